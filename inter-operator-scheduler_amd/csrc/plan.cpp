@@ -589,6 +589,28 @@ private:
         return r ? r->at + ((offset & ~kRegionTag) - r->voff) : offset;
     }
 
+    // The prefix ends where its work covers the time the input takes on the link (57 GB/s measured), both estimated: 100 TFLOP/s
+    // and 3.5 TB/s are what the kernels of these layers reach at the batches in question.
+    void choose_prefix() {
+        constexpr double kMinBytes = 2 << 20;
+        const double input = 4.0 * batch_ * (double)plan_.input.image_floats();
+        plan_.prefix_stages = 0;
+        if (batch_ < 16 || input < kMinBytes) return;
+        double covered = 0.0;
+        for (const auto &groups : plan_.stages) {
+            if (groups.size() != 1 || covered > 1.2 * input / 57e9) break;
+            bool plain = true;
+            for (int index : groups[0]) {
+                const PlanOp &op = plan_.ops[index];
+                plain = plain && op.srcs.empty() && !op.has_residual && op.bias_conv < 0 &&
+                        (op.kind == OpKind::ConvMfma || op.kind == OpKind::ConvDirect || op.kind == OpKind::Pool);
+                covered += std::max(op.flops / 100e12, op.bytes / 3.5e12);
+            }
+            if (!plain) break;
+            plan_.prefix_stages++;
+        }
+    }
+
     // Lifetimes from the stages of the operations that read or write a region; then first-fit placement, largest regions
     // first, where two regions may share addresses when their lifetimes do not intersect (all operations of a stage have
     // finished before the next stage starts, under every executor); finally every offset of the plan is rewritten.
@@ -600,6 +622,14 @@ private:
             for (const ViewRef &v : op.srcs) touch(v.offset, op.stage);
             if (op.has_residual) touch(op.residual.offset, op.stage);
             if (op.conv >= 0 && plan_.convs[op.conv].ws_floats > 0) touch(plan_.convs[op.conv].ws_off, op.stage);
+        }
+        choose_prefix();
+        for (const PlanOp &op : plan_.ops) {   // parts of the batch are in different stages of the prefix at the same time
+            if (op.stage >= plan_.prefix_stages) continue;
+            for (int stage : {0, plan_.prefix_stages - 1}) {
+                touch(op.in.offset, stage);
+                touch(op.out.offset, stage);
+            }
         }
         if (Region *r = region_of(plan_.output.offset)) r->pinned = true;
         const bool reuse = planner_arena_reuse();

@@ -98,6 +98,9 @@ struct Plan {
     size_t activation_floats_without_reuse = 0;
     std::set<std::string> overwritten;
     bool output_single_group = true;                     // the last stage has one group
+    // Leading stages of one group that may run on a part of the batch at a time, while the images behind it are still on their
+    // way to the device (0: the input is too small for that); their tensors share no memory with each other.
+    int prefix_stages = 0;
 };
 
 enum class PlanMode { Graph, Block, Stage };

@@ -12,6 +12,7 @@
 
 #include "plan.h"
 #include "fused.h"
+#include "host_io.h"
 
 namespace ios {
 
@@ -30,6 +31,11 @@ public:
     const std::string &name() const { return name_; }
     const std::string &arch() const { return arch_; }
     hipStream_t stream(int group) { return streams_[group]; }
+    HostStage &stage() { return stage_; }
+    // the session whose last pass left its result in stage() (null: none)
+    const void *result_owner = nullptr;
+    // the sessions that laid out the shared arena and the static scratch last
+    const void *shared_owner = nullptr, *static_owner = nullptr;
 
     // a process-wide arena reused by the stateless latency / inference entry points
     float *shared_arena(size_t floats);
@@ -60,6 +66,8 @@ public:
     int forced_variant() const { return forced_variant_; }
     int forced_split_k() const { return forced_split_k_; }
     std::string info_json() const;
+    // changes with everything but the options that the choice of kernel configurations depends on
+    std::string plan_token() const { return std::to_string(tuned.size()) + (xcd_usable_ ? "x" : "-"); }
 
     // Kernel configuration for a matrix-path convolution: the measured best when autotuning is on (cached
     // per problem signature for the life of the process, and in the file named by IOS_TUNE_CACHE when set),
@@ -103,6 +111,7 @@ private:
     int num_cus_ = 0;
     std::string name_, arch_;
     hipStream_t streams_[kMaxGroups];
+    HostStage stage_;
     float *arena_ = nullptr;
     size_t arena_floats_ = 0;
     void *table_ = nullptr;
@@ -121,7 +130,9 @@ public:
     // a time), or the static scratch array (one at a time; such a session allocates nothing, creates no events, and
     // issues every operator on the main stream in schedule order whatever the executor option says).
     enum class Storage { Own, Shared, Static };
-    Session(Plan plan, Storage storage);
+    // pack_filters: lay out whatever the filter regions hold, so that a pass without weights reads initialised memory; a
+    // caller that sets the weights next packs with them (see finish_weights)
+    Session(Plan plan, Storage storage, bool pack_filters = true);
     Session(Plan plan, bool shared) : Session(std::move(plan), shared ? Storage::Shared : Storage::Own) {}
     ~Session();
     void release() noexcept;   // frees device memory, events and the captured graph; safe to call twice
@@ -131,9 +142,12 @@ public:
     const Plan &plan() const { return plan_; }
 
     void set_input(const float *host);
-    // returns false (and prints like the reference runtime) when no convolution has that name
-    bool set_conv_weights(const char *name, const float *weight, const float *bias);
+    // prints like the reference runtime, and skips the entry, when no convolution has a name
+    void set_conv_weights(int count, char **names, float **weights, float **biases);
+    void finish_weights();   // packs the filters of the convolutions that neither the constructor nor set_conv_weights has packed
     void get_output(float *host);
+    // set_input, set_conv_weights, run and get_output in one, the pass following the weights as they arrive
+    void infer(const float *input, int count, char **names, float **weights, float **biases, float *output);
     void get_tensor(const std::string &name, float *host);
 
     void run();   // one forward pass, synchronised
@@ -161,17 +175,29 @@ public:
     void profile_launches(int warmup, int repeat, float *ms, int capacity);
 
 private:
-    void setup();
-    void tune_convs();
-    void launch_op(const PlanOp &op, int group);   // on stream `group` of the pool
+    void setup(bool pack_filters);
+    void pack(const PlanConv &conv, hipStream_t stream);
+    void ensure_timers();
+    void ensure_fork_events();
+    // on stream `group` of the pool; images > 0: on that many images of the batch from `first` on
+    void launch_op(const PlanOp &op, int group, int first = 0, int images = 0);
     unsigned *counters_of(const PlanConv &c) const;
     const float *bias_of(const PlanConv &c) const { return base_ + (c.linear ? c.zero_bias_off : c.bias_off); }
-    void enqueue(bool stage_events);   // issue one forward pass according to the execution mode
-    void enqueue_streams(bool stage_events);
-    void enqueue_fused(bool stage_events);
-    void enqueue_serial();
+    void ready_executor();
+    void enqueue(size_t first, bool stage_events);   // issue the stages from `first` on according to the execution mode
+    void enqueue_stage(size_t s);
+    void enqueue_stage_streams(size_t s);
+    void enqueue_stage_fused(size_t s);
+    void enqueue_stage_serial(size_t s);
+    void enqueue_prefix(size_t stages);
+    size_t direct_stages() const;
     void build_fused();
-    void build_graph();
+    void build_graph(size_t first);
+    void drop_graph() noexcept;
+    void settle();
+    void finish_pass();
+    void advance();
+    void attach();
     void copy_out(const ViewRef &view, float *host);
     TensorView tv(const ViewRef &v) const;
 
@@ -180,6 +206,11 @@ private:
     float *base_ = nullptr;
     bool owns_memory_ = false;
     bool static_ = false;
+    std::vector<char> packed_;      // per convolution: its packed filters are laid out
+    int arriving_ = 0, arriving_images_ = 0;   // parts of the input on their way, images per part
+    bool advance_ = false;          // set_conv_weights issues the stages whose filters it has packed
+    size_t next_stage_ = 0;
+    bool fetches_result_ = true;    // the caller has fetched the last result (or there was none): the next pass delivers its own
     std::vector<hipEvent_t> fork_events_;                 // per stage (multi-group stages only)
     std::vector<std::vector<hipEvent_t>> join_events_;    // per stage, per extra group
     std::vector<hipEvent_t> stage_events_;                // per stage, profile mode

@@ -58,6 +58,7 @@ DeviceContext::DeviceContext() {
     for (int i = 0; i < kMaxGroups; i++) IOS_HIP(hipStreamCreateWithFlags(&streams_[i], hipStreamNonBlocking));
     // the library runs on device 0 only, which is current here: its copy of the array is the one ever used
     IOS_HIP(hipGetSymbolAddress(reinterpret_cast<void **>(&static_scratch_), HIP_SYMBOL(scratch)));
+    stage_.create();
     probe_xcd_placement();
     const char *mode = getenv("IOS_EXECUTOR");
     if (mode != nullptr) set_option("executor", mode);
@@ -472,24 +473,24 @@ std::string DeviceContext::info_json() const {
 }
 
 // ---- session ---------------------------------------------------------------------------------------------------------
-Session::Session(Plan plan, Storage storage) : plan_(std::move(plan)), ctx_(DeviceContext::get()) {
+Session::Session(Plan plan, Storage storage, bool pack_filters) : plan_(std::move(plan)), ctx_(DeviceContext::get()) {
     if (storage == Storage::Static) {
         const size_t need = plan_.arena_floats * sizeof(float);
         if (need > DeviceContext::static_scratch_bytes())
             throw std::runtime_error("graph needs " + std::to_string(need) + " bytes of device memory at this batch size; the static scratch of "
                                      "graph_inference_no_alloc holds " + std::to_string(DeviceContext::static_scratch_bytes()));
         base_ = ctx_.static_scratch();
-        owns_memory_ = false;
         static_ = true;
+        ctx_.static_owner = this;
     } else if (storage == Storage::Shared) {
         base_ = ctx_.shared_arena(plan_.arena_floats);
-        owns_memory_ = false;
+        ctx_.shared_owner = this;
     } else {
         IOS_HIP(hipMalloc(reinterpret_cast<void **>(&base_), std::max<size_t>(plan_.arena_floats, 64) * sizeof(float)));
         owns_memory_ = true;
     }
     try {
-        setup();
+        setup(pack_filters);
     } catch (...) {
         release();   // the destructor does not run for a constructor that throws
         throw;
@@ -499,20 +500,21 @@ Session::Session(Plan plan, Storage storage) : plan_(std::move(plan)), ctx_(Devi
 Session::~Session() { release(); }
 
 void Session::release() noexcept {
+    if (ctx_.result_owner == this) ctx_.result_owner = nullptr;
     (void)hipDeviceSynchronize();
-    if (graph_exec_ != nullptr) (void)hipGraphExecDestroy(graph_exec_);
-    if (graph_ != nullptr) (void)hipGraphDestroy(graph_);
+    drop_graph();
+    if (ctx_.shared_owner == this) ctx_.shared_owner = nullptr;
+    if (ctx_.static_owner == this) ctx_.static_owner = nullptr;
     for (hipEvent_t e : fork_events_)
         if (e != nullptr) (void)hipEventDestroy(e);
     for (auto &per_stage : join_events_)
-        for (hipEvent_t e : per_stage) (void)hipEventDestroy(e);
+        for (hipEvent_t e : per_stage)
+            if (e != nullptr) (void)hipEventDestroy(e);
     for (hipEvent_t e : stage_events_) (void)hipEventDestroy(e);
     if (start_ != nullptr) (void)hipEventDestroy(start_);
     if (stop_ != nullptr) (void)hipEventDestroy(stop_);
     if (owns_memory_ && fused_items_ != nullptr) (void)hipFree(fused_items_);
     if (owns_memory_ && base_ != nullptr) (void)hipFree(base_);
-    graph_exec_ = nullptr;
-    graph_ = nullptr;
     fork_events_.clear();
     join_events_.clear();
     stage_events_.clear();
@@ -531,80 +533,127 @@ TensorView Session::tv(const ViewRef &v) const {
     return t;
 }
 
-void Session::setup() {
+void Session::pack(const PlanConv &conv, hipStream_t stream) {
+    if (conv.matrix_path) launch_pack_filters(conv.problem, conv.launch, base_ + conv.weight_off, base_ + conv.packed_off, stream);
+    packed_[&conv - plan_.convs.data()] = 1;
+}
+
+void Session::setup(bool pack_filters) {
     hipStream_t main = ctx_.stream(0);
     if (owns_memory_) launch_fill_pattern(base_, plan_.arena_floats, 0x2468aceu, main);
+    packed_.assign(plan_.convs.size(), 0);
     for (const PlanConv &conv : plan_.convs) {
         // a convolution in front of the average pool it was exchanged with adds zeros; the pool adds the bias
         if (conv.linear) launch_fill_u32(reinterpret_cast<unsigned *>(base_ + conv.zero_bias_off), (size_t)conv.problem.OC, 0u, main);
-        if (!conv.matrix_path) continue;
-        // the probes never upload filters: pack whatever the filter region holds so that the matrix
-        // path reads initialised memory
-        launch_pack_filters(conv.problem, conv.launch, base_ + conv.weight_off, base_ + conv.packed_off, main);
         // split-K tickets start at zero; every launch leaves them at zero again
-        if (conv.ctr_count > 0) launch_fill_u32(reinterpret_cast<unsigned *>(base_ + conv.ctr_off), conv.ctr_count, 0u, main);
+        if (conv.matrix_path && conv.ctr_count > 0) launch_fill_u32(reinterpret_cast<unsigned *>(base_ + conv.ctr_off), conv.ctr_count, 0u, main);
     }
+    if (pack_filters) finish_weights();
+}
+
+void Session::finish_weights() {
+    for (size_t c = 0; c < plan_.convs.size(); c++)
+        if (!packed_[c]) pack(plan_.convs[c], ctx_.stream(0));
+}
+
+// events of the stream executors, created when the first pass needs them (a static session creates none)
+void Session::ensure_fork_events() {
     const size_t num_stages = plan_.stages.size();
-    if (static_) {   // no events: everything is issued on the main stream and the host waits for the stream
-        IOS_HIP(hipStreamSynchronize(main));
-        return;
-    }
+    if (fork_events_.size() == num_stages) return;
     fork_events_.assign(num_stages, nullptr);
     join_events_.assign(num_stages, {});
     for (size_t s = 0; s < num_stages; s++) {
         const size_t groups = plan_.stages[s].size();
         if (groups <= 1) continue;
         IOS_HIP(hipEventCreateWithFlags(&fork_events_[s], hipEventDisableTiming));
-        join_events_[s].resize(groups - 1);
+        join_events_[s].assign(groups - 1, nullptr);
         for (hipEvent_t &e : join_events_[s]) IOS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-    IOS_HIP(hipEventCreate(&start_));
-    IOS_HIP(hipEventCreate(&stop_));
-    IOS_HIP(hipStreamSynchronize(main));
+}
+
+void Session::ensure_timers() {
+    if (start_ == nullptr) IOS_HIP(hipEventCreate(&start_));
+    if (stop_ == nullptr) IOS_HIP(hipEventCreate(&stop_));
 }
 
 void Session::set_input(const float *host) {
     if (host == nullptr) throw std::runtime_error("input pointer is null");
-    hipStream_t main = ctx_.stream(0);
     const ViewRef &in = plan_.input;
-    IOS_HIP(hipMemcpyAsync(base_ + in.offset, host, (size_t)plan_.batch * in.image_floats() * sizeof(float), hipMemcpyHostToDevice, main));
-    IOS_HIP(hipStreamSynchronize(main));
+    const size_t image = in.image_floats() * sizeof(float), total = (size_t)plan_.batch * image;
+    if (plan_.prefix_stages > 0 && total <= HostStage::kBatch && !static_) {
+        // the first stages of the next pass start on the images that are there while the others are still on their way
+        arriving_images_ = (plan_.batch + HostStage::kMaxChunks - 1) / HostStage::kMaxChunks;
+        arriving_ = (plan_.batch + arriving_images_ - 1) / arriving_images_;
+        ctx_.stage().upload_chunks(base_ + in.offset, host, total, (size_t)arriving_images_ * image, ctx_.stream(1), ctx_.stream(0));
+        return;
+    }
+    ctx_.stage().upload(base_ + in.offset, host, total, ctx_.stream(0));
 }
 
-bool Session::set_conv_weights(const char *name, const float *weight, const float *bias) {
-    auto it = plan_.conv_index.find(name ? name : "");
-    if (it == plan_.conv_index.end()) {
-        printf("%s not found\n", name ? name : "(null)");
-        return false;
+// everything the next kernels of the main stream may read has arrived
+void Session::settle() {
+    if (arriving_ > 0) ctx_.stage().arrived(arriving_ - 1, ctx_.stream(0));
+    arriving_ = 0;
+}
+
+// Filters and biases lie next to each other in the arena (the planner reserves them first, in network order): they are gathered
+// by several threads and travel in large steps, on a stream of their own; the filters of a convolution are packed on the main
+// stream as soon as they have arrived.
+void Session::set_conv_weights(int count, char **names, float **weights, float **biases) {
+    std::vector<int> entry(plan_.convs.size(), -1);   // a name given twice: the last one counts
+    for (int i = 0; i < count; i++) {
+        auto it = plan_.conv_index.find(names[i] ? names[i] : "");
+        if (it == plan_.conv_index.end()) {
+            printf("%s not found\n", names[i] ? names[i] : "(null)");
+            continue;
+        }
+        if (weights[i] == nullptr || biases[i] == nullptr)
+            throw std::runtime_error(std::string("convolution '") + names[i] + "': weight or bias pointer is null");
+        entry[it->second] = i;
     }
-    if (weight == nullptr || bias == nullptr) throw std::runtime_error(std::string("convolution '") + name + "': weight or bias pointer is null");
-    const PlanConv &conv = plan_.convs[it->second];
-    const ConvProblem &p = conv.problem;
+    std::vector<int> order;
+    for (size_t c = 0; c < entry.size(); c++)
+        if (entry[c] >= 0) order.push_back((int)c);
+    std::sort(order.begin(), order.end(), [&](int a, int b) { return plan_.convs[a].weight_off < plan_.convs[b].weight_off; });
+    std::vector<HostStage::Piece> pieces;
+    std::vector<size_t> complete;   // per entry of `order`: the piece behind its bias
+    auto add = [&](size_t offset, size_t floats, const float *src) {
+        const size_t bytes = floats * sizeof(float);
+        for (size_t at = 0; at < bytes; at += HostCopier::kPiece)
+            pieces.push_back({offset * sizeof(float) + at, std::min(HostCopier::kPiece, bytes - at), reinterpret_cast<const char *>(src) + at});
+    };
+    for (int c : order) {   // (a filter lies in front of its bias)
+        const PlanConv &conv = plan_.convs[c];
+        add(conv.weight_off, (size_t)conv.problem.OC * conv.problem.K(), weights[entry[c]]);
+        add(conv.bias_off, (size_t)conv.problem.OC, biases[entry[c]]);
+        complete.push_back(pieces.size());
+    }
+    size_t next = 0;
     hipStream_t main = ctx_.stream(0);
-    IOS_HIP(hipMemcpyAsync(base_ + conv.weight_off, weight, (size_t)p.OC * p.K() * sizeof(float), hipMemcpyHostToDevice, main));
-    IOS_HIP(hipMemcpyAsync(base_ + conv.bias_off, bias, (size_t)p.OC * sizeof(float), hipMemcpyHostToDevice, main));
-    if (conv.matrix_path) launch_pack_filters(p, conv.launch, base_ + conv.weight_off, base_ + conv.packed_off, main);
-    IOS_HIP(hipStreamSynchronize(main));
-    return true;
+    ctx_.stage().upload_pieces(reinterpret_cast<char *>(base_), pieces, ctx_.stream(1), main, [&](size_t limit) {
+        for (; next < order.size() && complete[next] <= limit; next++) pack(plan_.convs[order[next]], main);
+        if (advance_) advance();
+    });
 }
 
 void Session::copy_out(const ViewRef &view, float *host) {
+    settle();
     hipStream_t main = ctx_.stream(0);
     const size_t image = view.image_floats();
     if (view.bstride == (long long)image) {
-        IOS_HIP(hipMemcpyAsync(host, base_ + view.offset, (size_t)plan_.batch * image * sizeof(float), hipMemcpyDeviceToHost, main));
-    } else {
-        for (int b = 0; b < plan_.batch; b++)
-            IOS_HIP(hipMemcpyAsync(host + (size_t)b * image, base_ + view.offset + (size_t)b * view.bstride, image * sizeof(float),
-                                   hipMemcpyDeviceToHost, main));
+        ctx_.stage().download(host, base_ + view.offset, (size_t)plan_.batch * image * sizeof(float), main);
+        return;
     }
-    IOS_HIP(hipStreamSynchronize(main));
+    for (int b = 0; b < plan_.batch; b++)
+        ctx_.stage().download(host + (size_t)b * image, base_ + view.offset + (size_t)b * view.bstride, image * sizeof(float), main);
 }
 
 void Session::get_output(float *host) {
     if (host == nullptr) throw std::runtime_error("output pointer is null");
     if (!plan_.output_single_group) throw std::runtime_error("the last stage of the schedule must have a single group");
-    copy_out(plan_.output, host);
+    fetches_result_ = true;
+    if (ctx_.result_owner == this) ctx_.stage().fetch(host, (size_t)plan_.batch * plan_.output.image_floats() * sizeof(float), ctx_.stream(0));
+    else copy_out(plan_.output, host);
 }
 
 void Session::get_tensor(const std::string &name, float *host) {
@@ -621,13 +670,21 @@ unsigned *Session::counters_of(const PlanConv &c) const {
     return reinterpret_cast<unsigned *>(base_ + c.ctr_off);
 }
 
-void Session::launch_op(const PlanOp &op, int group) {
+void Session::launch_op(const PlanOp &op, int group, int first, int images) {
     hipStream_t stream = ctx_.stream(group);
+    const int count = images > 0 ? images : plan_.batch;
+    auto part = [&](const ViewRef &v) {   // the images this launch works on
+        TensorView t = tv(v);
+        t.ptr += (long long)first * v.bstride;
+        return t;
+    };
     switch (op.kind) {
         case OpKind::ConvMfma: {
             const PlanConv &c = plan_.convs[op.conv];
-            const TensorView residual = op.has_residual ? tv(op.residual) : TensorView{};
-            launch_conv_mfma(c.problem, c.launch, tv(op.in), base_ + c.packed_off, bias_of(c), tv(op.out),
+            ConvProblem p = c.problem;
+            p.B = count;
+            const TensorView residual = op.has_residual ? part(op.residual) : TensorView{};
+            launch_conv_mfma(p, c.launch, part(op.in), base_ + c.packed_off, bias_of(c), part(op.out),
                              c.ws_floats ? base_ + c.ws_off : nullptr, ctx_.split_reduce(counters_of(c), group, !capturing_forks_), stream,
                              op.has_residual ? &residual : nullptr,
                              op.post_relu != 0);
@@ -635,72 +692,110 @@ void Session::launch_op(const PlanOp &op, int group) {
         }
         case OpKind::ConvDepthwise: {
             const PlanConv &c = plan_.convs[op.conv];
+            ConvProblem p = c.problem;
+            p.B = count;
             TensorView more[kMaxNaryInputs];
-            for (size_t i = 1; i < op.srcs.size(); i++) more[i - 1] = tv(op.srcs[i]);
-            launch_dwconv(c.problem, tv(op.in), base_ + c.weight_off, bias_of(c), tv(op.out), stream, more,
+            for (size_t i = 1; i < op.srcs.size(); i++) more[i - 1] = part(op.srcs[i]);
+            launch_dwconv(p, part(op.in), base_ + c.weight_off, bias_of(c), part(op.out), stream, more,
                           op.srcs.empty() ? 0 : (int)op.srcs.size() - 1);
             break;
         }
         case OpKind::ConvDirect: {
             const PlanConv &c = plan_.convs[op.conv];
-            launch_conv_direct(c.problem, tv(op.in), base_ + c.weight_off, bias_of(c), tv(op.out), stream, c.thin);
+            ConvProblem p = c.problem;
+            p.B = count;
+            launch_conv_direct(p, part(op.in), base_ + c.weight_off, bias_of(c), part(op.out), stream, c.thin);
             break;
         }
         case OpKind::Pool:
-            launch_pool(op.pool, tv(op.in), tv(op.out), stream, op.bias_conv >= 0 ? base_ + plan_.convs[op.bias_conv].bias_off : nullptr, op.act);
+        case OpKind::GlobalPool: {
+            PoolProblem p = op.pool;
+            p.B = count;
+            if (op.kind == OpKind::GlobalPool) launch_global_pool(p, part(op.in), part(op.out), stream);
+            else launch_pool(p, part(op.in), part(op.out), stream, op.bias_conv >= 0 ? base_ + plan_.convs[op.bias_conv].bias_off : nullptr, op.act);
             break;
-        case OpKind::GlobalPool: launch_global_pool(op.pool, tv(op.in), tv(op.out), stream); break;
+        }
         case OpKind::Nary: {
             NaryArgs a;
             a.count = (int)op.srcs.size();
             for (int i = 0; i < a.count; i++) {
-                a.src[i] = base_ + op.srcs[i].offset;
+                a.src[i] = part(op.srcs[i]).ptr;
                 a.src_bstride[i] = op.srcs[i].bstride;
             }
-            launch_nary(a, op.multiply, op.accumulate, op.act, plan_.batch, (long long)op.out.image_floats(), tv(op.out), stream);
+            launch_nary(a, op.multiply, op.accumulate, op.act, count, (long long)op.out.image_floats(), part(op.out), stream);
             break;
         }
-        case OpKind::Unary: launch_unary(tv(op.in), tv(op.out), op.act, plan_.batch, stream); break;
+        case OpKind::Unary: launch_unary(part(op.in), part(op.out), op.act, count, stream); break;
     }
 }
 
-void Session::enqueue_streams(bool stage_events) {
+void Session::enqueue_stage_streams(size_t s) {
     hipStream_t main = ctx_.stream(0);
-    for (size_t s = 0; s < plan_.stages.size(); s++) {
-        const auto &groups = plan_.stages[s];
-        const bool fork = groups.size() > 1;
-        if (fork) {
-            IOS_HIP(hipEventRecord(fork_events_[s], main));
-            for (size_t g = 1; g < groups.size(); g++) IOS_HIP(hipStreamWaitEvent(ctx_.stream((int)g), fork_events_[s], 0));
+    const auto &groups = plan_.stages[s];
+    const bool fork = groups.size() > 1;
+    if (fork) {
+        IOS_HIP(hipEventRecord(fork_events_[s], main));
+        for (size_t g = 1; g < groups.size(); g++) IOS_HIP(hipStreamWaitEvent(ctx_.stream((int)g), fork_events_[s], 0));
+    }
+    for (size_t g = 0; g < groups.size(); g++)
+        for (int op : groups[g]) launch_op(plan_.ops[op], (int)g);
+    if (fork) {
+        for (size_t g = 1; g < groups.size(); g++) {
+            IOS_HIP(hipEventRecord(join_events_[s][g - 1], ctx_.stream((int)g)));
+            IOS_HIP(hipStreamWaitEvent(main, join_events_[s][g - 1], 0));
         }
-        for (size_t g = 0; g < groups.size(); g++)
-            for (int op : groups[g]) launch_op(plan_.ops[op], (int)g);
-        if (fork) {
-            for (size_t g = 1; g < groups.size(); g++) {
-                IOS_HIP(hipEventRecord(join_events_[s][g - 1], ctx_.stream((int)g)));
-                IOS_HIP(hipStreamWaitEvent(main, join_events_[s][g - 1], 0));
-            }
-        }
-        if (stage_events) IOS_HIP(hipEventRecord(stage_events_[s], main));
     }
 }
 
-void Session::enqueue_serial() {
-    hipStream_t main = ctx_.stream(0);
-    for (const auto &groups : plan_.stages)
-        for (const auto &group : groups)
-            for (int op : group) launch_op(plan_.ops[op], 0);
+void Session::enqueue_stage_serial(size_t s) {
+    for (const auto &group : plan_.stages[s])
+        for (int op : group) launch_op(plan_.ops[op], 0);
 }
 
-void Session::enqueue(bool stage_events) {
-    if (static_) {
-        if (stage_events) throw std::runtime_error("a session in the static scratch cannot profile stages");
-        enqueue_serial();
+void Session::enqueue_stage(size_t s) {
+    if (static_) enqueue_stage_serial(s);
+    else if (ctx_.fused_executor()) enqueue_stage_fused(s);
+    else enqueue_stage_streams(s);
+}
+
+// what enqueue_stage needs beyond the plan: allocations, copies and events stay outside a graph capture
+void Session::ready_executor() {
+    if (static_) return;
+    if (ctx_.fused_executor()) build_fused();
+    else ensure_fork_events();
+}
+
+// issues the stages from `first` on in order
+void Session::enqueue(size_t first, bool stage_events) {
+    if (static_ && stage_events) throw std::runtime_error("a session in the static scratch cannot profile stages");
+    ready_executor();
+    for (size_t s = first; s < plan_.stages.size(); s++) {
+        enqueue_stage(s);
+        if (stage_events) IOS_HIP(hipEventRecord(stage_events_[s], ctx_.stream(0)));
+    }
+}
+
+// The leading stages, of one group each: on the whole batch, or part by part as the images arrive.
+void Session::enqueue_prefix(size_t stages) {
+    if (arriving_ == 0 || plan_.prefix_stages == 0) {
+        settle();
+        for (size_t s = 0; s < stages; s++) enqueue_stage(s);
         return;
     }
-    const ExecMode mode = ctx_.exec_mode();
-    if (mode == ExecMode::Fused || mode == ExecMode::FusedGraph) enqueue_fused(stage_events);
-    else enqueue_streams(stage_events);
+    // Two parts: staging a batch takes about as long as half of its transfer, so the first half is there, and the second arrives
+    // while the first is worked on.  (Eight parts, one per chunk, run the kernels on an eighth of the pixels: 0.4 ms slower.)
+    const size_t split = (size_t)plan_.prefix_stages;
+    for (int part = 0, chunk = 0; part < 2; part++) {
+        const int begin = chunk * arriving_images_;
+        chunk = part == 0 ? (arriving_ + 1) / 2 : arriving_;
+        const int images = std::min(chunk * arriving_images_, plan_.batch) - begin;
+        if (images <= 0) continue;
+        ctx_.stage().arrived(chunk - 1, ctx_.stream(0));
+        for (size_t s = 0; s < split; s++)
+            for (int op : plan_.stages[s][0]) launch_op(plan_.ops[op], 0, begin, images);
+    }
+    arriving_ = 0;
+    for (size_t s = split; s < stages; s++) enqueue_stage(s);
 }
 
 // ---- fused stage launches -----------------------------------------------------------------------------------------
@@ -894,37 +989,50 @@ void Session::build_fused() {
     if (!items.empty()) {
         if (owns_memory_) IOS_HIP(hipMalloc(&fused_items_, items.size() * sizeof(WorkItem)));
         else fused_items_ = ctx_.shared_table(items.size() * sizeof(WorkItem));
-        IOS_HIP(hipMemcpyAsync(fused_items_, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, ctx_.stream(0)));
-        IOS_HIP(hipStreamSynchronize(ctx_.stream(0)));
+        ctx_.stage().upload(fused_items_, items.data(), items.size() * sizeof(WorkItem), ctx_.stream(0));
     }
     fused_built_ = true;
 }
 
-void Session::enqueue_fused(bool stage_events) {
-    build_fused();
-    hipStream_t main = ctx_.stream(0);
+void Session::enqueue_stage_fused(size_t s) {
+    if (fused_stages_[s].empty()) {
+        enqueue_stage_serial(s);
+        return;
+    }
     const WorkItem *items = static_cast<const WorkItem *>(fused_items_);
-    for (size_t s = 0; s < plan_.stages.size(); s++) {
-        if (fused_stages_[s].empty()) {
-            for (const auto &group : plan_.stages[s])
-                for (int op : group) launch_op(plan_.ops[op], 0);
-        } else {
-            for (const FusedLaunch &l : fused_stages_[s]) {
-                if (l.single_op >= 0) launch_op(plan_.ops[l.single_op], 0);
-                else launch_fused(l.threads, items + l.first_item, fused_items_host_.data() + l.first_item, l.header, l.total_blocks, l.smem_bytes, ctx_.num_cus(), main);
-            }
-        }
-        if (stage_events) IOS_HIP(hipEventRecord(stage_events_[s], main));
+    for (const FusedLaunch &l : fused_stages_[s]) {
+        if (l.single_op >= 0) launch_op(plan_.ops[l.single_op], 0);
+        else launch_fused(l.threads, items + l.first_item, fused_items_host_.data() + l.first_item, l.header, l.total_blocks, l.smem_bytes, ctx_.num_cus(), ctx_.stream(0));
     }
 }
 
-void Session::build_graph() {
+// Leading stages that the graph executors launch directly.  Handing a graph to the device takes the host 14-22 us before its
+// first kernel starts (measured for 1 to 60 kernels; a kernel launch takes 1.6-2.5 us), so the first few kernels go ahead of
+// it and the device works on them meanwhile; a pass of a handful of kernels needs no graph at all.
+size_t Session::direct_stages() const {
+    constexpr size_t kAhead = 4, kNoGraph = 8;
+    auto launches_of = [&](size_t s) {
+        size_t ops = 0;
+        for (const auto &group : plan_.stages[s]) ops += group.size();
+        return ctx_.fused_executor() && !fused_stages_[s].empty() ? fused_stages_[s].size() : ops;
+    };
+    size_t total = 0, ahead = 0, stages = 0;
+    for (size_t s = 0; s < plan_.stages.size(); s++) total += launches_of(s);
+    if (ctx_.fused_executor() && total <= kNoGraph) return plan_.stages.size();
+    while (stages < plan_.stages.size() && ahead < kAhead) {
+        if (!ctx_.fused_executor() && plan_.stages[stages].size() > 1) break;
+        ahead += launches_of(stages++);
+    }
+    return std::max(stages, (size_t)plan_.prefix_stages);
+}
+
+void Session::build_graph(size_t first) {
     hipStream_t main = ctx_.stream(0);
     IOS_HIP(hipStreamBeginCapture(main, hipStreamCaptureModeRelaxed));
     // the stream executor forks inside the capture, and the replay runs the branches on streams of its own choice
     capturing_forks_ = ctx_.exec_mode() == ExecMode::Graph;
     try {
-        enqueue(false);
+        enqueue(first, false);
         capturing_forks_ = false;
     } catch (...) {
         capturing_forks_ = false;
@@ -937,33 +1045,105 @@ void Session::build_graph() {
     IOS_HIP(hipGraphInstantiate(&graph_exec_, graph_, nullptr, nullptr, 0));
 }
 
+void Session::drop_graph() noexcept {
+    if (graph_exec_ != nullptr) (void)hipGraphExecDestroy(graph_exec_);
+    if (graph_ != nullptr) (void)hipGraphDestroy(graph_);
+    graph_exec_ = nullptr;
+    graph_ = nullptr;
+}
+
 void Session::forward() {
-    if (static_) {
-        enqueue_serial();
+    if (ctx_.result_owner == this) ctx_.result_owner = nullptr;
+    ready_executor();
+    const ExecMode mode = ctx_.exec_mode();
+    if (static_ || (mode != ExecMode::Graph && mode != ExecMode::FusedGraph)) {
+        const size_t prefix = (size_t)plan_.prefix_stages;
+        enqueue_prefix(prefix);
+        enqueue(prefix, false);
         return;
     }
-    const ExecMode mode = ctx_.exec_mode();
-    if (mode == ExecMode::Graph || mode == ExecMode::FusedGraph) {
-        if (graph_exec_ != nullptr && graph_mode_ != mode) {   // the option changed since the capture
-            IOS_HIP(hipGraphExecDestroy(graph_exec_));
-            IOS_HIP(hipGraphDestroy(graph_));
-            graph_exec_ = nullptr;
-            graph_ = nullptr;
-        }
-        if (graph_exec_ == nullptr) {
-            if (mode == ExecMode::FusedGraph) build_fused();   // allocations and copies stay outside the capture
-            build_graph();
-            graph_mode_ = mode;
-        }
-        IOS_HIP(hipGraphLaunch(graph_exec_, ctx_.stream(0)));
-    } else {
-        enqueue(false);
+    const size_t direct = direct_stages();
+    if (graph_exec_ != nullptr && graph_mode_ != mode) drop_graph();   // the option changed since the capture
+    if (graph_exec_ == nullptr && direct < plan_.stages.size()) {
+        build_graph(direct);
+        graph_mode_ = mode;
     }
+    enqueue_prefix(direct);
+    if (direct < plan_.stages.size()) IOS_HIP(hipGraphLaunch(graph_exec_, ctx_.stream(0)));
 }
 
 void Session::run() {
     forward();
-    synchronize();
+    finish_pass();
+}
+
+// waits for the pass that was queued last
+void Session::finish_pass() {
+    // A result of a few pages costs the last kernel nothing; a larger one travels with the pass unless the caller has left the
+    // one before where it was (it is then copied when it is asked for).
+    constexpr size_t kAlways = size_t(64) << 10;
+    const size_t bytes = (size_t)plan_.batch * plan_.output.image_floats() * sizeof(float);
+    const bool deliver = plan_.output_single_group && (bytes <= kAlways || (fetches_result_ && bytes <= HostStage::kResult));
+    fetches_result_ = false;
+    HostStage::Result result;
+    if (deliver) result = {base_ + plan_.output.offset, plan_.batch, (long long)plan_.output.image_floats(), plan_.output.bstride};
+    hipStream_t main = ctx_.stream(0);
+    ctx_.stage().signal(result, main);
+    ctx_.stage().wait(main);
+    ctx_.check_xcd_fault();
+    if (deliver) ctx_.result_owner = this;
+}
+
+// One inference with everything crossing the boundary.  The weights of a network take longer on the link than the pass itself
+// (87 MB, 1.5 ms against 0.4 ms for Inception-v3 at batch 1), so a stage is issued as soon as the filters of its convolutions
+// have been: the pass runs behind the transfer and ends with the stages of the last part.
+void Session::infer(const float *input, int count, char **names, float **weights, float **biases, float *output) {
+    attach();
+    if (ctx_.result_owner == this) ctx_.result_owner = nullptr;
+    set_input(input);
+    settle();
+    ready_executor();
+    packed_.assign(plan_.convs.size(), 0);
+    next_stage_ = 0;
+    advance_ = true;
+    try {
+        set_conv_weights(count, names, weights, biases);
+        finish_weights();
+        advance();
+    } catch (...) {
+        advance_ = false;
+        throw;
+    }
+    advance_ = false;
+    fetches_result_ = true;
+    finish_pass();
+    get_output(output);
+}
+
+// issues the stages whose filters are packed
+void Session::advance() {
+    for (; next_stage_ < plan_.stages.size(); next_stage_++) {
+        for (const auto &group : plan_.stages[next_stage_])
+            for (int op : group)
+                if (plan_.ops[op].conv >= 0 && !packed_[plan_.ops[op].conv]) return;
+        for (const auto &group : plan_.stages[next_stage_])
+            for (int op : group)
+                if (plan_.ops[op].bias_conv >= 0 && !packed_[plan_.ops[op].bias_conv]) return;
+        enqueue_stage(next_stage_);
+    }
+}
+
+// A session in memory that others use in between (the shared arena, the static scratch) lays out again what it keeps there.
+void Session::attach() {
+    if (owns_memory_) return;
+    float *base = static_ ? ctx_.static_scratch() : ctx_.shared_arena(plan_.arena_floats);
+    const void *&owner = static_ ? ctx_.static_owner : ctx_.shared_owner;
+    if (base == base_ && owner == this) return;
+    base_ = base;
+    owner = this;
+    drop_graph();
+    fused_built_ = false;
+    setup(false);
 }
 
 void Session::synchronize() {
@@ -974,6 +1154,7 @@ void Session::synchronize() {
 void Session::measure(int warmup, int number, int repeat, bool profile_stage, float *results, float *stage_results) {
     if (static_) throw std::runtime_error("a session in the static scratch has no timers");
     if (number < 1 || repeat < 1 || warmup < 0) throw std::runtime_error("measure: warmup >= 0, number >= 1, repeat >= 1 required");
+    ensure_timers();
     hipStream_t main = ctx_.stream(0);
     const size_t num_stages = plan_.stages.size();
     if (profile_stage && stage_events_.empty()) {
@@ -981,7 +1162,10 @@ void Session::measure(int warmup, int number, int repeat, bool profile_stage, fl
         for (hipEvent_t &e : stage_events_) IOS_HIP(hipEventCreate(&e));
     }
     auto pass = [&]() {
-        if (profile_stage) enqueue(true);
+        if (profile_stage) {
+            settle();
+            enqueue(0, true);
+        }
         else forward();
     };
     for (int i = 0; i < warmup; i++) pass();
@@ -1017,6 +1201,7 @@ void Session::measure(int warmup, int number, int repeat, bool profile_stage, fl
 void Session::measure_back_to_back(int warmup, int number, int repeat, float *results) {
     if (static_) throw std::runtime_error("a session in the static scratch has no timers");
     if (number < 1 || repeat < 1 || warmup < 0) throw std::runtime_error("measure: warmup >= 0, number >= 1, repeat >= 1 required");
+    ensure_timers();
     hipStream_t main = ctx_.stream(0);
     for (int i = 0; i < warmup; i++) forward();
     for (int i = 0; i < repeat; i++) {
@@ -1036,6 +1221,7 @@ void Session::measure_back_to_back(int warmup, int number, int repeat, float *re
 void Session::profile_ops(int warmup, int repeat, float *ms_out) {
     if (static_) throw std::runtime_error("a session in the static scratch has no timers");
     if (repeat < 1 || warmup < 0) throw std::runtime_error("profile_ops: warmup >= 0 and repeat >= 1 required");
+    ensure_timers();
     hipStream_t main = ctx_.stream(0);
     run();   // every operator sees the inputs it has in a real pass
     for (size_t i = 0; i < plan_.ops.size(); i++) {
@@ -1136,6 +1322,7 @@ void Session::profile_launches(int warmup, int repeat, float *ms_out, int capaci
     if (repeat < 1 || warmup < 0) throw std::runtime_error("profile_launches: warmup >= 0 and repeat >= 1 required");
     const std::vector<LaunchRecord> list = launches();
     if ((int)list.size() > capacity) throw std::runtime_error("profile_launches: output array too small");
+    ensure_timers();
     hipStream_t main = ctx_.stream(0);
     run();   // every launch sees the inputs it has in a real pass
     const WorkItem *items = static_cast<const WorkItem *>(fused_items_);

@@ -32,13 +32,14 @@ def c_ndarray(a: np.ndarray):
 
 def c_ndarray_list(arrays: List[Optional[np.ndarray]]):
     """``float **``: element i points at arrays[i] (or is NULL when arrays[i] is not an ndarray)."""
-    pointers = [a.ctypes.data_as(ctypes.c_void_p) if isinstance(a, np.ndarray) else ctypes.c_void_p(None)
-                for a in arrays]
+    pointers = [a.ctypes.data if isinstance(a, np.ndarray) else None for a in arrays]
     return (ctypes.c_void_p * len(arrays))(*pointers)
 
 
 def as_f32(a) -> np.ndarray:
     """C-contiguous float32 view or copy of ``a``."""
+    if type(a) is np.ndarray and a.dtype == np.float32 and a.flags.c_contiguous:
+        return a
     return np.ascontiguousarray(a, dtype=np.float32)
 
 

@@ -13,6 +13,7 @@ resident on the device and the forward pass can be run, timed and profiled repea
 import ctypes
 import json
 import os
+import sys
 from typing import List, Optional
 
 import numpy as np
@@ -240,14 +241,9 @@ def graph_inference(graph: Graph, batch_size, input: np.ndarray, no_alloc=False)
         raise ValueError(f'input has shape {x.shape}, expected {expected}')
     output = np.empty(shape=(batch_size, *graph.blocks[-1].exit_node.output_shape), dtype=np.float32)
     names, weights, biases = _weight_lists(graph)
-    name_array = c_string_list(names)
     entry = handle.graph_inference_no_alloc if no_alloc else handle.graph_inference
-    status = entry(c_string(json.dumps(graph.export_config())), c_int(batch_size),
-                                    x.ctypes.data_as(ctypes.c_void_p), c_int(len(names)),
-                                    ctypes.cast(name_array, ctypes.POINTER(ctypes.c_char_p)),
-                                    ctypes.cast(c_ndarray_list(weights), ctypes.POINTER(ctypes.c_void_p)),
-                                    ctypes.cast(c_ndarray_list(biases), ctypes.POINTER(ctypes.c_void_p)),
-                                    output.ctypes.data_as(ctypes.c_void_p))
+    status = entry(c_string(json.dumps(graph.export_config())), batch_size, x.ctypes.data, len(names), c_string_list(names),
+                   c_ndarray_list(weights), c_ndarray_list(biases), output.ctypes.data)
     _check(status, 'graph_inference_no_alloc' if no_alloc else 'graph_inference')
     return output
 
@@ -261,7 +257,9 @@ class Session:
         self._handle = self._lib.ios_session_create(c_string(json.dumps(graph.export_config())), c_int(batch_size))
         if not self._handle:
             _check(1, 'ios_session_create')
+        self.input_shape = (batch_size, *graph.enter_node.output_shape)
         self.output_shape = (batch_size, *graph.blocks[-1].exit_node.output_shape)
+        self._results = []   # result arrays handed out, see _result_array
 
     def close(self):
         if self._handle:
@@ -282,19 +280,14 @@ class Session:
 
     def load_weights(self):
         names, weights, biases = _weight_lists(self.graph)
-        name_array = c_string_list(names)
-        _check(self._lib.ios_session_set_conv_weights(
-            self._handle, c_int(len(names)), ctypes.cast(name_array, ctypes.POINTER(ctypes.c_char_p)),
-            ctypes.cast(c_ndarray_list(weights), ctypes.POINTER(ctypes.c_void_p)),
-            ctypes.cast(c_ndarray_list(biases), ctypes.POINTER(ctypes.c_void_p))), 'ios_session_set_conv_weights')
+        _check(self._lib.ios_session_set_conv_weights(self._handle, len(names), c_string_list(names), c_ndarray_list(weights),
+                                                      c_ndarray_list(biases)), 'ios_session_set_conv_weights')
 
     def set_input(self, x: np.ndarray):
         x = as_f32(x)
-        expected = (self.batch_size, *self.graph.enter_node.output_shape)
-        if tuple(x.shape) != tuple(expected):
-            raise ValueError(f'input has shape {x.shape}, expected {expected}')
-        _check(self._lib.ios_session_set_input(self._handle, x.ctypes.data_as(ctypes.c_void_p)),
-               'ios_session_set_input')
+        if x.shape != self.input_shape:
+            raise ValueError(f'input has shape {x.shape}, expected {self.input_shape}')
+        _check(self._lib.ios_session_set_input(self._handle, x.ctypes.data), 'ios_session_set_input')
 
     def run(self):
         _check(self._lib.ios_session_run(self._handle), 'ios_session_run')
@@ -306,10 +299,22 @@ class Session:
     def synchronize(self):
         _check(self._lib.ios_session_synchronize(self._handle), 'ios_session_synchronize')
 
+    def _result_array(self) -> np.ndarray:
+        """
+        An uninitialised array for a result.  A large one that the caller has let go of (nothing but this list refers to it)
+        is handed out again: touching the fresh pages of a new 2 MB array takes longer than copying the result into it.
+        """
+        for array in self._results:
+            if sys.getrefcount(array) == 3:   # the list, the loop variable and the argument of getrefcount
+                return array
+        array = np.empty(self.output_shape, dtype=np.float32)
+        if array.nbytes >= 1 << 16:
+            self._results = self._results[-1:] + [array]
+        return array
+
     def output(self) -> np.ndarray:
-        out = np.empty(self.output_shape, dtype=np.float32)
-        _check(self._lib.ios_session_get_output(self._handle, out.ctypes.data_as(ctypes.c_void_p)),
-               'ios_session_get_output')
+        out = self._result_array()
+        _check(self._lib.ios_session_get_output(self._handle, out.ctypes.data), 'ios_session_get_output')
         return out
 
     def tensor(self, node: Node) -> np.ndarray:

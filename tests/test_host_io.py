@@ -1,0 +1,101 @@
+"""Transfers between a caller's arrays and the device at the sizes where the paths of csrc/host_io.hip change over."""
+import numpy as np
+import pytest
+
+import ios
+from ios.contrib import ios_runtime as rt
+from ios.ir import Graph
+
+pytestmark = pytest.mark.gpu
+
+
+def relu_graph(channels, height, width):
+    """y = max(x, 0): what comes back is what went there."""
+    ios.reset_name()
+    v = ios.placeholder((channels, height, width))
+    block = ios.Block(v.node)
+    ios.relu(block, [[v]], is_exit=True)
+    graph = Graph('t', v.node, [block])
+    graph.sequential_schedule()
+    return graph
+
+
+# floats: one value; the ends of one-kernel results (16 KB, 64 KB) and of results fetched by one thread; uploads in one, in several
+# and in shared-out steps; the largest result a pass delivers and the largest upload a kernel pulls (4 MB); beyond both
+@pytest.mark.parametrize('floats', [1, 4095, 4096, 4097, 16383, 16385, 49152, 49153, 65537, 98305, 393215, 393217, 1 << 20, (1 << 20) + 1, 3000001])
+def test_input_and_result_of_every_size(floats):
+    session = rt.Session(relu_graph(1, 1, floats) if floats < 65536 else relu_graph(floats // 65536 + 1, 256, 256), 1)
+    rng = np.random.default_rng(floats)
+    for _ in range(3):   # delivered, delivered again, and after a result that nobody fetched
+        x = rng.standard_normal(session.input_shape, dtype=np.float32)
+        session.set_input(x)
+        session.run()
+        assert np.array_equal(session.output(), np.maximum(x, 0))
+    session.run()
+    session.set_input(-x)
+    session.run()
+    assert np.array_equal(session.output(), np.maximum(-x, 0))
+
+
+@pytest.mark.parametrize('batch', [16, 17, 23, 64])
+@pytest.mark.parametrize('executor', ['fused', 'fused_graph', 'streams', 'graph'])
+def test_batches_arrive_in_parts(batch, executor):
+    """Leading stages on the parts of a batch, against the same images one by one."""
+    rt.set_option('executor', executor)
+    rt.set_option('autotune', 0)
+    try:
+        ios.reset_name()
+        v = ios.placeholder((3, 161, 159))
+        block = ios.Block(v.node)
+        w = ios.conv2d(block, [[v]], 19, (3, 3), (2, 2))
+        w = ios.pool2d(block, [[w]], 'max', (3, 3), (2, 2))
+        w = ios.conv2d(block, [[w]], 33, (3, 3), (1, 1), (1, 1))
+        ios.pool2d(block, [[w]], 'global_avg', is_exit=True)
+        graph = Graph('t', v.node, [block])
+        graph.init_weights(seed=1, scheme='he_normal_bias')
+        graph.sequential_schedule()
+        session, single = rt.Session(graph, batch), rt.Session(graph, 1)
+        session.load_weights()
+        single.load_weights()
+        rng = np.random.default_rng(batch)
+        for _ in range(2):
+            x = rng.standard_normal(session.input_shape, dtype=np.float32)
+            session.set_input(x)
+            session.run()
+            got = session.output()
+            session.run()   # the same input again, now resident
+            assert np.array_equal(got, session.output())
+            for i in (0, batch // 2 - 1, batch // 2, batch // 2 + 1, batch - 1):
+                single.set_input(x[i:i + 1])
+                single.run()
+                assert np.allclose(got[i:i + 1], single.output(), rtol=1e-4, atol=1e-5)
+    finally:
+        rt.set_option('executor', 'fused')
+        rt.set_option('autotune', 1)
+
+
+@pytest.mark.parametrize('no_alloc', [False, True])
+def test_inference_calls_take_turns(no_alloc):
+    """Networks, batches, weights and inputs change from call to call; every call computes with its own."""
+    graphs = []
+    for width in (20, 33, 48, 64, 70, 96):   # more documents than plans are kept
+        ios.reset_name()
+        v = ios.placeholder((5, 14, 15))
+        block = ios.Block(v.node)
+        a = ios.conv2d(block, [[v]], width, (3, 3), (1, 1), (1, 1))
+        b = ios.conv2d(block, [[v]], 24, (1, 1))
+        ios.conv2d(block, [[a], [b]], 17, (1, 1), is_exit=True)
+        graph = Graph('t', v.node, [block])
+        graph.greedy_schedule(4)
+        graphs.append(graph)
+    for step in range(14):
+        graph, batch = graphs[(step * step) % 6], 1 + step % 3
+        graph.init_weights(seed=step, scheme='he_normal_bias')
+        x = np.random.default_rng(step).standard_normal((batch, 5, 14, 15)).astype(np.float32)
+        got = rt.graph_inference(graph, batch, x, no_alloc=no_alloc)
+        session = rt.Session(graph, batch)
+        session.load_weights()
+        session.set_input(x)
+        session.run()
+        assert np.allclose(got, session.output(), rtol=1e-4, atol=1e-5)
+        session.close()
