@@ -10,10 +10,9 @@
 //   m = output channel inside the group (OCg), n = flattened (image, oh, ow) pixel,
 //   k = (kh, kw, c) tap-major with the channels of every tap zero-padded to a multiple of the K tile.
 // The filter matrix is pre-packed k-major (launch_pack_filters) so that a block's BK x BM slice is read
-// with 16-byte loads along m.  The BK x BN input slice is gathered straight from the NCHW input view:
-// consecutive lanes take consecutive pixels; because a K tile lies inside one filter tap, the tap's
-// (kh, kw), its padding test and its base offset are computed once per tile and an element costs one
-// address add (with k = (c, kh, kw) the gather spent ~17 VALU instructions per MFMA).  Global loads run PD tiles
+// with 16-byte loads along m.  The BK x BN input slice is gathered straight from the NHWC input view:
+// consecutive lanes take consecutive quads of channels of a pixel, then the next pixel; because a K tile lies inside one
+// filter tap, the tap's (kh, kw), its padding test and its base offset are computed once per tile.  Global loads run PD tiles
 // ahead of the math in registers (the loop is latency bound at batch 1, where a block sees only a few
 // K tiles), tiles are staged in LDS (double buffered, one barrier per K tile) and consumed by
 // v_mfma_f32_32x32x2_f32 / v_mfma_f32_16x16x4_f32: lane l supplies A[k = l / MT][m = l % MT] and
@@ -37,27 +36,6 @@ namespace ios {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// Division of a 32-bit unsigned by a divisor fixed at launch time (Granlund-Montgomery): exact for every dividend,
-// five instructions instead of the ~20 of a hardware-less integer division.
-struct FastDiv {
-    unsigned m, s1, s2;
-};
-
-inline FastDiv make_fast_div(unsigned d) {   // d >= 1
-    unsigned l = 0;
-    while ((1ull << l) < d) l++;   // ceil(log2(d))
-    FastDiv f;
-    f.m = (unsigned)((((1ull << l) - d) << 32) / d + 1);
-    f.s1 = l < 1 ? l : 1;
-    f.s2 = l > 0 ? l - 1 : 0;
-    return f;
-}
-
-__device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv &f) {
-    const unsigned t = __umulhi(f.m, n);
-    return (t + ((n - t) >> f.s1)) >> f.s2;
-}
-
 struct ConvKernelArgs {
     const float *x;
     const float *wp;
@@ -69,8 +47,8 @@ struct ConvKernelArgs {
     int KW;
     int xcd_local;                    // split-K inside one XCD, see below
     unsigned magic_icgp, magic_kw;    // floor(2^32 / d) + 1: exact quotients for dividends < 2^16
-    int ICg, ICgP, OCg, OCgP, Kq, HW, OHW, groups;   // Kq = taps * ICgP rows of the packed filter matrix
-    long long x_bs, y_bs;
+    int ICg, ICgP, OCg, OCgP, Kq, OHW, groups;   // Kq = taps * ICgP rows of the packed filter matrix
+    int x_ps, y_ps;                   // elements between neighbouring pixels of input and output
     unsigned x_bytes, w_bytes;        // extents of the input view and of the packed filters, both < 2^31
     int Npix;
     int act, pre_relu;
@@ -83,7 +61,7 @@ struct ConvKernelArgs {
     FastDiv div_tile;    // by tile_div
     FastDiv div_ohw, div_ow;
     // Either the residual form (stand-alone kernels only): y = res + act(conv + bias), then max(., 0) when post_relu; res is a
-    // dense view of the output's shape (batch stride res_bs elements), null for a plain convolution.
+    // view of the output's shape (res_ps elements between pixels), null for a plain convolution.
     // Or split-K inside one XCD (xcd_local != 0; plain convolutions without groups, counters set): the grid is numbered so
     // that all K slices of an output tile run on the same XCD and meet in that XCD's L2 (see XcdSlot).  xcd_map: the XCC id
     // that blocks with index % 8 == c run on, four bits per c, as measured when the device context was created; fault: a
@@ -92,7 +70,7 @@ struct ConvKernelArgs {
     union {
         struct {
             const float *res;
-            int res_bs, post_relu;
+            int res_ps, post_relu;
         };
         struct {
             unsigned *fault;
@@ -166,17 +144,6 @@ __device__ __forceinline__ int draw_ticket(unsigned *counter, int split_k) {
     return last;
 }
 
-// v = act(conv + bias) of output element (image b, channel, pixel r): adds the residual operand.  The residual form is a
-// compile-time property of a body (RES): the plain form, which every fused stage launch uses, carries no test for it.
-template <bool RES>
-__device__ __forceinline__ float add_residual(const ConvKernelArgs &a, float v, int b, int channel, int r) {
-    if constexpr (RES) {
-        v += a.res[(long long)b * a.res_bs + (long long)channel * a.OHW + r];
-        if (a.post_relu) v = fmaxf(v, 0.0f);
-    }
-    return v;
-}
-
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Tiles are renumbered so that an XCD
 // receives a contiguous range of them, and the range runs along the operand that is cheaper to duplicate: the
 // more expensive operand (filters at batch 1, activations at large batch) is then fetched into one L2 only.
@@ -190,16 +157,47 @@ __device__ __forceinline__ void xcd_tile(const ConvKernelArgs &a, int block, int
     tn = a.weights_major ? rest : q2;
 }
 
-__device__ __forceinline__ float apply_act(float v, int act) {
-    switch (act) {
-        case ACT_RELU: return fmaxf(v, 0.0f);
-        case ACT_TANH: return tanhf(v);
-        case ACT_SIGMOID: return 1.0f / (1.0f + __expf(-v));
-        default: return v;
+typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4_u __attribute__((ext_vector_type(4), aligned(4)));   // 16 bytes at any 4-byte boundary
+
+// Epilogue of four consecutive output channels m ... m + 3 of group g at pixel nn (all four accumulators of a lane that belong
+// together, see Mfma::row): bias, activation, residual operand, one 16-byte store (element by element where the group ends
+// inside).  RES, the residual form, is a compile-time property of a body: the plain form, which every fused stage launch uses,
+// carries no test for it.
+template <bool RES>
+__device__ __forceinline__ void finish_quad(const ConvKernelArgs &a, floatx4 v, floatx4 bias, int g, int m, int nn) {
+    const int channel = g * a.OCg + m;
+    float out[4] = {v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
+    apply_activation(out, a.act);
+    v = floatx4{out[0], out[1], out[2], out[3]};
+    float *y = a.y + (long long)nn * a.y_ps + channel;
+    const float *res = nullptr;
+    if constexpr (RES) res = a.res + (long long)nn * a.res_ps + channel;
+    if (m + 3 < a.OCg) {
+        if constexpr (RES) {
+            v += (floatx4)*reinterpret_cast<const floatx4_u *>(res);
+            if (a.post_relu)
+#pragma unroll
+                for (int c = 0; c < 4; c++) v[c] = fmaxf(v[c], 0.0f);
+        }
+        *reinterpret_cast<floatx4_u *>(y) = v;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (m + c < a.OCg) {
+                if constexpr (RES) {
+                    v[c] += res[c];
+                    if (a.post_relu) v[c] = fmaxf(v[c], 0.0f);
+                }
+                y[c] = v[c];
+            }
     }
 }
 
-typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
+// bias of output channels m ... m + 3 of group g (what lies behind the last bias value is not used; the arena goes on there)
+__device__ __forceinline__ floatx4 bias_quad(const ConvKernelArgs &a, int g, int m) {
+    return *reinterpret_cast<const floatx4_u *>(a.bias + g * a.OCg + min(m, a.OCg - 1));
+}
 
 // Raw buffer loads: a 32-bit byte offset against a base + extent descriptor; offsets at or beyond the extent
 // read as zero, so an invalid element (padding, channel padding, tile overhang) is a load from kOutOfRange
@@ -267,7 +265,8 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
     if (a.split_k > 1) {
         if (a.counters == nullptr) {
             // two-kernel form: store this slice's partial tile; splitk_reduce_kernel adds the slices, bias and activation
-            float *wsz = a.ws + ((size_t)z * a.groups + g) * a.OCg * (size_t)a.Npix;
+            const size_t channels = (size_t)a.groups * a.OCg;
+            float *wsz = a.ws + (size_t)z * channels * (size_t)a.Npix + (size_t)g * a.OCg;
             if (wk == 0) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
@@ -278,7 +277,7 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
 #pragma unroll
                         for (int v = 0; v < M::ACC; v++) {
                             const int m = m0 + wm * WTM + i * MT + M::row(v, lane);
-                            if (m < a.OCg) wsz[(size_t)m * a.Npix + nn] = acc[i][j][v];
+                            if (m < a.OCg) wsz[(size_t)nn * channels + m] = acc[i][j][v];
                         }
                 }
             }
@@ -339,21 +338,20 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
     // ---- epilogue -------------------------------------------------------------------------------------------
     if (wk == 0) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int nn = n0 + wn * WTN + j * MT + lc;
-            if (nn >= a.Npix) continue;
-            const int b = (int)fast_div((unsigned)nn, a.div_ohw);
-            const int r = nn - b * a.OHW;
-            float *yb = a.y + (long long)b * a.y_bs + (long long)g * a.OCg * a.OHW + r;
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+            for (int q = 0; q < M::ACC / 4; q++) {
+                const int m = m0 + wm * WTM + i * MT + M::row(4 * q, lane);
+                if (m >= a.OCg) continue;
+                const floatx4 bias = bias_quad(a, g, m);
 #pragma unroll
-                for (int v = 0; v < M::ACC; v++) {
-                    const int m = m0 + wm * WTM + i * MT + M::row(v, lane);
-                    if (m < a.OCg)
-                        yb[(long long)m * a.OHW] = add_residual<RES>(a, apply_act(acc[i][j][v] + a.bias[g * a.OCg + m], a.act), b, g * a.OCg + m, r);
+                for (int j = 0; j < TN; j++) {
+                    const int nn = n0 + wn * WTN + j * MT + lc;
+                    if (nn >= a.Npix) continue;
+                    const floatx4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    finish_quad<RES>(a, v, bias, g, m, nn);
                 }
-        }
+            }
     }
 }
 
@@ -382,11 +380,11 @@ struct ConvTiled {
     constexpr int A_VEC_PER_ROW = BM / 4;
     constexpr int A_SLOTS = BK * A_VEC_PER_ROW;
     constexpr int A_ITERS = (A_SLOTS + T - 1) / T;
-    constexpr int B_ROWS_PER_PASS = T / BN;
-    constexpr int B_ITERS = BK / B_ROWS_PER_PASS;
+    constexpr int B_QUADS = BK / 4;                      // quads of channels of a pixel in a K tile
+    constexpr int B_ITERS = B_QUADS * BN / T;            // pixels a thread stages, T / B_QUADS apart
     static_assert(WTM % MT == 0 && WTN % MT == 0, "wave tile must be a multiple of the MFMA tile");
     static_assert(KSLICE % M::KSTEP == 0, "K slice per wavefront must be a multiple of the MFMA depth");
-    static_assert(T % BN == 0 && BK % B_ROWS_PER_PASS == 0, "input loader shape");
+    static_assert(T % B_QUADS == 0 && B_QUADS * BN % T == 0 && BN % (T / B_QUADS) == 0, "input loader shape");
     float *As = smem;                  // [2][BK][LDA]
     float *Bs = smem + 2 * BK * LDA;   // [2][BK][LDB]
 
@@ -406,21 +404,22 @@ struct ConvTiled {
     const int nkt = (k_end - k_begin) / BK;   // Kq and k_chunk are multiples of BK
 
     // ---- per-thread loader state ---------------------------------------------------------------------
-    const int bn_l = tid % BN;
-    const int bk_l = tid / BN;
-    const int n = n0 + bn_l;
-    const bool n_ok = n < a.Npix;
-    int ih0 = 0, iw0 = 0;
-    unsigned x_thread = 0;   // byte offset of (image, group, ih0, iw0); may wrap below zero, the tap offset brings it back
-    {
-        const int nn = n_ok ? n : 0;
+    const int bq = tid % B_QUADS;   // this thread's quad of channels inside a K tile
+    const int bn_l = tid / B_QUADS; // its first pixel inside the output tile
+    int ih0[B_ITERS], iw0[B_ITERS];
+    unsigned n_kill[B_ITERS], b_off[B_ITERS];   // byte offset of (image, ih0, iw0, group, quad); may wrap below zero, the tap offset brings it back
+#pragma unroll
+    for (int i = 0; i < B_ITERS; i++) {
+        const int n = n0 + bn_l + i * (T / B_QUADS);
+        n_kill[i] = n < a.Npix ? 0u : kOutOfRange;
+        const int nn = n < a.Npix ? n : 0;
         const int b = (int)fast_div((unsigned)nn, a.div_ohw);
         const int r = nn - b * a.OHW;
         const int oh = (int)fast_div((unsigned)r, a.div_ow);
         const int ow = r - oh * a.OW;
-        ih0 = oh * a.sh - a.ph;
-        iw0 = ow * a.sw - a.pw;
-        x_thread = (unsigned)(((long long)b * a.x_bs + (long long)g * a.ICg * a.HW + (long long)ih0 * a.W + iw0) * 4);
+        ih0[i] = oh * a.sh - a.ph;
+        iw0[i] = ow * a.sw - a.pw;
+        b_off[i] = (((unsigned)(b * a.H + ih0[i]) * (unsigned)a.W + (unsigned)iw0[i]) * (unsigned)a.x_ps + (unsigned)(g * a.ICg + 4 * bq)) * 4u;
     }
     const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
     const __amdgpu_buffer_rsrc_t wr = buffer_of(a.wp, a.w_bytes);
@@ -434,17 +433,13 @@ struct ConvTiled {
         const bool ok = (A_SLOTS % T == 0 || slot < A_SLOTS) && m0 + c4 * 4 < a.OCgP;
         a_off[i] = ok ? (unsigned)(((size_t)g * a.Kq * a.OCgP + (size_t)row * a.OCgP + m0 + c4 * 4) * 4) : kOutOfRange;
     }
-    unsigned b_off[B_ITERS];
-#pragma unroll
-    for (int i = 0; i < B_ITERS; i++) b_off[i] = x_thread + (unsigned)((bk_l + i * B_ROWS_PER_PASS) * a.HW) * 4u;
-
     floatx4 a_reg[PD][A_ITERS];
-    float b_reg[PD][B_ITERS];
+    floatx4 b_reg[PD][B_ITERS];
 
     // K is ordered tap-major: row k of the packed filters is (tap = k / ICgP, c = k % ICgP) with ICgP a
-    // multiple of BK, so a K tile lies inside one filter tap: (kh, kw) and the tile's base offsets are scalar,
-    // the padding test is one compare pair per thread, and an element costs an add and a select of its offset.
-    auto load_tile = [&](int kt, floatx4(&ar)[A_ITERS], float(&br)[B_ITERS]) {
+    // multiple of BK, so a K tile lies inside one filter tap: (kh, kw) and the tile's base offsets are scalar and
+    // the padding test is one compare pair per pixel.
+    auto load_tile = [&](int kt, floatx4(&ar)[A_ITERS], floatx4(&br)[B_ITERS]) {
         const int k0 = k_begin + kt * BK;
         const int tap = (int)__umulhi((unsigned)k0, a.magic_icgp);
         const int c0 = k0 - tap * a.ICgP;
@@ -456,20 +451,22 @@ struct ConvTiled {
         for (int i = 0; i < A_ITERS; i++) ar[i] = buffer_load_f32x4(wr, (a_off[i] + w_tile) | tile_kill);
         // invalid elements get the top offset bit set, which is beyond every extent; plain bit arithmetic keeps
         // the loads of a tile in one basic block so that they are issued back to back
-        const unsigned in_h = (unsigned)(ih0 + kh) < (unsigned)a.H ? 1u : 0u;
-        const unsigned in_w = (unsigned)(iw0 + kw) < (unsigned)a.W ? 1u : 0u;
-        const unsigned kill = (((in_h & in_w & (n_ok ? 1u : 0u)) ^ 1u) << 31) | tile_kill;
-        const unsigned x_tile = (unsigned)(c0 * a.HW + kh * a.W + kw) * 4u;
-        const int c_last = a.ICg - c0 - 1 - bk_l;   // this thread's rows beyond c_last are channel padding
+        const unsigned x_tile = (unsigned)((kh * a.W + kw) * a.x_ps + c0) * 4u;
+        const int c_left = a.ICg - c0 - 4 * bq;   // real channels from this quad on
+        const unsigned pad = (unsigned)(c_left - 1) & kOutOfRange;   // sign bit: the quad is channel padding
 #pragma unroll
         for (int i = 0; i < B_ITERS; i++) {
-            const unsigned pad = (unsigned)(c_last - i * B_ROWS_PER_PASS) & kOutOfRange;   // sign bit
-            br[i] = buffer_load_f32(xr, (b_off[i] + x_tile) | kill | pad);
+            const unsigned in_h = (unsigned)(ih0[i] + kh) < (unsigned)a.H ? 1u : 0u;
+            const unsigned in_w = (unsigned)(iw0[i] + kw) < (unsigned)a.W ? 1u : 0u;
+            const unsigned kill = (((in_h & in_w) ^ 1u) << 31) | n_kill[i] | tile_kill | pad;
+            br[i] = buffer_load_f32x4(xr, (b_off[i] + x_tile) | kill);
+#pragma unroll
+            for (int u = 1; u < 4; u++) br[i][u] = u < c_left ? br[i][u] : 0.f;   // channels of the quad beyond the group's
         }
     };
 
     const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
-    auto store_tile = [&](int buf, const floatx4(&ar)[A_ITERS], const float(&br)[B_ITERS]) {
+    auto store_tile = [&](int buf, const floatx4(&ar)[A_ITERS], const floatx4(&br)[B_ITERS]) {
         float *Ab = As + buf * BK * LDA;
         float *Bb = Bs + buf * BK * LDB;
 #pragma unroll
@@ -484,7 +481,9 @@ struct ConvTiled {
 #pragma unroll
         for (int i = 0; i < B_ITERS; i++) {
             // folded ReLU of the producer as one integer max (negative floats are negative integers)
-            Bb[(bk_l + i * B_ROWS_PER_PASS) * LDB + bn_l] = __int_as_float(max(__float_as_int(br[i]), relu_floor));
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                Bb[(4 * bq + u) * LDB + bn_l + i * (T / B_QUADS)] = __int_as_float(max(__float_as_int(br[i][u]), relu_floor));
         }
     };
 
@@ -579,8 +578,8 @@ struct ConvTiled {
 // which is the operand layout of the instruction (lane l: row l % 32, k = 8 * (l / 32) ... + 7): a wavefront reads the filter
 // operand of a 32 x 32 tile straight from global memory, one 16-byte load per lane and plane, PD K tiles ahead (the filters
 // are small and stay in the caches; the LDS, whose bandwidth bounds this kernel, carries the inputs only).  Inputs are split
-// by the thread that stages them: eight channels of one pixel, loaded PD K tiles ahead into registers, three 16-byte LDS
-// stores into [plane][octet][pixel][8 k], again the operand layout: an input operand is one conflict-free 16-byte LDS load
+// by the thread that stages them: eight channels of one pixel, two 16-byte loads PD K tiles ahead into registers, three 16-byte
+// LDS stores into [plane][pixel][octet][8 k], again the operand layout: an input operand is one conflict-free 16-byte LDS load
 // per lane and plane.  K tiles are 16 deep and lie inside one filter tap (channels padded to 16); LDS is double buffered, one
 // barrier per K tile.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -644,7 +643,7 @@ struct ConvSplit3 {
     static constexpr int SMEM_FLOATS = 2 * STAGE * 4;
     static constexpr int B_OCT = 2 * BN;
     static constexpr int B_IT = (B_OCT + T - 1) / T;                   // octets a thread stages per K tile
-    static_assert(T % BN == 0, "a thread stages the same pixel in every pass");
+    static_assert(B_OCT % T == 0 || B_IT == 1, "whole passes, or one with surplus threads");
 
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
@@ -678,30 +677,34 @@ struct ConvSplit3 {
         a_off[i] = m < a.OCgP ? (unsigned)(((((size_t)g * (a.Kq >> 3) + lk) * TERMS) * a.OCgP + m) * 16) : kOutOfRange;
     }
     const unsigned a_plane = (unsigned)a.OCgP * 16u;
-    // ---- inputs: this thread's pixel and octets ----------------------------------------------------------------------------
-    const int pix = tid % BN;
-    const int n = n0 + pix;
-    const bool n_ok = n < a.Npix;
-    int ih0, iw0;
-    unsigned x_thread;
-    {
-        const int nn = n_ok ? n : 0;
+    // ---- inputs: this thread's pixels and its octet of channels ----------------------------------------------------------
+    // Two neighbouring threads take the two octets of a pixel: 64 contiguous bytes of the input.
+    const int oct = tid & 1;
+    int ih0[B_IT], iw0[B_IT];
+    unsigned x_off[B_IT], n_kill[B_IT];
+#pragma unroll
+    for (int i = 0; i < B_IT; i++) {
+        const int n = n0 + ((tid + i * T) >> 1);
+        // (more threads than octets: the surplus stages nothing)
+        const bool ok = n < a.Npix && (B_OCT % T == 0 || tid < B_OCT);
+        n_kill[i] = ok ? 0u : kOutOfRange;
+        const int nn = ok ? n : 0;
         const int b = (int)fast_div((unsigned)nn, a.div_ohw);
         const int r = nn - b * a.OHW;
         const int oh = (int)fast_div((unsigned)r, a.div_ow);
         const int ow = r - oh * a.OW;
-        ih0 = oh * a.sh - a.ph;
-        iw0 = ow * a.sw - a.pw;
-        x_thread = (unsigned)(((long long)b * a.x_bs + (long long)g * a.ICg * a.HW + (long long)ih0 * a.W + iw0) * 4);
+        ih0[i] = oh * a.sh - a.ph;
+        iw0[i] = ow * a.sw - a.pw;
+        x_off[i] = (((unsigned)(b * a.H + ih0[i]) * (unsigned)a.W + (unsigned)iw0[i]) * (unsigned)a.x_ps + (unsigned)(g * a.ICg + 8 * oct)) * 4u;
     }
-    int b_oct[B_IT];       // which half of the K tile (channels 8 * b_oct ... + 7 of the tile) a pass of this thread stages
-#pragma unroll
-    for (int i = 0; i < B_IT; i++) b_oct[i] = (tid + i * T) / BN;
-    const unsigned b_surplus = B_OCT % T == 0 || tid < B_OCT ? 0u : kOutOfRange;   // (more threads than octets: the surplus stages nothing)
+    // LDS slot of (pixel, octet) inside a plane: the two octets of a pixel side by side, exchanged in every other group of four
+    // pixels, so that eight consecutive pixels of one octet (an operand read) and four pixels of both (a store) use all banks
+    auto slot_of = [](int pixel, int octet) { return 2 * pixel + (octet ^ ((pixel >> 2) & 1)); };
 
     uintx4 a_reg[PD][TERMS][TM];
-    float b_reg[PD][B_IT][8];
-    auto load_tile = [&](int kt, uintx4 (&ar)[TERMS][TM], float (&br)[B_IT][8]) {
+    floatx4 b_reg[PD][B_IT][2];
+    int b_left[PD];   // real channels of this thread's octet in the stage's K tile
+    auto load_tile = [&](int kt, uintx4 (&ar)[TERMS][TM], floatx4 (&br)[B_IT][2], int &left) {
         const int k0 = k_begin + kt * BK;
         const int tap = (int)__umulhi((unsigned)k0, a.magic_icgp);
         const int c0 = k0 - tap * a.ICgP;
@@ -713,37 +716,42 @@ struct ConvSplit3 {
         for (int p = 0; p < TERMS; p++)
 #pragma unroll
             for (int i = 0; i < TM; i++) ar[p][i] = __builtin_amdgcn_raw_buffer_load_b128(wr, (a_off[i] + w_tile) | tile_kill, (unsigned)p * a_plane, 0);
-        const unsigned in_h = (unsigned)(ih0 + kh) < (unsigned)a.H ? 1u : 0u;
-        const unsigned in_w = (unsigned)(iw0 + kw) < (unsigned)a.W ? 1u : 0u;
-        const unsigned kill = (((in_h & in_w & (n_ok ? 1u : 0u)) ^ 1u) << 31) | tile_kill | b_surplus;
-        const unsigned x_tile = x_thread + (unsigned)(c0 * a.HW + kh * a.W + kw) * 4u;
-        const unsigned plane = (unsigned)a.HW * 4u;
+        const unsigned x_tile = (unsigned)((kh * a.W + kw) * a.x_ps + c0) * 4u;
+        const int c_left = a.ICg - c0 - 8 * oct;   // real channels from this octet on
+        const unsigned pad0 = (unsigned)(c_left - 1) & kOutOfRange, pad1 = (unsigned)(c_left - 5) & kOutOfRange;   // sign bits
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
-            const int c_left = a.ICg - 1 - c0 - b_oct[i] * 8;   // channels of this octet beyond c_left are padding
-            const unsigned at = (x_tile + (unsigned)(b_oct[i] * 8) * plane) | kill;
+            const unsigned in_h = (unsigned)(ih0[i] + kh) < (unsigned)a.H ? 1u : 0u;
+            const unsigned in_w = (unsigned)(iw0[i] + kw) < (unsigned)a.W ? 1u : 0u;
+            const unsigned at = (x_off[i] + x_tile) | (((in_h & in_w) ^ 1u) << 31) | n_kill[i] | tile_kill;
             // (no branch around loads inside the loop: where paths that issued loads join, the compiler waits for all of them)
-#pragma unroll
-            for (int j = 0; j < 8; j++) br[i][j] = buffer_load_f32(xr, at | ((unsigned)(c_left - j) & kOutOfRange), (unsigned)j * plane);
+            br[i][0] = buffer_load_f32x4(xr, at | pad0);
+            br[i][1] = buffer_load_f32x4(xr, at | pad1, 16u);
         }
+        left = c_left;
     };
     const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
-    auto store_inputs = [&](int buf, const float (&br)[B_IT][8]) {
+    const bool ragged = (a.ICg & 3) != 0;   // a quad of channels may straddle the end of the group's
+    auto store_inputs = [&](int buf, const floatx4 (&br)[B_IT][2], int left) {
         uintx4 *stage = lds + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
             if (B_OCT % T != 0 && tid + i * T >= B_OCT) continue;
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(br[i][j]), relu_floor));   // folded ReLU of the producer
+            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(br[i][j >> 2][j & 3]), relu_floor));   // folded ReLU of the producer
+            if (ragged)
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = j < left ? v[j] : 0.f;
+            const int slot = slot_of((tid + i * T) >> 1, oct);
             if constexpr (TERMS == 3) {
                 uintx4 hi, mid, lo;
                 split_bf16x3(v, hi, mid, lo);
-                stage[(0 + b_oct[i]) * BN + pix] = hi;
-                stage[(2 + b_oct[i]) * BN + pix] = mid;
-                stage[(4 + b_oct[i]) * BN + pix] = lo;
+                stage[slot] = hi;
+                stage[2 * BN + slot] = mid;
+                stage[4 * BN + slot] = lo;
             } else {
-                stage[b_oct[i] * BN + pix] = round_bf16x8(v);
+                stage[slot] = round_bf16x8(v);
             }
         }
     };
@@ -761,22 +769,22 @@ struct ConvSplit3 {
     // kt: the matrix work of tile kt from registers (filters) and LDS stage kt & 1 (inputs), the stage's registers requested
     // again for tile kt + PD, the inputs of tile kt + 1 split and stored into the other LDS stage, one barrier.
 #pragma unroll
-    for (int s = 0; s < PD; s++) load_tile(s, a_reg[s], b_reg[s]);
-    store_inputs(0, b_reg[0]);
+    for (int s = 0; s < PD; s++) load_tile(s, a_reg[s], b_reg[s], b_left[s]);
+    store_inputs(0, b_reg[0], b_left[0]);
     __syncthreads();
     for (int kt0 = 0; kt0 < nkt; kt0 += PD) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
             const int kt = kt0 + s;
             const int buf = kt & 1;
-            const uintx4 *Bb = lds + buf * STAGE + lk * BN + wn * WTN + lc;
+            const uintx4 *Bb = lds + buf * STAGE + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
             bf16x8 av[TERMS][TM], bv[TERMS][TN];
 #pragma unroll
             for (int p = 0; p < TERMS; p++) {
 #pragma unroll
                 for (int i = 0; i < TM; i++) av[p][i] = __builtin_bit_cast(bf16x8, a_reg[s][p][i]);
 #pragma unroll
-                for (int j = 0; j < TN; j++) bv[p][j] = __builtin_bit_cast(bf16x8, Bb[p * 2 * BN + j * MT]);
+                for (int j = 0; j < TN; j++) bv[p][j] = __builtin_bit_cast(bf16x8, Bb[p * 2 * BN + j * 2 * MT]);
             }
             // all LDS reads of the tile are requested before its first matrix instruction (left to itself the scheduler
             // requests each operand right in front of its first use and the wavefront pays the LDS latency once per plane)
@@ -790,8 +798,8 @@ struct ConvSplit3 {
                 for (int i = 0; i < TM; i++)
 #pragma unroll
                     for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[TA[t]][i], bv[TB[t]][j], acc[i][j], 0, 0, 0);
-            store_inputs(buf ^ 1, b_reg[(s + 1) % PD]);
-            load_tile(kt + PD, a_reg[s], b_reg[s]);
+            store_inputs(buf ^ 1, b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+            load_tile(kt + PD, a_reg[s], b_reg[s], b_left[s]);
             __syncthreads();
         }
     }
@@ -799,32 +807,32 @@ struct ConvSplit3 {
     }   // run
 };
 
-// y[b][oc][r] = act(bias[oc] + sum_s ws[s][oc][n]) (+ residual),  n = b * OHW + r; slices are added in index order
+// y[n][oc] = act(bias[oc] + sum_s ws[s][n][oc]) (+ residual); slices are added in index order
 struct ReduceArgs {
     const float *ws;
     const float *bias;
     float *y;
-    int slices, OC, Npix, OHW, act;
-    long long slice_floats, y_bs;
+    int slices, OC, Npix, y_ps, act;
+    long long slice_floats;
     const float *res;      // residual operand as in ConvKernelArgs, or null
-    int res_bs, post_relu;
+    int res_ps, post_relu;
 };
 
 __device__ __forceinline__ void splitk_reduce_body(const ReduceArgs &a, int block, int num_blocks, unsigned threads) {
     const long long total = (long long)a.OC * a.Npix;
     for (long long i = block * (long long)threads + threadIdx.x; i < total; i += (long long)num_blocks * threads) {
-        const int oc = (int)(i / a.Npix);
-        const int n = (int)(i - (long long)oc * a.Npix);
+        const int n = (int)(i / a.OC);
+        const int oc = (int)(i - (long long)n * a.OC);
         float sum = 0.f;
         for (int s = 0; s < a.slices; s++) sum += a.ws[s * a.slice_floats + i];
-        const int b = n / a.OHW;
-        const int r = n - b * a.OHW;
-        float v = apply_act(sum + a.bias[oc], a.act);
+        float out[1] = {sum + a.bias[oc]};
+        apply_activation(out, a.act);
+        float v = out[0];
         if (a.res != nullptr) {
-            v += a.res[(long long)b * a.res_bs + (long long)oc * a.OHW + r];
+            v += a.res[(long long)n * a.res_ps + oc];
             if (a.post_relu) v = fmaxf(v, 0.0f);
         }
-        a.y[b * a.y_bs + (long long)oc * a.OHW + r] = v;
+        a.y[(long long)n * a.y_ps + oc] = v;
     }
 }
 
@@ -897,7 +905,7 @@ struct ConvWsplit {
     const int s_end = min(s_hi, s_begin + a.steps_per_wave);
 
     int ih0[TN], iw0[TN];
-    unsigned x_lane[TN];   // byte offset of (image, group channel lk, ih0, iw0); wraps like x_thread above
+    unsigned x_lane[TN];   // byte offset of (image, ih0, iw0, first channel of the lane); may wrap below zero, the tap offset brings it back
     bool n_ok[TN];
 #pragma unroll
     for (int j = 0; j < TN; j++) {
@@ -913,8 +921,8 @@ struct ConvWsplit {
         ih0[j] = __mul24(oh, a.sh) - a.ph;
         iw0[j] = __mul24(ow, a.sw) - a.pw;
         const int lane_channel = QUAD ? U * lk : lk;   // first channel of this lane inside a step / batch
-        x_lane[j] = ((unsigned)b * (unsigned)a.x_bs + (unsigned)(g * a.ICg + lane_channel) * (unsigned)a.HW +
-                     (unsigned)(__mul24(ih0[j], a.W) + iw0[j])) * 4u;
+        x_lane[j] = ((unsigned)(__mul24(b, a.H) + ih0[j]) * (unsigned)a.W + (unsigned)iw0[j]) * (unsigned)(a.x_ps * 4) +
+                    (unsigned)(g * a.ICg + lane_channel) * 4u;
     }
     const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
     const __amdgpu_buffer_rsrc_t wr = buffer_of(a.wp, a.w_bytes);
@@ -934,14 +942,13 @@ struct ConvWsplit {
     for (int j = 0; j < TN; j++) n_kill[j] = n_ok[j] ? 0u : kOutOfRange;
 
     // the bias of the outputs this lane finishes in the epilogue, requested now so that its latency hides behind the K loop
-    constexpr int EPW = (E + NW - 1) / NW;
-    float bias_pre[EPW];
+    // (a wavefront finishes whole quads of consecutive output channels)
+    constexpr int G = E / 4;
+    constexpr int GPW = (G + NW - 1) / NW;
+    auto quad_row = [&](int e4) { return m0 + (4 * e4 / (M::ACC * TN)) * MT + M::row((4 * e4) % M::ACC, lane); };
+    floatx4 bias_pre[GPW];
 #pragma unroll
-    for (int t = 0; t < EPW; t++) {
-        const int e = min(wave + t * NW, E - 1);
-        const int m = m0 + (e / (M::ACC * TN)) * MT + M::row(e % M::ACC, lane);
-        bias_pre[t] = a.bias[g * a.OCg + min(m, a.OCg - 1)];
-    }
+    for (int t = 0; t < GPW; t++) bias_pre[t] = bias_quad(a, g, quad_row(min(wave + t * NW, G - 1)));
     typename M::acc_t acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -963,6 +970,7 @@ struct ConvWsplit {
     using FilterStage = std::conditional_t<(RP >= 3), FilterStageX3, std::conditional_t<(RP != 0), FilterStageBf16, FilterStageF32>>;
     FilterStage av[D];
     float bv[D][U][TN];
+    int left[D];
 
     // k-step s covers rows k = s * KSTEP + lk of the tap-major packed filters; ICgP is a multiple of KSTEP, so a
     // step lies inside one filter tap and (tap, kh, kw, first channel) are wavefront-uniform
@@ -982,10 +990,9 @@ struct ConvWsplit {
     // descriptors of extent zero, and return zeros without touching memory.  Loads are never skipped by a branch inside
     // the K loop: where a path with and a path without newly issued loads join, the compiler can only wait for *all*
     // outstanding loads before the next use of an older one, which serialises load latency and matrix work.
-    // `ragged` (a std::bool_constant, QUAD only): the group's channel count is not a multiple of U, so the U channels of a lane
-    // can straddle the end of the real channels and every k-step needs its own test; otherwise a lane's channels are real or
-    // padding together and one test per batch, folded into the lane's offsets, covers them.
-    auto load_batch = [&](int s0, FilterStage &A, float(&B)[U][TN], bool live, auto ragged) {
+    // `left` (QUAD): the last real channel among those the lane has loaded, counted from its first one; where the group's channel
+    // count is no multiple of four, the quad that straddles its end holds a neighbour's channels and is masked before use.
+    auto load_batch = [&](int s0, FilterStage &A, float(&B)[U][TN], int &left, bool live) {
         if constexpr (QUAD) {
             // The whole batch lies inside one tap (channels are padded to the batch).  Batches are requested in K
             // order, so (first channel, kh, kw) and the filter offset advance incrementally on the SALU.  Lane-constant
@@ -1017,32 +1024,23 @@ struct ConvWsplit {
                         A.v[q * 4 + 3][i] = w4.w;
                     }
             }
-            const unsigned x_tap = (unsigned)(q_kh * a.W + q_kw) * 4u;
-            const unsigned x_chan = (unsigned)(q_cb * a.HW) * 4u;
-            unsigned voff[TN];
+            const unsigned x_tap = (unsigned)((q_kh * a.W + q_kw) * a.x_ps) * 4u;
+            const unsigned x_chan = (unsigned)q_cb * 4u;
+            const int c_left = c_lane_last - q_cb;   // the lane's channels beyond c_left are padding (the tap's last batch)
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const unsigned in_h = (unsigned)(ih0[j] + q_kh) < (unsigned)a.H ? 1u : 0u;
                 const unsigned in_w = (unsigned)(iw0[j] + q_kw) < (unsigned)a.W ? 1u : 0u;
-                voff[j] = (x_lane[j] + x_tap) | (((in_h & in_w) ^ 1u) << 31);
-            }
-            const int c_left = c_lane_last - q_cb;   // channels of this lane beyond c_left are padding (the tap's last batch)
-            if constexpr (decltype(ragged)::value) {
+                const unsigned voff = (x_lane[j] + x_tap) | (((in_h & in_w) ^ 1u) << 31);
 #pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const unsigned c_kill = (unsigned)(c_left - u) & kOutOfRange;   // sign bit
+                for (int q = 0; q < U / 4; q++) {
+                    const unsigned c_kill = (unsigned)(c_left - 4 * q) & kOutOfRange;   // sign bit: the whole quad is padding
+                    const floatx4 x4 = buffer_load_f32x4(xr, voff | c_kill, x_chan + (unsigned)(16 * q));
 #pragma unroll
-                    for (int j = 0; j < TN; j++) B[u][j] = buffer_load_f32(xr, voff[j] | c_kill, x_chan + (unsigned)(u * a.HW) * 4u);
+                    for (int u = 0; u < 4; u++) B[4 * q + u][j] = x4[u];
                 }
-            } else {
-                const unsigned c_kill = (unsigned)c_left & kOutOfRange;   // all U channels of the lane at once
-#pragma unroll
-                for (int j = 0; j < TN; j++) voff[j] |= c_kill;
-#pragma unroll
-                for (int u = 0; u < U; u++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++) B[u][j] = buffer_load_f32(xr, voff[j], x_chan + (unsigned)(u * a.HW) * 4u);
             }
+            left = c_left;
             // next batch (selects, not branches: the loop body stays one basic block)
             q_w += RP >= 3 ? (unsigned)((U * M::KSTEP / 8) * PLANES * a.OCgP) * 16u : (unsigned)((U * M::KSTEP / 4) * a.OCgP) * (RP != 0 ? 8u : 16u);
             q_cb += U * M::KSTEP;
@@ -1055,6 +1053,7 @@ struct ConvWsplit {
             return;
         }
         (void)live;   // steps at or beyond s_end are dead by their index
+        (void)left;
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const bool s_ok = (s0 + u) < s_end;
@@ -1067,7 +1066,7 @@ struct ConvWsplit {
             const unsigned step_kill = s_ok ? 0u : kOutOfRange;   // wavefront-uniform
 #pragma unroll
             for (int i = 0; i < TM; i++) A.v[u][i] = buffer_load_f32(wr, (w_lane[i] + w_step) | w_kill[i] | step_kill);
-            const unsigned x_step = (unsigned)(cb * a.HW + kh * a.W + kw) * 4u;
+            const unsigned x_step = (unsigned)((kh * a.W + kw) * a.x_ps + cb) * 4u;
             const unsigned c_kill = (unsigned)(a.ICg - 1 - cb - lk) & kOutOfRange;   // sign bit: channel padding
 #pragma unroll
             for (int j = 0; j < TN; j++) {
@@ -1080,7 +1079,14 @@ struct ConvWsplit {
     };
     // folded ReLU of the producer: as integers, negative floats are below 0 and everything is above INT_MIN
     const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
-    auto compute = [&](const FilterStage &A, const float(&B)[U][TN]) {
+    const bool ragged = QUAD && (a.ICg & 3) != 0;   // (a branch around register work only, see load_batch)
+    auto compute = [&](const FilterStage &A, float(&B)[U][TN], int left) {
+        if (ragged) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) B[u][j] = u <= left ? B[u][j] : 0.f;
+        }
         if constexpr (RP == 3) {
             bf16x8 bq[3][TN];
 #pragma unroll
@@ -1149,87 +1155,88 @@ struct ConvWsplit {
     };
 
     const int batches = (s_end - s_begin + U - 1) / U;   // <= 0 for wavefronts beyond the end of K
-    auto k_loop = [&](auto ragged) {
+    auto k_loop = [&]() {
         if (batches <= 0) return;
-        if constexpr (decltype(ragged)::value) {
-            // channel counts that are no multiple of U (a few tiny layers): one batch at a time
-            for (int b = 0; b < batches; b++) {
-                load_batch(s_begin + b * U, av[0], bv[0], true, ragged);
-                compute(av[0], bv[0]);
-            }
-        } else if constexpr (D == 2) {
+        if constexpr (D == 2) {
             // Two stages, peeled so that every load sits in straight-line code: the steady state requests batch b + 1,
             // consumes batch b, requests b + 2, consumes b + 1 with both requests known to be in range; the last one or two
             // batches are consumed behind the loop.  The waits in front of the matrix instructions then count exactly the
             // loads issued since, and the next batch's latency overlaps this batch's matrix work.  (The scheduling fences
             // keep a stage's requests behind the matrix work that still reads the stage: moved ahead of it they need a
             // second set of registers.)
-            load_batch(s_begin, av[0], bv[0], true, ragged);
+            load_batch(s_begin, av[0], bv[0], left[0], true);
             int b = 0;
             for (; b + 2 < batches; b += 2) {
-                load_batch(s_begin + (b + 1) * U, av[1], bv[1], true, ragged);
+                load_batch(s_begin + (b + 1) * U, av[1], bv[1], left[1], true);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(av[0], bv[0]);
+                compute(av[0], bv[0], left[0]);
                 __builtin_amdgcn_sched_barrier(0);
-                load_batch(s_begin + (b + 2) * U, av[0], bv[0], true, ragged);
+                load_batch(s_begin + (b + 2) * U, av[0], bv[0], left[0], true);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(av[1], bv[1]);
+                compute(av[1], bv[1], left[1]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (b + 1 < batches) {
-                load_batch(s_begin + (b + 1) * U, av[1], bv[1], true, ragged);
+                load_batch(s_begin + (b + 1) * U, av[1], bv[1], left[1], true);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(av[0], bv[0]);
-                compute(av[1], bv[1]);
+                compute(av[0], bv[0], left[0]);
+                compute(av[1], bv[1], left[1]);
             } else {
-                compute(av[0], bv[0]);
+                compute(av[0], bv[0], left[0]);
             }
         } else {
             // deeper pipeline: D batches requested before the first one is consumed.  The loop body is straight-line
             // (requests beyond the range are issued dead, see load_batch: at most D - 1 of them in the last round that
             // requests anything); the last D batches are consumed behind the loop, where nothing is requested any more.
 #pragma unroll
-            for (int st = 0; st < D; st++) load_batch(s_begin + st * U, av[st], bv[st], st < batches, ragged);
+            for (int st = 0; st < D; st++) load_batch(s_begin + st * U, av[st], bv[st], left[st], st < batches);
             int b = 0;
             for (; b + D < batches; b += D) {
 #pragma unroll
                 for (int st = 0; st < D; st++) {
-                    compute(av[st], bv[st]);
+                    compute(av[st], bv[st], left[st]);
                     __builtin_amdgcn_sched_barrier(0);
-                    load_batch(s_begin + (b + st + D) * U, av[st], bv[st], b + st + D < batches, ragged);
+                    load_batch(s_begin + (b + st + D) * U, av[st], bv[st], left[st], b + st + D < batches);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
 #pragma unroll
             for (int st = 0; st < D; st++)
-                if (b + st < batches) compute(av[st], bv[st]);
+                if (b + st < batches) compute(av[st], bv[st], left[st]);
         }
     };
-    if constexpr (QUAD) {
-        if ((a.ICg & (U - 1)) == 0) k_loop(std::false_type{});
-        else k_loop(std::true_type{});
-    } else {
-        k_loop(std::false_type{});
-    }
+    k_loop();
 
-    // partial tiles meet in LDS: element e of lane l of wavefront w lives at red[(w * E + e) * 64 + l]
+    // partial tiles meet in LDS: quad e4 (accumulator elements 4 * e4 ... + 3) of lane l of wavefront w lives in
+    // red4[(w * G + e4) * 64 + l]
+    floatx4 *red4 = reinterpret_cast<floatx4 *>(red);
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int v = 0; v < M::ACC; v++) red[(wave * E + (i * TN + j) * M::ACC + v) * 64 + lane] = acc[i][j][v];
+            for (int q = 0; q < M::ACC / 4; q++) {
+                const floatx4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                red4[(wave * G + (i * TN + j) * (M::ACC / 4) + q) * 64 + lane] = v;
+            }
     __syncthreads();
-    if (a.split_k > 1 && a.counters == nullptr) {
-        // two-kernel split-K: this slice's partial outputs as [slice][group][m][pixel] for splitk_reduce_kernel
-        float *wsz = a.ws + ((size_t)z * a.groups + g) * a.OCg * (size_t)a.Npix;
-        for (int e = wave; e < E; e += NW) {
-            float sum = 0.f;
+    auto meet = [&](int e4) {   // wavefronts in ascending order
+        floatx4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int w = 0; w < NW; w++) sum += red[(w * E + e) * 64 + lane];
-            const int m = m0 + (e / (M::ACC * TN)) * MT + M::row(e % M::ACC, lane);
-            const int nn = n0 + ((e / M::ACC) % TN) * MT + lc;
-            if (m < a.OCg && nn < a.Npix) wsz[(size_t)m * a.Npix + nn] = sum;
+        for (int w = 0; w < NW; w++) sum += red4[(w * G + e4) * 64 + lane];
+        return sum;
+    };
+    auto quad_pixel = [&](int e4) { return n0 + ((4 * e4 / M::ACC) % TN) * MT + lc; };
+    if (a.split_k > 1 && a.counters == nullptr) {
+        // two-kernel split-K: this slice's partial outputs as [slice][pixel][channel] for splitk_reduce_kernel
+        const size_t channels = (size_t)a.groups * a.OCg;
+        float *wsz = a.ws + (size_t)z * channels * (size_t)a.Npix + (size_t)g * a.OCg;
+        for (int e4 = wave; e4 < G; e4 += NW) {
+            const floatx4 sum = meet(e4);
+            const int m = quad_row(e4), nn = quad_pixel(e4);
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                if (m + c < a.OCg && nn < a.Npix) wsz[(size_t)nn * channels + m + c] = sum[c];
         }
         return;
     }
@@ -1244,11 +1251,10 @@ struct ConvWsplit {
         auto hand_in = [&](auto local) {
             constexpr bool LOCAL = decltype(local)::value;
             float *mine = slices + (size_t)z * (BM * BN) + lane;
-            for (int e = wave; e < E; e += NW) {
-                float sum = 0.f;
+            for (int e4 = wave; e4 < G; e4 += NW) {
+                const floatx4 sum = meet(e4);
 #pragma unroll
-                for (int w = 0; w < NW; w++) sum += red[(w * E + e) * 64 + lane];
-                partial_store<LOCAL>(mine + e * 64, sum);
+                for (int c = 0; c < 4; c++) partial_store<LOCAL>(mine + (4 * e4 + c) * 64, sum[c]);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
@@ -1261,31 +1267,23 @@ struct ConvWsplit {
     }
     const bool xcd_local = a.xcd_local != 0;
 #pragma unroll
-    for (int t = 0; t < EPW; t++) {
-        const int e = wave + t * NW;
-        if (e >= E) break;
-        float sum = 0.f;
+    for (int t = 0; t < GPW; t++) {
+        const int e4 = wave + t * NW;
+        if (e4 >= G) break;
+        floatx4 sum = {0.f, 0.f, 0.f, 0.f};
         if (a.split_k > 1) {
-            const float *theirs = slices + e * 64 + lane;
-            if (xcd_local)
-                for (int s2 = 0; s2 < a.split_k; s2++) sum += partial_load<true>(theirs + (size_t)s2 * (BM * BN));
-            else
-                for (int s2 = 0; s2 < a.split_k; s2++) sum += partial_load<false>(theirs + (size_t)s2 * (BM * BN));
-        } else {
+            const float *theirs = slices + 4 * e4 * 64 + lane;
+            for (int s2 = 0; s2 < a.split_k; s2++)
 #pragma unroll
-            for (int w = 0; w < NW; w++) sum += red[(w * E + e) * 64 + lane];
+                for (int c = 0; c < 4; c++) {
+                    const float *p = theirs + (size_t)s2 * (BM * BN) + c * 64;
+                    sum[c] += xcd_local ? partial_load<true>(p) : partial_load<false>(p);
+                }
+        } else {
+            sum = meet(e4);
         }
-        const int v = e % M::ACC;
-        const int j = (e / M::ACC) % TN;
-        const int i = e / (M::ACC * TN);
-        const int m = m0 + i * MT + M::row(v, lane);
-        const int nn = n0 + j * MT + lc;
-        if (m < a.OCg && nn < a.Npix) {
-            const int b = (int)fast_div((unsigned)nn, a.div_ohw);
-            const int r = nn - b * a.OHW;
-            a.y[(long long)b * a.y_bs + ((long long)g * a.OCg + m) * a.OHW + r] =
-                add_residual<RES>(a, apply_act(sum + bias_pre[t], a.act), b, g * a.OCg + m, r);
-        }
+        const int m = quad_row(e4), nn = quad_pixel(e4);
+        if (m < a.OCg && nn < a.Npix) finish_quad<RES>(a, sum, bias_pre[t], g, m, nn);
     }
 }   // run
 };

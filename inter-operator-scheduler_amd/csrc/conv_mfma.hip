@@ -195,7 +195,7 @@ ConvLaunch conv_pick_launch(const ConvProblem &p, int num_cus, bool fusable_only
 
 bool conv_matrix_path_supported(const ConvProblem &p) {
     // packed filter rows are indexed with 16 bits, input and filter byte offsets with 31 bits
-    const unsigned long long x_bytes = (unsigned long long)p.B * p.IC * p.H * p.W * 4ull;
+    const unsigned long long x_bytes = (unsigned long long)p.B * ((p.IC + 3) & ~3) * p.H * p.W * 4ull;
     const unsigned long long w_bytes = (unsigned long long)p.groups * p.Kq(128) * p.OCgP() * 4ull;
     // image sides below 2^15 and output planes below 2^23 elements keep the kernels' signed 24-bit index multiplies exact
     return p.Kq(128) < 65536 && p.Npix() < (1LL << 31) && x_bytes < (1ull << 30) && w_bytes < (1ull << 31) && p.H < 32768 && p.W < 32768 &&
@@ -225,9 +225,9 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     a.ICg = p.ICg(); a.ICgP = p.ICgP(e.v.cpad); a.OCg = p.OCg(); a.OCgP = p.OCgP(); a.Kq = p.Kq(e.v.cpad);
     a.magic_icgp = (unsigned)((1ULL << 32) / (unsigned)a.ICgP + 1);   // ICgP >= 8
     a.magic_kw = (unsigned)((1ULL << 32) / (unsigned)a.KW + 1);       // unused when KW == 1
-    a.HW = p.H * p.W; a.OHW = p.OH * p.OW; a.groups = p.groups;
-    a.x_bs = x.bstride; a.y_bs = y.bstride;
-    const unsigned long long x_bytes = ((unsigned long long)(p.B - 1) * x.bstride + (unsigned long long)p.IC * p.H * p.W) * 4ull;
+    a.OHW = p.OH * p.OW; a.groups = p.groups;
+    a.x_ps = x.pstride; a.y_ps = y.pstride;
+    const unsigned long long x_bytes = conv_input_extent(p, x.pstride);
     const unsigned long long w_bytes = (unsigned long long)p.groups * p.Kq(e.v.cpad) * p.OCgP() * (e.v.koct ? 2ull * e.v.koct : e.v.precision != PREC_FP32 ? 2ull : 4ull);
     if (x_bytes >= (1ull << 31) || w_bytes >= (1ull << 31)) throw std::runtime_error("conv: tensor too large for 31-bit buffer offsets");
     a.x_bytes = (unsigned)x_bytes;
@@ -254,14 +254,12 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     a.div_ohw = make_fast_div((unsigned)a.OHW);
     a.div_ow = make_fast_div((unsigned)a.OW);
     a.res = nullptr;
-    a.res_bs = 0;
+    a.res_ps = 0;
     a.post_relu = post_relu ? 1 : 0;
     if (residual != nullptr) {
         if (residual->C != p.OC || residual->H != p.OH || residual->W != p.OW) throw std::runtime_error("conv: residual view does not match the output");
-        if ((unsigned long long)(p.B - 1) * residual->bstride + (unsigned long long)p.OC * p.OH * p.OW >= (1ull << 31))
-            throw std::runtime_error("conv: residual view too large");
         a.res = residual->ptr;
-        a.res_bs = (int)residual->bstride;
+        a.res_ps = residual->pstride;
     } else if (post_relu) {
         throw std::runtime_error("conv: activation after a residual that is not there");
     }
@@ -296,12 +294,11 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
         r.slices = a.split_k;
         r.OC = p.OC;
         r.Npix = a.Npix;
-        r.OHW = a.OHW;
         r.act = p.act;
         r.slice_floats = (long long)p.OC * a.Npix;
-        r.y_bs = y.bstride;
+        r.y_ps = y.pstride;
         r.res = a.res;
-        r.res_bs = a.res_bs;
+        r.res_ps = a.res_ps;
         r.post_relu = a.post_relu;
         d.reduce_blocks = (int)std::min<long long>((r.slice_floats + 255) / 256, 4096);
     }
@@ -333,8 +330,8 @@ __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int 
                                     int precision, int planes) {
     // packed[g][k][m] = w[g * OCg + m][c][tap] with k = tap * ICgP + c;  rows with c >= ICg and columns with m >= OCg are zero.
     // kvec = 4: packed[g][k / 4][m][k % 4] instead (ICgP is a multiple of 4)
-    // kvec = 8: planes of bfloat16, packed[g][k / 8][plane][m][k % 8]: three planes with the exact three-term split of every filter
-    // value, or one plane with the value rounded to nearest even (the reduced-precision mode)
+    // kvec = 8: planes of 16-bit values, packed[g][k / 8][plane][m][k % 8]: three planes with the exact three-term split of every
+    // filter value, or one plane with the value rounded to nearest even (the reduced-precision modes)
     const size_t total = (size_t)groups * taps * ICgP * OCgP;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         int m;

@@ -133,7 +133,7 @@ __device__ __forceinline__ int fused_item_index(const WorkItem *items, int bid, 
 // -amdgpu-kernarg-preload-count the command processor hands them to a wavefront in registers, so a block knows its item
 // without a load and its first load is the item itself.
 template <int T>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(6))) void fused_kernel(const WorkItem *__restrict__ items, int num_items, int b1, int b2,
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4))) void fused_kernel(const WorkItem *__restrict__ items, int num_items, int b1, int b2,
                                                                                             int b3, int b4, int b5, int b6, int b7) {
     extern __shared__ floatx4 fused_smem[];
     float *smem = reinterpret_cast<float *>(fused_smem);
@@ -173,7 +173,7 @@ __device__ __forceinline__ void fused_inline_block(int b1, int b2, int b3, int b
 }
 
 template <int T>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(6))) void fused_kernel_inline(int num_items, int b1, int b2, int b3, int b4, int b5, int b6,
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4))) void fused_kernel_inline(int num_items, int b1, int b2, int b3, int b4, int b5, int b6,
                                                                                                    int b7, const InlineItems inl) {
     fused_inline_block<T, true>(b1, b2, b3, b4, b5, b6, b7);
 }

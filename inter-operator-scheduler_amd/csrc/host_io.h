@@ -12,35 +12,39 @@
 #include <functional>
 #include <vector>
 
+#include "plan.h"
+
 namespace ios {
 
-// Shares out copies of host memory over several threads.  They are started on the first large copy, sleep between copies
-// (on a futex: waking seven threads through a mutex took longer than their share of an 8 MB copy), and stay with the process
-// (the pool is never destroyed: a sleeping thread must not touch it while the process unloads).
+// Shares out copies of host memory over several threads.  They are started on the first large copy, sleep between copies (on
+// futexes) and stay with the process (the pool is never destroyed: a sleeping thread must not touch it while the process
+// unloads).  Waking a thread takes 20-40 us, longer than a 1 MB copy: three of them, the near ones, stay awake for half a
+// millisecond behind a copy, so that a caller who serves one request after the other finds them; the far ones join large copies
+// only.
 class HostCopier {
 public:
     static HostCopier &get();
     // `pieces` bodies, taken in order by the calling thread and the workers; `idle`, if given, is called by the calling thread
-    // between its pieces and until all are done
-    void parallel(int pieces, const std::function<void(int)> &body, const std::function<void()> *idle = nullptr);
+    // between its pieces and until all are done; `large`: the far workers take part
+    void parallel(int pieces, bool large, const std::function<void(int)> &body, const std::function<void()> *idle = nullptr);
     void copy(void *dst, const void *src, size_t bytes);
-    // A few workers wake up and wait, awake, for a copy that is to come within a millisecond (waking a sleeping thread takes 20 to
-    // 40 us, as long as copying a 1.7 MB result).
-    void rouse();
-    // below this one thread is faster than waking others (2.5 MB: 33 us with one thread, 4-11 us with workers that are awake)
-    static constexpr size_t kParallelBytes = size_t(3) << 19;
-    static constexpr size_t kPiece = size_t(256) << 10;
+    void rouse();   // a copy is to come within half a millisecond: the near workers wake up for it
+    static constexpr size_t kAloneBytes = size_t(192) << 10;   // one thread's copy (8 us) up to here
+    static constexpr size_t kLargeBytes = size_t(8) << 20;
+    static constexpr size_t kPiece = size_t(512) << 10;
 
 private:
     HostCopier() = default;
     void start();
-    void worker();
+    void worker(bool near);
+    static constexpr int kNear = 3;
     bool started_ = false;
     const std::function<void(int)> *body_ = nullptr;
     int pieces_ = 0;
-    std::atomic<unsigned> generation_{0};   // number of the copy
-    std::atomic<unsigned> calls_{0};        // the futex word: changes with every copy and every rouse()
-    std::atomic<unsigned> open_{0};         // generation of the copy that workers may join (0: none)
+    std::atomic<unsigned> generation_{0};                        // number of the copy
+    std::atomic<unsigned> open_{0};                              // generation of the copy that workers may join (0: none)
+    std::atomic<unsigned> near_calls_{0}, far_calls_{0};         // futex words
+    std::atomic<int> near_asleep_{0}, far_asleep_{0};
     std::atomic<int> next_{0}, busy_{0};
 };
 
@@ -48,20 +52,22 @@ class HostStage {
 public:
     static constexpr size_t kPart = size_t(4) << 20;      // bytes per staging buffer of the ring, and per step of a large transfer
     static constexpr int kParts = 4;
-    static constexpr int kMaxChunks = 8;                  // steps in which a batch arrives
-    static constexpr size_t kBatch = size_t(256) << 20;   // largest transfer that is staged as a whole
-    static constexpr size_t kPull = kPart;                // largest upload that a kernel reads from host memory
+    static constexpr int kMaxChunks = 4;                  // steps in which a batch arrives (the copy engine takes 25-35 us from one to the next)
+    static constexpr size_t kBatch = size_t(256) << 20;   // largest transfer that is staged as a whole (or one image)
     static constexpr size_t kChunk = size_t(64) << 10;   // bytes of the result that are announced together
     static constexpr size_t kAlone = 3 * kChunk;          // results up to this size are fetched by one thread
-    static constexpr size_t kResult = size_t(4) << 20;    // largest result a pass delivers to host memory by itself
+    static constexpr size_t kResult = kDeliveredFloats * sizeof(float);   // largest result a pass delivers to host memory by itself
 
     void create();   // with the device context (pinned memory goes with the process: the runtime may be unloaded before static objects are)
 
     // Copies `bytes` to the device behind what `stream` holds.  Returns when the caller's memory may change again; the
     // last part may still be on its way (in stream order).
     void upload(void *dst, const void *src, size_t bytes, hipStream_t stream);
-    // The same for a batch of `total` <= kBatch bytes in chunks of `bytes` bytes each (the last may be shorter), on the stream
-    // `link` behind what `stream` holds: chunk c has arrived for a stream that called arrived(c, stream).
+    // The same for a batch of images in the host's layout, which kernels read from the staging buffer and write as a view.
+    void upload_images(const TensorView &dst, int batch, const float *src, hipStream_t stream);
+    // A batch of `total` <= kBatch bytes to device memory as it is, in chunks of `bytes` bytes (the last may be shorter), by the
+    // copy engine and on the stream `link`, which waits for what `stream` holds: chunk c has arrived for a stream that called
+    // arrived(c, stream).  (Kernels that read host memory would share the device with those of `stream`.)
     void upload_chunks(void *dst, const void *src, size_t total, size_t bytes, hipStream_t link, hipStream_t stream);
     void arrived(int chunk, hipStream_t stream);
     // Scattered sources that lie next to each other on the device: `pieces` ascending by `to`, an offset from `dst`, without
@@ -80,9 +86,8 @@ public:
     // it, the same kernel then writes it to pinned memory, chunk after chunk with a word for each, so that copying a chunk
     // to the caller runs beside the transfer of the ones behind it.
     struct Result {
-        const float *src = nullptr;   // null: only the word
+        TensorView view;   // ptr null: only the word
         int batch = 0;
-        long long image = 0, bstride = 0;   // floats
     };
     void signal(const Result &result, hipStream_t stream);
     void wait(hipStream_t stream);                                  // for the pass behind the last signal()

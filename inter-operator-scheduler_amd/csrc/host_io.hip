@@ -11,7 +11,7 @@
 #include <sys/syscall.h>
 #include <unistd.h>
 #if defined(__x86_64__)
-#include <emmintrin.h>
+#include <immintrin.h>
 #endif
 
 #include "runtime.h"
@@ -30,34 +30,39 @@ static inline void pause() {
 #endif
 }
 
-void HostCopier::rouse() {
-    if (!started_) start();
-    calls_.fetch_add(1);
-    syscall(SYS_futex, reinterpret_cast<unsigned *>(&calls_), FUTEX_WAKE_PRIVATE, 3, nullptr, nullptr, 0);
+static void futex_wait(std::atomic<unsigned> &word, unsigned value) {
+    syscall(SYS_futex, reinterpret_cast<unsigned *>(&word), FUTEX_WAIT_PRIVATE, value, nullptr, nullptr, 0);
+}
+static void futex_wake(std::atomic<unsigned> &word) {
+    syscall(SYS_futex, reinterpret_cast<unsigned *>(&word), FUTEX_WAKE_PRIVATE, INT_MAX, nullptr, nullptr, 0);
 }
 
 void HostCopier::start() {
     started_ = true;
-    // half of the processors this process may use, eight at most: past that the copies are bound by memory, not by threads
-    const int n = std::min(8, std::max(1, (int)std::thread::hardware_concurrency() / 2));
-    for (int i = 1; i < n; i++) std::thread([this]() { worker(); }).detach();
+    // three quarters of the processors, twelve threads at most: large copies are bound by memory from there on (69 MB that lie in no
+    // cache: 530 us with 8 threads, 420 with 12 and with 15)
+    const int n = std::min(12, std::max(1, (int)std::thread::hardware_concurrency() * 3 / 4));
+    for (int i = 1; i < n; i++) std::thread([this, i]() { worker(i <= kNear); }).detach();
 }
 
-void HostCopier::worker() {
-    unsigned seen = 0, heard = 0;
+void HostCopier::worker(bool near) {
+    using clock = std::chrono::steady_clock;
+    std::atomic<unsigned> &calls = near ? near_calls_ : far_calls_;
+    std::atomic<int> &asleep = near ? near_asleep_ : far_asleep_;
+    unsigned seen = 0;
     for (;;) {
-        const unsigned call = calls_.load();
+        const unsigned call = calls.load();
         unsigned now = generation_.load();
-        if (now == seen && call == heard) {
-            syscall(SYS_futex, reinterpret_cast<unsigned *>(&calls_), FUTEX_WAIT_PRIVATE, call, nullptr, nullptr, 0);
-            continue;
+        if (now == seen && near) {
+            const auto until = clock::now() + std::chrono::microseconds(500);
+            while ((now = generation_.load()) == seen && clock::now() < until)
+                for (int i = 0; i < 32; i++) pause();
         }
-        heard = call;
-        if (now == seen) {   // roused
-            const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-            while ((now = generation_.load()) == seen && std::chrono::steady_clock::now() < until)
-                for (int i = 0; i < 16; i++) pause();
-            if (now == seen) continue;
+        if (now == seen) {
+            asleep.fetch_add(1);
+            futex_wait(calls, call);
+            asleep.fetch_sub(1);
+            continue;
         }
         seen = now;
         // either the owner sees this thread in busy_ and waits for it, or this thread sees that the copy is closed
@@ -68,7 +73,13 @@ void HostCopier::worker() {
     }
 }
 
-void HostCopier::parallel(int pieces, const std::function<void(int)> &body, const std::function<void()> *idle) {
+void HostCopier::rouse() {
+    if (!started_) start();
+    near_calls_.fetch_add(1);
+    if (near_asleep_.load() > 0) futex_wake(near_calls_);
+}
+
+void HostCopier::parallel(int pieces, bool large, const std::function<void(int)> &body, const std::function<void()> *idle) {
     if (pieces <= 1) {
         if (pieces == 1) body(0);
         if (idle != nullptr) (*idle)();
@@ -82,8 +93,12 @@ void HostCopier::parallel(int pieces, const std::function<void(int)> &body, cons
     if (generation == 0) generation = 1;
     open_.store(generation);
     generation_.store(generation);
-    calls_.fetch_add(1);
-    syscall(SYS_futex, reinterpret_cast<unsigned *>(&calls_), FUTEX_WAKE_PRIVATE, INT_MAX, nullptr, nullptr, 0);
+    near_calls_.fetch_add(1);
+    if (near_asleep_.load() > 0) futex_wake(near_calls_);
+    if (large) {
+        far_calls_.fetch_add(1);
+        if (far_asleep_.load() > 0) futex_wake(far_calls_);
+    }
     for (int i; (i = next_.fetch_add(1)) < pieces;) {
         body(i);
         if (idle != nullptr) (*idle)();
@@ -97,35 +112,49 @@ void HostCopier::parallel(int pieces, const std::function<void(int)> &body, cons
 }
 
 void HostCopier::copy(void *dst, const void *src, size_t bytes) {
-    if (bytes < kParallelBytes) {
+    if (bytes <= kAloneBytes) {
         memcpy(dst, src, bytes);
         return;
     }
-    parallel((int)((bytes + kPiece - 1) / kPiece), [&](int i) {
-        const size_t at = (size_t)i * kPiece;
-        memcpy(static_cast<char *>(dst) + at, static_cast<const char *>(src) + at, std::min(kPiece, bytes - at));
+    const size_t piece = std::min(kPiece, std::max(size_t(32) << 10, bytes / 16));
+    parallel((int)((bytes + piece - 1) / piece), bytes >= kLargeBytes, [&](int i) {
+        const size_t at = (size_t)i * piece;
+        memcpy(static_cast<char *>(dst) + at, static_cast<const char *>(src) + at, std::min(piece, bytes - at));
     });
 }
 
 // Fills a buffer that only the link will read and that is larger than the caches: stores past the caches save reading every
 // line of the buffer first (a third of the copy's memory traffic).
-static void copy_past_caches(char *dst, const char *src, size_t bytes) {
 #if defined(__x86_64__)
-    if ((reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-        const size_t lines = bytes / 64;
-        for (size_t i = 0; i < lines; i++, dst += 64, src += 64) {
-            const __m128i a = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src)), b = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + 16));
-            const __m128i c = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + 32)), d = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + 48));
-            _mm_stream_si128(reinterpret_cast<__m128i *>(dst), a);
-            _mm_stream_si128(reinterpret_cast<__m128i *>(dst + 16), b);
-            _mm_stream_si128(reinterpret_cast<__m128i *>(dst + 32), c);
-            _mm_stream_si128(reinterpret_cast<__m128i *>(dst + 48), d);
-        }
-        _mm_sfence();
-        bytes -= 64 * lines;
+__attribute__((target("avx512f"))) static size_t stream_lines_512(char *dst, const char *src, size_t bytes) {
+    const size_t whole = bytes & ~size_t(255);
+    for (size_t i = 0; i < whole; i += 256) {
+        const __m512i a = _mm512_loadu_si512(src + i), b = _mm512_loadu_si512(src + i + 64);
+        const __m512i c = _mm512_loadu_si512(src + i + 128), d = _mm512_loadu_si512(src + i + 192);
+        _mm512_stream_si512(reinterpret_cast<__m512i *>(dst + i), a);
+        _mm512_stream_si512(reinterpret_cast<__m512i *>(dst + i + 64), b);
+        _mm512_stream_si512(reinterpret_cast<__m512i *>(dst + i + 128), c);
+        _mm512_stream_si512(reinterpret_cast<__m512i *>(dst + i + 192), d);
     }
+    _mm_sfence();
+    return whole;
+}
+static size_t stream_lines_128(char *dst, const char *src, size_t bytes) {
+    const size_t whole = bytes & ~size_t(63);
+    for (size_t i = 0; i < whole; i += 16)
+        _mm_stream_si128(reinterpret_cast<__m128i *>(dst + i), _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + i)));
+    _mm_sfence();
+    return whole;
+}
 #endif
-    memcpy(dst, src, bytes);
+
+static void copy_past_caches(char *dst, const char *src, size_t bytes) {
+    size_t done = 0;
+#if defined(__x86_64__)
+    static const bool wide = __builtin_cpu_supports("avx512f");
+    if ((reinterpret_cast<uintptr_t>(dst) & 63) == 0) done = wide ? stream_lines_512(dst, src, bytes) : stream_lines_128(dst, src, bytes);
+#endif
+    memcpy(dst + done, src + done, bytes - done);
 }
 
 // ---- pinned buffers ------------------------------------------------------------------------------------------------------
@@ -175,6 +204,106 @@ char *HostStage::Batch::take(size_t need) {
 
 void HostStage::arrived(int chunk, hipStream_t stream) { IOS_HIP(hipStreamWaitEvent(stream, chunk_events_[chunk], 0)); }
 
+// Kernels read the staging buffer at the link's rate, like the copy engine, turn the images into the layout of views on the
+// way, and follow and precede the kernels of their stream without the hand-over between engines (600 KB: 25 us less per pass).
+void HostStage::upload_images(const TensorView &dst, int batch, const float *src, hipStream_t stream) {
+    const size_t pixels = (size_t)dst.H * dst.W, image = pixels * dst.C;   // floats
+    const int group = (int)std::max<size_t>(1, std::min<size_t>((size_t)batch, kBatch / (image * sizeof(float))));
+    struct Step {
+        TensorView part;
+        const float *from;
+        int images, pieces;
+        long long plane;
+    };
+    struct Copy {
+        size_t at, floats;   // in the group
+        int step;
+    };
+    std::vector<Step> steps;
+    std::vector<Copy> copies;
+    for (int first = 0; first < batch; first += group) {
+        const int images = std::min(group, batch - first);
+        const size_t floats = (size_t)images * image, bytes = floats * sizeof(float);
+        const bool ring = bytes <= kPart;
+        float *memory = reinterpret_cast<float *>(ring ? acquire() : inputs_.take(bytes));
+        const float *host = src + (size_t)first * image;
+        TensorView view = dst;
+        view.ptr += (size_t)first * pixels * dst.pstride;
+        // Steps, so that the link starts before everything is staged (a third at a time and 768 KB at least: a step of 150 KB takes
+        // 5 us and the launch of the next one another 5): whole images, or bands of pixels (few channels) or of channels of a
+        // single one.  Every step is copied in pieces.
+        steps.clear();
+        copies.clear();
+        const size_t step_floats = std::max(size_t(192) << 10, std::min((floats + 2) / 3, size_t(512) << 10));
+        const size_t piece_floats = std::max(size_t(8) << 10, std::min(floats / 16, HostCopier::kPiece / sizeof(float)));
+        auto add_copy = [&](size_t at, size_t n) {
+            for (size_t p = 0; p < n; p += piece_floats) {
+                copies.push_back({at + p, std::min(piece_floats, n - p), (int)steps.size() - 1});
+                steps.back().pieces++;
+            }
+        };
+        if (images > 1) {
+            const int per_step = (int)std::max<size_t>(1, step_floats / image);
+            for (int i = 0; i < images; i += per_step) {
+                Step s{view, memory + i * image, std::min(per_step, images - i), 0, 0};
+                s.part.ptr += (size_t)i * pixels * dst.pstride;
+                steps.push_back(s);
+                add_copy(i * image, s.images * image);
+            }
+        } else if (dst.C <= 4) {
+            const size_t band = (step_floats / dst.C + 63) & ~size_t(63);
+            for (size_t p = 0; p < pixels; p += band) {
+                const size_t n = std::min(band, pixels - p);
+                Step s{view, memory + p, 1, 0, (long long)pixels};
+                s.part.ptr += p * dst.pstride;
+                s.part.H = 1;
+                s.part.W = (int)n;
+                steps.push_back(s);
+                for (int c = 0; c < dst.C; c++) add_copy(c * pixels + p, n);
+            }
+        } else {
+            const int band = (int)((step_floats / pixels + 32) & ~size_t(31));
+            for (int c = 0; c < dst.C; c += band) {
+                Step s{view, memory + c * pixels, 1, 0, 0};
+                s.part.ptr += c;
+                s.part.C = std::min(band, dst.C - c);
+                steps.push_back(s);
+                add_copy(c * pixels, s.part.C * pixels);
+            }
+        }
+        auto copy = [&](const Copy &c) {
+            char *to = reinterpret_cast<char *>(memory + c.at);
+            const char *from = reinterpret_cast<const char *>(host + c.at);
+            if (ring) memcpy(to, from, c.floats * sizeof(float));
+            else copy_past_caches(to, from, c.floats * sizeof(float));
+        };
+        if (bytes <= HostCopier::kAloneBytes) {
+            size_t next = 0;
+            for (size_t s = 0; s < steps.size(); s++) {
+                for (; next < copies.size() && copies[next].step == (int)s; next++) copy(copies[next]);
+                launch_to_view(steps[s].from, steps[s].part, steps[s].images, stream, steps[s].plane);
+            }
+        } else {
+            // one shared-out copy; the calling thread hands a step to the link as soon as its pieces are staged
+            std::vector<std::atomic<int>> staged(steps.size());
+            for (auto &count : staged) count.store(0, std::memory_order_relaxed);
+            size_t sent = 0;
+            const std::function<void()> hand_over = [&]() {
+                for (; sent < steps.size() && staged[sent].load(std::memory_order_acquire) == steps[sent].pieces; sent++)
+                    launch_to_view(steps[sent].from, steps[sent].part, steps[sent].images, stream, steps[sent].plane);
+            };
+            HostCopier::get().parallel((int)copies.size(), bytes >= HostCopier::kLargeBytes, [&](int i) {
+                copy(copies[i]);
+                staged[copies[i].step].fetch_add(1, std::memory_order_release);
+            }, &hand_over);
+        }
+        IOS_HIP(hipGetLastError());
+        IOS_HIP(hipEventRecord(ring ? drained_[turn_] : inputs_.drained, stream));
+        if (ring) used_[turn_] = true;
+        else inputs_.used = true;
+    }
+}
+
 void HostStage::upload_chunks(void *dst, const void *src, size_t total, size_t bytes, hipStream_t link, hipStream_t stream) {
     char *memory = inputs_.take(total);
     IOS_HIP(hipEventRecord(order_, stream));
@@ -195,7 +324,7 @@ void HostStage::upload_chunks(void *dst, const void *src, size_t total, size_t b
             sent++;
         }
     };
-    HostCopier::get().parallel(chunks * per_chunk, [&](int piece) {
+    HostCopier::get().parallel(chunks * per_chunk, true, [&](int piece) {
         const int c = piece / per_chunk;
         const size_t at = (size_t)(piece - c * per_chunk) * HostCopier::kPiece, limit = chunk_bytes(c), from = (size_t)c * bytes + at;
         if (at < limit) copy_past_caches(memory + from, static_cast<const char *>(src) + from, std::min(HostCopier::kPiece, limit - at));
@@ -250,7 +379,7 @@ void HostStage::upload_pieces(char *dst, const std::vector<Piece> &all, hipStrea
             sent = limit;
             if (failed == hipSuccess) step(limit);
         };
-        HostCopier::get().parallel(runs, [&](int run) {
+        HostCopier::get().parallel(runs, span >= HostCopier::kLargeBytes, [&](int run) {
             for (size_t i = cuts[run]; i < cuts[run + 1]; i++) copy_past_caches(memory + (all[i].to - base), all[i].src, all[i].bytes);
             staged[run].store(1, std::memory_order_release);
         }, &hand_over);
@@ -261,68 +390,15 @@ void HostStage::upload_pieces(char *dst, const std::vector<Piece> &all, hipStrea
     }
 }
 
-// Bound by the link; a kernel that reads host memory reaches its rate with 256 blocks, like the copy engine, and follows and
-// precedes the kernels of its stream without the hand-over between engines (600 KB: 25 us less per pass).
-__global__ __launch_bounds__(256) void pull_kernel(float *dst, const float *src, unsigned words) {
-    const unsigned thread = blockIdx.x * blockDim.x + threadIdx.x, threads = gridDim.x * blockDim.x, quads = words >> 2;
-    const float4 *from = reinterpret_cast<const float4 *>(src);
-    float4 *to = reinterpret_cast<float4 *>(dst);
-    for (unsigned i = thread; i < quads; i += threads) to[i] = from[i];
-    for (unsigned i = 4 * quads + thread; i < words; i += threads) dst[i] = src[i];
-}
-
 void HostStage::upload(void *dst, const void *src, size_t bytes, hipStream_t stream) {
-    if (bytes > kPull || bytes % sizeof(float) != 0) {
-        for (size_t at = 0; at < bytes; at += kPart) {
-            const size_t n = std::min(kPart, bytes - at);
-            char *buffer = acquire();
-            HostCopier::get().copy(buffer, static_cast<const char *>(src) + at, n);
-            IOS_HIP(hipMemcpyAsync(static_cast<char *>(dst) + at, buffer, n, hipMemcpyHostToDevice, stream));
-            IOS_HIP(hipEventRecord(drained_[turn_], stream));
-            used_[turn_] = true;
-        }
-        return;
+    for (size_t at = 0; at < bytes; at += kPart) {
+        const size_t n = std::min(kPart, bytes - at);
+        char *buffer = acquire();
+        HostCopier::get().copy(buffer, static_cast<const char *>(src) + at, n);
+        IOS_HIP(hipMemcpyAsync(static_cast<char *>(dst) + at, buffer, n, hipMemcpyHostToDevice, stream));
+        IOS_HIP(hipEventRecord(drained_[turn_], stream));
+        used_[turn_] = true;
     }
-    // steps of a size that lets the link start before everything is staged
-    char *buffer = acquire();
-    const size_t step = bytes > (size_t(256) << 10) ? std::max(size_t(128) << 10, (bytes / 4 + 255) & ~size_t(255)) : bytes;
-    auto pull = [&](size_t at, size_t n) {
-        const unsigned words = (unsigned)(n / sizeof(float));
-        hipLaunchKernelGGL(pull_kernel, dim3(std::min(256u, words / 1024 + 1)), dim3(256), 0, stream,
-                           reinterpret_cast<float *>(static_cast<char *>(dst) + at), reinterpret_cast<const float *>(buffer + at), words);
-    };
-    const int steps = (int)((bytes + step - 1) / step);
-    auto stage = [&](int s) {
-        const size_t at = (size_t)s * step;
-        memcpy(buffer + at, static_cast<const char *>(src) + at, std::min(step, bytes - at));
-    };
-    if (bytes < HostCopier::kParallelBytes) {
-        for (int s = 0; s < steps; s++) {
-            stage(s);
-            pull((size_t)s * step, std::min(step, bytes - (size_t)s * step));
-        }
-    } else {
-        constexpr size_t kSlice = size_t(128) << 10;
-        const int slices = (int)((bytes + kSlice - 1) / kSlice);
-        std::atomic<char> staged[kPart / kSlice] = {};
-        int ready = 0;
-        size_t sent = 0;
-        const std::function<void()> hand_over = [&]() {
-            while (ready < slices && staged[ready].load(std::memory_order_acquire) != 0) ready++;
-            const size_t limit = std::min(bytes, (size_t)ready * kSlice);
-            if (limit == sent || (limit - sent < step && limit < bytes)) return;
-            pull(sent, limit - sent);
-            sent = limit;
-        };
-        HostCopier::get().parallel(slices, [&](int i) {
-            const size_t at = (size_t)i * kSlice;
-            memcpy(buffer + at, static_cast<const char *>(src) + at, std::min(kSlice, bytes - at));
-            staged[i].store(1, std::memory_order_release);
-        }, &hand_over);
-    }
-    IOS_HIP(hipGetLastError());
-    IOS_HIP(hipEventRecord(drained_[turn_], stream));
-    used_[turn_] = true;
 }
 
 void HostStage::download(void *dst, const void *src, size_t bytes, hipStream_t stream) {
@@ -358,52 +434,70 @@ void HostStage::download(void *dst, const void *src, size_t bytes, hipStream_t s
 // Four groups of 16 blocks take the chunks in turn: enough stores in flight for the link's rate while a group waits for the
 // acknowledgement of its chunk, and the chunks still complete nearly in order (eight groups: 52 instead of 39 us for 1.7 MB).
 constexpr int kGroups = 4, kGroupBlocks = 16;
-__global__ __launch_bounds__(256) void signal_kernel(float *dst, const float *src, unsigned batch, unsigned image, long long bstride, unsigned chunk,
-                                                     unsigned *tickets, unsigned *words, unsigned pass) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(words, pass, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (src == nullptr) return;
-    const unsigned total = batch * image;
+struct SignalArgs {
+    float *dst;
+    const float *src;
+    unsigned total, image, plane, chunk;   // floats of the result, of an image, pixels of an image; floats of a chunk
+    int pstride;
+    unsigned *tickets, *words, pass;
+    FastDiv div_image, div_plane;
+};
+__global__ __launch_bounds__(256) void signal_kernel(SignalArgs a) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(a.words, a.pass, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (a.src == nullptr) return;
     const unsigned group_blocks = gridDim.x < kGroupBlocks ? gridDim.x : kGroupBlocks;   // (one block for a single small chunk)
     const unsigned groups = gridDim.x / group_blocks, group = blockIdx.x / group_blocks;
     const unsigned thread = (blockIdx.x - group * group_blocks) * blockDim.x + threadIdx.x, threads = group_blocks * blockDim.x;
-    const bool dense = bstride == (long long)image;
+    // element i of the host's layout (gathered through the caches: the link is the bound)
+    auto element = [&](unsigned i) -> float {
+        const unsigned b = fast_div(i, a.div_image), rest = i - b * a.image;
+        const unsigned c = fast_div(rest, a.div_plane), r = rest - c * a.plane;
+        return a.src[(long long)(b * a.plane + r) * a.pstride + c];
+    };
     unsigned c = group;
-    for (unsigned begin = c * chunk; begin < total; begin += groups * chunk, c += groups) {
-        const unsigned end = begin + chunk < total ? begin + chunk : total;
+    for (unsigned begin = c * a.chunk; begin < a.total; begin += groups * a.chunk, c += groups) {
+        const unsigned end = begin + a.chunk < a.total ? begin + a.chunk : a.total;
         // stores at system scope go to host memory by themselves: the fence that would send plain ones there writes back the whole
         // L2, block after block (1.7 MB to the caller: 54 instead of 39 us)
-        if (dense) {
-            const unsigned pairs = (end - begin) >> 1;
-            const unsigned long long *from = reinterpret_cast<const unsigned long long *>(src + begin);
-            unsigned long long *to = reinterpret_cast<unsigned long long *>(dst + begin);
-            for (unsigned i = thread; i < pairs; i += threads) __hip_atomic_store(to + i, from[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            if ((end - begin) & 1u && thread == 0) __hip_atomic_store(dst + end - 1, src[end - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        } else {
-            for (unsigned i = begin + thread; i < end; i += threads) {
-                const unsigned b = i / image;
-                __hip_atomic_store(dst + i, src[(long long)b * bstride + (i - b * image)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
+        const unsigned pairs = (end - begin) >> 1;
+        unsigned long long *to = reinterpret_cast<unsigned long long *>(a.dst + begin);
+        for (unsigned i = thread; i < pairs; i += threads) {
+            const unsigned low = __float_as_uint(element(begin + 2 * i)), high = __float_as_uint(element(begin + 2 * i + 1));
+            __hip_atomic_store(to + i, (unsigned long long)high << 32 | low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
+        if ((end - begin) & 1u && thread == 0) __hip_atomic_store(a.dst + end - 1, element(end - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         // a block's stores are acknowledged before its ticket is drawn; the chunk's last ticket announces it
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (threadIdx.x != 0) continue;
         if (group_blocks > 1) {
-            if (__hip_atomic_fetch_add(tickets + c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != group_blocks - 1) continue;
-            __hip_atomic_store(tickets + c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__hip_atomic_fetch_add(a.tickets + c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != group_blocks - 1) continue;
+            __hip_atomic_store(a.tickets + c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __hip_atomic_store(words + 1 + c, pass, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(a.words + 1 + c, a.pass, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
 void HostStage::signal(const Result &result, hipStream_t stream) {
-    const size_t bytes = result.src != nullptr ? sizeof(float) * (size_t)result.batch * (size_t)result.image : 0;
+    const TensorView &v = result.view;
+    SignalArgs a{};
+    a.dst = result_;
+    a.src = v.ptr;
+    a.plane = v.ptr != nullptr ? (unsigned)(v.H * v.W) : 1;
+    a.image = v.ptr != nullptr ? a.plane * (unsigned)v.C : 1;
+    a.total = v.ptr != nullptr ? (unsigned)result.batch * a.image : 0;
+    a.chunk = (unsigned)(kChunk / sizeof(float));
+    a.pstride = v.pstride;
+    a.tickets = tickets_;
+    a.words = words_;
+    a.pass = ++pass_;
+    a.div_image = make_fast_div(a.image);
+    a.div_plane = make_fast_div(a.plane);
+    const size_t bytes = sizeof(float) * (size_t)a.total;
     if (bytes > kResult) throw std::runtime_error("internal: result larger than its staging buffer");
-    pass_++;
     if (bytes > kAlone) HostCopier::get().rouse();
     const int blocks = bytes <= (size_t(16) << 10) ? 1 : bytes <= kChunk ? kGroupBlocks : kGroups * kGroupBlocks;
-    hipLaunchKernelGGL(signal_kernel, dim3(blocks), dim3(256), 0, stream, result_, result.src, (unsigned)result.batch, (unsigned)result.image,
-                       result.bstride, (unsigned)(kChunk / sizeof(float)), tickets_, words_, pass_);
+    hipLaunchKernelGGL(signal_kernel, dim3(blocks), dim3(256), 0, stream, a);
     IOS_HIP(hipGetLastError());
 }
 
@@ -439,7 +533,7 @@ void HostStage::fetch(void *dst, size_t bytes, hipStream_t stream) {
     if (bytes <= kAlone) {
         for (int c = 0; c < chunks; c++) body(c);
     } else {
-        HostCopier::get().parallel(chunks, body);
+        HostCopier::get().parallel(chunks, false, body);
     }
     IOS_HIP((hipError_t)failed.load());
 }

@@ -1,9 +1,12 @@
 // Device kernels of the runtime and their host-side launchers (gfx950 / CDNA4 only).
 //
-// All tensors are fp32 NCHW *views*: a base pointer to (n=0, c=0), the extents C/H/W and a batch stride
-// in elements.  The channel stride is always H*W, so a channel slice or a window inside a wider concat
-// buffer is again a view; producers write straight into such windows and consumers read slices without
-// copies.
+// All tensors are fp32 NHWC *views*: a pointer to element (n=0, h=0, w=0, c=0), the extents C/H/W and the distance of
+// neighbouring pixels in elements.  Pixels follow each other in (n, h, w) order without gaps of their own, so a channel slice or
+// a window inside a wider concat buffer is again a view; producers write straight into such windows and consumers read
+// slices without copies.  The channels of a pixel lie side by side because that is what every kernel reads: four consecutive
+// k of an implicit GEMM, four channels of a pool or of a sum are one 16-byte load, where a channel-major tensor takes four.
+// Loads and stores assume 4-byte alignment only (a window may start at any channel).  A 16-byte load of a pixel's last channels
+// may run up to twelve bytes past them, into the next pixel, a neighbouring window or the padding behind a tensor.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -20,8 +23,50 @@ constexpr int kMaxNaryInputs = 8;   // views one launch adds (or multiplies)
 struct TensorView {
     float *ptr = nullptr;  // element (0, 0, 0, 0)
     int C = 0, H = 0, W = 0;
-    long long bstride = 0;  // elements between images
+    int pstride = 0;       // elements between pixels
 };
+
+// Division of a 32-bit unsigned by a divisor fixed at launch time (Granlund-Montgomery): exact for every dividend,
+// five instructions instead of the ~20 of a hardware-less integer division.
+struct FastDiv {
+    unsigned m, s1, s2;
+};
+
+inline FastDiv make_fast_div(unsigned d) {   // d >= 1
+    unsigned l = 0;
+    while ((1ull << l) < d) l++;   // ceil(log2(d))
+    FastDiv f;
+    f.m = (unsigned)((((1ull << l) - d) << 32) / d + 1);
+    f.s1 = l < 1 ? l : 1;
+    f.s2 = l > 0 ? l - 1 : 0;
+    return f;
+}
+
+__device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv &f) {
+    const unsigned t = __umulhi(f.m, n);
+    return (t + ((n - t) >> f.s1)) >> f.s2;
+}
+
+// Activation of V values of a lane.  The usual ones (none, ReLU) are one integer maximum per value (negative floats are negative
+// integers); the others go through one copy of their code in turn: inlined once per value, tanh and sigmoid put kilobytes of
+// code between a kernel's last load and its store, and skipping them cost a batch-1 launch a microsecond of instruction fetches.
+template <int V>
+__device__ __forceinline__ void apply_activation(float (&v)[V], int act) {
+    if (__builtin_expect(act <= ACT_RELU, 1)) {
+        const int floor = act == ACT_RELU ? 0 : (int)0x80000000;
+#pragma unroll
+        for (int k = 0; k < V; k++) v[k] = __int_as_float(max(__float_as_int(v[k]), floor));
+        return;
+    }
+#pragma unroll 1
+    for (int n = 0; n < V; n++) {
+        const float x = v[0];
+        const float y = act == ACT_TANH ? tanhf(x) : 1.0f / (1.0f + __expf(-x));
+#pragma unroll
+        for (int k = 0; k + 1 < V; k++) v[k] = v[k + 1];
+        v[V - 1] = y;
+    }
+}
 
 // ---- convolution ------------------------------------------------------------------------------------
 struct ConvProblem {
@@ -78,6 +123,10 @@ size_t conv_workspace_floats(const ConvProblem &p, const ConvLaunch &l);
 // Ticket counters the one-kernel split-K form needs: one unsigned per (group, output tile), zero before the
 // first launch (the kernel leaves them zero); 0 when the configuration does not split K.
 size_t conv_counter_count(const ConvProblem &p, const ConvLaunch &l);
+// Bytes from a convolution's first input element to the end of the last quad of channels of its last pixel.
+inline unsigned long long conv_input_extent(const ConvProblem &p, int pstride) {
+    return (((unsigned long long)p.B * p.H * p.W - 1) * (unsigned long long)pstride + (unsigned long long)((p.IC + 3) & ~3)) * 4ull;
+}
 // The matrix path indexes packed filter rows with 16 bits and pixels / input offsets with 31 bits.
 bool conv_matrix_path_supported(const ConvProblem &p);
 
@@ -111,7 +160,10 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
                       const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce, hipStream_t stream,
                       const TensorView *residual = nullptr, bool post_relu = false);
 
-// Depth-wise convolution (groups == IC == OC), filters in their original [C][1][KH][KW] layout.  With `more`, the input is
+// Filters of a depth-wise convolution: w[C][1][KH][KW] -> packed[tap][C rounded up to 4] (padding zero).
+inline size_t dwconv_packed_floats(const ConvProblem &p) { return (size_t)p.KH * p.KW * ((p.OC + 3) & ~3); }
+void launch_pack_depthwise(const ConvProblem &p, const float *w, float *packed, hipStream_t stream);
+// Depth-wise convolution (groups == IC == OC), filters from launch_pack_depthwise.  With `more`, the input is
 // x + more[0] + ... + more[nmore - 1] (at most kMaxNaryInputs views in all, added left to right before the folded ReLU).
 void launch_dwconv(const ConvProblem &p, const TensorView &x, const float *w, const float *bias,
                    const TensorView &y, hipStream_t stream, const TensorView *more = nullptr, int nmore = 0);
@@ -138,15 +190,18 @@ void launch_global_pool(const PoolProblem &p, const TensorView &x, const TensorV
 // ---- element-wise -----------------------------------------------------------------------------------
 struct NaryArgs {
     const float *src[kMaxNaryInputs];
-    long long src_bstride[kMaxNaryInputs];
+    int src_pstride[kMaxNaryInputs];
     int count;
 };
 // y = act(src0 (+|*) src1 (+|*) ...), left to right; more than kMaxNaryInputs inputs are handled by the
 // caller through accumulation (accumulate != 0 also combines the current contents of y first).
-void launch_nary(const NaryArgs &a, int multiply, int accumulate, int act, int B, long long chw,
-                 const TensorView &y, hipStream_t stream);
+void launch_nary(const NaryArgs &a, int multiply, int accumulate, int act, int B, const TensorView &y, hipStream_t stream);
 // y = act(x) for views; act == ACT_NONE is a strided copy.
 void launch_unary(const TensorView &x, const TensorView &y, int act, int B, hipStream_t stream);
+// Between a host tensor's layout (NCHW, dense) and a view: x -> y and back.  `nchw` may lie in host memory.  plane > 0: elements
+// between the channels of `nchw` where the view is a part of its pixels (one image).
+void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t stream, long long plane = 0);
+void launch_from_view(const TensorView &x, float *nchw, int B, hipStream_t stream);
 // Fill n floats with a deterministic pattern in [-1, 1) (seeded), or with a constant.
 void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream);
 void launch_fill_u32(unsigned *dst, size_t n, unsigned value, hipStream_t stream);

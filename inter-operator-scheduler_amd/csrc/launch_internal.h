@@ -26,8 +26,7 @@ PoolArgs make_pool_args(const PoolProblem &p, const TensorView &x, const TensorV
 DirectConvArgs make_direct_conv_args(const ConvProblem &p, const TensorView &x, const float *w, const float *bias,
                                      const TensorView &y, int *blocks, bool thin = false);
 // further inputs of a depth-wise convolution of a sum (see DirectConvArgs::more)
-void add_dwconv_sources(DirectConvArgs &a, const TensorView *more, int count);
-NaryKernelArgs make_nary_args(const NaryArgs &in, int multiply, int accumulate, int act, int B, long long chw,
-                              const TensorView &y, int *blocks);
+void add_dwconv_sources(DirectConvArgs &a, const TensorView *more, int count, int *blocks);
+NaryKernelArgs make_nary_args(const NaryArgs &in, int multiply, int accumulate, int act, int B, const TensorView &y, int *blocks);
 
 }  // namespace ios

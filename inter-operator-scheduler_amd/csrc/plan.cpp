@@ -589,6 +589,11 @@ private:
         return r ? r->at + ((offset & ~kRegionTag) - r->voff) : offset;
     }
 
+    void place(ViewRef &v) {
+        v.offset = placed(v.offset);
+        v.base = placed(v.base);
+    }
+
     // The prefix ends where its work covers the time the input takes on the link (57 GB/s measured), both estimated: 100 TFLOP/s
     // and 3.5 TB/s are what the kernels of these layers reach at the batches in question.
     void choose_prefix() {
@@ -624,6 +629,7 @@ private:
             if (op.conv >= 0 && plan_.convs[op.conv].ws_floats > 0) touch(plan_.convs[op.conv].ws_off, op.stage);
         }
         choose_prefix();
+        if (plan_.prefix_stages > 0) plan_.landing_off = reserve_region((size_t)batch_ * plan_.input.image_floats(), /*pinned=*/true);
         for (const PlanOp &op : plan_.ops) {   // parts of the batch are in different stages of the prefix at the same time
             if (op.stage >= plan_.prefix_stages) continue;
             for (int stage : {0, plan_.prefix_stages - 1}) {
@@ -632,6 +638,12 @@ private:
             }
         }
         if (Region *r = region_of(plan_.output.offset)) r->pinned = true;
+        const size_t result = (size_t)batch_ * plan_.output.image_floats();
+        if (result > kDeliveredFloats && plan_.output.H * plan_.output.W > 1) {   // written behind the last stage
+            plan_.result_floats = result;
+            plan_.result_off = reserve_region(result);
+            touch(plan_.result_off, last_stage);
+        }
         const bool reuse = planner_arena_reuse();
         for (Region &r : regions_)
             if (r.pinned || !reuse || r.last < 0) {   // (an untouched region belongs to an operator nobody reads: keep it apart)
@@ -662,8 +674,8 @@ private:
         plan_.persistent_floats = base;
         plan_.activation_floats_without_reuse = region_floats_;
         for (Region &r : regions_) r.at += base;
-        // (the vectorised pooling kernel reads up to eight floats past the end of a tensor and discards them: the arena ends
-        // in padding so that such a read stays inside the allocation)
+        // (16-byte loads of a pixel's last channels may run past the end of a tensor: the arena ends in padding so that such a read
+        // stays inside the allocation)
         plan_.arena_floats = base + extent + 64;
         // names of the outputs that a later region overwrites
         for (auto &entry : plan_.tensors) {
@@ -676,28 +688,31 @@ private:
                 }
         }
         for (PlanOp &op : plan_.ops) {
-            op.in.offset = placed(op.in.offset);
-            op.out.offset = placed(op.out.offset);
-            for (ViewRef &v : op.srcs) v.offset = placed(v.offset);
-            if (op.has_residual) op.residual.offset = placed(op.residual.offset);
+            place(op.in);
+            place(op.out);
+            for (ViewRef &v : op.srcs) place(v);
+            if (op.has_residual) place(op.residual);
         }
         for (PlanConv &c : plan_.convs)
             if (c.ws_floats > 0) c.ws_off = placed(c.ws_off);
-        for (auto &entry : plan_.tensors) entry.second.offset = placed(entry.second.offset);
-        plan_.input.offset = placed(plan_.input.offset);
-        plan_.output.offset = placed(plan_.output.offset);
+        for (auto &entry : plan_.tensors) place(entry.second);
+        place(plan_.input);
+        place(plan_.output);
+        if (plan_.prefix_stages > 0) plan_.landing_off = placed(plan_.landing_off);
+        if (plan_.result_floats > 0) plan_.result_off = placed(plan_.result_off);
     }
 
     void allocate_outputs() {
         for (PNode &n : nodes_)
-            if (n.own) n.own_offset = reserve_region((size_t)batch_ * n.C * n.H * n.W, /*pinned=*/n.type == NodeType::Placeholder);
+            if (n.own) n.own_offset = reserve_region((size_t)batch_ * n.H * n.W * padded_channels(n.C), /*pinned=*/n.type == NodeType::Placeholder);
     }
 
     ViewRef view_of(int index) const {
         const PNode &n = nodes_[index];
         if (n.own) {
             ViewRef v;
-            v.offset = n.own_offset;
+            v.base = v.offset = n.own_offset;
+            v.pstride = padded_channels(n.C);
             v.C = n.C;
             v.H = n.H;
             v.W = n.W;
@@ -716,7 +731,8 @@ private:
 
     ViewRef dense_temp(int C, int H, int W) {
         ViewRef v;
-        v.offset = reserve_region((size_t)batch_ * C * H * W);
+        v.base = v.offset = reserve_region((size_t)batch_ * H * W * padded_channels(C));
+        v.pstride = padded_channels(C);
         v.C = C;
         v.H = H;
         v.W = W;
@@ -868,7 +884,7 @@ private:
         if (p.is_depthwise()) {
             kind = OpKind::ConvDepthwise;
         } else if ((p.groups > 1 && (p.ICg() < 4 || p.OCg() < 8)) || !conv_matrix_path_supported(p) ||
-                   ((unsigned long long)(batch_ - 1) * in.bstride + in.image_floats()) * 4ull >= (1ull << 31)) {
+                   conv_input_extent(p, in.pstride) >= (1ull << 31)) {
             // thin groups, or an input view whose extent does not fit the matrix path's 31-bit byte offsets
             kind = OpKind::ConvDirect;
         } else {
@@ -938,7 +954,7 @@ private:
         const ViewRef in = input_view(pool, C, H, W, nullptr);
         ConvProblem p = problem_of(c);
         p.act = ACT_NONE;
-        const bool wide = ((unsigned long long)(batch_ - 1) * in.bstride + in.image_floats()) * 4ull >= (1ull << 31);
+        const bool wide = conv_input_extent(p, in.pstride) >= (1ull << 31);
         const int conv = add_plan_conv(c, p);
         plan_.convs[conv].matrix_path = !wide;
         plan_.convs[conv].linear = true;
@@ -1076,6 +1092,7 @@ private:
         }
         for (size_t i = 0; i < plan_.convs.size(); i++) {
             PlanConv &conv = plan_.convs[i];
+            if (conv.problem.is_depthwise()) conv.packed_off = reserve(dwconv_packed_floats(conv.problem));
             if (!conv.matrix_path) continue;
             conv.launch = chooser_(conv.problem, share[i]);
             conv.packed_off = reserve(conv_packed_floats(conv.problem, conv.launch));

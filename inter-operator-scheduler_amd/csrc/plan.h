@@ -2,8 +2,8 @@
 // block or stage document compiles to.  Planning is pure host code; nothing here touches the device.
 //
 // Memory model: one arena of 4-byte words.  Every operator output, temporary, filter, bias and split-K
-// workspace is a region of it at a 256-byte aligned offset.  Tensor views are
-// (offset, C, H, W, batch stride); a channel slice or a window of a concat buffer is again a view, so
+// workspace is a region of it at a 256-byte aligned offset.  Tensors are NHWC, the channels of a pixel padded to a multiple of
+// four (16-byte boundaries); a channel slice or a window of a concat buffer is again a view, so
 //   * an identity with one input value is an alias (no memory, no work),
 //   * a producer whose whole output is one term of a concat writes directly into the concat buffer,
 //   * a channel slice of a merged convolution is read in place at any batch size,
@@ -24,15 +24,25 @@ namespace ios {
 
 constexpr int kMaxGroups = 16;   // concurrent groups (streams) per stage
 constexpr int kMaxExtent = 1 << 16;     // image sides, filter sides, strides and padding a document may ask for
+constexpr size_t kDeliveredFloats = size_t(1) << 20;   // largest result that a pass writes to host memory by itself
 constexpr int kMaxChannels = 1 << 20;   // channels of a tensor
 
+// elements between the pixels of a tensor of its own
+inline int padded_channels(int C) { return C < 3 ? C : (C + 3) & ~3; }
+
 struct ViewRef {
-    size_t offset = 0;   // in floats from the arena base
+    size_t base = 0;      // of the tensor the view lies in, in floats from the arena base
+    int first = 0;        // channel of that tensor the view begins at
+    int pstride = 0;      // elements between its pixels
     int C = 0, H = 0, W = 0;
+    // The view's place in the tensor as if channels were the outermost dimension of an image: [offset, offset + C * H * W) and
+    // bstride further for every image.  Two views of a tensor overlap where these ranges do (plans are described by them).
+    size_t offset = 0;
     long long bstride = 0;
     ViewRef window(int begin, int end) const {
         ViewRef v = *this;
         v.offset += (size_t)begin * H * W;
+        v.first += begin;
         v.C = end - begin;
         return v;
     }
@@ -46,7 +56,7 @@ struct PlanConv {
     std::string name;
     ConvProblem problem;
     size_t weight_off = 0, bias_off = 0;       // original layouts
-    size_t packed_off = 0;                     // matrix path only
+    size_t packed_off = 0;                     // matrix path and depth-wise
     size_t ws_off = 0, ws_floats = 0;          // split-K only
     size_t ctr_off = 0, ctr_count = 0;         // split-K ticket counters (32-bit words at float offsets), zeroed at session setup
     ConvLaunch launch;
@@ -101,6 +111,9 @@ struct Plan {
     // Leading stages of one group that may run on a part of the batch at a time, while the images behind it are still on their
     // way to the device (0: the input is too small for that); their tensors share no memory with each other.
     int prefix_stages = 0;
+    size_t landing_off = 0;   // where the images of a plan with a prefix land, in the host's layout
+    // place for the result in the host's layout where it is too large for the pass to deliver it (else 0 floats)
+    size_t result_off = 0, result_floats = 0;
 };
 
 enum class PlanMode { Graph, Block, Stage };

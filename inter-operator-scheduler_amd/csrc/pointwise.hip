@@ -23,6 +23,9 @@ static int blocks_for(long long n, int per_block, int cap) {
 }
 
 // ---- argument builders (shared with the fused stage kernel) ---------------------------------------------------------
+// Channels per thread: four where the device is full with a quarter of the threads (64 threads per compute unit), else one.
+static int channels_per_thread(long long pixels, int C) { return pixels * ((C + 3) / 4) >= (1LL << 14) && C > 2 ? 4 : 1; }
+
 PoolArgs make_pool_args(const PoolProblem &p, const TensorView &x, const TensorView &y, bool global, int *blocks, const float *bias, int act) {
     if (x.C != p.C || x.H != p.H || x.W != p.W || y.C != p.C || y.H != p.OH || y.W != p.OW)
         throw std::runtime_error("pool: tensor views do not match the problem");
@@ -32,51 +35,34 @@ PoolArgs make_pool_args(const PoolProblem &p, const TensorView &x, const TensorV
     PoolArgs a;
     a.x = x.ptr;
     a.y = y.ptr;
-    a.x_bs = x.bstride;
-    a.y_bs = y.bstride;
+    a.x_ps = x.pstride;
+    a.y_ps = y.pstride;
     a.p = p;
     a.strip_rows = 0;
-    a.vec_columns = 1;
     a.bias = bias;
     a.act = act;
+    const long long pixels = (long long)p.B * p.OH * p.OW;
+    a.channels = channels_per_thread(pixels, p.C);
+    int lines = p.OH;
     if (global) {
-        // from 2^14 planes on (a lane per plane still gives every compute unit a wavefront) the row form, else a wavefront per plane
-        const long long planes = (long long)p.B * p.C;
-        if (planes >= (1LL << 14) && p.H * p.W <= 1024) {
-            a.strip_rows = 1;
-            *blocks = blocks_for(planes, 256, 4096);
-        } else {
-            *blocks = blocks_for(planes, 4, 4096);
-        }
-    } else if (p.KH == 3 && p.KW == 3 && (p.sh == 1 || p.sh == 2)) {
-        // one thread per strip of output rows; the longest strip that still leaves a million threads
-        int rows = kPoolStripRows;
-        while (rows > 1 && (long long)p.B * p.C * ((p.OH + rows - 1) / rows) * p.OW < (1LL << 20)) rows >>= 1;
-        a.strip_rows = rows;
-        long long threads = (long long)p.B * p.C * ((p.OH + rows - 1) / rows) * p.OW;
-        // larger tensors: four output columns per thread (16-byte loads and stores) while that leaves 65536 threads
-        if ((p.sw == 1 || p.sw == 2) && p.pw <= 1 && p.W >= 8) {
-            const long long kVecMinThreads = 1LL << 16;   // measured: 2^16 beats the one-column form from 64x147x147 at batch 1 on, 2^14 loses
-            auto quads = [&](int r) { return (long long)p.B * p.C * ((p.OH + r - 1) / r) * ((p.OW + kPoolVecColumns - 1) / kPoolVecColumns); };
-            // Tensors that give half a million threads even with the shortest strips (batch 16 and more) are bound by how many
-            // loads the device has in flight, not by the rows neighbouring strips read twice: one output row per thread for
-            // stride 2, two for stride 1 (batch 64, launched back to back: 64x147x147 stride 2 101.9 -> 89.7 us = 4.9 TB/s,
-            // 192x71x71 87.5 -> 77.3, 288x35x35 26.8 -> 22.3, 768x17x17 17.8 -> 15.9; stride 1 on 32x35x35 9.2 -> 7.5,
-            // 192x17x17 10.8 -> 9.7 us; longer strips there are 5-15 % slower, one column per thread 30-60 %)
-            const long long kShortStripThreads = 1LL << 19;
-            int vrows = kPoolStripRows;
-            if (quads(1) >= kShortStripThreads) vrows = p.sh == 2 ? 1 : 2;
-            while (vrows > 1 && quads(vrows) < kVecMinThreads) vrows >>= 1;
-            if (quads(vrows) >= kVecMinThreads) {
-                a.vec_columns = kPoolVecColumns;
-                a.strip_rows = vrows;
-                threads = quads(vrows);
-            }
-        }
-        *blocks = blocks_for(threads, 256, 16384);
+        *blocks = blocks_for((long long)p.B * ((p.C + kGlobalPoolChannels - 1) / kGlobalPoolChannels), 4, 8192);
     } else {
-        *blocks = blocks_for((long long)p.B * p.C * p.OH * p.OW, 256, 8192);
+        const int cv = (p.C + a.channels - 1) / a.channels;
+        long long threads = pixels * cv;
+        if (p.KH == 3 && p.KW == 3 && (p.sh == 1 || p.sh == 2)) {
+            // one thread per strip of output rows; the longest strip that still leaves half a million threads
+            int rows = p.sh == 1 ? kPoolStripRows : 2;
+            auto strips = [&](int r) { return (long long)p.B * ((p.OH + r - 1) / r) * p.OW * cv; };
+            while (rows > 1 && strips(rows) < (1LL << 19)) rows >>= 1;
+            a.strip_rows = rows;
+            threads = strips(rows);
+            lines = (p.OH + rows - 1) / rows;
+        }
+        *blocks = blocks_for(threads, 256, 1 << 16);
     }
+    a.div_cv = make_fast_div((unsigned)((p.C + a.channels - 1) / a.channels));
+    a.div_ow = make_fast_div((unsigned)p.OW);
+    a.div_strips = make_fast_div((unsigned)lines);
     return a;
 }
 
@@ -90,24 +76,27 @@ DirectConvArgs make_direct_conv_args(const ConvProblem &p, const TensorView &x, 
     a.w = w;
     a.bias = bias;
     a.y = y.ptr;
-    a.x_bs = x.bstride;
-    a.y_bs = y.bstride;
+    a.x_ps = x.pstride;
+    a.y_ps = y.pstride;
     a.p = p;
-    const unsigned long long x_bytes = ((unsigned long long)(p.B - 1) * x.bstride + (unsigned long long)p.IC * p.H * p.W) * 4ull;
+    const unsigned long long x_bytes = conv_input_extent(p, x.pstride);
     a.x_bytes = x_bytes < (1ull << 31) ? (unsigned)x_bytes : 0u;
     a.nmore = 0;
     for (int s = 0; s < kMaxNaryInputs - 1; s++) {
         a.more[s] = x.ptr;
-        a.more_bs[s] = x.bstride;
+        a.more_ps[s] = x.pstride;
         a.more_bytes[s] = 0;
     }
-    *blocks = blocks_for((long long)p.B * p.OC * p.OH * p.OW, 256, 8192);
-    a.thin = 0;
+    const long long pixels = (long long)p.B * p.OH * p.OW;
+    a.channels = p.is_depthwise() ? channels_per_thread(pixels, p.OC) : 1;
+    a.div_cv = make_fast_div((unsigned)((p.OC + a.channels - 1) / a.channels));
+    a.div_ow = make_fast_div((unsigned)p.OW);
+    a.div_oh = make_fast_div((unsigned)p.OH);
+    *blocks = blocks_for(pixels * ((p.OC + a.channels - 1) / a.channels), 256, 8192);
     if (thin) {
         if (!conv_thin_applies(p)) throw std::runtime_error("conv: the thin-input kernel serves 3 x 3 convolutions of 3-channel inputs");
-        a.thin = 1;
         // one block per 256 pixels and 32 output channels (sized for 256-thread blocks like the other bodies)
-        const long long units = (((long long)p.B * p.OH * p.OW + 255) / 256) * ((p.OC + kThinConvChannels - 1) / kThinConvChannels);
+        const long long units = ((pixels + 255) / 256) * ((p.OC + kThinConvChannels - 1) / kThinConvChannels);
         *blocks = (int)std::min<long long>(units, 1 << 20);
     }
     return a;
@@ -115,36 +104,43 @@ DirectConvArgs make_direct_conv_args(const ConvProblem &p, const TensorView &x, 
 
 bool dwconv_sums_inputs(const ConvProblem &p) { return p.is_depthwise() && p.KH == p.KW && (p.KH == 3 || p.KH == 5); }
 
-void add_dwconv_sources(DirectConvArgs &a, const TensorView *more, int count) {
+void add_dwconv_sources(DirectConvArgs &a, const TensorView *more, int count, int *blocks) {
     if (count < 0 || count > kMaxNaryInputs - 1) throw std::runtime_error("dwconv: too many summed inputs");
     const ConvProblem &p = a.p;
-    if (count > 0 && !dwconv_sums_inputs(p)) throw std::runtime_error("dwconv: this window does not add inputs in its loader");
+    if (count == 0) return;
+    if (!dwconv_sums_inputs(p)) throw std::runtime_error("dwconv: this window does not add inputs in its loader");
     for (int s = 0; s < count; s++) {
         if (more[s].C != p.IC || more[s].H != p.H || more[s].W != p.W) throw std::runtime_error("dwconv: summed inputs of different shapes");
-        const unsigned long long bytes = ((unsigned long long)(p.B - 1) * more[s].bstride + (unsigned long long)p.IC * p.H * p.W) * 4ull;
+        const unsigned long long bytes = conv_input_extent(p, more[s].pstride);
         if (bytes >= (1ull << 31) || a.x_bytes == 0) throw std::runtime_error("dwconv: summed inputs beyond 31-bit offsets");
         a.more[s] = more[s].ptr;
-        a.more_bs[s] = more[s].bstride;
+        a.more_ps[s] = more[s].pstride;
         a.more_bytes[s] = (unsigned)bytes;
     }
     a.nmore = count;
+    // the summing form holds whole windows of several inputs in registers: two channels per thread at most, for 3 x 3 windows
+    a.channels = a.channels == 4 && p.KH == 3 ? 2 : 1;
+    const int cv = (p.OC + a.channels - 1) / a.channels;
+    a.div_cv = make_fast_div((unsigned)cv);
+    *blocks = blocks_for((long long)p.B * p.OH * p.OW * cv, 256, 8192);
 }
 
-static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
-NaryKernelArgs make_nary_args(const NaryArgs &in, int multiply, int accumulate, int act, int B, long long chw,
-                              const TensorView &y, int *blocks) {
+NaryKernelArgs make_nary_args(const NaryArgs &in, int multiply, int accumulate, int act, int B, const TensorView &y, int *blocks) {
     if (in.count < 1 || in.count > kMaxNaryInputs) throw std::runtime_error("nary: bad input count");
-    bool vec = (chw % 4 == 0) && (y.bstride % 4 == 0) && aligned16(y.ptr);
-    for (int j = 0; j < in.count; j++) vec = vec && (in.src_bstride[j] % 4 == 0) && aligned16(in.src[j]);
-    if ((long long)B * chw >= (1LL << 31)) throw std::runtime_error("nary: tensor too large for 32-bit indexing");
+    const long long pixels = (long long)B * y.H * y.W;
+    if (pixels * y.C >= (1LL << 31)) throw std::runtime_error("nary: tensor too large for 32-bit indexing");
     NaryKernelArgs a;
     a.in = in;
     a.y = y.ptr;
-    a.y_bs = y.bstride;
-    a.chw = chw;
-    a.vec = vec ? 4 : 1;
-    a.total = (long long)B * chw / a.vec;
+    a.y_ps = y.pstride;
+    bool dense = y.pstride == y.C;
+    for (int j = 0; j < in.count; j++) dense = dense && in.src_pstride[j] == y.C;
+    const long long rows = dense ? 1 : pixels, length = dense ? pixels * y.C : y.C;
+    a.vec = length >= 4 && rows * ((length + 3) / 4) >= (1LL << 14) ? 4 : 1;
+    a.C = (int)length;
+    a.row = (unsigned)((length + a.vec - 1) / a.vec);
+    a.total = (unsigned)(rows * a.row);
+    a.div_row = make_fast_div(a.row);
     a.multiply = multiply;
     a.accumulate = accumulate;
     a.act = act;
@@ -170,7 +166,7 @@ void launch_dwconv(const ConvProblem &p, const TensorView &x, const float *w, co
     if (!p.is_depthwise()) throw std::runtime_error("dwconv: not a depth-wise problem");
     int blocks;
     DirectConvArgs a = make_direct_conv_args(p, x, w, bias, y, &blocks);
-    add_dwconv_sources(a, more, nmore);
+    add_dwconv_sources(a, more, nmore, &blocks);
     hipLaunchKernelGGL(dwconv_kernel, dim3(blocks), dim3(256), 0, stream, a);
 }
 
@@ -182,10 +178,9 @@ void launch_conv_direct(const ConvProblem &p, const TensorView &x, const float *
     else hipLaunchKernelGGL(conv_direct_kernel, dim3(blocks), dim3(256), 0, stream, a);
 }
 
-void launch_nary(const NaryArgs &in, int multiply, int accumulate, int act, int B, long long chw, const TensorView &y,
-                 hipStream_t stream) {
+void launch_nary(const NaryArgs &in, int multiply, int accumulate, int act, int B, const TensorView &y, hipStream_t stream) {
     int blocks;
-    const NaryKernelArgs a = make_nary_args(in, multiply, accumulate, act, B, chw, y, &blocks);
+    const NaryKernelArgs a = make_nary_args(in, multiply, accumulate, act, B, y, &blocks);
     hipLaunchKernelGGL(nary_kernel, dim3(blocks), dim3(256), 0, stream, a);
 }
 
@@ -194,8 +189,104 @@ void launch_unary(const TensorView &x, const TensorView &y, int act, int B, hipS
     NaryArgs a;
     a.count = 1;
     a.src[0] = x.ptr;
-    a.src_bstride[0] = x.bstride;
-    launch_nary(a, 0, 0, act, B, (long long)x.C * x.H * x.W, y, stream);
+    a.src_pstride[0] = x.pstride;
+    launch_nary(a, 0, 0, act, B, y, stream);
+}
+
+// ---- depth-wise filters -------------------------------------------------------------------------------------------------
+__global__ void pack_depthwise_kernel(const float *w, float *packed, int C, int padded, int taps) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < taps * padded; i += gridDim.x * blockDim.x) {
+        const int tap = i / padded, c = i - tap * padded;
+        packed[i] = c < C ? w[c * taps + tap] : 0.f;
+    }
+}
+
+void launch_pack_depthwise(const ConvProblem &p, const float *w, float *packed, hipStream_t stream) {
+    const int padded = (p.OC + 3) & ~3, taps = p.KH * p.KW;
+    hipLaunchKernelGGL(pack_depthwise_kernel, dim3(blocks_for((long long)padded * taps, 256, 1024)), dim3(256), 0, stream, w, packed, p.OC, padded, taps);
+}
+
+// ---- between the host's layout and views ---------------------------------------------------------------------------------
+// Bound by bytes (or by the link, where `nchw` lies in host memory).  Few channels (images): a thread takes a pixel, reads its
+// channels from their planes, consecutive threads consecutive pixels, and writes one pixel.  Otherwise a block turns a
+// tile of 32 channels x 64 pixels through LDS.
+template <bool TO_VIEW>
+__global__ __launch_bounds__(256) void layout_kernel(float *nchw, float *view, int B, int C, int HW, long long plane, int ps) {
+    if (C <= 4) {
+        const long long total = (long long)B * HW;
+        for (long long i = blockIdx.x * 256LL + threadIdx.x; i < total; i += gridDim.x * 256LL) {
+            const long long b = i / HW, r = i - b * HW;
+            float *first = nchw + b * C * plane + r, *pixel = view + i * ps;
+            if (TO_VIEW) {
+                float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (c < C) v[c] = first[c * plane];
+                if (ps == 4) {
+                    const pw_floatx4 q = {v[0], v[1], v[2], v[3]};
+                    *reinterpret_cast<pw_floatx4_u *>(pixel) = q;
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        if (c < C) pixel[c] = v[c];
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (c < C) first[c * plane] = pixel[c];
+            }
+        }
+        return;
+    }
+    // (64 pixels: 256 bytes of a plane at a time, which the link carries at 45 GB/s where pieces of 128 bytes at odd places come
+    // to 26)
+    __shared__ float tile[32][65];
+    const int tiles_c = (C + 31) / 32, tiles_p = (HW + 63) / 64;
+    const long long tiles = (long long)B * tiles_c * tiles_p;
+    const int px = threadIdx.x & 63, c4 = threadIdx.x >> 6;    // of the host's layout: pixel, channel of four
+    const int cx = threadIdx.x & 31, p8 = threadIdx.x >> 5;    // of the view: channel, pixel of eight
+    for (long long t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const long long bt = t / tiles_p;
+        const int p0 = (int)(t - bt * tiles_p) * 64;
+        const int b = (int)(bt / tiles_c), c0 = (int)(bt - (long long)b * tiles_c) * 32;
+        float *planes = nchw + ((long long)b * C + c0) * plane + p0, *pixels = view + ((long long)b * HW + p0) * ps + c0;
+        __syncthreads();
+        if (TO_VIEW) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = c0 + c4 + 4 * i < C && p0 + px < HW ? planes[(c4 + 4 * i) * plane + px] : 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) tile[c4 + 4 * i][px] = v[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (c0 + cx < C && p0 + p8 + 8 * i < HW) tile[cx][p8 + 8 * i] = pixels[(long long)(p8 + 8 * i) * ps + cx];
+        }
+        __syncthreads();
+        if (TO_VIEW) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (c0 + cx < C && p0 + p8 + 8 * i < HW) pixels[(long long)(p8 + 8 * i) * ps + cx] = tile[cx][p8 + 8 * i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (c0 + c4 + 4 * i < C && p0 + px < HW) planes[(c4 + 4 * i) * plane + px] = tile[c4 + 4 * i][px];
+        }
+    }
+}
+
+static int layout_blocks(int B, int C, int HW) {
+    return C <= 4 ? blocks_for((long long)B * HW, 256, 1024) : blocks_for((long long)B * ((C + 31) / 32) * ((HW + 63) / 64), 1, 2048);
+}
+
+void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t stream, long long plane) {
+    hipLaunchKernelGGL(layout_kernel<true>, dim3(layout_blocks(B, y.C, y.H * y.W)), dim3(256), 0, stream, const_cast<float *>(nchw), y.ptr, B, y.C,
+                       y.H * y.W, plane > 0 ? plane : (long long)y.H * y.W, y.pstride);
+}
+
+void launch_from_view(const TensorView &x, float *nchw, int B, hipStream_t stream) {
+    hipLaunchKernelGGL(layout_kernel<false>, dim3(layout_blocks(B, x.C, x.H * x.W)), dim3(256), 0, stream, nchw, x.ptr, B, x.C, x.H * x.W,
+                       (long long)x.H * x.W, x.pstride);
 }
 
 // ---- fills ---------------------------------------------------------------------------------------------------------

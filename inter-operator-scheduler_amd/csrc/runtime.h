@@ -39,6 +39,7 @@ public:
 
     // a process-wide arena reused by the stateless latency / inference entry points
     float *shared_arena(size_t floats);
+    float *turning_buffer(size_t floats);   // for a tensor on its way out in the host's layout
     void *shared_table(size_t bytes);   // companion buffer for the launch tables of such sessions
 
     void set_option(const std::string &key, const std::string &value);
@@ -112,6 +113,8 @@ private:
     std::string name_, arch_;
     hipStream_t streams_[kMaxGroups];
     HostStage stage_;
+    float *turning_ = nullptr;
+    size_t turning_floats_ = 0;
     float *arena_ = nullptr;
     size_t arena_floats_ = 0;
     void *table_ = nullptr;
@@ -195,6 +198,7 @@ private:
     void build_graph(size_t first);
     void drop_graph() noexcept;
     void settle();
+    void take_images(int first, int images, int chunk);
     void finish_pass();
     void advance();
     void attach();

@@ -224,10 +224,10 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
     static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
     const size_t kMaxWorkspace = size_t(96) << 20;   // floats
     TensorView x, y;
-    x.C = p.IC; x.H = p.H; x.W = p.W; x.bstride = (long long)p.IC * p.H * p.W;
-    y.C = p.OC; y.H = p.OH; y.W = p.OW; y.bstride = (long long)p.OC * p.OH * p.OW;
-    x.ptr = tuning_buffer(0, (size_t)p.B * x.bstride);
-    y.ptr = tuning_buffer(1, (size_t)p.B * y.bstride);
+    x.C = p.IC; x.H = p.H; x.W = p.W; x.pstride = padded_channels(p.IC);
+    y.C = p.OC; y.H = p.OH; y.W = p.OW; y.pstride = padded_channels(p.OC);
+    x.ptr = tuning_buffer(0, (size_t)p.B * p.H * p.W * x.pstride + 64);   // (a 16-byte load may run past the last channel)
+    y.ptr = tuning_buffer(1, (size_t)p.B * p.OH * p.OW * y.pstride);
     float *packed = tuning_buffer(2, conv_packed_floats_max(p) + p.OC);
     float *bias = packed + conv_packed_floats_max(p);
     hipStream_t stream = streams_[0];
@@ -402,6 +402,18 @@ float *DeviceContext::shared_arena(size_t floats) {
     return arena_;
 }
 
+float *DeviceContext::turning_buffer(size_t floats) {
+    if (floats > turning_floats_) {
+        IOS_HIP(hipDeviceSynchronize());
+        if (turning_ != nullptr) IOS_HIP(hipFree(turning_));
+        turning_ = nullptr;
+        turning_floats_ = 0;
+        IOS_HIP(hipMalloc(reinterpret_cast<void **>(&turning_), floats * sizeof(float)));
+        turning_floats_ = floats;
+    }
+    return turning_;
+}
+
 void *DeviceContext::shared_table(size_t bytes) {
     if (bytes > table_bytes_) {
         IOS_HIP(hipDeviceSynchronize());
@@ -525,16 +537,17 @@ void Session::release() noexcept {
 
 TensorView Session::tv(const ViewRef &v) const {
     TensorView t;
-    t.ptr = base_ + v.offset;
+    t.ptr = base_ + v.base + v.first;
     t.C = v.C;
     t.H = v.H;
     t.W = v.W;
-    t.bstride = v.bstride;
+    t.pstride = v.pstride;
     return t;
 }
 
 void Session::pack(const PlanConv &conv, hipStream_t stream) {
     if (conv.matrix_path) launch_pack_filters(conv.problem, conv.launch, base_ + conv.weight_off, base_ + conv.packed_off, stream);
+    else if (conv.problem.is_depthwise()) launch_pack_depthwise(conv.problem, base_ + conv.weight_off, base_ + conv.packed_off, stream);
     packed_[&conv - plan_.convs.data()] = 1;
 }
 
@@ -578,21 +591,33 @@ void Session::ensure_timers() {
 
 void Session::set_input(const float *host) {
     if (host == nullptr) throw std::runtime_error("input pointer is null");
-    const ViewRef &in = plan_.input;
-    const size_t image = in.image_floats() * sizeof(float), total = (size_t)plan_.batch * image;
-    if (plan_.prefix_stages > 0 && total <= HostStage::kBatch && !static_) {
+    const TensorView in = tv(plan_.input);
+    hipStream_t main = ctx_.stream(0);
+    if (plan_.prefix_stages > 0 && !static_ && plan_.batch * plan_.input.image_floats() * sizeof(float) <= HostStage::kBatch) {
         // the first stages of the next pass start on the images that are there while the others are still on their way
-        arriving_images_ = (plan_.batch + HostStage::kMaxChunks - 1) / HostStage::kMaxChunks;
+        const size_t image = plan_.input.image_floats() * sizeof(float);
+        const int chunks = plan_.batch * image < (size_t(32) << 20) ? 2 : HostStage::kMaxChunks;
+        arriving_images_ = (plan_.batch + chunks - 1) / chunks;
         arriving_ = (plan_.batch + arriving_images_ - 1) / arriving_images_;
-        ctx_.stage().upload_chunks(base_ + in.offset, host, total, (size_t)arriving_images_ * image, ctx_.stream(1), ctx_.stream(0));
+        ctx_.stage().upload_chunks(base_ + plan_.landing_off, host, plan_.batch * image, arriving_images_ * image, ctx_.stream(1), main);
         return;
     }
-    ctx_.stage().upload(base_ + in.offset, host, total, ctx_.stream(0));
+    arriving_ = 0;
+    ctx_.stage().upload_images(in, plan_.batch, host, main);
+}
+
+// images that have landed in the host's layout, the last of them with `chunk`, go to their place
+void Session::take_images(int first, int images, int chunk) {
+    hipStream_t main = ctx_.stream(0);
+    ctx_.stage().arrived(chunk, main);
+    TensorView in = tv(plan_.input);
+    in.ptr += (size_t)first * in.H * in.W * in.pstride;
+    launch_to_view(base_ + plan_.landing_off + (size_t)first * plan_.input.image_floats(), in, images, main);
 }
 
 // everything the next kernels of the main stream may read has arrived
 void Session::settle() {
-    if (arriving_ > 0) ctx_.stage().arrived(arriving_ - 1, ctx_.stream(0));
+    if (arriving_ > 0) take_images(0, plan_.batch, arriving_ - 1);
     arriving_ = 0;
 }
 
@@ -636,16 +661,19 @@ void Session::set_conv_weights(int count, char **names, float **weights, float *
     });
 }
 
+// Dense copy of a view in the host's layout.
 void Session::copy_out(const ViewRef &view, float *host) {
     settle();
     hipStream_t main = ctx_.stream(0);
-    const size_t image = view.image_floats();
-    if (view.bstride == (long long)image) {
-        ctx_.stage().download(host, base_ + view.offset, (size_t)plan_.batch * image * sizeof(float), main);
-        return;
+    const size_t floats = (size_t)plan_.batch * view.image_floats();
+    const TensorView t = tv(view);
+    const float *from = t.ptr;
+    if (view.H * view.W > 1 || t.pstride != t.C) {
+        float *turned = &view == &plan_.output && plan_.result_floats > 0 ? base_ + plan_.result_off : ctx_.turning_buffer(floats);
+        launch_from_view(t, turned, plan_.batch, main);
+        from = turned;
     }
-    for (int b = 0; b < plan_.batch; b++)
-        ctx_.stage().download(host + (size_t)b * image, base_ + view.offset + (size_t)b * view.bstride, image * sizeof(float), main);
+    ctx_.stage().download(host, from, floats * sizeof(float), main);
 }
 
 void Session::get_output(float *host) {
@@ -675,7 +703,7 @@ void Session::launch_op(const PlanOp &op, int group, int first, int images) {
     const int count = images > 0 ? images : plan_.batch;
     auto part = [&](const ViewRef &v) {   // the images this launch works on
         TensorView t = tv(v);
-        t.ptr += (long long)first * v.bstride;
+        t.ptr += (long long)first * v.H * v.W * v.pstride;
         return t;
     };
     switch (op.kind) {
@@ -696,7 +724,7 @@ void Session::launch_op(const PlanOp &op, int group, int first, int images) {
             p.B = count;
             TensorView more[kMaxNaryInputs];
             for (size_t i = 1; i < op.srcs.size(); i++) more[i - 1] = part(op.srcs[i]);
-            launch_dwconv(p, part(op.in), base_ + c.weight_off, bias_of(c), part(op.out), stream, more,
+            launch_dwconv(p, part(op.in), base_ + c.packed_off, bias_of(c), part(op.out), stream, more,
                           op.srcs.empty() ? 0 : (int)op.srcs.size() - 1);
             break;
         }
@@ -720,9 +748,9 @@ void Session::launch_op(const PlanOp &op, int group, int first, int images) {
             a.count = (int)op.srcs.size();
             for (int i = 0; i < a.count; i++) {
                 a.src[i] = part(op.srcs[i]).ptr;
-                a.src_bstride[i] = op.srcs[i].bstride;
+                a.src_pstride[i] = op.srcs[i].pstride;
             }
-            launch_nary(a, op.multiply, op.accumulate, op.act, count, (long long)op.out.image_floats(), part(op.out), stream);
+            launch_nary(a, op.multiply, op.accumulate, op.act, count, part(op.out), stream);
             break;
         }
         case OpKind::Unary: launch_unary(part(op.in), part(op.out), op.act, count, stream); break;
@@ -790,7 +818,7 @@ void Session::enqueue_prefix(size_t stages) {
         chunk = part == 0 ? (arriving_ + 1) / 2 : arriving_;
         const int images = std::min(chunk * arriving_images_, plan_.batch) - begin;
         if (images <= 0) continue;
-        ctx_.stage().arrived(chunk - 1, ctx_.stream(0));
+        take_images(begin, images, chunk - 1);
         for (size_t s = 0; s < split; s++)
             for (int op : plan_.stages[s][0]) launch_op(plan_.ops[op], 0, begin, images);
     }
@@ -895,11 +923,12 @@ void Session::build_fused() {
                         const PlanConv &c = plan_.convs[op.conv];
                         pend.item.kind = op.kind == OpKind::ConvDepthwise ? WORK_DWCONV : WORK_CONV_DIRECT;
                         if (c.thin) throw std::runtime_error("internal: the thin-input convolution kernel is planned for single-group stages only");
-                        pend.item.direct = make_direct_conv_args(c.problem, tv(op.in), base_ + c.weight_off, bias_of(c), tv(op.out), &blocks);
+                        pend.item.direct = make_direct_conv_args(c.problem, tv(op.in), base_ + (op.kind == OpKind::ConvDepthwise ? c.packed_off : c.weight_off),
+                                                                 bias_of(c), tv(op.out), &blocks);
                         if (op.kind == OpKind::ConvDepthwise && op.srcs.size() > 1) {
                             TensorView more[kMaxNaryInputs];
                             for (size_t i = 1; i < op.srcs.size(); i++) more[i - 1] = tv(op.srcs[i]);
-                            add_dwconv_sources(pend.item.direct, more, (int)op.srcs.size() - 1);
+                            add_dwconv_sources(pend.item.direct, more, (int)op.srcs.size() - 1, &blocks);
                         }
                         break;
                     }
@@ -914,18 +943,17 @@ void Session::build_fused() {
                         NaryArgs in;
                         if (op.kind == OpKind::Unary) {
                             in.count = 1;
-                            in.src[0] = base_ + op.in.offset;
-                            in.src_bstride[0] = op.in.bstride;
+                            in.src[0] = tv(op.in).ptr;
+                            in.src_pstride[0] = op.in.pstride;
                         } else {
                             in.count = (int)op.srcs.size();
                             for (int i = 0; i < in.count; i++) {
-                                in.src[i] = base_ + op.srcs[i].offset;
-                                in.src_bstride[i] = op.srcs[i].bstride;
+                                in.src[i] = tv(op.srcs[i]).ptr;
+                                in.src_pstride[i] = op.srcs[i].pstride;
                             }
                         }
                         pend.item.kind = WORK_NARY;
-                        pend.item.nary = make_nary_args(in, op.multiply, op.accumulate, op.act, plan_.batch,
-                                                        (long long)op.out.image_floats(), tv(op.out), &blocks);
+                        pend.item.nary = make_nary_args(in, op.multiply, op.accumulate, op.act, plan_.batch, tv(op.out), &blocks);
                         break;
                     }
                 }
@@ -1086,7 +1114,7 @@ void Session::finish_pass() {
     const bool deliver = plan_.output_single_group && (bytes <= kAlways || (fetches_result_ && bytes <= HostStage::kResult));
     fetches_result_ = false;
     HostStage::Result result;
-    if (deliver) result = {base_ + plan_.output.offset, plan_.batch, (long long)plan_.output.image_floats(), plan_.output.bstride};
+    if (deliver) result = {tv(plan_.output), plan_.batch};
     hipStream_t main = ctx_.stream(0);
     ctx_.stage().signal(result, main);
     ctx_.stage().wait(main);
