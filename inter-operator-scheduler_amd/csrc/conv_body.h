@@ -1435,6 +1435,4 @@ struct ConvWsplit {
     X(116, "wb_x1w_m64n64_w4", 2, 2, 4, 2)     \
     X(117, "wb_x1w_m32n32_w8", 1, 1, 8, 2)     \
     X(118, "wb_x1w_m64n64_w2", 2, 2, 2, 2)
-constexpr int kNumConvVariants = 119;
-
 }  // namespace ios

@@ -1,5 +1,5 @@
 // Stand-alone convolution kernels, the configuration table and the launchers.  Device code: conv_body.h.
-#include "conv_body.h"
+#include "conv_pipe.h"
 #include "launch_internal.h"
 
 #include <algorithm>
@@ -72,11 +72,22 @@ struct VariantEntry {
      conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>, true>,              \
      ConvWsplit<32, TM, TN, NW, 8, true, D, 4>::SMEM_FLOATS},
 
+#define IOS_PIPE_ENTRY(TERMS, HALF, PRECISION, NAME, KU, PD, TMW, TNW, WM, WN)                                                       \
+    {{NAME, ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::BM, ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::BN, 16 * KU, WM, WN, 1, 32, \
+      false, 16, false, false, PRECISION, TERMS},                                                                                     \
+     conv_kernel<ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>>, conv_kernel<ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>, true>,  \
+     ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::SMEM_FLOATS},
+#define IOS_PIPE3_ENTRY(IDX, ...) IOS_PIPE_ENTRY(3, false, PREC_FP32, __VA_ARGS__)
+#define IOS_PIPE_BF16_ENTRY(IDX, ...) IOS_PIPE_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
+#define IOS_PIPE_FP16_ENTRY(IDX, ...) IOS_PIPE_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
+
 static const VariantEntry kVariants[] = {IOS_TILED_VARIANTS(IOS_TILED_ENTRY) IOS_WSPLIT_VARIANTS(IOS_WSPLIT_ENTRY)
                                              IOS_WSPLIT_C4_VARIANTS(IOS_WSPLIT_C4_ENTRY)
                                              IOS_WSPLIT_T32_VARIANTS(IOS_WSPLIT_ENTRY) IOS_WSPLIT_F16_VARIANTS(IOS_WSPLIT_ENTRY)
                                              IOS_WSPLIT_LONGK_VARIANTS(IOS_WSPLIT_ENTRY) IOS_SPLIT3_VARIANTS(IOS_SPLIT3_ENTRY) IOS_WSPLIT_X3_VARIANTS(IOS_WSPLIT_X3_ENTRY)
-                                             IOS_SPLIT1_VARIANTS(IOS_SPLIT1_ENTRY) IOS_WSPLIT_X1_VARIANTS(IOS_WSPLIT_X1_ENTRY)};
+                                             IOS_SPLIT1_VARIANTS(IOS_SPLIT1_ENTRY) IOS_WSPLIT_X1_VARIANTS(IOS_WSPLIT_X1_ENTRY)
+                                             IOS_PIPE3_VARIANTS(IOS_PIPE3_ENTRY) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_ENTRY)
+                                             IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_ENTRY)};
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 static_assert(kNumVariants == kNumConvVariants, "variant lists and count disagree");
 
@@ -359,6 +370,8 @@ __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int 
                 out[at] = (unsigned short)(hi >> 16);
                 out[at + (size_t)OCgP * 8] = (unsigned short)(mid >> 16);
                 out[at + (size_t)OCgP * 16] = (unsigned short)(lo >> 16);
+            } else if (precision == PREC_FP16) {
+                reinterpret_cast<_Float16 *>(packed)[at] = (_Float16)value;   // round to nearest even
             } else {
                 reinterpret_cast<__bf16 *>(packed)[at] = (__bf16)value;   // round to nearest even
             }

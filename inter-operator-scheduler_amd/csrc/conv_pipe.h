@@ -1,0 +1,254 @@
+// LDS-tiled convolution for large batches with both operands staged in LDS: ConvPipe.
+//
+// The GEMM view, K order and tails are those of conv_body.h; the operands are the sixteen-bit ones of ConvSplit3: three exact
+// bfloat16 terms of an fp32 value (TERMS = 3, fp32 accuracy) or one rounded term, bfloat16 or IEEE half (TERMS = 1, the
+// reduced-precision modes), on v_mfma_f32_32x32x16.  ConvSplit3 reads its filters from global memory, once per wavefront: at 32 x 64
+// outputs per wavefront the L1 delivers 64 bytes per cycle and compute unit for them alone, its limit.  Here a block reads its
+// filter tile once, and a wavefront computes up to 64 x 64 or 96 x 64 outputs per operand read (24 or 36 matrix instructions of 32
+// cycles for 12 or 15 LDS reads of 8).
+//
+// A stage holds KU units of 16 k (a unit lies inside one filter tap).  One stage is two or more matrix times ahead in
+// registers, the next one in LDS; one barrier per stage.  What a stage has to cover is the latency of its loads: with three terms
+// the matrix work of one unit does (768 cycles per wavefront), with one term it takes four units (a one-unit stage is gone in 128).
+#pragma once
+
+#include "conv_body.h"
+
+namespace ios {
+
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+
+template <int TERMS, bool HALF, int KU, int PD, int TMW, int TNW, int WM, int WN>
+struct ConvPipe {
+    static_assert(TERMS == 3 || TERMS == 1, "three exact terms or one rounded term");
+    static_assert(!HALF || TERMS == 1, "half operands are rounded");
+    static constexpr int MT = 32;
+    using M = Mfma<32>;
+    static constexpr int BM = 32 * TMW * WM, BN = 32 * TNW * WN, BK = 16 * KU;
+    static constexpr int T = 64 * WM * WN;
+    static constexpr int THREADS = T;
+    static constexpr int CPAD = 16;
+    static constexpr bool FUSABLE = false;
+    static constexpr int OCT = 2 * KU;                 // octets (eight consecutive k) of a pixel or filter row in a stage
+    static constexpr int B_IT = OCT * BN / T;          // pixels a thread stages, T / OCT apart
+    static constexpr int A_SLOTS = OCT * TERMS * BM;   // slots of 16 bytes (eight 16-bit values)
+    static constexpr int A_IT = (A_SLOTS + T - 1) / T;
+    // inputs of one unit and plane: two slots per pixel; units are two slots out of step, so that the octets of a pixel, which
+    // neighbouring lanes store, fall into different banks
+    static constexpr int UNIT = 2 * BN + (KU > 1 ? 2 : 0);
+    static constexpr int STAGE = A_SLOTS + KU * TERMS * UNIT;
+    static constexpr int SMEM_FLOATS = 2 * STAGE * 4;
+    static_assert(OCT * BN % T == 0 && T % OCT == 0, "input loader shape");
+
+    template <bool RES = false>
+    __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
+    constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
+    uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave % WN;
+    const int wm = wave / WN;
+    const int lk = lane >> 5;
+    const int lc = lane & 31;
+    int tm, tn;
+    xcd_tile(a, tile, tm, tn);
+    const int m0 = tm * BM;
+    const int n0 = tn * BN;
+    const int k_begin = z * a.k_chunk;
+    const int k_end = min(a.Kq, k_begin + a.k_chunk);
+    const int stages = (k_end - k_begin + BK - 1) / BK;
+
+    const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
+    const __amdgpu_buffer_rsrc_t wr = buffer_of(a.wp, a.w_bytes);
+    // ---- filters: packed [g][k / 8][plane][OCgP] slots; slot s of a stage is (octet, plane, row) = (s / BM / TERMS, s / BM % TERMS, s % BM)
+    unsigned a_off[A_IT];
+    int a_oct[A_IT];
+#pragma unroll
+    for (int i = 0; i < A_IT; i++) {
+        const int s = tid + i * T;
+        const int row = s % BM, op = s / BM, m = m0 + row;
+        a_oct[i] = op / TERMS;
+        const bool ok = (A_SLOTS % T == 0 || s < A_SLOTS) && m < a.OCgP;
+        a_off[i] = ok ? (((unsigned)g * ((unsigned)a.Kq >> 3) * TERMS + (unsigned)op) * (unsigned)a.OCgP + (unsigned)m) * 16u : kOutOfRange;
+    }
+    // ---- inputs: this thread's octet and pixels; the octets of a pixel go to neighbouring threads
+    const int oct = tid % OCT;
+    const int unit = KU == 1 ? 0 : oct >> 1;
+    const int half = oct & 1;
+    int ih0[B_IT], iw0[B_IT];
+    unsigned x_off[B_IT], n_kill[B_IT];
+#pragma unroll
+    for (int i = 0; i < B_IT; i++) {
+        const int n = n0 + tid / OCT + i * (T / OCT);
+        n_kill[i] = n < a.Npix ? 0u : kOutOfRange;
+        const int nn = n < a.Npix ? n : 0;
+        const int b = (int)fast_div((unsigned)nn, a.div_ohw);
+        const int r = nn - b * a.OHW;
+        const int oh = (int)fast_div((unsigned)r, a.div_ow);
+        const int ow = r - oh * a.OW;
+        ih0[i] = oh * a.sh - a.ph;
+        iw0[i] = ow * a.sw - a.pw;
+        x_off[i] = (((unsigned)(b * a.H + ih0[i]) * (unsigned)a.W + (unsigned)iw0[i]) * (unsigned)a.x_ps + (unsigned)(g * a.ICg + 8 * half)) * 4u;
+    }
+    auto slot_of = [](int pixel, int octet) { return 2 * pixel + (octet ^ ((pixel >> 2) & 1)); };
+
+    uintx4 a_reg[PD][A_IT];
+    floatx4 b_reg[PD][B_IT][2];
+    int b_left[PD];
+    auto load_stage = [&](int st, uintx4 (&ar)[A_IT], floatx4 (&br)[B_IT][2], int &left) {
+        const int k0 = k_begin + st * BK;
+        const unsigned w_stage = (unsigned)((k0 >> 3) * TERMS) * (unsigned)a.OCgP * 16u;
+#pragma unroll
+        for (int i = 0; i < A_IT; i++) {
+            const unsigned kill = k0 + 8 * a_oct[i] < k_end ? 0u : kOutOfRange;   // beyond the K range: zeros
+            ar[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, (a_off[i] + w_stage) | kill, 0, 0);
+        }
+        const int k = k0 + 16 * unit;
+        const int tap = (int)__umulhi((unsigned)k, a.magic_icgp);
+        const int c0 = k - tap * a.ICgP;
+        const int kh = a.KW == 1 ? tap : (int)__umulhi((unsigned)tap, a.magic_kw);
+        const int kw = tap - kh * a.KW;
+        const unsigned dead = k < k_end ? 0u : kOutOfRange;
+        const unsigned x_unit = (unsigned)((kh * a.W + kw) * a.x_ps + c0) * 4u;
+        const int c_left = a.ICg - c0 - 8 * half;   // real channels from this octet on
+        const unsigned pad0 = (unsigned)(c_left - 1) & kOutOfRange, pad1 = (unsigned)(c_left - 5) & kOutOfRange;   // sign bits
+#pragma unroll
+        for (int i = 0; i < B_IT; i++) {
+            const unsigned in_h = (unsigned)(ih0[i] + kh) < (unsigned)a.H ? 1u : 0u;
+            const unsigned in_w = (unsigned)(iw0[i] + kw) < (unsigned)a.W ? 1u : 0u;
+            const unsigned at = (x_off[i] + x_unit) | (((in_h & in_w) ^ 1u) << 31) | n_kill[i] | dead;
+            br[i][0] = buffer_load_f32x4(xr, at | pad0);
+            br[i][1] = buffer_load_f32x4(xr, at | pad1, 16u);
+        }
+        left = c_left;
+    };
+    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const bool ragged = (a.ICg & 3) != 0;
+    auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
+        uintx4 *As = lds + buf * STAGE;
+        uintx4 *Bs = As + A_SLOTS + unit * (TERMS * UNIT);
+#pragma unroll
+        for (int i = 0; i < A_IT; i++)
+            if (A_SLOTS % T == 0 || tid + i * T < A_SLOTS) As[tid + i * T] = ar[i];
+#pragma unroll
+        for (int i = 0; i < B_IT; i++) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(br[i][j >> 2][j & 3]), relu_floor));   // folded ReLU of the producer
+            if (ragged)
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = j < left ? v[j] : 0.f;
+            const int slot = slot_of(tid / OCT + i * (T / OCT), half);
+            if constexpr (TERMS == 3) {
+                uintx4 hi, mid, lo;
+                split_bf16x3(v, hi, mid, lo);
+                Bs[slot] = hi;
+                Bs[UNIT + slot] = mid;
+                Bs[2 * UNIT + slot] = lo;
+            } else if constexpr (HALF) {
+                const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+                Bs[slot] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));   // round to nearest even, overflow to infinity
+            } else {
+                Bs[slot] = round_bf16x8(v);
+            }
+        }
+    };
+
+    typename M::acc_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
+
+    // Register set s holds stage st with st % PD == s.  Iteration st: the matrix work of stage st from LDS buffer st & 1, the
+    // registers of stage st + 1 into the other buffer, stage st + 1 + PD requested into the same registers.  The loop runs in
+    // rounds of PD stages with a straight-line body; stages past the end are loaded as zeros.
+#pragma unroll
+    for (int s = 0; s < PD; s++) load_stage(s, a_reg[s], b_reg[s], b_left[s]);
+    store_stage(0, a_reg[0], b_reg[0], b_left[0]);
+    load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
+    __syncthreads();
+    for (int st0 = 0; st0 < stages; st0 += PD) {
+#pragma unroll
+        for (int s = 0; s < PD; s++) {
+            const int st = st0 + s;
+            const int buf = st & 1;
+            const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
+            const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
+#pragma unroll
+            for (int u = 0; u < KU; u++) {
+                uintx4 av[TERMS][TM], bv[TERMS][TN];
+#pragma unroll
+                for (int p = 0; p < TERMS; p++) {
+#pragma unroll
+                    for (int i = 0; i < TM; i++) av[p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
+#pragma unroll
+                    for (int j = 0; j < TN; j++) bv[p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
+                }
+                // all LDS reads of the unit are requested before its first matrix instruction
+                if (TERMS == 3) __builtin_amdgcn_sched_barrier(0);
+                // the six terms, smallest first; the tiles of a term are independent instructions
+                constexpr int NT = TERMS == 3 ? 6 : 1;
+                constexpr int TA[6] = {TERMS == 3 ? 2 : 0, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++) {
+                            if constexpr (HALF)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, av[TA[t]][i]),
+                                                                                   __builtin_bit_cast(halfx8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
+                            else
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[TA[t]][i]),
+                                                                                    __builtin_bit_cast(bf16x8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
+                        }
+            }
+            store_stage(buf ^ 1, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+            load_stage(st + 1 + PD, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+            __syncthreads();
+        }
+    }
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0);
+    }   // run
+};
+
+// X(index, name, KU, PD, TMW, TNW, WM, WN): three exact terms
+#define IOS_PIPE3_VARIANTS(X)                          \
+    X(119, "x3p_m128n128_w2x2", 1, 2, 2, 2, 2, 2)      \
+    X(120, "x3p_m192n128_w2x2", 1, 2, 3, 2, 2, 2)      \
+    X(121, "x3p_m64n256_w1x4", 1, 2, 2, 2, 1, 4)       \
+    X(122, "x3p_m64n128_w1x2", 1, 2, 2, 2, 1, 2)       \
+    X(123, "x3p_m96n128_w1x4", 1, 2, 3, 1, 1, 4)       \
+    X(124, "x3p_m96n128_w1x2", 1, 2, 3, 2, 1, 2)       \
+    X(125, "x3p_m32n256_w1x4", 1, 2, 1, 2, 1, 4)       \
+    X(126, "x3p_m64n128_w1x4", 1, 2, 2, 1, 1, 4)       \
+    X(127, "x3p_m128n64_w2x2", 2, 1, 2, 1, 2, 2)       \
+    X(128, "x3p_m64n64_w2x2", 2, 1, 1, 1, 2, 2)        \
+    X(129, "x3p_m128n128_w2x2_k32", 2, 1, 2, 2, 2, 2)
+// one rounded term, bfloat16 (option precision=bf16)
+#define IOS_PIPE_BF16_VARIANTS(X)                      \
+    X(130, "wb_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
+    X(131, "wb_p_m192n128_w2x2", 4, 1, 3, 2, 2, 2)     \
+    X(132, "wb_p_m64n256_w1x4", 2, 1, 2, 2, 1, 4)      \
+    X(133, "wb_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
+    X(134, "wb_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
+    X(135, "wb_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
+    X(136, "wb_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
+    X(137, "wb_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)       \
+    X(138, "wb_p_m192n64_w2x2", 4, 1, 3, 1, 2, 2)
+// one rounded term, IEEE half (option precision=fp16)
+#define IOS_PIPE_FP16_VARIANTS(X)                      \
+    X(139, "wh_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
+    X(140, "wh_p_m192n128_w2x2", 4, 1, 3, 2, 2, 2)     \
+    X(141, "wh_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
+    X(142, "wh_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
+    X(143, "wh_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
+    X(144, "wh_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
+    X(145, "wh_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
+constexpr int kNumConvVariants = 146;
+
+}  // namespace ios
