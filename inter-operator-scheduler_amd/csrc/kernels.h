@@ -205,5 +205,6 @@ void launch_from_view(const TensorView &x, float *nchw, int B, hipStream_t strea
 // Fill n floats with a deterministic pattern in [-1, 1) (seeded), or with a constant.
 void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream);
 void launch_fill_u32(unsigned *dst, size_t n, unsigned value, hipStream_t stream);
+void launch_delay(int steps, hipStream_t stream);   // keeps the stream waiting about 4 us per step
 
 }  // namespace ios

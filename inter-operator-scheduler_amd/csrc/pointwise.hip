@@ -316,4 +316,11 @@ void launch_fill_u32(unsigned *dst, size_t n, unsigned value, hipStream_t stream
     hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for((long long)n, 256, 65535)), dim3(256), 0, stream, dst, n, value);
 }
 
+// One wavefront that sleeps for about 4 us per step (8128 clocks at 2.1 to 2.4 GHz).
+__global__ void delay_kernel(int steps) {
+    for (int i = 0; i < steps; i++) __builtin_amdgcn_s_sleep(127);
+}
+
+void launch_delay(int steps, hipStream_t stream) { hipLaunchKernelGGL(delay_kernel, dim3(1), dim3(64), 0, stream, steps); }
+
 }  // namespace ios

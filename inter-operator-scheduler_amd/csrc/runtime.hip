@@ -254,9 +254,13 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         const size_t ws = conv_workspace_floats(p, l);
         float *workspace = ws ? tuning_buffer(3, ws) : nullptr;
         const SplitKReduce counters = split_reduce(tuning_counters(conv_counter_count(p, l)));
-        launch_conv_mfma(p, l, x, packed, bias, y, workspace, counters, stream);   // warm-up
+        auto issue = [&] { launch_conv_mfma(p, l, x, packed, bias, y, workspace, counters, stream); };
+        issue();   // warm-up
+        // A launch costs the host 3 to 5 us, more than most kernels of a batch-1 network run: the device waits until all of
+        // them are queued, so that the events time the kernels and not the host.
+        launch_delay(reps + 3, stream);
         IOS_HIP(hipEventRecord(start, stream));
-        for (int r = 0; r < reps; r++) launch_conv_mfma(p, l, x, packed, bias, y, workspace, counters, stream);
+        for (int r = 0; r < reps; r++) issue();
         IOS_HIP(hipEventRecord(stop, stream));
         IOS_HIP(hipEventSynchronize(stop));
         float ms = 0.f;
