@@ -52,7 +52,7 @@ class HostStage {
 public:
     static constexpr size_t kPart = size_t(4) << 20;      // bytes per staging buffer of the ring, and per step of a large transfer
     static constexpr int kParts = 4;
-    static constexpr int kMaxChunks = 4;                  // steps in which a batch arrives (the copy engine takes 25-35 us from one to the next)
+    static constexpr int kMaxChunks = 5;                  // steps in which a batch arrives (the copy engine takes 25-35 us from one to the next)
     static constexpr size_t kBatch = size_t(256) << 20;   // largest transfer that is staged as a whole (or one image)
     static constexpr size_t kChunk = size_t(64) << 10;   // bytes of the result that are announced together
     static constexpr size_t kAlone = 3 * kChunk;          // results up to this size are fetched by one thread
@@ -65,10 +65,10 @@ public:
     void upload(void *dst, const void *src, size_t bytes, hipStream_t stream);
     // The same for a batch of images in the host's layout, which kernels read from the staging buffer and write as a view.
     void upload_images(const TensorView &dst, int batch, const float *src, hipStream_t stream);
-    // A batch of `total` <= kBatch bytes to device memory as it is, in chunks of `bytes` bytes (the last may be shorter), by the
+    // A batch of at most kBatch bytes to device memory as it is, in up to kMaxChunks chunks that end at `ends` (bytes), by the
     // copy engine and on the stream `link`, which waits for what `stream` holds: chunk c has arrived for a stream that called
     // arrived(c, stream).  (Kernels that read host memory would share the device with those of `stream`.)
-    void upload_chunks(void *dst, const void *src, size_t total, size_t bytes, hipStream_t link, hipStream_t stream);
+    void upload_chunks(void *dst, const void *src, const std::vector<size_t> &ends, hipStream_t link, hipStream_t stream);
     void arrived(int chunk, hipStream_t stream);
     // Scattered sources that lie next to each other on the device: `pieces` ascending by `to`, an offset from `dst`, without
     // overlap, gaps of less than a cache line's worth of padding that may be overwritten.  `step` is called by the calling thread

@@ -304,30 +304,33 @@ void HostStage::upload_images(const TensorView &dst, int batch, const float *src
     }
 }
 
-void HostStage::upload_chunks(void *dst, const void *src, size_t total, size_t bytes, hipStream_t link, hipStream_t stream) {
-    char *memory = inputs_.take(total);
+void HostStage::upload_chunks(void *dst, const void *src, const std::vector<size_t> &ends, hipStream_t link, hipStream_t stream) {
+    const int chunks = (int)ends.size();
+    if (chunks < 1 || chunks > kMaxChunks) throw std::runtime_error("internal: a batch arrives in too many chunks");
+    char *memory = inputs_.take(ends.back());
     IOS_HIP(hipEventRecord(order_, stream));
     IOS_HIP(hipStreamWaitEvent(link, order_, 0));
     // one shared-out copy of the whole batch; the calling thread hands a chunk to the link as soon as its pieces are staged
-    const int chunks = (int)((total + bytes - 1) / bytes);
-    const int per_chunk = (int)((bytes + HostCopier::kPiece - 1) / HostCopier::kPiece);
+    auto begin_of = [&](int c) { return c == 0 ? 0 : ends[c - 1]; };
+    int first_piece[kMaxChunks + 1] = {};
+    for (int c = 0; c < chunks; c++) first_piece[c + 1] = first_piece[c] + (int)((ends[c] - begin_of(c) + HostCopier::kPiece - 1) / HostCopier::kPiece);
     std::atomic<int> staged[kMaxChunks] = {};
-    auto chunk_bytes = [&](int c) { return std::min(bytes, total - (size_t)c * bytes); };
     int sent = 0;
     hipError_t failed = hipSuccess;
     const std::function<void()> hand_over = [&]() {
-        while (sent < chunks && staged[sent].load(std::memory_order_acquire) == per_chunk) {
-            const size_t at = (size_t)sent * bytes;
-            hipError_t status = hipMemcpyAsync(static_cast<char *>(dst) + at, memory + at, chunk_bytes(sent), hipMemcpyHostToDevice, link);
+        while (sent < chunks && staged[sent].load(std::memory_order_acquire) == first_piece[sent + 1] - first_piece[sent]) {
+            const size_t at = begin_of(sent);
+            hipError_t status = hipMemcpyAsync(static_cast<char *>(dst) + at, memory + at, ends[sent] - at, hipMemcpyHostToDevice, link);
             if (status == hipSuccess) status = hipEventRecord(chunk_events_[sent], link);
             if (failed == hipSuccess) failed = status;
             sent++;
         }
     };
-    HostCopier::get().parallel(chunks * per_chunk, true, [&](int piece) {
-        const int c = piece / per_chunk;
-        const size_t at = (size_t)(piece - c * per_chunk) * HostCopier::kPiece, limit = chunk_bytes(c), from = (size_t)c * bytes + at;
-        if (at < limit) copy_past_caches(memory + from, static_cast<const char *>(src) + from, std::min(HostCopier::kPiece, limit - at));
+    HostCopier::get().parallel(first_piece[chunks], true, [&](int piece) {
+        int c = 0;
+        while (piece >= first_piece[c + 1]) c++;
+        const size_t from = begin_of(c) + (size_t)(piece - first_piece[c]) * HostCopier::kPiece;
+        copy_past_caches(memory + from, static_cast<const char *>(src) + from, std::min(HostCopier::kPiece, ends[c] - from));
         staged[c].fetch_add(1, std::memory_order_release);
     }, &hand_over);
     IOS_HIP(failed);

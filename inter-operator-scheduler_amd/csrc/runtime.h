@@ -211,7 +211,7 @@ private:
     bool owns_memory_ = false;
     bool static_ = false;
     std::vector<char> packed_;      // per convolution: its packed filters are laid out
-    int arriving_ = 0, arriving_images_ = 0;   // parts of the input on their way, images per part
+    std::vector<int> arriving_;     // parts of the input on their way: images up to the end of each
     bool advance_ = false;          // set_conv_weights issues the stages whose filters it has packed
     size_t next_stage_ = 0;
     bool fetches_result_ = true;    // the caller has fetched the last result (or there was none): the next pass delivers its own
