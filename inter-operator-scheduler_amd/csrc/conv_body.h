@@ -29,6 +29,7 @@
 
 #include "kernels.h"
 
+#include <climits>
 #include <type_traits>
 
 namespace ios {
@@ -255,8 +256,9 @@ struct Mfma<16> {
 // barriers): the split-K exchange in its three forms, then bias, activation and the store through the output view.
 template <int MT, int BM, int BN, int TM, int TN, int WM, int WN, bool RES>
 __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem, typename Mfma<MT>::acc_t (&acc)[TM][TN], int tile, int g, int z,
-                                           int m0, int n0, int wm, int wn, int wk) {
+                                           int m0, int n0, int wm, int wn, int wk, int n_limit = INT_MAX) {
     using M = Mfma<MT>;
+    const int n_end = min(a.Npix, n_limit);   // (a tile that ends before the tensor does)
     constexpr int WTM = BM / WM, WTN = BN / WN;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -271,7 +273,7 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
                     const int nn = n0 + wn * WTN + j * MT + lc;
-                    if (nn >= a.Npix) continue;
+                    if (nn >= n_end) continue;
 #pragma unroll
                     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -347,7 +349,7 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
                     const int nn = n0 + wn * WTN + j * MT + lc;
-                    if (nn >= a.Npix) continue;
+                    if (nn >= n_end) continue;
                     const floatx4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
                     finish_quad<RES>(a, v, bias, g, m, nn);
                 }

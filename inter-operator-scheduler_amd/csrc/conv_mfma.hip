@@ -1,5 +1,6 @@
 // Stand-alone convolution kernels, the configuration table and the launchers.  Device code: conv_body.h.
-#include "conv_pipe.h"
+#include "conv_kernel.h"
+#include "conv_window.h"
 #include "launch_internal.h"
 
 #include <algorithm>
@@ -7,20 +8,6 @@
 #include <string>
 
 namespace ios {
-
-// stand-alone kernel around a body: grid = (tiles, groups, K slices), dynamic LDS = Body::SMEM_FLOATS floats
-// RES: the residual form of the epilogue (a.res is not null)
-template <typename Body, bool RES = false>
-__global__ __launch_bounds__(Body::THREADS) void conv_kernel(ConvKernelArgs a) {
-    extern __shared__ floatx4 conv_smem[];
-    if (a.xcd_local) {   // one-dimensional grid numbered for split-K inside an XCD
-        const XcdSlot slot = xcd_enter(a, blockIdx.x, blockIdx.x);
-        if (slot.idle) return;
-        Body::template run<RES>(a, reinterpret_cast<float *>(conv_smem), slot.tile, 0, slot.slice);
-        return;
-    }
-    Body::template run<RES>(a, reinterpret_cast<float *>(conv_smem), blockIdx.x, blockIdx.y, blockIdx.z);
-}
 
 __global__ void splitk_reduce_kernel(ReduceArgs a) { splitk_reduce_body(a, blockIdx.x, gridDim.x, blockDim.x); }
 
@@ -81,13 +68,23 @@ struct VariantEntry {
 #define IOS_PIPE_BF16_ENTRY(IDX, ...) IOS_PIPE_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
 #define IOS_PIPE_FP16_ENTRY(IDX, ...) IOS_PIPE_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
 
+#define IOS_WINDOW_ENTRY(TERMS, HALF, PRECISION, IDX, NAME, TMW, TNW, WM, WN, P_IT, NBUF)                                                 \
+    {{NAME, 32 * TMW * WM, 32 * TNW * WN, 16, WM, WN, 1, 32, false, 16, false, false, PRECISION, TERMS, false,                            \
+      ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SPAN},                                                                     \
+     kWindowKernels[IDX - kFirstWindowVariant].kernel, kWindowKernels[IDX - kFirstWindowVariant].kernel_residual,                          \
+     ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SMEM_FLOATS},
+#define IOS_WINDOW3_ENTRY(...) IOS_WINDOW_ENTRY(3, false, PREC_FP32, __VA_ARGS__)
+#define IOS_WINDOW_BF16_ENTRY(...) IOS_WINDOW_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
+#define IOS_WINDOW_FP16_ENTRY(...) IOS_WINDOW_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
+
 static const VariantEntry kVariants[] = {IOS_TILED_VARIANTS(IOS_TILED_ENTRY) IOS_WSPLIT_VARIANTS(IOS_WSPLIT_ENTRY)
                                              IOS_WSPLIT_C4_VARIANTS(IOS_WSPLIT_C4_ENTRY)
                                              IOS_WSPLIT_T32_VARIANTS(IOS_WSPLIT_ENTRY) IOS_WSPLIT_F16_VARIANTS(IOS_WSPLIT_ENTRY)
                                              IOS_WSPLIT_LONGK_VARIANTS(IOS_WSPLIT_ENTRY) IOS_SPLIT3_VARIANTS(IOS_SPLIT3_ENTRY) IOS_WSPLIT_X3_VARIANTS(IOS_WSPLIT_X3_ENTRY)
                                              IOS_SPLIT1_VARIANTS(IOS_SPLIT1_ENTRY) IOS_WSPLIT_X1_VARIANTS(IOS_WSPLIT_X1_ENTRY)
                                              IOS_PIPE3_VARIANTS(IOS_PIPE3_ENTRY) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_ENTRY)
-                                             IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_ENTRY)};
+                                             IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_ENTRY) IOS_WINDOW3_VARIANTS(IOS_WINDOW3_ENTRY)
+                                             IOS_WINDOW_BF16_VARIANTS(IOS_WINDOW_BF16_ENTRY) IOS_WINDOW_FP16_VARIANTS(IOS_WINDOW_FP16_ENTRY)};
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 static_assert(kNumVariants == kNumConvVariants, "variant lists and count disagree");
 
@@ -100,8 +97,42 @@ const ConvVariant &conv_variant(int index) {
 
 static int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
+static int variant_by_name(const char *name) {
+    for (int i = 0; i < kNumVariants; i++)
+        if (std::string(kVariants[i].v.name) == name) return i;
+    throw std::runtime_error(std::string("conv: no kernel configuration named ") + name);
+}
+
+// Input pixels that a block of `outputs` outputs reads at stride 1, as one run: to the last output's place, over the pixels that
+// every row of outputs leaves out, and the rows and columns the filter reaches over.
+static long long window_span(const ConvProblem &p, int outputs) {
+    return outputs - 1 + (long long)ceil_div(outputs - 1, p.OW) * (p.W - p.OW) + (long long)(p.KH - 1) * p.W + p.KW;
+}
+
+bool conv_variant_takes(const ConvProblem &p, int variant) {
+    const ConvVariant &v = conv_variant(variant);
+    if (v.window == 0) return true;
+    const int taps = p.KH * p.KW;   // odd, and a bit each
+    return p.sh == 1 && p.sw == 1 && taps % 2 == 1 && taps >= 3 && taps < 32 && p.OH <= p.H && p.OW <= p.W && window_span(p, v.BN) <= v.window;
+}
+
+// The entry that serves the problem: where a window kernel is asked for and does not take it, one that reads the same packed filters.
+static int variant_for(const ConvProblem &p, const ConvLaunch &l) {
+    if (l.variant < 0 || l.variant >= kNumVariants) throw std::runtime_error("conv: bad variant");
+    if (conv_variant_takes(p, l.variant)) return l.variant;
+    const int precision = kVariants[l.variant].v.precision;
+    static const int plain[] = {variant_by_name("x3p_m64n128_w1x4"), variant_by_name("wb_p_m64n128_w1x4"), variant_by_name("wh_p_m64n128_w1x4")};
+    return plain[precision == PREC_FP32 ? 0 : precision == PREC_BF16 ? 1 : 2];
+}
+
+// tiles of output pixels; a window kernel takes its tiles from one image at a time where the maps shrink (see ConvWindow)
+static int tiles_of_pixels(const ConvProblem &p, const ConvVariant &v) {
+    return v.window != 0 && p.OH != p.H ? p.B * ceil_div((long long)p.OH * p.OW, v.BN) : ceil_div(p.Npix(), v.BN);
+}
+
 static int k_chunk_of(const ConvProblem &p, const ConvLaunch &l) {
-    const ConvVariant &v = kVariants[l.variant].v;
+    const ConvVariant &v = kVariants[variant_for(p, l)].v;
+    if (v.window != 0) return ceil_div(p.ICgP(v.cpad) / 16, std::max(1, l.split_k)) * 16 * p.KH * p.KW;   // chunks of channels, all taps of each
     const int kq = p.Kq(v.cpad);
     // for the wave-split kernels BK is the K extent of one register batch, which may not divide kq
     const int tiles_k = ceil_div(kq, v.BK);
@@ -110,7 +141,7 @@ static int k_chunk_of(const ConvProblem &p, const ConvLaunch &l) {
 
 // split_k may ask for more slices than there are K tiles; the effective count leaves no slice empty
 static int effective_split(const ConvProblem &p, const ConvLaunch &l) {
-    return std::max(1, ceil_div(p.Kq(kVariants[l.variant].v.cpad), k_chunk_of(p, l)));
+    return std::max(1, ceil_div(p.Kq(kVariants[variant_for(p, l)].v.cpad), k_chunk_of(p, l)));
 }
 
 int conv_effective_split(const ConvProblem &p, const ConvLaunch &l) { return effective_split(p, l); }
@@ -120,22 +151,16 @@ size_t conv_workspace_floats(const ConvProblem &p, const ConvLaunch &l) {
     if (s <= 1) return 0;
     // two-kernel form: [slice][OC][pixels]; one-kernel forms: [group][tile][slice][BM * BN] with the tile count rounded up
     // to a multiple of 8 (the numbering of the XCD-local form, see XcdSlot)
-    const ConvVariant &v = kVariants[l.variant].v;
-    const size_t tiles = (size_t)xcd_padded_tiles(ceil_div(p.OCg(), v.BM) * ceil_div(p.Npix(), v.BN));
+    const ConvVariant &v = kVariants[variant_for(p, l)].v;
+    const size_t tiles = (size_t)xcd_padded_tiles(ceil_div(p.OCg(), v.BM) * tiles_of_pixels(p, v));
     const size_t padded = (size_t)p.groups * tiles * v.BM * v.BN;
     return (size_t)s * std::max((size_t)p.OC * (size_t)p.Npix(), padded);
 }
 
 size_t conv_counter_count(const ConvProblem &p, const ConvLaunch &l) {
     if (effective_split(p, l) <= 1) return 0;
-    const ConvVariant &v = kVariants[l.variant].v;
-    return (size_t)p.groups * (size_t)xcd_padded_tiles(ceil_div(p.OCg(), v.BM) * ceil_div(p.Npix(), v.BN));
-}
-
-static int variant_by_name(const char *name) {
-    for (int i = 0; i < kNumVariants; i++)
-        if (std::string(kVariants[i].v.name) == name) return i;
-    throw std::runtime_error(std::string("conv: no kernel configuration named ") + name);
+    const ConvVariant &v = kVariants[variant_for(p, l)].v;
+    return (size_t)p.groups * (size_t)xcd_padded_tiles(ceil_div(p.OCg(), v.BM) * tiles_of_pixels(p, v));
 }
 
 ConvLaunch conv_pick_launch(const ConvProblem &p, int num_cus, bool fusable_only, int precision) {
@@ -216,8 +241,8 @@ bool conv_matrix_path_supported(const ConvProblem &p) {
 ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed,
                                 const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce,
                                 const TensorView *residual, bool post_relu) {
-    if (l.variant < 0 || l.variant >= kNumVariants) throw std::runtime_error("conv: bad variant");
-    const VariantEntry &e = kVariants[l.variant];
+    const int variant = variant_for(p, l);
+    const VariantEntry &e = kVariants[variant];
     if (x.C != p.IC || x.H != p.H || x.W != p.W || y.C != p.OC || y.H != p.OH || y.W != p.OW)
         throw std::runtime_error("conv: tensor views do not match the problem");
     if (p.IC % p.groups != 0 || p.OC % p.groups != 0) throw std::runtime_error("conv: channels not divisible by groups");
@@ -256,7 +281,7 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
         a.steps_per_wave = e.v.kquad ? ceil_div(ceil_div(a.steps_chunk, u), e.v.WK) * u : ceil_div(a.steps_chunk, e.v.WK);
     }
     a.tiles_m = ceil_div(p.OCg(), e.v.BM);
-    a.tiles_n = ceil_div(p.Npix(), e.v.BN);
+    a.tiles_n = tiles_of_pixels(p, e.v);
     a.weights_major = (double)p.OC * p.K() > (double)p.B * p.IC * p.H * p.W ? 1 : 0;
     a.tile_div = a.weights_major ? a.tiles_n : a.tiles_m;
     a.xcd_q = (a.tiles_m * a.tiles_n) >> 3;
@@ -276,7 +301,7 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     }
     if (a.split_k > 1 && workspace == nullptr) throw std::runtime_error("conv: split-K launch without workspace");
     if (p.groups > 65535 || a.split_k > 65535) throw std::runtime_error("conv: grid too large");
-    d.variant = l.variant;
+    d.variant = variant;
     d.threads = e.v.threads();
     d.smem_bytes = e.smem_floats * (int)sizeof(float);
     d.tiles = a.tiles_m * a.tiles_n;

@@ -249,6 +249,5 @@ struct ConvPipe {
     X(143, "wh_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
     X(144, "wh_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
     X(145, "wh_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
-constexpr int kNumConvVariants = 146;
 
 }  // namespace ios

@@ -1,0 +1,272 @@
+// Convolutions of stride 1 with several taps at large batches, on a window of the input that is staged once: ConvWindow.
+//
+// The LDS-tiled kernels of conv_body.h and conv_pipe.h walk K tap by tap: for a 3 x 3 filter they load, convert (into three bfloat16
+// terms, some 50 instructions per eight values) and store every input value nine times.  At stride 1 the pixels that the BN
+// outputs of a block read lie in one run of the input, BN plus the rows the filter reaches over: 200 pixels for 128 outputs of a
+// 3 x 3 filter on 35 x 35 maps.  Here K is walked in chunks of 16 channels with all taps inside, and the run is staged once per
+// chunk; a tap is a constant shift of the LDS address, and a lane whose tap falls outside the image reads a slot of zeros (a bit
+// per tap, known from the start).  Filters are operands straight from memory, one unit (16 k of one tap) ahead in registers, so
+// the only barriers are those around the staging.
+//
+// What is left per unit is matrix work, TNW LDS reads per plane and three address instructions per 32 pixels.  With three
+// terms that reaches the rate at which random operands from LDS keep the matrix cores of this chip at their power limit (1.2 to
+// 1.3 PFLOP/s of bfloat16 with some vector work beside it, 205 to 220 TFLOP/s of fp32).  Measured at batch 64, tap by tap -> on
+// the window: 80 -> 192 channels 3 x 3 on 73 x 73 478 -> 434 us (205 TFLOP/s) in fp32, 225 -> 182 us in bfloat16; 32 -> 64 on 147 x 147
+// 370 -> 323 us (216 -> 206, bound by 530 MB of activations); 32 -> 32 on 149 x 149 291 -> 208 us (158 -> 130).
+#pragma once
+
+#include "conv_pipe.h"
+
+namespace ios {
+
+// TMW x TNW MFMA tiles per wavefront, WM x WN wavefronts per block; P_IT: rounds of T / 2 pixels in which a block stages its window;
+// NBUF: windows in LDS (2: one barrier per chunk, for tiles whose windows are small)
+template <int TERMS, bool HALF, int TMW, int TNW, int WM, int WN, int P_IT, int NBUF>
+struct ConvWindow {
+    static_assert(TERMS == 3 || TERMS == 1, "three exact terms or one rounded term");
+    static_assert(!HALF || TERMS == 1, "half operands are rounded");
+    static constexpr int MT = 32;
+    using M = Mfma<32>;
+    static constexpr int BM = 32 * TMW * WM, BN = 32 * TNW * WN;
+    static constexpr int T = 64 * WM * WN;
+    static constexpr int THREADS = T;
+    static constexpr int CPAD = 16;
+    static constexpr bool FUSABLE = false;
+    static constexpr int SPAN = P_IT * (T / 2);       // pixels of the input a block holds
+    // slots of 16 bytes per plane and octet (eight consecutive channels), the last one zero; the octets of a pixel, which
+    // neighbouring lanes store, fall into different banks
+    static constexpr int S = SPAN + 4;
+    static constexpr int BUF = 2 * TERMS * S;
+    static constexpr int SMEM_FLOATS = NBUF * BUF * 4;
+
+    template <bool RES = false>
+    __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
+    constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
+    uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave % WN;
+    const int wm = wave / WN;
+    const int lk = lane >> 5;
+    const int lc = lane & 31;
+    int tm, tn;
+    xcd_tile(a, tile, tm, tn);
+    const int m0 = tm * BM;
+    int n0 = tn * BN, n_end = a.Npix;
+    if (a.OH != a.H) {   // tiles of one image each (the host counts them so): the input pixels of two images do not follow each other
+        const int per_image = (a.OHW + BN - 1) / BN;
+        const int image = tn / per_image;
+        n0 = image * a.OHW + (tn - image * per_image) * BN;
+        n_end = (image + 1) * a.OHW;
+    }
+    const int taps = a.Kq / a.ICgP;   // odd
+    // K slice z of the grid: a range of chunks of 16 channels, all taps of each
+    const int chunks_all = a.ICgP >> 4;
+    const int per_slice = (chunks_all + a.split_k - 1) / a.split_k;
+    const int ch_begin = z * per_slice, ch_end = min(chunks_all, ch_begin + per_slice);
+
+    const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
+    // ---- filters: packed [g][k / 8][plane][OCgP] slots of 16 bytes, k = tap * ICgP + channel
+    unsigned a_off[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int m = m0 + wm * WTM + i * 32 + lc;
+        a_off[i] = m < a.OCgP ? (((unsigned)g * ((unsigned)a.Kq >> 3) + (unsigned)lk) * TERMS * (unsigned)a.OCgP + (unsigned)m) * 16u : kOutOfRange;
+    }
+    const unsigned plane_bytes = (unsigned)a.OCgP * 16u;
+    const unsigned tap_bytes = (unsigned)(a.ICgP >> 3) * TERMS * plane_bytes, chunk_bytes = 2u * TERMS * plane_bytes;
+
+    // ---- window: first input pixel of the block: tap (0, 0) of output pixel n0
+    auto input_of = [&](int n, int &oh, int &ow) {
+        const int b = (int)fast_div((unsigned)n, a.div_ohw);
+        const int r = n - b * a.OHW;
+        oh = (int)fast_div((unsigned)r, a.div_ow);
+        ow = r - oh * a.OW;
+        return (b * a.H + oh - a.ph) * a.W + ow - a.pw;
+    };
+    int oh_, ow_;
+    const int p0 = input_of(n0, oh_, ow_);
+    const int half = tid & 1;
+    unsigned x_off = (unsigned)((p0 + (tid >> 1)) * a.x_ps + g * a.ICg + 8 * half) * 4u;   // may wrap below zero: beyond the extent
+    const unsigned x_step = (unsigned)(T / 2) * (unsigned)a.x_ps * 4u;
+    floatx4 b_reg[P_IT][2];
+    int b_left;   // real channels of this thread's octet
+    auto load_window = [&](int ch) {
+        const int c0 = ch * 16;
+        b_left = a.ICg - c0 - 8 * half;
+        const unsigned dead = ch < ch_end ? 0u : kOutOfRange;
+        const unsigned pad0 = ((unsigned)(b_left - 1) & kOutOfRange) | dead, pad1 = ((unsigned)(b_left - 5) & kOutOfRange) | dead;
+#pragma unroll
+        for (int i = 0; i < P_IT; i++) {
+            const unsigned at = x_off + (unsigned)c0 * 4u + (unsigned)i * x_step;
+            b_reg[i][0] = buffer_load_f32x4(xr, at | pad0);
+            b_reg[i][1] = buffer_load_f32x4(xr, at | pad1, 16u);
+        }
+    };
+    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const bool ragged = (a.ICg & 3) != 0;
+    auto store_window = [&](int buf) {
+        uintx4 *at = lds + buf * BUF + half * S + (tid >> 1);
+#pragma unroll
+        for (int i = 0; i < P_IT; i++) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(b_reg[i][j >> 2][j & 3]), relu_floor));
+            if (ragged)
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = j < b_left ? v[j] : 0.f;
+            if constexpr (TERMS == 3) {
+                uintx4 hi, mid, lo;
+                split_bf16x3(v, hi, mid, lo);
+                at[i * (T / 2)] = hi;
+                at[i * (T / 2) + 2 * S] = mid;
+                at[i * (T / 2) + 4 * S] = lo;
+            } else if constexpr (HALF) {
+                const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+                at[i * (T / 2)] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));
+            } else {
+                at[i * (T / 2)] = round_bf16x8(v);
+            }
+        }
+    };
+    // this lane's outputs: place of tap (0, 0) in the patch, and the taps that fall inside the image
+    unsigned at0[TN], inside[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int n = n0 + wn * WTN + j * 32 + lc;
+        int oh, ow;
+        const int first = input_of(n < n_end ? n : n0, oh, ow);
+        at0[j] = (unsigned)((first - p0) * 16 + lk * S * 16);
+        unsigned mask = 0;
+        int kh = 0, kw = 0;
+        for (int t = 0; t < taps; t++) {
+            const bool ok = n < n_end && (unsigned)(oh - a.ph + kh) < (unsigned)a.H && (unsigned)(ow - a.pw + kw) < (unsigned)a.W;
+            mask |= (ok ? 1u : 0u) << t;
+            const bool wrap = ++kw == a.KW;
+            kw = wrap ? 0 : kw;
+            kh += wrap ? 1 : 0;
+        }
+        inside[j] = mask;
+    }
+    if (tid < NBUF * TERMS) lds[(tid / TERMS) * BUF + (tid % TERMS) * 2 * S + S - 1] = uintx4{0, 0, 0, 0};
+    constexpr unsigned kZero = (S - 1) * 16;
+
+    typename M::acc_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
+
+    uintx4 av[2][TERMS][TM];
+    // next filter operands to request
+    int r_tap = 0, r_ch = ch_begin;
+    unsigned r_at = (unsigned)ch_begin * chunk_bytes;
+    auto load_filters = [&](uintx4 (&v)[TERMS][TM]) {
+        const __amdgpu_buffer_rsrc_t wr = buffer_of(a.wp, r_ch < ch_end ? a.w_bytes : 0u);
+#pragma unroll
+        for (int p = 0; p < TERMS; p++)
+#pragma unroll
+            for (int i = 0; i < TM; i++) v[p][i] = __builtin_amdgcn_raw_buffer_load_b128(wr, a_off[i], r_at + (unsigned)p * plane_bytes, 0);
+        const bool wrap = ++r_tap == taps;
+        r_tap = wrap ? 0 : r_tap;
+        r_ch += wrap ? 1 : 0;
+        r_at = wrap ? (unsigned)r_ch * chunk_bytes : r_at + tap_bytes;
+    };
+    // tap of the unit at hand, its offset in the patch in bytes
+    int u_tap = 0, u_kw = 0, u_shift = 0;
+    auto unit = [&](const char *buf, const uintx4 (&fv)[TERMS][TM], uintx4 (&next)[TERMS][TM]) {
+        uintx4 bv[TERMS][TN];
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const unsigned valid = (unsigned)((int)(inside[j] << (31 - u_tap)) >> 31);
+            const unsigned at = ((at0[j] + (unsigned)u_shift) & valid) | (kZero & ~valid);
+            const uintx4 *p = reinterpret_cast<const uintx4 *>(buf + at);
+#pragma unroll
+            for (int q = 0; q < TERMS; q++) bv[q][j] = p[q * 2 * S];
+        }
+        load_filters(next);
+        const bool wrap = ++u_kw == a.KW;
+        u_shift += wrap ? (a.W - a.KW + 1) * 16 : 16;
+        u_kw = wrap ? 0 : u_kw;
+        u_tap++;
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int NT = TERMS == 3 ? 6 : 1;
+        constexpr int TA[6] = {TERMS == 3 ? 2 : 0, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    if constexpr (HALF)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, fv[TA[t]][i]), __builtin_bit_cast(halfx8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
+                    else
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fv[TA[t]][i]), __builtin_bit_cast(bf16x8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
+                }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // One chunk: its window from registers into LDS, the next one requested, then one unit of matrix work per tap, each with the
+    // filters of the next unit requested first.  (The first three units lie outside the loop: inside it every wait for filters
+    // would also wait for the window requested in front of it.)  P: the filter registers the chunk starts with; the number of taps
+    // is odd, so the next chunk starts with the other ones.
+    const char *bytes = reinterpret_cast<const char *>(smem);
+    auto chunk = [&](int ch, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        const int b = NBUF == 2 ? (ch & 1) : 0;
+        store_window(b);
+        __syncthreads();
+        load_window(ch + 1);
+        u_tap = 0; u_kw = 0; u_shift = 0;
+        const char *buf = bytes + b * BUF * 16;
+        unit(buf, av[P], av[P ^ 1]);
+        unit(buf, av[P ^ 1], av[P]);
+        for (int t = 3; t < taps; t += 2) {
+            unit(buf, av[P], av[P ^ 1]);
+            unit(buf, av[P ^ 1], av[P]);
+        }
+        unit(buf, av[P], av[P ^ 1]);
+        if (NBUF == 1) __syncthreads();
+    };
+    load_filters(av[0]);
+    load_window(ch_begin);
+    for (int ch = ch_begin; ch < ch_end; ch += 2) {
+        chunk(ch, std::integral_constant<int, 0>{});
+        if (ch + 1 >= ch_end) break;
+        chunk(ch + 1, std::integral_constant<int, 1>{});
+    }
+    __syncthreads();
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, n_end);
+    }   // run
+};
+
+// X(index, name, TMW, TNW, WM, WN, P_IT, NBUF).  A window of a 3 x 3 filter on wide maps takes 300 pixels beyond the outputs, so
+// the tall-and-narrow blocks are for few channels on large maps; the 128-output blocks serve the smaller maps.
+#define IOS_WINDOW3_VARIANTS(X)                          \
+    X(146, "x3_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(147, "x3_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(148, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)    \
+    X(149, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+#define IOS_WINDOW_BF16_VARIANTS(X)                      \
+    X(150, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(151, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(152, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(153, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(154, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+#define IOS_WINDOW_FP16_VARIANTS(X)                      \
+    X(155, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(156, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(157, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(158, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(159, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+constexpr int kFirstWindowVariant = 146, kNumConvVariants = 160;
+
+// The window kernels (conv_window.hip), in the order of the lists above
+struct WindowKernel {
+    void (*kernel)(ConvKernelArgs), (*kernel_residual)(ConvKernelArgs);
+};
+extern const WindowKernel kWindowKernels[];
+
+}  // namespace ios

@@ -103,6 +103,7 @@ struct ConvVariant {
     int koct = 0;
     // fits a fused stage launch of the wide-register kernel family only (the three-term wave-split configurations)
     bool fusable_wide_ = false;
+    int window = 0;   // > 0: stages a window of up to this many input pixels (conv_window.h); for the shapes conv_variant_takes allows
     bool fusable() const { return fusable_ || fusable_wide_; }
     bool needs_wide() const { return fusable_wide_ && !fusable_; }
     int kvec() const { return koct ? 8 : kquad ? 4 : 1; }   // consecutive k of one output channel that lie together
@@ -110,6 +111,7 @@ struct ConvVariant {
 
 int conv_num_variants();
 const ConvVariant &conv_variant(int index);
+bool conv_variant_takes(const ConvProblem &p, int variant);   // (a launch of another shape runs on a configuration that reads the same packed filters)
 
 struct ConvLaunch {
     int variant = 0;

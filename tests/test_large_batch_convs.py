@@ -1,0 +1,68 @@
+"""The convolution kernels for large batches that stage both operands (x3p_*, wb_p_*, wh_p_*) or a window of the input
+(x3_win_*, wb_win_*, wh_win_*) in LDS, at the edges of their tiles and windows, against the oracle."""
+import numpy as np
+import pytest
+
+import ios
+from ios.contrib import ios_runtime as rt
+from ios.ir import Block, Graph, Value
+from test_gpu_parity import assert_close, ios_oracle, matrix_path_convs
+
+pytestmark = pytest.mark.gpu
+
+FAMILIES = [('fp32', ('x3p_', 'x3_win_'), None), ('bf16', ('wb_p_', 'wb_win_'), 'bf16_convs'), ('fp16', ('wh_p_', 'wh_win_'), 'fp16_convs')]
+NAMES = [(name, precision, key) for precision, prefixes, key in FAMILIES for name in rt.conv_variant_names() if name.startswith(prefixes)]
+
+# in_shape, out channels, kernel, padding, batch
+CASES = [
+    ((18, 9, 11), 33, (3, 3), (1, 1), 5),       # tiles over several images, channels that end inside a quad and a tile
+    ((17, 13, 7), 64, (3, 3), (0, 0), 3),       # shrinking maps: tiles of one image each, the last one short
+    ((40, 16, 17), 96, (1, 7), (0, 3), 2),      # one row, the taps beside the image masked
+    ((35, 17, 9), 65, (7, 1), (3, 0), 2),
+    ((16, 12, 12), 20, (5, 5), (2, 2), 4),      # 25 taps
+    ((5, 3, 3), 200, (3, 3), (1, 1), 1),        # fewer pixels than any tile, one chunk of channels
+    ((33, 6, 80), 31, (3, 3), (2, 0), 1),       # a map that grows in height: not for the window kernels
+    ((20, 8, 200), 40, (3, 3), (1, 1), 1),      # rows too wide for the smaller windows
+    ((24, 10, 10), 48, (2, 2), (0, 0), 2),      # an even number of taps
+]
+
+
+@pytest.fixture(autouse=True)
+def default_options():
+    yield
+    for key, value in (('conv_variant', -1), ('conv_split_k', 0), ('precision', 'fp32'), ('split_k_reduce', 'xcd')):
+        rt.set_option(key, value)
+
+
+def build(case, reader):
+    """The convolution reads a channel window of the input (from an odd channel on) and writes one of a concatenation."""
+    in_shape, oc, kernel, pad, _ = case
+    ios.reset_name()
+    holder = ios.placeholder((in_shape[0] + 3, *in_shape[1:]))
+    block = Block(holder.node, None, [], None)
+    window = Value(holder.node, 1, in_shape[0] + 1)
+    conv = ios.conv2d(block, [[window]], oc, kernel, (1, 1), pad, act='relu')
+    if reader:
+        other = ios.pool2d(block, [[conv]], 'max', (3, 3), (1, 1), (1, 1))
+        ios.identity(block, [[other], [conv]], is_exit=True)
+    else:
+        ios.identity(block, [[conv]], is_exit=True)
+    graph = Graph('large', holder.node, [block])
+    graph.init_weights(3, 'he_normal_bias')
+    graph.sequential_schedule()
+    return graph
+
+
+@pytest.mark.parametrize('name,precision,key', NAMES, ids=[n[0] for n in NAMES])
+def test_edges(name, precision, key):
+    rt.set_option('precision', precision)
+    rt.set_option('conv_variant', rt.device_info()['conv_variants'].index(name))
+    for index, case in enumerate(CASES):
+        graph = build(case, reader=index % 2 == 0)
+        x = np.random.default_rng(index).standard_normal((case[4], *graph.enter_node.output_shape)).astype(np.float32)
+        want = ios_oracle.run(graph, x, **({key: matrix_path_convs(graph, case[4])} if key else {}))
+        for split, reduce in ((1, 'xcd'), (2, ('xcd', 'inline', 'kernel')[index % 3])):
+            rt.set_option('conv_split_k', split)
+            rt.set_option('split_k_reduce', reduce)
+            got = rt.graph_inference(graph, case[4], x)
+            assert_close(got, want, f'{name} {case} split {split} {reduce}')
