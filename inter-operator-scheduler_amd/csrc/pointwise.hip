@@ -13,8 +13,7 @@ __global__ void global_pool_kernel(PoolArgs a) { global_pool_body(a, blockIdx.x,
 __global__ void dwconv_kernel(DirectConvArgs a) { dwconv_dispatch(a, blockIdx.x, gridDim.x, blockDim.x); }
 __global__ void conv_direct_kernel(DirectConvArgs a) { conv_direct_body(a, blockIdx.x, gridDim.x, blockDim.x); }
 __global__ __launch_bounds__(256) void conv_thin_kernel(DirectConvArgs a) {
-    __shared__ float filters[kThinConvSmemFloats];
-    conv_thin_body(a, filters, blockIdx.x, gridDim.x);
+    conv_thin_body(a, blockIdx.x, gridDim.x);
 }
 __global__ void nary_kernel(NaryKernelArgs a) { nary_dispatch(a, blockIdx.x, gridDim.x, blockDim.x); }
 
@@ -95,9 +94,8 @@ DirectConvArgs make_direct_conv_args(const ConvProblem &p, const TensorView &x, 
     *blocks = blocks_for(pixels * ((p.OC + a.channels - 1) / a.channels), 256, 8192);
     if (thin) {
         if (!conv_thin_applies(p)) throw std::runtime_error("conv: the thin-input kernel serves 3 x 3 convolutions of 3-channel inputs");
-        // one block per 256 pixels and 32 output channels (sized for 256-thread blocks like the other bodies)
-        const long long units = ((pixels + 255) / 256) * ((p.OC + kThinConvChannels - 1) / kThinConvChannels);
-        *blocks = (int)std::min<long long>(units, 1 << 20);
+        // up to eight blocks of four wavefronts per compute unit, each on several tiles of pixels
+        *blocks = (int)std::min<long long>((pixels + kThinConvPixels - 1) / kThinConvPixels, 2048);
     }
     return a;
 }
