@@ -356,6 +356,24 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         }
         if (!found[c]) result.best[c] = conv_pick_launch(p, std::max(1, num_cus_ >> c), c > 0, precision_);
     }
+    // A convolution large enough for a kernel that no fused launch can hold is launched by itself also where it shares its stage:
+    // when that kernel and the gap in front of it take less than the device time of the best fusable one, which is its time
+    // or, where its blocks do not fill the device, their share of it.  (Allowing 5 us for the gap; Inception-v3 under the greedy
+    // schedule: bfloat16 at batch 24 1970 -> 1840 us, fp32 at batch 32 3335 -> 3270, half at batch 12 1115 -> 1090; SqueezeNet, half,
+    // batch 50 585 -> 480.  With 3 us the middle sizes lose up to 1 %, with 8 the small maps 7 %.)
+    constexpr float kGapMs = 0.005f;
+    if (fused_executor() && found[0] && !conv_variant(result.best[0].variant).fusable()) {
+        auto device_time = [&](const ConvLaunch &l) {
+            for (const Candidate &cand : candidates)
+                if (cand.launch.variant == l.variant && cand.launch.split_k == l.split_k) return cand.ms * (float)std::min(1.0, cand.footprint / capacity);
+            return 0.f;
+        };
+        float alone = 0.f;
+        for (const Candidate &cand : candidates)
+            if (cand.launch.variant == result.best[0].variant && cand.launch.split_k == result.best[0].split_k) alone = cand.ms;
+        for (int c = 1; c < kShareClasses; c++)
+            if (found[c] && alone + kGapMs < device_time(result.best[c])) result.best[c] = result.best[0];
+    }
     if (!tune_cache_path_.empty()) {
         FILE *f = fopen(tune_cache_path_.c_str(), "a");
         if (f != nullptr) {
@@ -901,7 +919,7 @@ void Session::build_fused() {
                                                                   tv(op.out), c.ws_floats ? base_ + c.ws_off : nullptr, ctx_.split_reduce(counters_of(c)),
                                                                   op.has_residual ? &residual : nullptr, op.post_relu != 0);
                         pend.fusable = conv_variant(d.variant).fusable() && !op.has_residual;   // (the fused kernel holds the plain epilogue)
-                        if (!pend.fusable && !solo)
+                        if (!pend.fusable && !solo && (op.has_residual || ctx_.forced_variant() >= 0))
                             throw std::runtime_error(op.has_residual ? std::string("internal: a residual convolution is planned for single-group stages only")
                                                                      : std::string("convolution kernel configuration ") + conv_variant(d.variant).name +
                                                                            " cannot run inside a fused stage launch");
@@ -917,7 +935,7 @@ void Session::build_fused() {
                         pend.smem_bytes = d.smem_bytes;
                         if (d.has_reduce && solo) pend.fusable = false;   // launched stand-alone, reduction included
                         level_of(op).push_back(pend);
-                        if (d.has_reduce && !solo) {
+                        if (d.has_reduce && pend.fusable) {
                             Pending red;
                             memset(&red.item, 0, sizeof(WorkItem));
                             red.item.kind = WORK_REDUCE;
@@ -984,6 +1002,10 @@ void Session::build_fused() {
             for (auto &chain : chains)
                 if (level < chain.size())
                     for (Pending &pend : chain[level]) {
+                        if (!solo && !pend.fusable) {   // fills the device by itself (see tune_conv); the others of the level share launches
+                            fused_stages_[s].push_back(FusedLaunch{0, 0, 0, 0, 0, pend.op, {}, {pend.op}});
+                            continue;
+                        }
                         here.push_back(&pend);
                         widest = std::max(widest, pend.threads);
                         all_fusable = all_fusable && pend.fusable;

@@ -29,8 +29,9 @@ CASES = [
 
 @pytest.fixture(autouse=True)
 def default_options():
+    rt.set_option('autotune', 0)
     yield
-    for key, value in (('conv_variant', -1), ('conv_split_k', 0), ('precision', 'fp32'), ('split_k_reduce', 'xcd')):
+    for key, value in (('autotune', 0), ('executor', 'fused'), ('conv_variant', -1), ('conv_split_k', 0), ('precision', 'fp32'), ('split_k_reduce', 'xcd')):
         rt.set_option(key, value)
 
 
@@ -66,3 +67,35 @@ def test_edges(name, precision, key):
             rt.set_option('split_k_reduce', reduce)
             got = rt.graph_inference(graph, case[4], x)
             assert_close(got, want, f'{name} {case} split {split} {reduce}')
+
+
+@pytest.mark.parametrize('executor', ['fused', 'fused_graph'])
+@pytest.mark.parametrize('precision,key', [('bf16', 'bf16_convs'), ('fp16', 'fp16_convs')])
+def test_parallel_stage_launches_large_convolutions_by_themselves(precision, key, executor):
+    """Measured configurations: two large convolutions of a parallel stage take kernels no fused launch holds; the small convolution
+    and the pool beside them share one launch."""
+    ios.reset_name()
+    holder = ios.placeholder((64, 35, 35))
+    block = Block(holder.node, None, [], None)
+    first = ios.conv2d(block, [[holder]], 96, (3, 3), (1, 1), (1, 1))
+    second = ios.conv2d(block, [[holder]], 96, (3, 3), (1, 1), (1, 1), act='identity')
+    small = ios.conv2d(block, [[Value(holder.node, 3, 11)]], 7, (1, 1))
+    pool = ios.pool2d(block, [[holder]], 'max', (3, 3), (1, 1), (1, 1))
+    ios.identity(block, [[first], [second], [small], [pool]], is_exit=True)
+    graph = Graph('stage', holder.node, [block])
+    graph.init_weights(4, 'he_normal_bias')
+    graph.greedy_schedule(8)
+    x = np.random.default_rng(9).standard_normal((24, 64, 35, 35)).astype(np.float32)
+    rt.set_option('precision', precision)
+    rt.set_option('executor', executor)
+    rt.set_option('autotune', 1)
+    with rt.Session(graph, 24) as session:
+        session.load_weights()
+        session.set_input(x)
+        kernels = [launch['kernel'] for launch in session.launches()]
+        assert sum(name.startswith('conv_kernel<') for name in kernels) == 2 and sum(name.startswith('fused_kernel') for name in kernels) == 1, kernels
+        for _ in range(3):
+            session.run()
+            got = session.output()
+        convs = frozenset(op['node'] for op in session.describe() if op['kind'] == 'conv_mfma')
+    assert_close(got, ios_oracle.run(graph, x, **{key: convs}), f'{precision} {executor}')
