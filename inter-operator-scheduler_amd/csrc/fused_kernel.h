@@ -132,6 +132,8 @@ __device__ __forceinline__ int fused_item_index(const WorkItem *items, int bid, 
 // The first blocks of the items travel as scalar kernel arguments (b1 ... b7; item 0 starts at block 0): with
 // -amdgpu-kernarg-preload-count the command processor hands them to a wavefront in registers, so a block knows its item
 // without a load and its first load is the item itself.
+// Four wavefronts per SIMD, 128 registers: with six (80 registers) the channels-last loaders spill, and four, five and six
+// measured the same (launches of a batch-1 network rarely have two wavefronts for a SIMD).
 template <int T>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4))) void fused_kernel(const WorkItem *__restrict__ items, int num_items, int b1, int b2,
                                                                                             int b3, int b4, int b5, int b6, int b7) {
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4))) void fus
 // block's first load (its item) then hits, where the table costs a miss all the way to memory at the start of every launch
 // (the caches do not keep it from one launch to the next): 1.0 % of an Inception-v3 pass, 1.2 % of NASNet-A mobile, 2 % of
 // SqueezeNet 1.1 in same-device A/B runs.  With the items there the compiler loads all eight source descriptors of the
-// summing depth-wise body ahead of its loop, which does not fit beside the matrix-path bodies in 80 registers, so the form
+// summing depth-wise body ahead of its loop, which does not fit beside the matrix-path bodies in 128 registers, so the form
 // comes as two kernels: fused_kernel_inline holds the matrix-path convolution bodies and no depth-wise / direct ones,
 // fused_kernel_inline_direct the other way round with four wavefronts per SIMD (another 1.9 % of NASNet-A mobile).
 // fused_launch_form() chooses.
