@@ -13,7 +13,6 @@ resident on the device and the forward pass can be run, timed and profiled repea
 import ctypes
 import json
 import os
-import sys
 from typing import List, Optional
 
 import numpy as np
@@ -259,7 +258,6 @@ class Session:
             _check(1, 'ios_session_create')
         self.input_shape = (batch_size, *graph.enter_node.output_shape)
         self.output_shape = (batch_size, *graph.blocks[-1].exit_node.output_shape)
-        self._results = []   # result arrays handed out, see _result_array
 
     def close(self):
         if self._handle:
@@ -299,21 +297,8 @@ class Session:
     def synchronize(self):
         _check(self._lib.ios_session_synchronize(self._handle), 'ios_session_synchronize')
 
-    def _result_array(self) -> np.ndarray:
-        """
-        An uninitialised array for a result.  A large one that the caller has let go of (nothing but this list refers to it)
-        is handed out again: touching the fresh pages of a new 2 MB array takes longer than copying the result into it.
-        """
-        for array in self._results:
-            if sys.getrefcount(array) == 3:   # the list, the loop variable and the argument of getrefcount
-                return array
-        array = np.empty(self.output_shape, dtype=np.float32)
-        if array.nbytes >= 1 << 16:
-            self._results = self._results[-1:] + [array]
-        return array
-
     def output(self) -> np.ndarray:
-        out = self._result_array()
+        out = np.empty(self.output_shape, dtype=np.float32)
         _check(self._lib.ios_session_get_output(self._handle, out.ctypes.data), 'ios_session_get_output')
         return out
 

@@ -461,3 +461,46 @@ def test_average_pools_change_places_with_the_pointwise_convolution_behind_them(
     nasnet = ios.models.nasnet_mobile()
     nasnet.sequential_schedule()
     assert not any(op.get('linear') for op in rt.plan_describe(nasnet, 1))
+
+
+class _WritesZeros:
+    """Stands in for the library: every result is zeros."""
+
+    def __init__(self, floats):
+        self.floats = floats
+
+    def ios_session_get_output(self, handle, pointer):
+        ctypes.memset(pointer, 0, 4 * self.floats)
+        return 0
+
+    def ios_session_destroy(self, handle):
+        pass
+
+
+def test_result_arrays_belong_to_the_caller():
+    """Whatever a caller does to a result, the next one is an array of its own in the result's shape."""
+    session = object.__new__(rt.Session)
+    session.output_shape = (1, 64, 64, 64)
+    session._lib, session._handle = _WritesZeros(1 << 18), None
+
+    def check(y):
+        assert y.shape == (1, 64, 64, 64) and y.dtype == np.float32 and y.flags.writeable and y.flags.c_contiguous and y.flags.owndata
+        assert not y.any()
+        return y
+
+    y = check(session.output())
+    y.shape = (-1,)
+    del y
+    y = check(session.output())
+    y.dtype = np.uint32
+    del y
+    y = check(session.output())
+    y.flags.writeable = False
+    del y
+    check(session.output()).resize((2, 3))
+    y = check(session.output())
+    address, row = y.ctypes.data, y[0, 3]
+    row[:] = 7
+    del y
+    later = [check(session.output()) for _ in range(4)]
+    assert all(address != z.ctypes.data for z in later) and (row == 7).all()
