@@ -78,8 +78,9 @@ public:
         const char *src;
     };
     void upload_pieces(char *dst, const std::vector<Piece> &pieces, hipStream_t link, hipStream_t stream, const std::function<void(size_t)> &step);
-    // Device to host, complete on return.
-    void download(void *dst, const void *src, size_t bytes, hipStream_t stream);
+    // A tensor to the caller in the host's layout, complete on return.  Kernels gather it into the staging buffers, so it needs
+    // no device memory.
+    void download(float *dst, const TensorView &src, int batch, hipStream_t stream);
 
     // Waiting for a pass: a last small kernel raises a word in host memory that the caller watches (a kernel and this
     // wait take 5.8 us where hipStreamSynchronize takes 9.5).  Where the result is small or the caller is known to fetch

@@ -200,10 +200,9 @@ struct NaryArgs {
 void launch_nary(const NaryArgs &a, int multiply, int accumulate, int act, int B, const TensorView &y, hipStream_t stream);
 // y = act(x) for views; act == ACT_NONE is a strided copy.
 void launch_unary(const TensorView &x, const TensorView &y, int act, int B, hipStream_t stream);
-// Between a host tensor's layout (NCHW, dense) and a view: x -> y and back.  `nchw` may lie in host memory.  plane > 0: elements
-// between the channels of `nchw` where the view is a part of its pixels (one image).
+// From a host tensor's layout (NCHW, dense) to a view.  `nchw` may lie in host memory.  plane > 0: elements between the channels
+// of `nchw` where the view is a part of its pixels (one image).
 void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t stream, long long plane = 0);
-void launch_from_view(const TensorView &x, float *nchw, int B, hipStream_t stream);
 // Fill n floats with a deterministic pattern in [-1, 1) (seeded), or with a constant.
 void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream);
 void launch_fill_u32(unsigned *dst, size_t n, unsigned value, hipStream_t stream);

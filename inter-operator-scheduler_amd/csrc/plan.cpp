@@ -638,12 +638,6 @@ private:
             }
         }
         if (Region *r = region_of(plan_.output.offset)) r->pinned = true;
-        const size_t result = (size_t)batch_ * plan_.output.image_floats();
-        if (result > kDeliveredFloats && plan_.output.H * plan_.output.W > 1) {   // written behind the last stage
-            plan_.result_floats = result;
-            plan_.result_off = reserve_region(result);
-            touch(plan_.result_off, last_stage);
-        }
         const bool reuse = planner_arena_reuse();
         for (Region &r : regions_)
             if (r.pinned || !reuse || r.last < 0) {   // (an untouched region belongs to an operator nobody reads: keep it apart)
@@ -699,7 +693,6 @@ private:
         place(plan_.input);
         place(plan_.output);
         if (plan_.prefix_stages > 0) plan_.landing_off = placed(plan_.landing_off);
-        if (plan_.result_floats > 0) plan_.result_off = placed(plan_.result_off);
     }
 
     void allocate_outputs() {

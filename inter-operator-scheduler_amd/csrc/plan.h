@@ -112,8 +112,6 @@ struct Plan {
     // way to the device (0: the input is too small for that); their tensors share no memory with each other.
     int prefix_stages = 0;
     size_t landing_off = 0;   // where the images of a plan with a prefix land, in the host's layout
-    // place for the result in the host's layout where it is too large for the pass to deliver it (else 0 floats)
-    size_t result_off = 0, result_floats = 0;
 };
 
 enum class PlanMode { Graph, Block, Stage };

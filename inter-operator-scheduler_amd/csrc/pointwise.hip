@@ -204,34 +204,28 @@ void launch_pack_depthwise(const ConvProblem &p, const float *w, float *packed, 
     hipLaunchKernelGGL(pack_depthwise_kernel, dim3(blocks_for((long long)padded * taps, 256, 1024)), dim3(256), 0, stream, w, packed, p.OC, padded, taps);
 }
 
-// ---- between the host's layout and views ---------------------------------------------------------------------------------
+// ---- from the host's layout to views -------------------------------------------------------------------------------------
 // Bound by bytes (or by the link, where `nchw` lies in host memory).  Few channels (images): a thread takes a pixel, reads its
 // channels from their planes, consecutive threads consecutive pixels, and writes one pixel.  Otherwise a block turns a
 // tile of 32 channels x 64 pixels through LDS.
-template <bool TO_VIEW>
-__global__ __launch_bounds__(256) void layout_kernel(float *nchw, float *view, int B, int C, int HW, long long plane, int ps) {
+__global__ __launch_bounds__(256) void to_view_kernel(const float *nchw, float *view, int B, int C, int HW, long long plane, int ps) {
     if (C <= 4) {
         const long long total = (long long)B * HW;
         for (long long i = blockIdx.x * 256LL + threadIdx.x; i < total; i += gridDim.x * 256LL) {
             const long long b = i / HW, r = i - b * HW;
-            float *first = nchw + b * C * plane + r, *pixel = view + i * ps;
-            if (TO_VIEW) {
-                float v[4] = {0.f, 0.f, 0.f, 0.f};
+            const float *first = nchw + b * C * plane + r;
+            float *pixel = view + i * ps;
+            float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int c = 0; c < 4; c++)
-                    if (c < C) v[c] = first[c * plane];
-                if (ps == 4) {
-                    const pw_floatx4 q = {v[0], v[1], v[2], v[3]};
-                    *reinterpret_cast<pw_floatx4_u *>(pixel) = q;
-                } else {
-#pragma unroll
-                    for (int c = 0; c < 4; c++)
-                        if (c < C) pixel[c] = v[c];
-                }
+            for (int c = 0; c < 4; c++)
+                if (c < C) v[c] = first[c * plane];
+            if (ps == 4) {
+                const pw_floatx4 q = {v[0], v[1], v[2], v[3]};
+                *reinterpret_cast<pw_floatx4_u *>(pixel) = q;
             } else {
 #pragma unroll
                 for (int c = 0; c < 4; c++)
-                    if (c < C) first[c * plane] = pixel[c];
+                    if (c < C) pixel[c] = v[c];
             }
         }
         return;
@@ -247,29 +241,18 @@ __global__ __launch_bounds__(256) void layout_kernel(float *nchw, float *view, i
         const long long bt = t / tiles_p;
         const int p0 = (int)(t - bt * tiles_p) * 64;
         const int b = (int)(bt / tiles_c), c0 = (int)(bt - (long long)b * tiles_c) * 32;
-        float *planes = nchw + ((long long)b * C + c0) * plane + p0, *pixels = view + ((long long)b * HW + p0) * ps + c0;
+        const float *planes = nchw + ((long long)b * C + c0) * plane + p0;
+        float *pixels = view + ((long long)b * HW + p0) * ps + c0;
         __syncthreads();
-        if (TO_VIEW) {
-            float v[8];
+        float v[8];
 #pragma unroll
-            for (int i = 0; i < 8; i++) v[i] = c0 + c4 + 4 * i < C && p0 + px < HW ? planes[(c4 + 4 * i) * plane + px] : 0.f;
+        for (int i = 0; i < 8; i++) v[i] = c0 + c4 + 4 * i < C && p0 + px < HW ? planes[(c4 + 4 * i) * plane + px] : 0.f;
 #pragma unroll
-            for (int i = 0; i < 8; i++) tile[c4 + 4 * i][px] = v[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (c0 + cx < C && p0 + p8 + 8 * i < HW) tile[cx][p8 + 8 * i] = pixels[(long long)(p8 + 8 * i) * ps + cx];
-        }
+        for (int i = 0; i < 8; i++) tile[c4 + 4 * i][px] = v[i];
         __syncthreads();
-        if (TO_VIEW) {
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (c0 + cx < C && p0 + p8 + 8 * i < HW) pixels[(long long)(p8 + 8 * i) * ps + cx] = tile[cx][p8 + 8 * i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (c0 + c4 + 4 * i < C && p0 + px < HW) planes[(c4 + 4 * i) * plane + px] = tile[c4 + 4 * i][px];
-        }
+        for (int i = 0; i < 8; i++)
+            if (c0 + cx < C && p0 + p8 + 8 * i < HW) pixels[(long long)(p8 + 8 * i) * ps + cx] = tile[cx][p8 + 8 * i];
     }
 }
 
@@ -278,13 +261,8 @@ static int layout_blocks(int B, int C, int HW) {
 }
 
 void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t stream, long long plane) {
-    hipLaunchKernelGGL(layout_kernel<true>, dim3(layout_blocks(B, y.C, y.H * y.W)), dim3(256), 0, stream, const_cast<float *>(nchw), y.ptr, B, y.C,
+    hipLaunchKernelGGL(to_view_kernel, dim3(layout_blocks(B, y.C, y.H * y.W)), dim3(256), 0, stream, nchw, y.ptr, B, y.C,
                        y.H * y.W, plane > 0 ? plane : (long long)y.H * y.W, y.pstride);
-}
-
-void launch_from_view(const TensorView &x, float *nchw, int B, hipStream_t stream) {
-    hipLaunchKernelGGL(layout_kernel<false>, dim3(layout_blocks(B, x.C, x.H * x.W)), dim3(256), 0, stream, nchw, x.ptr, B, x.C, x.H * x.W,
-                       (long long)x.H * x.W, x.pstride);
 }
 
 // ---- fills ---------------------------------------------------------------------------------------------------------

@@ -39,7 +39,6 @@ public:
 
     // a process-wide arena reused by the stateless latency / inference entry points
     float *shared_arena(size_t floats);
-    float *turning_buffer(size_t floats);   // for a tensor on its way out in the host's layout
     void *shared_table(size_t bytes);   // companion buffer for the launch tables of such sessions
 
     void set_option(const std::string &key, const std::string &value);
@@ -113,8 +112,6 @@ private:
     std::string name_, arch_;
     hipStream_t streams_[kMaxGroups];
     HostStage stage_;
-    float *turning_ = nullptr;
-    size_t turning_floats_ = 0;
     float *arena_ = nullptr;
     size_t arena_floats_ = 0;
     void *table_ = nullptr;

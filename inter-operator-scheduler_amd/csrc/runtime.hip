@@ -424,18 +424,6 @@ float *DeviceContext::shared_arena(size_t floats) {
     return arena_;
 }
 
-float *DeviceContext::turning_buffer(size_t floats) {
-    if (floats > turning_floats_) {
-        IOS_HIP(hipDeviceSynchronize());
-        if (turning_ != nullptr) IOS_HIP(hipFree(turning_));
-        turning_ = nullptr;
-        turning_floats_ = 0;
-        IOS_HIP(hipMalloc(reinterpret_cast<void **>(&turning_), floats * sizeof(float)));
-        turning_floats_ = floats;
-    }
-    return turning_;
-}
-
 void *DeviceContext::shared_table(size_t bytes) {
     if (bytes > table_bytes_) {
         IOS_HIP(hipDeviceSynchronize());
@@ -699,16 +687,7 @@ void Session::set_conv_weights(int count, char **names, float **weights, float *
 // Dense copy of a view in the host's layout.
 void Session::copy_out(const ViewRef &view, float *host) {
     settle();
-    hipStream_t main = ctx_.stream(0);
-    const size_t floats = (size_t)plan_.batch * view.image_floats();
-    const TensorView t = tv(view);
-    const float *from = t.ptr;
-    if (view.H * view.W > 1 || t.pstride != t.C) {
-        float *turned = &view == &plan_.output && plan_.result_floats > 0 ? base_ + plan_.result_off : ctx_.turning_buffer(floats);
-        launch_from_view(t, turned, plan_.batch, main);
-        from = turned;
-    }
-    ctx_.stage().download(host, from, floats * sizeof(float), main);
+    ctx_.stage().download(host, tv(view), plan_.batch, ctx_.stream(0));
 }
 
 void Session::get_output(float *host) {

@@ -99,3 +99,25 @@ def test_inference_calls_take_turns(no_alloc):
         session.run()
         assert np.allclose(got, session.output(), rtol=1e-4, atol=1e-5)
         session.close()
+
+
+# beyond what a pass delivers, in one and in several parts, ends of parts inside images, planes and quads of channels
+@pytest.mark.parametrize('batch,shape', [(5, (37, 101, 103)), (2, (1, 1024, 1031)), (2100, (501, 1, 1)), (3, (350, 32, 32)), (70001, (15, 1, 1))])
+def test_large_results_of_several_images(batch, shape):
+    """A tensor that shares its pixels with another one's channels, and a result that does not fit the pass's delivery."""
+    ios.reset_name()
+    v = ios.placeholder(shape)
+    block = ios.Block(v.node)
+    a = ios.relu(block, [[v]])
+    b = ios.pool2d(block, [[v]], 'max', (1, 1), (1, 1), (0, 0))
+    ios.identity(block, [[a], [b]], is_exit=True)
+    graph = Graph('t', v.node, [block])
+    graph.sequential_schedule()
+    x = np.random.default_rng(batch).standard_normal((batch, *shape), dtype=np.float32)
+    with rt.Session(graph, batch) as session:
+        session.set_input(x)
+        session.run()
+        want = np.concatenate([np.maximum(x, 0), x], axis=1)
+        assert np.array_equal(session.output(), want)
+        assert np.array_equal(session.tensor(a.node), want[:, :shape[0]])
+        assert np.array_equal(session.tensor(b.node), want[:, shape[0]:])

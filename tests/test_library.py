@@ -9,6 +9,7 @@ import pytest
 
 import ios
 from ios.contrib import ios_runtime as rt
+from ios.ir import Block, Graph
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -504,3 +505,17 @@ def test_result_arrays_belong_to_the_caller():
     del y
     later = [check(session.output()) for _ in range(4)]
     assert all(address != z.ctypes.data for z in later) and (row == 7).all()
+
+
+@pytest.mark.parametrize('shape,batch', [((37, 101, 103), 5), ((64, 56, 56), 32)])
+def test_a_large_result_is_laid_out_once(shape, batch):
+    """The result in the host's layout takes no device memory of its own, however large it is."""
+    ios.reset_name()
+    v = ios.placeholder(shape)
+    block = Block(v.node)
+    ios.relu(block, [[v]], is_exit=True)
+    graph = Graph('t', v.node, [block])
+    graph.sequential_schedule()
+    channels = (shape[0] + 3) // 4 * 4
+    tensor = 4 * batch * channels * shape[1] * shape[2]
+    assert rt.plan_arena_bytes(graph, batch) <= 2 * tensor + 4 * batch * int(np.prod(shape)) // 2 + 1024

@@ -100,3 +100,10 @@ def test_a_graph_beyond_the_static_array_is_refused_and_the_next_call_works():
     sample.sequential_schedule()
     both(sample, 1, seed=4)
     both(sample, 2, seed=4)
+
+
+def test_large_batches_that_fit_the_scratch_are_accepted():
+    """The result of a batch, 2.5 MB an image here, is in the scratch once."""
+    graph = ios.models.sample_network(init_seed=0, init_scheme='he_normal_bias')
+    graph.sequential_schedule()
+    both(graph, 60, 3)
