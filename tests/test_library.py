@@ -478,14 +478,21 @@ class _WritesZeros:
         pass
 
 
-def test_result_arrays_belong_to_the_caller():
-    """Whatever a caller does to a result, the next one is an array of its own in the result's shape."""
+def session_without_device(shape):
     session = object.__new__(rt.Session)
-    session.output_shape = (1, 64, 64, 64)
-    session._lib, session._handle = _WritesZeros(1 << 18), None
+    session.output_shape, session._result_bytes = shape, 4 * int(np.prod(shape))
+    session._lib, session._handle, session._free = _WritesZeros(int(np.prod(shape))), None, []
+    return session
+
+
+# arrays of malloc's own reuse, and arrays over memory that the session keeps
+@pytest.mark.parametrize('shape', [(1, 64, 64, 64), (5, 35, 300, 161)])
+def test_result_arrays_belong_to_the_caller(shape):
+    """Whatever a caller does to a result, the next one is an array of its own in the result's shape."""
+    session = session_without_device(shape)
 
     def check(y):
-        assert y.shape == (1, 64, 64, 64) and y.dtype == np.float32 and y.flags.writeable and y.flags.c_contiguous and y.flags.owndata
+        assert type(y) is np.ndarray and y.shape == shape and y.dtype == np.float32 and y.flags.writeable and y.flags.c_contiguous
         assert not y.any()
         return y
 
@@ -497,14 +504,31 @@ def test_result_arrays_belong_to_the_caller():
     del y
     y = check(session.output())
     y.flags.writeable = False
+    y.flags.writeable = True
+    y.flags.writeable = False
     del y
-    check(session.output()).resize((2, 3))
+    if 4 * np.prod(shape) <= 32 << 20:
+        check(session.output()).resize((2, 3))
     y = check(session.output())
-    address, row = y.ctypes.data, y[0, 3]
+    row, held = y[0, 3], memoryview(y[0, 4])
     row[:] = 7
+    held.obj[:] = 8
     del y
     later = [check(session.output()) for _ in range(4)]
-    assert all(address != z.ctypes.data for z in later) and (row == 7).all()
+    assert not any(np.shares_memory(row, z) for z in later) and (row == 7).all()
+    assert not any(np.shares_memory(a, b) for a in later for b in later if a is not b)
+    del later, row
+    check(session.output())
+    assert (np.asarray(held) == 8).all() and len(session._free) <= 2
+
+
+def test_memory_of_large_results_is_used_again():
+    session = session_without_device((1, 3, 2000, 1500))
+    first, second = session.output(), session.output()
+    addresses = {first.ctypes.data, second.ctypes.data}
+    del first, second
+    assert {memory.ctypes.data for memory in session._free} == addresses
+    assert {session.output().ctypes.data for _ in range(5)} <= addresses
 
 
 @pytest.mark.parametrize('shape,batch', [((37, 101, 103), 5), ((64, 56, 56), 32)])
