@@ -156,7 +156,10 @@ int ios_session_get_output(ios_session *session, float *output);
 /* Dense copy of an operator's output (batch x C x H x W) after a run.  Fails, with a message that says which, for an
  * operator whose output is never written as such (a ReLU applied by the convolution that reads it, a sum added by the
  * depth-wise convolution or the activation that reads it, the convolution and the addition of a residual unit whose result
- * the convolution's epilogue writes) and, under "arena_reuse" = "1", for one whose memory a later operator took over. */
+ * the convolution's epilogue writes) and, under "arena_reuse" = "1", for one whose memory a later operator took over.  The
+ * leading operators of a large batch may have worked on parts of it while the images arrived, and have held some outputs for
+ * one part at a time: asking for one of these runs the pass again on the whole batch, and fails where the input or a weight
+ * has been set since. */
 int ios_session_get_tensor(ios_session *session, const char *node_name, float *output);
 /* Same protocol and outputs as graph_latency, on the resident session. */
 int ios_session_measure(ios_session *session, int warmup, int number, int repeat, int profile_stage_latency,

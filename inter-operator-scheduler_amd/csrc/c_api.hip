@@ -87,7 +87,8 @@ int inference_call(ios::Session::Storage storage, const char *graph_json, int ba
             // the call that allocates nothing takes measured kernel configurations where they are known and measures none
             const bool tune = storage != ios::Session::Storage::Static;
             ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size,
-                                             [&ctx, tune](const ios::ConvProblem &p, int share) { return ctx.choose_launch(p, share, tune); });
+                                             [&ctx, tune](const ios::ConvProblem &p, int share) { return ctx.choose_launch(p, share, tune); },
+                                             ios::InputUse::Once);
             InferencePlan entry;
             entry.key = std::to_string((int)storage) + '/' + std::to_string(batch_size) + '/' + ctx.plan_token();   // (measuring changes it)
             entry.document = graph_json;
@@ -221,8 +222,7 @@ int ios_plan_describe(const char *graph_json, int batch_size, char *buf, int cap
     guarded([&]() {
         const ios::Json doc = ios::Json::parse(graph_json);
         // host-only: the closed-form configuration model for a 256-CU device, no device is touched
-        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size,
-                                         host_chooser());
+        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, host_chooser(), ios::InputUse::InParts);
         const std::string text = ios::describe_plan(plan);
         needed = (int)text.size();
         if (buf != nullptr && cap > needed) memcpy(buf, text.c_str(), text.size() + 1);
@@ -234,8 +234,7 @@ long long ios_plan_arena_bytes(const char *graph_json, int batch_size) {
     long long bytes = -1;
     guarded([&]() {
         const ios::Json doc = ios::Json::parse(graph_json);
-        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size,
-                                         host_chooser());
+        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, host_chooser(), ios::InputUse::InParts);
         bytes = (long long)(plan.arena_floats * sizeof(float));
     });
     return bytes;
@@ -245,7 +244,7 @@ ios_session *ios_session_create(const char *graph_json, int batch_size) {
     SessionBox *box = nullptr;
     const int status = guarded([&]() {
         const ios::Json doc = ios::Json::parse(graph_json);
-        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, device_chooser());
+        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, device_chooser(), ios::InputUse::InParts);
         box = new SessionBox();
         box->description = ios::describe_plan(plan);
         box->session.reset(new ios::Session(std::move(plan), /*shared=*/false));

@@ -53,7 +53,7 @@ public:
     static constexpr size_t kPart = size_t(4) << 20;      // bytes per staging buffer of the ring, and per step of a large transfer
     static constexpr int kParts = 4;
     static constexpr int kMaxChunks = 5;                  // steps in which a batch arrives (the copy engine takes 25-35 us from one to the next)
-    static constexpr size_t kBatch = size_t(256) << 20;   // largest transfer that is staged as a whole (or one image)
+    static constexpr size_t kBatch = kStagedBytes;        // largest transfer that is staged as a whole (or one image)
     static constexpr size_t kChunk = size_t(64) << 10;   // bytes of the result that are announced together
     static constexpr size_t kAlone = 3 * kChunk;          // results up to this size are fetched by one thread
     static constexpr size_t kResult = kDeliveredFloats * sizeof(float);   // largest result a pass delivers to host memory by itself

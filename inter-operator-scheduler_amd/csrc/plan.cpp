@@ -79,7 +79,7 @@ int act_code(const std::string &name) {
 
 class Planner {
 public:
-    Planner(int batch, const LaunchChooser &chooser) : batch_(batch), chooser_(chooser) {
+    Planner(int batch, const LaunchChooser &chooser, InputUse input) : batch_(batch), input_use_(input), chooser_(chooser) {
         if (batch < 1) throw std::runtime_error("batch size must be positive");
         plan_.batch = batch;
     }
@@ -556,13 +556,19 @@ private:
     static constexpr size_t kRegionTag = size_t(1) << 62;
     struct Region {
         size_t voff, floats;
+        size_t exact = 0;                 // floats before rounding up
         int first = INT_MAX, last = -1;   // stages that touch it
         bool pinned = false;              // lives for the whole pass (inputs, the result)
         size_t at = 0;                    // final offset
+        // The same where the pass works on parts of the batch: the parts take the stages of the prefix one after the other, so
+        // that these count as often as there are parts.
+        int part_first = INT_MAX, part_last = -1;
+        int held = -1;                    // region that holds this tensor for a part at a time
     };
     size_t reserve_region(size_t floats, bool pinned = false) {
         Region r;
         r.voff = region_floats_;
+        r.exact = floats;
         r.floats = (std::max<size_t>(floats, 1) + 63) & ~size_t(63);
         r.pinned = pinned;
         region_floats_ += r.floats;
@@ -594,13 +600,13 @@ private:
         v.base = placed(v.base);
     }
 
-    // The prefix ends where its work covers the time the input takes on the link (57 GB/s measured), both estimated: 100 TFLOP/s
+    // Leading stages whose work covers the time the input takes on the link (57 GB/s measured), both estimated: 100 TFLOP/s
     // and 3.5 TB/s are what the kernels of these layers reach at the batches in question.
-    void choose_prefix() {
+    int choose_prefix() {
         constexpr double kMinBytes = 2 << 20;
         const double input = 4.0 * batch_ * (double)plan_.input.image_floats();
-        plan_.prefix_stages = 0;
-        if (batch_ < 16 || input < kMinBytes) return;
+        if (input_use_ != InputUse::InParts || batch_ < 16 || input < kMinBytes || input > (double)kStagedBytes) return 0;
+        int stages = 0;
         double covered = 0.0;
         for (const auto &groups : plan_.stages) {
             if (groups.size() != 1 || covered > 1.2 * input / 57e9) break;
@@ -612,40 +618,33 @@ private:
                 covered += std::max(op.flops / 100e12, op.bytes / 3.5e12);
             }
             if (!plain) break;
-            plan_.prefix_stages++;
+            stages++;
         }
+        return stages;
     }
 
-    // Lifetimes from the stages of the operations that read or write a region; then first-fit placement, largest regions
-    // first, where two regions may share addresses when their lifetimes do not intersect (all operations of a stage have
-    // finished before the next stage starts, under every executor); finally every offset of the plan is rewritten.
-    void place_regions() {
-        const int last_stage = (int)plan_.stages.size() - 1;
-        for (const PlanOp &op : plan_.ops) {
-            touch(op.in.offset, op.stage);
-            touch(op.out.offset, op.stage);
-            for (const ViewRef &v : op.srcs) touch(v.offset, op.stage);
-            if (op.has_residual) touch(op.residual.offset, op.stage);
-            if (op.conv >= 0 && plan_.convs[op.conv].ws_floats > 0) touch(plan_.convs[op.conv].ws_off, op.stage);
-        }
-        choose_prefix();
-        if (plan_.prefix_stages > 0) plan_.landing_off = reserve_region((size_t)batch_ * plan_.input.image_floats(), /*pinned=*/true);
-        for (const PlanOp &op : plan_.ops) {   // parts of the batch are in different stages of the prefix at the same time
-            if (op.stage >= plan_.prefix_stages) continue;
-            for (int stage : {0, plan_.prefix_stages - 1}) {
-                touch(op.in.offset, stage);
-                touch(op.out.offset, stage);
-            }
-        }
-        if (Region *r = region_of(plan_.output.offset)) r->pinned = true;
-        const bool reuse = planner_arena_reuse();
-        for (Region &r : regions_)
-            if (r.pinned || !reuse || r.last < 0) {   // (an untouched region belongs to an operator nobody reads: keep it apart)
-                r.first = 0;
-                r.last = last_stage;
-            }
+    // A small first part, so that work starts early, and a small last one, so that little of it is left when the link is done;
+    // every part costs the copy engine 25 to 35 us, and kernels on a few images fill the device badly.  Inception-v3, against two
+    // halves: batch 64 6.68 -> 6.54 ms in fp32, 4.45 -> 4.11 ms in bfloat16 (four equal parts: 4.17); batch 16, 17 MB, 2.32 -> 2.28 ms
+    // with three parts (2.33 with five).
+    std::vector<int> choose_parts() const {
+        std::vector<int> ends;
+        auto part = [&](int of64) {
+            const int end = (batch_ * of64 + 63) / 64;
+            if (ends.empty() || end > ends.back()) ends.push_back(end);
+        };
+        if (4 * batch_ * plan_.input.image_floats() >= (size_t(32) << 20))
+            for (int of64 : {8, 22, 38, 52, 64}) part(of64);
+        else
+            for (int of64 : {12, 32, 64}) part(of64);
+        return ends;
+    }
+
+    // First-fit placement of the first `count` regions, largest first: two may share addresses when they are never alive at the
+    // same time, neither in a pass on the whole batch nor in one on parts of it.  Returns the floats they take.
+    size_t lay_out(size_t count) {
         std::vector<Region *> order;
-        for (Region &r : regions_) order.push_back(&r);
+        for (size_t i = 0; i < count; i++) order.push_back(&regions_[i]);
         std::stable_sort(order.begin(), order.end(), [](const Region *a, const Region *b) { return a->floats > b->floats; });
         std::vector<Region *> done;
         size_t extent = 0;
@@ -653,7 +652,8 @@ private:
             // candidate offsets: 0 and the end of every placed region that is alive at the same time
             std::vector<std::pair<size_t, size_t>> busy;   // [begin, end) of conflicting regions
             for (Region *o : done)
-                if (o->first <= r->last && r->first <= o->last) busy.push_back({o->at, o->at + o->floats});
+                if ((o->first <= r->last && r->first <= o->last) || (o->part_first <= r->part_last && r->part_first <= o->part_last))
+                    busy.push_back({o->at, o->at + o->floats});
             std::sort(busy.begin(), busy.end());
             size_t at = 0;
             for (const auto &b : busy) {
@@ -664,9 +664,72 @@ private:
             extent = std::max(extent, at + r->floats);
             done.push_back(r);
         }
-        const size_t base = plan_.arena_floats;
-        plan_.persistent_floats = base;
+        return extent;
+    }
+
+    // What a pass on parts of the batch needs beyond the regions of a pass on the whole batch.  A tensor that outlives the prefix
+    // is filled part by part: it is alive from the first stage on.  One that does not is held for one part at a time, in a region
+    // of that size.  (Inception-v3 at batch 64: 1492 MB with all of them whole, 866 MB this way, 797 MB without a prefix.)
+    void plan_parts(int stages, bool reuse) {
+        plan_.part_ends = choose_parts();
+        int most = 0;
+        for (size_t i = 0; i < plan_.part_ends.size(); i++) most = std::max(most, plan_.part_ends[i] - (i ? plan_.part_ends[i - 1] : 0));
+        plan_.landing_off = reserve_region((size_t)batch_ * plan_.input.image_floats(), /*pinned=*/true);
+        const int last_stage = (int)plan_.stages.size() - 1;
+        regions_.back().first = regions_.back().part_first = 0;
+        regions_.back().last = regions_.back().part_last = last_stage;
+        std::set<size_t> partial_tiles;   // (alive in the stage of their convolution, whatever the part)
+        for (const PlanConv &c : plan_.convs)
+            if (c.ws_floats > 0) partial_tiles.insert(c.ws_off);
+        for (size_t i = 0, n = regions_.size(); i < n; i++) {
+            if (regions_[i].pinned || !reuse || regions_[i].first >= stages || partial_tiles.count(regions_[i].voff | kRegionTag)) continue;
+            if (regions_[i].last >= stages) {
+                regions_[i].part_first = 0;
+                continue;
+            }
+            const int first = regions_[i].first, last = regions_[i].last;
+            reserve_region(regions_[i].exact / (size_t)batch_ * (size_t)most);
+            Region &held = regions_.back();
+            held.part_first = first;
+            held.part_last = last;
+            regions_[i].part_first = INT_MAX;
+            regions_[i].part_last = -1;
+            regions_[i].held = (int)regions_.size() - 1;
+        }
+        plan_.prefix_stages = stages;
+    }
+
+    // Lifetimes from the stages of the operations that read or write a region; then placement, where two regions may share addresses
+    // when their lifetimes do not intersect (all operations of a stage have finished before the next stage starts, under every
+    // executor); finally every offset of the plan is rewritten.
+    void place_regions() {
+        const int last_stage = (int)plan_.stages.size() - 1;
+        for (const PlanOp &op : plan_.ops) {
+            touch(op.in.offset, op.stage);
+            touch(op.out.offset, op.stage);
+            for (const ViewRef &v : op.srcs) touch(v.offset, op.stage);
+            if (op.has_residual) touch(op.residual.offset, op.stage);
+            if (op.conv >= 0 && plan_.convs[op.conv].ws_floats > 0) touch(plan_.convs[op.conv].ws_off, op.stage);
+        }
+        if (Region *r = region_of(plan_.output.offset)) r->pinned = true;
+        if (Region *r = region_of(plan_.input.offset)) r->first = 0;   // (there before the pass)
+        const bool reuse = planner_arena_reuse();
+        for (Region &r : regions_) {
+            if (r.pinned || !reuse || r.last < 0) {   // (an untouched region belongs to an operator nobody reads: keep it apart)
+                r.first = 0;
+                r.last = last_stage;
+            }
+            r.part_first = r.first;
+            r.part_last = r.last;
+        }
+        const size_t base = plan_.arena_floats, whole = regions_.size();
         plan_.activation_floats_without_reuse = region_floats_;
+        size_t extent = lay_out(whole);
+        if (const int stages = choose_prefix()) {
+            plan_parts(stages, reuse);
+            extent = lay_out(regions_.size());
+        }
+        plan_.persistent_floats = base;
         for (Region &r : regions_) r.at += base;
         // (16-byte loads of a pixel's last channels may run past the end of a tensor: the arena ends in padding so that such a read
         // stays inside the allocation)
@@ -675,13 +738,30 @@ private:
         for (auto &entry : plan_.tensors) {
             const Region *r = region_of(entry.second.offset);
             if (r == nullptr) continue;
-            for (const Region &o : regions_)
+            if (r->held >= 0) plan_.in_parts.insert(entry.first);
+            for (size_t i = 0; i < whole; i++) {
+                const Region &o = regions_[i];
                 if (&o != r && o.first > r->last && o.at < r->at + r->floats && r->at < o.at + o.floats) {
                     plan_.overwritten.insert(entry.first);
                     break;
                 }
+            }
         }
+        auto part_view = [&](const ViewRef &v, ViewRef &part, bool &whole_batch) {
+            const Region *r = region_of(v.offset);
+            part = v;
+            place(part);
+            whole_batch = r->held < 0;
+            if (whole_batch) return;
+            const Region &held = regions_[r->held];
+            part.base = part.base - r->at + held.at;
+            part.offset = part.offset - r->at + held.at;
+        };
         for (PlanOp &op : plan_.ops) {
+            if (op.stage < plan_.prefix_stages) {
+                part_view(op.in, op.part_in, op.part_in_whole);
+                part_view(op.out, op.part_out, op.part_out_whole);
+            }
             place(op.in);
             place(op.out);
             for (ViewRef &v : op.srcs) place(v);
@@ -697,7 +777,7 @@ private:
 
     void allocate_outputs() {
         for (PNode &n : nodes_)
-            if (n.own) n.own_offset = reserve_region((size_t)batch_ * n.H * n.W * padded_channels(n.C), /*pinned=*/n.type == NodeType::Placeholder);
+            if (n.own) n.own_offset = reserve_region((size_t)batch_ * n.H * n.W * padded_channels(n.C), /*pinned=*/n.type == NodeType::Placeholder && input_use_ != InputUse::Once);
     }
 
     ViewRef view_of(int index) const {
@@ -1098,6 +1178,7 @@ private:
     }
 
     int batch_;
+    InputUse input_use_;
     int level_unit_ = -2, level_base_ = 0, level_top_ = 0;   // PlanOp::level of the operations being emitted
     const LaunchChooser &chooser_;
     Plan plan_;
@@ -1163,8 +1244,8 @@ long long planner_thin_conv_min_pixels() { return g_thin_conv_min_pixels; }
 int planner_host_split_k() { return g_host_split_k; }
 bool planner_commute_pool_conv() { return g_commute_pool_conv; }
 
-Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser) {
-    Planner planner(batch, chooser);
+Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input) {
+    Planner planner(batch, chooser, mode == PlanMode::Graph ? input : InputUse::Resident);
     return planner.run(mode, doc, extra);
 }
 
@@ -1218,6 +1299,17 @@ std::string describe_plan(const Plan &plan) {
         if (op.has_residual) reads.push_back(op.residual);
         ranges("writes", {op.out});
         ranges("reads", reads);
+        if (op.stage < plan.prefix_stages) {   // the same for a pass on parts of the batch: [first image, floats per image, whole batch]
+            auto part = [&](const char *key, const ViewRef &v, bool whole) {
+                os << ",\"" << key << "\":[" << v.offset << ',' << v.bstride << ',' << (whole ? "true" : "false") << ']';
+            };
+            part("part_reads", op.part_in, op.part_in_whole);
+            part("part_writes", op.part_out, op.part_out_whole);
+            os << ",\"landing\":[" << plan.landing_off << ',' << plan.landing_off + (size_t)plan.batch * plan.input.image_floats() << ']';
+            os << ",\"part_ends\":[";
+            for (size_t p = 0; p < plan.part_ends.size(); p++) os << (p ? "," : "") << plan.part_ends[p];
+            os << ']';
+        }
         // a split-K convolution first writes, then reads its partial tiles: a region that shares addresses with other tensors
         // like any other
         if (op.conv >= 0 && plan.convs[op.conv].ws_floats > 0) {

@@ -24,6 +24,7 @@ namespace ios {
 
 constexpr int kMaxGroups = 16;   // concurrent groups (streams) per stage
 constexpr int kMaxExtent = 1 << 16;     // image sides, filter sides, strides and padding a document may ask for
+constexpr size_t kStagedBytes = size_t(256) << 20;   // largest transfer that is staged as a whole
 constexpr size_t kDeliveredFloats = size_t(1) << 20;   // largest result that a pass writes to host memory by itself
 constexpr int kMaxChannels = 1 << 20;   // channels of a tensor
 
@@ -86,6 +87,10 @@ struct PlanOp {
     bool has_residual = false;
     ViewRef residual;
     int post_relu = 0;
+    // Where the operation reads and writes when the pass works on parts of the batch (operations of Plan::prefix_stages): a tensor
+    // of the whole batch, or one that holds a part at a time.
+    ViewRef part_in, part_out;
+    bool part_in_whole = true, part_out_whole = true;
     double flops = 0.0, bytes = 0.0;
 };
 
@@ -109,12 +114,20 @@ struct Plan {
     std::set<std::string> overwritten;
     bool output_single_group = true;                     // the last stage has one group
     // Leading stages of one group that may run on a part of the batch at a time, while the images behind it are still on their
-    // way to the device (0: the input is too small for that); their tensors share no memory with each other.
+    // way to the device (0: the input is too small for that, or the plan is not for a session that is given its input while it
+    // works).  A tensor that only these stages read is then held for one part at a time: `in_parts` names the operators whose
+    // output no pass on parts leaves as a whole.
     int prefix_stages = 0;
-    size_t landing_off = 0;   // where the images of a plan with a prefix land, in the host's layout
+    std::vector<int> part_ends;   // images up to the end of each part
+    size_t landing_off = 0;       // where the images of a plan with a prefix land, in the host's layout
+    std::set<std::string> in_parts;
 };
 
 enum class PlanMode { Graph, Block, Stage };
+
+// Resident: the input stays where it is for any number of passes.  InParts: the same, and it may arrive while the first stages work
+// (Plan::prefix_stages).  Once: every pass is given its input, whose memory is free once its last reader has run.
+enum class InputUse { Resident, InParts, Once };
 
 // Picks the kernel configuration of a matrix-path convolution (closed-form model or measured).  `share` is the
 // number of groups that run concurrently in the convolution's stage: a kernel that shares the device with
@@ -124,7 +137,7 @@ typedef std::function<ConvLaunch(const ConvProblem &, int share)> LaunchChooser;
 // Compile a document.  `extra` is the input-shape document of stage mode ({name: [C, H, W]}).
 // Throws std::runtime_error on malformed documents, unknown operator types, non-topological schedules
 // and stages with too many groups.
-Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser);
+Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input = InputUse::Resident);
 
 std::string describe_plan(const Plan &plan);   // JSON array, one object per op
 

@@ -209,6 +209,8 @@ private:
     bool static_ = false;
     std::vector<char> packed_;      // per convolution: its packed filters are laid out
     std::vector<int> arriving_;     // parts of the input on their way: images up to the end of each
+    bool ran_in_parts_ = false;     // the last pass worked on parts of the batch as they arrived
+    bool input_changed_ = false;    // the input or a weight has been set since the last pass
     bool advance_ = false;          // set_conv_weights issues the stages whose filters it has packed
     size_t next_stage_ = 0;
     bool fetches_result_ = true;    // the caller has fetched the last result (or there was none): the next pass delivers its own

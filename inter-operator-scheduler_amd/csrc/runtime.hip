@@ -603,26 +603,15 @@ void Session::set_input(const float *host) {
     if (host == nullptr) throw std::runtime_error("input pointer is null");
     const TensorView in = tv(plan_.input);
     hipStream_t main = ctx_.stream(0);
-    if (plan_.prefix_stages > 0 && !static_ && plan_.batch * plan_.input.image_floats() * sizeof(float) <= HostStage::kBatch) {
+    input_changed_ = true;
+    if (plan_.prefix_stages > 0) {
         // the first stages of the next pass start on the images that are there while the others are still on their way
         const size_t image = plan_.input.image_floats() * sizeof(float);
         arriving_.clear();
         std::vector<size_t> ends;
-        auto part = [&](int of64) {
-            const int end = (plan_.batch * of64 + 63) / 64;
-            if (!arriving_.empty() && end <= arriving_.back()) return;
-            arriving_.push_back(end);
-            ends.push_back(end * image);
-        };
-        // A small first part, so that work starts early, and a small last one, so that little of it is left when the link is
-        // done; every part costs the copy engine 25 to 35 us, and kernels on a few images fill the device badly.  Inception-v3,
-        // against two halves: batch 64 6.68 -> 6.54 ms in fp32, 4.45 -> 4.11 ms in bfloat16 (four equal parts: 4.17); batch 16,
-        // 17 MB, 2.32 -> 2.28 ms with three parts (2.33 with five).
-        if (plan_.batch * image >= (size_t(32) << 20))
-            for (int of64 : {8, 22, 38, 52, 64}) part(of64);
-        else
-            for (int of64 : {12, 32, 64}) part(of64);
+        for (int end : plan_.part_ends) ends.push_back(end * image);
         ctx_.stage().upload_chunks(base_ + plan_.landing_off, host, ends, ctx_.stream(1), main);
+        arriving_ = plan_.part_ends;
         return;
     }
     arriving_.clear();
@@ -648,6 +637,7 @@ void Session::settle() {
 // by several threads and travel in large steps, on a stream of their own; the filters of a convolution are packed on the main
 // stream as soon as they have arrived.
 void Session::set_conv_weights(int count, char **names, float **weights, float **biases) {
+    input_changed_ = true;
     std::vector<int> entry(plan_.convs.size(), -1);   // a name given twice: the last one counts
     for (int i = 0; i < count; i++) {
         auto it = plan_.conv_index.find(names[i] ? names[i] : "");
@@ -704,6 +694,12 @@ void Session::get_tensor(const std::string &name, float *host) {
     if (plan_.overwritten.count(name))
         throw std::runtime_error("the output of operator '" + name + "' shares its memory with a later operator and does not survive the pass "
                                  "(option arena_reuse=0 keeps every output)");
+    if (ran_in_parts_ && plan_.in_parts.count(name)) {   // never whole in that pass: the same pass on the whole batch
+        if (input_changed_)
+            throw std::runtime_error("the last pass worked on parts of the batch, held the output of operator '" + name + "' for one part at a time, and its "
+                                     "input or weights have changed since (option arena_reuse=0 keeps every output)");
+        forward();
+    }
     copy_out(it->second, host);
 }
 
@@ -715,18 +711,20 @@ unsigned *Session::counters_of(const PlanConv &c) const {
 void Session::launch_op(const PlanOp &op, int group, int first, int images) {
     hipStream_t stream = ctx_.stream(group);
     const int count = images > 0 ? images : plan_.batch;
-    auto part = [&](const ViewRef &v) {   // the images this launch works on
-        TensorView t = tv(v);
-        t.ptr += (long long)first * v.H * v.W * v.pstride;
+    auto part = [&](const ViewRef &whole_view, const ViewRef &part_view, bool whole) {   // the images this launch works on
+        if (images <= 0) return tv(whole_view);
+        TensorView t = tv(part_view);
+        if (whole) t.ptr += (long long)first * t.H * t.W * t.pstride;
         return t;
     };
+    const TensorView in = part(op.in, op.part_in, op.part_in_whole), out = part(op.out, op.part_out, op.part_out_whole);
     switch (op.kind) {
         case OpKind::ConvMfma: {
             const PlanConv &c = plan_.convs[op.conv];
             ConvProblem p = c.problem;
             p.B = count;
-            const TensorView residual = op.has_residual ? part(op.residual) : TensorView{};
-            launch_conv_mfma(p, c.launch, part(op.in), base_ + c.packed_off, bias_of(c), part(op.out),
+            const TensorView residual = op.has_residual ? tv(op.residual) : TensorView{};
+            launch_conv_mfma(p, c.launch, in, base_ + c.packed_off, bias_of(c), out,
                              c.ws_floats ? base_ + c.ws_off : nullptr, ctx_.split_reduce(counters_of(c), group, !capturing_forks_), stream,
                              op.has_residual ? &residual : nullptr,
                              op.post_relu != 0);
@@ -737,8 +735,8 @@ void Session::launch_op(const PlanOp &op, int group, int first, int images) {
             ConvProblem p = c.problem;
             p.B = count;
             TensorView more[kMaxNaryInputs];
-            for (size_t i = 1; i < op.srcs.size(); i++) more[i - 1] = part(op.srcs[i]);
-            launch_dwconv(p, part(op.in), base_ + c.packed_off, bias_of(c), part(op.out), stream, more,
+            for (size_t i = 1; i < op.srcs.size(); i++) more[i - 1] = tv(op.srcs[i]);
+            launch_dwconv(p, in, base_ + c.packed_off, bias_of(c), out, stream, more,
                           op.srcs.empty() ? 0 : (int)op.srcs.size() - 1);
             break;
         }
@@ -746,28 +744,28 @@ void Session::launch_op(const PlanOp &op, int group, int first, int images) {
             const PlanConv &c = plan_.convs[op.conv];
             ConvProblem p = c.problem;
             p.B = count;
-            launch_conv_direct(p, part(op.in), base_ + c.weight_off, bias_of(c), part(op.out), stream, c.thin);
+            launch_conv_direct(p, in, base_ + c.weight_off, bias_of(c), out, stream, c.thin);
             break;
         }
         case OpKind::Pool:
         case OpKind::GlobalPool: {
             PoolProblem p = op.pool;
             p.B = count;
-            if (op.kind == OpKind::GlobalPool) launch_global_pool(p, part(op.in), part(op.out), stream);
-            else launch_pool(p, part(op.in), part(op.out), stream, op.bias_conv >= 0 ? base_ + plan_.convs[op.bias_conv].bias_off : nullptr, op.act);
+            if (op.kind == OpKind::GlobalPool) launch_global_pool(p, in, out, stream);
+            else launch_pool(p, in, out, stream, op.bias_conv >= 0 ? base_ + plan_.convs[op.bias_conv].bias_off : nullptr, op.act);
             break;
         }
         case OpKind::Nary: {
             NaryArgs a;
             a.count = (int)op.srcs.size();
             for (int i = 0; i < a.count; i++) {
-                a.src[i] = part(op.srcs[i]).ptr;
+                a.src[i] = tv(op.srcs[i]).ptr;
                 a.src_pstride[i] = op.srcs[i].pstride;
             }
-            launch_nary(a, op.multiply, op.accumulate, op.act, count, part(op.out), stream);
+            launch_nary(a, op.multiply, op.accumulate, op.act, count, out, stream);
             break;
         }
-        case OpKind::Unary: launch_unary(part(op.in), part(op.out), op.act, count, stream); break;
+        case OpKind::Unary: launch_unary(in, out, op.act, count, stream); break;
     }
 }
 
@@ -819,13 +817,16 @@ void Session::enqueue(size_t first, bool stage_events) {
 
 // The leading stages, of one group each: on the whole batch, or part by part as the images arrive.
 void Session::enqueue_prefix(size_t stages) {
-    if (arriving_.empty() || plan_.prefix_stages == 0) {
+    input_changed_ = false;
+    ran_in_parts_ = !arriving_.empty() && plan_.prefix_stages > 0;
+    if (!ran_in_parts_) {
         settle();
         for (size_t s = 0; s < stages; s++) enqueue_stage(s);
         return;
     }
     const size_t split = (size_t)plan_.prefix_stages;
     int begin = 0;
+    // (a part's stages follow those of the part before it: they write over the tensors that hold one part at a time)
     for (size_t part = 0; part < arriving_.size(); part++) {
         const int images = arriving_[part] - begin;
         take_images(begin, images, (int)part);

@@ -121,3 +121,82 @@ def test_large_results_of_several_images(batch, shape):
         assert np.array_equal(session.output(), want)
         assert np.array_equal(session.tensor(a.node), want[:, :shape[0]])
         assert np.array_equal(session.tensor(b.node), want[:, shape[0]:])
+
+
+# three parts; five parts, which take 32 MB and more
+@pytest.mark.parametrize('batch,side', [(17, 161), (64, 225), (61, 231)])
+@pytest.mark.parametrize('executor', ['fused', 'fused_graph'])
+def test_tensors_of_a_batch_that_arrived_in_parts(batch, side, executor):
+    """The result and every tensor that can be asked for, among them those that a pass on parts holds for one part at a time."""
+    rt.set_option('executor', executor)
+    rt.set_option('autotune', 0)
+    try:
+        ios.reset_name()
+        v = ios.placeholder((3, side, side - 2))
+        block = ios.Block(v.node)
+        a = ios.conv2d(block, [[v]], 19, (3, 3), (2, 2))
+        b = ios.pool2d(block, [[a]], 'max', (3, 3), (1, 1), (1, 1))
+        c = ios.conv2d(block, [[a], [b]], 26, (3, 3), (2, 2))
+        d = ios.conv2d(block, [[c]], 33, (3, 3), (1, 1), (1, 1))
+        ios.pool2d(block, [[d], [c]], 'global_avg', is_exit=True)
+        graph = Graph('t', v.node, [block])
+        graph.init_weights(seed=1, scheme='he_normal_bias')
+        graph.sequential_schedule()
+        parts = [op['part_ends'] for op in rt.plan_describe(graph, batch) if 'part_ends' in op]
+        assert parts and len(parts[0]) == (5 if batch * 3 * side * (side - 2) >= 8 << 20 else 3)
+        with rt.Session(graph, batch) as session, rt.Session(graph, 1) as single:
+            session.load_weights()
+            single.load_weights()
+            x = np.random.default_rng(batch).standard_normal(session.input_shape, dtype=np.float32)
+            for step in range(2):
+                x = x[::-1].copy()
+                session.set_input(x)
+                session.run()
+                got = session.output()
+                asked = 0
+                for value in (a, b, c, d):
+                    try:
+                        tensor = session.tensor(value.node)
+                    except RuntimeError as e:
+                        assert 'shares its memory' in str(e)
+                        continue
+                    asked += 1
+                    for i in (0, batch // 3, batch - 1):
+                        single.set_input(x[i:i + 1])
+                        single.run()
+                        try:
+                            assert np.allclose(tensor[i:i + 1], single.tensor(value.node), rtol=1e-4, atol=1e-5)
+                        except RuntimeError as e:
+                            assert 'shares its memory' in str(e)
+                        assert np.allclose(got[i:i + 1], single.output(), rtol=1e-4, atol=1e-5)
+                assert asked > 0 and np.array_equal(got, session.output())
+                session.run()   # the same input again, now resident
+                assert np.array_equal(got, session.output())
+            # an input that no pass has worked on: tensors of the last pass are there or are refused, the result is the last pass's
+            session.set_input(-x)
+            session.run()
+            negative = session.output()
+            session.set_input(x)
+            for value in (a, b, c, d):
+                try:
+                    session.tensor(value.node)
+                except RuntimeError as e:
+                    assert 'shares its memory' in str(e) or 'changed since' in str(e)
+            assert np.array_equal(negative, session.output())
+            session.run()
+            assert np.array_equal(got, session.output())
+    finally:
+        rt.set_option('executor', 'fused')
+        rt.set_option('autotune', 1)
+
+
+def test_an_input_beyond_the_staging_buffer():
+    """335 MB go through the 256 MB buffer in two groups of images."""
+    session = rt.Session(relu_graph(1, 4096, 4096), 5)
+    x = np.random.default_rng(5).standard_normal(session.input_shape, dtype=np.float32)
+    for _ in range(2):
+        x = -x
+        session.set_input(x)
+        session.run()
+        assert np.array_equal(session.output(), np.maximum(x, 0))
+    session.close()

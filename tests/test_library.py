@@ -543,3 +543,102 @@ def test_a_large_result_is_laid_out_once(shape, batch):
     channels = (shape[0] + 3) // 4 * 4
     tensor = 4 * batch * channels * shape[1] * shape[2]
     assert rt.plan_arena_bytes(graph, batch) <= 2 * tensor + 4 * batch * int(np.prod(shape)) // 2 + 1024
+
+
+def _simulate_parts(ops, batch):
+    """
+    A pass on parts of the batch on an arena that remembers, for every float, which operation wrote it for which image.  Returns
+    what every operation read, per image.
+    """
+    prefix = [op for op in ops if 'part_ends' in op]
+    ends, landing = prefix[0]['part_ends'], prefix[0]['landing']
+    extent = max([landing[1]] + [stop for op in ops for key in ('reads', 'writes', 'scratch') for _, stop in op.get(key, [])] +
+                 [op[key][0] + batch * op[key][1] for op in prefix for key in ('part_reads', 'part_writes')])
+    writer = np.full(extent, -1, np.int32)
+    seen = {}
+
+    def read(index, image, begin, stop):
+        seen.setdefault((index, image), set()).update(np.unique(writer[begin:stop]).tolist())
+
+    image_floats = (landing[1] - landing[0]) // batch
+    for n in range(batch):
+        writer[landing[0] + n * image_floats:landing[0] + (n + 1) * image_floats] = 100000000 + n
+    first_in, _, whole = prefix[0]['part_reads']
+    assert whole
+    begin_image = 0
+    for end_image in ends:
+        for n in range(begin_image, end_image):
+            found = np.unique(writer[landing[0] + n * image_floats:landing[0] + (n + 1) * image_floats])
+            assert found.tolist() == [100000000 + n]
+            begin, stop = ops[0]['reads'][n]
+            writer[begin:stop] = 200000000 + n
+        for index, op in enumerate(ops):
+            if 'part_ends' not in op:
+                continue
+            for begin, stop in op.get('scratch', []):
+                writer[begin:stop] = -2
+            for key in ('part_reads', 'part_writes'):
+                at, stride, whole = op[key]
+                floats = op[key[5:]][0][1] - op[key[5:]][0][0]
+                for n in range(begin_image, end_image):
+                    begin = at + (n if whole else n - begin_image) * stride
+                    if key == 'part_reads':
+                        read(index, n, begin, begin + floats)
+                    else:
+                        writer[begin:begin + floats] = index * 1000 + n
+        begin_image = end_image
+    assert begin_image == batch
+    for index, op in enumerate(ops):
+        if 'part_ends' in op:
+            continue
+        for begin, stop in op.get('scratch', []):
+            writer[begin:stop] = -2
+        for i, (begin, stop) in enumerate(op['reads']):
+            read(index, i % batch, begin, stop)
+        for i, (begin, stop) in enumerate(op['writes']):
+            writer[begin:stop] = index * 1000 + i % batch
+    # the input and what landed are whole at the end
+    for n, (begin, stop) in enumerate(ops[0]['reads']):
+        assert np.unique(writer[begin:stop]).tolist() == [200000000 + n]
+    assert (writer[landing[0]:landing[1]] >= 100000000).all() and (writer[landing[0]:landing[1]] < 200000000).all()
+    return seen
+
+
+def _branching_front(channels):
+    """A concatenation of a convolution and a pool among the leading stages, read by two operators."""
+    ios.reset_name()
+    v = ios.placeholder((3, 131, 127))
+    block = Block(v.node)
+    a = ios.conv2d(block, [[v]], channels, (3, 3), (1, 1), (1, 1))
+    b = ios.pool2d(block, [[a]], 'max', (3, 3), (1, 1), (1, 1))
+    both = ios.identity(block, [[a], [b]])
+    c = ios.conv2d(block, [[both]], 24, (3, 3), (2, 2))
+    d = ios.pool2d(block, [[both]], 'max', (3, 3), (2, 2))
+    e = ios.conv2d(block, [[c], [d]], 40, (5, 5), (1, 1), (2, 2))
+    ios.pool2d(block, [[e], [c]], 'global_avg', is_exit=True)
+    return Graph('t', v.node, [block])
+
+
+@pytest.mark.parametrize('name,batch,split_k', [('front', 16, 0), ('front', 23, 3), ('front', 64, 2), ('squeezenet_1_1', 17, 0)])
+def test_parts_of_a_batch_share_the_arena(name, batch, split_k):
+    """Where the first stages work on parts of the batch, every operation still reads what the operations before it wrote for the
+    same image, and the tensors of one part at a time cost next to no memory."""
+    graph = _branching_front(21) if name == 'front' else getattr(ios.models, name)()
+    graph.sequential_schedule()
+    try:
+        rt.set_option('host_plan_split_k', split_k)
+        ops, arena = rt.plan_describe(graph, batch), rt.plan_arena_bytes(graph, batch)
+        below = rt.plan_arena_bytes(graph, 15)   # the largest batch that arrives as a whole
+        rt.set_option('arena_reuse', 0)
+        plain = rt.plan_describe(graph, batch)
+    finally:
+        rt.set_option('arena_reuse', 1)
+        rt.set_option('host_plan_split_k', 0)
+    prefix = [op for op in ops if 'part_ends' in op]
+    assert len(prefix) >= 2 and any(not op['part_writes'][2] for op in prefix)
+    assert all(op['part_writes'][2] for op in plain if 'part_ends' in op)
+    expected = _simulate_parts(plain, batch)
+    assert -1 not in set().union(*expected.values())
+    assert _simulate_parts(ops, batch) == expected
+    image = 4 * int(np.prod(graph.enter_node.output_shape))
+    assert arena < below * batch / 15 * 1.05 + batch * image

@@ -102,8 +102,11 @@ def test_a_graph_beyond_the_static_array_is_refused_and_the_next_call_works():
     both(sample, 2, seed=4)
 
 
-def test_large_batches_that_fit_the_scratch_are_accepted():
-    """The result of a batch, 2.5 MB an image here, is in the scratch once."""
-    graph = ios.models.sample_network(init_seed=0, init_scheme='he_normal_bias')
-    graph.sequential_schedule()
-    both(graph, 60, 3)
+@pytest.mark.parametrize('name,schedule,batch', [('sample_network', 'sequential', 87), ('squeezenet_1_1', 'sequential', 57), ('inception_v3', 'sequential', 10),
+                                                 ('nasnet_mobile', 'sequential', 54), ('nasnet_mobile', 'greedy', 45),
+                                                 ('randwire_small', 'sequential', 38), ('randwire_small', 'greedy', 27)])
+def test_batches_that_fit_the_scratch(name, schedule, batch):
+    """The tensors of these fill the scratch nearly: it holds the result once, and the input until its last reader has run."""
+    graph = getattr(ios.models, name)(init_seed=0, init_scheme='he_normal_bias')
+    graph.sequential_schedule() if schedule == 'sequential' else graph.greedy_schedule(8)
+    both(graph, batch, 3)
