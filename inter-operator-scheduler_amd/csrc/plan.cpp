@@ -379,10 +379,13 @@ private:
     // output tensor disappear (the reference adds them with a kernel of its own, src/ios/ios_runtime.cu:1047-1057).
     void find_depthwise_sums() {
         // The summing loader addresses every source with 31-bit byte offsets.  Where the sources will live is decided later
-        // (a source may become a window of a wider concatenation buffer), so the test assumes the widest tensor of the graph
-        // as the batch stride; a sum that could exceed the range keeps its own launch and the generic depth-wise path.
-        unsigned long long widest = 0;
-        for (const PNode &n : nodes_) widest = std::max(widest, (unsigned long long)n.C * n.H * n.W);
+        // (a source may become a window of a wider concatenation buffer), so the test assumes the pixels of the widest tensor with
+        // maps of this size; a sum that could exceed the range keeps its own launch and the generic depth-wise path.
+        std::map<std::pair<int, int>, int> widest;   // (H, W) -> elements between pixels
+        for (const PNode &n : nodes_) {
+            int &stride = widest[{n.H, n.W}];
+            stride = std::max(stride, padded_channels(n.C));
+        }
         for (const auto &seq : sequentials_) {
             for (int i = seq.first; i <= seq.second; i++) {
                 PNode &dw = nodes_[i];
@@ -401,7 +404,7 @@ private:
                 }
                 const PNode &f = nodes_[front];
                 if (f.inputs.size() != 1 || f.inputs[0].size() < 2 || f.inputs[0].size() > (size_t)kMaxNaryInputs) continue;
-                if (((unsigned long long)(batch_ - 1) * widest + (unsigned long long)pd.IC * pd.H * pd.W) * 4ull >= (1ull << 31)) continue;
+                if (conv_input_extent(pd, widest.at({pd.H, pd.W})) >= (1ull << 31)) continue;
                 dw.sum_front = front;
                 dw.sum_relu = relu;
                 if (front != i) {

@@ -642,3 +642,25 @@ def test_parts_of_a_batch_share_the_arena(name, batch, split_k):
     assert _simulate_parts(ops, batch) == expected
     image = 4 * int(np.prod(graph.enter_node.output_shape))
     assert arena < below * batch / 15 * 1.05 + batch * image
+
+
+@pytest.mark.parametrize('channels,width,batch,folds', [(5, 5, 100, False), (5, 5, 63, True), (8, 8, 63, True), (8, 8, 64, False),
+                                                        (4, 4, 127, True), (4, 4, 128, False), (4, 9, 100, False), (4, 9, 42, True)])
+def test_sums_beyond_the_offsets_of_the_depthwise_loader_keep_their_launch(channels, width, batch, folds):
+    """The loader's 31-bit offsets count the padding of every pixel; a source may be a window of a wider tensor."""
+    ios.reset_name()
+    v = ios.placeholder((channels, 1024, 1024))
+    block = Block(v.node)
+    a = ios.relu(block, [[v]])
+    b = ios.pool2d(block, [[v]], 'max', (3, 3), (1, 1), (1, 1))
+    d = ios.relu_sep_conv(block, [[a, b]], channels, (3, 3), (1, 1), (1, 1))
+    if width > channels:
+        ios.identity(block, [[d], [a], [ios.conv2d(block, [[v]], width - 2 * channels, (1, 1))]], is_exit=True)
+    else:
+        ios.pool2d(block, [[d]], 'global_avg', is_exit=True)
+    graph = Graph('t', v.node, [block])
+    graph.sequential_schedule()
+    ops = rt.plan_describe(graph, batch)
+    sums = [op for op in ops if op['kind'] == 'conv_depthwise']
+    assert [op['inputs'] for op in sums] == [2 if folds else 1]
+    assert sum(op['kind'] == 'nary' for op in ops) == (0 if folds else 1)
