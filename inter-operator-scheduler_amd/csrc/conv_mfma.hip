@@ -230,8 +230,9 @@ ConvLaunch conv_pick_launch(const ConvProblem &p, int num_cus, bool fusable_only
 }
 
 bool conv_matrix_path_supported(const ConvProblem &p) {
-    // packed filter rows are indexed with 16 bits, input and filter byte offsets with 31 bits
-    const unsigned long long x_bytes = (unsigned long long)p.B * ((p.IC + 3) & ~3) * p.H * p.W * 4ull;
+    // packed filter rows are indexed with 16 bits, input and filter byte offsets with 31 bits (an input of less than 2^30 bytes has
+    // at most 1.6 * 2^30 with its pixels padded, five channels to eight; a window of a wider tensor is checked where it is known)
+    const unsigned long long x_bytes = (unsigned long long)p.B * p.IC * p.H * p.W * 4ull;
     const unsigned long long w_bytes = (unsigned long long)p.groups * p.Kq(128) * p.OCgP() * 4ull;
     // image sides below 2^15 and output planes below 2^23 elements keep the kernels' signed 24-bit index multiplies exact
     return p.Kq(128) < 65536 && p.Npix() < (1LL << 31) && x_bytes < (1ull << 30) && w_bytes < (1ull << 31) && p.H < 32768 && p.W < 32768 &&

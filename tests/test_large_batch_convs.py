@@ -99,3 +99,27 @@ def test_parallel_stage_launches_large_convolutions_by_themselves(precision, key
             got = session.output()
         convs = frozenset(op['node'] for op in session.describe() if op['kind'] == 'conv_mfma')
     assert_close(got, ios_oracle.run(graph, x, **{key: convs}), f'{precision} {executor}')
+
+
+@pytest.mark.parametrize('variant', [None, 'x3p_m64n128_w1x2', 'wq_m64n32_w4_t32', 'm64n64k32_w2x2x1_t32'])
+def test_an_input_of_a_gigabyte(variant):
+    """85 images of 3 x 1024 x 1024: 1.07 GB of values, 1.43 GB with the pixels padded."""
+    if variant is not None:
+        rt.set_option('conv_variant', rt.conv_variant_names().index(variant))
+    ios.reset_name()
+    holder = ios.placeholder((3, 1024, 1024))
+    block = Block(holder.node, None, [], None)
+    ios.conv2d(block, [[holder]], 32, (5, 5), (4, 4), (2, 2), is_exit=True)
+    graph = Graph('gigabyte', holder.node, [block])
+    graph.init_weights(3, 'he_normal_bias')
+    graph.sequential_schedule()
+    x = np.tile(np.random.default_rng(0).standard_normal((5, 3, 1024, 1024), dtype=np.float32), (17, 1, 1, 1))
+    with rt.Session(graph, 85) as session:
+        assert [op['kind'] for op in session.describe()] == ['conv_mfma']
+        session.load_weights()
+        session.set_input(x)
+        session.run()
+        got = session.output()
+    want = ios_oracle.run(graph, x[:5])
+    for image in (0, 1, 42, 63, 83, 84):   # 2^30 bytes of padded pixels end inside image 64
+        assert_close(got[image], want[image % 5], f'image {image}')

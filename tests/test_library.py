@@ -664,3 +664,16 @@ def test_sums_beyond_the_offsets_of_the_depthwise_loader_keep_their_launch(chann
     sums = [op for op in ops if op['kind'] == 'conv_depthwise']
     assert [op['inputs'] for op in sums] == [2 if folds else 1]
     assert sum(op['kind'] == 'nary' for op in ops) == (0 if folds else 1)
+
+
+@pytest.mark.parametrize('channels,batch,kind', [(3, 85, 'conv_mfma'), (3, 86, 'conv_direct'), (5, 51, 'conv_mfma'), (5, 52, 'conv_direct'),
+                                                 (1, 255, 'conv_mfma'), (4, 63, 'conv_mfma'), (4, 64, 'conv_direct')])
+def test_inputs_of_a_gigabyte_stay_on_the_matrix_path(channels, batch, kind):
+    """The limit is 2^30 bytes of values; their padding is inside the kernels' 31-bit offsets."""
+    ios.reset_name()
+    v = ios.placeholder((channels, 1024, 1024))
+    block = Block(v.node)
+    ios.conv2d(block, [[v]], 32, (5, 5), (4, 4), (2, 2), is_exit=True)
+    graph = Graph('t', v.node, [block])
+    graph.sequential_schedule()
+    assert [op['kind'] for op in rt.plan_describe(graph, batch)] == [kind]
