@@ -17,8 +17,10 @@ for src in conv_mfma.hip conv_window.hip pointwise.hip fused.hip fused_512.hip f
     hipcc $FLAGS ${FILE_FLAGS[$src]:-} -Rpass-analysis=kernel-resource-usage -c "$src" -o "build/${src%.hip}.o" 2> "build/${src%.hip}.log" &
     pids+=($!)
 done
-hipcc $FLAGS -x hip -c plan.cpp -o build/plan.o &
-pids+=($!)
+for src in plan.cpp host_copier.cpp; do
+    hipcc $FLAGS -x hip -c "$src" -o "build/${src%.cpp}.o" &
+    pids+=($!)
+done
 status=0
 for pid in "${pids[@]}"; do wait "$pid" || status=1; done
 if [ "$status" -ne 0 ]; then
@@ -30,5 +32,5 @@ if grep -h "ScratchSize \[bytes/lane\]: [1-9]" build/*.log > /dev/null; then
     awk '/Function Name:/ { name = $0; sub(/.*Function Name: /, "", name); sub(/ \[-R.*/, "", name) }
          /ScratchSize \[bytes\/lane\]: [1-9]/ { size = $0; sub(/.*lane\]: /, "", size); sub(/ .*/, "", size); print "  " size "  " name }' build/*.log >&2
 fi
-hipcc --offload-arch=gfx950 -shared -fPIC -o build/libios_runtime.so build/conv_mfma.o build/conv_window.o build/pointwise.o build/fused.o build/fused_512.o build/fused_wide.o build/runtime.o build/host_io.o build/c_api.o build/plan.o
+hipcc --offload-arch=gfx950 -shared -fPIC -o build/libios_runtime.so build/conv_mfma.o build/conv_window.o build/pointwise.o build/fused.o build/fused_512.o build/fused_wide.o build/runtime.o build/host_io.o build/host_copier.o build/c_api.o build/plan.o
 echo "built $(pwd)/build/libios_runtime.so"

@@ -2,14 +2,9 @@
 
 #include <algorithm>
 #include <chrono>
-#include <climits>
 #include <cstring>
 #include <stdexcept>
-#include <thread>
 
-#include <linux/futex.h>
-#include <sys/syscall.h>
-#include <unistd.h>
 #if defined(__x86_64__)
 #include <immintrin.h>
 #endif
@@ -17,111 +12,6 @@
 #include "runtime.h"
 
 namespace ios {
-
-// ---- threads -----------------------------------------------------------------------------------------------------------
-HostCopier &HostCopier::get() {
-    static HostCopier *instance = new HostCopier();
-    return *instance;
-}
-
-static inline void pause() {
-#if defined(__x86_64__)
-    __builtin_ia32_pause();
-#endif
-}
-
-static void futex_wait(std::atomic<unsigned> &word, unsigned value) {
-    syscall(SYS_futex, reinterpret_cast<unsigned *>(&word), FUTEX_WAIT_PRIVATE, value, nullptr, nullptr, 0);
-}
-static void futex_wake(std::atomic<unsigned> &word) {
-    syscall(SYS_futex, reinterpret_cast<unsigned *>(&word), FUTEX_WAKE_PRIVATE, INT_MAX, nullptr, nullptr, 0);
-}
-
-void HostCopier::start() {
-    started_ = true;
-    // three quarters of the processors, twelve threads at most: large copies are bound by memory from there on (69 MB that lie in no
-    // cache: 530 us with 8 threads, 420 with 12 and with 15)
-    const int n = std::min(12, std::max(1, (int)std::thread::hardware_concurrency() * 3 / 4));
-    for (int i = 1; i < n; i++) std::thread([this, i]() { worker(i <= kNear); }).detach();
-}
-
-void HostCopier::worker(bool near) {
-    using clock = std::chrono::steady_clock;
-    std::atomic<unsigned> &calls = near ? near_calls_ : far_calls_;
-    std::atomic<int> &asleep = near ? near_asleep_ : far_asleep_;
-    unsigned seen = 0;
-    for (;;) {
-        const unsigned call = calls.load();
-        unsigned now = generation_.load();
-        if (now == seen && near) {
-            const auto until = clock::now() + std::chrono::microseconds(500);
-            while ((now = generation_.load()) == seen && clock::now() < until)
-                for (int i = 0; i < 32; i++) pause();
-        }
-        if (now == seen) {
-            asleep.fetch_add(1);
-            futex_wait(calls, call);
-            asleep.fetch_sub(1);
-            continue;
-        }
-        seen = now;
-        // either the owner sees this thread in busy_ and waits for it, or this thread sees that the copy is closed
-        busy_.fetch_add(1);
-        if (open_.load() == now)
-            for (int i; (i = next_.fetch_add(1)) < pieces_;) (*body_)(i);
-        busy_.fetch_sub(1);
-    }
-}
-
-void HostCopier::rouse() {
-    if (!started_) start();
-    near_calls_.fetch_add(1);
-    if (near_asleep_.load() > 0) futex_wake(near_calls_);
-}
-
-void HostCopier::parallel(int pieces, bool large, const std::function<void(int)> &body, const std::function<void()> *idle) {
-    if (pieces <= 1) {
-        if (pieces == 1) body(0);
-        if (idle != nullptr) (*idle)();
-        return;
-    }
-    if (!started_) start();
-    next_.store(0);
-    body_ = &body;
-    pieces_ = pieces;
-    unsigned generation = generation_.load() + 1;
-    if (generation == 0) generation = 1;
-    open_.store(generation);
-    generation_.store(generation);
-    near_calls_.fetch_add(1);
-    if (near_asleep_.load() > 0) futex_wake(near_calls_);
-    if (large) {
-        far_calls_.fetch_add(1);
-        if (far_asleep_.load() > 0) futex_wake(far_calls_);
-    }
-    for (int i; (i = next_.fetch_add(1)) < pieces;) {
-        body(i);
-        if (idle != nullptr) (*idle)();
-    }
-    open_.store(0);
-    while (busy_.load() != 0) {
-        if (idle != nullptr) (*idle)();
-        pause();
-    }
-    if (idle != nullptr) (*idle)();
-}
-
-void HostCopier::copy(void *dst, const void *src, size_t bytes) {
-    if (bytes <= kAloneBytes) {
-        memcpy(dst, src, bytes);
-        return;
-    }
-    const size_t piece = std::min(kPiece, std::max(size_t(32) << 10, bytes / 16));
-    parallel((int)((bytes + piece - 1) / piece), bytes >= kLargeBytes, [&](int i) {
-        const size_t at = (size_t)i * piece;
-        memcpy(static_cast<char *>(dst) + at, static_cast<const char *>(src) + at, std::min(piece, bytes - at));
-    });
-}
 
 // Fills a buffer that only the link will read and that is larger than the caches: stores past the caches save reading every
 // line of the buffer first (a third of the copy's memory traffic).
@@ -156,6 +46,18 @@ static void copy_past_caches(char *dst, const char *src, size_t bytes) {
 #endif
     memcpy(dst + done, src + done, bytes - done);
 }
+
+// A transfer that fails midway may have queued steps on `stream` that still read the staging buffers: they end before the buffers
+// are used again.
+namespace {
+struct SettleOnFailure {
+    hipStream_t stream;
+    bool armed = true;
+    ~SettleOnFailure() {
+        if (armed) (void)hipStreamSynchronize(stream);
+    }
+};
+}  // namespace
 
 // ---- pinned buffers ------------------------------------------------------------------------------------------------------
 void HostStage::create() {
@@ -207,6 +109,7 @@ void HostStage::arrived(int chunk, hipStream_t stream) { IOS_HIP(hipStreamWaitEv
 // Kernels read the staging buffer at the link's rate, like the copy engine, turn the images into the layout of views on the
 // way, and follow and precede the kernels of their stream without the hand-over between engines (600 KB: 25 us less per pass).
 void HostStage::upload_images(const TensorView &dst, int batch, const float *src, hipStream_t stream) {
+    SettleOnFailure settle{stream};
     const size_t pixels = (size_t)dst.H * dst.W, image = pixels * dst.C;   // floats
     const int group = (int)std::max<size_t>(1, std::min<size_t>((size_t)batch, kBatch / (image * sizeof(float))));
     struct Step {
@@ -302,9 +205,11 @@ void HostStage::upload_images(const TensorView &dst, int batch, const float *src
         if (ring) used_[turn_] = true;
         else inputs_.used = true;
     }
+    settle.armed = false;
 }
 
 void HostStage::upload_chunks(void *dst, const void *src, const std::vector<size_t> &ends, hipStream_t link, hipStream_t stream) {
+    SettleOnFailure settle{link};
     const int chunks = (int)ends.size();
     if (chunks < 1 || chunks > kMaxChunks) throw std::runtime_error("internal: a batch arrives in too many chunks");
     char *memory = inputs_.take(ends.back());
@@ -336,9 +241,11 @@ void HostStage::upload_chunks(void *dst, const void *src, const std::vector<size
     IOS_HIP(failed);
     IOS_HIP(hipEventRecord(inputs_.drained, link));
     inputs_.used = true;
+    settle.armed = false;
 }
 
 void HostStage::upload_pieces(char *dst, const std::vector<Piece> &all, hipStream_t link, hipStream_t stream, const std::function<void(size_t)> &step) {
+    SettleOnFailure settle{link};
     IOS_HIP(hipEventRecord(order_, stream));   // queued passes read what they were queued with
     IOS_HIP(hipStreamWaitEvent(link, order_, 0));
     for (size_t begin = 0; begin < all.size();) {
@@ -391,9 +298,11 @@ void HostStage::upload_pieces(char *dst, const std::vector<Piece> &all, hipStrea
         weights_.used = true;
         begin = end;
     }
+    settle.armed = false;
 }
 
 void HostStage::upload(void *dst, const void *src, size_t bytes, hipStream_t stream) {
+    SettleOnFailure settle{stream};
     for (size_t at = 0; at < bytes; at += kPart) {
         const size_t n = std::min(kPart, bytes - at);
         char *buffer = acquire();
@@ -402,6 +311,7 @@ void HostStage::upload(void *dst, const void *src, size_t bytes, hipStream_t str
         IOS_HIP(hipEventRecord(drained_[turn_], stream));
         used_[turn_] = true;
     }
+    settle.armed = false;
 }
 
 // Elements [first, first + count) of a view in the host's layout, to host memory (count <= 2^20).  Bound by the link: a part of
@@ -416,6 +326,7 @@ __global__ __launch_bounds__(256) void gather_kernel(float *__restrict__ dst, co
 }
 
 void HostStage::download(float *dst, const TensorView &src, int batch, hipStream_t stream) {
+    SettleOnFailure settle{stream};
     // one part is gathered while the one before it is copied to the caller; small transfers take one step
     struct Part {
         size_t at, n;   // floats
@@ -445,6 +356,7 @@ void HostStage::download(float *dst, const TensorView &src, int batch, hipStream
         }
         last = now;
     }
+    settle.armed = false;
 }
 
 // ---- end of a pass -------------------------------------------------------------------------------------------------------
@@ -525,7 +437,7 @@ hipError_t HostStage::watch(int word, hipStream_t stream) {
     auto next = clock::now() + std::chrono::microseconds(500);
     for (unsigned spins = 0;; spins++) {
         if (__atomic_load_n(words_ + word, __ATOMIC_ACQUIRE) == pass_) return hipSuccess;
-        pause();
+        spin_pause();
         if ((spins & 63) != 63 || clock::now() < next) continue;
         const hipError_t status = hipStreamQuery(stream);
         if (status != hipErrorNotReady) return status;
