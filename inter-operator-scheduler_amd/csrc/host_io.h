@@ -58,9 +58,10 @@ public:
         TensorView view;   // ptr null: only the word
         int batch = 0;
     };
-    void signal(const Result &result, hipStream_t stream);
-    void wait(hipStream_t stream);                                  // for the pass behind the last signal()
-    void fetch(void *dst, size_t bytes, hipStream_t stream);        // that pass's result
+    unsigned signal(const Result &result, hipStream_t stream);      // the number of the pass
+    void wait(unsigned pass, hipStream_t stream);
+    // The result of a pass that delivered one, until the next pass that does.
+    void fetch(void *dst, size_t bytes, unsigned pass, hipStream_t stream);
 
 private:
     char *acquire();   // the ring's next buffer, once the link has drained it
@@ -71,7 +72,7 @@ private:
         bool used = false;
         char *take(size_t need);
     };
-    hipError_t watch(int word, hipStream_t stream);
+    hipError_t watch(int word, unsigned pass, hipStream_t stream);
     char *part_[kParts] = {};
     hipEvent_t drained_[kParts] = {};
     bool used_[kParts] = {};

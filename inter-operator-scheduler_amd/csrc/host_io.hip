@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256) void signal_kernel(SignalArgs a) {
     }
 }
 
-void HostStage::signal(const Result &result, hipStream_t stream) {
+unsigned HostStage::signal(const Result &result, hipStream_t stream) {
     const TensorView &v = result.view;
     SignalArgs a{};
     a.dst = result_;
@@ -429,14 +429,15 @@ void HostStage::signal(const Result &result, hipStream_t stream) {
     const int blocks = bytes <= (size_t(16) << 10) ? 1 : bytes <= kChunk ? kGroupBlocks : kGroups * kGroupBlocks;
     hipLaunchKernelGGL(signal_kernel, dim3(blocks), dim3(256), 0, stream, a);
     IOS_HIP(hipGetLastError());
+    return a.pass;
 }
 
-hipError_t HostStage::watch(int word, hipStream_t stream) {
+hipError_t HostStage::watch(int word, unsigned pass, hipStream_t stream) {
     using clock = std::chrono::steady_clock;
     // the stream itself is asked every now and then: a failed pass never raises the word
     auto next = clock::now() + std::chrono::microseconds(500);
     for (unsigned spins = 0;; spins++) {
-        if (__atomic_load_n(words_ + word, __ATOMIC_ACQUIRE) == pass_) return hipSuccess;
+        if (__atomic_load_n(words_ + word, __ATOMIC_ACQUIRE) == pass) return hipSuccess;
         spin_pause();
         if ((spins & 63) != 63 || clock::now() < next) continue;
         const hipError_t status = hipStreamQuery(stream);
@@ -445,14 +446,14 @@ hipError_t HostStage::watch(int word, hipStream_t stream) {
     }
 }
 
-void HostStage::wait(hipStream_t stream) { IOS_HIP(watch(0, stream)); }
+void HostStage::wait(unsigned pass, hipStream_t stream) { IOS_HIP(watch(0, pass, stream)); }
 
-void HostStage::fetch(void *dst, size_t bytes, hipStream_t stream) {
+void HostStage::fetch(void *dst, size_t bytes, unsigned pass, hipStream_t stream) {
     // memory that a device has just written is read at 25-30 GB/s by one thread: several threads, each waiting for its chunk
     const int chunks = (int)((bytes + kChunk - 1) / kChunk);
     std::atomic<int> failed{hipSuccess};
     const auto body = [&](int c) {
-        const hipError_t status = watch(1 + c, stream);
+        const hipError_t status = watch(1 + c, pass, stream);
         if (status != hipSuccess) {
             failed.store(status);
             return;

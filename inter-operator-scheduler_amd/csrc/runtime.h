@@ -213,6 +213,7 @@ private:
     bool input_changed_ = false;    // the input or a weight has been set since the last pass
     bool advance_ = false;          // set_conv_weights issues the stages whose filters it has packed
     size_t next_stage_ = 0;
+    unsigned delivered_pass_ = 0;   // the pass whose result is in the context's stage, where this session owns that
     bool fetches_result_ = true;    // the caller has fetched the last result (or there was none): the next pass delivers its own
     std::vector<hipEvent_t> fork_events_;                 // per stage (multi-group stages only)
     std::vector<std::vector<hipEvent_t>> join_events_;    // per stage, per extra group

@@ -684,7 +684,7 @@ void Session::get_output(float *host) {
     if (host == nullptr) throw std::runtime_error("output pointer is null");
     if (!plan_.output_single_group) throw std::runtime_error("the last stage of the schedule must have a single group");
     fetches_result_ = true;
-    if (ctx_.result_owner == this) ctx_.stage().fetch(host, (size_t)plan_.batch * plan_.output.image_floats() * sizeof(float), ctx_.stream(0));
+    if (ctx_.result_owner == this) ctx_.stage().fetch(host, (size_t)plan_.batch * plan_.output.image_floats() * sizeof(float), delivered_pass_, ctx_.stream(0));
     else copy_out(plan_.output, host);
 }
 
@@ -1132,10 +1132,13 @@ void Session::finish_pass() {
     HostStage::Result result;
     if (deliver) result = {tv(plan_.output), plan_.batch};
     hipStream_t main = ctx_.stream(0);
-    ctx_.stage().signal(result, main);
-    ctx_.stage().wait(main);
+    if (deliver) ctx_.result_owner = nullptr;   // what is there is written over, also by a pass that then fails
+    const unsigned pass = ctx_.stage().signal(result, main);
+    ctx_.stage().wait(pass, main);
     ctx_.check_xcd_fault();
-    if (deliver) ctx_.result_owner = this;
+    if (!deliver) return;
+    ctx_.result_owner = this;
+    delivered_pass_ = pass;
 }
 
 // One inference with everything crossing the boundary.  The weights of a network take longer on the link than the pass itself

@@ -1,4 +1,6 @@
 """Transfers between a caller's arrays and the device at the sizes where the paths of csrc/host_io.hip change over."""
+import time
+
 import numpy as np
 import pytest
 
@@ -200,3 +202,46 @@ def test_an_input_beyond_the_staging_buffer():
         session.run()
         assert np.array_equal(session.output(), np.maximum(x, 0))
     session.close()
+
+
+@pytest.mark.parametrize('floats', [4096, 65537, 640000])
+def test_sessions_take_turns(floats):
+    """A result that a pass has delivered stays there until another pass delivers one, whatever passes run in between."""
+    channels = floats // 65536 + 1
+    first, second, large = (rt.Session(relu_graph(c, h, w), 1) for c, h, w in
+                            ((1, 1, floats) if floats < 65536 else (channels, 256, 256), (channels, 256, 255), (17, 256, 257)))
+    rng = np.random.default_rng(floats)
+    x, y, z = (rng.standard_normal(s.input_shape, dtype=np.float32) for s in (first, second, large))
+    for session, data in ((first, x), (second, y), (large, z)):
+        session.set_input(data)
+        session.run()
+        assert np.array_equal(session.output(), np.maximum(data, 0))
+    for step in range(4):
+        first.set_input(x + step)
+        first.run()
+        if step % 2:
+            large.run()     # too large to be delivered
+            second.enqueue()
+            second.synchronize()
+        if step == 3:
+            second.run()    # delivers: the first one's result is copied from its own tensor
+        assert np.array_equal(first.output(), np.maximum(x + step, 0))
+        assert np.array_equal(first.output(), np.maximum(x + step, 0))
+        assert np.array_equal(second.output(), np.maximum(y, 0))
+        assert np.array_equal(large.output(), np.maximum(z, 0))
+
+
+def test_a_delivered_result_is_fetched_at_once_after_passes_that_deliver_nothing():
+    """2.5 MB, 40 chunks: the wait for chunks of another pass would take half a millisecond for each."""
+    first, large = rt.Session(relu_graph(10, 256, 256), 1), rt.Session(relu_graph(17, 256, 257), 1)
+    x = np.random.default_rng(0).standard_normal(first.input_shape, dtype=np.float32)
+    first.set_input(x)
+    times = []
+    for _ in range(12):
+        first.run()
+        large.run()
+        start = time.perf_counter()
+        y = first.output()
+        times.append(time.perf_counter() - start)
+        assert np.array_equal(y, np.maximum(x, 0))
+    assert min(times) < 2e-3, times
