@@ -467,7 +467,7 @@ struct ConvTiled {
         }
     };
 
-    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const float floor = relu_floor(a.pre_relu != 0);
     auto store_tile = [&](int buf, const floatx4(&ar)[A_ITERS], const floatx4(&br)[B_ITERS]) {
         float *Ab = As + buf * BK * LDA;
         float *Bb = Bs + buf * BK * LDB;
@@ -482,10 +482,10 @@ struct ConvTiled {
         }
 #pragma unroll
         for (int i = 0; i < B_ITERS; i++) {
-            // folded ReLU of the producer as one integer max (negative floats are negative integers)
+            // folded ReLU of the producer
 #pragma unroll
             for (int u = 0; u < 4; u++)
-                Bb[(4 * bq + u) * LDB + bn_l + i * (T / B_QUADS)] = __int_as_float(max(__float_as_int(br[i][u]), relu_floor));
+                Bb[(4 * bq + u) * LDB + bn_l + i * (T / B_QUADS)] = relu_above(floor, br[i][u]);
         }
     };
 
@@ -732,7 +732,7 @@ struct ConvSplit3 {
         }
         left = c_left;
     };
-    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;   // a quad of channels may straddle the end of the group's
     auto store_inputs = [&](int buf, const floatx4 (&br)[B_IT][2], int left) {
         uintx4 *stage = lds + buf * STAGE;
@@ -741,7 +741,7 @@ struct ConvSplit3 {
             if (B_OCT % T != 0 && tid + i * T >= B_OCT) continue;
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(br[i][j >> 2][j & 3]), relu_floor));   // folded ReLU of the producer
+            for (int j = 0; j < 8; j++) v[j] = relu_above(floor, br[i][j >> 2][j & 3]);   // folded ReLU of the producer
             if (ragged)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = j < left ? v[j] : 0.f;
@@ -1080,7 +1080,7 @@ struct ConvWsplit {
         }
     };
     // folded ReLU of the producer: as integers, negative floats are below 0 and everything is above INT_MIN
-    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = QUAD && (a.ICg & 3) != 0;   // (a branch around register work only, see load_batch)
     auto compute = [&](const FilterStage &A, float(&B)[U][TN], int left) {
         if (ragged) {
@@ -1095,7 +1095,7 @@ struct ConvWsplit {
             for (int j = 0; j < TN; j++) {
                 float v[8];
 #pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = __int_as_float(max(__float_as_int(B[u][j]), relu_floor));
+                for (int u = 0; u < 8; u++) v[u] = relu_above(floor, B[u][j]);
                 uintx4 hi, mid, lo;
                 split_bf16x3(v, hi, mid, lo);
                 bq[0][j] = __builtin_bit_cast(bf16x8, hi);
@@ -1118,7 +1118,7 @@ struct ConvWsplit {
             for (int j = 0; j < TN; j++) {
                 float v[8];
 #pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = __int_as_float(max(__float_as_int(B[u][j]), relu_floor));
+                for (int u = 0; u < 8; u++) v[u] = relu_above(floor, B[u][j]);
                 const bf16x8 bq = __builtin_bit_cast(bf16x8, round_bf16x8(v));
 #pragma unroll
                 for (int i = 0; i < TM; i++)
@@ -1128,8 +1128,8 @@ struct ConvWsplit {
         } else if constexpr (RP != 0) {
 #pragma unroll
             for (int j = 0; j < TN; j++) {
-                const floatx4 b32 = {__int_as_float(max(__float_as_int(B[0][j]), relu_floor)), __int_as_float(max(__float_as_int(B[1][j]), relu_floor)),
-                                     __int_as_float(max(__float_as_int(B[2][j]), relu_floor)), __int_as_float(max(__float_as_int(B[3][j]), relu_floor))};
+                const floatx4 b32 = {relu_above(floor, B[0][j]), relu_above(floor, B[1][j]),
+                                     relu_above(floor, B[2][j]), relu_above(floor, B[3][j])};
                 if constexpr (RP == 1) {
                     const bf16x4 b4 = __builtin_convertvector(b32, bf16x4);   // round to nearest even
 #pragma unroll
@@ -1150,7 +1150,7 @@ struct ConvWsplit {
                 for (int i = 0; i < TM; i++)
 #pragma unroll
                     for (int j = 0; j < TN; j++) {
-                        const float bval = __int_as_float(max(__float_as_int(B[u][j]), relu_floor));   // one integer max
+                        const float bval = relu_above(floor, B[u][j]);
                         acc[i][j] = M::run(A.v[u][i], bval, acc[i][j]);
                     }
         }

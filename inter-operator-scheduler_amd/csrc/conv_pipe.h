@@ -123,7 +123,7 @@ struct ConvPipe {
         }
         left = c_left;
     };
-    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;
     auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
         uintx4 *As = lds + buf * STAGE;
@@ -135,7 +135,7 @@ struct ConvPipe {
         for (int i = 0; i < B_IT; i++) {
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(br[i][j >> 2][j & 3]), relu_floor));   // folded ReLU of the producer
+            for (int j = 0; j < 8; j++) v[j] = relu_above(floor, br[i][j >> 2][j & 3]);   // folded ReLU of the producer
             if (ragged)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = j < left ? v[j] : 0.f;

@@ -104,7 +104,7 @@ struct ConvWindow {
             b_reg[i][1] = buffer_load_f32x4(xr, at | pad1, 16u);
         }
     };
-    const int relu_floor = a.pre_relu ? 0 : (int)0x80000000;
+    const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;
     auto store_window = [&](int buf) {
         uintx4 *at = lds + buf * BUF + half * S + (tid >> 1);
@@ -112,7 +112,7 @@ struct ConvWindow {
         for (int i = 0; i < P_IT; i++) {
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = __int_as_float(max(__float_as_int(b_reg[i][j >> 2][j & 3]), relu_floor));
+            for (int j = 0; j < 8; j++) v[j] = relu_above(floor, b_reg[i][j >> 2][j & 3]);
             if (ragged)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = j < b_left ? v[j] : 0.f;

@@ -47,15 +47,23 @@ __device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv &f) {
     return (t + ((n - t) >> f.s1)) >> f.s2;
 }
 
-// Activation of V values of a lane.  The usual ones (none, ReLU) are one integer maximum per value (negative floats are negative
-// integers); the others go through one copy of their code in turn: inlined once per value, tanh and sigmoid put kilobytes of
-// code between a kernel's last load and its store, and skipping them cost a batch-1 launch a microsecond of instruction fetches.
+// max(x, 0) or x, chosen by a floor that does not depend on the lane.  NaN gives 0, as in the reference (its descriptors say
+// NOT_PROPAGATE_NAN).  For the loaders of convolutions, whose values come from memory, in one instruction: v_med3_f32 of 0, |x| and
+// x is x above zero and 0 below it, and the smallest of those that are numbers, 0, where x is not; with a floor that is NaN
+// itself it is the smaller of |x| and x: x as it is.  (A floating-point maximum takes a second instruction for a value that may be
+// a signalling NaN; an integer maximum keeps a NaN whose sign is clear.)
+__device__ __forceinline__ float relu_floor(bool relu) { return relu ? 0.f : __builtin_nanf(""); }
+__device__ __forceinline__ float relu_above(float floor, float x) { return __builtin_amdgcn_fmed3f(floor, __builtin_fabsf(x), x); }
+
+// Activation of V values of a lane.  The usual ones (none, ReLU) are one maximum per value; the others go through one copy of
+// their code in turn: inlined once per value, tanh and sigmoid put kilobytes of code between a kernel's last load and its store,
+// and skipping them cost a batch-1 launch a microsecond of instruction fetches.
 template <int V>
 __device__ __forceinline__ void apply_activation(float (&v)[V], int act) {
     if (__builtin_expect(act <= ACT_RELU, 1)) {
-        const int floor = act == ACT_RELU ? 0 : (int)0x80000000;
+        const float floor = relu_floor(act == ACT_RELU);
 #pragma unroll
-        for (int k = 0; k < V; k++) v[k] = __int_as_float(max(__float_as_int(v[k]), floor));
+        for (int k = 0; k < V; k++) v[k] = fmaxf(v[k], floor);   // (the maximum of a number and NaN is the number)
         return;
     }
 #pragma unroll 1

@@ -294,7 +294,7 @@ __device__ __forceinline__ void dwconv_body(const DirectConvArgs &a, int block, 
     const unsigned cv = (unsigned)((p.OC + V - 1) / V);
     const unsigned total = (unsigned)(p.B * p.OH * p.OW) * cv;
     const int w_ps = (p.OC + 3) & ~3;
-    const int relu_floor = p.pre_relu ? 0 : (int)0x80000000;   // folded ReLU as an integer max
+    const float floor = relu_floor(p.pre_relu != 0);
     for (unsigned i = block * threads + threadIdx.x; i < total; i += num_blocks * threads) {
         const unsigned pixel = fast_div(i, a.div_cv);
         const int c = (int)(i - pixel * cv) * V;
@@ -310,7 +310,7 @@ __device__ __forceinline__ void dwconv_body(const DirectConvArgs &a, int block, 
         auto add_tap = [&](const Channels<V> &x, int tap) {
             const Channels<V> f = load_channels<V>(wc + tap * w_ps);
 #pragma unroll
-            for (int k = 0; k < V; k++) acc.v[k] = fmaf(__int_as_float(max(__float_as_int(x.v[k]), relu_floor)), f.v[k], acc.v[k]);
+            for (int k = 0; k < V; k++) acc.v[k] = fmaf(relu_above(floor, x.v[k]), f.v[k], acc.v[k]);
         };
         bool done = false;
         if constexpr (KH > 0) if (a.x_bytes != 0) {
