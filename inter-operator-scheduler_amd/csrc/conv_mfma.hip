@@ -116,6 +116,33 @@ bool conv_variant_takes(const ConvProblem &p, int variant) {
     return p.sh == 1 && p.sw == 1 && taps % 2 == 1 && taps >= 3 && taps < 32 && p.OH <= p.H && p.OW <= p.W && window_span(p, v.BN) <= v.window;
 }
 
+// Configurations that the tuner leaves out.  None of them was the fastest in any share class over 3030 problems: the convolutions of
+// nine networks (Inception-v3, SqueezeNet, ResNet-18 / 50, RandWire, NASNet, VGG-16, AlexNet, the sample network) at batch 1 to 64 and
+// of multi-branch blocks on odd sizes, in each precision.  (The fp32 matrix instructions lose to three bfloat16 terms from a few
+// microseconds on.)  They serve the closed-form choice, which knows none of the others, and the option that pins a configuration.
+static const char *const kNotMeasured[] = {
+    "m64n64k32_w2x2x1_t32", "m128n128k16_w2x2x1_t32", "m32n32k64_w1x1x4_t32", "m64n32k32_w2x1x2_t32", "m32n64k32_w1x2x2_t32",
+    "m128n64k16_w2x2x1_t32", "m64n16k64_w4x1x1_t16", "m32n16k64_w2x1x2_t16", "m16n16k128_w1x1x4_t16", "m64n128k16_w2x2x1_t32",
+    "m64n64k16_w2x2x1_t32", "m32n128k16_w1x4x1_t32", "m192n64k16_w2x2x1_t32", "m96n128k16_w1x4x1_t32", "m192n128k16_w2x2x1_t32",
+    "m160n128k16_w1x4x1_t32", "ws_m32n16_w16_t16", "ws_m16n16_w16_t16", "ws_m32n32_w16_t16", "ws_m64n16_w16_t16",
+    "ws_m32n16_w8_t16", "ws_m32n16_w4_t16", "ws_m32n32_w16_t32", "ws_m16n32_w16_t16", "wq_m32n32_w16_t16", "wq_m64n32_w8_t16",
+    "wq_m64n64_w4_t16", "wq_m64n32_w4_t16", "wq_m32n32_w8_t16", "wq_m64n64_w4_t32", "wq_m16n16_w16_t16_d4",
+    "wq_m32n16_w16_t16_d4", "wq_m32n32_w2_t16_d4", "wq_m64n32_w2_t16", "wq_m64n32_w4_t16_d4", "wb_m64n64_w4",
+    "ws_m32n64_w1_t16_c4", "wq_m32n32_w8_t32", "wq_m32n32_w16_t32", "wq_m64n32_w8_t32", "wq_m64n32_w4_t32", "wq_m32n64_w8_t32",
+    "wq_m32n64_w4_t32", "wq_m64n64_w8_t32", "wq_m64n32_w2_t32", "wq_m64n32_w1_t32", "wq_m32n64_w2_t32", "wq_m32n32_w2_t32_d4",
+    "wq_m32n32_w1_t16_d4", "wq_m64n64_w2_t32", "x3_m64n64_w2x2", "x3_m64n64_w1x1", "x3_m64n128_w1x2", "x3_m192n128_w6x2",
+    "wb_x1_m64n128_w2x2", "wb_x1_m128n256_w2x4", "wb_x1_m64n128_w1x2", "wb_x1_m64n256_w2x4",
+};
+
+bool conv_variant_measured(int variant) {
+    static const std::vector<char> measured = [] {
+        std::vector<char> flags(kNumVariants, 1);
+        for (const char *name : kNotMeasured) flags[variant_by_name(name)] = 0;
+        return flags;
+    }();
+    return measured.at(variant) != 0;
+}
+
 // The entry that serves the problem: where a window kernel is asked for and does not take it, one that reads the same packed filters.
 static int variant_for(const ConvProblem &p, const ConvLaunch &l) {
     if (l.variant < 0 || l.variant >= kNumVariants) throw std::runtime_error("conv: bad variant");

@@ -218,36 +218,24 @@ struct ConvPipe {
 
 // X(index, name, KU, PD, TMW, TNW, WM, WN): three exact terms
 #define IOS_PIPE3_VARIANTS(X)                          \
-    X(119, "x3p_m128n128_w2x2", 1, 2, 2, 2, 2, 2)      \
-    X(120, "x3p_m192n128_w2x2", 1, 2, 3, 2, 2, 2)      \
-    X(121, "x3p_m64n256_w1x4", 1, 2, 2, 2, 1, 4)       \
-    X(122, "x3p_m64n128_w1x2", 1, 2, 2, 2, 1, 2)       \
-    X(123, "x3p_m96n128_w1x4", 1, 2, 3, 1, 1, 4)       \
-    X(124, "x3p_m96n128_w1x2", 1, 2, 3, 2, 1, 2)       \
-    X(125, "x3p_m32n256_w1x4", 1, 2, 1, 2, 1, 4)       \
-    X(126, "x3p_m64n128_w1x4", 1, 2, 2, 1, 1, 4)       \
-    X(127, "x3p_m128n64_w2x2", 2, 1, 2, 1, 2, 2)       \
-    X(128, "x3p_m64n64_w2x2", 2, 1, 1, 1, 2, 2)        \
-    X(129, "x3p_m128n128_w2x2_k32", 2, 1, 2, 2, 2, 2)
+    X(119, "x3p_m96n128_w1x4", 1, 2, 3, 1, 1, 4)       \
+    X(120, "x3p_m64n128_w1x4", 1, 2, 2, 1, 1, 4)       \
+    X(121, "x3p_m64n64_w2x2", 2, 1, 1, 1, 2, 2)
 // one rounded term, bfloat16 (option precision=bf16)
 #define IOS_PIPE_BF16_VARIANTS(X)                      \
-    X(130, "wb_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
-    X(131, "wb_p_m192n128_w2x2", 4, 1, 3, 2, 2, 2)     \
-    X(132, "wb_p_m64n256_w1x4", 2, 1, 2, 2, 1, 4)      \
-    X(133, "wb_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
-    X(134, "wb_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
-    X(135, "wb_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
-    X(136, "wb_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
-    X(137, "wb_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)       \
-    X(138, "wb_p_m192n64_w2x2", 4, 1, 3, 1, 2, 2)
+    X(122, "wb_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
+    X(123, "wb_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
+    X(124, "wb_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
+    X(125, "wb_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
+    X(126, "wb_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
+    X(127, "wb_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
 // one rounded term, IEEE half (option precision=fp16)
 #define IOS_PIPE_FP16_VARIANTS(X)                      \
-    X(139, "wh_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
-    X(140, "wh_p_m192n128_w2x2", 4, 1, 3, 2, 2, 2)     \
-    X(141, "wh_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
-    X(142, "wh_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
-    X(143, "wh_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
-    X(144, "wh_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
-    X(145, "wh_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
+    X(128, "wh_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
+    X(129, "wh_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
+    X(130, "wh_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
+    X(131, "wh_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
+    X(132, "wh_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
+    X(133, "wh_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
 
 }  // namespace ios

@@ -245,23 +245,23 @@ struct ConvWindow {
 // X(index, name, TMW, TNW, WM, WN, P_IT, NBUF).  A window of a 3 x 3 filter on wide maps takes 300 pixels beyond the outputs, so
 // the tall-and-narrow blocks are for few channels on large maps; the 128-output blocks serve the smaller maps.
 #define IOS_WINDOW3_VARIANTS(X)                          \
-    X(146, "x3_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(147, "x3_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(148, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)    \
-    X(149, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+    X(134, "x3_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(135, "x3_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(136, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)    \
+    X(137, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
 #define IOS_WINDOW_BF16_VARIANTS(X)                      \
-    X(150, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
-    X(151, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
-    X(152, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(153, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(154, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+    X(138, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(139, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(140, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(141, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(142, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
 #define IOS_WINDOW_FP16_VARIANTS(X)                      \
-    X(155, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
-    X(156, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
-    X(157, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(158, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(159, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
-constexpr int kFirstWindowVariant = 146, kNumConvVariants = 160;
+    X(143, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(144, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(145, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(146, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(147, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+constexpr int kFirstWindowVariant = 134, kNumConvVariants = 148;
 
 // The window kernels (conv_window.hip), in the order of the lists above
 struct WindowKernel {

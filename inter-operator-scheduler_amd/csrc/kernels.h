@@ -119,6 +119,7 @@ struct ConvVariant {
 
 int conv_num_variants();
 const ConvVariant &conv_variant(int index);
+bool conv_variant_measured(int variant);   // the tuner tries it
 bool conv_variant_takes(const ConvProblem &p, int variant);   // (a launch of another shape runs on a configuration that reads the same packed filters)
 
 struct ConvLaunch {

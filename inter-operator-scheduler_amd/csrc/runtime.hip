@@ -250,6 +250,9 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         double footprint;
         bool fusable;
     };
+    std::vector<Candidate> candidates;
+    float fastest = 1e30f;
+    constexpr float kQueuedMs = 0.008f, kLongMs = 0.04f;
     auto measure = [&](const ConvLaunch &l, int reps) {
         const size_t ws = conv_workspace_floats(p, l);
         float *workspace = ws ? tuning_buffer(3, ws) : nullptr;
@@ -257,8 +260,8 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         auto issue = [&] { launch_conv_mfma(p, l, x, packed, bias, y, workspace, counters, stream); };
         issue();   // warm-up
         // A launch costs the host 3 to 5 us, more than most kernels of a batch-1 network run: the device waits until all of
-        // them are queued, so that the events time the kernels and not the host.
-        launch_delay(reps + 3, stream);
+        // them are queued, so that the events time the kernels and not the host.  Where no kernel is that short, until the first.
+        launch_delay(fastest < kQueuedMs || candidates.empty() ? reps + 3 : 2, stream);
         IOS_HIP(hipEventRecord(start, stream));
         for (int r = 0; r < reps; r++) issue();
         IOS_HIP(hipEventRecord(stop, stream));
@@ -268,11 +271,9 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         return ms / reps;
     };
     // first pass: every configuration and split factor, a few launches each
-    std::vector<Candidate> candidates;
-    float fastest = 1e30f;
     for (int v = 0; v < conv_num_variants(); v++) {
         const ConvVariant &cv = conv_variant(v);
-        if (cv.precision != precision_ || !conv_variant_takes(p, v)) continue;   // the precision mode decides which family of configurations competes
+        if (cv.precision != precision_ || !conv_variant_measured(v) || !conv_variant_takes(p, v)) continue;   // the precision mode decides which family of configurations competes
         // tiles more than twice as tall / wide as the problem only waste lanes
         if (cv.BM >= 2 * p.OCg() + 32 || cv.BN >= 2 * p.Npix() + 32) continue;
         int last_effective = -1;
@@ -284,7 +285,7 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
             if (effective == last_effective) continue;   // asks for more slices than there are K tiles
             last_effective = effective;
             if (conv_workspace_floats(p, l) > kMaxWorkspace) break;
-            const float ms = measure(l, 4);
+            const float ms = measure(l, fastest < kLongMs ? 4 : 2);
             const double footprint = (double)cv.threads() * ((p.OCg() + cv.BM - 1) / cv.BM) * (double)((p.Npix() + cv.BN - 1) / cv.BN) *
                                      p.groups * effective;
             candidates.push_back({l, ms, footprint, cv.fusable()});

@@ -101,7 +101,7 @@ def test_parallel_stage_launches_large_convolutions_by_themselves(precision, key
     assert_close(got, ios_oracle.run(graph, x, **{key: convs}), f'{precision} {executor}')
 
 
-@pytest.mark.parametrize('variant', [None, 'x3p_m64n128_w1x2', 'wq_m64n32_w4_t32', 'm64n64k32_w2x2x1_t32'])
+@pytest.mark.parametrize('variant', [None, 'x3p_m64n128_w1x4', 'wq_m64n32_w4_t32', 'm64n64k32_w2x2x1_t32'])
 def test_an_input_of_a_gigabyte(variant):
     """85 images of 3 x 1024 x 1024: 1.07 GB of values, 1.43 GB with the pixels padded."""
     if variant is not None:
