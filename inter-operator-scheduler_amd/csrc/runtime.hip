@@ -473,6 +473,10 @@ void DeviceContext::set_option(const std::string &key, const std::string &value)
         else if (value == "inline") reduce_mode_ = ReduceMode::Inline;
         else if (value == "kernel") reduce_mode_ = ReduceMode::Kernel;
         else throw std::runtime_error("option split_k_reduce: expected xcd, inline or kernel, got '" + value + "'");
+    } else if (key == "host_threads") {
+        const int v = atoi(value.c_str());
+        if (v < 0 || v > 1024) throw std::runtime_error("option host_threads: expected 0..1024");
+        HostCopier::get().set_threads(v);
     } else if (key == "clear_tuning") {
         tuned.clear();
     } else {
@@ -488,6 +492,7 @@ std::string DeviceContext::info_json() const {
        << ",\"xcd_placement_probe\":" << (xcd_usable_ ? "true" : "false") << ",\"xcd_map\":" << xcd_map_[0]
        << ",\"precision\":\"" << (precision_ == PREC_BF16 ? "bf16" : precision_ == PREC_FP16 ? "fp16" : "fp32") << "\""
        << ",\"conv_variant\":" << forced_variant_ << ",\"conv_split_k\":" << forced_split_k_
+       << ",\"host_threads\":" << HostCopier::get().threads()
        << ",\"arena_reuse\":" << (planner_arena_reuse() ? "true" : "false")
        << ",\"max_groups\":" << kMaxGroups << ",\"conv_variants\":[";
     for (int i = 0; i < conv_num_variants(); i++) os << (i ? "," : "") << '"' << conv_variant(i).name << '"';

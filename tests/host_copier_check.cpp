@@ -1,7 +1,10 @@
 // Copies shared out over threads (csrc/host_copier.h) whose pieces or whose work between the pieces fail.
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
+#include <set>
 #include <stdexcept>
 #include <thread>
 #include <vector>
@@ -62,15 +65,43 @@ static void check_failure(int who, bool large) {
         threw = true;
     }
     CHECK(inside.load() == 0);
-    CHECK(threw == (who != 3) || (who == 2 && std::thread::hardware_concurrency() < 3));
+    CHECK(threw == (who != 3) || (who == 2 && HostCopier::get().threads() < 2));
     CHECK(threw ? begun.load() < 64 : begun.load() == 64);
     const int then = begun.load();
     doze(2000);
     CHECK(begun.load() == then);   // nobody begins a piece behind the caller's back
 }
 
-int main() {
+// the pool with another number of threads
+static void check_threads(int count) {
+    HostCopier::get().set_threads(count);
+    std::mutex mutex;
+    std::set<std::thread::id> seen;
+    for (int round = 0; round < 5; round++) {
+        if (round) doze(1000);   // the workers are asleep, or awake
+        HostCopier::get().parallel(40, true, [&](int) {
+            doze(200);
+            std::lock_guard<std::mutex> lock(mutex);
+            seen.insert(std::this_thread::get_id());
+        });
+    }
+    CHECK((int)seen.size() <= HostCopier::get().threads());
+    CHECK(count == 0 || (int)seen.size() <= count);
+    CHECK(count != 1 || seen.size() == 1);
     check_copies();
+}
+
+int main() {
+    CHECK(ios::processors_of_quota("max 100000") == 0);
+    CHECK(ios::processors_of_quota("400000 100000") == 4);
+    CHECK(ios::processors_of_quota("50000 100000") == 1);
+    CHECK(ios::processors_of_quota("150000 100000") == 2);
+    CHECK(ios::processors_of_quota("-1 100000") == 0);
+    CHECK(ios::processors_of_quota("") == 0);
+    CHECK(ios::available_processors() >= 1 && ios::available_processors() <= (int)std::thread::hardware_concurrency());
+    check_copies();
+    CHECK(HostCopier::get().threads() <= std::max(1, ios::available_processors() * 3 / 4));
+    for (int count : {1, 3, 2, 0, 1, 7, 0}) check_threads(count);
     for (int round = 0; round < 12; round++)
         for (int who = 0; who < 4; who++) {
             check_failure(who, round % 2 == 0);

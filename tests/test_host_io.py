@@ -245,3 +245,17 @@ def test_a_delivered_result_is_fetched_at_once_after_passes_that_deliver_nothing
         times.append(time.perf_counter() - start)
         assert np.array_equal(y, np.maximum(x, 0))
     assert min(times) < 2e-3, times
+
+
+def test_host_threads():
+    """Copies shared out over other numbers of threads, the caller alone among them."""
+    try:
+        for threads in (1, 2, 5, 0):
+            rt.set_option('host_threads', threads)
+            assert threads == 0 or rt.device_info()['host_threads'] == threads
+            test_input_and_result_of_every_size(3000001)
+            test_input_and_result_of_every_size(98305)
+        with pytest.raises(RuntimeError, match='host_threads'):
+            rt.set_option('host_threads', -1)
+    finally:
+        rt.set_option('host_threads', 0)
