@@ -285,7 +285,7 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
             if (effective == last_effective) continue;   // asks for more slices than there are K tiles
             last_effective = effective;
             if (conv_workspace_floats(p, l) > kMaxWorkspace) break;
-            const float ms = measure(l, fastest < kLongMs ? 4 : 2);
+            const float ms = measure(l, fastest < kQueuedMs ? 8 : fastest < kLongMs ? 4 : 2);
             const double footprint = (double)cv.threads() * ((p.OCg() + cv.BM - 1) / cv.BM) * (double)((p.Npix() + cv.BN - 1) / cv.BN) *
                                      p.groups * effective;
             candidates.push_back({l, ms, footprint, cv.fusable()});
@@ -293,7 +293,11 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
             if (ms > 3.f * fastest) break;   // more slices only add reduction work from here on
         }
     }
-    // second pass: the three fastest of every class again with more launches (the first pass is noisy at 5-10 us)
+    // second pass: the fastest of every class again with more launches.  The first pass is noisy at 5-10 us, and many of the
+    // configurations that are measured at all are close to each other.  Inception-v3 at batch 1, mean over 6 to 16 processes that
+    // measure anew: 399 us with four launches in the first pass and three finalists, 396 with four and five, 392 with eight and five
+    // (392 too with all 102 configurations, four launches and three finalists).
+    constexpr int kFinalists = 5;
     std::sort(candidates.begin(), candidates.end(), [](const Candidate &a, const Candidate &b) { return a.ms < b.ms; });
     std::vector<char> refined(candidates.size(), 0);
     TunedConv result;
@@ -325,7 +329,7 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
                 if ((candidates[i].fusable || any_kernel) && !wide_too_short(candidates[i])) order.push_back(i);
             std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return score(candidates[a]) < score(candidates[b]); });
             double best = 1e300;
-            for (size_t n = 0; n < order.size() && n < 3; n++) {
+            for (size_t n = 0; n < order.size() && n < kFinalists; n++) {
                 Candidate &cand = candidates[order[n]];
                 if (!refined[order[n]]) {
                     cand.ms = std::min(cand.ms, measure(cand.launch, 16));
@@ -341,7 +345,7 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         for (int pass = 0; pass < 2 && !found[c]; pass++) {
             int taken = 0;
             float best = 1e30f;
-            for (size_t i = 0; i < candidates.size() && taken < 3; i++) {
+            for (size_t i = 0; i < candidates.size() && taken < kFinalists; i++) {
                 if (!eligible(candidates[i], pass == 0)) continue;
                 taken++;
                 if (!refined[i]) {
