@@ -120,6 +120,8 @@ const char *ios_last_error(void);
  *   "host_threads" = N: threads that share a large copy between a caller's arrays and pinned memory, the caller among them
  *       (12 at most; 1: the caller alone).  "0" (default): three quarters of the processors the process is bound to or that its
  *       control group leaves it.  Up to three of them stay awake for half a millisecond behind a copy;
+ *   "release_staging" = anything: frees the pinned memory that inputs and weights are staged in (up to 256 MB each).  It stays as
+ *       long as there is a session; a program that only makes inference calls keeps it between them;
  *   "thin_conv_min_pixels" = count (default 262144; negative: never): a 3 x 3 convolution of a 3-channel image with at least
  *       this many output pixels (batch x OH x OW) that has its stage to itself runs on a direct kernel bound by the bytes of
  *       its output instead of the matrix path (first layers at large batches); needs no device;

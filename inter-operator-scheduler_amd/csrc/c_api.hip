@@ -153,7 +153,13 @@ const char *ios_last_error(void) { return g_last_error.c_str(); }
 int ios_set_option(const char *key, const char *value) {
     return guarded([&]() {
         if (key == nullptr || value == nullptr) throw std::runtime_error("option key or value is null");
-        g_inference_plans.clear();
+        if (!g_inference_plans.empty()) {
+            // the next inference call stages as much as the last one: the memory for that stays (option release_staging frees it)
+            ios::DeviceContext &ctx = ios::DeviceContext::get();
+            ctx.sessions++;
+            g_inference_plans.clear();
+            ctx.sessions--;
+        }
         if (ios::set_planner_option(key, value)) return;   // needs no device
         ios::DeviceContext::get().set_option(key, value);
     });

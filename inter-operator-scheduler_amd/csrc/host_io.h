@@ -22,10 +22,14 @@ public:
     static constexpr int kParts = 4;
     static constexpr int kMaxChunks = 5;                  // steps in which a batch arrives (the copy engine takes 25-35 us from one to the next)
     static constexpr size_t kBatch = kStagedBytes;        // largest transfer that is staged as a whole (or one image)
+    static constexpr size_t kIdle = size_t(16) << 20;     // of each growing buffer that stays while there is no session
     static constexpr size_t kChunk = size_t(64) << 10;   // bytes of the result that are announced together
     static constexpr size_t kAlone = 3 * kChunk;          // results up to this size are fetched by one thread
     static constexpr size_t kResult = kDeliveredFloats * sizeof(float);   // largest result a pass delivers to host memory by itself
 
+    // Frees what the growing buffers hold beyond kIdle.  Nothing may be on its way.
+    void give_back() noexcept;
+    size_t staged_bytes() const { return inputs_.bytes + weights_.bytes; }
     void create();   // with the device context (pinned memory goes with the process: the runtime may be unloaded before static objects are)
 
     // Copies `bytes` to the device behind what `stream` holds.  Returns when the caller's memory may change again; the
@@ -65,7 +69,7 @@ public:
 
 private:
     char *acquire();   // the ring's next buffer, once the link has drained it
-    struct Batch {     // a buffer that grows to the transfer it stages, and is kept
+    struct Batch {     // a buffer that grows to the transfer it stages, and is kept while there are sessions
         char *memory = nullptr;
         size_t bytes = 0;
         hipEvent_t drained = nullptr;

@@ -88,6 +88,16 @@ char *HostStage::acquire() {
     return part_[turn_];
 }
 
+void HostStage::give_back() noexcept {
+    for (Batch *b : {&inputs_, &weights_}) {
+        if (b->bytes <= kIdle) continue;
+        (void)hipHostFree(b->memory);
+        b->memory = nullptr;
+        b->bytes = 0;
+        b->used = false;
+    }
+}
+
 char *HostStage::Batch::take(size_t need) {
     if (used) {
         used = false;

@@ -36,6 +36,7 @@ public:
     const void *result_owner = nullptr;
     // the sessions that laid out the shared arena and the static scratch last
     const void *shared_owner = nullptr, *static_owner = nullptr;
+    int sessions = 0;   // that there are
 
     // a process-wide arena reused by the stateless latency / inference entry points
     float *shared_arena(size_t floats);
@@ -175,6 +176,7 @@ public:
     void profile_launches(int warmup, int repeat, float *ms, int capacity);
 
 private:
+    void acquire(Storage storage, bool pack_filters);
     void setup(bool pack_filters);
     void pack(const PlanConv &conv, hipStream_t stream);
     void ensure_timers();
@@ -207,6 +209,7 @@ private:
     float *base_ = nullptr;
     bool owns_memory_ = false;
     bool static_ = false;
+    bool released_ = false;
     std::vector<char> packed_;      // per convolution: its packed filters are laid out
     std::vector<int> arriving_;     // parts of the input on their way: images up to the end of each
     bool ran_in_parts_ = false;     // the last pass worked on parts of the batch as they arrived

@@ -481,6 +481,9 @@ void DeviceContext::set_option(const std::string &key, const std::string &value)
         const int v = atoi(value.c_str());
         if (v < 0 || v > 1024) throw std::runtime_error("option host_threads: expected 0..1024");
         HostCopier::get().set_threads(v);
+    } else if (key == "release_staging") {
+        IOS_HIP(hipDeviceSynchronize());
+        stage_.give_back();
     } else if (key == "clear_tuning") {
         tuned.clear();
     } else {
@@ -496,7 +499,7 @@ std::string DeviceContext::info_json() const {
        << ",\"xcd_placement_probe\":" << (xcd_usable_ ? "true" : "false") << ",\"xcd_map\":" << xcd_map_[0]
        << ",\"precision\":\"" << (precision_ == PREC_BF16 ? "bf16" : precision_ == PREC_FP16 ? "fp16" : "fp32") << "\""
        << ",\"conv_variant\":" << forced_variant_ << ",\"conv_split_k\":" << forced_split_k_
-       << ",\"host_threads\":" << HostCopier::get().threads()
+       << ",\"staged_bytes\":" << stage_.staged_bytes() << ",\"host_threads\":" << HostCopier::get().threads()
        << ",\"arena_reuse\":" << (planner_arena_reuse() ? "true" : "false")
        << ",\"max_groups\":" << kMaxGroups << ",\"conv_variants\":[";
     for (int i = 0; i < conv_num_variants(); i++) os << (i ? "," : "") << '"' << conv_variant(i).name << '"';
@@ -506,6 +509,16 @@ std::string DeviceContext::info_json() const {
 
 // ---- session ---------------------------------------------------------------------------------------------------------
 Session::Session(Plan plan, Storage storage, bool pack_filters) : plan_(std::move(plan)), ctx_(DeviceContext::get()) {
+    ctx_.sessions++;
+    try {
+        acquire(storage, pack_filters);
+    } catch (...) {
+        release();   // the destructor does not run for a constructor that throws
+        throw;
+    }
+}
+
+void Session::acquire(Storage storage, bool pack_filters) {
     if (storage == Storage::Static) {
         const size_t need = plan_.arena_floats * sizeof(float);
         if (need > DeviceContext::static_scratch_bytes())
@@ -521,12 +534,7 @@ Session::Session(Plan plan, Storage storage, bool pack_filters) : plan_(std::mov
         IOS_HIP(hipMalloc(reinterpret_cast<void **>(&base_), std::max<size_t>(plan_.arena_floats, 64) * sizeof(float)));
         owns_memory_ = true;
     }
-    try {
-        setup(pack_filters);
-    } catch (...) {
-        release();   // the destructor does not run for a constructor that throws
-        throw;
-    }
+    setup(pack_filters);
 }
 
 Session::~Session() { release(); }
@@ -553,6 +561,8 @@ void Session::release() noexcept {
     start_ = stop_ = nullptr;
     fused_items_ = nullptr;
     base_ = nullptr;
+    if (!released_ && --ctx_.sessions == 0) ctx_.stage().give_back();   // (pinned memory for inputs and weights: up to 256 MB each)
+    released_ = true;
 }
 
 TensorView Session::tv(const ViewRef &v) const {

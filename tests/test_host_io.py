@@ -1,4 +1,5 @@
 """Transfers between a caller's arrays and the device at the sizes where the paths of csrc/host_io.hip change over."""
+import gc
 import time
 
 import numpy as np
@@ -259,3 +260,36 @@ def test_host_threads():
             rt.set_option('host_threads', -1)
     finally:
         rt.set_option('host_threads', 0)
+
+
+def test_staging_memory_goes_with_the_last_session():
+    """67 MB of input: its staging buffer stays while there is a session, and shrinks to 16 MB at most behind the last one."""
+    gc.collect()
+    rt.set_option('release_staging', 1)
+    assert rt.device_info()['staged_bytes'] <= 32 << 20
+    small, large = rt.Session(relu_graph(1, 1, 100), 1), rt.Session(relu_graph(1, 4096, 4096), 1)
+    x = np.random.default_rng(0).standard_normal(large.input_shape, dtype=np.float32)
+    for _ in range(2):
+        large.set_input(x)
+        large.run()
+        assert np.array_equal(large.output(), np.maximum(x, 0))
+    assert rt.device_info()['staged_bytes'] >= 64 << 20
+    large.close()
+    assert rt.device_info()['staged_bytes'] >= 64 << 20
+    small.close()
+    assert rt.device_info()['staged_bytes'] <= 32 << 20
+    with rt.Session(relu_graph(1, 4096, 4096), 1) as again:
+        again.set_input(-x)
+        again.run()
+        assert np.array_equal(again.output(), np.maximum(-x, 0))
+    # inference calls alone keep it, also where an option makes them plan anew
+    graph = relu_graph(1, 4096, 4096)
+    for _ in range(2):
+        assert np.array_equal(rt.graph_inference(graph, 1, x), np.maximum(x, 0))
+        assert rt.device_info()['staged_bytes'] >= 64 << 20
+        rt.set_option('executor', 'fused')
+        assert rt.device_info()['staged_bytes'] >= 64 << 20
+    rt.set_option('release_staging', 1)
+    assert rt.device_info()['staged_bytes'] <= 32 << 20
+    assert np.array_equal(rt.graph_inference(graph, 1, -x), np.maximum(-x, 0))
+    rt.set_option('release_staging', 1)
