@@ -1231,6 +1231,7 @@ void Session::measure(int warmup, int number, int repeat, bool profile_stage, fl
     auto pass = [&]() {
         if (profile_stage) {
             settle();
+            ran_in_parts_ = input_changed_ = false;
             enqueue(0, true);
         }
         else forward();
@@ -1290,7 +1291,8 @@ void Session::profile_ops(int warmup, int repeat, float *ms_out) {
     if (repeat < 1 || warmup < 0) throw std::runtime_error("profile_ops: warmup >= 0 and repeat >= 1 required");
     ensure_timers();
     hipStream_t main = ctx_.stream(0);
-    run();   // every operator sees the inputs it has in a real pass
+    settle();
+    run();   // every operator sees the inputs it has in a real pass, on the whole batch
     for (size_t i = 0; i < plan_.ops.size(); i++) {
         const PlanOp &op = plan_.ops[i];
         for (int w = 0; w < warmup; w++) launch_op(op, 0);
@@ -1391,7 +1393,8 @@ void Session::profile_launches(int warmup, int repeat, float *ms_out, int capaci
     if ((int)list.size() > capacity) throw std::runtime_error("profile_launches: output array too small");
     ensure_timers();
     hipStream_t main = ctx_.stream(0);
-    run();   // every launch sees the inputs it has in a real pass
+    settle();
+    run();   // every launch sees the inputs it has in a real pass, on the whole batch
     const WorkItem *items = static_cast<const WorkItem *>(fused_items_);
     for (size_t i = 0; i < list.size(); i++) {
         const LaunchRecord &r = list[i];

@@ -156,14 +156,14 @@ def test_tensors_of_a_batch_that_arrived_in_parts(batch, side, executor):
                 session.set_input(x)
                 session.run()
                 got = session.output()
-                asked = 0
+                held = []
                 for value in (a, b, c, d):
                     try:
                         tensor = session.tensor(value.node)
                     except RuntimeError as e:
                         assert 'shares its memory' in str(e)
                         continue
-                    asked += 1
+                    held.append(value)
                     for i in (0, batch // 3, batch - 1):
                         single.set_input(x[i:i + 1])
                         single.run()
@@ -172,8 +172,16 @@ def test_tensors_of_a_batch_that_arrived_in_parts(batch, side, executor):
                         except RuntimeError as e:
                             assert 'shares its memory' in str(e)
                         assert np.allclose(got[i:i + 1], single.output(), rtol=1e-4, atol=1e-5)
-                assert asked > 0 and np.array_equal(got, session.output())
+                assert held and np.array_equal(got, session.output())
                 session.run()   # the same input again, now resident
+                assert np.array_equal(got, session.output())
+            # a timed pass and a profile work on the whole batch, also where the input has only just been set
+            for profile in (lambda: session.measure(0, 1, 1, profile_stage=True), session.profile_ops, session.profile_launches):
+                session.set_input(x)
+                profile()
+                tensors = [session.tensor(value.node) for value in held]
+                session.run()
+                assert held and all(np.array_equal(t, session.tensor(value.node)) for t, value in zip(tensors, held))
                 assert np.array_equal(got, session.output())
             # an input that no pass has worked on: tensors of the last pass are there or are refused, the result is the last pass's
             session.set_input(-x)
