@@ -719,6 +719,7 @@ void Session::get_tensor(const std::string &name, float *host) {
             throw std::runtime_error("the last pass worked on parts of the batch, held the output of operator '" + name + "' for one part at a time, and its "
                                      "input or weights have changed since (option arena_reuse=0 keeps every output)");
         forward();
+        synchronize();
     }
     copy_out(it->second, host);
 }
