@@ -618,11 +618,214 @@ __device__ __forceinline__ void split_bf16x3(const float (&x)[8], uintx4 &hi, ui
     }
 }
 
+// ---- fp32 operands as two terms of IEEE half -------------------------------------------------------------------------------
+// x = hi + lo with hi the nearest half of x and lo the nearest half of the remainder holds 23 of an fp32 value's 24 significant
+// bits (the remainder has twelve bits and a sign, a half takes eleven of them: the last one is lost for a quarter of the values,
+// the other values are exact).  A product is then the sum of three products of halves, each exact in fp32 (hi * hi, hi * lo,
+// lo * hi; the fourth is below 2^-22 of it), against the six of three bfloat16 terms: half the matrix instructions, two operand
+// planes instead of three, four vector instructions per split value instead of seven.  What bounds an fp32 result is the rounding of
+// its sum, and a sum of half as many terms is rounded half as often.  Relative error (2-norm) against 64 bits, three terms -> two, of
+// the LDS-tiled kernels: 1.8e-7 -> 1.5e-7 at K = 131, 4.2e-7 -> 3.1e-7 at 768, 9.5e-7 -> 6.6e-7 at 4032; of four wavefronts that share K: 1.14e-7 ->
+// 1.10e-7, 2.2e-7 -> 1.7e-7, 4.8e-7 -> 3.5e-7.  Below K = 64 the lost bits of the operands weigh more (7.1e-8 -> 8.3e-8 at 16): the tuner does
+// not let the two-term kernels compete there.
+//
+// A half has five bits of exponent, so operands are scaled by powers of two (exact).  Filters: every output channel by its own
+// factor, which puts its largest filter value into [2^14, 2^15); the factors that undo it follow the packed planes.  Inputs: by
+// kHalfScale, their lower term by 2^11 more, which keeps it out of the subnormal halves (its partner, the upper term of the filter,
+// is taken times 2^-11).  That represents inputs up to kHalfMost, with 23 bits from 2^-10 on and to within 2^-32 below.  A
+// wavefront keeps the largest magnitude it has seen; where that is beyond kHalfMost, or so small that 2^-32 would show in the
+// result (below kHalfLeast), the tile is computed again with a factor made for it, and from kHalfWide on (and for
+// infinities) with plain fp32 multiply-adds, which have no limit.
+constexpr float kHalfScale = 0.0625f;
+constexpr float kHalfMost = 65504.f * 16.f;
+constexpr float kHalfLeast = 0.0078125f;
+constexpr float kHalfWide = 67108864.f;
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+
+// the two terms of eight values times `scale` (the lower one times 2^11), each as four words of two halves (lower k in the lower
+// half).  The additions of zero make every step one mixed-precision multiply-add (v_fma_mix*, three per value; products that are
+// converted take five instructions).  No assembly: the compiler does not know what wait the matrix instructions need behind that.
+__device__ __forceinline__ void split_half2(const float (&x)[8], float scale, uintx4 &hi, uintx4 &lo) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        halfx2 h, l;
+#pragma unroll
+        for (int u = 0; u < 2; u++) h[u] = (_Float16)__builtin_fmaf(x[2 * i + u], scale, 0.f);
+#pragma unroll
+        for (int u = 0; u < 2; u++) l[u] = (_Float16)__builtin_fmaf(__builtin_fmaf(x[2 * i + u], scale, -(float)h[u]), 2048.f, 0.f);   // (the inner one is exact)
+        hi[i] = __builtin_bit_cast(unsigned, h);
+        lo[i] = __builtin_bit_cast(unsigned, l);
+    }
+}
+// the upper term of a filter operand times 2^-11
+__device__ __forceinline__ uintx4 half_down(uintx4 v) {
+    return __builtin_bit_cast(uintx4, __builtin_bit_cast(halfx8, v) * (_Float16)0.00048828125f);
+}
+// Largest magnitude of eight values and `peak`; NaN does not count.  (The empty assembly keeps the maximum where the values are: put
+// off to the end of the loop that stages them, it keeps all of them in registers.)
+__device__ __forceinline__ float half_peak(const float (&x)[8], float peak) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) peak = fmaxf(fmaxf(fabsf(x[i]), fabsf(x[i + 1])), peak);
+    asm("" : "+v"(peak));
+    return peak;
+}
+// factor for inputs of magnitude `peak` > 0 at most: puts them below 2^15
+__device__ __forceinline__ float half_scale_for(float peak) {
+    const int e = (int)(__float_as_uint(peak) >> 23) - 127;   // -127 for subnormal values
+    return __uint_as_float((unsigned)(min(14 - e, 120) + 127) << 23);
+}
+// A tile is computed with kHalfScale first and where its inputs want that once more with the factor the first attempt returns (0: by
+// plain multiply-adds).  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to
+// 100 registers.  again() keeps it from sharing what both attempts derive from the lane.
+constexpr float kHalfDone = -1.f;
+template <typename Attempt>
+__device__ __forceinline__ void half_attempts(Attempt attempt) {
+    const float next = attempt(kHalfScale);
+    if (__builtin_expect(next >= 0.f, 0)) attempt(next);
+}
+__device__ __forceinline__ int again(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+// what half_attempts runs after an attempt with kHalfScale whose largest input was `peak`
+__device__ __forceinline__ float half_next_scale(float peak) {
+    if (peak == 0.f || (peak >= kHalfLeast && peak <= kHalfMost)) return kHalfDone;
+    return peak >= kHalfWide ? 0.f : half_scale_for(peak);
+}
+// Largest peak of the lanes of a wavefront; cheaper than that (and only some value half_next_scale lets pass) in the usual case.
+__device__ __forceinline__ float half_wave_peak(float peak) {
+    if (__ballot(peak > kHalfMost) == 0 && __ballot(peak >= kHalfLeast) != 0) return kHalfLeast;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) peak = fmaxf(peak, __shfl_xor(peak, d));
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
+}
+// The same over the wavefronts of a block: a barrier in the usual case.  `words`: one per wavefront that nothing else uses until the
+// next barrier.
+template <int WAVES>
+__device__ __forceinline__ float half_block_peak(float peak, float *words) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned *flags = reinterpret_cast<unsigned *>(words);
+    const unsigned mine = (__ballot(peak > kHalfMost) != 0 ? 1u : 0u) | (__ballot(peak >= kHalfLeast) != 0 ? 2u : 0u);
+    if ((threadIdx.x & 63) == 0) flags[wave] = mine;
+    __syncthreads();
+    unsigned all = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) all |= flags[w];
+    if (__builtin_amdgcn_readfirstlane(all) == 2u) return kHalfLeast;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) peak = fmaxf(peak, __shfl_xor(peak, d));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) words[wave] = peak;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) peak = fmaxf(peak, words[w]);
+    __syncthreads();
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
+}
+
+// Factors that undo the scaling of output channels m ... m + 3 of group g (behind the packed planes; the quad that straddles the end
+// reads on into the padding the host reserves).
+__device__ __forceinline__ floatx4 channel_scale_quad(const ConvKernelArgs &a, int g, int m) {
+    const float *scales = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.wp) + a.w_bytes);
+    return *reinterpret_cast<const floatx4_u *>(scales + g * a.OCg + min(m, a.OCg - 1));
+}
+
+// sums of scaled filters -> sums of the filters as they were given, times `more` (exact); m_base: row 0 of the tiles
+template <int TM, int TN>
+__device__ __forceinline__ void scale_channels(const ConvKernelArgs &a, floatx16 (&acc)[TM][TN], int g, int m_base, float more) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const floatx4 factor = channel_scale_quad(a, g, m_base + i * 32 + Mfma<32>::row(4 * q, lane)) * more;
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[i][j][4 * q + v] *= factor[v];
+        }
+}
+
+// The accumulators of TM x TN tiles of 32 x 32 by fp32 multiply-adds, from the packed halves: for inputs no factor serves.  m_base: row
+// 0 of the tiles; n: this lane's column in tile column j, or negative; K as [k_begin, k_end) of the packed rows, restricted to
+// channels [c_begin, c_end).  The sums are those of the filters as they were given.  Slow on purpose: it takes few registers and runs for values beyond 2^26.
+template <int TM, int TN, typename Pixel>
+__device__ __forceinline__ void half_exact_tiles(const ConvKernelArgs &a, floatx16 (&acc)[TM][TN], int g, int m_base, Pixel n_of, int k_begin,
+                                                 int k_end, int c_begin, int c_end) {
+    const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
+    const int lane = threadIdx.x & 63;
+    const float floor = relu_floor(a.pre_relu != 0);
+    const _Float16 *planes = reinterpret_cast<const _Float16 *>(a.wp);
+    const int taps = a.Kq / a.ICgP;
+#pragma unroll 1
+    for (int quad = 0; quad < TM * TN * 4; quad++) {
+        const int q = quad & 3, j = (quad >> 2) % TN, i = (quad >> 2) / TN;
+        const int m = min(m_base + i * 32 + 8 * q + 4 * (lane >> 5), a.OCgP - 4);   // (rows come in fours)
+        const int n = n_of(j);
+        const int nn = n >= 0 ? n : 0;
+        const int b = (int)fast_div((unsigned)nn, a.div_ohw);
+        const int r = nn - b * a.OHW;
+        const int oh = (int)fast_div((unsigned)r, a.div_ow);
+        const int ow = r - oh * a.OW;
+        floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+        const floatx4 factor = channel_scale_quad(a, g, m) * kHalfScale;
+#pragma unroll 1
+        for (int tap = 0; tap < taps; tap++) {
+            const int kh = tap / a.KW, kw = tap - kh * a.KW;
+            const int ih = oh * a.sh - a.ph + kh, iw = ow * a.sw - a.pw + kw;
+            const bool ok = n >= 0 && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
+            const unsigned at = (((unsigned)(b * a.H + ih) * (unsigned)a.W + (unsigned)iw) * (unsigned)a.x_ps + (unsigned)(g * a.ICg)) * 4u;
+            const int first = max(c_begin, k_begin - tap * a.ICgP), last = min(min(c_end, a.ICg), k_end - tap * a.ICgP);
+#pragma unroll 1
+            for (int c = first; c < last; c++) {
+                const float x = relu_above(floor, buffer_load_f32(xr, ok ? at + (unsigned)c * 4u : kOutOfRange));
+                const int k = tap * a.ICgP + c;
+                const size_t slot = (((size_t)g * (a.Kq >> 3) + (k >> 3)) * 2 * a.OCgP + m) * 8 + (k & 7);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float w = (float)planes[slot + v * 8] + (float)planes[slot + v * 8 + (size_t)a.OCgP * 8];
+                    sum[v] = __builtin_fmaf(w * factor[v], ok ? x : 0.f, sum[v]);
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < TM * TN * 4; e++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                floatx16 &to = acc[(e >> 2) / TN][(e >> 2) % TN];
+                to[4 * (e & 3) + v] = quad == e ? sum[v] : to[4 * (e & 3) + v];
+            }
+    }
+}
+
 // eight fp32 values rounded to bfloat16 (nearest even), as four words of two (lower k in the lower half)
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ uintx4 round_bf16x8(const float (&x)[8]) {
     const floatx8 v = {x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
     return __builtin_bit_cast(uintx4, __builtin_convertvector(v, bf16x8));
+}
+
+// TM x TN tiles of 32 x 32 and one unit of 16 k: filter operands av, input operands bv, a plane per term.  Two terms take three
+// instructions, smallest product first; the tiles of a product are independent instructions.
+template <int TERMS, bool HALF, int TM, int TN>
+__device__ __forceinline__ void multiply_terms(floatx16 (&acc)[TM][TN], const uintx4 (&av)[TERMS][TM], const uintx4 (&bv)[TERMS][TN]) {
+    auto product = [&](auto filter, int plane) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                if constexpr (HALF)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, filter(i)), __builtin_bit_cast(halfx8, bv[plane][j]), acc[i][j], 0, 0, 0);
+                else
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, filter(i)), __builtin_bit_cast(bf16x8, bv[plane][j]), acc[i][j], 0, 0, 0);
+            }
+    };
+    if constexpr (TERMS == 2) {
+        product([&](int i) { return av[1][i]; }, 0);
+        product([&](int i) { return half_down(av[0][i]); }, 1);
+    }
+    product([&](int i) { return av[0][i]; }, 0);
 }
 
 // TMW x TNW MFMA tiles of 32 x 32 per wavefront, WM x WN wavefronts per block
@@ -865,26 +1068,28 @@ struct ConvWsplit {
     static constexpr int BM = TM * MT, BN = TN * MT;
     static constexpr int E = TM * TN * M::ACC;
     static constexpr int THREADS = 64 * NW;
-    static constexpr int SMEM_FLOATS = NW * E * 64;
+    static constexpr int SMEM_FLOATS = NW * E * 64 + (RP == 3 ? NW : 0);   // (two terms: a flag per wavefront behind the tiles)
     static constexpr int CPAD = CP ? CP : (QUAD ? U * M::KSTEP : 8);   // channel padding of the packed filters this kernel expects
     static_assert(CP == 0 || (!QUAD && CP % M::KSTEP == 0), "a k-step must lie inside one filter tap");
     static constexpr bool KQUAD = QUAD;                    // packed filters are [k / 4][m][4] instead of [k][m]
     // accumulators + staged operands per lane decide whether the body fits the register budget of a fused launch
     // (the channel-padding-4 forms serve first layers, which are stages of their own: kept out of the fused launches)
     static constexpr bool FUSABLE = RP < 3 && CP == 0 && E + D * U * (TM + TN) <= (QUAD ? (MT == 32 ? 48 : 56) : 48);   // per-step addressing of the plain layout needs more registers, and so do the 16-register accumulator tuples of the 32 x 32 tiles
-    // the three-term bodies of up to two 32 x 32 tiles per wavefront (100-155 registers) run inside fused launches of the
+    // the two-term bodies of up to two 32 x 32 tiles per wavefront run inside fused launches of the
     // wide-register kernel family (fused_kernel_wide)
     static constexpr bool FUSABLE_WIDE = RP == 3 && NW <= 8 && TM * TN <= 2;
-    static constexpr int KREDUCED = RP;                    // 0: fp32 filters; 1: packed filters hold bfloat16; 2: IEEE half; 3: three bfloat16 planes; 4: one
-    static constexpr int PLANES = RP == 3 ? 3 : 1;
+    static constexpr int KREDUCED = RP;                    // 0: fp32 filters; 1: packed filters hold bfloat16; 2: IEEE half; 3: two planes of half; 4: one of bfloat16
+    static constexpr int PLANES = RP == 3 ? 2 : 1;
+    static constexpr int WAVES_PER_SIMD = RP != 3 ? 1 : TM * TN == 1 ? 5 : TM * TN == 2 ? 3 : 2;
     // RP == 4: the reduced-precision mode on the same instruction and layout: one plane of filters rounded to bfloat16, inputs
     // rounded after the load, one matrix instruction per tile and batch.
-    // RP == 3: fp32 results from the bfloat16 matrix pipe, as in ConvSplit3 (operands split exactly into three bfloat16 terms,
-    // six of the nine partial products on v_mfma_f32_32x32x16_bf16): filters are split when packed, [k / 8][plane][m][8], and read
-    // as operands straight from global memory; a lane splits the eight input values it loads for a batch itself.
+    // RP == 3: fp32 results from the half matrix pipe (operands as two terms, three products on v_mfma_f32_32x32x16_f16, see
+    // split_half2): filters are split when packed, [k / 8][plane][m][8], and read as operands straight from global memory; a lane
+    // splits the eight input values it loads for a batch itself.  Every wavefront decides by itself whether its inputs want another
+    // factor, or plain multiply-adds.
     static_assert(!QUAD || U % 4 == 0, "quad loads need whole groups of four k per lane");
     static_assert(RP >= 0 && RP <= 4 && (RP == 0 || (RP >= 3 ? QUAD && MT == 32 && U == 8 : QUAD && MT == 16 && U == 4)),
-                  "the 16-bit paths are the 16 x 16 x 16 form of the quad layout, the three-term path its 32 x 32 x 16 form");
+                  "the 16-bit paths are the 16 x 16 x 16 form of the quad layout, the two-term path its 32 x 32 x 16 form");
 
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *red, int tile, int g, int z) {
@@ -906,6 +1111,25 @@ struct ConvWsplit {
     const int s_begin = s_lo + wave * a.steps_per_wave;
     const int s_end = min(s_hi, s_begin + a.steps_per_wave);
 
+    // the bias of the outputs this lane finishes in the epilogue (and the factors of their channels, with two terms), requested
+    // ahead of the K loop so that its latency hides behind it (a wavefront finishes whole quads of consecutive output channels)
+    constexpr int G = E / 4;
+    constexpr int GPW = (G + NW - 1) / NW;
+    auto quad_row = [&](int e4) { return m0 + (4 * e4 / (M::ACC * TN)) * MT + M::row((4 * e4) % M::ACC, lane); };
+    floatx4 bias_pre[GPW], factor_pre[RP == 3 ? GPW : 1];
+    auto request_bias = [&] {
+#pragma unroll
+        for (int t = 0; t < GPW; t++) {
+            const int row = quad_row(min(wave + t * NW, G - 1));
+            bias_pre[t] = bias_quad(a, g, row);
+            if constexpr (RP == 3) factor_pre[t] = channel_scale_quad(a, g, row);
+        }
+    };
+    // the sums of this wavefront's K range into acc (two terms: of inputs times `scale`); returns the largest input magnitude (two terms)
+    auto sums = [&](typename M::acc_t (&acc)[TM][TN], const int lane, const float scale) {
+    const int lk = lane / MT;
+    const int lc = lane % MT;
+    float peak = 0.f;
     int ih0[TN], iw0[TN];
     unsigned x_lane[TN];   // byte offset of (image, ih0, iw0, first channel of the lane); may wrap below zero, the tap offset brings it back
     bool n_ok[TN];
@@ -943,15 +1167,7 @@ struct ConvWsplit {
 #pragma unroll
     for (int j = 0; j < TN; j++) n_kill[j] = n_ok[j] ? 0u : kOutOfRange;
 
-    // the bias of the outputs this lane finishes in the epilogue, requested now so that its latency hides behind the K loop
-    // (a wavefront finishes whole quads of consecutive output channels)
-    constexpr int G = E / 4;
-    constexpr int GPW = (G + NW - 1) / NW;
-    auto quad_row = [&](int e4) { return m0 + (4 * e4 / (M::ACC * TN)) * MT + M::row((4 * e4) % M::ACC, lane); };
-    floatx4 bias_pre[GPW];
-#pragma unroll
-    for (int t = 0; t < GPW; t++) bias_pre[t] = bias_quad(a, g, quad_row(min(wave + t * NW, G - 1)));
-    typename M::acc_t acc[TM][TN];
+    if constexpr (RP != 3) request_bias();
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -1090,27 +1306,16 @@ struct ConvWsplit {
                 for (int j = 0; j < TN; j++) B[u][j] = u <= left ? B[u][j] : 0.f;
         }
         if constexpr (RP == 3) {
-            bf16x8 bq[3][TN];
+            uintx4 bq[2][TN];
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 float v[8];
 #pragma unroll
                 for (int u = 0; u < 8; u++) v[u] = relu_above(floor, B[u][j]);
-                uintx4 hi, mid, lo;
-                split_bf16x3(v, hi, mid, lo);
-                bq[0][j] = __builtin_bit_cast(bf16x8, hi);
-                bq[1][j] = __builtin_bit_cast(bf16x8, mid);
-                bq[2][j] = __builtin_bit_cast(bf16x8, lo);
+                peak = half_peak(v, peak);
+                split_half2(v, scale, bq[0][j], bq[1][j]);
             }
-            // the six terms, smallest first; the tiles of a term are independent instructions
-            constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-            for (int t = 0; t < 6; t++)
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, A.v[TA[t]][i]), bq[TB[t]][j], acc[i][j], 0, 0, 0);
+            multiply_terms<2, true>(acc, A.v, bq);
             return;
         } else if constexpr (RP == 4) {
             // one rounded term: the reduced-precision mode on the 32 x 32 x 16 instruction
@@ -1208,24 +1413,70 @@ struct ConvWsplit {
         }
     };
     k_loop();
-
+    return peak;
+    };
     // partial tiles meet in LDS: quad e4 (accumulator elements 4 * e4 ... + 3) of lane l of wavefront w lives in
     // red4[(w * G + e4) * 64 + l]
     floatx4 *red4 = reinterpret_cast<floatx4 *>(red);
+    auto hand_over = [&](const typename M::acc_t (&acc)[TM][TN]) {
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+            for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int q = 0; q < M::ACC / 4; q++) {
-                const floatx4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                red4[(wave * G + (i * TN + j) * (M::ACC / 4) + q) * 64 + lane] = v;
+                for (int q = 0; q < M::ACC / 4; q++) {
+                    const floatx4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    red4[(wave * G + (i * TN + j) * (M::ACC / 4) + q) * 64 + lane] = v;
+                }
+    };
+    // two terms: whether a wavefront's sums are those of the filters as they were given (see half_exact_tiles), not of the scaled ones
+    int *exact_flags = reinterpret_cast<int *>(red) + NW * E * 64;
+    {
+        typename M::acc_t acc[TM][TN];
+        if constexpr (RP == 3 && GPW == 1) request_bias();
+        const float peak = sums(acc, lane, kHalfScale);
+        if constexpr (RP == 3 && GPW > 1) request_bias();   // (more of them wait until the K loop has given its registers back)
+        hand_over(acc);
+        if constexpr (RP == 3) {
+            const float next = half_next_scale(half_wave_peak(peak));
+            if (lane == 0) exact_flags[wave] = next == 0.f ? 1 : 0;
+            if (__builtin_expect(next >= 0.f, 0)) {   // again, with another factor or by plain multiply-adds
+                typename M::acc_t acc[TM][TN];
+                if (next == 0.f) {
+                    half_exact_tiles(a, acc, g, m0, [&](int j) {
+                        const int n = n0 + j * MT + lc;
+                        return n < a.Npix ? n : -1;
+                    }, s_begin * M::KSTEP, s_end * M::KSTEP, 0, a.ICgP);
+                } else {
+                    (void)sums(acc, again(lane), next);
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int j = 0; j < TN; j++) acc[i][j] *= kHalfScale / next;
+                }
+                hand_over(acc);
             }
+        }
+    }
     __syncthreads();
-    auto meet = [&](int e4) {   // wavefronts in ascending order
+    auto meet = [&](int t) {   // quad wave + t * NW of the tile: wavefronts in ascending order
+        const int e4 = wave + t * NW;
         floatx4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; w++) sum += red4[(w * G + e4) * 64 + lane];
+        if constexpr (RP == 3) {
+            int any = 0;
+#pragma unroll
+            for (int w = 0; w < NW; w++) any |= exact_flags[w];
+            sum *= factor_pre[t];
+            if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) != 0, 0)) {
+                sum = floatx4{0.f, 0.f, 0.f, 0.f};
+                for (int w = 0; w < NW; w++) {
+                    const floatx4 part = red4[(w * G + e4) * 64 + lane];
+                    sum += exact_flags[w] != 0 ? part : part * factor_pre[t];
+                }
+            }
+        }
         return sum;
     };
     auto quad_pixel = [&](int e4) { return n0 + ((4 * e4 / M::ACC) % TN) * MT + lc; };
@@ -1233,8 +1484,11 @@ struct ConvWsplit {
         // two-kernel split-K: this slice's partial outputs as [slice][pixel][channel] for splitk_reduce_kernel
         const size_t channels = (size_t)a.groups * a.OCg;
         float *wsz = a.ws + (size_t)z * channels * (size_t)a.Npix + (size_t)g * a.OCg;
-        for (int e4 = wave; e4 < G; e4 += NW) {
-            const floatx4 sum = meet(e4);
+#pragma unroll
+        for (int t = 0; t < GPW; t++) {
+            const int e4 = wave + t * NW;
+            if (e4 >= G) break;
+            const floatx4 sum = meet(t);
             const int m = quad_row(e4), nn = quad_pixel(e4);
 #pragma unroll
             for (int c = 0; c < 4; c++)
@@ -1253,8 +1507,11 @@ struct ConvWsplit {
         auto hand_in = [&](auto local) {
             constexpr bool LOCAL = decltype(local)::value;
             float *mine = slices + (size_t)z * (BM * BN) + lane;
-            for (int e4 = wave; e4 < G; e4 += NW) {
-                const floatx4 sum = meet(e4);
+#pragma unroll
+            for (int t = 0; t < GPW; t++) {
+                const int e4 = wave + t * NW;
+                if (e4 >= G) break;
+                const floatx4 sum = meet(t);
 #pragma unroll
                 for (int c = 0; c < 4; c++) partial_store<LOCAL>(mine + (4 * e4 + c) * 64, sum[c]);
             }
@@ -1282,7 +1539,7 @@ struct ConvWsplit {
                     sum[c] += xcd_local ? partial_load<true>(p) : partial_load<false>(p);
                 }
         } else {
-            sum = meet(e4);
+            sum = meet(t);
         }
         const int m = quad_row(e4), nn = quad_pixel(e4);
         if (m < a.OCg && nn < a.Npix) finish_quad<RES>(a, sum, bias_pre[t], g, m, nn);
@@ -1409,7 +1666,7 @@ struct ConvWsplit {
     X(95, "x3_m128n64_w4x1", 1, 2, 4, 1, 2)        \
     X(96, "x3_m128n128_w4x2", 1, 2, 4, 2, 2)       \
     X(97, "x3_m192n128_w6x2", 1, 2, 6, 2, 2)
-// X(index, name, TM, TN, NW, D): wave-split configurations with operands split into three bfloat16 terms (ConvWsplit, RP = 3),
+// X(index, name, TM, TN, NW, D): wave-split configurations with operands as two terms of half (ConvWsplit, RP = 3),
 // 32 x 32 x 16 tiles, 16 k per batch
 #define IOS_WSPLIT_X3_VARIANTS(X)            \
     X(98, "x3w_m32n32_w8", 1, 1, 8, 2)       \

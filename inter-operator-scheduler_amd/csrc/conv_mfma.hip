@@ -43,7 +43,7 @@ struct VariantEntry {
      ConvSplit3<TMW, TNW, WM, WN, PD>::SMEM_FLOATS},
 
 #define IOS_WSPLIT_X3_ENTRY(IDX, NAME, TM, TN, NW, D)                                                                        \
-    {{NAME, TM * 32, TN * 32, 16, 1, 1, NW, 32, true, ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::CPAD, true, false, PREC_FP32, 3, \
+    {{NAME, TM * 32, TN * 32, 16, 1, 1, NW, 32, true, ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::CPAD, true, false, PREC_FP32, 2, \
       ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::FUSABLE_WIDE},      \
      conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>, true>,              \
      ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::SMEM_FLOATS},
@@ -59,21 +59,21 @@ struct VariantEntry {
      conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>, true>,              \
      ConvWsplit<32, TM, TN, NW, 8, true, D, 4>::SMEM_FLOATS},
 
-#define IOS_PIPE_ENTRY(TERMS, HALF, PRECISION, NAME, KU, PD, TMW, TNW, WM, WN)                                                       \
+#define IOS_PIPE_ENTRY(TERMS, HALF, PRECISION, IDX, NAME, KU, PD, TMW, TNW, WM, WN)                                                       \
     {{NAME, ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::BM, ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::BN, 16 * KU, WM, WN, 1, 32, \
       false, 16, false, false, PRECISION, TERMS},                                                                                     \
-     conv_kernel<ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>>, conv_kernel<ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>, true>,  \
+     kPipeKernels[IDX - kFirstPipeVariant].kernel, kPipeKernels[IDX - kFirstPipeVariant].kernel_residual,                               \
      ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::SMEM_FLOATS},
-#define IOS_PIPE3_ENTRY(IDX, ...) IOS_PIPE_ENTRY(3, false, PREC_FP32, __VA_ARGS__)
-#define IOS_PIPE_BF16_ENTRY(IDX, ...) IOS_PIPE_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
-#define IOS_PIPE_FP16_ENTRY(IDX, ...) IOS_PIPE_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
+#define IOS_PIPE3_ENTRY(...) IOS_PIPE_ENTRY(2, true, PREC_FP32, __VA_ARGS__)
+#define IOS_PIPE_BF16_ENTRY(...) IOS_PIPE_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
+#define IOS_PIPE_FP16_ENTRY(...) IOS_PIPE_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
 
 #define IOS_WINDOW_ENTRY(TERMS, HALF, PRECISION, IDX, NAME, TMW, TNW, WM, WN, P_IT, NBUF)                                                 \
     {{NAME, 32 * TMW * WM, 32 * TNW * WN, 16, WM, WN, 1, 32, false, 16, false, false, PRECISION, TERMS, false,                            \
       ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SPAN},                                                                     \
      kWindowKernels[IDX - kFirstWindowVariant].kernel, kWindowKernels[IDX - kFirstWindowVariant].kernel_residual,                          \
      ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SMEM_FLOATS},
-#define IOS_WINDOW3_ENTRY(...) IOS_WINDOW_ENTRY(3, false, PREC_FP32, __VA_ARGS__)
+#define IOS_WINDOW3_ENTRY(...) IOS_WINDOW_ENTRY(2, true, PREC_FP32, __VA_ARGS__)
 #define IOS_WINDOW_BF16_ENTRY(...) IOS_WINDOW_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
 #define IOS_WINDOW_FP16_ENTRY(...) IOS_WINDOW_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
 
@@ -119,7 +119,7 @@ bool conv_variant_takes(const ConvProblem &p, int variant) {
 // Configurations that the tuner leaves out.  None of them was the fastest in any share class over 3030 problems: the convolutions of
 // nine networks (Inception-v3, SqueezeNet, ResNet-18 / 50, RandWire, NASNet, VGG-16, AlexNet, the sample network) at batch 1 to 64 and
 // of multi-branch blocks on odd sizes, in each precision; nor, each pinned in turn, on 31 more from 8 -> 8 channels on 8 x 8 pixels to
-// 4096 -> 4096 on one and 700 -> 300 on 80 x 80.  (The fp32 matrix instructions lose to three bfloat16 terms from a few
+// 4096 -> 4096 on one and 700 -> 300 on 80 x 80.  (The fp32 matrix instructions lose to two terms of half from a few
 // microseconds on.)  They serve the closed-form choice, which knows none of the others, and the option that pins a configuration.
 static const char *const kNotMeasured[] = {
     "m64n64k32_w2x2x1_t32", "m128n128k16_w2x2x1_t32", "m32n32k64_w1x1x4_t32", "m64n32k32_w2x1x2_t32", "m32n64k32_w1x2x2_t32",
@@ -135,12 +135,20 @@ static const char *const kNotMeasured[] = {
     "wb_x1_m64n128_w2x2", "wb_x1_m128n256_w2x4", "wb_x1_m64n128_w1x2", "wb_x1_m64n256_w2x4",
 };
 
-bool conv_variant_measured(int variant) {
+static bool precise_only(const ConvProblem &p) { return p.K() < 64; }
+
+bool conv_variant_measured(const ConvProblem &p, int variant) {
     static const std::vector<char> measured = [] {
         std::vector<char> flags(kNumVariants, 1);
         for (const char *name : kNotMeasured) flags[variant_by_name(name)] = 0;
         return flags;
     }();
+    // Two terms of half against three of bfloat16: half the matrix work, and half the roundings of the sum, but operands that are off in
+    // the last bit.  Below a K of 64 the second shows (errors 8.3e-8 against 7.1e-8 at K = 16), and nothing there is bound by matrix work
+    // (16 -> 64 channels on 55 x 55 at batch 50: 13.1 us by fp32 instructions, 15.2 by two terms); from 64 on the first (2.7e-7 against
+    // 3.6e-7 at K = 576), and the three-term kernels are slower or within 1 %.
+    const int planes = kVariants[variant].v.koct;
+    if (precise_only(p) ? planes == 2 : planes == 3) return false;
     return measured.at(variant) != 0;
 }
 
@@ -391,12 +399,35 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
 }
 
 // ---- filter packing ------------------------------------------------------------------------
+// factors behind the planes of two-term filters: channel m's filters are packed times 16 / scale[m], which puts the largest of them
+// (infinities and NaN aside) into [2^14, 2^15); a block per output channel
+__global__ void filter_scale_kernel(const float *w, float *scales, int fan) {
+    const float *row = w + (size_t)blockIdx.x * fan;
+    unsigned most = 0;   // magnitudes compare as integers
+    for (int i = threadIdx.x; i < fan; i += 256) {
+        const unsigned v = __float_as_uint(row[i]) & 0x7fffffffu;
+        if (v < 0x7f800000u) most = max(most, v);
+    }
+    __shared__ unsigned waves[4];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, d));
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = most;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        most = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
+        // filters times 2^up; their results times 2^-up / kHalfScale (a row of zeros or of subnormal values: as far as it goes)
+        const int up = most == 0 ? 0 : min(14 - ((int)(most >> 23) - 127), 127);
+        scales[blockIdx.x] = __uint_as_float((unsigned)(127 + 4 - up) << 23);
+    }
+}
+
 __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int OCgP, int ICg, int ICgP, int taps, int groups, int kvec,
-                                    int precision, int planes) {
+                                    int precision, int planes, const float *scales) {
     // packed[g][k][m] = w[g * OCg + m][c][tap] with k = tap * ICgP + c;  rows with c >= ICg and columns with m >= OCg are zero.
     // kvec = 4: packed[g][k / 4][m][k % 4] instead (ICgP is a multiple of 4)
     // kvec = 8: planes of 16-bit values, packed[g][k / 8][plane][m][k % 8]: three planes with the exact three-term split of every
-    // filter value, or one plane with the value rounded to nearest even (the reduced-precision modes)
+    // filter value, two with its two terms of half (scaled, see filter_scale_kernel), or one plane with the value rounded to nearest
+    // even (the reduced-precision modes)
     const size_t total = (size_t)groups * taps * ICgP * OCgP;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         int m;
@@ -424,6 +455,12 @@ __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int 
                 out[at] = (unsigned short)(hi >> 16);
                 out[at + (size_t)OCgP * 8] = (unsigned short)(mid >> 16);
                 out[at + (size_t)OCgP * 16] = (unsigned short)(lo >> 16);
+            } else if (planes == 2) {
+                const float scaled = m < OCg ? value * (16.f / scales[g * OCg + m]) : 0.f;   // (powers of two)
+                const _Float16 hi = (_Float16)scaled;
+                _Float16 *out = reinterpret_cast<_Float16 *>(packed);
+                out[at] = hi;
+                out[at + (size_t)OCgP * 8] = (_Float16)(scaled - (float)hi);
             } else if (precision == PREC_FP16) {
                 reinterpret_cast<_Float16 *>(packed)[at] = (_Float16)value;   // round to nearest even
             } else {
@@ -435,19 +472,21 @@ __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int 
     }
 }
 
+static size_t packed_floats(const ConvProblem &p, const ConvVariant &v) {
+    const size_t elements = (size_t)p.groups * p.Kq(v.cpad) * p.OCgP();
+    if (v.koct == 2) return elements + p.OC + 3;   // two planes of half, the factors of the channels (read in quads)
+    if (v.koct) return (elements * v.koct + 1) / 2;   // planes of bfloat16
+    return v.precision != PREC_FP32 ? (elements + 1) / 2 : elements;
+}
+
 size_t conv_packed_floats(const ConvProblem &p, const ConvLaunch &l) {
     if (l.variant < 0 || l.variant >= kNumVariants) throw std::runtime_error("conv: bad variant");
-    const size_t elements = (size_t)p.groups * p.Kq(kVariants[l.variant].v.cpad) * p.OCgP();
-    if (kVariants[l.variant].v.koct) return (elements * kVariants[l.variant].v.koct + 1) / 2;   // planes of bfloat16
-    return kVariants[l.variant].v.precision != PREC_FP32 ? (elements + 1) / 2 : elements;
+    return packed_floats(p, kVariants[l.variant].v);
 }
 
 size_t conv_packed_floats_max(const ConvProblem &p) {
     size_t most = 0;
-    for (const VariantEntry &e : kVariants) {
-        const size_t elements = (size_t)p.groups * p.Kq(e.v.cpad) * p.OCgP();
-        most = std::max(most, e.v.koct ? (elements * e.v.koct + 1) / 2 : elements);
-    }
+    for (const VariantEntry &e : kVariants) most = std::max(most, packed_floats(p, e.v));
     return most;
 }
 
@@ -455,8 +494,10 @@ void launch_pack_filters(const ConvProblem &p, const ConvLaunch &l, const float 
     const int cpad = kVariants[l.variant].v.cpad;
     const size_t total = (size_t)p.groups * p.Kq(cpad) * p.OCgP();   // elements
     const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 65535);
+    float *scales = packed + total;   // (two planes of half take the room of the elements)
+    if (kVariants[l.variant].v.koct == 2) hipLaunchKernelGGL(filter_scale_kernel, dim3((unsigned)p.OC), dim3(256), 0, stream, w, scales, p.K());
     hipLaunchKernelGGL(pack_filters_kernel, dim3(blocks), dim3(256), 0, stream, w, packed, p.OCg(), p.OCgP(), p.ICg(), p.ICgP(cpad),
-                       p.KH * p.KW, p.groups, kVariants[l.variant].v.kvec(), kVariants[l.variant].v.precision, kVariants[l.variant].v.koct);
+                       p.KH * p.KW, p.groups, kVariants[l.variant].v.kvec(), kVariants[l.variant].v.precision, kVariants[l.variant].v.koct, scales);
 }
 
 }  // namespace ios

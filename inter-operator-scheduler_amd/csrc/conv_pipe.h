@@ -1,27 +1,27 @@
 // LDS-tiled convolution for large batches with both operands staged in LDS: ConvPipe.
 //
-// The GEMM view, K order and tails are those of conv_body.h; the operands are the sixteen-bit ones of ConvSplit3: three exact
-// bfloat16 terms of an fp32 value (TERMS = 3, fp32 accuracy) or one rounded term, bfloat16 or IEEE half (TERMS = 1, the
+// The GEMM view, K order and tails are those of conv_body.h; the operands are sixteen-bit ones: two terms of IEEE half that hold
+// an fp32 value (TERMS = 2, fp32 accuracy, see split_half2) or one rounded term, bfloat16 or half (TERMS = 1, the
 // reduced-precision modes), on v_mfma_f32_32x32x16.  ConvSplit3 reads its filters from global memory, once per wavefront: at 32 x 64
 // outputs per wavefront the L1 delivers 64 bytes per cycle and compute unit for them alone, its limit.  Here a block reads its
 // filter tile once, and a wavefront computes up to 64 x 64 or 96 x 64 outputs per operand read (24 or 36 matrix instructions of 32
 // cycles for 12 or 15 LDS reads of 8).
 //
 // A stage holds KU units of 16 k (a unit lies inside one filter tap).  One stage is two or more matrix times ahead in
-// registers, the next one in LDS; one barrier per stage.  What a stage has to cover is the latency of its loads: with three terms
-// the matrix work of one unit does (768 cycles per wavefront), with one term it takes four units (a one-unit stage is gone in 128).
+// registers, the next one in LDS; one barrier per stage.  What a stage has to cover is the latency of its loads: with two terms one
+// or two units do (12 matrix instructions of 32 cycles per wavefront and unit at 64 x 64), with one term it takes four (a one-unit
+// stage is gone in 128 cycles).  Measured at batch 64 in fp32, three bfloat16 terms -> two terms of half: 288 -> 384 channels 3 x 3 stride 2 on
+// 35 x 35 222 -> 159 us (231 TFLOP/s, with 64 x 64 per wavefront, two units), 768 -> 192 on 17 x 17 44 -> 37 us, 192 -> 64 on 35 x 35
+// 22.7 -> 20.8 us (bound by its 110 MB).
 #pragma once
 
 #include "conv_body.h"
 
 namespace ios {
 
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-
 template <int TERMS, bool HALF, int KU, int PD, int TMW, int TNW, int WM, int WN>
 struct ConvPipe {
-    static_assert(TERMS == 3 || TERMS == 1, "three exact terms or one rounded term");
-    static_assert(!HALF || TERMS == 1, "half operands are rounded");
+    static_assert(TERMS == 1 || (TERMS == 2 && HALF), "one rounded term, or two terms of half");
     static constexpr int MT = 32;
     using M = Mfma<32>;
     static constexpr int BM = 32 * TMW * WM, BN = 32 * TNW * WN, BK = 16 * KU;
@@ -38,13 +38,21 @@ struct ConvPipe {
     static constexpr int UNIT = 2 * BN + (KU > 1 ? 2 : 0);
     static constexpr int STAGE = A_SLOTS + KU * TERMS * UNIT;
     static constexpr int SMEM_FLOATS = 2 * STAGE * 4;
+    static_assert(SMEM_FLOATS >= WM * WN, "a word per wavefront");
     static_assert(OCT * BN % T == 0 && T % OCT == 0, "input loader shape");
 
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
+        if constexpr (TERMS == 2) half_attempts([&](float scale) { return attempt<RES>(a, smem, tile, g, z, scale); });
+        else attempt<RES>(a, smem, tile, g, z, 1.f);
+    }
+
+    // the tile with inputs times `scale` (two terms); returns what half_attempts takes
+    template <bool RES>
+    __device__ static __forceinline__ float attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, const float scale) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
-    const int tid = threadIdx.x;
+    const int tid = TERMS == 2 ? again(threadIdx.x) : (int)threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % WN;
@@ -125,6 +133,7 @@ struct ConvPipe {
     };
     const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;
+    float peak = 0.f;   // two terms: largest magnitude this thread has staged
     auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
         uintx4 *As = lds + buf * STAGE;
         uintx4 *Bs = As + A_SLOTS + unit * (TERMS * UNIT);
@@ -140,12 +149,12 @@ struct ConvPipe {
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = j < left ? v[j] : 0.f;
             const int slot = slot_of(tid / OCT + i * (T / OCT), half);
-            if constexpr (TERMS == 3) {
-                uintx4 hi, mid, lo;
-                split_bf16x3(v, hi, mid, lo);
+            if constexpr (TERMS == 2) {
+                uintx4 hi, lo;
+                peak = half_peak(v, peak);
+                split_half2(v, scale, hi, lo);
                 Bs[slot] = hi;
-                Bs[UNIT + slot] = mid;
-                Bs[2 * UNIT + slot] = lo;
+                Bs[UNIT + slot] = lo;
             } else if constexpr (HALF) {
                 const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
                 Bs[slot] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));   // round to nearest even, overflow to infinity
@@ -162,80 +171,96 @@ struct ConvPipe {
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
-
-    // Register set s holds stage st with st % PD == s.  Iteration st: the matrix work of stage st from LDS buffer st & 1, the
-    // registers of stage st + 1 into the other buffer, stage st + 1 + PD requested into the same registers.  The loop runs in
-    // rounds of PD stages with a straight-line body; stages past the end are loaded as zeros.
+    bool exact = false;
+    if constexpr (TERMS == 2) {
+        exact = scale == 0.f;
+        if (exact)
+            half_exact_tiles(a, acc, g, m0 + wm * WTM, [&](int j) {
+                const int n = n0 + wn * WTN + j * 32 + lc;
+                return n < a.Npix ? n : -1;
+            }, k_begin, k_end, 0, a.ICgP);
+    }
+    if (!exact) {
+        // Register set s holds stage st with st % PD == s.  Iteration st: the matrix work of stage st from LDS buffer st & 1, the
+        // registers of stage st + 1 into the other buffer, stage st + 1 + PD requested into the same registers.  The loop runs in
+        // rounds of PD stages with a straight-line body; stages past the end are loaded as zeros.
 #pragma unroll
-    for (int s = 0; s < PD; s++) load_stage(s, a_reg[s], b_reg[s], b_left[s]);
-    store_stage(0, a_reg[0], b_reg[0], b_left[0]);
-    load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
-    __syncthreads();
-    for (int st0 = 0; st0 < stages; st0 += PD) {
+        for (int s = 0; s < PD; s++) load_stage(s, a_reg[s], b_reg[s], b_left[s]);
+        store_stage(0, a_reg[0], b_reg[0], b_left[0]);
+        load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
+        __syncthreads();
+        for (int st0 = 0; st0 < stages; st0 += PD) {
 #pragma unroll
-        for (int s = 0; s < PD; s++) {
-            const int st = st0 + s;
-            const int buf = st & 1;
-            const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
-            const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
+            for (int s = 0; s < PD; s++) {
+                const int st = st0 + s;
+                const int buf = st & 1;
+                const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
+                const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
 #pragma unroll
-            for (int u = 0; u < KU; u++) {
-                uintx4 av[TERMS][TM], bv[TERMS][TN];
+                for (int u = 0; u < KU; u++) {
+                    uintx4 av[TERMS][TM], bv[TERMS][TN];
 #pragma unroll
-                for (int p = 0; p < TERMS; p++) {
+                    for (int p = 0; p < TERMS; p++) {
 #pragma unroll
-                    for (int i = 0; i < TM; i++) av[p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
+                        for (int i = 0; i < TM; i++) av[p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
 #pragma unroll
-                    for (int j = 0; j < TN; j++) bv[p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
+                        for (int j = 0; j < TN; j++) bv[p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
+                    }
+                    // all LDS reads of the unit are requested before its first matrix instruction
+                    if (TERMS == 2) __builtin_amdgcn_sched_barrier(0);
+                    multiply_terms<TERMS, HALF>(acc, av, bv);
                 }
-                // all LDS reads of the unit are requested before its first matrix instruction
-                if (TERMS == 3) __builtin_amdgcn_sched_barrier(0);
-                // the six terms, smallest first; the tiles of a term are independent instructions
-                constexpr int NT = TERMS == 3 ? 6 : 1;
-                constexpr int TA[6] = {TERMS == 3 ? 2 : 0, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-                for (int t = 0; t < NT; t++)
-#pragma unroll
-                    for (int i = 0; i < TM; i++)
-#pragma unroll
-                        for (int j = 0; j < TN; j++) {
-                            if constexpr (HALF)
-                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, av[TA[t]][i]),
-                                                                                   __builtin_bit_cast(halfx8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
-                            else
-                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[TA[t]][i]),
-                                                                                    __builtin_bit_cast(bf16x8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
-                        }
+                store_stage(buf ^ 1, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+                load_stage(st + 1 + PD, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+                __syncthreads();
             }
-            store_stage(buf ^ 1, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
-            load_stage(st + 1 + PD, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
-            __syncthreads();
+        }
+        if constexpr (TERMS == 2) {
+            if (scale == kHalfScale) {
+                const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem));
+                if (next >= 0.f) return next;
+            }
+            scale_channels(a, acc, g, m0 + wm * WTM, kHalfScale / scale);
         }
     }
     tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0);
-    }   // run
+    return kHalfDone;
+    }   // attempt
 };
 
-// X(index, name, KU, PD, TMW, TNW, WM, WN): three exact terms
-#define IOS_PIPE3_VARIANTS(X)                          \
-    X(119, "x3p_m96n128_w1x4", 1, 2, 3, 1, 1, 4)       \
-    X(120, "x3p_m64n128_w1x4", 1, 2, 2, 1, 1, 4)       \
-    X(121, "x3p_m64n64_w2x2", 2, 1, 1, 1, 2, 2)
+// X(index, name, KU, PD, TMW, TNW, WM, WN): two terms of half, three products
+#define IOS_PIPE3_VARIANTS(X)                            \
+    X(119, "x3p_m96n128_w1x4", 1, 2, 3, 1, 1, 4)         \
+    X(120, "x3p_m64n128_w1x4", 1, 2, 2, 1, 1, 4)         \
+    X(121, "x3p_m64n64_w2x2", 2, 1, 1, 1, 2, 2)          \
+    X(122, "x3p_m128n128_w2x2_u2", 2, 1, 2, 2, 2, 2)     \
+    X(123, "x3p_m64n128_w1x4_u2", 2, 1, 2, 1, 1, 4)      \
+    X(124, "x3p_m128n64_w2x2_u2", 2, 1, 2, 1, 2, 2)      \
+    X(125, "x3p_m64n64_w2x2_u4", 4, 1, 1, 1, 2, 2)       \
+    X(126, "x3p_m32n128_w1x4_u2", 2, 1, 1, 1, 1, 4)
 // one rounded term, bfloat16 (option precision=bf16)
 #define IOS_PIPE_BF16_VARIANTS(X)                      \
-    X(122, "wb_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
-    X(123, "wb_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
-    X(124, "wb_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
-    X(125, "wb_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
-    X(126, "wb_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
-    X(127, "wb_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
+    X(127, "wb_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
+    X(128, "wb_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
+    X(129, "wb_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
+    X(130, "wb_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
+    X(131, "wb_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
+    X(132, "wb_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
 // one rounded term, IEEE half (option precision=fp16)
 #define IOS_PIPE_FP16_VARIANTS(X)                      \
-    X(128, "wh_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
-    X(129, "wh_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
-    X(130, "wh_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
-    X(131, "wh_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
-    X(132, "wh_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
-    X(133, "wh_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
+    X(133, "wh_p_m128n128_w2x2", 4, 1, 2, 2, 2, 2)     \
+    X(134, "wh_p_m64n128_w1x4", 4, 1, 2, 1, 1, 4)      \
+    X(135, "wh_p_m96n128_w1x4", 4, 1, 3, 1, 1, 4)      \
+    X(136, "wh_p_m32n256_w1x4", 2, 1, 1, 2, 1, 4)      \
+    X(137, "wh_p_m128n64_w2x2", 4, 1, 2, 1, 2, 2)      \
+    X(138, "wh_p_m64n64_w2x2", 4, 1, 1, 1, 2, 2)
+
+constexpr int kFirstPipeVariant = 119;
+
+// A kernel and its residual form; those of conv_pipe.hip, in the order of the lists above
+struct StagedKernel {
+    void (*kernel)(ConvKernelArgs), (*kernel_residual)(ConvKernelArgs);
+};
+extern const StagedKernel kPipeKernels[];
 
 }  // namespace ios

@@ -1,0 +1,14 @@
+// The convolution kernels that stage both operands (conv_pipe.h), compiled apart from the others.
+#include "conv_pipe.h"
+#include "conv_kernel.h"
+
+namespace ios {
+
+#define IOS_PIPE_KERNEL(TERMS, HALF, ...) {conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__>>, conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__>, true>},
+#define IOS_PIPE3_KERNEL(IDX, NAME, ...) IOS_PIPE_KERNEL(2, true, __VA_ARGS__)
+#define IOS_PIPE_BF16_KERNEL(IDX, NAME, ...) IOS_PIPE_KERNEL(1, false, __VA_ARGS__)
+#define IOS_PIPE_FP16_KERNEL(IDX, NAME, ...) IOS_PIPE_KERNEL(1, true, __VA_ARGS__)
+extern const StagedKernel kPipeKernels[] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_KERNEL) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_KERNEL)
+                                                IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_KERNEL)};
+
+}  // namespace ios

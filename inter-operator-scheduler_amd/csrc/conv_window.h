@@ -1,18 +1,19 @@
 // Convolutions of stride 1 with several taps at large batches, on a window of the input that is staged once: ConvWindow.
 //
-// The LDS-tiled kernels of conv_body.h and conv_pipe.h walk K tap by tap: for a 3 x 3 filter they load, convert (into three bfloat16
-// terms, some 50 instructions per eight values) and store every input value nine times.  At stride 1 the pixels that the BN
+// The LDS-tiled kernels of conv_body.h and conv_pipe.h walk K tap by tap: for a 3 x 3 filter they load, convert (into two terms of
+// half, some 40 instructions per eight values) and store every input value nine times.  At stride 1 the pixels that the BN
 // outputs of a block read lie in one run of the input, BN plus the rows the filter reaches over: 200 pixels for 128 outputs of a
 // 3 x 3 filter on 35 x 35 maps.  Here K is walked in chunks of 16 channels with all taps inside, and the run is staged once per
 // chunk; a tap is a constant shift of the LDS address, and a lane whose tap falls outside the image reads a slot of zeros (a bit
 // per tap, known from the start).  Filters are operands straight from memory, one unit (16 k of one tap) ahead in registers, so
 // the only barriers are those around the staging.
 //
-// What is left per unit is matrix work, TNW LDS reads per plane and three address instructions per 32 pixels.  With three
-// terms that reaches the rate at which random operands from LDS keep the matrix cores of this chip at their power limit (1.2 to
-// 1.3 PFLOP/s of bfloat16 with some vector work beside it, 205 to 220 TFLOP/s of fp32).  Measured at batch 64, tap by tap -> on
-// the window: 80 -> 192 channels 3 x 3 on 73 x 73 478 -> 434 us (205 TFLOP/s) in fp32, 225 -> 182 us in bfloat16; 32 -> 64 on 147 x 147
-// 370 -> 323 us (216 -> 206, bound by 530 MB of activations); 32 -> 32 on 149 x 149 291 -> 208 us (158 -> 130).
+// What is left per unit is matrix work, TNW LDS reads per plane and three address instructions per 32 pixels (two terms: four
+// more for the scaled filter operand).  Measured at batch 64, fp32 as three terms of bfloat16 (six products) -> two of half (three):
+// 80 -> 192 channels 3 x 3 on 73 x 73 484 -> 355 us (251 TFLOP/s, 750 of half products), 32 -> 64 on 147 x 147 360 -> 291 us, 32 -> 32 on
+// 149 x 149 232 -> 167 us, 48 -> 64 5 x 5 on 35 x 35 68 -> 47 us, 192 -> 192 1 x 7 on 17 x 17 56 -> 40 us; launched back to back, where the
+// clock settles lower than in a pass.  In bfloat16, tap by tap -> on the window, the same layers in a pass: 225 -> 182 us, 216 -> 206
+// (bound by 530 MB of activations), 158 -> 130.
 #pragma once
 
 #include "conv_pipe.h"
@@ -23,8 +24,7 @@ namespace ios {
 // NBUF: windows in LDS (2: one barrier per chunk, for tiles whose windows are small)
 template <int TERMS, bool HALF, int TMW, int TNW, int WM, int WN, int P_IT, int NBUF>
 struct ConvWindow {
-    static_assert(TERMS == 3 || TERMS == 1, "three exact terms or one rounded term");
-    static_assert(!HALF || TERMS == 1, "half operands are rounded");
+    static_assert(TERMS == 1 || (TERMS == 2 && HALF), "one rounded term, or two terms of half");
     static constexpr int MT = 32;
     using M = Mfma<32>;
     static constexpr int BM = 32 * TMW * WM, BN = 32 * TNW * WN;
@@ -37,13 +37,21 @@ struct ConvWindow {
     // neighbouring lanes store, fall into different banks
     static constexpr int S = SPAN + 4;
     static constexpr int BUF = 2 * TERMS * S;
-    static constexpr int SMEM_FLOATS = NBUF * BUF * 4;
+    static constexpr int FLAGS = NBUF * BUF * 4;      // two terms: a word per wavefront behind the windows
+    static constexpr int SMEM_FLOATS = FLAGS + (TERMS == 2 ? 4 * ((WM * WN + 3) / 4) : 0);
 
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
+        if constexpr (TERMS == 2) half_attempts([&](float scale) { return attempt<RES>(a, smem, tile, g, z, scale); });
+        else attempt<RES>(a, smem, tile, g, z, 1.f);
+    }
+
+    // the tile with inputs times `scale` (two terms); returns what half_attempts takes
+    template <bool RES>
+    __device__ static __forceinline__ float attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, const float scale) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
-    const int tid = threadIdx.x;
+    const int tid = TERMS == 2 ? again(threadIdx.x) : (int)threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % WN;
@@ -106,6 +114,7 @@ struct ConvWindow {
     };
     const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;
+    float peak = 0.f;   // two terms: largest magnitude this thread has staged
     auto store_window = [&](int buf) {
         uintx4 *at = lds + buf * BUF + half * S + (tid >> 1);
 #pragma unroll
@@ -116,12 +125,12 @@ struct ConvWindow {
             if (ragged)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = j < b_left ? v[j] : 0.f;
-            if constexpr (TERMS == 3) {
-                uintx4 hi, mid, lo;
-                split_bf16x3(v, hi, mid, lo);
+            if constexpr (TERMS == 2) {
+                uintx4 hi, lo;
+                peak = half_peak(v, peak);
+                split_half2(v, scale, hi, lo);
                 at[i * (T / 2)] = hi;
-                at[i * (T / 2) + 2 * S] = mid;
-                at[i * (T / 2) + 4 * S] = lo;
+                at[i * (T / 2) + 2 * S] = lo;
             } else if constexpr (HALF) {
                 const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
                 at[i * (T / 2)] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));
@@ -153,13 +162,6 @@ struct ConvWindow {
     constexpr unsigned kZero = (S - 1) * 16;
 
     typename M::acc_t acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
-
     uintx4 av[2][TERMS][TM];
     // next filter operands to request
     int r_tap = 0, r_ch = ch_begin;
@@ -193,19 +195,7 @@ struct ConvWindow {
         u_kw = wrap ? 0 : u_kw;
         u_tap++;
         __builtin_amdgcn_sched_barrier(0);
-        constexpr int NT = TERMS == 3 ? 6 : 1;
-        constexpr int TA[6] = {TERMS == 3 ? 2 : 0, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    if constexpr (HALF)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, fv[TA[t]][i]), __builtin_bit_cast(halfx8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
-                    else
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fv[TA[t]][i]), __builtin_bit_cast(bf16x8, bv[TB[t]][j]), acc[i][j], 0, 0, 0);
-                }
+        multiply_terms<TERMS, HALF>(acc, fv, bv);
         __builtin_amdgcn_sched_barrier(0);
     };
     // One chunk: its window from registers into LDS, the next one requested, then one unit of matrix work per tap, each with the
@@ -230,43 +220,69 @@ struct ConvWindow {
         unit(buf, av[P], av[P ^ 1]);
         if (NBUF == 1) __syncthreads();
     };
-    load_filters(av[0]);
-    load_window(ch_begin);
-    for (int ch = ch_begin; ch < ch_end; ch += 2) {
-        chunk(ch, std::integral_constant<int, 0>{});
-        if (ch + 1 >= ch_end) break;
-        chunk(ch + 1, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
+    bool exact = false;
+    if constexpr (TERMS == 2) {
+        exact = scale == 0.f;
+        if (exact)
+            half_exact_tiles(a, acc, g, m0 + wm * WTM, [&](int j) {
+                const int n = n0 + wn * WTN + j * 32 + lc;
+                return n < n_end ? n : -1;
+            }, 0, a.Kq, ch_begin * 16, ch_end * 16);
     }
-    __syncthreads();
+    if (!exact) {
+        load_filters(av[0]);
+        load_window(ch_begin);
+        for (int ch = ch_begin; ch < ch_end; ch += 2) {
+            chunk(ch, std::integral_constant<int, 0>{});
+            if (ch + 1 >= ch_end) break;
+            chunk(ch + 1, std::integral_constant<int, 1>{});
+        }
+        if constexpr (TERMS == 2) {
+            if (scale == kHalfScale) {
+                const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem + FLAGS));
+                if (next >= 0.f) return next;
+            } else {
+                __syncthreads();
+            }
+            scale_channels(a, acc, g, m0 + wm * WTM, kHalfScale / scale);
+        } else {
+            __syncthreads();
+        }
+    }
     tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, n_end);
-    }   // run
+    return kHalfDone;
+    }   // attempt
 };
 
 // X(index, name, TMW, TNW, WM, WN, P_IT, NBUF).  A window of a 3 x 3 filter on wide maps takes 300 pixels beyond the outputs, so
 // the tall-and-narrow blocks are for few channels on large maps; the 128-output blocks serve the smaller maps.
-#define IOS_WINDOW3_VARIANTS(X)                          \
-    X(134, "x3_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(135, "x3_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(136, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)    \
-    X(137, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+#define IOS_WINDOW3_VARIANTS(X)                           \
+    X(139, "x3_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)       \
+    X(140, "x3_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)       \
+    X(141, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)     \
+    X(142, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)       \
+    X(143, "x3_win_m96n128_w1x4_d", 3, 1, 1, 4, 2, 2)
 #define IOS_WINDOW_BF16_VARIANTS(X)                      \
-    X(138, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
-    X(139, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
-    X(140, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(141, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(142, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+    X(144, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(145, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(146, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(147, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(148, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
 #define IOS_WINDOW_FP16_VARIANTS(X)                      \
-    X(143, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
-    X(144, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
-    X(145, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(146, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(147, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
-constexpr int kFirstWindowVariant = 134, kNumConvVariants = 148;
+    X(149, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(150, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(151, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(152, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(153, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+constexpr int kFirstWindowVariant = 139, kNumConvVariants = 154;
 
 // The window kernels (conv_window.hip), in the order of the lists above
-struct WindowKernel {
-    void (*kernel)(ConvKernelArgs), (*kernel_residual)(ConvKernelArgs);
-};
-extern const WindowKernel kWindowKernels[];
+extern const StagedKernel kWindowKernels[];
 
 }  // namespace ios

@@ -8,7 +8,7 @@ namespace ios {
 
 // One block of a fused launch: the body of `item`.  MATRIX / DIRECT: the matrix-path convolution bodies / the depth-wise and
 // direct convolution bodies are part of the kernel.
-// WIDE: the kernel also holds the three-term wave-split bodies (fused_kernel_wide, no cap on registers).
+// WIDE: the kernel also holds the two-term wave-split bodies (fused_kernel_wide, no cap on registers).
 template <int T, bool MATRIX = true, bool DIRECT = true, bool WIDE = false>
 __device__ __forceinline__ void fused_item(const WorkItem &item, const int bid, float *smem) {
     // An item spans five 64-byte lines of the scalar cache, and the bodies read its fields in two or three dependent steps
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4))) void fus
     fused_inline_block<T, false>(b1, b2, b3, b4, b5, b6, b7);
 }
 
-// The family with room for the three-term wave-split bodies: no cap on registers (its heaviest body takes ~155, three
+// The family with room for the two-term wave-split bodies: no cap on registers (its heaviest body takes ~155, three
 // wavefronts per SIMD), every other body as well, items in the table.  For parallel stages at batch 16 and more, where those
 // bodies are the fastest convolution kernels and the launches run long enough for the lower occupancy not to matter.
 template <int T>

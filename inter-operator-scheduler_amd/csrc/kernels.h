@@ -106,10 +106,11 @@ struct ConvVariant {
     int threads() const { return 64 * WM * WN * WK; }
     bool fusable_;   // light enough on registers to run inside a fused stage launch
     int precision;   // PREC_FP32, or a reduced-precision mode: bfloat16 / IEEE half filters and inputs, fp32 accumulation
-    // packed filters as planes of bfloat16, [k / 8][plane][m][8]: 3 = the exact three-term split of fp32 values (fp32 results from
-    // the bfloat16 matrix pipe), 1 = one plane rounded to nearest even (the reduced-precision mode on the same kernels), 0 = neither
+    // packed filters as planes of 16-bit values, [k / 8][plane][m][8]: 3 = the exact split of fp32 values into three bfloat16 terms and
+    // 2 = their split into two terms of IEEE half, scaled per output channel (fp32 results from the 16-bit matrix pipe), 1 = one plane
+    // rounded to nearest even (the reduced-precision mode on the same kernels), 0 = neither
     int koct = 0;
-    // fits a fused stage launch of the wide-register kernel family only (the three-term wave-split configurations)
+    // fits a fused stage launch of the wide-register kernel family only (the two-term wave-split configurations)
     bool fusable_wide_ = false;
     int window = 0;   // > 0: stages a window of up to this many input pixels (conv_window.h); for the shapes conv_variant_takes allows
     bool fusable() const { return fusable_ || fusable_wide_; }
@@ -119,7 +120,7 @@ struct ConvVariant {
 
 int conv_num_variants();
 const ConvVariant &conv_variant(int index);
-bool conv_variant_measured(int variant);   // the tuner tries it
+bool conv_variant_measured(const ConvProblem &p, int variant);   // the tuner tries it
 bool conv_variant_takes(const ConvProblem &p, int variant);   // (a launch of another shape runs on a configuration that reads the same packed filters)
 
 struct ConvLaunch {
@@ -147,7 +148,8 @@ bool conv_matrix_path_supported(const ConvProblem &p);
 ConvLaunch conv_pick_launch(const ConvProblem &p, int num_cus, bool fusable_only = false, int precision = PREC_FP32);
 
 // Filter packing for a kernel configuration: w[OC][ICg][KH][KW] -> packed[g][k = (kh*KW + kw)*ICgP + c][OCgP]
-// (or [g][k / 4][OCgP][k % 4] for kquad configurations, three bfloat16 planes [g][k / 8][plane][OCgP][k % 8] for koct ones), ICgP = ICg rounded up to the configuration's channel
+// (or [g][k / 4][OCgP][k % 4] for kquad configurations, planes of 16-bit values [g][k / 8][plane][OCgP][k % 8] for koct ones, with the
+// factors of the output channels behind two planes), ICgP = ICg rounded up to the configuration's channel
 // padding (zero rows), OCgP = OCg rounded up to 4.  16-bit configurations pack bfloat16 or half (round to nearest even), two
 // per float of the returned size.
 size_t conv_packed_floats(const ConvProblem &p, const ConvLaunch &l);

@@ -273,7 +273,7 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
     // first pass: every configuration and split factor, a few launches each
     for (int v = 0; v < conv_num_variants(); v++) {
         const ConvVariant &cv = conv_variant(v);
-        if (cv.precision != precision_ || !conv_variant_measured(v) || !conv_variant_takes(p, v)) continue;   // the precision mode decides which family of configurations competes
+        if (cv.precision != precision_ || !conv_variant_measured(p, v) || !conv_variant_takes(p, v)) continue;   // the precision mode decides which family of configurations competes
         // tiles more than twice as tall / wide as the problem only waste lanes
         if (cv.BM >= 2 * p.OCg() + 32 || cv.BN >= 2 * p.Npix() + 32) continue;
         int last_effective = -1;
