@@ -29,6 +29,7 @@
 
 #include "kernels.h"
 
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -195,6 +196,47 @@ __device__ __forceinline__ void finish_quad(const ConvKernelArgs &a, floatx4 v, 
     }
 }
 
+// The same for N pixels STEP apart from `first` on, below n_end; factor: of the four channels.
+template <bool RES, int N, int STEP>
+__device__ __forceinline__ void finish_quads(const ConvKernelArgs &a, floatx4 (&v)[N], floatx4 bias, floatx4 factor, int g, int m, int first, int n_end) {
+    if (m >= a.OCg) return;
+    float out[4 * N];
+#pragma unroll
+    for (int r = 0; r < N; r++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) out[4 * r + c] = __builtin_fmaf(v[r][c], factor[c], bias[c]);
+    apply_activation(out, a.act);
+    const int channel = g * a.OCg + m;
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        const int nn = first + r * STEP;
+        if (nn >= n_end) break;
+        floatx4 w = {out[4 * r], out[4 * r + 1], out[4 * r + 2], out[4 * r + 3]};
+        float *y = a.y + (long long)nn * a.y_ps + channel;
+        const float *res = nullptr;
+        if constexpr (RES) res = a.res + (long long)nn * a.res_ps + channel;
+        if (m + 3 < a.OCg) {
+            if constexpr (RES) {
+                w += (floatx4)*reinterpret_cast<const floatx4_u *>(res);
+                if (a.post_relu)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) w[c] = fmaxf(w[c], 0.0f);
+            }
+            *reinterpret_cast<floatx4_u *>(y) = w;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                if (m + c < a.OCg) {
+                    if constexpr (RES) {
+                        w[c] += res[c];
+                        if (a.post_relu) w[c] = fmaxf(w[c], 0.0f);
+                    }
+                    y[c] = w[c];
+                }
+        }
+    }
+}
+
 // bias of output channels m ... m + 3 of group g (what lies behind the last bias value is not used; the arena goes on there)
 __device__ __forceinline__ floatx4 bias_quad(const ConvKernelArgs &a, int g, int m) {
     return *reinterpret_cast<const floatx4_u *>(a.bias + g * a.OCg + min(m, a.OCg - 1));
@@ -252,11 +294,61 @@ struct Mfma<16> {
     __device__ static __forceinline__ int row(int v, int lane) { return 4 * (lane >> 4) + v; }
 };
 
+// Factors that undo the scaling of output channels m ... m + 3 of group g (behind the packed planes; the quad that straddles the end
+// reads on into the padding the host reserves).
+__device__ __forceinline__ floatx4 channel_scale_quad(const ConvKernelArgs &a, int g, int m) {
+    const float *scales = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.wp) + a.w_bytes);
+    return *reinterpret_cast<const floatx4_u *>(scales + g * a.OCg + min(m, a.OCg - 1));
+}
+
+// sums of scaled filters -> sums of the filters as they were given, times `more` (exact); m_base: row 0 of the tiles
+template <int TM, int TN, typename Acc>
+__device__ __forceinline__ void scale_channels(const ConvKernelArgs &a, Acc (&acc)[TM][TN], int g, int m_base, float more) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const floatx4 factor = channel_scale_quad(a, g, m_base + i * 32 + Mfma<32>::row(4 * q, lane)) * more;
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[i][j][4 * q + v] *= factor[v];
+        }
+}
+
+// Bias (and factors, SCALED) of the four output channels per 32 rows that this lane finishes in the epilogue, m_base: row 0 of the
+// wavefront's tiles; requested before the last barriers of a body, which their latency then overlaps.
+template <int TM>
+struct TailConstants { floatx4 bias[TM], factor[TM]; };
+template <int MT, bool SCALED, int TM>
+__device__ __forceinline__ void tail_constants(const ConvKernelArgs &a, TailConstants<TM> &c, int g, int m_base) {
+    if constexpr (MT == 32) {
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            const int m = m_base + i * 32 + 4 * (threadIdx.x & 7);
+            c.bias[i] = bias_quad(a, g, m);
+            if constexpr (SCALED) c.factor[i] = channel_scale_quad(a, g, m);
+        }
+    }
+}
+
+// LDS of a wavefront in the epilogue: its tiles, pixel by pixel with the quads of channels exchanged so that eight pixels' quads and
+// eight quads of a pixel meet all banks, and the constants
+constexpr int tail_floats(int tm, int tn) { return tm * tn * 1024 + tm * 64; }
+// what the lanes of a wavefront have written to LDS is there for its other lanes (accesses of a wavefront are executed in order)
+__device__ __forceinline__ void wavefront_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Tail of the LDS-tiled kernels once a block holds its accumulators (wavefronts with wk == 0; the others only take part in the
 // barriers): the split-K exchange in its three forms, then bias, activation and the store through the output view.
-template <int MT, int BM, int BN, int TM, int TN, int WM, int WN, bool RES>
+// `smem` is free when this is called, for tail_floats floats per wavefront (32 x 32 tiles).
+// SCALED: the sums are those of scaled filters (see split_half2), times `more`; 0: of the filters as they were given.
+template <int MT, int BM, int BN, int TM, int TN, int WM, int WN, bool RES, bool SCALED = false>
 __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem, typename Mfma<MT>::acc_t (&acc)[TM][TN], int tile, int g, int z,
-                                           int m0, int n0, int wm, int wn, int wk, int n_limit = INT_MAX) {
+                                           int m0, int n0, int wm, int wn, int wk, const TailConstants<TM> &c, int n_limit = INT_MAX, float more = 0.f) {
     using M = Mfma<MT>;
     const int n_end = min(a.Npix, n_limit);   // (a tile that ends before the tensor does)
     constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -265,6 +357,10 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
     const int lc = lane % MT;
     // ---- split-K ----------------------------------------------------------------------------------------------
     if (a.split_k > 1) {
+        if (SCALED && more != 0.f) {   // (slices meet as sums of the filters as they were given)
+            scale_channels(a, acc, g, m0 + wm * WTM, more);
+            more = 0.f;
+        }
         if (a.counters == nullptr) {
             // two-kernel form: store this slice's partial tile; splitk_reduce_kernel adds the slices, bias and activation
             const size_t channels = (size_t)a.groups * a.OCg;
@@ -313,7 +409,9 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
             __syncthreads();
             if (tid == 0) *last_flag = draw_ticket<LOCAL>(counter, a.split_k);
             __syncthreads();
-            if (*last_flag == 0) return false;
+            const int last = *last_flag;
+            __syncthreads();   // (the flag's place is a wavefront's in the epilogue)
+            if (last == 0) return false;
             if (wk == 0) {
 #pragma unroll
                 for (int i = 0; i < TM; i++)
@@ -338,6 +436,41 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
     }
 
     // ---- epilogue -------------------------------------------------------------------------------------------
+    if constexpr (MT == 32) {
+        // A lane holds four channels of a pixel, its neighbour the next pixel's: stored like that, every 16 bytes of a wavefront's store
+        // go to another line, and the L2 takes a request for each.  So the tiles pass through LDS; eight lanes then take the 128 bytes
+        // of a pixel, a lane the same four channels of every pixel of a tile.  What runs once is short (one copy of the code for all
+        // tiles: instructions that a launch has not run yet come from memory, a line at a time).  64 x 128 tiles of 17 x 17 maps at
+        // batch 64, 14 MB of results: 6.2 -> 3.9 us behind the K loop.
+        if (wk != 0) return;
+        float *place = smem + (wm * WN + wn) * tail_floats(TM, TN), *constants = place + TM * TN * 1024;
+        const int quad = lane & 7, px = lane >> 3;
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            if (lane < 8) {
+                *reinterpret_cast<floatx4 *>(constants + i * 64 + 4 * lane) = c.bias[i];
+                if constexpr (SCALED) *reinterpret_cast<floatx4 *>(constants + i * 64 + 32 + 4 * lane) = c.factor[i];
+            }
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int q = 0; q < M::ACC / 4; q++)
+                    *reinterpret_cast<floatx4 *>(place + (i * TN + j) * 1024 + lc * 32 + ((2 * q + (lane >> 5)) ^ (lc & 7)) * 4) =
+                        floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        }
+        wavefront_lds_fence();
+#pragma unroll 1
+        for (int t = 0; t < TM * TN; t++) {
+            const int i = t / TN, j = t - i * TN;
+            const floatx4 bias = *reinterpret_cast<const floatx4 *>(constants + i * 64 + 4 * quad);
+            floatx4 factor = {1.f, 1.f, 1.f, 1.f};
+            if (SCALED && more != 0.f) factor = *reinterpret_cast<const floatx4 *>(constants + i * 64 + 32 + 4 * quad) * more;
+            floatx4 v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = *reinterpret_cast<const floatx4 *>(place + t * 1024 + (8 * r + px) * 32 + (quad ^ px) * 4);
+            finish_quads<RES, 4, 8>(a, v, bias, factor, g, m0 + wm * WTM + i * MT + 4 * quad, n0 + wn * WTN + j * MT + px, n_end);
+        }
+    } else {
     if (wk == 0) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -355,6 +488,7 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
                 }
             }
     }
+    }
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int WK, int MT, int PD>
@@ -371,7 +505,8 @@ struct ConvTiled {
     // occupancy of every other operator (the wave-split bodies that serve small problems need 32-72), so they
     // only run as stand-alone kernels.
     static constexpr bool FUSABLE = false;
-    static constexpr int SMEM_FLOATS = TILE_FLOATS > RED_FLOATS ? TILE_FLOATS : RED_FLOATS;
+    static constexpr int TAIL_FLOATS = MT == 32 ? WM * WN * tail_floats(BM / WM / MT, BN / WN / MT) : 0;
+    static constexpr int SMEM_FLOATS = std::max({TILE_FLOATS, RED_FLOATS, TAIL_FLOATS});
 
     // one block: output tile `tile` of group `g`, K slice `z`; smem holds SMEM_FLOATS floats, 16-byte aligned
     template <bool RES = false>
@@ -561,9 +696,12 @@ struct ConvTiled {
                         for (int v = 0; v < M::ACC; v++)
                             acc[i][j][v] += red[((size_t)s * PER_WAVE + (i * TN + j) * M::ACC + v) * (MN_WAVES * 64) + slot];
         }
+        __syncthreads();
     }
 
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, wk);
+    TailConstants<TM> constants;
+    tail_constants<MT, false>(a, constants, g, m0 + wm * WTM);
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, wk, constants);
     }   // run
 };
 
@@ -724,29 +862,6 @@ __device__ __forceinline__ float half_block_peak(float peak, float *words) {
     return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
 }
 
-// Factors that undo the scaling of output channels m ... m + 3 of group g (behind the packed planes; the quad that straddles the end
-// reads on into the padding the host reserves).
-__device__ __forceinline__ floatx4 channel_scale_quad(const ConvKernelArgs &a, int g, int m) {
-    const float *scales = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.wp) + a.w_bytes);
-    return *reinterpret_cast<const floatx4_u *>(scales + g * a.OCg + min(m, a.OCg - 1));
-}
-
-// sums of scaled filters -> sums of the filters as they were given, times `more` (exact); m_base: row 0 of the tiles
-template <int TM, int TN>
-__device__ __forceinline__ void scale_channels(const ConvKernelArgs &a, floatx16 (&acc)[TM][TN], int g, int m_base, float more) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const floatx4 factor = channel_scale_quad(a, g, m_base + i * 32 + Mfma<32>::row(4 * q, lane)) * more;
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) acc[i][j][4 * q + v] *= factor[v];
-        }
-}
-
 // The accumulators of TM x TN tiles of 32 x 32 by fp32 multiply-adds, from the packed halves: for inputs no factor serves.  m_base: row
 // 0 of the tiles; n: this lane's column in tile column j, or negative; K as [k_begin, k_end) of the packed rows, restricted to
 // channels [c_begin, c_end).  The sums are those of the filters as they were given.  Slow on purpose: it takes few registers and runs for values beyond 2^26.
@@ -845,7 +960,7 @@ struct ConvSplit3 {
     static constexpr bool FUSABLE = false;
     // LDS in slots of 16 bytes (eight bfloat16): per stage the input planes [TERMS][2][BN]
     static constexpr int STAGE = 2 * TERMS * BN;
-    static constexpr int SMEM_FLOATS = 2 * STAGE * 4;
+    static constexpr int SMEM_FLOATS = std::max(2 * STAGE * 4, WAVES * tail_floats(TMW, TNW));
     static constexpr int B_OCT = 2 * BN;
     static constexpr int B_IT = (B_OCT + T - 1) / T;                   // octets a thread stages per K tile
     static_assert(B_OCT % T == 0 || B_IT == 1, "whole passes, or one with surplus threads");
@@ -1008,7 +1123,9 @@ struct ConvSplit3 {
             __syncthreads();
         }
     }
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0);
+    TailConstants<TM> constants;
+    tail_constants<MT, false>(a, constants, g, m0 + wm * WTM);
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants);
     }   // run
 };
 
@@ -1694,4 +1811,12 @@ struct ConvWsplit {
     X(116, "wb_x1w_m64n64_w4", 2, 2, 4, 2)     \
     X(117, "wb_x1w_m32n32_w8", 1, 1, 8, 2)     \
     X(118, "wb_x1w_m64n64_w2", 2, 2, 2, 2)
+
+// A stand-alone kernel and its residual form
+struct KernelPair {
+    void (*kernel)(ConvKernelArgs) = nullptr, (*kernel_residual)(ConvKernelArgs) = nullptr;
+};
+// conv_tiled.hip, in the order of the lists above
+extern const KernelPair kTiledKernels[], kSplit3Kernels[], kSplit1Kernels[];
+constexpr int kFirstSplit3Variant = 89, kFirstSplit1Variant = 107;
 }  // namespace ios

@@ -16,54 +16,56 @@ typedef void (*ConvKernelFn)(ConvKernelArgs);
 
 struct VariantEntry {
     ConvVariant v;
-    ConvKernelFn kernel, kernel_residual;
+    KernelPair any;
     int smem_floats;
+    KernelPair special[2] = {};   // staged kernels for the filters that kernel_of() names
 };
 
 #define IOS_TILED_ENTRY(IDX, NAME, BM, BN, BK, WM, WN, WK, MT, PD)                                        \
     {{NAME, BM, BN, BK, WM, WN, WK, MT, false, ConvTiled<BM, BN, BK, WM, WN, WK, MT, PD>::CPAD, false, \
       ConvTiled<BM, BN, BK, WM, WN, WK, MT, PD>::FUSABLE, false},    \
-     conv_kernel<ConvTiled<BM, BN, BK, WM, WN, WK, MT, PD>>, conv_kernel<ConvTiled<BM, BN, BK, WM, WN, WK, MT, PD>, true>, \
+     kTiledKernels[IDX], \
      ConvTiled<BM, BN, BK, WM, WN, WK, MT, PD>::SMEM_FLOATS},
 #define IOS_WSPLIT_ENTRY(IDX, NAME, MT, TM, TN, NW, U, QUAD, D, BF16)                                                                  \
     {{NAME, TM * MT, TN * MT, U *(MT == 32 ? 2 : 4), 1, 1, NW, MT, true, ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>::CPAD, QUAD, \
       ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>::FUSABLE, BF16},      \
-     conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>>, conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>, true>,    \
+     {conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>>, conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>, true>}, \
      ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16>::SMEM_FLOATS},
 #define IOS_WSPLIT_C4_ENTRY(IDX, NAME, MT, TM, TN, NW, U, QUAD, D, BF16)                                                                  \
     {{NAME, TM * MT, TN * MT, U *(MT == 32 ? 2 : 4), 1, 1, NW, MT, true, ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>::CPAD, QUAD, \
       ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>::FUSABLE, BF16},                                                                 \
-     conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>>, conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>, true>,    \
+     {conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>>, conv_kernel<ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>, true>}, \
      ConvWsplit<MT, TM, TN, NW, U, QUAD, D, BF16, 4>::SMEM_FLOATS},
 
 #define IOS_SPLIT3_ENTRY(IDX, NAME, TMW, TNW, WM, WN, PD)                                                                              \
     {{NAME, ConvSplit3<TMW, TNW, WM, WN, PD>::BM, ConvSplit3<TMW, TNW, WM, WN, PD>::BN, 16, WM, WN, 1, 32, false,                         \
       ConvSplit3<TMW, TNW, WM, WN, PD>::CPAD, false, false, PREC_FP32, 3},                                                                \
-     conv_kernel<ConvSplit3<TMW, TNW, WM, WN, PD>>, conv_kernel<ConvSplit3<TMW, TNW, WM, WN, PD>, true>,                                  \
+     kSplit3Kernels[IDX - kFirstSplit3Variant], \
      ConvSplit3<TMW, TNW, WM, WN, PD>::SMEM_FLOATS},
 
 #define IOS_WSPLIT_X3_ENTRY(IDX, NAME, TM, TN, NW, D)                                                                        \
     {{NAME, TM * 32, TN * 32, 16, 1, 1, NW, 32, true, ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::CPAD, true, false, PREC_FP32, 2, \
       ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::FUSABLE_WIDE},      \
-     conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>, true>,              \
+     {conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>, true>}, \
      ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::SMEM_FLOATS},
 
 #define IOS_SPLIT1_ENTRY(IDX, NAME, TMW, TNW, WM, WN, PD)                                                                              \
     {{NAME, ConvSplit3<TMW, TNW, WM, WN, PD, 1>::BM, ConvSplit3<TMW, TNW, WM, WN, PD, 1>::BN, 16, WM, WN, 1, 32, false,                   \
       ConvSplit3<TMW, TNW, WM, WN, PD, 1>::CPAD, false, false, PREC_BF16, 1},                                                             \
-     conv_kernel<ConvSplit3<TMW, TNW, WM, WN, PD, 1>>, conv_kernel<ConvSplit3<TMW, TNW, WM, WN, PD, 1>, true>,                            \
+     kSplit1Kernels[IDX - kFirstSplit1Variant], \
      ConvSplit3<TMW, TNW, WM, WN, PD, 1>::SMEM_FLOATS},
 
 #define IOS_WSPLIT_X1_ENTRY(IDX, NAME, TM, TN, NW, D)                                                                        \
     {{NAME, TM * 32, TN * 32, 16, 1, 1, NW, 32, true, ConvWsplit<32, TM, TN, NW, 8, true, D, 4>::CPAD, true, false, PREC_BF16, 1},      \
-     conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>, true>,              \
+     {conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 4>, true>}, \
      ConvWsplit<32, TM, TN, NW, 8, true, D, 4>::SMEM_FLOATS},
 
 #define IOS_PIPE_ENTRY(TERMS, HALF, PRECISION, IDX, NAME, KU, PD, TMW, TNW, WM, WN)                                                       \
     {{NAME, ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::BM, ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::BN, 16 * KU, WM, WN, 1, 32, \
       false, 16, false, false, PRECISION, TERMS},                                                                                     \
-     kPipeKernels[IDX - kFirstPipeVariant].kernel, kPipeKernels[IDX - kFirstPipeVariant].kernel_residual,                               \
-     ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::SMEM_FLOATS},
+     kPipeKernels[IDX - kFirstPipeVariant][0], \
+     ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::SMEM_FLOATS,                                                                   \
+     {kPipeKernels[IDX - kFirstPipeVariant][1], {}}},
 #define IOS_PIPE3_ENTRY(...) IOS_PIPE_ENTRY(2, true, PREC_FP32, __VA_ARGS__)
 #define IOS_PIPE_BF16_ENTRY(...) IOS_PIPE_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
 #define IOS_PIPE_FP16_ENTRY(...) IOS_PIPE_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
@@ -71,8 +73,9 @@ struct VariantEntry {
 #define IOS_WINDOW_ENTRY(TERMS, HALF, PRECISION, IDX, NAME, TMW, TNW, WM, WN, P_IT, NBUF)                                                 \
     {{NAME, 32 * TMW * WM, 32 * TNW * WN, 16, WM, WN, 1, 32, false, 16, false, false, PRECISION, TERMS, false,                            \
       ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SPAN},                                                                     \
-     kWindowKernels[IDX - kFirstWindowVariant].kernel, kWindowKernels[IDX - kFirstWindowVariant].kernel_residual,                          \
-     ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SMEM_FLOATS},
+     kWindowKernels[IDX - kFirstWindowVariant], \
+     ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SMEM_FLOATS, \
+     {kWindow7Kernels[IDX - kFirstWindowVariant], kWindow9Kernels[IDX - kFirstWindowVariant]}},
 #define IOS_WINDOW3_ENTRY(...) IOS_WINDOW_ENTRY(2, true, PREC_FP32, __VA_ARGS__)
 #define IOS_WINDOW_BF16_ENTRY(...) IOS_WINDOW_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
 #define IOS_WINDOW_FP16_ENTRY(...) IOS_WINDOW_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
@@ -378,16 +381,28 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     return d;
 }
 
+// Which of an entry's kernels serves the problem: 0 any, 1 and 2 the special ones.  Pipelined kernels: [1] 1 x 1 filters without groups,
+// whose addresses stay the same over K (at batch 64 768 -> 192 on 17 x 17 39.7 -> 34.8 us, 2048 -> 320 on 8 x 8 51.2 -> 43.1).  Window kernels:
+// [1] seven taps, [2] nine (see known_chunk; other numbers are rare, 1 x 3 and 5 x 5).
+static int kernel_of(const ConvProblem &p, const VariantEntry &e) {
+    const int taps = p.KH * p.KW;
+    if (e.v.window != 0) return taps == 7 ? 1 : taps == 9 ? 2 : 0;
+    return e.special[0].kernel != nullptr && taps == 1 && p.groups == 1 ? 1 : 0;
+}
+
 void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed,
                       const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce, hipStream_t stream,
                       const TensorView *residual, bool post_relu) {
     const ConvDispatch d = make_conv_dispatch(p, l, x, packed, bias, y, workspace, reduce, residual, post_relu);
     const VariantEntry &e = kVariants[d.variant];
     const dim3 grid = d.xcd_blocks > 0 ? dim3((unsigned)d.xcd_blocks) : dim3((unsigned)d.tiles, (unsigned)d.groups, (unsigned)d.slices);
-    const ConvKernelFn kernel = !d.args.xcd_local && d.args.res != nullptr ? e.kernel_residual : e.kernel;
+    const int which = kernel_of(p, e);
+    const KernelPair &pair = which == 0 ? e.any : e.special[which - 1];
+    const bool with_residual = !d.args.xcd_local && d.args.res != nullptr;
+    const ConvKernelFn kernel = with_residual ? pair.kernel_residual : pair.kernel;
     if (d.smem_bytes > 64 * 1024) {   // beyond the default limit of dynamic LDS: raised once per kernel
-        static bool raised[kNumConvVariants][2] = {};
-        bool &done = raised[d.variant][kernel == e.kernel_residual ? 1 : 0];
+        static bool raised[kNumConvVariants][6] = {};
+        bool &done = raised[d.variant][2 * which + (with_residual ? 1 : 0)];
         if (!done) {
             if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, d.smem_bytes) != hipSuccess)
                 throw std::runtime_error(std::string("conv: cannot reserve LDS for configuration ") + e.v.name);

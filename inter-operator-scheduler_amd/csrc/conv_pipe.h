@@ -19,7 +19,7 @@
 
 namespace ios {
 
-template <int TERMS, bool HALF, int KU, int PD, int TMW, int TNW, int WM, int WN>
+template <int TERMS, bool HALF, int KU, int PD, int TMW, int TNW, int WM, int WN, bool POINT = false>
 struct ConvPipe {
     static_assert(TERMS == 1 || (TERMS == 2 && HALF), "one rounded term, or two terms of half");
     static constexpr int MT = 32;
@@ -29,6 +29,7 @@ struct ConvPipe {
     static constexpr int THREADS = T;
     static constexpr int CPAD = 16;
     static constexpr bool FUSABLE = false;
+    static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : 4;
     static constexpr int OCT = 2 * KU;                 // octets (eight consecutive k) of a pixel or filter row in a stage
     static constexpr int B_IT = OCT * BN / T;          // pixels a thread stages, T / OCT apart
     static constexpr int A_SLOTS = OCT * TERMS * BM;   // slots of 16 bytes (eight 16-bit values)
@@ -37,8 +38,8 @@ struct ConvPipe {
     // neighbouring lanes store, fall into different banks
     static constexpr int UNIT = 2 * BN + (KU > 1 ? 2 : 0);
     static constexpr int STAGE = A_SLOTS + KU * TERMS * UNIT;
-    static constexpr int SMEM_FLOATS = 2 * STAGE * 4;
-    static_assert(SMEM_FLOATS >= WM * WN, "a word per wavefront");
+    static constexpr int FLAGS = std::max(2 * STAGE * 4, WM * WN * tail_floats(TMW, TNW));   // two terms: a word per wavefront behind the operands
+    static constexpr int SMEM_FLOATS = FLAGS + (TERMS == 2 ? 4 * ((WM * WN + 3) / 4) : 0);
     static_assert(OCT * BN % T == 0 && T % OCT == 0, "input loader shape");
 
     template <bool RES = false>
@@ -97,7 +98,8 @@ struct ConvPipe {
         const int ow = r - oh * a.OW;
         ih0[i] = oh * a.sh - a.ph;
         iw0[i] = ow * a.sw - a.pw;
-        x_off[i] = (((unsigned)(b * a.H + ih0[i]) * (unsigned)a.W + (unsigned)iw0[i]) * (unsigned)a.x_ps + (unsigned)(g * a.ICg + 8 * half)) * 4u;
+        x_off[i] = (((unsigned)(b * a.H + ih0[i]) * (unsigned)a.W + (unsigned)iw0[i]) * (unsigned)a.x_ps + (unsigned)(g * a.ICg + 8 * half + (POINT ? 16 * unit : 0))) * 4u;
+        if constexpr (POINT) x_off[i] |= n_kill[i] | ((unsigned)ih0[i] < (unsigned)a.H && (unsigned)iw0[i] < (unsigned)a.W ? 0u : kOutOfRange);
     }
     auto slot_of = [](int pixel, int octet) { return 2 * pixel + (octet ^ ((pixel >> 2) & 1)); };
 
@@ -106,6 +108,23 @@ struct ConvPipe {
     int b_left[PD];
     auto load_stage = [&](int st, uintx4 (&ar)[A_IT], floatx4 (&br)[B_IT][2], int &left) {
         const int k0 = k_begin + st * BK;
+        if constexpr (POINT) {
+            // Addresses stay, the descriptors move on to the stage and end where K does (stages past the end: at once).  Channels past the
+            // end of a pixel's are masked by store_stage.
+            const bool live = k0 < k_end;
+            const unsigned w_stage = (unsigned)((k0 >> 3) * TERMS) * (unsigned)a.OCgP * 16u;
+            const __amdgpu_buffer_rsrc_t xs = buffer_of(a.x + k0, live ? a.x_bytes - (unsigned)k0 * 4u : 0u);
+            const __amdgpu_buffer_rsrc_t ws = buffer_of(a.wp + (w_stage >> 2), live ? a.w_bytes - w_stage : 0u);
+#pragma unroll
+            for (int i = 0; i < A_IT; i++) ar[i] = __builtin_amdgcn_raw_buffer_load_b128(ws, a_off[i], 0, 0);
+#pragma unroll
+            for (int i = 0; i < B_IT; i++) {
+                br[i][0] = buffer_load_f32x4(xs, x_off[i]);
+                br[i][1] = buffer_load_f32x4(xs, x_off[i], 16u);
+            }
+            left = a.ICg - k0;
+            return;
+        }
         const unsigned w_stage = (unsigned)((k0 >> 3) * TERMS) * (unsigned)a.OCgP * 16u;
 #pragma unroll
         for (int i = 0; i < A_IT; i++) {
@@ -131,7 +150,6 @@ struct ConvPipe {
         }
         left = c_left;
     };
-    const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;
     float peak = 0.f;   // two terms: largest magnitude this thread has staged
     auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
@@ -144,10 +162,15 @@ struct ConvPipe {
         for (int i = 0; i < B_IT; i++) {
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = relu_above(floor, br[i][j >> 2][j & 3]);   // folded ReLU of the producer
-            if (ragged)
+            for (int j = 0; j < 8; j++) v[j] = br[i][j >> 2][j & 3];
+            if (a.pre_relu != 0)
 #pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = j < left ? v[j] : 0.f;
+                for (int j = 0; j < 8; j++) v[j] = relu_above(0.f, v[j]);   // folded ReLU of the producer
+            if (POINT ? left < BK : ragged) {
+                const int mine = POINT ? left - 16 * unit - 8 * half : left;
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = j < mine ? v[j] : 0.f;
+            }
             const int slot = slot_of(tid / OCT + i * (T / OCT), half);
             if constexpr (TERMS == 2) {
                 uintx4 hi, lo;
@@ -171,9 +194,11 @@ struct ConvPipe {
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
+    TailConstants<TM> constants;
     bool exact = false;
     if constexpr (TERMS == 2) {
         exact = scale == 0.f;
+        if (exact) tail_constants<MT, true>(a, constants, g, m0 + wm * WTM);
         if (exact)
             half_exact_tiles(a, acc, g, m0 + wm * WTM, [&](int j) {
                 const int n = n0 + wn * WTN + j * 32 + lc;
@@ -215,15 +240,15 @@ struct ConvPipe {
                 __syncthreads();
             }
         }
+        tail_constants<MT, TERMS == 2>(a, constants, g, m0 + wm * WTM);
         if constexpr (TERMS == 2) {
             if (scale == kHalfScale) {
-                const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem));
+                const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem + FLAGS));
                 if (next >= 0.f) return next;
             }
-            scale_channels(a, acc, g, m0 + wm * WTM, kHalfScale / scale);
         }
     }
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0);
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, TERMS == 2>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants, INT_MAX, TERMS == 2 && !exact ? kHalfScale / scale : 0.f);
     return kHalfDone;
     }   // attempt
 };
@@ -257,10 +282,7 @@ struct ConvPipe {
 
 constexpr int kFirstPipeVariant = 119;
 
-// A kernel and its residual form; those of conv_pipe.hip, in the order of the lists above
-struct StagedKernel {
-    void (*kernel)(ConvKernelArgs), (*kernel_residual)(ConvKernelArgs);
-};
-extern const StagedKernel kPipeKernels[];
+// The kernels of conv_pipe.hip, in the order of the lists above; [0] any filter, [1] 1 x 1 filters without groups
+extern const KernelPair kPipeKernels[][2];
 
 }  // namespace ios

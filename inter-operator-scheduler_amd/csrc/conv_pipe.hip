@@ -4,11 +4,13 @@
 
 namespace ios {
 
-#define IOS_PIPE_KERNEL(TERMS, HALF, ...) {conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__>>, conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__>, true>},
+#define IOS_PIPE_KERNEL(TERMS, HALF, ...)                                                                             \
+    {{conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__>>, conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__>, true>},             \
+     {conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__, true>>, conv_kernel<ConvPipe<TERMS, HALF, __VA_ARGS__, true>, true>}},
 #define IOS_PIPE3_KERNEL(IDX, NAME, ...) IOS_PIPE_KERNEL(2, true, __VA_ARGS__)
 #define IOS_PIPE_BF16_KERNEL(IDX, NAME, ...) IOS_PIPE_KERNEL(1, false, __VA_ARGS__)
 #define IOS_PIPE_FP16_KERNEL(IDX, NAME, ...) IOS_PIPE_KERNEL(1, true, __VA_ARGS__)
-extern const StagedKernel kPipeKernels[] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_KERNEL) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_KERNEL)
+extern const KernelPair kPipeKernels[][2] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_KERNEL) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_KERNEL)
                                                 IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_KERNEL)};
 
 }  // namespace ios

@@ -22,7 +22,8 @@ namespace ios {
 
 // TMW x TNW MFMA tiles per wavefront, WM x WN wavefronts per block; P_IT: rounds of T / 2 pixels in which a block stages its window;
 // NBUF: windows in LDS (2: one barrier per chunk, for tiles whose windows are small)
-template <int TERMS, bool HALF, int TMW, int TNW, int WM, int WN, int P_IT, int NBUF>
+// TAPS: number of taps where it is known, 0 otherwise
+template <int TERMS, bool HALF, int TMW, int TNW, int WM, int WN, int P_IT, int NBUF, int TAPS = 0>
 struct ConvWindow {
     static_assert(TERMS == 1 || (TERMS == 2 && HALF), "one rounded term, or two terms of half");
     static constexpr int MT = 32;
@@ -32,12 +33,13 @@ struct ConvWindow {
     static constexpr int THREADS = T;
     static constexpr int CPAD = 16;
     static constexpr bool FUSABLE = false;
+    static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : TAPS > 0 ? 3 : 4;
     static constexpr int SPAN = P_IT * (T / 2);       // pixels of the input a block holds
     // slots of 16 bytes per plane and octet (eight consecutive channels), the last one zero; the octets of a pixel, which
     // neighbouring lanes store, fall into different banks
     static constexpr int S = SPAN + 4;
     static constexpr int BUF = 2 * TERMS * S;
-    static constexpr int FLAGS = NBUF * BUF * 4;      // two terms: a word per wavefront behind the windows
+    static constexpr int FLAGS = std::max(NBUF * BUF * 4, WM * WN * tail_floats(TMW, TNW));   // two terms: a word per wavefront behind the windows
     static constexpr int SMEM_FLOATS = FLAGS + (TERMS == 2 ? 4 * ((WM * WN + 3) / 4) : 0);
 
     template <bool RES = false>
@@ -68,7 +70,7 @@ struct ConvWindow {
         n0 = image * a.OHW + (tn - image * per_image) * BN;
         n_end = (image + 1) * a.OHW;
     }
-    const int taps = a.Kq / a.ICgP;   // odd
+    const int taps = TAPS > 0 ? TAPS : a.Kq / a.ICgP;   // odd
     // K slice z of the grid: a range of chunks of 16 channels, all taps of each
     const int chunks_all = a.ICgP >> 4;
     const int per_slice = (chunks_all + a.split_k - 1) / a.split_k;
@@ -95,6 +97,10 @@ struct ConvWindow {
     };
     int oh_, ow_;
     const int p0 = input_of(n0, oh_, ow_);
+    // pixels from the first to the last that the block's outputs read: what lies behind, in the rounds of T / 2, is neither loaded nor
+    // converted (a wavefront stages 32 neighbouring pixels a round)
+    const int span = input_of(min(n0 + BN, n_end) - 1, oh_, ow_) - p0 + (taps / a.KW - 1) * a.W + a.KW;
+    auto needed = [&](int i) { return wave * 32 + i * (T / 2) < span; };
     const int half = tid & 1;
     unsigned x_off = (unsigned)((p0 + (tid >> 1)) * a.x_ps + g * a.ICg + 8 * half) * 4u;   // may wrap below zero: beyond the extent
     const unsigned x_step = (unsigned)(T / 2) * (unsigned)a.x_ps * 4u;
@@ -107,21 +113,24 @@ struct ConvWindow {
         const unsigned pad0 = ((unsigned)(b_left - 1) & kOutOfRange) | dead, pad1 = ((unsigned)(b_left - 5) & kOutOfRange) | dead;
 #pragma unroll
         for (int i = 0; i < P_IT; i++) {
-            const unsigned at = x_off + (unsigned)c0 * 4u + (unsigned)i * x_step;
+            const unsigned at = (x_off + (unsigned)c0 * 4u + (unsigned)i * x_step) | (needed(i) ? 0u : kOutOfRange);
             b_reg[i][0] = buffer_load_f32x4(xr, at | pad0);
             b_reg[i][1] = buffer_load_f32x4(xr, at | pad1, 16u);
         }
     };
-    const float floor = relu_floor(a.pre_relu != 0);
     const bool ragged = (a.ICg & 3) != 0;
     float peak = 0.f;   // two terms: largest magnitude this thread has staged
     auto store_window = [&](int buf) {
         uintx4 *at = lds + buf * BUF + half * S + (tid >> 1);
 #pragma unroll
         for (int i = 0; i < P_IT; i++) {
+            if (!needed(i)) break;
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = relu_above(floor, b_reg[i][j >> 2][j & 3]);
+            for (int j = 0; j < 8; j++) v[j] = b_reg[i][j >> 2][j & 3];
+            if (a.pre_relu != 0)
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = relu_above(0.f, v[j]);
             if (ragged)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = j < b_left ? v[j] : 0.f;
@@ -177,6 +186,58 @@ struct ConvWindow {
         r_ch += wrap ? 1 : 0;
         r_at = wrap ? (unsigned)r_ch * chunk_bytes : r_at + tap_bytes;
     };
+    // With the number of taps known, the places of a lane's operands are computed once, and a unit is its loads, its LDS reads and its
+    // matrix work; otherwise address arithmetic takes as long as half of that (192 -> 192 1 x 7 on 17 x 17 at batch 64: 2.6 us a chunk, 0.8 of
+    // them with neither loads nor matrix work).  That layer with 64 x 256 outputs per block 40.0 -> 36.4 us with what follows, 96 -> 96 3 x 3 on
+    // 35 x 35 (32 x 256) 52.8 -> 49.0, 80 -> 192 on 73 x 73 304 -> 289.
+    unsigned place[TAPS > 0 ? TAPS : 1][TN];
+    if constexpr (TAPS > 0) {
+        int shift = 0, kw = 0;
+#pragma unroll
+        for (int t = 0; t < TAPS; t++) {
+#pragma unroll
+            for (int j = 0; j < TN; j++) place[t][j] = (inside[j] >> t & 1u) != 0 ? at0[j] + (unsigned)shift : kZero;
+            const bool wrap = ++kw == a.KW;
+            shift += wrap ? (a.W - a.KW + 1) * 16 : 16;
+            kw = wrap ? 0 : kw;
+        }
+    }
+    auto filters_at = [&](uintx4 (&v)[TERMS][TM], unsigned at, bool live) {
+        const __amdgpu_buffer_rsrc_t wr = buffer_of(a.wp, live ? a.w_bytes : 0u);
+#pragma unroll
+        for (int p = 0; p < TERMS; p++)
+#pragma unroll
+            for (int i = 0; i < TM; i++) v[p][i] = __builtin_amdgcn_raw_buffer_load_b128(wr, a_off[i], (live ? at : 0u) + (unsigned)p * plane_bytes, 0);
+    };
+    // Filters are requested two taps ahead and the next window behind the third tap's: loads return in order, so whoever waits for filters
+    // requested behind a window waits for the window.  SETS sets of registers take turns, tap t in set t % SETS; the first two taps of the
+    // next chunk find sets 0 and 1 free.  (With the filters of a chunk in LDS, staged like the window, no wait is left inside a chunk, and it
+    // was no faster: 36.4 against 35.4 us on the first of these layers.)
+    constexpr int SETS = TAPS % 3 == 0 ? 3 : TAPS % 4 == 3 ? 4 : 5;
+    static_assert(TAPS == 0 || (TAPS % SETS == 0) || (TAPS % SETS == SETS - 1), "the last taps leave the first sets alone");
+    uintx4 fv[TAPS > 0 ? SETS : 1][TERMS][TM];
+    auto known_chunk = [&](int ch, auto buffer) {
+        constexpr int B = decltype(buffer)::value;
+        store_window(B);
+        __syncthreads();
+        const char *buf = reinterpret_cast<const char *>(smem) + B * BUF * 16;
+        const unsigned at = (unsigned)ch * chunk_bytes;
+#pragma unroll
+        for (int t = 0; t < TAPS; t++) {
+            uintx4 bv[TERMS][TN];
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int q = 0; q < TERMS; q++) bv[q][j] = reinterpret_cast<const uintx4 *>(buf + place[t][j])[q * 2 * S];
+            if (t + 2 < TAPS) filters_at(fv[(t + 2) % SETS], at + (unsigned)(t + 2) * tap_bytes, true);
+            else filters_at(fv[t + 2 - TAPS], at + chunk_bytes + (unsigned)(t + 2 - TAPS) * tap_bytes, ch + 1 < ch_end);
+            if (t == 0) load_window(ch + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_terms<TERMS, HALF>(acc, fv[t % SETS], bv);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (NBUF == 1) __syncthreads();
+    };
     // tap of the unit at hand, its offset in the patch in bytes
     int u_tap = 0, u_kw = 0, u_shift = 0;
     auto unit = [&](const char *buf, const uintx4 (&fv)[TERMS][TM], uintx4 (&next)[TERMS][TM]) {
@@ -226,9 +287,11 @@ struct ConvWindow {
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
+    TailConstants<TM> constants;
     bool exact = false;
     if constexpr (TERMS == 2) {
         exact = scale == 0.f;
+        if (exact) tail_constants<MT, true>(a, constants, g, m0 + wm * WTM);
         if (exact)
             half_exact_tiles(a, acc, g, m0 + wm * WTM, [&](int j) {
                 const int n = n0 + wn * WTN + j * 32 + lc;
@@ -236,13 +299,25 @@ struct ConvWindow {
             }, 0, a.Kq, ch_begin * 16, ch_end * 16);
     }
     if (!exact) {
-        load_filters(av[0]);
-        load_window(ch_begin);
-        for (int ch = ch_begin; ch < ch_end; ch += 2) {
-            chunk(ch, std::integral_constant<int, 0>{});
-            if (ch + 1 >= ch_end) break;
-            chunk(ch + 1, std::integral_constant<int, 1>{});
+        if constexpr (TAPS > 0) {
+            filters_at(fv[0], (unsigned)ch_begin * chunk_bytes, true);
+            filters_at(fv[1], (unsigned)ch_begin * chunk_bytes + tap_bytes, true);
+            load_window(ch_begin);
+            for (int ch = ch_begin; ch < ch_end; ch += 2) {
+                known_chunk(ch, std::integral_constant<int, 0>{});
+                if (ch + 1 >= ch_end) break;
+                known_chunk(ch + 1, std::integral_constant<int, NBUF - 1>{});
+            }
+        } else {
+            load_filters(av[0]);
+            load_window(ch_begin);
+            for (int ch = ch_begin; ch < ch_end; ch += 2) {
+                chunk(ch, std::integral_constant<int, 0>{});
+                if (ch + 1 >= ch_end) break;
+                chunk(ch + 1, std::integral_constant<int, 1>{});
+            }
         }
+        tail_constants<MT, TERMS == 2>(a, constants, g, m0 + wm * WTM);
         if constexpr (TERMS == 2) {
             if (scale == kHalfScale) {
                 const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem + FLAGS));
@@ -250,39 +325,42 @@ struct ConvWindow {
             } else {
                 __syncthreads();
             }
-            scale_channels(a, acc, g, m0 + wm * WTM, kHalfScale / scale);
         } else {
             __syncthreads();
         }
     }
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, n_end);
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, TERMS == 2>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants, n_end, TERMS == 2 && !exact ? kHalfScale / scale : 0.f);
     return kHalfDone;
     }   // attempt
 };
 
 // X(index, name, TMW, TNW, WM, WN, P_IT, NBUF).  A window of a 3 x 3 filter on wide maps takes 300 pixels beyond the outputs, so
-// the tall-and-narrow blocks are for few channels on large maps; the 128-output blocks serve the smaller maps.
+// the tall-and-narrow blocks are for few channels on large maps; the 128-output blocks serve the smaller maps, those of eight and
+// twelve wavefronts where there is a block or two for a compute unit.
 #define IOS_WINDOW3_VARIANTS(X)                           \
     X(139, "x3_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)       \
-    X(140, "x3_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)       \
-    X(141, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)     \
-    X(142, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)       \
-    X(143, "x3_win_m96n128_w1x4_d", 3, 1, 1, 4, 2, 2)
+    X(140, "x3_win_m64n128_w1x4_d", 2, 1, 1, 4, 2, 2)     \
+    X(141, "x3_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)       \
+    X(142, "x3_win_m96n128_w1x4_d", 3, 1, 1, 4, 2, 2)     \
+    X(143, "x3_win_m64n128_w2x4_d", 1, 1, 2, 4, 1, 2)     \
+    X(144, "x3_win_m64n256_w2x4", 1, 2, 2, 4, 3, 1)       \
+    X(145, "x3_win_m96n128_w3x4_d", 1, 1, 3, 4, 1, 2)
 #define IOS_WINDOW_BF16_VARIANTS(X)                      \
-    X(144, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
-    X(145, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
-    X(146, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(147, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(148, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+    X(146, "wb_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(147, "wb_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(148, "wb_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(149, "wb_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(150, "wb_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
 #define IOS_WINDOW_FP16_VARIANTS(X)                      \
-    X(149, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
-    X(150, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
-    X(151, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
-    X(152, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
-    X(153, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
-constexpr int kFirstWindowVariant = 139, kNumConvVariants = 154;
+    X(151, "wh_win_m192n128_w2x2", 3, 2, 2, 2, 3, 1)     \
+    X(152, "wh_win_m96n128_w1x4", 3, 1, 1, 4, 2, 1)      \
+    X(153, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
+    X(154, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
+    X(155, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+constexpr int kFirstWindowVariant = 139, kNumConvVariants = 156;
 
-// The window kernels (conv_window.hip), in the order of the lists above
-extern const StagedKernel kWindowKernels[];
+// The window kernels in the order of the lists above: for any number of taps (conv_window.hip), for 7 and for 9 (conv_window7.hip,
+// conv_window9.hip)
+extern const KernelPair kWindowKernels[], kWindow7Kernels[], kWindow9Kernels[];
 
 }  // namespace ios

@@ -4,11 +4,12 @@
 
 namespace ios {
 
-#define IOS_WINDOW_KERNEL(TERMS, HALF, ...) {conv_kernel<ConvWindow<TERMS, HALF, __VA_ARGS__>>, conv_kernel<ConvWindow<TERMS, HALF, __VA_ARGS__>, true>},
+#define IOS_WINDOW_KERNEL(TERMS, HALF, ...) \
+    {conv_kernel<ConvWindow<TERMS, HALF, __VA_ARGS__, 0>>, conv_kernel<ConvWindow<TERMS, HALF, __VA_ARGS__, 0>, true>},
 #define IOS_WINDOW3_KERNEL(IDX, NAME, ...) IOS_WINDOW_KERNEL(2, true, __VA_ARGS__)
 #define IOS_WINDOW_BF16_KERNEL(IDX, NAME, ...) IOS_WINDOW_KERNEL(1, false, __VA_ARGS__)
 #define IOS_WINDOW_FP16_KERNEL(IDX, NAME, ...) IOS_WINDOW_KERNEL(1, true, __VA_ARGS__)
-extern const StagedKernel kWindowKernels[] = {IOS_WINDOW3_VARIANTS(IOS_WINDOW3_KERNEL) IOS_WINDOW_BF16_VARIANTS(IOS_WINDOW_BF16_KERNEL)
-                                                  IOS_WINDOW_FP16_VARIANTS(IOS_WINDOW_FP16_KERNEL)};
+extern const KernelPair kWindowKernels[] = {IOS_WINDOW3_VARIANTS(IOS_WINDOW3_KERNEL) IOS_WINDOW_BF16_VARIANTS(IOS_WINDOW_BF16_KERNEL)
+                                                 IOS_WINDOW_FP16_VARIANTS(IOS_WINDOW_FP16_KERNEL)};
 
 }  // namespace ios

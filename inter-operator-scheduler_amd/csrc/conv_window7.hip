@@ -1,0 +1,15 @@
+// The convolution kernels that stage a window of the input (conv_window.h) for seven taps, compiled apart from the others.
+#include "conv_window.h"
+#include "conv_kernel.h"
+
+namespace ios {
+
+#define IOS_WINDOW_KERNEL(TERMS, HALF, ...) \
+    {conv_kernel<ConvWindow<TERMS, HALF, __VA_ARGS__, 7>>, conv_kernel<ConvWindow<TERMS, HALF, __VA_ARGS__, 7>, true>},
+#define IOS_WINDOW3_KERNEL(IDX, NAME, ...) IOS_WINDOW_KERNEL(2, true, __VA_ARGS__)
+#define IOS_WINDOW_BF16_KERNEL(IDX, NAME, ...) IOS_WINDOW_KERNEL(1, false, __VA_ARGS__)
+#define IOS_WINDOW_FP16_KERNEL(IDX, NAME, ...) IOS_WINDOW_KERNEL(1, true, __VA_ARGS__)
+extern const KernelPair kWindow7Kernels[] = {IOS_WINDOW3_VARIANTS(IOS_WINDOW3_KERNEL) IOS_WINDOW_BF16_VARIANTS(IOS_WINDOW_BF16_KERNEL)
+                                                 IOS_WINDOW_FP16_VARIANTS(IOS_WINDOW_FP16_KERNEL)};
+
+}  // namespace ios
