@@ -862,21 +862,22 @@ __device__ __forceinline__ float half_block_peak(float peak, float *words) {
     return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
 }
 
-// The accumulators of TM x TN tiles of 32 x 32 by fp32 multiply-adds, from the packed halves: for inputs no factor serves.  m_base: row
+// The accumulators of TM x TN tiles of MT x MT by fp32 multiply-adds, from the packed halves: for inputs no factor serves.  m_base: row
 // 0 of the tiles; n: this lane's column in tile column j, or negative; K as [k_begin, k_end) of the packed rows, restricted to
 // channels [c_begin, c_end).  The sums are those of the filters as they were given.  Slow on purpose: it takes few registers and runs for values beyond 2^26.
-template <int TM, int TN, typename Pixel>
-__device__ __forceinline__ void half_exact_tiles(const ConvKernelArgs &a, floatx16 (&acc)[TM][TN], int g, int m_base, Pixel n_of, int k_begin,
+template <int MT, int TM, int TN, typename Pixel>
+__device__ __forceinline__ void half_exact_tiles(const ConvKernelArgs &a, typename Mfma<MT>::acc_t (&acc)[TM][TN], int g, int m_base, Pixel n_of, int k_begin,
                                                  int k_end, int c_begin, int c_end) {
     const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
     const int lane = threadIdx.x & 63;
     const float floor = relu_floor(a.pre_relu != 0);
     const _Float16 *planes = reinterpret_cast<const _Float16 *>(a.wp);
     const int taps = a.Kq / a.ICgP;
+    constexpr int Q = Mfma<MT>::ACC / 4;   // quads of rows of a tile that a lane holds
 #pragma unroll 1
-    for (int quad = 0; quad < TM * TN * 4; quad++) {
-        const int q = quad & 3, j = (quad >> 2) % TN, i = (quad >> 2) / TN;
-        const int m = min(m_base + i * 32 + 8 * q + 4 * (lane >> 5), a.OCgP - 4);   // (rows come in fours)
+    for (int quad = 0; quad < TM * TN * Q; quad++) {
+        const int q = quad % Q, j = quad / Q % TN, i = quad / Q / TN;
+        const int m = min(m_base + i * MT + Mfma<MT>::row(4 * q, lane), a.OCgP - 4);   // (rows come in fours)
         const int n = n_of(j);
         const int nn = n >= 0 ? n : 0;
         const int b = (int)fast_div((unsigned)nn, a.div_ohw);
@@ -905,11 +906,11 @@ __device__ __forceinline__ void half_exact_tiles(const ConvKernelArgs &a, floatx
             }
         }
 #pragma unroll
-        for (int e = 0; e < TM * TN * 4; e++)
+        for (int e = 0; e < TM * TN * Q; e++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                floatx16 &to = acc[(e >> 2) / TN][(e >> 2) % TN];
-                to[4 * (e & 3) + v] = quad == e ? sum[v] : to[4 * (e & 3) + v];
+                typename Mfma<MT>::acc_t &to = acc[e / Q / TN][e / Q % TN];
+                to[4 * (e % Q) + v] = quad == e ? sum[v] : to[4 * (e % Q) + v];
             }
     }
 }
@@ -921,17 +922,23 @@ __device__ __forceinline__ uintx4 round_bf16x8(const float (&x)[8]) {
     return __builtin_bit_cast(uintx4, __builtin_convertvector(v, bf16x8));
 }
 
-// TM x TN tiles of 32 x 32 and one unit of 16 k: filter operands av, input operands bv, a plane per term.  Two terms take three
+// TM x TN tiles of 32 x 32 and one unit of 16 k, or of 16 x 16 and 32 k: filter operands av, input operands bv, a plane per term.  Two terms take three
 // instructions, smallest product first; the tiles of a product are independent instructions.
-template <int TERMS, bool HALF, int TM, int TN>
-__device__ __forceinline__ void multiply_terms(floatx16 (&acc)[TM][TN], const uintx4 (&av)[TERMS][TM], const uintx4 (&bv)[TERMS][TN]) {
+__device__ __forceinline__ floatx16 multiply_half(uintx4 a, uintx4 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4 multiply_half(uintx4 a, uintx4 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+}
+template <int TERMS, bool HALF, int TM, int TN, typename Acc>
+__device__ __forceinline__ void multiply_terms(Acc (&acc)[TM][TN], const uintx4 (&av)[TERMS][TM], const uintx4 (&bv)[TERMS][TN]) {
     auto product = [&](auto filter, int plane) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 if constexpr (HALF)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, filter(i)), __builtin_bit_cast(halfx8, bv[plane][j]), acc[i][j], 0, 0, 0);
+                    acc[i][j] = multiply_half(filter(i), bv[plane][j], acc[i][j]);
                 else
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, filter(i)), __builtin_bit_cast(bf16x8, bv[plane][j]), acc[i][j], 0, 0, 0);
             }
@@ -1191,22 +1198,22 @@ struct ConvWsplit {
     static constexpr bool KQUAD = QUAD;                    // packed filters are [k / 4][m][4] instead of [k][m]
     // accumulators + staged operands per lane decide whether the body fits the register budget of a fused launch
     // (the channel-padding-4 forms serve first layers, which are stages of their own: kept out of the fused launches)
-    static constexpr bool FUSABLE = RP < 3 && CP == 0 && E + D * U * (TM + TN) <= (QUAD ? (MT == 32 ? 48 : 56) : 48);   // per-step addressing of the plain layout needs more registers, and so do the 16-register accumulator tuples of the 32 x 32 tiles
+    static constexpr bool FUSABLE = (RP == 3 && MT == 16 && TM * TN <= 2) || (RP < 3 && CP == 0 && E + D * U * (TM + TN) <= (QUAD ? (MT == 32 ? 48 : 56) : 48));   // per-step addressing of the plain layout needs more registers, and so do the 16-register accumulator tuples of the 32 x 32 tiles
     // the two-term bodies of up to two 32 x 32 tiles per wavefront run inside fused launches of the
     // wide-register kernel family (fused_kernel_wide)
-    static constexpr bool FUSABLE_WIDE = RP == 3 && NW <= 8 && TM * TN <= 2;
-    static constexpr int KREDUCED = RP;                    // 0: fp32 filters; 1: packed filters hold bfloat16; 2: IEEE half; 3: two planes of half; 4: one of bfloat16
+    static constexpr bool FUSABLE_WIDE = RP == 3 && NW <= 8 && TM * TN * MT <= 64;
+    static constexpr int KREDUCED = RP;                    // 0: fp32 filters; 1: packed filters hold bfloat16; 2: IEEE half; 3: two planes of half; 4: one of bfloat16; 5: one of half
     static constexpr int PLANES = RP == 3 ? 2 : 1;
-    static constexpr int WAVES_PER_SIMD = RP != 3 ? 1 : TM * TN == 1 ? 5 : TM * TN == 2 ? 3 : 2;
-    // RP == 4: the reduced-precision mode on the same instruction and layout: one plane of filters rounded to bfloat16, inputs
+    static constexpr int WAVES_PER_SIMD = RP != 3 || MT == 16 ? 1 : TM * TN == 1 ? 5 : TM * TN == 2 ? 3 : 2;
+    // RP == 4, 5: the reduced-precision modes on the same instruction and layout: one plane of filters rounded to bfloat16 or half, inputs
     // rounded after the load, one matrix instruction per tile and batch.
     // RP == 3: fp32 results from the half matrix pipe (operands as two terms, three products on v_mfma_f32_32x32x16_f16, see
     // split_half2): filters are split when packed, [k / 8][plane][m][8], and read as operands straight from global memory; a lane
     // splits the eight input values it loads for a batch itself.  Every wavefront decides by itself whether its inputs want another
     // factor, or plain multiply-adds.
     static_assert(!QUAD || U % 4 == 0, "quad loads need whole groups of four k per lane");
-    static_assert(RP >= 0 && RP <= 4 && (RP == 0 || (RP >= 3 ? QUAD && MT == 32 && U == 8 : QUAD && MT == 16 && U == 4)),
-                  "the 16-bit paths are the 16 x 16 x 16 form of the quad layout, the two-term path its 32 x 32 x 16 form");
+    static_assert(RP >= 0 && RP <= 5 && (RP == 0 || (RP >= 3 ? QUAD && U == 8 && (MT == 32 || RP == 3) : QUAD && MT == 16 && U == 4)),
+                  "the 16-bit paths are the 16 x 16 x 16 form of the quad layout, or the 32 x 32 x 16 and 16 x 16 x 32 forms of the octet layout");
 
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *red, int tile, int g, int z) {
@@ -1434,6 +1441,17 @@ struct ConvWsplit {
             }
             multiply_terms<2, true>(acc, A.v, bq);
             return;
+        } else if constexpr (RP == 5) {
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                floatx8 v;
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = relu_above(floor, B[u][j]);
+                const uintx4 bq = __builtin_bit_cast(uintx4, __builtin_convertvector(v, halfx8));   // round to nearest even, overflow to infinity
+#pragma unroll
+                for (int i = 0; i < TM; i++) acc[i][j] = multiply_half(A.v[0][i], bq, acc[i][j]);
+            }
+            return;
         } else if constexpr (RP == 4) {
             // one rounded term: the reduced-precision mode on the 32 x 32 x 16 instruction
 #pragma unroll
@@ -1560,7 +1578,7 @@ struct ConvWsplit {
             if (__builtin_expect(next >= 0.f, 0)) {   // again, with another factor or by plain multiply-adds
                 typename M::acc_t acc[TM][TN];
                 if (next == 0.f) {
-                    half_exact_tiles(a, acc, g, m0, [&](int j) {
+                    half_exact_tiles<MT>(a, acc, g, m0, [&](int j) {
                         const int n = n0 + j * MT + lc;
                         return n < a.Npix ? n : -1;
                     }, s_begin * M::KSTEP, s_end * M::KSTEP, 0, a.ICgP);
@@ -1811,6 +1829,29 @@ struct ConvWsplit {
     X(116, "wb_x1w_m64n64_w4", 2, 2, 4, 2)     \
     X(117, "wb_x1w_m32n32_w8", 1, 1, 8, 2)     \
     X(118, "wb_x1w_m64n64_w2", 2, 2, 2, 2)
+// X(index, name, TM, TN, NW, D): two terms of half on 16 x 16 tiles and 32 k per batch (v_mfma_f32_16x16x32_f16), three instructions of
+// 16 cycles where the fp32 form takes eight of 32: for problems of few tiles, bound by what the wavefronts of a SIMD issue one after the
+// other.  At most 100 registers up to 32 x 16: these run inside every fused launch.  Against the fp32 form, microseconds: 288 -> 384
+// 3 x 3 / 2 on 35 x 35 at batch 1 10.9 -> 10.1, 160 -> 192 7 x 1 on 17 x 17 5.9 -> 5.6, 448 -> 384 3 x 3 on 8 x 8 at batch 5 15.0 -> 13.5.
+#define IOS_WSPLIT_X3S_VARIANTS(X)                \
+    X(156, "x3w_m16n16_w16_t16", 1, 1, 16, 2)     \
+    X(157, "x3w_m16n16_w8_t16", 1, 1, 8, 2)       \
+    X(158, "x3w_m32n16_w16_t16", 2, 1, 16, 2)     \
+    X(159, "x3w_m32n16_w8_t16", 2, 1, 8, 2)       \
+    X(160, "x3w_m32n16_w4_t16", 2, 1, 4, 2)       \
+    X(161, "x3w_m32n32_w8_t16", 2, 2, 8, 2)       \
+    X(162, "x3w_m64n16_w8_t16", 4, 1, 8, 2)       \
+    X(163, "x3w_m64n32_w4_t16", 4, 2, 4, 2)
+// X(index, name, TM, TN, NW, D): the wave-split kernel with one term rounded to half (ConvWsplit, RP = 5; option precision=fp16).  Against the
+// 16 x 16 x 16 forms at batch 7: 192 -> 192 1 x 7 on 17 x 17 9.9 -> 8.6 us, 768 -> 192 7.2 -> 6.7.  (Inside the wide-register fused launches
+// they cost a pass of Inception-v3 at batch 7 more than they gain: 789 against 739 us.)
+#define IOS_WSPLIT_XH_VARIANTS(X)              \
+    X(164, "wh_x1w_m32n32_w4", 1, 1, 4, 2)     \
+    X(165, "wh_x1w_m64n32_w4", 2, 1, 4, 2)     \
+    X(166, "wh_x1w_m32n64_w4", 1, 2, 4, 2)     \
+    X(167, "wh_x1w_m64n64_w4", 2, 2, 4, 2)     \
+    X(168, "wh_x1w_m32n32_w8", 1, 1, 8, 2)     \
+    X(169, "wh_x1w_m64n32_w8", 2, 1, 8, 2)
 
 // A stand-alone kernel and its residual form
 struct KernelPair {
@@ -1818,5 +1859,7 @@ struct KernelPair {
 };
 // conv_tiled.hip, in the order of the lists above
 extern const KernelPair kTiledKernels[], kSplit3Kernels[], kSplit1Kernels[];
-constexpr int kFirstSplit3Variant = 89, kFirstSplit1Variant = 107;
+// conv_wsplit_half.hip, likewise
+extern const KernelPair kWsplitX3sKernels[], kWsplitXhKernels[];
+constexpr int kFirstSplit3Variant = 89, kFirstSplit1Variant = 107, kFirstWsplitX3sVariant = 156, kFirstWsplitXhVariant = 164;
 }  // namespace ios

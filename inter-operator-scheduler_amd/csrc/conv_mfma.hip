@@ -49,6 +49,13 @@ struct VariantEntry {
      {conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>>, conv_kernel<ConvWsplit<32, TM, TN, NW, 8, true, D, 3>, true>}, \
      ConvWsplit<32, TM, TN, NW, 8, true, D, 3>::SMEM_FLOATS},
 
+#define IOS_WSPLIT_HALF_ENTRY(KERNEL, BK, MT, RP, PRECISION, PLANES, NAME, TM, TN, NW, D)                                               \
+    {{NAME, TM * MT, TN * MT, BK, 1, 1, NW, MT, true, ConvWsplit<MT, TM, TN, NW, 8, true, D, RP>::CPAD, true,                            \
+      ConvWsplit<MT, TM, TN, NW, 8, true, D, RP>::FUSABLE, PRECISION, PLANES, ConvWsplit<MT, TM, TN, NW, 8, true, D, RP>::FUSABLE_WIDE},  \
+     KERNEL, ConvWsplit<MT, TM, TN, NW, 8, true, D, RP>::SMEM_FLOATS},
+#define IOS_WSPLIT_X3S_ENTRY(IDX, ...) IOS_WSPLIT_HALF_ENTRY(kWsplitX3sKernels[IDX - kFirstWsplitX3sVariant], 32, 16, 3, PREC_FP32, 2, __VA_ARGS__)
+#define IOS_WSPLIT_XH_ENTRY(IDX, ...) IOS_WSPLIT_HALF_ENTRY(kWsplitXhKernels[IDX - kFirstWsplitXhVariant], 16, 32, 5, PREC_FP16, 1, __VA_ARGS__)
+
 #define IOS_SPLIT1_ENTRY(IDX, NAME, TMW, TNW, WM, WN, PD)                                                                              \
     {{NAME, ConvSplit3<TMW, TNW, WM, WN, PD, 1>::BM, ConvSplit3<TMW, TNW, WM, WN, PD, 1>::BN, 16, WM, WN, 1, 32, false,                   \
       ConvSplit3<TMW, TNW, WM, WN, PD, 1>::CPAD, false, false, PREC_BF16, 1},                                                             \
@@ -87,7 +94,8 @@ static const VariantEntry kVariants[] = {IOS_TILED_VARIANTS(IOS_TILED_ENTRY) IOS
                                              IOS_SPLIT1_VARIANTS(IOS_SPLIT1_ENTRY) IOS_WSPLIT_X1_VARIANTS(IOS_WSPLIT_X1_ENTRY)
                                              IOS_PIPE3_VARIANTS(IOS_PIPE3_ENTRY) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_ENTRY)
                                              IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_ENTRY) IOS_WINDOW3_VARIANTS(IOS_WINDOW3_ENTRY)
-                                             IOS_WINDOW_BF16_VARIANTS(IOS_WINDOW_BF16_ENTRY) IOS_WINDOW_FP16_VARIANTS(IOS_WINDOW_FP16_ENTRY)};
+                                             IOS_WINDOW_BF16_VARIANTS(IOS_WINDOW_BF16_ENTRY) IOS_WINDOW_FP16_VARIANTS(IOS_WINDOW_FP16_ENTRY)
+                                             IOS_WSPLIT_X3S_VARIANTS(IOS_WSPLIT_X3S_ENTRY) IOS_WSPLIT_XH_VARIANTS(IOS_WSPLIT_XH_ENTRY)};
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 static_assert(kNumVariants == kNumConvVariants, "variant lists and count disagree");
 

@@ -200,7 +200,7 @@ struct ConvPipe {
         exact = scale == 0.f;
         if (exact) tail_constants<MT, true>(a, constants, g, m0 + wm * WTM);
         if (exact)
-            half_exact_tiles(a, acc, g, m0 + wm * WTM, [&](int j) {
+            half_exact_tiles<MT>(a, acc, g, m0 + wm * WTM, [&](int j) {
                 const int n = n0 + wn * WTN + j * 32 + lc;
                 return n < a.Npix ? n : -1;
             }, k_begin, k_end, 0, a.ICgP);

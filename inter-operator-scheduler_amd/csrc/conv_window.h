@@ -293,7 +293,7 @@ struct ConvWindow {
         exact = scale == 0.f;
         if (exact) tail_constants<MT, true>(a, constants, g, m0 + wm * WTM);
         if (exact)
-            half_exact_tiles(a, acc, g, m0 + wm * WTM, [&](int j) {
+            half_exact_tiles<MT>(a, acc, g, m0 + wm * WTM, [&](int j) {
                 const int n = n0 + wn * WTN + j * 32 + lc;
                 return n < n_end ? n : -1;
             }, 0, a.Kq, ch_begin * 16, ch_end * 16);
@@ -357,7 +357,7 @@ struct ConvWindow {
     X(153, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
     X(154, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
     X(155, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
-constexpr int kFirstWindowVariant = 139, kNumConvVariants = 156;
+constexpr int kFirstWindowVariant = 139, kNumConvVariants = 170;
 
 // The window kernels in the order of the lists above: for any number of taps (conv_window.hip), for 7 and for 9 (conv_window7.hip,
 // conv_window9.hip)
