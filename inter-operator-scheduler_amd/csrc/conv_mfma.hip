@@ -422,35 +422,64 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
 }
 
 // ---- filter packing ------------------------------------------------------------------------
-// factors behind the planes of two-term filters: channel m's filters are packed times 16 / scale[m], which puts the largest of them
-// (infinities and NaN aside) into [2^14, 2^15); a block per output channel
-__global__ void filter_scale_kernel(const float *w, float *scales, int fan) {
-    const float *row = w + (size_t)blockIdx.x * fan;
-    unsigned most = 0;   // magnitudes compare as integers
-    for (int i = threadIdx.x; i < fan; i += 256) {
-        const unsigned v = __float_as_uint(row[i]) & 0x7fffffffu;
-        if (v < 0x7f800000u) most = max(most, v);
-    }
-    __shared__ unsigned waves[4];
+// Filters as two terms of half, [g][k / 8][plane][m][8], and behind the planes a factor per channel: channel m's filters are packed times
+// 16 / scale[m], which puts the largest of them (infinities
+// and NaN aside) into [2^14, 2^15).  A block reads the filters of four channels twice, for the largest and
+// to pack them (from the L2), and writes 64 bytes at a time.  With a launch of its own for the
+// factors, which costs the host thread that queues the copies too, Inception-v3 at batch 1 that brings its weights along took 2952 us, like
+// this 2588.
+__global__ __launch_bounds__(512) void pack_half2_kernel(const float *w, float *packed, float *scales, int OCg, int OCgP, int ICg, int ICgP, int taps) {
+    const int quads = OCgP / 4, g = blockIdx.x / quads, m0 = 4 * (blockIdx.x - g * quads);
+    const int fan = ICg * taps, octets = taps * ICgP / 8;
+    __shared__ unsigned waves[8];
+    {
+        const int m = m0 + (threadIdx.x >> 7);
+        const float *row = w + ((size_t)g * OCg + min(m, OCg - 1)) * fan;
+        unsigned most = 0;   // magnitudes compare as integers
+#pragma unroll 4
+        for (int i = threadIdx.x & 127; i < fan; i += 128) {
+            const unsigned v = __float_as_uint(row[i]) & 0x7fffffffu;
+            if (v < 0x7f800000u) most = max(most, v);
+        }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, d));
-    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = most;
+        for (int d = 32; d > 0; d >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, d));
+        if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = most;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        most = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
-        // filters times 2^up; their results times 2^-up / kHalfScale (a row of zeros or of subnormal values: as far as it goes)
-        const int up = most == 0 ? 0 : min(14 - ((int)(most >> 23) - 127), 127);
-        scales[blockIdx.x] = __uint_as_float((unsigned)(127 + 4 - up) << 23);
+    const int m = m0 + (threadIdx.x & 3);
+    const unsigned most = max(waves[2 * (threadIdx.x & 3)], waves[2 * (threadIdx.x & 3) + 1]);
+    // filters times 2^up; their results times 2^-up / kHalfScale (a row of zeros or of subnormal values: as far as it goes)
+    const int up = most == 0 ? 0 : min(14 - ((int)(most >> 23) - 127), 127);
+    const float scale = __uint_as_float((unsigned)(127 + 4 - up) << 23);
+    if (threadIdx.x < 4 && m < OCg) scales[g * OCg + m] = scale;
+    const float factor = 16.f / scale;   // (powers of two)
+    const float *row = w + ((size_t)g * OCg + min(m, OCg - 1)) * fan;
+    halfx8 *out = reinterpret_cast<halfx8 *>(packed);
+#pragma unroll 1
+    for (int o = threadIdx.x >> 2; o < octets; o += 128) {
+        const int tap = o * 8 / ICgP, c = o * 8 - tap * ICgP;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = m < OCg && c + j < ICg ? row[(c + j) * taps + tap] : 0.f;
+        halfx8 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float scaled = v[j] * factor;
+            hi[j] = (_Float16)scaled;
+            lo[j] = (_Float16)(scaled - (float)hi[j]);
+        }
+        const size_t at = ((size_t)g * octets + o) * 2 * OCgP + m;
+        out[at] = hi;
+        out[at + OCgP] = lo;
     }
 }
 
 __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int OCgP, int ICg, int ICgP, int taps, int groups, int kvec,
-                                    int precision, int planes, const float *scales) {
+                                    int precision, int planes) {
     // packed[g][k][m] = w[g * OCg + m][c][tap] with k = tap * ICgP + c;  rows with c >= ICg and columns with m >= OCg are zero.
     // kvec = 4: packed[g][k / 4][m][k % 4] instead (ICgP is a multiple of 4)
     // kvec = 8: planes of 16-bit values, packed[g][k / 8][plane][m][k % 8]: three planes with the exact three-term split of every
-    // filter value, two with its two terms of half (scaled, see filter_scale_kernel), or one plane with the value rounded to nearest
-    // even (the reduced-precision modes)
+    // filter value, or one plane with the value rounded to nearest even (the reduced-precision modes)
     const size_t total = (size_t)groups * taps * ICgP * OCgP;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         int m;
@@ -478,12 +507,6 @@ __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int 
                 out[at] = (unsigned short)(hi >> 16);
                 out[at + (size_t)OCgP * 8] = (unsigned short)(mid >> 16);
                 out[at + (size_t)OCgP * 16] = (unsigned short)(lo >> 16);
-            } else if (planes == 2) {
-                const float scaled = m < OCg ? value * (16.f / scales[g * OCg + m]) : 0.f;   // (powers of two)
-                const _Float16 hi = (_Float16)scaled;
-                _Float16 *out = reinterpret_cast<_Float16 *>(packed);
-                out[at] = hi;
-                out[at + (size_t)OCgP * 8] = (_Float16)(scaled - (float)hi);
             } else if (precision == PREC_FP16) {
                 reinterpret_cast<_Float16 *>(packed)[at] = (_Float16)value;   // round to nearest even
             } else {
@@ -517,10 +540,13 @@ void launch_pack_filters(const ConvProblem &p, const ConvLaunch &l, const float 
     const int cpad = kVariants[l.variant].v.cpad;
     const size_t total = (size_t)p.groups * p.Kq(cpad) * p.OCgP();   // elements
     const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 65535);
-    float *scales = packed + total;   // (two planes of half take the room of the elements)
-    if (kVariants[l.variant].v.koct == 2) hipLaunchKernelGGL(filter_scale_kernel, dim3((unsigned)p.OC), dim3(256), 0, stream, w, scales, p.K());
+    if (kVariants[l.variant].v.koct == 2) {   // (two planes of half take the room of the elements)
+        hipLaunchKernelGGL(pack_half2_kernel, dim3((unsigned)(p.groups * (p.OCgP() / 4))), dim3(512), 0, stream, w, packed, packed + total, p.OCg(), p.OCgP(),
+                           p.ICg(), p.ICgP(cpad), p.KH * p.KW);
+        return;
+    }
     hipLaunchKernelGGL(pack_filters_kernel, dim3(blocks), dim3(256), 0, stream, w, packed, p.OCg(), p.OCgP(), p.ICg(), p.ICgP(cpad),
-                       p.KH * p.KW, p.groups, kVariants[l.variant].v.kvec(), kVariants[l.variant].v.precision, kVariants[l.variant].v.koct, scales);
+                       p.KH * p.KW, p.groups, kVariants[l.variant].v.kvec(), kVariants[l.variant].v.precision, kVariants[l.variant].v.koct);
 }
 
 }  // namespace ios
