@@ -148,6 +148,8 @@ static const char *const kNotMeasured[] = {
 
 static bool precise_only(const ConvProblem &p) { return p.K() < 64; }
 
+bool conv_variant_precise(const ConvProblem &p, int variant) { return !(precise_only(p) && kVariants[variant].v.koct == 2); }
+
 bool conv_variant_measured(const ConvProblem &p, int variant) {
     static const std::vector<char> measured = [] {
         std::vector<char> flags(kNumVariants, 1);
@@ -159,7 +161,7 @@ bool conv_variant_measured(const ConvProblem &p, int variant) {
     // (16 -> 64 channels on 55 x 55 at batch 50: 13.1 us by fp32 instructions, 15.2 by two terms); from 64 on the first (2.7e-7 against
     // 3.6e-7 at K = 576), and the three-term kernels are slower or within 1 %.
     const int planes = kVariants[variant].v.koct;
-    if (precise_only(p) ? planes == 2 : planes == 3) return false;
+    if (!conv_variant_precise(p, variant) || (planes == 3 && !precise_only(p))) return false;
     return measured.at(variant) != 0;
 }
 

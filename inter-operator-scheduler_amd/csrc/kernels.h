@@ -121,6 +121,7 @@ struct ConvVariant {
 int conv_num_variants();
 const ConvVariant &conv_variant(int index);
 bool conv_variant_measured(const ConvProblem &p, int variant);   // the tuner tries it
+bool conv_variant_precise(const ConvProblem &p, int variant);   // fp32 configurations: its operands are as good as fp32 ones for this K
 bool conv_variant_takes(const ConvProblem &p, int variant);   // (a launch of another shape runs on a configuration that reads the same packed filters)
 
 struct ConvLaunch {

@@ -176,6 +176,10 @@ void DeviceContext::load_tune_cache() {
             entry.best[c].split_k = split;
         }
         if (!ok) continue;
+        ConvProblem p{};
+        p.IC = v[1]; p.KH = v[5]; p.KW = v[6]; p.groups = std::max(1, v[11]);
+        for (const ConvLaunch &l : entry.best) ok = ok && conv_variant_precise(p, l.variant);
+        if (!ok) continue;   // (written when that name stood for three terms)
         std::ostringstream os;
         for (int i = 0; i < 12; i++) os << (i ? " " : "") << v[i];
         os << ' ' << token;
