@@ -69,6 +69,33 @@ def test_edges(name, precision, key):
             assert_close(got, want, f'{name} {case} split {split} {reduce}')
 
 
+# channels, out channels, map, stride, padding, batch of 1 x 1 filters: one channel short of a quad, of an octet and of a stage's units; one
+# channel beyond them; fewer channels than a stage; pixels beside the map
+POINTS = [(31, 33, (9, 11), 1, 0, 3), (65, 64, (7, 5), 2, 0, 5), (23, 200, (6, 6), 1, 1, 2), (3, 20, (13, 17), 3, 0, 1), (96, 97, (3, 3), 2, 1, 4)]
+
+
+@pytest.mark.parametrize('name,precision,key', [n for n in NAMES if '_win_' not in n[0]], ids=[n[0] for n in NAMES if '_win_' not in n[0]])
+def test_filters_of_one_pixel(name, precision, key):
+    """1 x 1 filters walk K by moving the ends of their buffers: what lies beside the channels they read is NaN and must not show."""
+    rt.set_option('precision', precision)
+    rt.set_option('conv_variant', rt.device_info()['conv_variants'].index(name))
+    for channels, oc, size, stride, pad, batch in POINTS:
+        ios.reset_name()
+        holder = ios.placeholder((channels + 3, *size))
+        block = Block(holder.node, None, [], None)
+        ios.conv2d(block, [[Value(holder.node, 1, channels + 1)]], oc, (1, 1), (stride, stride), (pad, pad), act='identity', is_exit=True)
+        graph = Graph('point', holder.node, [block])
+        graph.init_weights(3, 'he_normal_bias')
+        graph.sequential_schedule()
+        x = np.random.default_rng(channels).standard_normal((batch, channels + 3, *size)).astype(np.float32)
+        want = ios_oracle.run(graph, x, **({key: matrix_path_convs(graph, batch)} if key else {}))
+        x[:, 0] = x[:, channels + 1:] = np.nan
+        for split, reduce in ((1, 'xcd'), (2, 'inline'), (3, 'kernel')):
+            rt.set_option('conv_split_k', split)
+            rt.set_option('split_k_reduce', reduce)
+            assert_close(rt.graph_inference(graph, batch, x), want, f'{name} {channels} -> {oc} stride {stride} padding {pad} split {split} {reduce}')
+
+
 @pytest.mark.parametrize('executor', ['fused', 'fused_graph'])
 @pytest.mark.parametrize('precision,key', [('bf16', 'bf16_convs'), ('fp16', 'fp16_convs')])
 def test_parallel_stage_launches_large_convolutions_by_themselves(precision, key, executor):
