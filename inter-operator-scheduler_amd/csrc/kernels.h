@@ -216,7 +216,7 @@ void launch_unary(const TensorView &x, const TensorView &y, int act, int B, hipS
 // of `nchw` where the view is a part of its pixels (one image).
 void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t stream, long long plane = 0);
 // Fill n floats with a deterministic pattern in [-1, 1) (seeded), or with a constant.
-void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream);
+void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream, float most = 1.f);   // values up to +-most
 void launch_fill_u32(unsigned *dst, size_t n, unsigned value, hipStream_t stream);
 void launch_delay(int steps, hipStream_t stream);   // keeps the stream waiting about 4 us per step
 

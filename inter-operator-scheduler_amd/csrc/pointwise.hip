@@ -266,7 +266,7 @@ void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t s
 }
 
 // ---- fills ---------------------------------------------------------------------------------------------------------
-__global__ void fill_pattern_kernel(float *dst, size_t n, unsigned seed) {
+__global__ void fill_pattern_kernel(float *dst, size_t n, unsigned seed, float most) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         unsigned h = (unsigned)i * 2654435761u ^ seed;
         h ^= h >> 16;
@@ -274,7 +274,7 @@ __global__ void fill_pattern_kernel(float *dst, size_t n, unsigned seed) {
         h ^= h >> 13;
         h *= 0xc2b2ae35u;
         h ^= h >> 16;
-        dst[i] = (float)(h >> 8) * (1.0f / 8388608.0f) - 1.0f;
+        dst[i] = ((float)(h >> 8) * (1.0f / 8388608.0f) - 1.0f) * most;
     }
 }
 
@@ -282,9 +282,9 @@ __global__ void fill_u32_kernel(unsigned *dst, size_t n, unsigned value) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) dst[i] = value;
 }
 
-void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream) {
+void launch_fill_pattern(float *dst, size_t n, unsigned seed, hipStream_t stream, float most) {
     if (n == 0) return;
-    hipLaunchKernelGGL(fill_pattern_kernel, dim3(blocks_for((long long)n, 256, 65535)), dim3(256), 0, stream, dst, n, seed);
+    hipLaunchKernelGGL(fill_pattern_kernel, dim3(blocks_for((long long)n, 256, 65535)), dim3(256), 0, stream, dst, n, seed, most);
 }
 
 void launch_fill_u32(unsigned *dst, size_t n, unsigned value, hipStream_t stream) {

@@ -16,6 +16,7 @@
 #include "fused.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <sstream>
@@ -592,9 +593,15 @@ void Session::pack(const PlanConv &conv, hipStream_t stream) {
 
 void Session::setup(bool pack_filters) {
     hipStream_t main = ctx_.stream(0);
-    if (owns_memory_) launch_fill_pattern(base_, plan_.arena_floats, 0x2468aceu, main);
+    // (also where the memory is shared: a probe before this one left its tensors there)
+    if (owns_memory_ || pack_filters) launch_fill_pattern(base_, plan_.arena_floats, 0x2468aceu, main);
     packed_.assign(plan_.convs.size(), 0);
     for (const PlanConv &conv : plan_.convs) {
+        // A latency is measured without weights: filters with which the tensors neither grow from layer to layer nor with the sums
+        // between them (half of He's bound; the biases of +-1 keep them from vanishing).  With +-1 they grew past 2^26 within five layers,
+        // where the two-term kernels compute by plain multiply-adds: Inception-v3 at batch 1 was searched for 55 s instead of 8.
+        if (pack_filters)
+            launch_fill_pattern(base_ + conv.weight_off, (size_t)conv.problem.OC * conv.problem.K(), 0x2468aceu, main, 0.5f * std::sqrt(6.f / (float)conv.problem.K()));
         // a convolution in front of the average pool it was exchanged with adds zeros; the pool adds the bias
         if (conv.linear) launch_fill_u32(reinterpret_cast<unsigned *>(base_ + conv.zero_bias_off), (size_t)conv.problem.OC, 0u, main);
         // split-K tickets start at zero; every launch leaves them at zero again
