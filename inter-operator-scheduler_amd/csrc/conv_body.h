@@ -41,6 +41,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 struct ConvKernelArgs {
     const float *x;
     const float *wp;
+    const float *w;                   // the filters as they were given
     const float *bias;
     float *y;
     float *ws;
@@ -294,33 +295,15 @@ struct Mfma<16> {
     __device__ static __forceinline__ int row(int v, int lane) { return 4 * (lane >> 4) + v; }
 };
 
-// Factors that undo the scaling of output channels m ... m + 3 of group g (behind the packed planes; the quad that straddles the end
-// reads on into the padding the host reserves).
-__device__ __forceinline__ floatx4 channel_scale_quad(const ConvKernelArgs &a, int g, int m) {
-    const float *scales = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.wp) + a.w_bytes);
-    return *reinterpret_cast<const floatx4_u *>(scales + g * a.OCg + min(m, a.OCg - 1));
-}
+__device__ __forceinline__ floatx4 channel_scale_quad(const ConvKernelArgs &a, int g, int m);   // (with the two-term operands below)
+__device__ __forceinline__ floatx4 channel_least_quad(const ConvKernelArgs &a, int g, int m);
+template <int MT, int TM, int TN, typename Acc>
+__device__ __forceinline__ void scale_channels(const ConvKernelArgs &a, Acc (&acc)[TM][TN], int g, int m_base);
 
-// sums of scaled filters -> sums of the filters as they were given, times `more` (exact); m_base: row 0 of the tiles
-template <int TM, int TN, typename Acc>
-__device__ __forceinline__ void scale_channels(const ConvKernelArgs &a, Acc (&acc)[TM][TN], int g, int m_base, float more) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const floatx4 factor = channel_scale_quad(a, g, m_base + i * 32 + Mfma<32>::row(4 * q, lane)) * more;
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) acc[i][j][4 * q + v] *= factor[v];
-        }
-}
-
-// Bias (and factors, SCALED) of the four output channels per 32 rows that this lane finishes in the epilogue, m_base: row 0 of the
+// Bias (and what belongs to two terms, SCALED) of the four output channels per 32 rows that this lane finishes in the epilogue, m_base: row 0 of the
 // wavefront's tiles; requested before the last barriers of a body, which their latency then overlaps.
 template <int TM>
-struct TailConstants { floatx4 bias[TM], factor[TM]; };
+struct TailConstants { floatx4 bias[TM], factor[TM], least[TM]; };
 template <int MT, bool SCALED, int TM>
 __device__ __forceinline__ void tail_constants(const ConvKernelArgs &a, TailConstants<TM> &c, int g, int m_base) {
     if constexpr (MT == 32) {
@@ -328,7 +311,10 @@ __device__ __forceinline__ void tail_constants(const ConvKernelArgs &a, TailCons
         for (int i = 0; i < TM; i++) {
             const int m = m_base + i * 32 + 4 * (threadIdx.x & 7);
             c.bias[i] = bias_quad(a, g, m);
-            if constexpr (SCALED) c.factor[i] = channel_scale_quad(a, g, m);
+            if constexpr (SCALED) {
+                c.factor[i] = channel_scale_quad(a, g, m);
+                c.least[i] = channel_least_quad(a, g, m);
+            }
         }
     }
 }
@@ -345,10 +331,10 @@ __device__ __forceinline__ void wavefront_lds_fence() {
 // Tail of the LDS-tiled kernels once a block holds its accumulators (wavefronts with wk == 0; the others only take part in the
 // barriers): the split-K exchange in its three forms, then bias, activation and the store through the output view.
 // `smem` is free when this is called, for tail_floats floats per wavefront (32 x 32 tiles).
-// SCALED: the sums are those of scaled filters (see split_half2), times `more`; 0: of the filters as they were given.
+// SCALED: the sums are those of scaled filters (see split_half2) where `scaled` says so, of the filters as they were given otherwise.
 template <int MT, int BM, int BN, int TM, int TN, int WM, int WN, bool RES, bool SCALED = false>
 __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem, typename Mfma<MT>::acc_t (&acc)[TM][TN], int tile, int g, int z,
-                                           int m0, int n0, int wm, int wn, int wk, const TailConstants<TM> &c, int n_limit = INT_MAX, float more = 0.f) {
+                                           int m0, int n0, int wm, int wn, int wk, const TailConstants<TM> &c, int n_limit = INT_MAX, bool scaled = false) {
     using M = Mfma<MT>;
     const int n_end = min(a.Npix, n_limit);   // (a tile that ends before the tensor does)
     constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -357,9 +343,9 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
     const int lc = lane % MT;
     // ---- split-K ----------------------------------------------------------------------------------------------
     if (a.split_k > 1) {
-        if (SCALED && more != 0.f) {   // (slices meet as sums of the filters as they were given)
-            scale_channels(a, acc, g, m0 + wm * WTM, more);
-            more = 0.f;
+        if (SCALED && scaled) {   // (slices meet as sums of the filters as they were given)
+            scale_channels<MT>(a, acc, g, m0 + wm * WTM);
+            scaled = false;
         }
         if (a.counters == nullptr) {
             // two-kernel form: store this slice's partial tile; splitk_reduce_kernel adds the slices, bias and activation
@@ -464,7 +450,7 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
             const int i = t / TN, j = t - i * TN;
             const floatx4 bias = *reinterpret_cast<const floatx4 *>(constants + i * 64 + 4 * quad);
             floatx4 factor = {1.f, 1.f, 1.f, 1.f};
-            if (SCALED && more != 0.f) factor = *reinterpret_cast<const floatx4 *>(constants + i * 64 + 32 + 4 * quad) * more;
+            if (SCALED && scaled) factor = *reinterpret_cast<const floatx4 *>(constants + i * 64 + 32 + 4 * quad);
             floatx4 v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = *reinterpret_cast<const floatx4 *>(place + t * 1024 + (8 * r + px) * 32 + (quad ^ px) * 4);
@@ -761,27 +747,136 @@ __device__ __forceinline__ void split_bf16x3(const float (&x)[8], uintx4 &hi, ui
 // bits (the remainder has twelve bits and a sign, a half takes eleven of them: the last one is lost for a quarter of the values,
 // the other values are exact).  A product is then the sum of three products of halves, each exact in fp32 (hi * hi, hi * lo,
 // lo * hi; the fourth is below 2^-22 of it), against the six of three bfloat16 terms: half the matrix instructions, two operand
-// planes instead of three, four vector instructions per split value instead of seven.  What bounds an fp32 result is the rounding of
-// its sum, and a sum of half as many terms is rounded half as often.  Relative error (2-norm) against 64 bits, three terms -> two, of
-// the LDS-tiled kernels: 1.8e-7 -> 1.5e-7 at K = 131, 4.2e-7 -> 3.1e-7 at 768, 9.5e-7 -> 6.6e-7 at 4032; of four wavefronts that share K: 1.14e-7 ->
-// 1.10e-7, 2.2e-7 -> 1.7e-7, 4.8e-7 -> 3.5e-7.  Below K = 64 the lost bits of the operands weigh more (7.1e-8 -> 8.3e-8 at 16): the tuner does
-// not let the two-term kernels compete there.
+// planes instead of three.  What bounds an fp32 result is the rounding of its sum, and a sum of half as many terms is rounded half as
+// often.  Below K = 64 the lost bits of the operands weigh more (see conv_variant_precise): the tuner does not let the two-term
+// kernels compete there.
 //
-// A half has five bits of exponent, so operands are scaled by powers of two (exact).  Filters: every output channel by its own
-// factor, which puts its largest filter value into [2^14, 2^15); the factors that undo it follow the packed planes.  Inputs: by
-// kHalfScale, their lower term by 2^11 more, which keeps it out of the subnormal halves (its partner, the upper term of the filter,
-// is taken times 2^-11).  That represents inputs up to kHalfMost, with 23 bits from 2^-10 on and to within 2^-32 below.  A
-// wavefront keeps the largest magnitude it has seen; where that is beyond kHalfMost, or so small that 2^-32 would show in the
-// result (below kHalfLeast), the tile is computed again with a factor made for it, and from kHalfWide on (and for
-// infinities) with plain fp32 multiply-adds, which have no limit.
-constexpr float kHalfScale = 0.0625f;
-constexpr float kHalfMost = 65504.f * 16.f;
-constexpr float kHalfLeast = 0.0078125f;
-constexpr float kHalfWide = 67108864.f;
+// A half has five bits of exponent, so operands are scaled by powers of two (exact).  Filters: every output channel by its own factor,
+// which puts its largest filter value into [2^14, 2^15).  Inputs: a tile's by one that its first values choose, with room for two to four
+// more binades below 2^15; where a later value is beyond that, the tile is computed once more with another.  (In the wave-split kernels
+// the lanes that stage a pixel also hold its sums: every pixel has its own factor, and the sums follow when it shrinks.)  The lower terms
+// are taken times 2^8 (inputs) and 2^4 (filters) and their partners in a product, the upper terms, times 2^-8 and 2^-4: as far up from the
+// subnormal halves as the others come down to them.  So an input keeps its 23 bits down to 2^-11 scaled, 2^-22 of the largest or less, a filter
+// down to 2^-7, 2^-21 of the largest of its channel.
+//
+// What lies below is off by an amount that does not shrink with it.  No result may show that, whatever the others are: filters like that are
+// known when they are packed (channel_least), octets of inputs that are all below are counted where they are staged (InputWatch), and
+// a result of theirs that is not 2^22 times what they may have added to it is computed again in fp32 from the filters as they were given
+// (sums_hold), as is one that an infinite value takes part in.  (Of values of a normal distribution one filter in 10^6 is that small, one
+// octet in 10^7, and few of their results.  Every single input held against the window costs the pipelined kernels 8 % more; where the
+// largest of eight neighbouring channels is in it, the others are off by 2^-21 of that one at most.)
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+constexpr float kInputLift = 256.f, kFilterLift = 16.f, kFilterFloor = 0x1p-7f;
+constexpr unsigned kWindow = 26u << 23;   // binades from the limit of the inputs down to 2^-11 scaled, in bits of a float
+// An input below the window is off by 2^-33, its upper term times 2^-4 by 2^-21 against a lower one of 2^-11 of its filter, and the product of
+// lower terms that is left out is 2^-34 of its filter: 2^-31 together, against filters below 2^15.  Eight of them, times 2^22:
+constexpr float kLeastOfOctet = 512.f;
 
-// the two terms of eight values times `scale` (the lower one times 2^11), each as four words of two halves (lower k in the lower
+// A factor as the bits of the power of two that the values stay below: 2^n means a factor of 2^(15 - n).  Values too far from 1
+// (from 2^89 on, and infinities) share the last limit, and their results are computed again; 1 (the smallest subnormal): none chosen.
+constexpr unsigned kNoLimit = 1, kLeastLimit = 39u << 23, kMostLimit = 220u << 23;
+__device__ __forceinline__ float limit_scale(unsigned limit) { return __uint_as_float((269u << 23) - limit); }
+__device__ __forceinline__ float limit_unscale(unsigned limit) { return __uint_as_float(max(limit, kLeastLimit) - (15u << 23)); }
+// limit of values of which `peak` > 0 is the largest
+__device__ __forceinline__ unsigned limit_for(float peak) { return min(max(__float_as_uint(peak) & 0x7f800000u, kLeastLimit - (3u << 23)) + (3u << 23), kMostLimit); }
+
+// Largest magnitude of eight values; NaN does not count.  (The empty assembly keeps the maximum where the values are: put off to the end
+// of the loop that stages them, it keeps all of them in registers.)
+__device__ __forceinline__ float octet_peak(const float (&x)[8]) {
+    float peak = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) peak = fmaxf(fmaxf(fabsf(x[i]), fabsf(x[i + 1])), peak);
+    asm("" : "+v"(peak));
+    return peak;
+}
+// over the lanes of a wavefront that hold the octets of a pixel in the operand layout (lanes equal modulo MT)
+template <int MT>
+__device__ __forceinline__ float pixel_peak(float peak) {
+    uintx2 s = __builtin_bit_cast(uintx2, __builtin_amdgcn_permlane32_swap(__float_as_uint(peak), __float_as_uint(peak), false, false));
+    peak = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+    if constexpr (MT == 16) {
+        s = __builtin_bit_cast(uintx2, __builtin_amdgcn_permlane16_swap(__float_as_uint(peak), __float_as_uint(peak), false, false));
+        peak = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+    }
+    return peak;
+}
+// what a pixel's sums so far are multiplied by when its limit grows
+__device__ __forceinline__ float limit_ratio(unsigned from, unsigned to) {
+    const unsigned d = (to >> 23) - (from >> 23);
+    return d < 127u ? __uint_as_float((127u - d) << 23) : 0.f;
+}
+// so far that what they held may be lost, or to the last one
+__device__ __forceinline__ bool limit_loses(unsigned from, unsigned to) { return to >= kMostLimit || (from != kNoLimit && to - from > (60u << 23)); }
+// What a thread has seen of the inputs: their largest, and how many octets its wavefront staged that have any but zeros and all of those below
+// the window
+struct InputWatch {
+    float peak = 0.f;
+    unsigned below = 0;
+    __device__ __forceinline__ void octet(float most, unsigned limit) {
+        peak = fmaxf(peak, most);
+        below += (unsigned)__popcll(__ballot(__float_as_uint(most) - 1u < limit - (kWindow + 1u)));
+    }
+};
+
+// over a wavefront
+__device__ __forceinline__ float wave_peak(float peak) {
+    auto with = [&](auto control) {
+        return fmaxf(peak, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(peak), decltype(control)::value, 0xf, 0xf, true)));
+    };
+    peak = with(std::integral_constant<int, 0xb1>{});    // lanes 1 0 3 2 of every four
+    peak = with(std::integral_constant<int, 0x4e>{});    // 2 3 0 1
+    peak = with(std::integral_constant<int, 0x141>{});   // 7 ... 0 of every eight
+    peak = with(std::integral_constant<int, 0x140>{});   // 15 ... 0 of every sixteen
+    peak = pixel_peak<16>(peak);
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
+}
+
+// What the wavefronts of a block have seen, or-ed; words: one per wavefront that nothing else uses until the next barrier
+template <int WAVES>
+__device__ __forceinline__ unsigned block_or(unsigned mine, unsigned *words) {
+    if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    unsigned all = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) all |= words[w];
+    return __builtin_amdgcn_readfirstlane(all);
+}
+template <int WAVES>
+__device__ __forceinline__ unsigned block_sum(unsigned mine, unsigned *words) {   // of the wavefronts
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    unsigned all = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) all += words[w];
+    return __builtin_amdgcn_readfirstlane(all);
+}
+template <int WAVES>
+__device__ __forceinline__ float block_peak(float peak, unsigned *words) {
+    peak = wave_peak(peak);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = __float_as_uint(peak);
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) peak = fmaxf(peak, __uint_as_float(words[w]));
+    __syncthreads();
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
+}
+// A tile's limit by the largest of its first values in every thread, with room for two to four binades.  Magnitudes that are common find
+// theirs by a step of comparisons and a barrier.
+template <int WAVES>
+__device__ __forceinline__ unsigned first_limit(float most, unsigned *words) {
+    unsigned state = 0;
+#pragma unroll
+    for (int i = 0; i < 5; i++) state |= __ballot(most >= (i == 0 ? 32.f : i == 1 ? 8.f : i == 2 ? 2.f : i == 3 ? 0.5f : 0.125f)) != 0 ? 16u >> i : 0u;
+    state = block_or<WAVES>(state, words);
+    if (__builtin_expect(state != 0 && state < 16u, 1)) return (state >= 8u ? 134u : state >= 4u ? 132u : state >= 2u ? 130u : 128u) << 23;   // 2^7, 2^5, 2^3, 2
+    const float peak = block_peak<WAVES>(most, words);
+    return peak > 0.f ? limit_for(peak) : 132u << 23;
+}
+
+// the two terms of eight values times `scale` (the lower one times 2^8), each as four words of two halves (lower k in the lower
 // half).  The additions of zero make every step one mixed-precision multiply-add (v_fma_mix*, three per value; products that are
 // converted take five instructions).  No assembly: the compiler does not know what wait the matrix instructions need behind that.
 __device__ __forceinline__ void split_half2(const float (&x)[8], float scale, uintx4 &hi, uintx4 &lo) {
@@ -791,128 +886,278 @@ __device__ __forceinline__ void split_half2(const float (&x)[8], float scale, ui
 #pragma unroll
         for (int u = 0; u < 2; u++) h[u] = (_Float16)__builtin_fmaf(x[2 * i + u], scale, 0.f);
 #pragma unroll
-        for (int u = 0; u < 2; u++) l[u] = (_Float16)__builtin_fmaf(__builtin_fmaf(x[2 * i + u], scale, -(float)h[u]), 2048.f, 0.f);   // (the inner one is exact)
+        for (int u = 0; u < 2; u++) l[u] = (_Float16)__builtin_fmaf(__builtin_fmaf(x[2 * i + u], scale, -(float)h[u]), kInputLift, 0.f);   // (the inner one is exact)
         hi[i] = __builtin_bit_cast(unsigned, h);
         lo[i] = __builtin_bit_cast(unsigned, l);
     }
 }
-// the upper term of a filter operand times 2^-11
-__device__ __forceinline__ uintx4 half_down(uintx4 v) {
-    return __builtin_bit_cast(uintx4, __builtin_bit_cast(halfx8, v) * (_Float16)0.00048828125f);
+
+// upper terms, for their partners
+__device__ __forceinline__ uintx4 half_down(uintx4 v, float lift) { return __builtin_bit_cast(uintx4, __builtin_bit_cast(halfx8, v) * (_Float16)(1.f / lift)); }
+
+// What follows the packed planes: per output channel the factor that undoes its scaling, and 2^22 times what its filters below the window are
+// off by, 0 where it has none: what a sum must be, over the largest input, for that not to show (see above).  Both arrays are read in quads and end in three words of padding.
+__device__ __forceinline__ const float *channel_scales(const ConvKernelArgs &a) {
+    return reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.wp) + a.w_bytes);
 }
-// Largest magnitude of eight values and `peak`; NaN does not count.  (The empty assembly keeps the maximum where the values are: put
-// off to the end of the loop that stages them, it keeps all of them in registers.)
-__device__ __forceinline__ float half_peak(const float (&x)[8], float peak) {
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) peak = fmaxf(fmaxf(fabsf(x[i]), fabsf(x[i + 1])), peak);
-    asm("" : "+v"(peak));
-    return peak;
+__device__ __forceinline__ floatx4 channel_scale_quad(const ConvKernelArgs &a, int g, int m) {
+    return *reinterpret_cast<const floatx4_u *>(channel_scales(a) + g * a.OCg + min(m, a.OCg - 1));
 }
-// factor for inputs of magnitude `peak` > 0 at most: puts them below 2^15
-__device__ __forceinline__ float half_scale_for(float peak) {
-    const int e = (int)(__float_as_uint(peak) >> 23) - 127;   // -127 for subnormal values
-    return __uint_as_float((unsigned)(min(14 - e, 120) + 127) << 23);
-}
-// A tile is computed with kHalfScale first and where its inputs want that once more with the factor the first attempt returns (0: by
-// plain multiply-adds).  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to
-// 100 registers.  again() keeps it from sharing what both attempts derive from the lane.
-constexpr float kHalfDone = -1.f;
-template <typename Attempt>
-__device__ __forceinline__ void half_attempts(Attempt attempt) {
-    const float next = attempt(kHalfScale);
-    if (__builtin_expect(next >= 0.f, 0)) attempt(next);
-}
-__device__ __forceinline__ int again(int v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-// what half_attempts runs after an attempt with kHalfScale whose largest input was `peak`
-__device__ __forceinline__ float half_next_scale(float peak) {
-    if (peak == 0.f || (peak >= kHalfLeast && peak <= kHalfMost)) return kHalfDone;
-    return peak >= kHalfWide ? 0.f : half_scale_for(peak);
-}
-// Largest peak of the lanes of a wavefront; cheaper than that (and only some value half_next_scale lets pass) in the usual case.
-__device__ __forceinline__ float half_wave_peak(float peak) {
-    if (__ballot(peak > kHalfMost) == 0 && __ballot(peak >= kHalfLeast) != 0) return kHalfLeast;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) peak = fmaxf(peak, __shfl_xor(peak, d));
-    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
-}
-// The same over the wavefronts of a block: a barrier in the usual case.  `words`: one per wavefront that nothing else uses until the
-// next barrier.
-template <int WAVES>
-__device__ __forceinline__ float half_block_peak(float peak, float *words) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned *flags = reinterpret_cast<unsigned *>(words);
-    const unsigned mine = (__ballot(peak > kHalfMost) != 0 ? 1u : 0u) | (__ballot(peak >= kHalfLeast) != 0 ? 2u : 0u);
-    if ((threadIdx.x & 63) == 0) flags[wave] = mine;
-    __syncthreads();
-    unsigned all = 0;
-#pragma unroll
-    for (int w = 0; w < WAVES; w++) all |= flags[w];
-    if (__builtin_amdgcn_readfirstlane(all) == 2u) return kHalfLeast;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) peak = fmaxf(peak, __shfl_xor(peak, d));
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) words[wave] = peak;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < WAVES; w++) peak = fmaxf(peak, words[w]);
-    __syncthreads();
-    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(peak)));
+__device__ __forceinline__ floatx4 channel_least_quad(const ConvKernelArgs &a, int g, int m) {
+    return *reinterpret_cast<const floatx4_u *>(channel_scales(a) + a.groups * a.OCg + 3 + g * a.OCg + min(m, a.OCg - 1));
 }
 
-// The accumulators of TM x TN tiles of MT x MT by fp32 multiply-adds, from the packed halves: for inputs no factor serves.  m_base: row
-// 0 of the tiles; n: this lane's column in tile column j, or negative; K as [k_begin, k_end) of the packed rows, restricted to
-// channels [c_begin, c_end).  The sums are those of the filters as they were given.  Slow on purpose: it takes few registers and runs for values beyond 2^26.
-template <int MT, int TM, int TN, typename Pixel>
-__device__ __forceinline__ void half_exact_tiles(const ConvKernelArgs &a, typename Mfma<MT>::acc_t (&acc)[TM][TN], int g, int m_base, Pixel n_of, int k_begin,
-                                                 int k_end, int c_begin, int c_end) {
-    const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
+// sums of scaled filters -> sums of the filters as they were given (exact); m_base: row 0 of the tiles
+template <int MT, int TM, int TN, typename Acc>
+__device__ __forceinline__ void scale_channels(const ConvKernelArgs &a, Acc (&acc)[TM][TN], int g, int m_base) {
     const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < Mfma<MT>::ACC / 4; q++) {
+            const floatx4 factor = channel_scale_quad(a, g, m_base + i * MT + Mfma<MT>::row(4 * q, lane));
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[i][j][4 * q + v] *= factor[v];
+        }
+}
+
+// the scale of the inputs is undone
+template <int TM, int TN, typename Acc>
+__device__ __forceinline__ void unscale_inputs(Acc (&acc)[TM][TN], const unsigned (&limit)[TN]) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const float unscale = limit_unscale(limit[j]);
+#pragma unroll
+        for (int i = 0; i < TM; i++) acc[i][j] *= unscale;
+    }
+}
+
+// What a wavefront knows of its inputs: the limit of those of this lane's pixels, whether it did not serve them, and how many octets may
+// have been below the window.
+template <int TN>
+struct InputRange {
+    unsigned limit[TN];
+    bool wild[TN];
+    unsigned octets;
+};
+// The sums of a wavefront again that small operands may show in, in fp32 from the filters as they were given.  `tiles`: its unscaled sums in
+// LDS, quad q of lane l of tile e = i * TN + j at [(e * Q + q) * 64 + l]; m_base: row 0 of the tiles; n_of(j): this lane's pixel in tile column j, or negative; K as [k_begin, k_end) of the packed rows, restricted to channels [c_begin, c_end).  Returns false where there were any: all sums
+// of the wavefront have then become those of the filters as they were given.  Few of a tile are computed one by one, a lane every 64th
+// of the products, more of them by matrix instructions.  Rare, so the code is short.
+template <int MT, int TM, int TN, typename Pixel>
+__device__ __forceinline__ bool sums_hold(const ConvKernelArgs &a, floatx4 *tiles, const InputRange<TN> &in, int g, int m_base, Pixel n_of,
+                                          int k_begin, int k_end, int c_begin, int c_end) {
+    using M = Mfma<MT>;
+    constexpr int Q = M::ACC / 4, U = 8, kFew = 24;
+    const int lane = threadIdx.x & 63, lk = lane / MT, lc = lane % MT;
+    auto off_in = [&](int e) {   // a bit per sum of this lane in tile e
+        const int i = e / TN, j = e - i * TN;
+        unsigned limit = in.limit[0], bits = 0;
+        bool wild = in.wild[0];
+#pragma unroll
+        for (int c = 1; c < TN; c++) {
+            limit = j == c ? in.limit[c] : limit;
+            wild = j == c ? in.wild[c] : wild;
+        }
+        const bool counts = limit != kNoLimit && n_of(j) >= 0;
+        const float of_inputs = kLeastOfOctet * (float)in.octets * limit_unscale(limit);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int m = m_base + i * MT + M::row(4 * q, lane);
+            const floatx4 least = channel_least_quad(a, g, m), sum = tiles[(e * Q + q) * 64 + lane];
+#pragma unroll
+            for (int v = 0; v < 4; v++)   // (NaN comes from NaN inputs, unless the factors did not serve)
+                bits |= counts && m + v < a.OCg && (fabsf(sum[v]) < least[v] * __uint_as_float(limit) + of_inputs || wild || least[v] == __builtin_inff()) ? 1u << (4 * q + v) : 0u;
+        }
+        return bits;
+    };
+    unsigned any = 0;
+#pragma unroll 1
+    for (int e = 0; e < TM * TN; e++) any |= off_in(e);
+    if (__ballot(any != 0) == 0) return true;
+    const __amdgpu_buffer_rsrc_t xr = buffer_of(a.x, a.x_bytes);
     const float floor = relu_floor(a.pre_relu != 0);
-    const _Float16 *planes = reinterpret_cast<const _Float16 *>(a.wp);
     const int taps = a.Kq / a.ICgP;
-    constexpr int Q = Mfma<MT>::ACC / 4;   // quads of rows of a tile that a lane holds
+    const unsigned fan = (unsigned)(a.ICg * taps);
+    const __amdgpu_buffer_rsrc_t wr = buffer_of(a.w, (unsigned)(a.groups * a.OCg) * fan * 4u);
+    // channels [first, last) of a tap are within the K range
+    auto first_of = [&](int tap) { return max(c_begin, k_begin - tap * a.ICgP); };
+    auto last_of = [&](int tap) { return min(min(c_end, a.ICg), k_end - tap * a.ICgP); };
+    const int c_span = min(c_end, a.ICg) - c_begin;
 #pragma unroll 1
-    for (int quad = 0; quad < TM * TN * Q; quad++) {
-        const int q = quad % Q, j = quad / Q % TN, i = quad / Q / TN;
-        const int m = min(m_base + i * MT + Mfma<MT>::row(4 * q, lane), a.OCgP - 4);   // (rows come in fours)
-        const int n = n_of(j);
-        const int nn = n >= 0 ? n : 0;
-        const int b = (int)fast_div((unsigned)nn, a.div_ohw);
-        const int r = nn - b * a.OHW;
-        const int oh = (int)fast_div((unsigned)r, a.div_ow);
-        const int ow = r - oh * a.OW;
-        floatx4 sum = {0.f, 0.f, 0.f, 0.f};
-        const floatx4 factor = channel_scale_quad(a, g, m) * kHalfScale;
-#pragma unroll 1
-        for (int tap = 0; tap < taps; tap++) {
+    for (int e = 0; e < TM * TN; e++) {
+        const int i = e / TN, j = e - i * TN;
+        unsigned bits = off_in(e);   // (the next lines change the sums)
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            tiles[(e * Q + q) * 64 + lane] *= channel_scale_quad(a, g, m_base + i * MT + M::row(4 * q, lane));
+        }
+        const int n_mine = n_of(j);
+        // place of output pixel n's tap in the input, in bytes, or beyond the extent
+        auto input_at = [&](int n, int tap) {
+            const int nn = n >= 0 ? n : 0;
+            const int b = (int)fast_div((unsigned)nn, a.div_ohw);
+            const int r = nn - b * a.OHW;
+            const int oh = (int)fast_div((unsigned)r, a.div_ow), ow = r - oh * a.OW;
             const int kh = tap / a.KW, kw = tap - kh * a.KW;
             const int ih = oh * a.sh - a.ph + kh, iw = ow * a.sw - a.pw + kw;
             const bool ok = n >= 0 && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-            const unsigned at = (((unsigned)(b * a.H + ih) * (unsigned)a.W + (unsigned)iw) * (unsigned)a.x_ps + (unsigned)(g * a.ICg)) * 4u;
-            const int first = max(c_begin, k_begin - tap * a.ICgP), last = min(min(c_end, a.ICg), k_end - tap * a.ICgP);
-#pragma unroll 1
-            for (int c = first; c < last; c++) {
-                const float x = relu_above(floor, buffer_load_f32(xr, ok ? at + (unsigned)c * 4u : kOutOfRange));
-                const int k = tap * a.ICgP + c;
-                const size_t slot = (((size_t)g * (a.Kq >> 3) + (k >> 3)) * 2 * a.OCgP + m) * 8 + (k & 7);
+            return ok ? (((unsigned)(b * a.H + ih) * (unsigned)a.W + (unsigned)iw) * (unsigned)a.x_ps + (unsigned)(g * a.ICg)) * 4u : kOutOfRange;
+        };
+        // (a sum of zeros is as it should be)
+        unsigned zeros = 0;
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const float w = (float)planes[slot + v * 8] + (float)planes[slot + v * 8 + (size_t)a.OCgP * 8];
-                    sum[v] = __builtin_fmaf(w * factor[v], ok ? x : 0.f, sum[v]);
+        for (int q = 0; q < Q; q++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) zeros |= tiles[(e * Q + q) * 64 + lane][v] == 0.f ? bits & 1u << (4 * q + v) : 0u;
+        if (__ballot(zeros != 0) != 0) {
+            bool any_input = false;
+#pragma unroll 1
+            for (int tap = 0; tap < taps; tap++) {
+                const unsigned at = zeros != 0 ? input_at(n_mine, tap) : kOutOfRange;
+                const int last = last_of(tap);
+#pragma unroll 4
+                for (int c = first_of(tap); c < last; c += 4) {
+                    const floatx4 x = buffer_load_f32x4(xr, (at + (unsigned)c * 4u) | (at & kOutOfRange));
+#pragma unroll
+                    for (int u = 0; u < 4; u++) any_input = any_input || (c + u < last && relu_above(floor, x[u]) != 0.f);
                 }
+            }
+            if (!any_input) bits &= ~zeros;
+        }
+        int total = __popc(bits);
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d);
+        if (__builtin_amdgcn_readfirstlane(total) <= kFew) {
+            while (true) {
+                const unsigned long long lanes = __ballot(bits != 0);
+                if (lanes == 0) break;
+                const int owner = __builtin_ctzll(lanes);
+                const int v = __builtin_ctz((unsigned)__builtin_amdgcn_readlane((int)bits, owner)), n = __builtin_amdgcn_readlane(n_mine, owner);
+                const int m = m_base + i * MT + M::row(v, owner);
+                float sum = 0.f;
+                // (all of K, a value of another tap in every lane where the channels are few: the loads of eight rounds are under way together)
+                int tap = c_span > 0 ? lane / c_span : taps, c = lane - tap * c_span;
+#pragma unroll 1
+                while (__ballot(tap < taps) != 0) {
+                    float x[8], w[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const int channel = c_begin + c, k = tap * a.ICgP + channel;
+                        const bool ok = tap < taps && k >= k_begin && k < k_end;
+                        const unsigned at = input_at(ok ? n : -1, tap);
+                        x[u] = buffer_load_f32(xr, (at + (unsigned)channel * 4u) | (at & kOutOfRange));
+                        w[u] = buffer_load_f32(wr, ok ? ((unsigned)(g * a.OCg + m) * fan + (unsigned)(channel * taps + tap)) * 4u : kOutOfRange);
+                        c += 64;
+                        while (c >= c_span && tap < taps) {
+                            c -= c_span;
+                            tap++;
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; u++) sum = __builtin_fmaf(w[u], relu_above(floor, x[u]), sum);
+                }
+#pragma unroll
+                for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+                if (lane == owner) {
+                    tiles[(e * Q + (v >> 2)) * 64 + lane][v & 3] = sum;
+                    bits &= bits - 1u;
+                }
+            }
+            continue;
+        }
+        const int m = m_base + i * MT + lc;
+        const unsigned w_row = m < a.OCg ? (unsigned)(g * a.OCg + m) * fan * 4u : kOutOfRange;
+        typename M::acc_t sum;
+#pragma unroll
+        for (int v = 0; v < M::ACC; v++) sum[v] = 0.f;
+#pragma unroll 1
+        for (int tap = 0; tap < taps; tap++) {
+            const unsigned at = input_at(n_mine, tap);
+            const int last = last_of(tap);
+#pragma unroll 1
+            for (int c0 = first_of(tap); c0 < last; c0 += U * M::KSTEP) {
+                float w[U], x[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int c = c0 + u * M::KSTEP + lk;
+                    const unsigned kill = c < last ? 0u : kOutOfRange;
+                    w[u] = buffer_load_f32(wr, (w_row + (unsigned)(c * taps + tap) * 4u) | (w_row & kOutOfRange) | kill);
+                    x[u] = buffer_load_f32(xr, (at + (unsigned)c * 4u) | (at & kOutOfRange) | kill);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) sum = M::run(w[u], relu_above(floor, x[u]), sum);
             }
         }
 #pragma unroll
-        for (int e = 0; e < TM * TN * Q; e++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                typename Mfma<MT>::acc_t &to = acc[e / Q / TN][e / Q % TN];
-                to[4 * (e % Q) + v] = quad == e ? sum[v] : to[4 * (e % Q) + v];
-            }
+        for (int v = 0; v < M::ACC; v++)
+            if (bits >> v & 1u) tiles[(e * Q + (v >> 2)) * 64 + lane][v & 3] = sum[v];
     }
+    return false;
+}
+
+// Whether sums_hold need look at a wavefront's unscaled sums, in registers; in and n_of as there.  least: channel_least of the rows of the tiles, a
+// quad 4 * (lane % (MT / 4)) rows into each.  Few rows have one, if any: only theirs are looked at.
+template <int MT, int TM, int TN, typename Pixel>
+__device__ __forceinline__ bool sums_look_off(const ConvKernelArgs &a, const typename Mfma<MT>::acc_t (&acc)[TM][TN], const InputRange<TN> &in, const floatx4 (&least)[TM], int m_base,
+                                              Pixel n_of) {
+    using M = Mfma<MT>;
+    float most = 0.f;   // (what lies behind the last channel may be anything)
+    unsigned quads[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int m = m_base + i * MT + 4 * ((threadIdx.x & 63) % (MT / 4));
+        float mine = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) mine = fmaxf(mine, m + k < a.OCg ? least[i][k] : 0.f);
+        most = fmaxf(most, mine);
+        quads[i] = (unsigned)__ballot(mine > 0.f) & ((1u << (MT / 4)) - 1u);   // a bit per quad of rows
+    }
+    bool off = in.octets != 0;
+#pragma unroll
+    for (int j = 0; j < TN; j++) off = off || in.wild[j];
+    if (__builtin_expect(__ballot(off || most > 0.f) == 0, 1)) return false;
+    most = wave_peak(most);
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < M::ACC / 4; q++) {
+            unsigned mine = 0;   // the quads of rows that the lanes hold in these four registers
+#pragma unroll
+            for (int l = 0; l < 64; l += MT) mine |= 1u << (M::row(4 * q, l) / 4);
+            if ((quads[i] & mine) == 0) continue;
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int v = 4 * q; v < 4 * q + 4; v++)
+                    off = off || (n_of(j) >= 0 && in.limit[j] != kNoLimit && m_base + i * MT + M::row(v, threadIdx.x & 63) < a.OCg &&
+                                  !(fabsf(acc[i][j][v]) >= most * __uint_as_float(in.limit[j])));
+        }
+    return __ballot(off) != 0;
+}
+
+// Both, for sums in registers; `tiles` is free.
+template <int MT, int TM, int TN, typename Pixel>
+__device__ __forceinline__ bool check_sums(const ConvKernelArgs &a, typename Mfma<MT>::acc_t (&acc)[TM][TN], floatx4 *tiles, const InputRange<TN> &in, const floatx4 (&least)[TM], int g,
+                                           int m_base, Pixel n_of, int k_begin, int k_end, int c_begin, int c_end) {
+    constexpr int Q = Mfma<MT>::ACC / 4;
+    const int lane = threadIdx.x & 63;
+    if (__builtin_expect(!sums_look_off<MT>(a, acc, in, least, m_base, n_of), 1)) return true;
+#pragma unroll
+    for (int e = 0; e < TM * TN; e++)
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            tiles[(e * Q + q) * 64 + lane] = floatx4{acc[e / TN][e % TN][4 * q], acc[e / TN][e % TN][4 * q + 1], acc[e / TN][e % TN][4 * q + 2], acc[e / TN][e % TN][4 * q + 3]};
+    if (sums_hold<MT, TM, TN>(a, tiles, in, g, m_base, n_of, k_begin, k_end, c_begin, c_end)) return true;
+#pragma unroll
+    for (int e = 0; e < TM * TN; e++)
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[e / TN][e % TN][4 * q + v] = tiles[(e * Q + q) * 64 + lane][v];
+    return false;
 }
 
 // eight fp32 values rounded to bfloat16 (nearest even), as four words of two (lower k in the lower half)
@@ -923,31 +1168,37 @@ __device__ __forceinline__ uintx4 round_bf16x8(const float (&x)[8]) {
 }
 
 // TM x TN tiles of 32 x 32 and one unit of 16 k, or of 16 x 16 and 32 k: filter operands av, input operands bv, a plane per term.  Two terms take three
-// instructions, smallest product first; the tiles of a product are independent instructions.
+// instructions; the tiles of a product are independent instructions.
 __device__ __forceinline__ floatx16 multiply_half(uintx4 a, uintx4 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
 }
 __device__ __forceinline__ floatx4 multiply_half(uintx4 a, uintx4 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
 }
+template <bool HALF, int TM, int TN, typename Acc>
+__device__ __forceinline__ void multiply_planes(Acc (&acc)[TM][TN], const uintx4 (&av)[TM], const uintx4 (&bv)[TN]) {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            if constexpr (HALF)
+                acc[i][j] = multiply_half(av[i], bv[j], acc[i][j]);
+            else
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av[i]), __builtin_bit_cast(bf16x8, bv[j]), acc[i][j], 0, 0, 0);
+        }
+}
 template <int TERMS, bool HALF, int TM, int TN, typename Acc>
 __device__ __forceinline__ void multiply_terms(Acc (&acc)[TM][TN], const uintx4 (&av)[TERMS][TM], const uintx4 (&bv)[TERMS][TN]) {
-    auto product = [&](auto filter, int plane) {
+    if constexpr (TERMS == 2) {   // smallest products first
+        uintx4 ad[TM], bd[TN];
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+        for (int j = 0; j < TN; j++) bd[j] = half_down(bv[0][j], kFilterLift);
+        multiply_planes<HALF>(acc, av[1], bd);
 #pragma unroll
-            for (int j = 0; j < TN; j++) {
-                if constexpr (HALF)
-                    acc[i][j] = multiply_half(filter(i), bv[plane][j], acc[i][j]);
-                else
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, filter(i)), __builtin_bit_cast(bf16x8, bv[plane][j]), acc[i][j], 0, 0, 0);
-            }
-    };
-    if constexpr (TERMS == 2) {
-        product([&](int i) { return av[1][i]; }, 0);
-        product([&](int i) { return half_down(av[0][i]); }, 1);
+        for (int i = 0; i < TM; i++) ad[i] = half_down(av[0][i], kInputLift);
+        multiply_planes<HALF>(acc, ad, bv[1]);
     }
-    product([&](int i) { return av[0][i]; }, 0);
+    multiply_planes<HALF>(acc, av[0], bv[0]);
 }
 
 // TMW x TNW MFMA tiles of 32 x 32 per wavefront, WM x WN wavefronts per block
@@ -1204,13 +1455,12 @@ struct ConvWsplit {
     static constexpr bool FUSABLE_WIDE = RP == 3 && NW <= 8 && TM * TN * MT <= 64;
     static constexpr int KREDUCED = RP;                    // 0: fp32 filters; 1: packed filters hold bfloat16; 2: IEEE half; 3: two planes of half; 4: one of bfloat16; 5: one of half
     static constexpr int PLANES = RP == 3 ? 2 : 1;
-    static constexpr int WAVES_PER_SIMD = RP != 3 || MT == 16 ? 1 : TM * TN == 1 ? 5 : TM * TN == 2 ? 3 : 2;
+    static constexpr int WAVES_PER_SIMD = RP != 3 || MT == 16 ? 1 : TM * TN == 1 ? 4 : TM * TN == 2 ? 3 : 2;
     // RP == 4, 5: the reduced-precision modes on the same instruction and layout: one plane of filters rounded to bfloat16 or half, inputs
     // rounded after the load, one matrix instruction per tile and batch.
     // RP == 3: fp32 results from the half matrix pipe (operands as two terms, three products on v_mfma_f32_32x32x16_f16, see
     // split_half2): filters are split when packed, [k / 8][plane][m][8], and read as operands straight from global memory; a lane
-    // splits the eight input values it loads for a batch itself.  Every wavefront decides by itself whether its inputs want another
-    // factor, or plain multiply-adds.
+    // splits the eight input values it loads for a batch itself.  The scale of a pixel is kept by the lanes that hold its sums.
     static_assert(!QUAD || U % 4 == 0, "quad loads need whole groups of four k per lane");
     static_assert(RP >= 0 && RP <= 5 && (RP == 0 || (RP >= 3 ? QUAD && U == 8 && (MT == 32 || RP == 3) : QUAD && MT == 16 && U == 4)),
                   "the 16-bit paths are the 16 x 16 x 16 form of the quad layout, or the 32 x 32 x 16 and 16 x 16 x 32 forms of the octet layout");
@@ -1249,11 +1499,15 @@ struct ConvWsplit {
             if constexpr (RP == 3) factor_pre[t] = channel_scale_quad(a, g, row);
         }
     };
-    // the sums of this wavefront's K range into acc (two terms: of inputs times `scale`); returns the largest input magnitude (two terms)
-    auto sums = [&](typename M::acc_t (&acc)[TM][TN], const int lane, const float scale) {
-    const int lk = lane / MT;
-    const int lc = lane % MT;
-    float peak = 0.f;
+    typename M::acc_t acc[TM][TN];
+    // two terms: the limits of this lane's pixels, which follow their values
+    InputRange<TN> in;
+    unsigned below = 0;
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        in.limit[j] = kNoLimit;
+        in.wild[j] = false;
+    }
     int ih0[TN], iw0[TN];
     unsigned x_lane[TN];   // byte offset of (image, ih0, iw0, first channel of the lane); may wrap below zero, the tap offset brings it back
     bool n_ok[TN];
@@ -1291,7 +1545,7 @@ struct ConvWsplit {
 #pragma unroll
     for (int j = 0; j < TN; j++) n_kill[j] = n_ok[j] ? 0u : kOutOfRange;
 
-    if constexpr (RP != 3) request_bias();
+    if constexpr (RP != 3 || GPW == 1) request_bias();
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -1436,8 +1690,19 @@ struct ConvWsplit {
                 float v[8];
 #pragma unroll
                 for (int u = 0; u < 8; u++) v[u] = relu_above(floor, B[u][j]);
-                peak = half_peak(v, peak);
-                split_half2(v, scale, bq[0][j], bq[1][j]);
+                const float mine = octet_peak(v), peak = pixel_peak<MT>(mine);
+                unsigned &limit = in.limit[j];
+                if (__builtin_expect(__ballot(peak >= __uint_as_float(limit)) != 0, 0)) {   // the sums follow
+                    const unsigned next = peak >= __uint_as_float(limit) ? limit_for(peak) : limit;
+                    in.wild[j] = in.wild[j] || (next != limit && limit_loses(limit, next));
+                    const float ratio = limit_ratio(limit, next);
+                    limit = next;
+#pragma unroll
+                    for (int i = 0; i < TM; i++) acc[i][j] *= ratio;
+                }
+                const unsigned long long small = __ballot(__float_as_uint(mine) - 1u < limit - (kWindow + 1u));
+                if (__builtin_expect(small != 0, 0)) below += (unsigned)__popcll(small);
+                split_half2(v, limit_scale(limit), bq[0][j], bq[1][j]);
             }
             multiply_terms<2, true>(acc, A.v, bq);
             return;
@@ -1548,8 +1813,6 @@ struct ConvWsplit {
         }
     };
     k_loop();
-    return peak;
-    };
     // partial tiles meet in LDS: quad e4 (accumulator elements 4 * e4 ... + 3) of lane l of wavefront w lives in
     // red4[(w * G + e4) * 64 + l]
     floatx4 *red4 = reinterpret_cast<floatx4 *>(red);
@@ -1564,34 +1827,26 @@ struct ConvWsplit {
                     red4[(wave * G + (i * TN + j) * (M::ACC / 4) + q) * 64 + lane] = v;
                 }
     };
-    // two terms: whether a wavefront's sums are those of the filters as they were given (see half_exact_tiles), not of the scaled ones
+    // two terms: whether a wavefront's sums are those of the filters as they were given, not of the scaled ones
     int *exact_flags = reinterpret_cast<int *>(red) + NW * E * 64;
-    {
-        typename M::acc_t acc[TM][TN];
-        if constexpr (RP == 3 && GPW == 1) request_bias();
-        const float peak = sums(acc, lane, kHalfScale);
-        if constexpr (RP == 3 && GPW > 1) request_bias();   // (more of them wait until the K loop has given its registers back)
+    if constexpr (RP != 3) {
         hand_over(acc);
-        if constexpr (RP == 3) {
-            const float next = half_next_scale(half_wave_peak(peak));
-            if (lane == 0) exact_flags[wave] = next == 0.f ? 1 : 0;
-            if (__builtin_expect(next >= 0.f, 0)) {   // again, with another factor or by plain multiply-adds
-                typename M::acc_t acc[TM][TN];
-                if (next == 0.f) {
-                    half_exact_tiles<MT>(a, acc, g, m0, [&](int j) {
-                        const int n = n0 + j * MT + lc;
-                        return n < a.Npix ? n : -1;
-                    }, s_begin * M::KSTEP, s_end * M::KSTEP, 0, a.ICgP);
-                } else {
-                    (void)sums(acc, again(lane), next);
+    } else {
+        auto pixel_of = [&](int j) {
+            const int n = n0 + j * MT + lc;
+            return n < a.Npix ? n : -1;
+        };
+        unscale_inputs(acc, in.limit);
+        in.octets = below;
+        floatx4 least[TM];
 #pragma unroll
-                    for (int i = 0; i < TM; i++)
-#pragma unroll
-                        for (int j = 0; j < TN; j++) acc[i][j] *= kHalfScale / next;
-                }
-                hand_over(acc);
-            }
-        }
+        for (int i = 0; i < TM; i++) least[i] = channel_least_quad(a, g, m0 + i * MT + 4 * (lane % (MT / 4)));
+        const bool off = batches > 0 && sums_look_off<MT>(a, acc, in, least, m0, pixel_of);
+        hand_over(acc);
+        if constexpr (GPW > 1) request_bias();   // (more of them wait until the K loop has given its registers back)
+        bool scaled = true;
+        if (__builtin_expect(off, 0)) scaled = sums_hold<MT, TM, TN>(a, red4 + wave * G * 64, in, g, m0, pixel_of, s_begin * M::KSTEP, s_end * M::KSTEP, 0, a.ICgP);
+        if (lane == 0) exact_flags[wave] = scaled ? 0 : 1;
     }
     __syncthreads();
     auto meet = [&](int t) {   // quad wave + t * NW of the tile: wavefronts in ascending order

@@ -289,7 +289,7 @@ bool conv_matrix_path_supported(const ConvProblem &p) {
 }
 
 ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed,
-                                const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce,
+                                const float *filters, const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce,
                                 const TensorView *residual, bool post_relu) {
     const int variant = variant_for(p, l);
     const VariantEntry &e = kVariants[variant];
@@ -301,6 +301,7 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     ConvKernelArgs &a = d.args;
     a.x = x.ptr;
     a.wp = packed;
+    a.w = filters;
     a.bias = bias;
     a.y = y.ptr;
     a.ws = workspace;
@@ -400,10 +401,10 @@ static int kernel_of(const ConvProblem &p, const VariantEntry &e) {
     return e.special[0].kernel != nullptr && taps == 1 && p.groups == 1 ? 1 : 0;
 }
 
-void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed,
+void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed, const float *filters,
                       const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce, hipStream_t stream,
                       const TensorView *residual, bool post_relu) {
-    const ConvDispatch d = make_conv_dispatch(p, l, x, packed, bias, y, workspace, reduce, residual, post_relu);
+    const ConvDispatch d = make_conv_dispatch(p, l, x, packed, filters, bias, y, workspace, reduce, residual, post_relu);
     const VariantEntry &e = kVariants[d.variant];
     const dim3 grid = d.xcd_blocks > 0 ? dim3((unsigned)d.xcd_blocks) : dim3((unsigned)d.tiles, (unsigned)d.groups, (unsigned)d.slices);
     const int which = kernel_of(p, e);
@@ -424,16 +425,16 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
 }
 
 // ---- filter packing ------------------------------------------------------------------------
-// Filters as two terms of half, [g][k / 8][plane][m][8], and behind the planes a factor per channel: channel m's filters are packed times
-// 16 / scale[m], which puts the largest of them (infinities
-// and NaN aside) into [2^14, 2^15).  A block reads the filters of four channels twice, for the largest and
-// to pack them (from the L2), and writes 64 bytes at a time.  With a launch of its own for the
-// factors, which costs the host thread that queues the copies too, Inception-v3 at batch 1 that brings its weights along took 2952 us, like
-// this 2588.
-__global__ __launch_bounds__(512) void pack_half2_kernel(const float *w, float *packed, float *scales, int OCg, int OCgP, int ICg, int ICgP, int taps) {
+// Filters as two terms of half, [g][k / 8][plane][m][8], and behind the planes what channel_scale_quad and channel_least read: channel m's
+// filters are packed times 2^up, which puts the largest of them (infinities and NaN aside) into [2^14, 2^15).  A block reads the
+// filters of four channels twice, for the largest and to pack them (from the L2), and writes 64 bytes at a time.  With a launch of its own
+// for the factors, which costs the host thread that queues the copies too, Inception-v3 at batch 1 that brings its weights along took
+// 2952 us, like this 2588.
+__global__ __launch_bounds__(512) void pack_half2_kernel(const float *w, float *packed, float *scales, float *leasts, int OCg, int OCgP, int ICg, int ICgP, int taps) {
     const int quads = OCgP / 4, g = blockIdx.x / quads, m0 = 4 * (blockIdx.x - g * quads);
     const int fan = ICg * taps, octets = taps * ICgP / 8;
     __shared__ unsigned waves[8];
+    __shared__ float parts[8][4];
     {
         const int m = m0 + (threadIdx.x >> 7);
         const float *row = w + ((size_t)g * OCg + min(m, OCg - 1)) * fan;
@@ -450,13 +451,12 @@ __global__ __launch_bounds__(512) void pack_half2_kernel(const float *w, float *
     __syncthreads();
     const int m = m0 + (threadIdx.x & 3);
     const unsigned most = max(waves[2 * (threadIdx.x & 3)], waves[2 * (threadIdx.x & 3) + 1]);
-    // filters times 2^up; their results times 2^-up / kHalfScale (a row of zeros or of subnormal values: as far as it goes)
-    const int up = most == 0 ? 0 : min(14 - ((int)(most >> 23) - 127), 127);
-    const float scale = __uint_as_float((unsigned)(127 + 4 - up) << 23);
-    if (threadIdx.x < 4 && m < OCg) scales[g * OCg + m] = scale;
-    const float factor = 16.f / scale;   // (powers of two)
+    // (2^140 serves the smallest subnormal value and is undone by a subnormal factor; it takes two multiplications)
+    const int up = most == 0 ? 0 : min(14 - ((int)(most >> 23) - 127), 140);
+    const float first = __uint_as_float((unsigned)(127 + min(up, 100)) << 23), second = __uint_as_float((unsigned)(127 + max(up - 100, 0)) << 23);
     const float *row = w + ((size_t)g * OCg + min(m, OCg - 1)) * fan;
     halfx8 *out = reinterpret_cast<halfx8 *>(packed);
+    float least = 0.f;
 #pragma unroll 1
     for (int o = threadIdx.x >> 2; o < octets; o += 128) {
         const int tap = o * 8 / ICgP, c = o * 8 - tap * ICgP;
@@ -466,13 +466,29 @@ __global__ __launch_bounds__(512) void pack_half2_kernel(const float *w, float *
         halfx8 hi, lo;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const float scaled = v[j] * factor;
+            const float scaled = v[j] * first * second;
             hi[j] = (_Float16)scaled;
-            lo[j] = (_Float16)(scaled - (float)hi[j]);
+            lo[j] = (_Float16)((scaled - (float)hi[j]) * kFilterLift);
+            // what a filter below the window is off by, its upper term times 2^-8 against a lower one (2^-11 of the input, times 2^8), and
+            // the product of lower terms that is left out (infinite and NaN filters: all results of the channel are computed again)
+            const float upper = (float)hi[j], lower = (float)lo[j] / kFilterLift, down = upper / kInputLift;
+            const float off = fabsf(scaled - upper - lower) + (fabsf(down - (float)(_Float16)down) * kInputLift + fabsf(lower)) * 0x1p-11f;
+            least += __builtin_isfinite(scaled) ? fabsf(scaled) < kFilterFloor ? off : 0.f : __builtin_inff();
         }
         const size_t at = ((size_t)g * octets + o) * 2 * OCgP + m;
         out[at] = hi;
         out[at + OCgP] = lo;
+    }
+#pragma unroll
+    for (int d = 32; d >= 4; d >>= 1) least += __shfl_xor(least, d);
+    if ((threadIdx.x & 63) < 4) parts[threadIdx.x >> 6][threadIdx.x & 3] = least;
+    __syncthreads();
+    if (threadIdx.x < 4 && m < OCg) {
+        float all = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) all += parts[i][threadIdx.x];
+        scales[g * OCg + m] = __uint_as_float(up <= 126 ? (unsigned)(127 - up) << 23 : 1u << (149 - up));
+        leasts[g * OCg + m] = all * 4200000.f;   // 2^22, and what the sum is rounded by
     }
 }
 
@@ -522,7 +538,7 @@ __global__ void pack_filters_kernel(const float *w, float *packed, int OCg, int 
 
 static size_t packed_floats(const ConvProblem &p, const ConvVariant &v) {
     const size_t elements = (size_t)p.groups * p.Kq(v.cpad) * p.OCgP();
-    if (v.koct == 2) return elements + p.OC + 3;   // two planes of half, the factors of the channels (read in quads)
+    if (v.koct == 2) return elements + 2 * (p.OC + 3);   // two planes of half, two words per channel (read in quads)
     if (v.koct) return (elements * v.koct + 1) / 2;   // planes of bfloat16
     return v.precision != PREC_FP32 ? (elements + 1) / 2 : elements;
 }
@@ -543,7 +559,7 @@ void launch_pack_filters(const ConvProblem &p, const ConvLaunch &l, const float 
     const size_t total = (size_t)p.groups * p.Kq(cpad) * p.OCgP();   // elements
     const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 65535);
     if (kVariants[l.variant].v.koct == 2) {   // (two planes of half take the room of the elements)
-        hipLaunchKernelGGL(pack_half2_kernel, dim3((unsigned)(p.groups * (p.OCgP() / 4))), dim3(512), 0, stream, w, packed, packed + total, p.OCg(), p.OCgP(),
+        hipLaunchKernelGGL(pack_half2_kernel, dim3((unsigned)(p.groups * (p.OCgP() / 4))), dim3(512), 0, stream, w, packed, packed + total, packed + total + p.OC + 3, p.OCg(), p.OCgP(),
                            p.ICg(), p.ICgP(cpad), p.KH * p.KW);
         return;
     }

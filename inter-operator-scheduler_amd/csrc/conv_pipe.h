@@ -4,8 +4,8 @@
 // an fp32 value (TERMS = 2, fp32 accuracy, see split_half2) or one rounded term, bfloat16 or half (TERMS = 1, the
 // reduced-precision modes), on v_mfma_f32_32x32x16.  ConvSplit3 reads its filters from global memory, once per wavefront: at 32 x 64
 // outputs per wavefront the L1 delivers 64 bytes per cycle and compute unit for them alone, its limit.  Here a block reads its
-// filter tile once, and a wavefront computes up to 64 x 64 or 96 x 64 outputs per operand read (24 or 36 matrix instructions of 32
-// cycles for 12 or 15 LDS reads of 8).
+// filter tile once, and a wavefront computes up to 64 x 64 or 96 x 32 outputs per operand read (with two terms 12 or 9 matrix
+// instructions of 32 cycles for 8 LDS reads of 16 bytes per lane).
 //
 // A stage holds KU units of 16 k (a unit lies inside one filter tap).  One stage is two or more matrix times ahead in
 // registers, the next one in LDS; one barrier per stage.  What a stage has to cover is the latency of its loads: with two terms one
@@ -38,22 +38,26 @@ struct ConvPipe {
     // neighbouring lanes store, fall into different banks
     static constexpr int UNIT = 2 * BN + (KU > 1 ? 2 : 0);
     static constexpr int STAGE = A_SLOTS + KU * TERMS * UNIT;
-    static constexpr int FLAGS = std::max(2 * STAGE * 4, WM * WN * tail_floats(TMW, TNW));   // two terms: a word per wavefront behind the operands
-    static constexpr int SMEM_FLOATS = FLAGS + (TERMS == 2 ? 4 * ((WM * WN + 3) / 4) : 0);
+    static constexpr int WORDS = std::max(2 * STAGE * 4, WM * WN * tail_floats(TMW, TNW));
+    static constexpr int SMEM_FLOATS = WORDS + (TERMS == 2 ? WM * WN : 0);   // (two terms: a word per wavefront)
     static_assert(OCT * BN % T == 0 && T % OCT == 0, "input loader shape");
 
+    // Two terms: one limit for the inputs of the tile, by those of its first stage.  Where that does not serve all of them, the tile is
+    // computed again.  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to 100
+    // registers.
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
-        if constexpr (TERMS == 2) half_attempts([&](float scale) { return attempt<RES>(a, smem, tile, g, z, scale); });
-        else attempt<RES>(a, smem, tile, g, z, 1.f);
+        const unsigned limit = attempt<RES>(a, smem, tile, g, z, kNoLimit);
+        if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES>(a, smem, tile, g, z, limit);
     }
 
-    // the tile with inputs times `scale` (two terms); returns what half_attempts takes
+    // limit: kNoLimit for the first attempt.  Returns the limit for another one, or 0.
     template <bool RES>
-    __device__ static __forceinline__ float attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, const float scale) {
+    __device__ static __forceinline__ unsigned attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, unsigned limit) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
-    const int tid = TERMS == 2 ? again(threadIdx.x) : (int)threadIdx.x;
+    int tid = threadIdx.x;
+    if constexpr (TERMS == 2) asm volatile("" : "+v"(tid));   // (keeps the attempts from sharing what both derive from it)
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % WN;
@@ -151,7 +155,20 @@ struct ConvPipe {
         left = c_left;
     };
     const bool ragged = (a.ICg & 3) != 0;
-    float peak = 0.f;   // two terms: largest magnitude this thread has staged
+    InputWatch watch;   // two terms
+    unsigned *words = reinterpret_cast<unsigned *>(smem) + WORDS;
+    auto octet_of = [&](const floatx4 (&br)[2], int left, float (&v)[8]) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = br[j >> 2][j & 3];
+        if (a.pre_relu != 0)
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = relu_above(0.f, v[j]);   // folded ReLU of the producer
+        if (POINT ? left < BK : ragged) {
+            const int mine = POINT ? left - 16 * unit - 8 * half : left;
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = j < mine ? v[j] : 0.f;
+        }
+    };
     auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
         uintx4 *As = lds + buf * STAGE;
         uintx4 *Bs = As + A_SLOTS + unit * (TERMS * UNIT);
@@ -161,21 +178,12 @@ struct ConvPipe {
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
             float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = br[i][j >> 2][j & 3];
-            if (a.pre_relu != 0)
-#pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = relu_above(0.f, v[j]);   // folded ReLU of the producer
-            if (POINT ? left < BK : ragged) {
-                const int mine = POINT ? left - 16 * unit - 8 * half : left;
-#pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = j < mine ? v[j] : 0.f;
-            }
+            octet_of(br[i], left, v);
             const int slot = slot_of(tid / OCT + i * (T / OCT), half);
             if constexpr (TERMS == 2) {
                 uintx4 hi, lo;
-                peak = half_peak(v, peak);
-                split_half2(v, scale, hi, lo);
+                watch.octet(octet_peak(v), limit);
+                split_half2(v, limit_scale(limit), hi, lo);
                 Bs[slot] = hi;
                 Bs[UNIT + slot] = lo;
             } else if constexpr (HALF) {
@@ -186,6 +194,7 @@ struct ConvPipe {
             }
         }
     };
+    const bool first = limit == kNoLimit;
 
     typename M::acc_t acc[TM][TN];
 #pragma unroll
@@ -194,62 +203,75 @@ struct ConvPipe {
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
-    TailConstants<TM> constants;
-    bool exact = false;
+
+    // Register set s holds stage st with st % PD == s.  Iteration st: the matrix work of stage st from LDS buffer st & 1, the
+    // registers of stage st + 1 into the other buffer, stage st + 1 + PD requested into the same registers.  The loop runs in
+    // rounds of PD stages with a straight-line body; stages past the end are loaded as zeros.
+#pragma unroll
+    for (int s = 0; s < PD; s++) load_stage(s, a_reg[s], b_reg[s], b_left[s]);
     if constexpr (TERMS == 2) {
-        exact = scale == 0.f;
-        if (exact) tail_constants<MT, true>(a, constants, g, m0 + wm * WTM);
-        if (exact)
-            half_exact_tiles<MT>(a, acc, g, m0 + wm * WTM, [&](int j) {
-                const int n = n0 + wn * WTN + j * 32 + lc;
-                return n < a.Npix ? n : -1;
-            }, k_begin, k_end, 0, a.ICgP);
+        if (first) {
+            float most = 0.f;
+#pragma unroll
+            for (int i = 0; i < B_IT; i++) {
+                float v[8];
+                octet_of(b_reg[0][i], b_left[0], v);
+                most = fmaxf(most, octet_peak(v));
+            }
+            limit = first_limit<WM * WN>(most, words);
+        }
     }
-    if (!exact) {
-        // Register set s holds stage st with st % PD == s.  Iteration st: the matrix work of stage st from LDS buffer st & 1, the
-        // registers of stage st + 1 into the other buffer, stage st + 1 + PD requested into the same registers.  The loop runs in
-        // rounds of PD stages with a straight-line body; stages past the end are loaded as zeros.
+    store_stage(0, a_reg[0], b_reg[0], b_left[0]);
+    load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
+    __syncthreads();
+    for (int st0 = 0; st0 < stages; st0 += PD) {
 #pragma unroll
-        for (int s = 0; s < PD; s++) load_stage(s, a_reg[s], b_reg[s], b_left[s]);
-        store_stage(0, a_reg[0], b_reg[0], b_left[0]);
-        load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
-        __syncthreads();
-        for (int st0 = 0; st0 < stages; st0 += PD) {
+        for (int s = 0; s < PD; s++) {
+            const int st = st0 + s;
+            const int buf = st & 1;
+            const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
+            const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
 #pragma unroll
-            for (int s = 0; s < PD; s++) {
-                const int st = st0 + s;
-                const int buf = st & 1;
-                const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
-                const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
+            for (int u = 0; u < KU; u++) {
+                uintx4 av[TERMS][TM], bv[TERMS][TN];
 #pragma unroll
-                for (int u = 0; u < KU; u++) {
-                    uintx4 av[TERMS][TM], bv[TERMS][TN];
+                for (int p = 0; p < TERMS; p++) {
 #pragma unroll
-                    for (int p = 0; p < TERMS; p++) {
+                    for (int i = 0; i < TM; i++) av[p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
 #pragma unroll
-                        for (int i = 0; i < TM; i++) av[p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
-#pragma unroll
-                        for (int j = 0; j < TN; j++) bv[p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
-                    }
-                    // all LDS reads of the unit are requested before its first matrix instruction
-                    if (TERMS == 2) __builtin_amdgcn_sched_barrier(0);
-                    multiply_terms<TERMS, HALF>(acc, av, bv);
+                    for (int j = 0; j < TN; j++) bv[p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
                 }
-                store_stage(buf ^ 1, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
-                load_stage(st + 1 + PD, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
-                __syncthreads();
+                // all LDS reads of the unit are requested before its first matrix instruction
+                if (TERMS == 2) __builtin_amdgcn_sched_barrier(0);
+                multiply_terms<TERMS, HALF>(acc, av, bv);
             }
-        }
-        tail_constants<MT, TERMS == 2>(a, constants, g, m0 + wm * WTM);
-        if constexpr (TERMS == 2) {
-            if (scale == kHalfScale) {
-                const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem + FLAGS));
-                if (next >= 0.f) return next;
-            }
+            store_stage(buf ^ 1, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+            load_stage(st + 1 + PD, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
+            __syncthreads();
         }
     }
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, TERMS == 2>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants, INT_MAX, TERMS == 2 && !exact ? kHalfScale / scale : 0.f);
-    return kHalfDone;
+    TailConstants<TM> constants;
+    tail_constants<MT, TERMS == 2>(a, constants, g, m0 + wm * WTM);
+    bool scaled = false;
+    if constexpr (TERMS == 2) {
+        const unsigned state = block_or<WM * WN>((__ballot(watch.peak >= __uint_as_float(limit)) != 0 ? 1u : 0u) | (watch.below != 0 ? 2u : 0u), words);
+        if (__builtin_expect((state & 1u) != 0 && limit != kMostLimit, 0)) return limit_for(block_peak<WM * WN>(watch.peak, words));
+        InputRange<TN> in;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            in.limit[j] = limit;
+            in.wild[j] = limit == kMostLimit;
+        }
+        in.octets = __builtin_expect(state != 0, 0) ? block_sum<WM * WN>(watch.below, words) : 0u;
+        unscale_inputs(acc, in.limit);
+        scaled = check_sums<MT>(a, acc, reinterpret_cast<floatx4 *>(smem + (wm * WN + wn) * tail_floats(TM, TN)), in, constants.least, g, m0 + wm * WTM,
+                                [&](int j) {
+            const int n = n0 + wn * WTN + j * 32 + lc;
+            return n < a.Npix ? n : -1;
+        }, k_begin, k_end, 0, a.ICgP);
+    }
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, TERMS == 2>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants, INT_MAX, scaled);
+    return 0;
     }   // attempt
 };
 

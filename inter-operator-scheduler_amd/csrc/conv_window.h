@@ -33,27 +33,31 @@ struct ConvWindow {
     static constexpr int THREADS = T;
     static constexpr int CPAD = 16;
     static constexpr bool FUSABLE = false;
-    static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : TAPS > 0 ? 3 : 4;
+    static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : TAPS > 0 || TNW == 2 ? 3 : 4;
     static constexpr int SPAN = P_IT * (T / 2);       // pixels of the input a block holds
     // slots of 16 bytes per plane and octet (eight consecutive channels), the last one zero; the octets of a pixel, which
     // neighbouring lanes store, fall into different banks
     static constexpr int S = SPAN + 4;
     static constexpr int BUF = 2 * TERMS * S;
-    static constexpr int FLAGS = std::max(NBUF * BUF * 4, WM * WN * tail_floats(TMW, TNW));   // two terms: a word per wavefront behind the windows
-    static constexpr int SMEM_FLOATS = FLAGS + (TERMS == 2 ? 4 * ((WM * WN + 3) / 4) : 0);
+    static constexpr int WORDS = std::max(NBUF * BUF * 4, WM * WN * tail_floats(TMW, TNW));
+    static constexpr int SMEM_FLOATS = WORDS + (TERMS == 2 ? WM * WN : 0);   // (two terms: a word per wavefront)
 
+    // Two terms: one limit for all pixels of the block (an output reads many of them), by the values of its first window.  Where that does
+    // not serve all of them, the tile is computed again.  The code is there twice: a limit that changes inside the K loop costs it 30 to
+    // 60 registers, a loop around it as many, for addresses and masks that are held for the second time.
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
-        if constexpr (TERMS == 2) half_attempts([&](float scale) { return attempt<RES>(a, smem, tile, g, z, scale); });
-        else attempt<RES>(a, smem, tile, g, z, 1.f);
+        const unsigned limit = attempt<RES>(a, smem, tile, g, z, kNoLimit);
+        if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES>(a, smem, tile, g, z, limit);
     }
 
-    // the tile with inputs times `scale` (two terms); returns what half_attempts takes
+    // limit: kNoLimit for the first attempt.  Returns the limit for another one, or 0.
     template <bool RES>
-    __device__ static __forceinline__ float attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, const float scale) {
+    __device__ static __forceinline__ unsigned attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, unsigned limit) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
-    const int tid = TERMS == 2 ? again(threadIdx.x) : (int)threadIdx.x;
+    int tid = threadIdx.x;
+    if constexpr (TERMS == 2) asm volatile("" : "+v"(tid));   // (keeps the attempts from sharing what both derive from it)
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % WN;
@@ -119,24 +123,29 @@ struct ConvWindow {
         }
     };
     const bool ragged = (a.ICg & 3) != 0;
-    float peak = 0.f;   // two terms: largest magnitude this thread has staged
+    InputWatch watch;   // two terms
+    unsigned *words = reinterpret_cast<unsigned *>(smem) + WORDS;
+    auto octet_of = [&](int i, float (&v)[8]) {   // of the window in registers
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = b_reg[i][j >> 2][j & 3];
+        if (a.pre_relu != 0)
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = relu_above(0.f, v[j]);
+        if (ragged)
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = j < b_left ? v[j] : 0.f;
+    };
     auto store_window = [&](int buf) {
         uintx4 *at = lds + buf * BUF + half * S + (tid >> 1);
+        const float scale = limit_scale(limit);
 #pragma unroll
         for (int i = 0; i < P_IT; i++) {
             if (!needed(i)) break;
             float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = b_reg[i][j >> 2][j & 3];
-            if (a.pre_relu != 0)
-#pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = relu_above(0.f, v[j]);
-            if (ragged)
-#pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = j < b_left ? v[j] : 0.f;
+            octet_of(i, v);
             if constexpr (TERMS == 2) {
                 uintx4 hi, lo;
-                peak = half_peak(v, peak);
+                watch.octet(octet_peak(v), limit);
                 split_half2(v, scale, hi, lo);
                 at[i * (T / 2)] = hi;
                 at[i * (T / 2) + 2 * S] = lo;
@@ -171,6 +180,20 @@ struct ConvWindow {
     constexpr unsigned kZero = (S - 1) * 16;
 
     typename M::acc_t acc[TM][TN];
+    const bool first = limit == kNoLimit;
+    auto begin = [&] {   // behind the request for the first window
+        if constexpr (TERMS == 2) {
+            if (!first) return;
+            float most = 0.f;
+#pragma unroll
+            for (int i = 0; i < P_IT; i++) {
+                float v[8];
+                octet_of(i, v);
+                most = needed(i) ? fmaxf(most, octet_peak(v)) : most;
+            }
+            limit = first_limit<WM * WN>(most, words);
+        }
+    };
     uintx4 av[2][TERMS][TM];
     // next filter operands to request
     int r_tap = 0, r_ch = ch_begin;
@@ -287,50 +310,49 @@ struct ConvWindow {
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int v = 0; v < M::ACC; v++) acc[i][j][v] = 0.f;
+    if constexpr (TAPS > 0) {
+        filters_at(fv[0], (unsigned)ch_begin * chunk_bytes, true);
+        filters_at(fv[1], (unsigned)ch_begin * chunk_bytes + tap_bytes, true);
+        load_window(ch_begin);
+        begin();
+        for (int ch = ch_begin; ch < ch_end; ch += 2) {
+            known_chunk(ch, std::integral_constant<int, 0>{});
+            if (ch + 1 >= ch_end) break;
+            known_chunk(ch + 1, std::integral_constant<int, NBUF - 1>{});
+        }
+    } else {
+        load_filters(av[0]);
+        load_window(ch_begin);
+        begin();
+        for (int ch = ch_begin; ch < ch_end; ch += 2) {
+            chunk(ch, std::integral_constant<int, 0>{});
+            if (ch + 1 >= ch_end) break;
+            chunk(ch + 1, std::integral_constant<int, 1>{});
+        }
+    }
     TailConstants<TM> constants;
-    bool exact = false;
+    tail_constants<MT, TERMS == 2>(a, constants, g, m0 + wm * WTM);
+    bool scaled = false;
     if constexpr (TERMS == 2) {
-        exact = scale == 0.f;
-        if (exact) tail_constants<MT, true>(a, constants, g, m0 + wm * WTM);
-        if (exact)
-            half_exact_tiles<MT>(a, acc, g, m0 + wm * WTM, [&](int j) {
-                const int n = n0 + wn * WTN + j * 32 + lc;
-                return n < n_end ? n : -1;
-            }, 0, a.Kq, ch_begin * 16, ch_end * 16);
-    }
-    if (!exact) {
-        if constexpr (TAPS > 0) {
-            filters_at(fv[0], (unsigned)ch_begin * chunk_bytes, true);
-            filters_at(fv[1], (unsigned)ch_begin * chunk_bytes + tap_bytes, true);
-            load_window(ch_begin);
-            for (int ch = ch_begin; ch < ch_end; ch += 2) {
-                known_chunk(ch, std::integral_constant<int, 0>{});
-                if (ch + 1 >= ch_end) break;
-                known_chunk(ch + 1, std::integral_constant<int, NBUF - 1>{});
-            }
-        } else {
-            load_filters(av[0]);
-            load_window(ch_begin);
-            for (int ch = ch_begin; ch < ch_end; ch += 2) {
-                chunk(ch, std::integral_constant<int, 0>{});
-                if (ch + 1 >= ch_end) break;
-                chunk(ch + 1, std::integral_constant<int, 1>{});
-            }
+        const unsigned state = block_or<WM * WN>((__ballot(watch.peak >= __uint_as_float(limit)) != 0 ? 1u : 0u) | (watch.below != 0 ? 2u : 0u), words);
+        if (__builtin_expect((state & 1u) != 0 && limit != kMostLimit, 0)) return limit_for(block_peak<WM * WN>(watch.peak, words));
+        InputRange<TN> in;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            in.limit[j] = limit;
+            in.wild[j] = limit == kMostLimit;
         }
-        tail_constants<MT, TERMS == 2>(a, constants, g, m0 + wm * WTM);
-        if constexpr (TERMS == 2) {
-            if (scale == kHalfScale) {
-                const float next = half_next_scale(half_block_peak<WM * WN>(peak, smem + FLAGS));
-                if (next >= 0.f) return next;
-            } else {
-                __syncthreads();
-            }
-        } else {
-            __syncthreads();
-        }
+        in.octets = __builtin_expect(state != 0, 0) ? block_sum<WM * WN>(watch.below, words) : 0u;
+        unscale_inputs(acc, in.limit);
+        scaled = check_sums<MT>(a, acc, reinterpret_cast<floatx4 *>(smem + (wm * WN + wn) * tail_floats(TM, TN)), in, constants.least, g, m0 + wm * WTM, [&](int j) {
+            const int n = n0 + wn * WTN + j * 32 + lc;
+            return n < n_end ? n : -1;
+        }, 0, a.Kq, ch_begin * 16, ch_end * 16);
+    } else {
+        __syncthreads();
     }
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, TERMS == 2>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants, n_end, TERMS == 2 && !exact ? kHalfScale / scale : 0.f);
-    return kHalfDone;
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, TERMS == 2>(a, smem, acc, tile, g, z, m0, n0, wm, wn, 0, constants, n_end, scaled);
+    return 0;
     }   // attempt
 };
 

@@ -168,9 +168,9 @@ struct SplitKReduce {
     unsigned *fault = nullptr;   // device-visible word in host memory, set to 1 by a block that runs on an unexpected XCC
 };
 
-// y = act(conv(x, w) + bias).  `packed` comes from launch_pack_filters.  `workspace` holds the split_k
+// y = act(conv(x, w) + bias).  `packed` comes from launch_pack_filters, `filters` are those it packed.  `workspace` holds the split_k
 // partial outputs (conv_workspace_floats).
-void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed,
+void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed, const float *filters,
                       const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce, hipStream_t stream,
                       const TensorView *residual = nullptr, bool post_relu = false);
 

@@ -233,8 +233,12 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
     y.C = p.OC; y.H = p.OH; y.W = p.OW; y.pstride = padded_channels(p.OC);
     x.ptr = tuning_buffer(0, (size_t)p.B * p.H * p.W * x.pstride + 64);   // (a 16-byte load may run past the last channel)
     y.ptr = tuning_buffer(1, (size_t)p.B * p.OH * p.OW * y.pstride);
-    float *packed = tuning_buffer(2, conv_packed_floats_max(p) + p.OC);
-    float *bias = packed + conv_packed_floats_max(p);
+    // Any values do for packed filters, except where two-term kernels read what belongs to a channel behind them: those are packed.
+    const size_t packed_floats = conv_packed_floats_max(p);
+    float *packed = tuning_buffer(2, 2 * packed_floats + p.OC + (size_t)p.OC * p.K());
+    float *two_terms = packed + packed_floats, *bias = two_terms + packed_floats, *filters = bias + p.OC;
+    int two_terms_cpad = 0;
+    launch_fill_pattern(packed, 2 * packed_floats + p.OC + (size_t)p.OC * p.K(), 0x51f15e, streams_[0]);
     hipStream_t stream = streams_[0];
     struct EventPair {   // destroyed on every way out, a failing launch included
         hipEvent_t start = nullptr, stop = nullptr;
@@ -262,7 +266,12 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         const size_t ws = conv_workspace_floats(p, l);
         float *workspace = ws ? tuning_buffer(3, ws) : nullptr;
         const SplitKReduce counters = split_reduce(tuning_counters(conv_counter_count(p, l)));
-        auto issue = [&] { launch_conv_mfma(p, l, x, packed, bias, y, workspace, counters, stream); };
+        const ConvVariant &cv = conv_variant(l.variant);
+        if (cv.koct == 2 && cv.cpad != two_terms_cpad) {
+            launch_pack_filters(p, l, filters, two_terms, stream);
+            two_terms_cpad = cv.cpad;
+        }
+        auto issue = [&] { launch_conv_mfma(p, l, x, cv.koct == 2 ? two_terms : packed, filters, bias, y, workspace, counters, stream); };
         issue();   // warm-up
         // A launch costs the host 3 to 5 us, more than most kernels of a batch-1 network run: the device waits until all of
         // them are queued, so that the events time the kernels and not the host.  Where no kernel is that short, until the first.
@@ -761,7 +770,7 @@ void Session::launch_op(const PlanOp &op, int group, int first, int images) {
             ConvProblem p = c.problem;
             p.B = count;
             const TensorView residual = op.has_residual ? tv(op.residual) : TensorView{};
-            launch_conv_mfma(p, c.launch, in, base_ + c.packed_off, bias_of(c), out,
+            launch_conv_mfma(p, c.launch, in, base_ + c.packed_off, base_ + c.weight_off, bias_of(c), out,
                              c.ws_floats ? base_ + c.ws_off : nullptr, ctx_.split_reduce(counters_of(c), group, !capturing_forks_), stream,
                              op.has_residual ? &residual : nullptr,
                              op.post_relu != 0);
@@ -932,7 +941,7 @@ void Session::build_fused() {
                     case OpKind::ConvMfma: {
                         const PlanConv &c = plan_.convs[op.conv];
                         const TensorView residual = op.has_residual ? tv(op.residual) : TensorView{};
-                        const ConvDispatch d = make_conv_dispatch(c.problem, c.launch, tv(op.in), base_ + c.packed_off, bias_of(c),
+                        const ConvDispatch d = make_conv_dispatch(c.problem, c.launch, tv(op.in), base_ + c.packed_off, base_ + c.weight_off, bias_of(c),
                                                                   tv(op.out), c.ws_floats ? base_ + c.ws_off : nullptr, ctx_.split_reduce(counters_of(c)),
                                                                   op.has_residual ? &residual : nullptr, op.post_relu != 0);
                         pend.fusable = conv_variant(d.variant).fusable() && !op.has_residual;   // (the fused kernel holds the plain epilogue)
