@@ -1449,10 +1449,10 @@ struct ConvWsplit {
     static constexpr bool KQUAD = QUAD;                    // packed filters are [k / 4][m][4] instead of [k][m]
     // accumulators + staged operands per lane decide whether the body fits the register budget of a fused launch
     // (the channel-padding-4 forms serve first layers, which are stages of their own: kept out of the fused launches)
-    static constexpr bool FUSABLE = (RP == 3 && MT == 16 && TM * TN <= 2) || (RP < 3 && CP == 0 && E + D * U * (TM + TN) <= (QUAD ? (MT == 32 ? 48 : 56) : 48));   // per-step addressing of the plain layout needs more registers, and so do the 16-register accumulator tuples of the 32 x 32 tiles
+    static constexpr bool FUSABLE = RP < 3 && CP == 0 && E + D * U * (TM + TN) <= (QUAD ? (MT == 32 ? 48 : 56) : 48);   // per-step addressing of the plain layout needs more registers, and so do the 16-register accumulator tuples of the 32 x 32 tiles
     // the two-term bodies of up to two 32 x 32 tiles per wavefront run inside fused launches of the
     // wide-register kernel family (fused_kernel_wide)
-    static constexpr bool FUSABLE_WIDE = RP == 3 && NW <= 8 && TM * TN * MT <= 64;
+    static constexpr bool FUSABLE_WIDE = RP == 3 && MT == 32 && NW <= 8 && TM * TN <= 2;
     static constexpr int KREDUCED = RP;                    // 0: fp32 filters; 1: packed filters hold bfloat16; 2: IEEE half; 3: two planes of half; 4: one of bfloat16; 5: one of half
     static constexpr int PLANES = RP == 3 ? 2 : 1;
     static constexpr int WAVES_PER_SIMD = RP != 3 || MT == 16 ? 1 : TM * TN == 1 ? 4 : TM * TN == 2 ? 3 : 2;

@@ -65,13 +65,6 @@ __device__ __forceinline__ void fused_item(const WorkItem &item, const int bid, 
         break;
                 IOS_WSPLIT_X3_VARIANTS(IOS_CASE_X3)
 #undef IOS_CASE_X3
-#define IOS_CASE_X3S(IDX, NAME, TM, TN, NW, D)                                                        \
-    case IDX:                                                                                      \
-        if constexpr (64 * NW <= T && (ConvWsplit<16, TM, TN, NW, 8, true, D, 3>::FUSABLE || (WIDE && ConvWsplit<16, TM, TN, NW, 8, true, D, 3>::FUSABLE_WIDE))) \
-            ConvWsplit<16, TM, TN, NW, 8, true, D, 3>::run(a, smem, tile, g, z);                   \
-        break;
-                IOS_WSPLIT_X3S_VARIANTS(IOS_CASE_X3S)
-#undef IOS_CASE_X3S
                 IOS_TILED_VARIANTS(IOS_CASE_TILED)
                 IOS_WSPLIT_VARIANTS(IOS_CASE_WSPLIT)
                 IOS_WSPLIT_C4_VARIANTS(IOS_CASE_WSPLIT_C4)

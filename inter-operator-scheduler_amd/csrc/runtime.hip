@@ -323,20 +323,16 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
         // fastest such configuration
         const bool any_kernel = !fused_executor();
         // A configuration of the wide-register fused family (three wavefronts per SIMD, items fetched from the table) only
-        // competes when it runs for 12 us or more by itself: below that the family's slower start costs more than the
-        // kernel gains (Inception-v3 at batch 1, same device: 0.379-0.385 ms with it against 0.375-0.377 ms without).
-        constexpr float kWideMinMs = 0.012f;
-        // The two-term configurations of the plain families (16 x 16 and 32 x 16 tiles) compete below 9 us: they read their operands twice
-        // as often as the larger tiles of the wide one, which their neighbours in the launch pay for (three convolutions of 375 ... 768
-        // channels on 15 x 15 at batch 1, 11 to 15 us each: 31.3 us with them, 24.7 with 64 x 32 tiles).
-        constexpr float kSmallMaxMs = 0.009f;
-        auto wrong_family = [&](const Candidate &cand) {
-            const ConvVariant &v = conv_variant(cand.launch.variant);
-            return !any_kernel && (v.needs_wide() ? cand.ms < kWideMinMs : v.koct == 2 && v.fusable() && cand.ms >= kSmallMaxMs);
+        // competes when it runs for 9 us or more by itself: below that the family's slower start costs more than the
+        // kernel gains.  (Inception-v3 at batch 1, two runs each: 423 and 413 us from 12 us on, 423 and 421 from 9; at batch 16 2015 and 2000 against
+        // 1946 and 1953, ResNet-50 at batch 5 748 and 751 against 743 and 761.)
+        constexpr float kWideMinMs = 0.009f;
+        auto wide_too_short = [&](const Candidate &cand) {
+            return !any_kernel && conv_variant(cand.launch.variant).needs_wide() && cand.ms < kWideMinMs;
         };
         auto eligible = [&](const Candidate &cand, bool fit) {
             if (c == 0) return true;
-            if (wrong_family(cand)) return false;
+            if (wide_too_short(cand)) return false;
             return (cand.fusable || any_kernel) && (!fit || cand.footprint <= capacity / (1 << c));
         };
         found[c] = false;
@@ -345,7 +341,7 @@ DeviceContext::TunedConv DeviceContext::tune_conv(const ConvProblem &p) {
             auto score = [&](const Candidate &cand) { return cand.ms * (1.0 + ((1 << c) - 1) * cand.footprint / capacity); };
             std::vector<size_t> order;
             for (size_t i = 0; i < candidates.size(); i++)
-                if ((candidates[i].fusable || any_kernel) && !wrong_family(candidates[i])) order.push_back(i);
+                if ((candidates[i].fusable || any_kernel) && !wide_too_short(candidates[i])) order.push_back(i);
             std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return score(candidates[a]) < score(candidates[b]); });
             double best = 1e300;
             for (size_t n = 0; n < order.size() && n < kFinalists; n++) {
