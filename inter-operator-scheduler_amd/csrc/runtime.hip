@@ -177,10 +177,16 @@ void DeviceContext::load_tune_cache() {
             entry.best[c].split_k = split;
         }
         if (!ok) continue;
+        for (int i : {0, 1, 2, 3, 4, 5, 6, 7, 8, 11}) ok = ok && v[i] >= 1;   // (the paddings may be 0)
+        ok = ok && v[9] >= 0 && v[10] >= 0;
+        if (!ok) continue;
         ConvProblem p{};
-        p.IC = v[1]; p.KH = v[5]; p.KW = v[6]; p.groups = std::max(1, v[11]);
-        for (const ConvLaunch &l : entry.best) ok = ok && conv_variant_precise(p, l.variant);
-        if (!ok) continue;   // (written when that name stood for three terms)
+        p.B = v[0]; p.IC = v[1]; p.H = v[2]; p.W = v[3]; p.OC = v[4]; p.KH = v[5]; p.KW = v[6]; p.sh = v[7]; p.sw = v[8]; p.ph = v[9]; p.pw = v[10];
+        p.groups = v[11];
+        p.OH = (p.H + 2 * p.ph - p.KH) / p.sh + 1;
+        p.OW = (p.W + 2 * p.pw - p.KW) / p.sw + 1;
+        for (const ConvLaunch &l : entry.best) ok = ok && conv_variant_measured(p, l.variant) && conv_variant_takes(p, l.variant);
+        if (!ok) continue;   // (a configuration that is not measured for this shape now: written by a build that had other kernels)
         std::ostringstream os;
         for (int i = 0; i < 12; i++) os << (i ? " " : "") << v[i];
         os << ' ' << token;
