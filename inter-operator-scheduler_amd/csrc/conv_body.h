@@ -330,9 +330,10 @@ __device__ __forceinline__ void wavefront_lds_fence() {
 
 // Tail of the LDS-tiled kernels once a block holds its accumulators (wavefronts with wk == 0; the others only take part in the
 // barriers): the split-K exchange in its three forms, then bias, activation and the store through the output view.
-// `smem` is free when this is called, for tail_floats floats per wavefront (32 x 32 tiles).
+// `smem` is free when this is called.
 // SCALED: the sums are those of scaled filters (see split_half2) where `scaled` says so, of the filters as they were given otherwise.
-template <int MT, int BM, int BN, int TM, int TN, int WM, int WN, bool RES, bool SCALED = false>
+// THROUGH_LDS: `smem` holds tail_floats per wavefront too, and results are stored by whole lines of channels.
+template <int MT, int BM, int BN, int TM, int TN, int WM, int WN, bool RES, bool SCALED = false, bool THROUGH_LDS = MT == 32>
 __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem, typename Mfma<MT>::acc_t (&acc)[TM][TN], int tile, int g, int z,
                                            int m0, int n0, int wm, int wn, int wk, const TailConstants<TM> &c, int n_limit = INT_MAX, bool scaled = false) {
     using M = Mfma<MT>;
@@ -422,7 +423,7 @@ __device__ __forceinline__ void tiled_tail(const ConvKernelArgs &a, float *smem,
     }
 
     // ---- epilogue -------------------------------------------------------------------------------------------
-    if constexpr (MT == 32) {
+    if constexpr (THROUGH_LDS) {
         // A lane holds four channels of a pixel, its neighbour the next pixel's: stored like that, every 16 bytes of a wavefront's store
         // go to another line, and the L2 takes a request for each.  So the tiles pass through LDS; eight lanes then take the 128 bytes
         // of a pixel, a lane the same four channels of every pixel of a tile.  What runs once is short (one copy of the code for all
@@ -491,8 +492,11 @@ struct ConvTiled {
     // occupancy of every other operator (the wave-split bodies that serve small problems need 32-72), so they
     // only run as stand-alone kernels.
     static constexpr bool FUSABLE = false;
-    static constexpr int TAIL_FLOATS = MT == 32 ? WM * WN * tail_floats(BM / WM / MT, BN / WN / MT) : 0;
-    static constexpr int SMEM_FLOATS = std::max({TILE_FLOATS, RED_FLOATS, TAIL_FLOATS});
+    // Results go through LDS where two blocks still fit a compute unit (128 x 128 tiles, 33 -> 66 KB: 48 -> 192 channels 1 x 1 on 35 x 35 at
+    // batch 64 41 -> 35 us, 192 -> 256 94 -> 90, 96 -> 192 3 x 3 313 -> 310; 192 x 128 tiles, 41 -> 99 KB: 41 -> 37, but 120 -> 136 and 268 -> 293).
+    static constexpr int TAIL_FLOATS = WM * WN * tail_floats(BM / WM / MT, BN / WN / MT);
+    static constexpr bool THROUGH_LDS = MT == 32 && TAIL_FLOATS <= 20480;
+    static constexpr int SMEM_FLOATS = std::max({TILE_FLOATS, RED_FLOATS, THROUGH_LDS ? TAIL_FLOATS : 0});
 
     // one block: output tile `tile` of group `g`, K slice `z`; smem holds SMEM_FLOATS floats, 16-byte aligned
     template <bool RES = false>
@@ -687,7 +691,7 @@ struct ConvTiled {
 
     TailConstants<TM> constants;
     tail_constants<MT, false>(a, constants, g, m0 + wm * WTM);
-    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES>(a, smem, acc, tile, g, z, m0, n0, wm, wn, wk, constants);
+    tiled_tail<MT, BM, BN, TM, TN, WM, WN, RES, false, THROUGH_LDS>(a, smem, acc, tile, g, z, m0, n0, wm, wn, wk, constants);
     }   // run
 };
 
