@@ -1,5 +1,5 @@
 """The kernels that multiply fp32 operands as two terms of IEEE half (x3p_*, x3_win_*, x3w_*): the powers of two that bring inputs
-and filters into a half's range, the second attempt with another one, and the plain multiply-adds behind it."""
+and filters into a half's range, the second attempt with another one, and the results that are computed again in fp32."""
 import numpy as np
 import pytest
 import torch
@@ -61,7 +61,7 @@ def test_magnitudes(name):
     for e in (-100, -60, -12, -8, 0, 17, 19, 20, 25, 26, 40, 100):   # largest inputs on both sides of every limit
         check(graph, conv, np.ldexp(x, e).astype(np.float32), f'inputs times 2^{e}', 1)
     check(graph, conv, np.ldexp(x, 22).astype(np.float32), 'a second attempt', 3)
-    check(graph, conv, np.ldexp(x, 40).astype(np.float32), 'multiply-adds', 3, 'kernel')
+    check(graph, conv, np.ldexp(x, 40).astype(np.float32), 'far from 1', 3, 'kernel')
     # filters of every channel on another scale
     conv.weight = np.ldexp(weight, rng.integers(-90, 60, (OC, 1, 1, 1))).astype(np.float32)
     check(graph, conv, x, 'filters', 1)
@@ -69,7 +69,7 @@ def test_magnitudes(name):
     conv.weight = np.zeros_like(weight)
     check(graph, conv, x, 'no filters', 1)
     conv.weight = weight
-    # the limits of the first attempt, and the first values beyond them
+    # values on both sides of powers of two and of the largest half
     for value in (65504.0 * 16, 65505.0 * 16, 2.0 ** 26, np.nextafter(np.float32(2.0 ** 26), np.float32(0)), 2.0 ** -7, np.nextafter(np.float32(2.0 ** -7), np.float32(0))):
         check(graph, conv, np.clip(x * np.float32(1e30), -value, value).astype(np.float32), f'largest input {value}', 1)
     check(graph, conv, np.zeros_like(x), 'zeros', 2)
@@ -87,10 +87,10 @@ def test_a_large_value_spares_the_others(name):
     check(graph, conv, x, 'a large value', 2)
     plain = x.copy()
     plain[1, 20, 2, 3] = 0
-    for value in (np.inf, np.nan):
+    for value, split in ((np.inf, 1), (np.inf, 2), (np.nan, 1), (np.nan, 2)):
         x[1, 20, 2, 3] = value
+        rt.set_option('conv_split_k', split)
         got = rt.graph_inference(graph, BATCH, x)
-        rt.set_option('conv_split_k', 1)
         seen = np.zeros(got.shape, bool)
         seen[1, :, 1:4, 2:5] = True
         assert not np.isfinite(got[seen]).any()
