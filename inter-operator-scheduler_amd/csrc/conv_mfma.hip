@@ -129,9 +129,10 @@ bool conv_variant_takes(const ConvProblem &p, int variant) {
 
 // Configurations that the tuner leaves out.  None of them was the fastest in any share class over 3030 problems: the convolutions of
 // nine networks (Inception-v3, SqueezeNet, ResNet-18 / 50, RandWire, NASNet, VGG-16, AlexNet, the sample network) at batch 1 to 64 and
-// of multi-branch blocks on odd sizes, in each precision; nor, each pinned in turn, on 31 more from 8 -> 8 channels on 8 x 8 pixels to
-// 4096 -> 4096 on one and 700 -> 300 on 80 x 80.  (The fp32 matrix instructions lose to two terms of half from a few
-// microseconds on.)  They serve the closed-form choice, which knows none of the others, and the option that pins a configuration.
+// of multi-branch blocks on odd sizes, in each precision, with three bfloat16 terms where two of half are now.  Against the kernels of
+// now, each pinned in turn on 30 fp32 layers (K from 4 to 4608, those below 64 that the two-term kernels do not serve among them) at batch
+// 1, 16 and 64: the best of them takes 1.0 to 2.5 times the time of the best measured one, but for 60 -> 60 1 x 1 on 33 x 33 (5.6 against
+// 5.7 us at batch 16, 11.0 against 11.3 at 64) and 64 -> 16 on 55 x 55 at batch 16 (5.8 against 6.1).  They serve the closed-form choice, which knows none of the others, and the option that pins a configuration.
 static const char *const kNotMeasured[] = {
     "m64n64k32_w2x2x1_t32", "m128n128k16_w2x2x1_t32", "m32n32k64_w1x1x4_t32", "m64n32k32_w2x1x2_t32", "m32n64k32_w1x2x2_t32",
     "m128n64k16_w2x2x1_t32", "m64n16k64_w4x1x1_t16", "m32n16k64_w2x1x2_t16", "m16n16k128_w1x1x4_t16", "m64n128k16_w2x2x1_t32",

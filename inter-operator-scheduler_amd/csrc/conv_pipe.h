@@ -11,8 +11,8 @@
 // registers, the next one in LDS; one barrier per stage.  What a stage has to cover is the latency of its loads: with two terms one
 // or two units do (12 matrix instructions of 32 cycles per wavefront and unit at 64 x 64), with one term it takes four (a one-unit
 // stage is gone in 128 cycles).  Measured at batch 64 in fp32, three bfloat16 terms -> two terms of half: 288 -> 384 channels 3 x 3 stride 2 on
-// 35 x 35 222 -> 159 us (231 TFLOP/s, with 64 x 64 per wavefront, two units), 768 -> 192 on 17 x 17 44 -> 37 us, 192 -> 64 on 35 x 35
-// 22.7 -> 20.8 us (bound by its 110 MB).
+// 35 x 35 207 -> 149 us (247 TFLOP/s, with 64 x 64 per wavefront, two units), 768 -> 192 on 17 x 17 42 -> 34 us, 192 -> 64 on 35 x 35
+// 20.7 -> 18.5 us (bound by its 80 MB).
 #pragma once
 
 #include "conv_body.h"

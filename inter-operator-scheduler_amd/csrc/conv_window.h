@@ -10,9 +10,8 @@
 //
 // What is left per unit is matrix work, TNW LDS reads per plane and three address instructions per 32 pixels (two terms: four
 // more for the scaled filter operand).  Measured at batch 64, fp32 as three terms of bfloat16 (six products) -> two of half (three):
-// 80 -> 192 channels 3 x 3 on 73 x 73 484 -> 355 us (251 TFLOP/s, 750 of half products), 32 -> 64 on 147 x 147 360 -> 291 us, 32 -> 32 on
-// 149 x 149 232 -> 167 us, 48 -> 64 5 x 5 on 35 x 35 68 -> 47 us, 192 -> 192 1 x 7 on 17 x 17 56 -> 40 us; launched back to back, where the
-// clock settles lower than in a pass.  In bfloat16, tap by tap -> on the window, the same layers in a pass: 225 -> 182 us, 216 -> 206
+// 80 -> 192 channels 3 x 3 on 73 x 73 463 -> 306 us (308 TFLOP/s, 924 of half products), 32 -> 64 on 147 x 147 317 -> 233 us, 32 -> 32 on
+// 149 x 149 203 -> 155 us, 48 -> 64 5 x 5 on 35 x 35 66 -> 48 us, 192 -> 192 1 x 7 on 17 x 17 55 -> 36 us.  In bfloat16, tap by tap -> on the window, the same layers in a pass: 225 -> 182 us, 216 -> 206
 // (bound by 530 MB of activations), 158 -> 130.
 #pragma once
 

@@ -149,8 +149,8 @@ bool conv_matrix_path_supported(const ConvProblem &p);
 ConvLaunch conv_pick_launch(const ConvProblem &p, int num_cus, bool fusable_only = false, int precision = PREC_FP32);
 
 // Filter packing for a kernel configuration: w[OC][ICg][KH][KW] -> packed[g][k = (kh*KW + kw)*ICgP + c][OCgP]
-// (or [g][k / 4][OCgP][k % 4] for kquad configurations, planes of 16-bit values [g][k / 8][plane][OCgP][k % 8] for koct ones, with the
-// factors of the output channels behind two planes), ICgP = ICg rounded up to the configuration's channel
+// (or [g][k / 4][OCgP][k % 4] for kquad configurations, planes of 16-bit values [g][k / 8][plane][OCgP][k % 8] for koct ones, with two
+// words per output channel behind two planes: the factor that undoes its scale, and a bound for what its smallest filters are off by), ICgP = ICg rounded up to the configuration's channel
 // padding (zero rows), OCgP = OCg rounded up to 4.  16-bit configurations pack bfloat16 or half (round to nearest even), two
 // per float of the returned size.
 size_t conv_packed_floats(const ConvProblem &p, const ConvLaunch &l);

@@ -609,8 +609,8 @@ void Session::setup(bool pack_filters) {
     packed_.assign(plan_.convs.size(), 0);
     for (const PlanConv &conv : plan_.convs) {
         // A latency is measured without weights: filters with which the tensors neither grow from layer to layer nor with the sums
-        // between them (half of He's bound; the biases of +-1 keep them from vanishing).  With +-1 they grew past 2^26 within five layers,
-        // where the two-term kernels compute by plain multiply-adds: Inception-v3 at batch 1 was searched for 55 s instead of 8.
+        // between them (half of He's bound; the biases of +-1 keep them from vanishing).  With +-1 they grow past 2^26 within five layers and
+        // on to infinity, and sums of infinities are computed twice where two-term kernels meet them: no network's time.
         if (pack_filters)
             launch_fill_pattern(base_ + conv.weight_off, (size_t)conv.problem.OC * conv.problem.K(), 0x2468aceu, main, 0.5f * std::sqrt(6.f / (float)conv.problem.K()));
         // a convolution in front of the average pool it was exchanged with adds zeros; the pool adds the bias
