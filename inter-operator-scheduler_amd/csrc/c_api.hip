@@ -25,6 +25,13 @@ ios::LaunchChooser device_chooser() {
     return [&ctx](const ios::ConvProblem &p, int share) { return ctx.choose_launch(p, share); };
 }
 
+ios::BatchChooser device_batches() {
+    ios::DeviceContext &ctx = ios::DeviceContext::get();
+    return [&ctx](const std::vector<ios::ConvProblem> &problems, const std::vector<int> &share, bool remains) {
+        return ctx.choose_batch(problems, share, remains);
+    };
+}
+
 template <typename F>
 int guarded(F &&body) {
     std::lock_guard<std::recursive_mutex> lock(g_api_mutex);
@@ -47,7 +54,7 @@ int latency_call(ios::PlanMode mode, const char *doc_json, const char *extra_jso
         const ios::Json doc = ios::Json::parse(doc_json);
         ios::Json extra;
         if (extra_json != nullptr) extra = ios::Json::parse(extra_json);
-        ios::Plan plan = ios::build_plan(mode, doc, extra_json ? &extra : nullptr, batch_size, device_chooser());
+        ios::Plan plan = ios::build_plan(mode, doc, extra_json ? &extra : nullptr, batch_size, device_chooser(), ios::InputUse::Resident, device_batches());
         ios::Session session(std::move(plan), /*shared=*/true);
         if (mode == ios::PlanMode::Stage) {
             if (profile_stage_latency) throw std::runtime_error("stage_latency cannot profile stages (profile_stage_latency must be 0)");
@@ -88,7 +95,9 @@ int inference_call(ios::Session::Storage storage, const char *graph_json, int ba
             const bool tune = storage != ios::Session::Storage::Static;
             ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size,
                                              [&ctx, tune](const ios::ConvProblem &p, int share) { return ctx.choose_launch(p, share, tune); },
-                                             ios::InputUse::Once);
+                                             ios::InputUse::Once,
+                                             // (a batch holds outputs for longer: what fits the static scratch goes on fitting it)
+                                             tune ? device_batches() : nullptr);
             InferencePlan entry;
             entry.key = std::to_string((int)storage) + '/' + std::to_string(batch_size) + '/' + ctx.plan_token();   // (measuring changes it)
             entry.document = graph_json;
@@ -223,12 +232,21 @@ static ios::LaunchChooser host_chooser() {
     };
 }
 
+static ios::BatchChooser host_batches() {
+    if (!ios::planner_host_batches()) return nullptr;
+    return [](const std::vector<ios::ConvProblem> &, const std::vector<int> &, bool) {
+        int v = 0;
+        while (!ios::conv_variant_batches(v)) v++;
+        return v;
+    };
+}
+
 int ios_plan_describe(const char *graph_json, int batch_size, char *buf, int cap) {
     int needed = -1;
     guarded([&]() {
         const ios::Json doc = ios::Json::parse(graph_json);
         // host-only: the closed-form configuration model for a 256-CU device, no device is touched
-        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, host_chooser(), ios::InputUse::InParts);
+        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, host_chooser(), ios::InputUse::InParts, host_batches());
         const std::string text = ios::describe_plan(plan);
         needed = (int)text.size();
         if (buf != nullptr && cap > needed) memcpy(buf, text.c_str(), text.size() + 1);
@@ -240,7 +258,7 @@ long long ios_plan_arena_bytes(const char *graph_json, int batch_size) {
     long long bytes = -1;
     guarded([&]() {
         const ios::Json doc = ios::Json::parse(graph_json);
-        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, host_chooser(), ios::InputUse::InParts);
+        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, host_chooser(), ios::InputUse::InParts, host_batches());
         bytes = (long long)(plan.arena_floats * sizeof(float));
     });
     return bytes;
@@ -250,7 +268,7 @@ ios_session *ios_session_create(const char *graph_json, int batch_size) {
     SessionBox *box = nullptr;
     const int status = guarded([&]() {
         const ios::Json doc = ios::Json::parse(graph_json);
-        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, device_chooser(), ios::InputUse::InParts);
+        ios::Plan plan = ios::build_plan(ios::PlanMode::Graph, doc, nullptr, batch_size, device_chooser(), ios::InputUse::InParts, device_batches());
         box = new SessionBox();
         box->description = ios::describe_plan(plan);
         box->session.reset(new ios::Session(std::move(plan), /*shared=*/false));

@@ -4,6 +4,7 @@
 #include "launch_internal.h"
 
 #include <algorithm>
+#include <climits>
 #include <stdexcept>
 #include <string>
 
@@ -423,6 +424,56 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
     }
     hipLaunchKernelGGL(kernel, grid, dim3(d.threads), d.smem_bytes, stream, d.args);
     if (d.has_reduce) hipLaunchKernelGGL(splitk_reduce_kernel, dim3(d.reduce_blocks), dim3(256), 0, stream, d.reduce);
+}
+
+// ---- several convolutions in a launch ------------------------------------------------------
+bool conv_variant_batches(int variant) { return variant >= kFirstPipeVariant && variant < kFirstWindowVariant; }
+
+bool conv_batchable(const ConvProblem &a, const ConvProblem &b) {
+    return a.KH == 1 && a.KW == 1 && b.KH == 1 && b.KW == 1 && a.groups == 1 && b.groups == 1 && a.B == b.B && a.IC == b.IC && a.H == b.H && a.W == b.W &&
+           a.sh == b.sh && a.sw == b.sw && a.ph == b.ph && a.pw == b.pw;
+}
+
+void launch_conv_batch(const ConvBatchMember *members, int count, int variant, const TensorView &x, hipStream_t stream) {
+    if (count < 1 || count > kMaxConvBatch || !conv_variant_batches(variant)) throw std::runtime_error("conv: no such batch");
+    const VariantEntry &e = kVariants[variant];
+    ConvLaunch l;
+    l.variant = variant;
+    ConvBatchArgs b;
+    int tiles_m = 0, tiles_n = 0, threads = 0, smem_bytes = 0;
+    double filters = 0.0;
+    for (int i = 0; i < kMaxConvBatch; i++) {
+        const ConvBatchMember &m = members[std::min(i, count - 1)];
+        if (!conv_batchable(members[0].p, m.p)) throw std::runtime_error("conv: a batch of convolutions that do not fit each other");
+        const ConvDispatch d = make_conv_dispatch(m.p, l, x, m.packed, m.filters, m.bias, m.y, nullptr, SplitKReduce{});
+        b.item[i] = d.args;
+        b.item[i].xcd_q = b.item[i].xcd_r = b.item[i].weights_major = 0;
+        b.item[i].tile_div = d.args.tiles_m;
+        b.item[i].div_tile = make_fast_div((unsigned)d.args.tiles_m);
+        b.first[i] = i < count ? tiles_m : INT_MAX;
+        if (i >= count) continue;
+        tiles_m += d.args.tiles_m;
+        tiles_n = d.args.tiles_n;
+        threads = d.threads;
+        smem_bytes = d.smem_bytes;
+        filters += (double)m.p.OC * m.p.K();
+    }
+    const ConvProblem &p = members[0].p;
+    b.weights_major = filters > (double)p.B * p.IC * p.H * p.W ? 1 : 0;
+    b.tile_div = b.weights_major ? tiles_n : tiles_m;
+    b.div_tile = make_fast_div((unsigned)b.tile_div);
+    b.xcd_q = (tiles_m * tiles_n) >> 3;
+    b.xcd_r = (tiles_m * tiles_n) & 7;
+    const ConvBatchKernelFn kernel = kPipeBatchKernels[variant - kFirstPipeVariant];
+    if (smem_bytes > 64 * 1024) {
+        static bool raised[kNumConvVariants] = {};
+        if (!raised[variant]) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes) != hipSuccess)
+                throw std::runtime_error(std::string("conv: cannot reserve LDS for a batch on configuration ") + e.v.name);
+            raised[variant] = true;
+        }
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(threads), smem_bytes, stream, b);
 }
 
 // ---- filter packing ------------------------------------------------------------------------

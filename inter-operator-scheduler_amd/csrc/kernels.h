@@ -174,6 +174,18 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
                       const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce, hipStream_t stream,
                       const TensorView *residual = nullptr, bool post_relu = false);
 
+// Several convolutions of one input in a launch: they read the same view through the same window, without groups or a residual.
+// Every member has the packed filters, bias and output of its own.
+struct ConvBatchMember {
+    ConvProblem p;
+    const float *packed, *filters, *bias;
+    TensorView y;
+};
+constexpr int kMaxConvBatch = 4;
+bool conv_variant_batches(int variant);                              // there is a batched kernel on this configuration
+bool conv_batchable(const ConvProblem &a, const ConvProblem &b);     // two convolutions of one view may share a launch
+void launch_conv_batch(const ConvBatchMember *members, int count, int variant, const TensorView &x, hipStream_t stream);
+
 // Filters of a depth-wise convolution: w[C][1][KH][KW] -> packed[tap][C rounded up to 4] (padding zero).
 inline size_t dwconv_packed_floats(const ConvProblem &p) { return (size_t)p.KH * p.KW * ((p.OC + 3) & ~3); }
 void launch_pack_depthwise(const ConvProblem &p, const float *w, float *packed, hipStream_t stream);

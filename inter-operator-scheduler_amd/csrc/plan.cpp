@@ -79,7 +79,8 @@ int act_code(const std::string &name) {
 
 class Planner {
 public:
-    Planner(int batch, const LaunchChooser &chooser, InputUse input) : batch_(batch), input_use_(input), chooser_(chooser) {
+    Planner(int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches)
+        : batch_(batch), input_use_(input), chooser_(chooser), batch_chooser_(batches) {
         if (batch < 1) throw std::runtime_error("batch size must be positive");
         plan_.batch = batch;
     }
@@ -614,7 +615,10 @@ private:
         for (const auto &groups : plan_.stages) {
             if (groups.size() != 1 || covered > 1.2 * input / 57e9) break;
             bool plain = true;
-            for (int index : groups[0]) {
+            std::vector<int> here = groups[0];
+            for (const PlanBatch &batch : plan_.batches)
+                if (batch.stage == stages) here.insert(here.end(), batch.ops.begin(), batch.ops.end());
+            for (int index : here) {
                 const PlanOp &op = plan_.ops[index];
                 plain = plain && op.srcs.empty() && !op.has_residual && op.bias_conv < 0 &&
                         (op.kind == OpKind::ConvMfma || op.kind == OpKind::ConvDirect || op.kind == OpKind::Pool);
@@ -1131,18 +1135,8 @@ private:
         plan_.output_single_group = stage_names.back().size() == 1;
     }
 
-    void finish() {
-        for (size_t i = 0; i < nodes_.size(); i++) {
-            const PNode &n = nodes_[i];
-            if (n.pre_relu_alias || n.no_storage || n.residual_into >= 0) continue;   // never materialised
-            plan_.tensors[n.name] = view_of(static_cast<int>(i));
-        }
-        plan_.input = view_of(0);
-        // the result is the last operator of the last stage's last group
-        const auto &last_stage_units = unit_result_;
-        int out_node = last_stage_units.back();
-        plan_.output = view_of(out_node);
-        plan_.output_name = nodes_[out_node].name;
+    // per convolution: the operators that run beside it, itself among them
+    std::vector<int> shares() const {
         std::vector<int> share(plan_.convs.size(), 1);
         // a convolution shares the device with the operators at the same position of the other groups of its stage
         // (the fused executor runs position after position); in a multi-group stage it counts at least two, because
@@ -1156,6 +1150,79 @@ private:
                     for (const auto &other : stage) busy += other.size() > pos ? 1 : 0;
                     share[op.conv] = stage.size() > 1 ? std::max(2, busy) : 1;
                 }
+        return share;
+    }
+
+    // Convolutions of one view through the same window (the 1 x 1 convolutions at the head of the branches of a block) may share a
+    // launch, whichever branches, groups or stages they lie in: from the stage on before which the view is complete, the first of
+    // them takes the others along.  A staged kernel at these sizes waits for its loads and barriers, with one or two blocks on a
+    // compute unit; the blocks of a batch fill them up, and read the input tile that their neighbours on the XCD read.  Measured, four
+    // branches, each on its fastest kernel -> together: 768 channels on 17 x 17 at batch 64 fp32 133 -> 99 us, bfloat16 77 -> 52, at batch 7 half
+    // 27 -> 12; 2048 on 8 x 8 at batch 64 151 -> 97, bfloat16 94 -> 47; 192 on 35 x 35 at batch 16 30 -> 19.
+    void find_batches() {
+        const std::vector<int> share = shares();
+        std::map<std::vector<long long>, std::vector<int>> readers;   // operations by view and window
+        for (size_t i = 0; i < plan_.ops.size(); i++) {
+            const PlanOp &op = plan_.ops[i];
+            if (op.kind != OpKind::ConvMfma || op.has_residual || !plan_.convs[op.conv].matrix_path) continue;
+            const ConvProblem &p = plan_.convs[op.conv].problem;
+            if (!conv_batchable(p, p)) continue;
+            readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W, p.sh, p.sw, p.ph, p.pw}].push_back((int)i);
+        }
+        for (auto &entry : readers) {
+            std::vector<int> &ops = entry.second;
+            if (ops.size() < 2) continue;
+            const ViewRef in = plan_.ops[ops[0]].in;
+            int ready = -1;   // the last stage that writes into the view
+            for (const PlanOp &op : plan_.ops)
+                if (op.out.base == in.base && op.out.first < in.first + in.C && in.first < op.out.first + op.out.C) ready = std::max(ready, op.stage);
+            ops.erase(std::remove_if(ops.begin(), ops.end(), [&](int i) { return plan_.ops[i].stage <= ready; }), ops.end());
+            std::stable_sort(ops.begin(), ops.end(), [&](int a, int b) { return plan_.ops[a].stage < plan_.ops[b].stage; });
+            for (size_t first = 0; first + 1 < ops.size(); first += kMaxConvBatch) {
+                const size_t last = std::min(ops.size(), first + kMaxConvBatch);
+                PlanBatch batch;
+                batch.ops.assign(ops.begin() + first, ops.begin() + last);
+                batch.stage = plan_.ops[batch.ops[0]].stage;
+                std::vector<ConvProblem> problems;
+                std::vector<int> their_share;
+                bool remains = false;
+                for (int i : batch.ops) {
+                    problems.push_back(plan_.convs[plan_.ops[i].conv].problem);
+                    their_share.push_back(share[plan_.ops[i].conv]);
+                    if (plan_.stages[plan_.ops[i].stage].size() == 1) continue;
+                    for (const auto &group : plan_.stages[plan_.ops[i].stage])   // (what runs at the beginning of their stages)
+                        remains = remains || (!group.empty() && std::find(batch.ops.begin(), batch.ops.end(), group[0]) == batch.ops.end());
+                }
+                batch.variant = batch_chooser_(problems, their_share, remains);
+                if (batch.variant < 0) continue;
+                for (int i : batch.ops) {
+                    PlanOp &op = plan_.ops[i];
+                    auto &group = plan_.stages[op.stage][op.group];
+                    group.erase(std::find(group.begin(), group.end(), i));
+                    op.stage = batch.stage;
+                    op.batch = (int)plan_.batches.size();
+                    PlanConv &conv = plan_.convs[op.conv];
+                    conv.launch.variant = batch.variant;
+                    conv.launch.split_k = 1;
+                    batched_.insert(op.conv);
+                }
+                plan_.batches.push_back(batch);
+            }
+        }
+    }
+
+    void finish() {
+        for (size_t i = 0; i < nodes_.size(); i++) {
+            const PNode &n = nodes_[i];
+            if (n.pre_relu_alias || n.no_storage || n.residual_into >= 0) continue;   // never materialised
+            plan_.tensors[n.name] = view_of(static_cast<int>(i));
+        }
+        plan_.input = view_of(0);
+        // the result is the last operator of the last stage's last group
+        const auto &last_stage_units = unit_result_;
+        int out_node = last_stage_units.back();
+        plan_.output = view_of(out_node);
+        plan_.output_name = nodes_[out_node].name;
         for (PlanOp &op : plan_.ops) {
             if (op.conv < 0 || !plan_.convs[op.conv].thin) continue;
             PlanConv &conv = plan_.convs[op.conv];
@@ -1166,11 +1233,13 @@ private:
                 conv.thin = false;
             }
         }
+        if (batch_chooser_ && planner_batch_convs()) find_batches();
+        const std::vector<int> share = shares();
         for (size_t i = 0; i < plan_.convs.size(); i++) {
             PlanConv &conv = plan_.convs[i];
             if (conv.problem.is_depthwise()) conv.packed_off = reserve(dwconv_packed_floats(conv.problem));
             if (!conv.matrix_path) continue;
-            conv.launch = chooser_(conv.problem, share[i]);
+            if (!batched_.count((int)i)) conv.launch = chooser_(conv.problem, share[i]);
             conv.packed_off = reserve(conv_packed_floats(conv.problem, conv.launch));
             conv.ws_floats = conv_workspace_floats(conv.problem, conv.launch);
             if (conv.ws_floats > 0) conv.ws_off = reserve_region(conv.ws_floats);
@@ -1184,6 +1253,7 @@ private:
     InputUse input_use_;
     int level_unit_ = -2, level_base_ = 0, level_top_ = 0;   // PlanOp::level of the operations being emitted
     const LaunchChooser &chooser_;
+    const BatchChooser &batch_chooser_;
     Plan plan_;
     std::vector<PNode> nodes_;
     std::map<std::string, int> by_name_;
@@ -1196,6 +1266,7 @@ private:
     std::vector<int> groups_in_stage_;
     struct SeqRange { int first, second; };
     std::vector<SeqRange> sequentials_;
+    std::set<int> batched_;   // convolutions that share a launch
     std::vector<Region> regions_;   // ascending virtual offsets
     size_t region_floats_ = 0;
     std::map<int, ViewRef> commuted_z_;   // commuted pool node -> the temporary between the convolution and the pool
@@ -1218,6 +1289,7 @@ bool g_arena_reuse = true;
 long long g_thin_conv_min_pixels = 1LL << 18;
 int g_host_split_k = 0;
 bool g_commute_pool_conv = true;
+bool g_batch_convs = true, g_host_batches = false;
 }
 
 bool set_planner_option(const std::string &key, const std::string &value) {
@@ -1227,6 +1299,14 @@ bool set_planner_option(const std::string &key, const std::string &value) {
     }
     if (key == "commute_pool_conv") {
         g_commute_pool_conv = !(value == "0" || value == "false" || value == "off" || value.empty());
+        return true;
+    }
+    if (key == "batch_convs") {
+        g_batch_convs = !(value == "0" || value == "false" || value == "off" || value.empty());
+        return true;
+    }
+    if (key == "host_plan_batches") {   // plans made without a device put every convolution that may share a launch into one
+        g_host_batches = !(value == "0" || value == "false" || value == "off" || value.empty());
         return true;
     }
     if (key == "thin_conv_min_pixels") {
@@ -1245,10 +1325,12 @@ bool set_planner_option(const std::string &key, const std::string &value) {
 bool planner_arena_reuse() { return g_arena_reuse; }
 long long planner_thin_conv_min_pixels() { return g_thin_conv_min_pixels; }
 int planner_host_split_k() { return g_host_split_k; }
+bool planner_batch_convs() { return g_batch_convs; }
+bool planner_host_batches() { return g_host_batches; }
 bool planner_commute_pool_conv() { return g_commute_pool_conv; }
 
-Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input) {
-    Planner planner(batch, chooser, mode == PlanMode::Graph ? input : InputUse::Resident);
+Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches) {
+    Planner planner(batch, chooser, mode == PlanMode::Graph ? input : InputUse::Resident, batches);
     return planner.run(mode, doc, extra);
 }
 
@@ -1283,6 +1365,7 @@ std::string describe_plan(const Plan &plan) {
         if (op.bias_conv >= 0) os << ",\"adds_bias_of\":\"" << plan.convs[op.bias_conv].name << "\",\"act\":" << op.act;
         if (op.conv >= 0 && plan.convs[op.conv].linear) os << ",\"linear\":true";
         if (op.has_residual) os << ",\"residual\":true,\"post_relu\":" << op.post_relu;
+        if (op.batch >= 0) os << ",\"batch\":" << op.batch;
         os << ",\"level\":" << op.level;
         // arena extents in floats, one [begin, end) per image: what the operation writes and what it reads
         auto ranges = [&](const char *key, const std::vector<ViewRef> &views) {

@@ -91,14 +91,24 @@ struct PlanOp {
     // of the whole batch, or one that holds a part at a time.
     ViewRef part_in, part_out;
     bool part_in_whole = true, part_out_whole = true;
+    int batch = -1;       // index into Plan::batches
     double flops = 0.0, bytes = 0.0;
+};
+
+// Convolutions of one view through the same window that share a launch (launch_conv_batch).  They run at the beginning of their
+// stage, before its groups: an operation that the schedule puts into a later stage moves here.
+struct PlanBatch {
+    int stage = 0;
+    int variant = -1;
+    std::vector<int> ops;
 };
 
 struct Plan {
     int batch = 1;
     std::vector<PlanOp> ops;
     std::vector<PlanConv> convs;
-    std::vector<std::vector<std::vector<int>>> stages;   // stage -> group -> op indices in launch order
+    std::vector<std::vector<std::vector<int>>> stages;   // stage -> group -> op indices in launch order (without those of batches)
+    std::vector<PlanBatch> batches;                      // by stage
     std::vector<std::string> unit_names;
     std::map<std::string, ViewRef> tensors;              // operator name -> materialised output view
     std::map<std::string, int> conv_index;               // convolution name -> index into convs
@@ -134,10 +144,15 @@ enum class InputUse { Resident, InParts, Once };
 // share - 1 others should occupy about 1 / share of it rather than all of it.
 typedef std::function<ConvLaunch(const ConvProblem &, int share)> LaunchChooser;
 
+// Kernel configuration on which convolutions of one input run in a launch of their own, or -1 where they are faster by themselves;
+// `share` of each as above.  `remains`: other operations of their stage lose the launch that they shared with them.
+typedef std::function<int(const std::vector<ConvProblem> &, const std::vector<int> &share, bool remains)> BatchChooser;
+
 // Compile a document.  `extra` is the input-shape document of stage mode ({name: [C, H, W]}).
 // Throws std::runtime_error on malformed documents, unknown operator types, non-topological schedules
 // and stages with too many groups.
-Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input = InputUse::Resident);
+Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input = InputUse::Resident,
+                const BatchChooser &batches = nullptr);
 
 std::string describe_plan(const Plan &plan);   // JSON array, one object per op
 
@@ -149,6 +164,8 @@ bool set_planner_option(const std::string &key, const std::string &value);
 bool planner_arena_reuse();
 long long planner_thin_conv_min_pixels();
 int planner_host_split_k();   // option host_plan_split_k
+bool planner_batch_convs();     // option batch_convs (default 1)
+bool planner_host_batches();    // option host_plan_batches
 bool planner_commute_pool_conv();   // option commute_pool_conv (default 1): see PlanConv::linear
 
 }  // namespace ios

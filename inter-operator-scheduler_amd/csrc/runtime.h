@@ -68,7 +68,7 @@ public:
     int forced_split_k() const { return forced_split_k_; }
     std::string info_json() const;
     // changes with everything but the options that the choice of kernel configurations depends on
-    std::string plan_token() const { return std::to_string(tuned.size()) + (xcd_usable_ ? "x" : "-"); }
+    std::string plan_token() const { return std::to_string(tuned.size()) + '/' + std::to_string(batched.size()) + (xcd_usable_ ? "x" : "-"); }
 
     // Kernel configuration for a matrix-path convolution: the measured best when autotuning is on (cached
     // per problem signature for the life of the process, and in the file named by IOS_TUNE_CACHE when set),
@@ -77,6 +77,10 @@ public:
     // allow_tuning = false never measures (measuring allocates scratch tensors): a shape that has no cached winner
     // gets the closed-form choice.
     ConvLaunch choose_launch(const ConvProblem &p, int share, bool allow_tuning = true);
+
+    // Kernel configuration on which these convolutions of one input share a launch, or -1 where the measurement finds them faster by
+    // themselves (as choose_launch has them); see BatchChooser.  Without autotuning there are no batches, but on a forced configuration.
+    int choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains);
 
     // Static device scratch of the entry point that allocates nothing: address on device 0 (resolved once, when the
     // context is created) and size in bytes.
@@ -87,8 +91,10 @@ public:
         ConvLaunch best[kShareClasses];
     };
     std::map<std::string, TunedConv> tuned;
+    std::map<std::string, int> batched;   // choose_batch by its arguments
 
 private:
+    int tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains);
     DeviceContext();
     TunedConv tune_conv(const ConvProblem &p);
     float *tuning_buffer(int which, size_t floats);
@@ -169,6 +175,7 @@ public:
         std::vector<int> ops;    // indices into plan().ops
         int blocks = 0, threads = 0;
         int fused_level = -1;    // index into the stage's fused launches, -1 for a stand-alone kernel
+        int batch = -1;          // index into plan().batches
     };
     std::vector<LaunchRecord> launches();
     std::string describe_launches();   // JSON array with the algorithmic flops and bytes of every launch
@@ -183,6 +190,9 @@ private:
     void ensure_fork_events();
     // on stream `group` of the pool; images > 0: on that many images of the batch from `first` on
     void launch_op(const PlanOp &op, int group, int first = 0, int images = 0);
+    TensorView part_of(const ViewRef &whole_view, const ViewRef &part_view, bool whole, int first, int images) const;
+    void launch_batch(const PlanBatch &batch, int first = 0, int images = 0);   // on the main stream
+    void launch_batches(size_t stage, int first = 0, int images = 0);           // those at the beginning of a stage
     unsigned *counters_of(const PlanConv &c) const;
     const float *bias_of(const PlanConv &c) const { return base_ + (c.linear ? c.zero_bias_off : c.bias_off); }
     void ready_executor();

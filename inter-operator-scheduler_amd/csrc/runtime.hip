@@ -130,6 +130,7 @@ void DeviceContext::check_xcd_fault() {
     *xcd_fault_ = 0;
     xcd_usable_ = false;
     tuned.clear();
+    batched.clear();
     throw std::runtime_error("a split-K convolution found a workgroup on another XCD than the round-robin placement it relies on: results since the "
                              "last synchronisation may be wrong.  The XCD-local form is switched off for the rest of this process; create the session again");
 }
@@ -158,6 +159,18 @@ void DeviceContext::load_tune_cache() {
     // does not parse (truncated write, a configuration name this build no longer has) is skipped: its shape is measured again.
     char line[1024];
     while (fgets(line, sizeof(line), f) != nullptr) {
+        // or "batch", the arguments of choose_batch and a configuration name or "none", with tabs between them
+        if (strncmp(line, "batch\t", 6) == 0) {
+            const std::string text(line + 6, strcspn(line + 6, "\n"));
+            const size_t tab = text.find('\t');
+            if (tab == std::string::npos) continue;
+            const std::string name = text.substr(tab + 1);
+            int variant = name == "none" ? -1 : -2;
+            for (int i = 0; i < conv_num_variants(); i++)
+                if (name == conv_variant(i).name && conv_variant_batches(i)) variant = i;
+            if (variant >= -1) batched[text.substr(0, tab)] = variant;   // (whether it serves the shapes is seen when it is asked for)
+            continue;
+        }
         std::istringstream in(line);
         int v[12];
         bool ok = true;
@@ -434,6 +447,162 @@ ConvLaunch DeviceContext::choose_launch(const ConvProblem &p, int share, bool al
     return launch;
 }
 
+static WorkItem conv_work_item(const ConvDispatch &d) {
+    WorkItem item;
+    memset(&item, 0, sizeof(WorkItem));
+    item.kind = WORK_CONV;
+    item.variant = d.variant;
+    item.threads = d.threads;
+    item.tiles = d.tiles;
+    item.groups = d.groups;
+    item.div_tiles = make_fast_div((unsigned)d.tiles);
+    item.div_groups = make_fast_div((unsigned)d.groups);
+    item.num_blocks = d.grid_blocks();
+    item.conv = d.args;
+    return item;
+}
+
+// Both ways on scratch tensors of the real shapes: every convolution as it runs without a batch (beside the others where one of them
+// shares its stage), and all of them in a launch on every configuration that has such a kernel.
+int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains) {
+    const ConvProblem &p = problems[0];
+    const size_t count = problems.size();
+    bool parallel = false;
+    for (int s : share) parallel = parallel || s > 1;
+    std::vector<ConvLaunch> alone;
+    for (size_t i = 0; i < count; i++) alone.push_back(choose_launch(problems[i], share[i]));
+    TensorView x;
+    x.C = p.IC; x.H = p.H; x.W = p.W; x.pstride = padded_channels(p.IC);
+    x.ptr = tuning_buffer(0, (size_t)p.B * p.H * p.W * x.pstride + 64);
+    std::vector<TensorView> y(count);
+    std::vector<size_t> y_at(count), packed_at(count), filters_at(count), ws_at(count), ctr_at(count);
+    size_t y_floats = 0, floats = 0, ws_floats = 0, counters = 0, items_at = 0;
+    for (size_t i = 0; i < count; i++) {
+        const ConvProblem &q = problems[i];
+        y[i].C = q.OC; y[i].H = q.OH; y[i].W = q.OW; y[i].pstride = padded_channels(q.OC);
+        y_at[i] = y_floats;
+        y_floats += ((size_t)q.B * q.OH * q.OW * y[i].pstride + 63) & ~size_t(63);
+        packed_at[i] = floats;
+        floats += (conv_packed_floats_max(q) + 63) & ~size_t(63);
+        filters_at[i] = floats;   // (the first of them serve as its bias)
+        floats += ((size_t)q.OC * q.K() + 63) & ~size_t(63);
+        ws_at[i] = ws_floats;
+        ws_floats += conv_workspace_floats(q, alone[i]);
+        ctr_at[i] = counters;
+        counters += conv_counter_count(q, alone[i]);
+    }
+    items_at = floats;
+    floats += (count * sizeof(WorkItem) + sizeof(float) - 1) / sizeof(float);
+    float *y_memory = tuning_buffer(1, y_floats), *memory = tuning_buffer(2, floats), *workspace = ws_floats ? tuning_buffer(3, ws_floats) : nullptr;
+    unsigned *tickets = tuning_counters(counters);
+    hipStream_t stream = streams_[0];
+    launch_fill_pattern(memory, items_at, 0x51f15e, stream, 0.5f);
+    for (size_t i = 0; i < count; i++) y[i].ptr = y_memory + y_at[i];
+    struct EventPair {   // destroyed on every way out, a failing launch included
+        hipEvent_t start = nullptr, stop = nullptr;
+        ~EventPair() {
+            if (start != nullptr) (void)hipEventDestroy(start);
+            if (stop != nullptr) (void)hipEventDestroy(stop);
+        }
+    } events;
+    IOS_HIP(hipEventCreate(&events.start));
+    IOS_HIP(hipEventCreate(&events.stop));
+    auto measure = [&](int reps, int launches, const std::function<void()> &issue) {
+        issue();
+        launch_delay(reps * launches + 3, stream);   // (as in tune_conv: the events time the kernels and not the host)
+        IOS_HIP(hipEventRecord(events.start, stream));
+        for (int r = 0; r < reps; r++) issue();
+        IOS_HIP(hipEventRecord(events.stop, stream));
+        IOS_HIP(hipEventSynchronize(events.stop));
+        float ms = 0.f;
+        IOS_HIP(hipEventElapsedTime(&ms, events.start, events.stop));
+        return ms / reps;
+    };
+    constexpr int kReps = 8;
+    // by themselves
+    std::vector<WorkItem> items;
+    FusedHeader header{};
+    int blocks = 0, smem_bytes = 0, threads = 256;
+    std::vector<size_t> single;
+    bool wide = false;
+    for (size_t i = 0; i < count; i++) {
+        launch_pack_filters(problems[i], alone[i], memory + filters_at[i], memory + packed_at[i], stream);
+        const ConvDispatch d = make_conv_dispatch(problems[i], alone[i], x, memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
+                                                  workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr));
+        if (!parallel || !fused_executor() || !conv_variant(d.variant).fusable() || d.has_reduce) {
+            single.push_back(i);
+            continue;
+        }
+        WorkItem item = conv_work_item(d);
+        item.first_block = blocks;
+        header.first_block[items.size()] = blocks;
+        blocks += item.num_blocks;
+        smem_bytes = std::max(smem_bytes, d.smem_bytes);
+        threads = std::max(threads, d.threads);
+        wide = wide || conv_variant(d.variant).needs_wide();
+        items.push_back(item);
+    }
+    if (wide && threads > 512) return -1;   // (a level of such operators is not one launch: see build_fused)
+    header.num_items = (int)items.size();
+    WorkItem *device_items = reinterpret_cast<WorkItem *>(memory + items_at);
+    if (!items.empty()) stage_.upload(device_items, items.data(), items.size() * sizeof(WorkItem), stream);
+    const float apart = measure(kReps, (int)single.size() + 1, [&] {
+        if (!items.empty()) launch_fused(threads, device_items, items.data(), header, blocks, smem_bytes, num_cus_, stream);
+        for (size_t i : single)
+            launch_conv_mfma(problems[i], alone[i], x, memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
+                             workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr), stream);
+    });
+    // together
+    float best = 1e30f;
+    int variant = -1;
+    std::vector<ConvBatchMember> members(count);
+    for (size_t i = 0; i < count; i++) members[i] = {problems[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i]};
+    bool packed = false;
+    for (int v = 0; v < conv_num_variants(); v++) {
+        if (!conv_variant_batches(v) || conv_variant(v).precision != precision_) continue;
+        bool precise = true;
+        for (const ConvProblem &q : problems) precise = precise && conv_variant_precise(q, v);
+        if (!precise) continue;
+        ConvLaunch l;
+        l.variant = v;
+        for (size_t i = 0; i < count && !packed; i++) launch_pack_filters(problems[i], l, memory + filters_at[i], memory + packed_at[i], stream);
+        packed = true;   // (they all read the same layout)
+        const float ms = measure(kReps, 1, [&] { launch_conv_batch(members.data(), (int)count, v, x, stream); });
+        if (ms < best) {
+            best = ms;
+            variant = v;
+        }
+    }
+    // What is left of a stage takes a launch of its own: 3 us.  A gain within the noise of the measurement is none.
+    constexpr float kLaunchMs = 0.003f, kNoise = 0.97f;
+    return best + (remains ? kLaunchMs : 0.f) < kNoise * apart ? variant : -1;
+}
+
+int DeviceContext::choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains) {
+    if (forced_variant_ >= 0) return forced_split_k_ <= 1 && conv_variant_batches(forced_variant_) ? forced_variant_ : -1;
+    if (!autotune_ || forced_split_k_ > 0) return -1;
+    std::string key = settings_token() + (precision_ == PREC_BF16 ? " bf16" : precision_ == PREC_FP16 ? " fp16" : "") + (remains ? " remains" : "");
+    for (size_t i = 0; i < problems.size(); i++) key += " | " + conv_signature(problems[i]) + " " + std::to_string(share[i]);
+    auto it = batched.find(key);
+    if (it != batched.end() && it->second >= 0) {   // (a saved choice that would not be measured here: written by a build that had other kernels)
+        bool serves = conv_variant(it->second).precision == precision_;
+        for (const ConvProblem &p : problems) serves = serves && conv_variant_precise(p, it->second);
+        if (!serves) {
+            batched.erase(it);
+            it = batched.end();
+        }
+    }
+    if (it == batched.end()) {
+        it = batched.emplace(key, tune_batch(problems, share, remains)).first;
+        FILE *f = tune_cache_path_.empty() ? nullptr : fopen(tune_cache_path_.c_str(), "a");
+        if (f != nullptr) {
+            fprintf(f, "batch\t%s\t%s\n", key.c_str(), it->second >= 0 ? conv_variant(it->second).name : "none");
+            fclose(f);
+        }
+    }
+    return it->second;
+}
+
 float *DeviceContext::shared_arena(size_t floats) {
     if (floats > arena_floats_) {
         IOS_HIP(hipDeviceSynchronize());
@@ -507,6 +676,7 @@ void DeviceContext::set_option(const std::string &key, const std::string &value)
         stage_.give_back();
     } else if (key == "clear_tuning") {
         tuned.clear();
+        batched.clear();
     } else {
         throw std::runtime_error("unknown option '" + key + "'");
     }
@@ -756,16 +926,42 @@ unsigned *Session::counters_of(const PlanConv &c) const {
     return reinterpret_cast<unsigned *>(base_ + c.ctr_off);
 }
 
+// the images that a launch works on
+TensorView Session::part_of(const ViewRef &whole_view, const ViewRef &part_view, bool whole, int first, int images) const {
+    if (images <= 0) return tv(whole_view);
+    TensorView t = tv(part_view);
+    if (whole) t.ptr += (long long)first * t.H * t.W * t.pstride;
+    return t;
+}
+
+void Session::launch_batch(const PlanBatch &batch, int first, int images) {
+    ConvBatchMember members[kMaxConvBatch];
+    TensorView in;
+    int count = 0;
+    for (int index : batch.ops) {
+        const PlanOp &op = plan_.ops[index];
+        const PlanConv &c = plan_.convs[op.conv];
+        ConvBatchMember &m = members[count++];
+        m.p = c.problem;
+        if (images > 0) m.p.B = images;
+        m.packed = base_ + c.packed_off;
+        m.filters = base_ + c.weight_off;
+        m.bias = bias_of(c);
+        m.y = part_of(op.out, op.part_out, op.part_out_whole, first, images);
+        in = part_of(op.in, op.part_in, op.part_in_whole, first, images);
+    }
+    launch_conv_batch(members, count, batch.variant, in, ctx_.stream(0));
+}
+
+void Session::launch_batches(size_t stage, int first, int images) {
+    for (const PlanBatch &batch : plan_.batches)
+        if (batch.stage == (int)stage) launch_batch(batch, first, images);
+}
+
 void Session::launch_op(const PlanOp &op, int group, int first, int images) {
     hipStream_t stream = ctx_.stream(group);
     const int count = images > 0 ? images : plan_.batch;
-    auto part = [&](const ViewRef &whole_view, const ViewRef &part_view, bool whole) {   // the images this launch works on
-        if (images <= 0) return tv(whole_view);
-        TensorView t = tv(part_view);
-        if (whole) t.ptr += (long long)first * t.H * t.W * t.pstride;
-        return t;
-    };
-    const TensorView in = part(op.in, op.part_in, op.part_in_whole), out = part(op.out, op.part_out, op.part_out_whole);
+    const TensorView in = part_of(op.in, op.part_in, op.part_in_whole, first, images), out = part_of(op.out, op.part_out, op.part_out_whole, first, images);
     switch (op.kind) {
         case OpKind::ConvMfma: {
             const PlanConv &c = plan_.convs[op.conv];
@@ -841,6 +1037,7 @@ void Session::enqueue_stage_serial(size_t s) {
 }
 
 void Session::enqueue_stage(size_t s) {
+    launch_batches(s);
     if (static_) enqueue_stage_serial(s);
     else if (ctx_.fused_executor()) enqueue_stage_fused(s);
     else enqueue_stage_streams(s);
@@ -878,8 +1075,10 @@ void Session::enqueue_prefix(size_t stages) {
     for (size_t part = 0; part < arriving_.size(); part++) {
         const int images = arriving_[part] - begin;
         take_images(begin, images, (int)part);
-        for (size_t s = 0; s < split; s++)
+        for (size_t s = 0; s < split; s++) {
+            launch_batches(s, begin, images);
             for (int op : plan_.stages[s][0]) launch_op(plan_.ops[op], 0, begin, images);
+        }
         begin = arriving_[part];
     }
     arriving_.clear();
@@ -951,14 +1150,7 @@ void Session::build_fused() {
                             throw std::runtime_error(op.has_residual ? std::string("internal: a residual convolution is planned for single-group stages only")
                                                                      : std::string("convolution kernel configuration ") + conv_variant(d.variant).name +
                                                                            " cannot run inside a fused stage launch");
-                        pend.item.kind = WORK_CONV;
-                        pend.item.variant = d.variant;
-                        pend.item.tiles = d.tiles;
-                        pend.item.groups = d.groups;
-                        pend.item.div_tiles = make_fast_div((unsigned)d.tiles);
-                        pend.item.div_groups = make_fast_div((unsigned)d.groups);
-                        pend.item.num_blocks = d.grid_blocks();
-                        pend.item.conv = d.args;
+                        pend.item = conv_work_item(d);
                         pend.threads = d.threads;
                         pend.smem_bytes = d.smem_bytes;
                         if (d.has_reduce && solo) pend.fusable = false;   // launched stand-alone, reduction included
@@ -1104,9 +1296,10 @@ void Session::enqueue_stage_fused(size_t s) {
 size_t Session::direct_stages() const {
     constexpr size_t kAhead = 4, kNoGraph = 8;
     auto launches_of = [&](size_t s) {
-        size_t ops = 0;
+        size_t ops = 0, batches = 0;
         for (const auto &group : plan_.stages[s]) ops += group.size();
-        return ctx_.fused_executor() && !fused_stages_[s].empty() ? fused_stages_[s].size() : ops;
+        for (const PlanBatch &batch : plan_.batches) batches += batch.stage == (int)s ? 1 : 0;
+        return batches + (ctx_.fused_executor() && !fused_stages_[s].empty() ? fused_stages_[s].size() : ops);
     };
     size_t total = 0, ahead = 0, stages = 0;
     for (size_t s = 0; s < plan_.stages.size(); s++) total += launches_of(s);
@@ -1218,6 +1411,10 @@ void Session::infer(const float *input, int count, char **names, float **weights
 // issues the stages whose filters are packed
 void Session::advance() {
     for (; next_stage_ < plan_.stages.size(); next_stage_++) {
+        for (const PlanBatch &batch : plan_.batches)
+            if (batch.stage == (int)next_stage_)
+                for (int op : batch.ops)
+                    if (!packed_[plan_.ops[op].conv]) return;
         for (const auto &group : plan_.stages[next_stage_])
             for (int op : group)
                 if (plan_.ops[op].conv >= 0 && !packed_[plan_.ops[op].conv]) return;
@@ -1356,6 +1553,15 @@ std::vector<Session::LaunchRecord> Session::launches() {
     std::vector<LaunchRecord> out;
     for (size_t s = 0; s < plan_.stages.size(); s++) {
         const auto &groups = plan_.stages[s];
+        for (size_t b = 0; b < plan_.batches.size(); b++) {
+            if (plan_.batches[b].stage != (int)s) continue;
+            LaunchRecord r;
+            r.stage = (int)s;
+            r.kernel = std::string("conv_batch_kernel<") + conv_variant(plan_.batches[b].variant).name + ">";
+            r.ops = plan_.batches[b].ops;
+            r.batch = (int)b;
+            out.push_back(r);
+        }
         if (fused && !fused_stages_[s].empty()) {
             for (size_t l = 0; l < fused_stages_[s].size(); l++) {
                 const FusedLaunch &f = fused_stages_[s][l];
@@ -1427,7 +1633,9 @@ void Session::profile_launches(int warmup, int repeat, float *ms_out, int capaci
     for (size_t i = 0; i < list.size(); i++) {
         const LaunchRecord &r = list[i];
         auto issue = [&]() {
-            if (r.fused_level >= 0) {
+            if (r.batch >= 0) {
+                launch_batch(plan_.batches[r.batch]);
+            } else if (r.fused_level >= 0) {
                 const FusedLaunch &l = fused_stages_[r.stage][r.fused_level];
                 launch_fused(l.threads, items + l.first_item, fused_items_host_.data() + l.first_item, l.header, l.total_blocks, l.smem_bytes, ctx_.num_cus(), main);
             } else {
