@@ -771,6 +771,7 @@ __device__ __forceinline__ void split_bf16x3(const float (&x)[8], uintx4 &hi, ui
 // largest of eight neighbouring channels is in it, the others are off by 2^-21 of that one at most.)
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 constexpr float kInputLift = 256.f, kFilterLift = 16.f, kFilterFloor = 0x1p-7f;
 constexpr unsigned kWindow = 26u << 23;   // binades from the limit of the inputs down to 2^-11 scaled, in bits of a float
 // An input below the window is off by 2^-33, its upper term times 2^-4 by 2^-21 against a lower one of 2^-11 of its filter, and the product of
@@ -794,14 +795,16 @@ __device__ __forceinline__ float octet_peak(const float (&x)[8]) {
     asm("" : "+v"(peak));
     return peak;
 }
+// of two magnitudes that are numbers (they compare as integers; a maximum of floats is preceded by one of each for signalling NaN)
+__device__ __forceinline__ float larger(float a, float b) { return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b))); }
 // over the lanes of a wavefront that hold the octets of a pixel in the operand layout (lanes equal modulo MT)
 template <int MT>
 __device__ __forceinline__ float pixel_peak(float peak) {
     uintx2 s = __builtin_bit_cast(uintx2, __builtin_amdgcn_permlane32_swap(__float_as_uint(peak), __float_as_uint(peak), false, false));
-    peak = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+    peak = larger(__uint_as_float(s.x), __uint_as_float(s.y));
     if constexpr (MT == 16) {
         s = __builtin_bit_cast(uintx2, __builtin_amdgcn_permlane16_swap(__float_as_uint(peak), __float_as_uint(peak), false, false));
-        peak = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+        peak = larger(__uint_as_float(s.x), __uint_as_float(s.y));
     }
     return peak;
 }
@@ -818,7 +821,7 @@ struct InputWatch {
     float peak = 0.f;
     unsigned below = 0;
     __device__ __forceinline__ void octet(float most, unsigned limit) {
-        peak = fmaxf(peak, most);
+        peak = larger(peak, most);
         below += (unsigned)__popcll(__ballot(__float_as_uint(most) - 1u < limit - (kWindow + 1u)));
     }
 };
@@ -881,18 +884,21 @@ __device__ __forceinline__ unsigned first_limit(float most, unsigned *words) {
 }
 
 // the two terms of eight values times `scale` (the lower one times 2^8), each as four words of two halves (lower k in the lower
-// half).  The additions of zero make every step one mixed-precision multiply-add (v_fma_mix*, three per value; products that are
-// converted take five instructions).  No assembly: the compiler does not know what wait the matrix instructions need behind that.
+// half): four multiplications, two conversions of pairs and two mixed-precision multiply-adds for two values, four cycles each.  (As
+// v_fma_mixlo_f16 / v_fma_mixhi_f16, seven instructions, it takes 48 instead of 32: these two are issued at half the rate.  Four 1 x 1 convolutions
+// of 768 channels on 17 x 17 at batch 64, 704 outputs: 100 -> 94 us; 2048 on 8 x 8, batch 7: 33.7 -> 31.8.)  No assembly: the compiler does not know
+// what wait the matrix instructions need behind that.
 __device__ __forceinline__ void split_half2(const float (&x)[8], float scale, uintx4 &hi, uintx4 &lo) {
+    const float lifted = scale * kInputLift;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        halfx2 h, l;
+        const floatx2 scaled = {x[2 * i] * scale, x[2 * i + 1] * scale};
+        const halfx2 h = __builtin_convertvector(scaled, halfx2);
+        floatx2 rest;
 #pragma unroll
-        for (int u = 0; u < 2; u++) h[u] = (_Float16)__builtin_fmaf(x[2 * i + u], scale, 0.f);
-#pragma unroll
-        for (int u = 0; u < 2; u++) l[u] = (_Float16)__builtin_fmaf(__builtin_fmaf(x[2 * i + u], scale, -(float)h[u]), kInputLift, 0.f);   // (the inner one is exact)
+        for (int u = 0; u < 2; u++) rest[u] = __builtin_fmaf((float)h[u], -kInputLift, x[2 * i + u] * lifted);   // (exact)
         hi[i] = __builtin_bit_cast(unsigned, h);
-        lo[i] = __builtin_bit_cast(unsigned, l);
+        lo[i] = __builtin_bit_cast(unsigned, __builtin_convertvector(rest, halfx2));
     }
 }
 
