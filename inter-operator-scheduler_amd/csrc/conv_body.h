@@ -888,17 +888,21 @@ __device__ __forceinline__ unsigned first_limit(float most, unsigned *words) {
 // v_fma_mixlo_f16 / v_fma_mixhi_f16, seven instructions, it takes 48 instead of 32: these two are issued at half the rate.  Four 1 x 1 convolutions
 // of 768 channels on 17 x 17 at batch 64, 704 outputs: 100 -> 94 us; 2048 on 8 x 8, batch 7: 33.7 -> 31.8.)  No assembly: the compiler does not know
 // what wait the matrix instructions need behind that.
-__device__ __forceinline__ void split_half2(const float (&x)[8], float scale, uintx4 &hi, uintx4 &lo) {
+__device__ __forceinline__ void split_pair(float x0, float x1, float scale, unsigned &hi, unsigned &lo) {
     const float lifted = scale * kInputLift;
+    const floatx2 scaled = {x0 * scale, x1 * scale};
+    const halfx2 h = __builtin_convertvector(scaled, halfx2);
+    const floatx2 rest = {__builtin_fmaf((float)h[0], -kInputLift, x0 * lifted), __builtin_fmaf((float)h[1], -kInputLift, x1 * lifted)};   // (exact)
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, __builtin_convertvector(rest, halfx2));
+}
+__device__ __forceinline__ void split_half2(const float (&x)[8], float scale, uintx4 &hi, uintx4 &lo) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const floatx2 scaled = {x[2 * i] * scale, x[2 * i + 1] * scale};
-        const halfx2 h = __builtin_convertvector(scaled, halfx2);
-        floatx2 rest;
-#pragma unroll
-        for (int u = 0; u < 2; u++) rest[u] = __builtin_fmaf((float)h[u], -kInputLift, x[2 * i + u] * lifted);   // (exact)
-        hi[i] = __builtin_bit_cast(unsigned, h);
-        lo[i] = __builtin_bit_cast(unsigned, __builtin_convertvector(rest, halfx2));
+        unsigned h, l;
+        split_pair(x[2 * i], x[2 * i + 1], scale, h, l);
+        hi[i] = h;
+        lo[i] = l;
     }
 }
 
@@ -1209,6 +1213,31 @@ __device__ __forceinline__ void multiply_terms(Acc (&acc)[TM][TN], const uintx4 
         multiply_planes<HALF>(acc, ad, bv[1]);
     }
     multiply_planes<HALF>(acc, av[0], bv[0]);
+}
+
+// The same for two terms in a fixed order, between(n) behind the n-th of 3 TM TN matrix instructions: what it does is issued while they run (an
+// instruction waits for the one before it in the matrix pipe, and all that follows in the wavefront with it).
+template <int TM, int TN, typename Acc, typename Between>
+__device__ __forceinline__ void multiply_terms_between(Acc (&acc)[TM][TN], const uintx4 (&av)[2][TM], const uintx4 (&bv)[2][TN], Between between) {
+    uintx4 ad[TM], bd[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) bd[j] = half_down(bv[0][j], kFilterLift);
+    __builtin_amdgcn_sched_barrier(0);
+    int n = 0;
+#pragma unroll
+    for (int t = 0; t < 3; t++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                acc[i][j] = multiply_half(t == 0 ? av[1][i] : t == 1 ? ad[i] : av[0][i], t == 0 ? bd[j] : t == 1 ? bv[1][j] : bv[0][j], acc[i][j]);
+                if (t == 0 && j == 0) {
+                    ad[i] = half_down(av[0][i], kInputLift);
+                    asm volatile("" : "+v"(ad[i]));
+                }
+                between(n++);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 }
 
 // TMW x TNW MFMA tiles of 32 x 32 per wavefront, WM x WN wavefronts per block

@@ -44,15 +44,23 @@ struct ConvPipe {
 
     // Two terms: one limit for the inputs of the tile, by those of its first stage.  Where that does not serve all of them, the tile is
     // computed again.  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to 100
-    // registers.
+    // registers.  And a third time, PLAIN, for inputs that need neither a ReLU nor channels masked: what a tile with nothing beside it on its
+    // compute unit waits for is the sum of its steps (768 -> 192 on 17 x 17, a block of 64 x 128, per 16 k: 230 cycles for the operands from LDS, 320 for the
+    // matrix instructions, 450 to split an octet, 250 to store and for the barrier), and without the branches between them the split work lies
+    // under the matrix instructions.  That layer at batch 3 23.6 -> 21.7 us, at batch 64 31.8 -> 29.0; four such convolutions in a launch, 704 outputs,
+    // batch 16 31.6 -> 29.2, batch 64 94.2 -> 92.2.
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
-        const unsigned limit = attempt<RES>(a, smem, tile, g, z, kNoLimit);
-        if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES>(a, smem, tile, g, z, limit);
+        bool plain = false;
+        if constexpr (TERMS == 2) plain = a.pre_relu == 0 && (POINT ? a.ICg % BK == 0 : (a.ICg & 3) == 0);
+        unsigned limit;
+        if (plain) limit = attempt<RES, true, TERMS == 2>(a, smem, tile, g, z, kNoLimit);
+        else limit = attempt<RES, true, false>(a, smem, tile, g, z, kNoLimit);
+        if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES, false, false>(a, smem, tile, g, z, limit);
     }
 
     // limit: kNoLimit for the first attempt.  Returns the limit for another one, or 0.
-    template <bool RES>
+    template <bool RES, bool FIRST, bool PLAIN>
     __device__ static __forceinline__ unsigned attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, unsigned limit) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
@@ -169,7 +177,7 @@ struct ConvPipe {
             for (int j = 0; j < 8; j++) v[j] = j < mine ? v[j] : 0.f;
         }
     };
-    auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
+    auto store_octets = [&](int buf, const uintx4 (&ar)[A_IT], const uintx4 (&hi)[B_IT], const uintx4 (&lo)[B_IT]) {
         uintx4 *As = lds + buf * STAGE;
         uintx4 *Bs = As + A_SLOTS + unit * (TERMS * UNIT);
 #pragma unroll
@@ -177,24 +185,29 @@ struct ConvPipe {
             if (A_SLOTS % T == 0 || tid + i * T < A_SLOTS) As[tid + i * T] = ar[i];
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
-            float v[8];
-            octet_of(br[i], left, v);
             const int slot = slot_of(tid / OCT + i * (T / OCT), half);
-            if constexpr (TERMS == 2) {
-                uintx4 hi, lo;
-                watch.octet(octet_peak(v), limit);
-                split_half2(v, limit_scale(limit), hi, lo);
-                Bs[slot] = hi;
-                Bs[UNIT + slot] = lo;
-            } else if constexpr (HALF) {
-                const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
-                Bs[slot] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));   // round to nearest even, overflow to infinity
-            } else {
-                Bs[slot] = round_bf16x8(v);
-            }
+            Bs[slot] = hi[i];
+            if constexpr (TERMS == 2) Bs[UNIT + slot] = lo[i];
         }
     };
-    const bool first = limit == kNoLimit;
+    auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
+        uintx4 hi[B_IT], lo[B_IT];
+#pragma unroll
+        for (int i = 0; i < B_IT; i++) {
+            float v[8];
+            octet_of(br[i], left, v);
+            if constexpr (TERMS == 2) {
+                watch.octet(octet_peak(v), limit);
+                split_half2(v, limit_scale(limit), hi[i], lo[i]);
+            } else if constexpr (HALF) {
+                const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+                hi[i] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));   // round to nearest even, overflow to infinity
+            } else {
+                hi[i] = round_bf16x8(v);
+            }
+        }
+        store_octets(buf, ar, hi, lo);
+    };
 
     typename M::acc_t acc[TM][TN];
 #pragma unroll
@@ -210,7 +223,7 @@ struct ConvPipe {
 #pragma unroll
     for (int s = 0; s < PD; s++) load_stage(s, a_reg[s], b_reg[s], b_left[s]);
     if constexpr (TERMS == 2) {
-        if (first) {
+        if constexpr (FIRST) {
             float most = 0.f;
 #pragma unroll
             for (int i = 0; i < B_IT; i++) {
@@ -224,6 +237,8 @@ struct ConvPipe {
     store_stage(0, a_reg[0], b_reg[0], b_left[0]);
     load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
     __syncthreads();
+    // (otherwise the compiler waits for all loads in every round, for registers that hold loads only on the way in)
+    if constexpr (PLAIN) __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
     for (int st0 = 0; st0 < stages; st0 += PD) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
@@ -231,21 +246,62 @@ struct ConvPipe {
             const int buf = st & 1;
             const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
             const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
-#pragma unroll
-            for (int u = 0; u < KU; u++) {
-                uintx4 av[TERMS][TM], bv[TERMS][TN];
+            // operands of the next unit are read ahead of a unit's matrix work, where registers allow it
+            constexpr int TURN = PLAIN && KU > 1 && TMW * TNW != 2 ? 1 : 0;
+            uintx4 av[TURN + 1][TERMS][TM], bv[TURN + 1][TERMS][TN];
+            auto read_unit = [&](int u) {
 #pragma unroll
                 for (int p = 0; p < TERMS; p++) {
 #pragma unroll
-                    for (int i = 0; i < TM; i++) av[p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
+                    for (int i = 0; i < TM; i++) av[u & TURN][p][i] = Ab[(2 * u * TERMS + p) * BM + i * MT];
 #pragma unroll
-                    for (int j = 0; j < TN; j++) bv[p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
+                    for (int j = 0; j < TN; j++) bv[u & TURN][p][j] = Bb[(u * TERMS + p) * UNIT + j * 2 * MT];
                 }
-                // all LDS reads of the unit are requested before its first matrix instruction
-                if (TERMS == 2) __builtin_amdgcn_sched_barrier(0);
-                multiply_terms<TERMS, HALF>(acc, av, bv);
+            };
+            const uintx4 (&ar)[A_IT] = a_reg[(s + 1) % PD];
+            const floatx4 (&br)[B_IT][2] = b_reg[(s + 1) % PD];
+            if constexpr (PLAIN) {
+                // The octets of the next stage are split between the matrix instructions of this one, a pair of values at a time.
+                constexpr int SLOTS = 3 * TM * TN * KU, PIECES = 5 * B_IT;
+                uintx4 hi[B_IT], lo[B_IT];
+#pragma unroll
+                for (int u = 0; u < KU; u++) {
+                    if (TURN == 0 || u == 0) {
+                        read_unit(u);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (TURN == 1 && u + 1 < KU) read_unit(u + 1);
+                    multiply_terms_between(acc, av[u & TURN], bv[u & TURN], [&](int n) {
+                        const int slot = u * 3 * TM * TN + n;
+#pragma unroll
+                        for (int piece = slot * PIECES / SLOTS; piece < (slot + 1) * PIECES / SLOTS; piece++) {
+                            const int i = piece / 5, q = piece % 5;
+                            if (q < 4) {
+                                unsigned h, l;
+                                split_pair(br[i][q >> 1][2 * (q & 1)], br[i][q >> 1][2 * (q & 1) + 1], limit_scale(limit), h, l);
+                                asm volatile("" : "+v"(h), "+v"(l));   // (here, and not where they are stored)
+                                hi[i][q] = h;
+                                lo[i][q] = l;
+                            } else {
+                                float v[8];
+#pragma unroll
+                                for (int j = 0; j < 8; j++) v[j] = br[i][j >> 2][j & 3];
+                                watch.octet(octet_peak(v), limit);
+                            }
+                        }
+                    });
+                }
+                store_octets(buf ^ 1, ar, hi, lo);
+            } else {
+#pragma unroll
+                for (int u = 0; u < KU; u++) {
+                    read_unit(u);
+                    // all LDS reads of the unit are requested before its first matrix instruction
+                    if (TERMS == 2) __builtin_amdgcn_sched_barrier(0);
+                    multiply_terms<TERMS, HALF>(acc, av[0], bv[0]);
+                }
+                store_stage(buf ^ 1, ar, br, b_left[(s + 1) % PD]);
             }
-            store_stage(buf ^ 1, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
             load_stage(st + 1 + PD, a_reg[(s + 1) % PD], b_reg[(s + 1) % PD], b_left[(s + 1) % PD]);
             __syncthreads();
         }

@@ -152,12 +152,14 @@ def test_measured_batches_under_every_executor(executor, schedule):
     rt.set_option('autotune', 1)
     try:
         rt.set_option('executor', executor)
-        graph = heads((192, 17, 17), (96, 64, 96, 48), 1, 0, schedule)
+        graph = heads((384, 17, 17), (192, 160, 160, 192), 1, 0, schedule)
         rng = np.random.default_rng(1)
         with rt.Session(graph, 12) as session:
             session.load_weights()
-            assert sum('batch' in op for op in session.describe()) == 4
-            assert sum(launch['kernel'].startswith('conv_batch_kernel') for launch in session.launches()) == 1
+            # (one after the other they take twice as long as together; beside each other the measurement decides)
+            batched = sum('batch' in op for op in session.describe())
+            assert batched == 4 or (batched == 0 and schedule == 'greedy')
+            assert sum(launch['kernel'].startswith('conv_batch_kernel') for launch in session.launches()) == batched // 4
             for _ in range(3):
                 x = rng.standard_normal((12, *graph.enter_node.output_shape)).astype(np.float32)
                 session.set_input(x)
