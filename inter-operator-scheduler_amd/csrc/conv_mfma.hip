@@ -19,7 +19,7 @@ struct VariantEntry {
     ConvVariant v;
     KernelPair any;
     int smem_floats;
-    KernelPair special[2] = {};   // staged kernels for the filters that kernel_of() names
+    KernelPair special[4] = {};   // staged kernels for the filters that kernel_of() names
 };
 
 #define IOS_TILED_ENTRY(IDX, NAME, BM, BN, BK, WM, WN, WK, MT, PD)                                        \
@@ -83,7 +83,8 @@ struct VariantEntry {
       ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SPAN},                                                                     \
      kWindowKernels[IDX - kFirstWindowVariant], \
      ConvWindow<TERMS, HALF, TMW, TNW, WM, WN, P_IT, NBUF>::SMEM_FLOATS, \
-     {kWindow7Kernels[IDX - kFirstWindowVariant], kWindow9Kernels[IDX - kFirstWindowVariant]}},
+     {kWindow7Kernels[IDX - kFirstWindowVariant], kWindow9Kernels[IDX - kFirstWindowVariant], \
+      kWindow7ShortKernels[IDX - kFirstWindowVariant], kWindow9ShortKernels[IDX - kFirstWindowVariant]}},
 #define IOS_WINDOW3_ENTRY(...) IOS_WINDOW_ENTRY(2, true, PREC_FP32, __VA_ARGS__)
 #define IOS_WINDOW_BF16_ENTRY(...) IOS_WINDOW_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
 #define IOS_WINDOW_FP16_ENTRY(...) IOS_WINDOW_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
@@ -394,12 +395,15 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     return d;
 }
 
-// Which of an entry's kernels serves the problem: 0 any, 1 and 2 the special ones.  Pipelined kernels: [1] 1 x 1 filters without groups,
+// Which of an entry's kernels serves the problem: 0 any, else the special ones.  Pipelined kernels: [1] 1 x 1 filters without groups,
 // whose addresses stay the same over K (at batch 64 768 -> 192 on 17 x 17 39.7 -> 34.8 us, 2048 -> 320 on 8 x 8 51.2 -> 43.1).  Window kernels:
-// [1] seven taps, [2] nine (see known_chunk; other numbers are rare, 1 x 3 and 5 x 5).
+// [1] seven taps, [2] nine (see known_chunk; other numbers are rare, 1 x 3 and 5 x 5), [3] and [4] the same where the window fits three rounds.
 static int kernel_of(const ConvProblem &p, const VariantEntry &e) {
     const int taps = p.KH * p.KW;
-    if (e.v.window != 0) return taps == 7 ? 1 : taps == 9 ? 2 : 0;
+    if (e.v.window != 0) {
+        const int known = taps == 7 ? 1 : taps == 9 ? 2 : 0;
+        return known != 0 && window_span(p, e.v.BN) <= short_rounds(INT_MAX) * (e.v.threads() / 2) ? known + 2 : known;
+    }
     return e.special[0].kernel != nullptr && taps == 1 && p.groups == 1 ? 1 : 0;
 }
 
@@ -414,7 +418,7 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
     const bool with_residual = !d.args.xcd_local && d.args.res != nullptr;
     const ConvKernelFn kernel = with_residual ? pair.kernel_residual : pair.kernel;
     if (d.smem_bytes > 64 * 1024) {   // beyond the default limit of dynamic LDS: raised once per kernel
-        static bool raised[kNumConvVariants][6] = {};
+        static bool raised[kNumConvVariants][10] = {};
         bool &done = raised[d.variant][2 * which + (with_residual ? 1 : 0)];
         if (!done) {
             if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, d.smem_bytes) != hipSuccess)

@@ -46,12 +46,18 @@ struct ConvWindow {
     // 60 registers, a loop around it as many, for addresses and masks that are held for the second time.
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
-        const unsigned limit = attempt<RES>(a, smem, tile, g, z, kNoLimit);
-        if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES>(a, smem, tile, g, z, limit);
+        // Inputs that need neither a ReLU nor channels masked: a test a round, and the copies that its two ways out take, cost as much as the
+        // conversion (192 -> 192 1 x 7 on 17 x 17 at batch 64 in bfloat16: 290 cycles a round, 24.8 -> 21.1 us).  Not for two terms in windows of
+        // two rounds, whose code comes out slower that way (160 -> 160 1 x 7 32.0 -> 34.1 us).
+        constexpr bool KNOWN = TAPS > 0 && (TERMS == 1 || NBUF == 1);
+        unsigned limit;
+        if (KNOWN && a.pre_relu == 0 && (a.ICg & 3) == 0) limit = attempt<RES, true, KNOWN>(a, smem, tile, g, z, kNoLimit);
+        else limit = attempt<RES, true, false>(a, smem, tile, g, z, kNoLimit);
+        if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES, false, false>(a, smem, tile, g, z, limit);
     }
 
     // limit: kNoLimit for the first attempt.  Returns the limit for another one, or 0.
-    template <bool RES>
+    template <bool RES, bool FIRST, bool PLAIN>
     __device__ static __forceinline__ unsigned attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, unsigned limit) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
@@ -141,7 +147,12 @@ struct ConvWindow {
         for (int i = 0; i < P_IT; i++) {
             if (!needed(i)) break;
             float v[8];
-            octet_of(i, v);
+            if constexpr (PLAIN) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = b_reg[i][j >> 2][j & 3];
+            } else {
+                octet_of(i, v);
+            }
             if constexpr (TERMS == 2) {
                 uintx4 hi, lo;
                 watch.octet(octet_peak(v), limit);
@@ -179,10 +190,9 @@ struct ConvWindow {
     constexpr unsigned kZero = (S - 1) * 16;
 
     typename M::acc_t acc[TM][TN];
-    const bool first = limit == kNoLimit;
     auto begin = [&] {   // behind the request for the first window
         if constexpr (TERMS == 2) {
-            if (!first) return;
+            if constexpr (!FIRST) return;
             float most = 0.f;
 #pragma unroll
             for (int i = 0; i < P_IT; i++) {
@@ -378,10 +388,13 @@ struct ConvWindow {
     X(153, "wh_win_m64n128_w1x4", 2, 1, 1, 4, 3, 1)      \
     X(154, "wh_win_m64n256_w1x4", 2, 2, 1, 4, 5, 1)      \
     X(155, "wh_win_m32n256_w1x4", 1, 2, 1, 4, 5, 1)
+// Rounds of a kernel for windows of at most three: loads of rounds that no output needs return zeros, but the L1 takes 16 cycles for each like
+// for any other, and what a tap with one term waits for is the L1 (96 -> 96 3 x 3 on 35 x 35 at batch 64 52.2 -> 48.1 us, bfloat16 29.0 -> 27.2, with PLAIN).
+constexpr int short_rounds(int rounds) { return std::min(rounds, 3); }
 constexpr int kFirstWindowVariant = 139, kNumConvVariants = 170;
 
 // The window kernels in the order of the lists above: for any number of taps (conv_window.hip), for 7 and for 9 (conv_window7.hip,
-// conv_window9.hip)
-extern const KernelPair kWindowKernels[], kWindow7Kernels[], kWindow9Kernels[];
+// conv_window9.hip), the latter two also with windows of three rounds
+extern const KernelPair kWindowKernels[], kWindow7Kernels[], kWindow9Kernels[], kWindow7ShortKernels[], kWindow9ShortKernels[];
 
 }  // namespace ios
