@@ -206,12 +206,30 @@ void launch_pack_depthwise(const ConvProblem &p, const float *w, float *packed, 
 
 // ---- from the host's layout to views -------------------------------------------------------------------------------------
 // Bound by bytes (or by the link, where `nchw` lies in host memory).  Few channels (images): a thread takes a pixel, reads its
-// channels from their planes, consecutive threads consecutive pixels, and writes one pixel.  Otherwise a block turns a
-// tile of 32 channels x 64 pixels through LDS.
-__global__ __launch_bounds__(256) void to_view_kernel(const float *nchw, float *view, int B, int C, int HW, long long plane, int ps) {
+// channels from their planes, consecutive threads consecutive pixels, and writes one pixel.  Otherwise a block turns a tile of
+// 32 channels x 240 pixels through LDS: a row of the tile is read from line to line, 64 lanes of 16 bytes, wherever it begins.
+// Rows of 64 pixels at odd places straddle five lines instead of four, and no cache keeps host memory for the block that reads
+// the rest: three images of 131 channels x 37 x 53 took 115 us until they were there and take 96 like this (3.1 MB; 54 is the
+// link).  Up to four channels the planes' rows are long: whole lines through LDS gave nothing there (seven images of 299 x 299
+// 209 us against 203, five of 224 x 224 93 against 87).
+constexpr int kLine = 16;   // floats
+constexpr int kTileRow = 240, kTileChannels = 32;
+
+// Floats [at, at + 4) of `total`, at a multiple of four; those outside are zero.
+__device__ __forceinline__ pw_floatx4 line_quad(const float *nchw, long long at, long long total) {
+    if (at + 4 <= total) return *reinterpret_cast<const pw_floatx4 *>(nchw + at);
+    pw_floatx4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (at + j < total) v[j] = nchw[at + j];
+    return v;
+}
+
+// lead: floats from the last multiple of a line in memory to the first element; total: floats from there to behind the last
+__global__ __launch_bounds__(256) void to_view_kernel(const float *nchw, float *view, int B, int C, int HW, long long plane, int ps, int lead, long long total) {
     if (C <= 4) {
-        const long long total = (long long)B * HW;
-        for (long long i = blockIdx.x * 256LL + threadIdx.x; i < total; i += gridDim.x * 256LL) {
+        const long long pixels = (long long)B * HW;
+        for (long long i = blockIdx.x * 256LL + threadIdx.x; i < pixels; i += gridDim.x * 256LL) {
             const long long b = i / HW, r = i - b * HW;
             const float *first = nchw + b * C * plane + r;
             float *pixel = view + i * ps;
@@ -230,39 +248,50 @@ __global__ __launch_bounds__(256) void to_view_kernel(const float *nchw, float *
         }
         return;
     }
-    // (64 pixels: 256 bytes of a plane at a time, which the link carries at 45 GB/s where pieces of 128 bytes at odd places come
-    // to 26)
-    __shared__ float tile[32][65];
-    const int tiles_c = (C + 31) / 32, tiles_p = (HW + 63) / 64;
-    const long long tiles = (long long)B * tiles_c * tiles_p;
-    const int px = threadIdx.x & 63, c4 = threadIdx.x >> 6;    // of the host's layout: pixel, channel of four
-    const int cx = threadIdx.x & 31, p8 = threadIdx.x >> 5;    // of the view: channel, pixel of eight
-    for (long long t = blockIdx.x; t < tiles; t += gridDim.x) {
+    nchw -= lead;
+    constexpr int STRIDE = kTileRow + kLine + 4;
+    __shared__ float rows[kTileChannels * STRIDE];
+    const int tid = threadIdx.x;
+    const int tiles_c = (C + kTileChannels - 1) / kTileChannels, tiles_p = (HW + kTileRow - 1) / kTileRow;
+    const int lane = tid & 63, wave = tid >> 6;              // of the host's layout: four floats of a row, a channel of four
+    const int cx = tid & 31, p8 = tid >> 5;                  // of the view: channel, pixel of eight
+    for (long long t = blockIdx.x; t < (long long)B * tiles_c * tiles_p; t += gridDim.x) {
         const long long bt = t / tiles_p;
-        const int p0 = (int)(t - bt * tiles_p) * 64;
-        const int b = (int)(bt / tiles_c), c0 = (int)(bt - (long long)b * tiles_c) * 32;
-        const float *planes = nchw + ((long long)b * C + c0) * plane + p0;
-        float *pixels = view + ((long long)b * HW + p0) * ps + c0;
+        const int p0 = (int)(t - bt * tiles_p) * kTileRow, pixels = min(kTileRow, HW - p0);
+        const long long b = bt / tiles_c;
+        const int c0 = (int)(bt - b * tiles_c) * kTileChannels;
+        const long long first = lead + (b * C + c0) * plane + p0;
+        pw_floatx4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int c = wave + 4 * i;
+            const long long at = first + c * plane, from = at & ~(long long)(kLine - 1);
+            v[i] = pw_floatx4{0.f, 0.f, 0.f, 0.f};
+            if (c0 + c < C && 4 * lane < (int)(at - from) + pixels) v[i] = line_quad(nchw, from + 4 * lane, total);
+        }
         __syncthreads();
-        float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = c0 + c4 + 4 * i < C && p0 + px < HW ? planes[(c4 + 4 * i) * plane + px] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) tile[c4 + 4 * i][px] = v[i];
+        for (int i = 0; i < 8; i++) *reinterpret_cast<pw_floatx4 *>(rows + (wave + 4 * i) * STRIDE + 4 * lane) = v[i];
         __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (c0 + cx < C && p0 + p8 + 8 * i < HW) pixels[(long long)(p8 + 8 * i) * ps + cx] = tile[cx][p8 + 8 * i];
+        if (c0 + cx < C) {
+            const float *row = rows + cx * STRIDE + (int)((first + cx * plane) & (kLine - 1));
+            float *out = view + (b * HW + p0) * ps + c0 + cx;
+            for (int p = p8; p < pixels; p += 8) out[(long long)p * ps] = row[p];
+        }
     }
 }
 
 static int layout_blocks(int B, int C, int HW) {
-    return C <= 4 ? blocks_for((long long)B * HW, 256, 1024) : blocks_for((long long)B * ((C + 31) / 32) * ((HW + 63) / 64), 1, 2048);
+    return C <= 4 ? blocks_for((long long)B * HW, 256, 1024)
+                  : blocks_for((long long)B * ((C + kTileChannels - 1) / kTileChannels) * ((HW + kTileRow - 1) / kTileRow), 1, 2048);
 }
 
 void launch_to_view(const float *nchw, const TensorView &y, int B, hipStream_t stream, long long plane) {
-    hipLaunchKernelGGL(to_view_kernel, dim3(layout_blocks(B, y.C, y.H * y.W)), dim3(256), 0, stream, nchw, y.ptr, B, y.C,
-                       y.H * y.W, plane > 0 ? plane : (long long)y.H * y.W, y.pstride);
+    const int HW = y.H * y.W;
+    const long long step = plane > 0 ? plane : HW;
+    const int lead = (int)(reinterpret_cast<uintptr_t>(nchw) / sizeof(float) % kLine);
+    const long long total = lead + ((long long)B * y.C - 1) * step + HW;
+    hipLaunchKernelGGL(to_view_kernel, dim3(layout_blocks(B, y.C, HW)), dim3(256), 0, stream, nchw, y.ptr, B, y.C, HW, step, y.pstride, lead, total);
 }
 
 // ---- fills ---------------------------------------------------------------------------------------------------------
