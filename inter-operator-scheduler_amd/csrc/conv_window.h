@@ -33,6 +33,7 @@ struct ConvWindow {
     static constexpr int CPAD = 16;
     static constexpr bool FUSABLE = false;
     static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : TAPS > 0 || TNW == 2 ? 3 : 4;
+    static constexpr int kTouches = 4;                 // lines of 128 bytes of the filters a thread requests at the start
     static constexpr int SPAN = P_IT * (T / 2);       // pixels of the input a block holds
     // slots of 16 bytes per plane and octet (eight consecutive channels), the last one zero; the octets of a pixel, which
     // neighbouring lanes store, fall into different banks
@@ -95,6 +96,33 @@ struct ConvWindow {
     }
     const unsigned plane_bytes = (unsigned)a.OCgP * 16u;
     const unsigned tap_bytes = (unsigned)(a.ICgP >> 3) * TERMS * plane_bytes, chunk_bytes = 2u * TERMS * plane_bytes;
+
+    // The filters of a pass fit no L2: all of what the block will read is requested at once, a word of every line, shared out over the
+    // blocks of the XCD that read the same.  Requested two taps ahead only, each of them waits for memory.  With filters that no cache
+    // holds, bfloat16 at batch 64, 192 -> 192 1 x 7 on 17 x 17 took 25.7 us (20.6 with filters in the L2) and takes 20.2, 256 -> 256 3 x 3 on
+    // 14 x 14 38.8 (26.8) -> 27.2, 448 -> 384 3 x 3 on 8 x 8 48.7 (32.3) -> 34.3; two terms at batch 7, 256 -> 256 38.5 -> 32.8.  It costs
+    // 0.2 to 1 us where they are in the L2.
+    unsigned touched[FIRST ? kTouches : 1];
+    if constexpr (FIRST) {
+        const int slot = tile >> 3;
+        int share, mine;
+        if (a.weights_major) {
+            share = min(a.xcd_q, a.tile_div);
+            mine = a.xcd_q <= a.tile_div ? slot : tn;
+        } else {
+            share = (int)fast_div((unsigned)a.xcd_q, a.div_tile);
+            mine = (int)fast_div((unsigned)slot, a.div_tile);
+        }
+        constexpr int LINES = BM / 8;   // of 128 bytes, for eight consecutive k of a plane
+        const int lines = a.split_k == 1 ? (a.Kq >> 3) * TERMS * LINES : 0, step = max(share, 1) * T;
+        const __amdgpu_buffer_rsrc_t wr = buffer_of(a.wp, a.w_bytes);
+        const unsigned base = (unsigned)g * ((unsigned)a.Kq >> 3) * TERMS * plane_bytes + (unsigned)m0 * 16u;
+#pragma unroll
+        for (int i = 0; i < kTouches; i++) {
+            const int line = mine * T + tid + i * step;
+            touched[i] = __builtin_amdgcn_raw_buffer_load_b32(wr, line < lines ? base + (unsigned)(line / LINES) * plane_bytes + (unsigned)(line % LINES) * 128u : kOutOfRange, 0, 0);
+        }
+    }
 
     // ---- window: first input pixel of the block: tap (0, 0) of output pixel n0
     auto input_of = [&](int n, int &oh, int &ow) {
@@ -202,6 +230,11 @@ struct ConvWindow {
             }
             limit = first_limit<WM * WN>(most, words);
         }
+    };
+    auto touches_end = [&] {
+        if constexpr (FIRST)
+#pragma unroll
+            for (int i = 0; i < kTouches; i++) asm volatile("" ::"v"(touched[i]));
     };
     uintx4 av[2][TERMS][TM];
     // next filter operands to request
@@ -324,6 +357,7 @@ struct ConvWindow {
         filters_at(fv[1], (unsigned)ch_begin * chunk_bytes + tap_bytes, true);
         load_window(ch_begin);
         begin();
+        touches_end();
         for (int ch = ch_begin; ch < ch_end; ch += 2) {
             known_chunk(ch, std::integral_constant<int, 0>{});
             if (ch + 1 >= ch_end) break;
@@ -333,6 +367,7 @@ struct ConvWindow {
         load_filters(av[0]);
         load_window(ch_begin);
         begin();
+        touches_end();
         for (int ch = ch_begin; ch < ch_end; ch += 2) {
             chunk(ch, std::integral_constant<int, 0>{});
             if (ch + 1 >= ch_end) break;
