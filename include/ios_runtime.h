@@ -121,7 +121,9 @@ const char *ios_last_error(void);
  *   "batch_convs" = "1" (default) | "0": 1 x 1 convolutions of one view through the same window (the heads of the branches of a
  *       block) share a launch where a measurement finds that faster (with "autotune" = "1"; pinned configurations that have such a
  *       kernel always).  They then run in the stage of the first of them; the same results bit for bit as apart on the same
- *       configuration.  "host_plan_batches" = "1" | "0" (default): plans made without a device batch whatever they may;
+ *       configuration.  Convolutions that the groups of a stage begin with, and those of one view through different windows, share
+ *       launches by the same rule, and a pool beside them goes along.  "host_plan_batches" = "0" (default) | "1" | "2": plans made
+ *       without a device batch the former ("1") or both ("2") wherever they may;
  *   "host_threads" = N: threads that share a large copy between a caller's arrays and pinned memory, the caller among them
  *       (12 at most; 1: the caller alone).  "0" (default): three quarters of the processors the process is bound to or that its
  *       control group leaves it.  Up to three of them stay awake for half a millisecond behind a copy;

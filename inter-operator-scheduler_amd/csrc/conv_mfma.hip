@@ -1,10 +1,12 @@
 // Stand-alone convolution kernels, the configuration table and the launchers.  Device code: conv_body.h.
 #include "conv_kernel.h"
+#include "conv_mixed.h"
 #include "conv_window.h"
 #include "launch_internal.h"
 
 #include <algorithm>
 #include <climits>
+#include <cstring>
 #include <stdexcept>
 #include <string>
 
@@ -438,7 +440,7 @@ bool conv_batchable(const ConvProblem &a, const ConvProblem &b) {
            a.sh == b.sh && a.sw == b.sw && a.ph == b.ph && a.pw == b.pw;
 }
 
-void launch_conv_batch(const ConvBatchMember *members, int count, int variant, const TensorView &x, hipStream_t stream) {
+void launch_conv_batch(const ConvBatchMember *members, int count, int variant, hipStream_t stream) {
     if (count < 1 || count > kMaxConvBatch || !conv_variant_batches(variant)) throw std::runtime_error("conv: no such batch");
     const VariantEntry &e = kVariants[variant];
     ConvLaunch l;
@@ -449,7 +451,7 @@ void launch_conv_batch(const ConvBatchMember *members, int count, int variant, c
     for (int i = 0; i < kMaxConvBatch; i++) {
         const ConvBatchMember &m = members[std::min(i, count - 1)];
         if (!conv_batchable(members[0].p, m.p)) throw std::runtime_error("conv: a batch of convolutions that do not fit each other");
-        const ConvDispatch d = make_conv_dispatch(m.p, l, x, m.packed, m.filters, m.bias, m.y, nullptr, SplitKReduce{});
+        const ConvDispatch d = make_conv_dispatch(m.p, l, members[0].x, m.packed, m.filters, m.bias, m.y, nullptr, SplitKReduce{});
         b.item[i] = d.args;
         b.item[i].xcd_q = b.item[i].xcd_r = b.item[i].weights_major = 0;
         b.item[i].tile_div = d.args.tiles_m;
@@ -478,6 +480,59 @@ void launch_conv_batch(const ConvBatchMember *members, int count, int variant, c
         }
     }
     hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(threads), smem_bytes, stream, b);
+}
+
+bool conv_variant_mixes(int variant) { return variant >= kFirstPipeVariant && variant < kFirstWindowVariant + kWindowVariants; }
+
+bool conv_mixable(const ConvProblem &p, int variant) {
+    return conv_variant_mixes(variant) && p.groups == 1 && conv_variant_takes(p, variant) && conv_variant_precise(p, variant);
+}
+
+void launch_conv_mixed(const ConvBatchMember *members, int count, const MixedPool *pool, int variant, hipStream_t stream) {
+    if (count < 1 || count > kMaxConvBatch || !conv_variant_mixes(variant)) throw std::runtime_error("conv: no such launch of mixed convolutions");
+    const VariantEntry &e = kVariants[variant];
+    ConvLaunch l;
+    l.variant = variant;
+    ConvMixedArgs b;
+    long long blocks = 0;
+    int threads = 0, smem_bytes = 0, which = -1;
+    for (int i = 0; i < kMaxConvBatch; i++) {
+        const ConvBatchMember &m = members[std::min(i, count - 1)];
+        if (!conv_mixable(m.p, variant)) throw std::runtime_error(std::string("conv: configuration ") + e.v.name + " does not take a member of a launch");
+        const ConvDispatch d = make_conv_dispatch(m.p, l, m.x, m.packed, m.filters, m.bias, m.y, nullptr, SplitKReduce{});
+        b.item[i] = d.args;
+        b.first[i] = i < count ? (int)blocks : INT_MAX;
+        if (i >= count) continue;
+        blocks += ((long long)d.tiles + 7) & ~7ll;
+        threads = d.threads;
+        smem_bytes = d.smem_bytes;
+        const int here = e.v.window != 0 ? kernel_of(m.p, e) : 0;
+        which = which < 0 || which == here ? here : 0;
+    }
+    b.pool_first = INT_MAX;
+    b.pool_blocks = 0;
+    memset(&b.pool, 0, sizeof(b.pool));
+    if (pool != nullptr) {
+        b.pool = make_pool_args(pool->p, pool->x, pool->y, false, &b.pool_blocks, pool->bias, pool->act);
+        b.pool_blocks = std::max(1, (b.pool_blocks * 256 + threads - 1) / threads);   // (counted for 256 threads)
+        b.pool_first = (int)std::min<long long>(blocks, INT_MAX);
+        blocks += b.pool_blocks;
+    }
+    if (blocks >= INT_MAX) throw std::runtime_error("conv: grid too large");
+    const int index = variant - (e.v.window != 0 ? kFirstWindowVariant : kFirstPipeVariant);
+    // (windows of more than three rounds with a known number of taps are rare here: the kernel for any number serves them)
+    const ConvMixedKernelFn *kernels = e.v.window == 0 ? kPipeMixedKernels : which == 3 ? kWindow7MixedKernels : which == 4 ? kWindow9MixedKernels : kWindowMixedKernels;
+    const ConvMixedKernelFn kernel = kernels[index];
+    if (smem_bytes > 64 * 1024) {
+        static bool raised[kNumConvVariants][3] = {};
+        bool &done = raised[variant][which >= 3 ? which - 2 : 0];
+        if (!done) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes) != hipSuccess)
+                throw std::runtime_error(std::string("conv: cannot reserve LDS for mixed convolutions on configuration ") + e.v.name);
+            done = true;
+        }
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), smem_bytes, stream, b);
 }
 
 // ---- filter packing ------------------------------------------------------------------------

@@ -426,7 +426,7 @@ struct ConvWindow {
 // Rounds of a kernel for windows of at most three: loads of rounds that no output needs return zeros, but the L1 takes 16 cycles for each like
 // for any other, and what a tap with one term waits for is the L1 (96 -> 96 3 x 3 on 35 x 35 at batch 64 52.2 -> 48.1 us, bfloat16 29.0 -> 27.2, with PLAIN).
 constexpr int short_rounds(int rounds) { return std::min(rounds, 3); }
-constexpr int kFirstWindowVariant = 139, kNumConvVariants = 170;
+constexpr int kFirstWindowVariant = 139, kWindowVariants = 17, kNumConvVariants = 170;
 
 // The window kernels in the order of the lists above: for any number of taps (conv_window.hip), for 7 and for 9 (conv_window7.hip,
 // conv_window9.hip), the latter two also with windows of three rounds

@@ -174,17 +174,20 @@ void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorVie
                       const float *bias, const TensorView &y, float *workspace, const SplitKReduce &reduce, hipStream_t stream,
                       const TensorView *residual = nullptr, bool post_relu = false);
 
-// Several convolutions of one input in a launch: they read the same view through the same window, without groups or a residual.
-// Every member has the packed filters, bias and output of its own.
+// Several convolutions in a launch, without groups or a residual, each with the packed filters, bias and output of its own.
+// A batch: they read the same view (the first member's x) through the same 1 x 1 window.  A mixed one: no two need be alike, and a pool may
+// run beside them.
 struct ConvBatchMember {
     ConvProblem p;
     const float *packed, *filters, *bias;
-    TensorView y;
+    TensorView x, y;
 };
 constexpr int kMaxConvBatch = 4;
 bool conv_variant_batches(int variant);                              // there is a batched kernel on this configuration
 bool conv_batchable(const ConvProblem &a, const ConvProblem &b);     // two convolutions of one view may share a launch
-void launch_conv_batch(const ConvBatchMember *members, int count, int variant, const TensorView &x, hipStream_t stream);
+void launch_conv_batch(const ConvBatchMember *members, int count, int variant, hipStream_t stream);
+bool conv_variant_mixes(int variant);                                // there is a kernel for mixed members on this configuration
+bool conv_mixable(const ConvProblem &p, int variant);                // and it takes this one
 
 // Filters of a depth-wise convolution: w[C][1][KH][KW] -> packed[tap][C rounded up to 4] (padding zero).
 inline size_t dwconv_packed_floats(const ConvProblem &p) { return (size_t)p.KH * p.KW * ((p.OC + 3) & ~3); }
@@ -211,6 +214,13 @@ struct PoolProblem {
 void launch_pool(const PoolProblem &p, const TensorView &x, const TensorView &y, hipStream_t stream, const float *bias = nullptr,
                  int act = ACT_NONE);
 // Window == whole map: one wavefront reduces one (n, c) plane.
+struct MixedPool {   // a pool beside mixed convolutions
+    PoolProblem p;
+    TensorView x, y;
+    const float *bias;
+    int act;
+};
+void launch_conv_mixed(const ConvBatchMember *members, int count, const MixedPool *pool, int variant, hipStream_t stream);
 void launch_global_pool(const PoolProblem &p, const TensorView &x, const TensorView &y, hipStream_t stream);
 
 // ---- element-wise -----------------------------------------------------------------------------------

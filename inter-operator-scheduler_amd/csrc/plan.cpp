@@ -1170,45 +1170,114 @@ private:
             readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W, p.sh, p.sw, p.ph, p.pw}].push_back((int)i);
         }
         for (auto &entry : readers) {
-            std::vector<int> &ops = entry.second;
-            if (ops.size() < 2) continue;
-            const ViewRef in = plan_.ops[ops[0]].in;
-            int ready = -1;   // the last stage that writes into the view
-            for (const PlanOp &op : plan_.ops)
-                if (op.out.base == in.base && op.out.first < in.first + in.C && in.first < op.out.first + op.out.C) ready = std::max(ready, op.stage);
-            ops.erase(std::remove_if(ops.begin(), ops.end(), [&](int i) { return plan_.ops[i].stage <= ready; }), ops.end());
-            std::stable_sort(ops.begin(), ops.end(), [&](int a, int b) { return plan_.ops[a].stage < plan_.ops[b].stage; });
+            const std::vector<int> ops = behind_their_view(entry.second);
+            for (size_t first = 0; first + 1 < ops.size(); first += kMaxConvBatch)
+                share_launch({ops.begin() + first, ops.begin() + std::min(ops.size(), first + kMaxConvBatch)}, share, /*mixed=*/false);
+        }
+        find_mixed(share);
+    }
+
+    // Convolutions that parallel groups begin with, and of one view through different windows in whichever stages (1 x 3 and 3 x 1), may
+    // share a launch as well, and a pool that another group begins with goes along: by itself it takes 5 to 8 us, as much as two
+    // convolutions gain by each other.  The other way is a fused launch, which holds kernels without staging only.  1 x 7 and 7 x 1, 160
+    // channels on 17 x 17, and a pool: at batch 16 29.3 -> 21.5 us, half at batch 7 15.4 -> 13.2; 5 x 5 (48 -> 64 channels), 3 x 3 (64 -> 96)
+    // and a pool on 35 x 35 43.1 -> 29.7 and 20.1 -> 15.1; at batch 1 the fused launch is measured to be the faster one.
+    void find_mixed(const std::vector<int> &share) {
+        auto alike = [&](const std::vector<int> &ops) {   // (they had their chance)
+            const PlanOp &a = plan_.ops[ops[0]];
+            for (int i : ops) {
+                const PlanOp &b = plan_.ops[i];
+                if (a.in.base != b.in.base || a.in.first != b.in.first || !conv_batchable(plan_.convs[a.conv].problem, plan_.convs[b.conv].problem)) return false;
+            }
+            return true;
+        };
+        for (size_t s = 0; s < plan_.stages.size(); s++) {
+            if (plan_.stages[s].size() < 2) continue;
+            std::vector<int> ops;
+            int pool = -1;
+            for (const auto &group : plan_.stages[s]) {
+                if (group.empty()) continue;
+                if (may_share(plan_.ops[group[0]], share)) ops.push_back(group[0]);
+                else if (plan_.ops[group[0]].kind == OpKind::Pool) pool = group[0];
+            }
             for (size_t first = 0; first + 1 < ops.size(); first += kMaxConvBatch) {
-                const size_t last = std::min(ops.size(), first + kMaxConvBatch);
-                PlanBatch batch;
-                batch.ops.assign(ops.begin() + first, ops.begin() + last);
-                batch.stage = plan_.ops[batch.ops[0]].stage;
-                std::vector<ConvProblem> problems;
-                std::vector<int> their_share;
-                bool remains = false;
-                for (int i : batch.ops) {
-                    problems.push_back(plan_.convs[plan_.ops[i].conv].problem);
-                    their_share.push_back(share[plan_.ops[i].conv]);
-                    if (plan_.stages[plan_.ops[i].stage].size() == 1) continue;
-                    for (const auto &group : plan_.stages[plan_.ops[i].stage])   // (what runs at the beginning of their stages)
-                        remains = remains || (!group.empty() && std::find(batch.ops.begin(), batch.ops.end(), group[0]) == batch.ops.end());
-                }
-                batch.variant = batch_chooser_(problems, their_share, remains);
-                if (batch.variant < 0) continue;
-                for (int i : batch.ops) {
-                    PlanOp &op = plan_.ops[i];
-                    auto &group = plan_.stages[op.stage][op.group];
-                    group.erase(std::find(group.begin(), group.end(), i));
-                    op.stage = batch.stage;
-                    op.batch = (int)plan_.batches.size();
-                    PlanConv &conv = plan_.convs[op.conv];
-                    conv.launch.variant = batch.variant;
-                    conv.launch.split_k = 1;
-                    batched_.insert(op.conv);
-                }
-                plan_.batches.push_back(batch);
+                std::vector<int> few(ops.begin() + first, ops.begin() + std::min(ops.size(), first + kMaxConvBatch));
+                if (alike(few)) continue;
+                if (pool >= 0) few.push_back(pool);
+                const size_t before = plan_.batches.size();
+                share_launch(few, share, /*mixed=*/true);
+                if (plan_.batches.size() > before) pool = -1;
             }
         }
+        std::map<std::vector<long long>, std::vector<int>> readers;
+        for (size_t i = 0; i < plan_.ops.size(); i++) {
+            const PlanOp &op = plan_.ops[i];
+            if (may_share(op, share)) readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W}].push_back((int)i);
+        }
+        for (auto &entry : readers) {
+            const std::vector<int> ops = behind_their_view(entry.second);
+            for (size_t first = 0; first + 1 < ops.size(); first += kMaxConvBatch) {
+                const std::vector<int> few(ops.begin() + first, ops.begin() + std::min(ops.size(), first + kMaxConvBatch));
+                if (!alike(few)) share_launch(few, share, /*mixed=*/true);
+            }
+        }
+    }
+
+    // of operations that read one view: those of later stages than the last that writes into it, by stage
+    std::vector<int> behind_their_view(std::vector<int> ops) const {
+        const ViewRef in = plan_.ops[ops[0]].in;
+        int ready = -1;
+        for (const PlanOp &op : plan_.ops)
+            if (op.out.base == in.base && op.out.first < in.first + in.C && in.first < op.out.first + op.out.C) ready = std::max(ready, op.stage);
+        ops.erase(std::remove_if(ops.begin(), ops.end(), [&](int i) { return plan_.ops[i].stage <= ready; }), ops.end());
+        std::stable_sort(ops.begin(), ops.end(), [&](int a, int b) { return plan_.ops[a].stage < plan_.ops[b].stage; });
+        return ops;
+    }
+
+    // (among parallel groups not one that fills the device by itself, see tune_conv: no fused launch would hold it)
+    bool may_share(const PlanOp &op, const std::vector<int> &share) const {
+        if (op.kind != OpKind::ConvMfma || op.batch >= 0 || op.has_residual) return false;
+        const PlanConv &conv = plan_.convs[op.conv];
+        if (!conv.matrix_path || conv.problem.groups != 1) return false;
+        return plan_.stages[op.stage].size() == 1 || conv_variant(chooser_(conv.problem, share[op.conv]).variant).fusable();
+    }
+
+    // a launch of these operations (by stage, the first of them at the beginning of its) where it is the faster way
+    void share_launch(std::vector<int> ops, const std::vector<int> &share, bool mixed) {
+        PlanBatch batch;
+        batch.mixed = mixed;
+        batch.ops = std::move(ops);
+        batch.stage = plan_.ops[batch.ops[0]].stage;
+        std::vector<ConvProblem> problems;
+        std::vector<int> their_share;
+        bool remains = false;
+        const PoolProblem *pool = nullptr;
+        for (int i : batch.ops) {
+            if (plan_.ops[i].kind == OpKind::Pool) {
+                pool = &plan_.ops[i].pool;
+                continue;
+            }
+            problems.push_back(plan_.convs[plan_.ops[i].conv].problem);
+            their_share.push_back(share[plan_.ops[i].conv]);
+            if (plan_.stages[plan_.ops[i].stage].size() == 1) continue;
+            for (const auto &group : plan_.stages[plan_.ops[i].stage])   // (what runs at the beginning of their stages)
+                remains = remains || (!group.empty() && std::find(batch.ops.begin(), batch.ops.end(), group[0]) == batch.ops.end());
+        }
+        batch.variant = batch_chooser_(problems, their_share, remains, mixed, pool);
+        if (batch.variant < 0) return;
+        for (int i : batch.ops) {
+            PlanOp &op = plan_.ops[i];
+            auto &group = plan_.stages[op.stage][op.group];
+            group.erase(std::find(group.begin(), group.end(), i));
+            op.stage = batch.stage;
+            op.batch = (int)plan_.batches.size();
+            if (op.conv < 0) continue;
+            PlanConv &conv = plan_.convs[op.conv];
+            conv.launch.variant = batch.variant;
+            conv.launch.split_k = 1;
+            batched_.insert(op.conv);
+        }
+        plan_.batches.push_back(batch);
     }
 
     void finish() {
@@ -1289,7 +1358,8 @@ bool g_arena_reuse = true;
 long long g_thin_conv_min_pixels = 1LL << 18;
 int g_host_split_k = 0;
 bool g_commute_pool_conv = true;
-bool g_batch_convs = true, g_host_batches = false;
+bool g_batch_convs = true;
+int g_host_batches = 0;
 }
 
 bool set_planner_option(const std::string &key, const std::string &value) {
@@ -1305,8 +1375,8 @@ bool set_planner_option(const std::string &key, const std::string &value) {
         g_batch_convs = !(value == "0" || value == "false" || value == "off" || value.empty());
         return true;
     }
-    if (key == "host_plan_batches") {   // plans made without a device put every convolution that may share a launch into one
-        g_host_batches = !(value == "0" || value == "false" || value == "off" || value.empty());
+    if (key == "host_plan_batches") {   // plans made without a device put every convolution that may share a launch into one ("2": mixed ones too)
+        g_host_batches = value == "2" ? 2 : value == "0" || value == "false" || value == "off" || value.empty() ? 0 : 1;
         return true;
     }
     if (key == "thin_conv_min_pixels") {
@@ -1326,7 +1396,7 @@ bool planner_arena_reuse() { return g_arena_reuse; }
 long long planner_thin_conv_min_pixels() { return g_thin_conv_min_pixels; }
 int planner_host_split_k() { return g_host_split_k; }
 bool planner_batch_convs() { return g_batch_convs; }
-bool planner_host_batches() { return g_host_batches; }
+int planner_host_batches() { return g_host_batches; }
 bool planner_commute_pool_conv() { return g_commute_pool_conv; }
 
 Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches) {

@@ -95,11 +95,12 @@ struct PlanOp {
     double flops = 0.0, bytes = 0.0;
 };
 
-// Convolutions of one view through the same window that share a launch (launch_conv_batch).  They run at the beginning of their
-// stage, before its groups: an operation that the schedule puts into a later stage moves here.
+// Convolutions that share a launch: of one view through the same window (launch_conv_batch), or mixed ones (launch_conv_mixed).  They run at
+// the beginning of their stage, before its groups: an operation that the schedule puts into a later stage moves here.
 struct PlanBatch {
     int stage = 0;
     int variant = -1;
+    bool mixed = false;     // (a pool may be among its operations, the last of them)
     std::vector<int> ops;
 };
 
@@ -144,9 +145,10 @@ enum class InputUse { Resident, InParts, Once };
 // share - 1 others should occupy about 1 / share of it rather than all of it.
 typedef std::function<ConvLaunch(const ConvProblem &, int share)> LaunchChooser;
 
-// Kernel configuration on which convolutions of one input run in a launch of their own, or -1 where they are faster by themselves;
-// `share` of each as above.  `remains`: other operations of their stage lose the launch that they shared with them.
-typedef std::function<int(const std::vector<ConvProblem> &, const std::vector<int> &share, bool remains)> BatchChooser;
+// Kernel configuration on which convolutions of one input (`mixed`: of any inputs and windows) run in a launch of their own, or -1 where
+// they are faster by themselves; `share` of each as above.  `remains`: other operations of their stage lose the launch that they shared
+// with them.  `pool`: it runs beside mixed convolutions.
+typedef std::function<int(const std::vector<ConvProblem> &, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool)> BatchChooser;
 
 // Compile a document.  `extra` is the input-shape document of stage mode ({name: [C, H, W]}).
 // Throws std::runtime_error on malformed documents, unknown operator types, non-topological schedules
@@ -165,7 +167,7 @@ bool planner_arena_reuse();
 long long planner_thin_conv_min_pixels();
 int planner_host_split_k();   // option host_plan_split_k
 bool planner_batch_convs();     // option batch_convs (default 1)
-bool planner_host_batches();    // option host_plan_batches
+int planner_host_batches();     // option host_plan_batches
 bool planner_commute_pool_conv();   // option commute_pool_conv (default 1): see PlanConv::linear
 
 }  // namespace ios

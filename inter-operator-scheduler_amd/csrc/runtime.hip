@@ -167,7 +167,7 @@ void DeviceContext::load_tune_cache() {
             const std::string name = text.substr(tab + 1);
             int variant = name == "none" ? -1 : -2;
             for (int i = 0; i < conv_num_variants(); i++)
-                if (name == conv_variant(i).name && conv_variant_batches(i)) variant = i;
+                if (name == conv_variant(i).name && (conv_variant_batches(i) || conv_variant_mixes(i))) variant = i;
             if (variant >= -1) batched[text.substr(0, tab)] = variant;   // (whether it serves the shapes is seen when it is asked for)
             continue;
         }
@@ -462,19 +462,49 @@ static WorkItem conv_work_item(const ConvDispatch &d) {
     return item;
 }
 
+// a configuration that a launch of these convolutions may be measured on
+bool DeviceContext::serves_batch(const std::vector<ConvProblem> &problems, int variant, bool mixed) const {
+    if (conv_variant(variant).precision != precision_ || !(mixed ? conv_variant_mixes(variant) : conv_variant_batches(variant))) return false;
+    for (const ConvProblem &p : problems)
+        if (!(mixed ? conv_mixable(p, variant) : conv_variant_precise(p, variant))) return false;
+    return true;
+}
+
 // Both ways on scratch tensors of the real shapes: every convolution as it runs without a batch (beside the others where one of them
 // shares its stage), and all of them in a launch on every configuration that has such a kernel.
-int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains) {
-    const ConvProblem &p = problems[0];
+int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool) {
     const size_t count = problems.size();
     bool parallel = false;
     for (int s : share) parallel = parallel || s > 1;
+    if (mixed && parallel && !fused_executor()) return -1;   // (they run beside each other, on streams)
     std::vector<ConvLaunch> alone;
     for (size_t i = 0; i < count; i++) alone.push_back(choose_launch(problems[i], share[i]));
-    TensorView x;
-    x.C = p.IC; x.H = p.H; x.W = p.W; x.pstride = padded_channels(p.IC);
-    x.ptr = tuning_buffer(0, (size_t)p.B * p.H * p.W * x.pstride + 64);
-    std::vector<TensorView> y(count);
+    std::vector<TensorView> x(count), y(count);
+    std::vector<size_t> x_at(count);
+    size_t x_floats = 0;
+    for (size_t i = 0; i < count; i++) {
+        const ConvProblem &p = problems[i];
+        x[i].C = p.IC; x[i].H = p.H; x[i].W = p.W; x[i].pstride = padded_channels(p.IC);
+        if (!mixed && i > 0) continue;   // (one input)
+        x_at[i] = x_floats;
+        x_floats += ((size_t)p.B * p.H * p.W * x[i].pstride + 64 + 63) & ~size_t(63);
+    }
+    MixedPool beside{};
+    size_t pool_x_at = 0, pool_y_at = 0;
+    if (pool != nullptr) {
+        beside.p = *pool;
+        beside.x.C = beside.y.C = pool->C;
+        beside.x.H = pool->H; beside.x.W = pool->W; beside.y.H = pool->OH; beside.y.W = pool->OW;
+        beside.x.pstride = beside.y.pstride = padded_channels(pool->C);
+        pool_x_at = x_floats;
+        x_floats += ((size_t)pool->B * pool->H * pool->W * beside.x.pstride + 64 + 63) & ~size_t(63);
+        pool_y_at = x_floats;
+        x_floats += ((size_t)pool->B * pool->OH * pool->OW * beside.y.pstride + 64 + 63) & ~size_t(63);
+    }
+    float *x_memory = tuning_buffer(0, x_floats);
+    beside.x.ptr = x_memory + pool_x_at;
+    beside.y.ptr = x_memory + pool_y_at;
+    for (size_t i = 0; i < count; i++) x[i].ptr = x_memory + x_at[i];
     std::vector<size_t> y_at(count), packed_at(count), filters_at(count), ws_at(count), ctr_at(count);
     size_t y_floats = 0, floats = 0, ws_floats = 0, counters = 0, items_at = 0;
     for (size_t i = 0; i < count; i++) {
@@ -492,7 +522,7 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
         counters += conv_counter_count(q, alone[i]);
     }
     items_at = floats;
-    floats += (count * sizeof(WorkItem) + sizeof(float) - 1) / sizeof(float);
+    floats += ((count + 1) * sizeof(WorkItem) + sizeof(float) - 1) / sizeof(float);
     float *y_memory = tuning_buffer(1, y_floats), *memory = tuning_buffer(2, floats), *workspace = ws_floats ? tuning_buffer(3, ws_floats) : nullptr;
     unsigned *tickets = tuning_counters(counters);
     hipStream_t stream = streams_[0];
@@ -527,7 +557,7 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
     bool wide = false;
     for (size_t i = 0; i < count; i++) {
         launch_pack_filters(problems[i], alone[i], memory + filters_at[i], memory + packed_at[i], stream);
-        const ConvDispatch d = make_conv_dispatch(problems[i], alone[i], x, memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
+        const ConvDispatch d = make_conv_dispatch(problems[i], alone[i], x[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
                                                   workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr));
         if (!parallel || !fused_executor() || !conv_variant(d.variant).fusable() || d.has_reduce) {
             single.push_back(i);
@@ -542,32 +572,46 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
         wide = wide || conv_variant(d.variant).needs_wide();
         items.push_back(item);
     }
+    if (pool != nullptr && !items.empty()) {
+        WorkItem item;
+        memset(&item, 0, sizeof(item));
+        item.kind = WORK_POOL;
+        item.pool = make_pool_args(beside.p, beside.x, beside.y, false, &item.num_blocks);
+        item.num_blocks = std::max(1, (item.num_blocks * 256 + threads - 1) / threads);
+        item.threads = threads;
+        item.first_block = blocks;
+        header.first_block[items.size()] = blocks;
+        blocks += item.num_blocks;
+        items.push_back(item);
+    }
+    const bool pool_alone = pool != nullptr && items.empty();
     if (wide && threads > 512) return -1;   // (a level of such operators is not one launch: see build_fused)
     header.num_items = (int)items.size();
     WorkItem *device_items = reinterpret_cast<WorkItem *>(memory + items_at);
     if (!items.empty()) stage_.upload(device_items, items.data(), items.size() * sizeof(WorkItem), stream);
     const float apart = measure(kReps, (int)single.size() + 1, [&] {
+        if (pool_alone) launch_pool(beside.p, beside.x, beside.y, stream);
         if (!items.empty()) launch_fused(threads, device_items, items.data(), header, blocks, smem_bytes, num_cus_, stream);
         for (size_t i : single)
-            launch_conv_mfma(problems[i], alone[i], x, memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
+            launch_conv_mfma(problems[i], alone[i], x[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
                              workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr), stream);
     });
     // together
     float best = 1e30f;
     int variant = -1;
     std::vector<ConvBatchMember> members(count);
-    for (size_t i = 0; i < count; i++) members[i] = {problems[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i]};
+    for (size_t i = 0; i < count; i++) members[i] = {problems[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], x[i], y[i]};
     bool packed = false;
     for (int v = 0; v < conv_num_variants(); v++) {
-        if (!conv_variant_batches(v) || conv_variant(v).precision != precision_) continue;
-        bool precise = true;
-        for (const ConvProblem &q : problems) precise = precise && conv_variant_precise(q, v);
-        if (!precise) continue;
+        if (!serves_batch(problems, v, mixed)) continue;
         ConvLaunch l;
         l.variant = v;
         for (size_t i = 0; i < count && !packed; i++) launch_pack_filters(problems[i], l, memory + filters_at[i], memory + packed_at[i], stream);
         packed = true;   // (they all read the same layout)
-        const float ms = measure(kReps, 1, [&] { launch_conv_batch(members.data(), (int)count, v, x, stream); });
+        const float ms = measure(kReps, 1, [&] {
+            if (mixed) launch_conv_mixed(members.data(), (int)count, pool != nullptr ? &beside : nullptr, v, stream);
+            else launch_conv_batch(members.data(), (int)count, v, stream);
+        });
         if (ms < best) {
             best = ms;
             variant = v;
@@ -578,22 +622,28 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
     return best + (remains ? kLaunchMs : 0.f) < kNoise * apart ? variant : -1;
 }
 
-int DeviceContext::choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains) {
-    if (forced_variant_ >= 0) return forced_split_k_ <= 1 && conv_variant_batches(forced_variant_) ? forced_variant_ : -1;
+int DeviceContext::choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool) {
+    if (forced_variant_ >= 0) {
+        const bool serves = mixed ? serves_batch(problems, forced_variant_, true) : conv_variant_batches(forced_variant_);
+        return forced_split_k_ <= 1 && serves ? forced_variant_ : -1;
+    }
     if (!autotune_ || forced_split_k_ > 0) return -1;
-    std::string key = settings_token() + (precision_ == PREC_BF16 ? " bf16" : precision_ == PREC_FP16 ? " fp16" : "") + (remains ? " remains" : "");
+    std::string key = (mixed ? "mixed " : "") + settings_token() + (precision_ == PREC_BF16 ? " bf16" : precision_ == PREC_FP16 ? " fp16" : "") + (remains ? " remains" : "");
     for (size_t i = 0; i < problems.size(); i++) key += " | " + conv_signature(problems[i]) + " " + std::to_string(share[i]);
+    if (pool != nullptr) {
+        key += " | pool";
+        for (int n : {pool->C, pool->H, pool->W, pool->KH, pool->KW, pool->sh, pool->sw, pool->ph, pool->pw, pool->is_max})
+            key += ' ' + std::to_string(n);
+    }
     auto it = batched.find(key);
     if (it != batched.end() && it->second >= 0) {   // (a saved choice that would not be measured here: written by a build that had other kernels)
-        bool serves = conv_variant(it->second).precision == precision_;
-        for (const ConvProblem &p : problems) serves = serves && conv_variant_precise(p, it->second);
-        if (!serves) {
+        if (!serves_batch(problems, it->second, mixed)) {
             batched.erase(it);
             it = batched.end();
         }
     }
     if (it == batched.end()) {
-        it = batched.emplace(key, tune_batch(problems, share, remains)).first;
+        it = batched.emplace(key, tune_batch(problems, share, remains, mixed, pool)).first;
         FILE *f = tune_cache_path_.empty() ? nullptr : fopen(tune_cache_path_.c_str(), "a");
         if (f != nullptr) {
             fprintf(f, "batch\t%s\t%s\n", key.c_str(), it->second >= 0 ? conv_variant(it->second).name : "none");
@@ -936,10 +986,16 @@ TensorView Session::part_of(const ViewRef &whole_view, const ViewRef &part_view,
 
 void Session::launch_batch(const PlanBatch &batch, int first, int images) {
     ConvBatchMember members[kMaxConvBatch];
-    TensorView in;
     int count = 0;
+    MixedPool pool{};
     for (int index : batch.ops) {
         const PlanOp &op = plan_.ops[index];
+        if (op.kind == OpKind::Pool) {
+            pool = {op.pool, part_of(op.in, op.part_in, op.part_in_whole, first, images), part_of(op.out, op.part_out, op.part_out_whole, first, images),
+                    op.bias_conv >= 0 ? base_ + plan_.convs[op.bias_conv].bias_off : nullptr, op.act};
+            if (images > 0) pool.p.B = images;
+            continue;
+        }
         const PlanConv &c = plan_.convs[op.conv];
         ConvBatchMember &m = members[count++];
         m.p = c.problem;
@@ -948,9 +1004,10 @@ void Session::launch_batch(const PlanBatch &batch, int first, int images) {
         m.filters = base_ + c.weight_off;
         m.bias = bias_of(c);
         m.y = part_of(op.out, op.part_out, op.part_out_whole, first, images);
-        in = part_of(op.in, op.part_in, op.part_in_whole, first, images);
+        m.x = part_of(op.in, op.part_in, op.part_in_whole, first, images);
     }
-    launch_conv_batch(members, count, batch.variant, in, ctx_.stream(0));
+    if (batch.mixed) launch_conv_mixed(members, count, pool.x.ptr != nullptr ? &pool : nullptr, batch.variant, ctx_.stream(0));
+    else launch_conv_batch(members, count, batch.variant, ctx_.stream(0));
 }
 
 void Session::launch_batches(size_t stage, int first, int images) {
@@ -1413,8 +1470,10 @@ void Session::advance() {
     for (; next_stage_ < plan_.stages.size(); next_stage_++) {
         for (const PlanBatch &batch : plan_.batches)
             if (batch.stage == (int)next_stage_)
-                for (int op : batch.ops)
-                    if (!packed_[plan_.ops[op].conv]) return;
+                for (int op : batch.ops) {
+                    const int conv = plan_.ops[op].conv >= 0 ? plan_.ops[op].conv : plan_.ops[op].bias_conv;
+                    if (conv >= 0 && !packed_[conv]) return;
+                }
         for (const auto &group : plan_.stages[next_stage_])
             for (int op : group)
                 if (plan_.ops[op].conv >= 0 && !packed_[plan_.ops[op].conv]) return;
@@ -1557,7 +1616,7 @@ std::vector<Session::LaunchRecord> Session::launches() {
             if (plan_.batches[b].stage != (int)s) continue;
             LaunchRecord r;
             r.stage = (int)s;
-            r.kernel = std::string("conv_batch_kernel<") + conv_variant(plan_.batches[b].variant).name + ">";
+            r.kernel = std::string(plan_.batches[b].mixed ? "conv_mixed_kernel<" : "conv_batch_kernel<") + conv_variant(plan_.batches[b].variant).name + ">";
             r.ops = plan_.batches[b].ops;
             r.batch = (int)b;
             out.push_back(r);
