@@ -44,17 +44,17 @@ struct ConvPipe {
 
     // Two terms: one limit for the inputs of the tile, by those of its first stage.  Where that does not serve all of them, the tile is
     // computed again.  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to 100
-    // registers.  And a third time, PLAIN, for inputs that need neither a ReLU nor channels masked: what a tile with nothing beside it on its
+    // registers.  And once more, PLAIN, for inputs that need neither a ReLU nor channels masked: what a tile with nothing beside it on its
     // compute unit waits for is the sum of its steps (768 -> 192 on 17 x 17, a block of 64 x 128, per 16 k: 230 cycles for the operands from LDS, 320 for the
     // matrix instructions, 450 to split an octet, 250 to store and for the barrier), and without the branches between them the split work lies
     // under the matrix instructions.  That layer at batch 3 23.6 -> 21.7 us, at batch 64 31.8 -> 29.0; four such convolutions in a launch, 704 outputs,
-    // batch 16 31.6 -> 29.2, batch 64 94.2 -> 92.2.
+    // batch 16 31.6 -> 29.2, batch 64 94.2 -> 92.2.  With one term the matrix work is a third of that and the two ways out of each test cost as much as the
+    // conversion: passes of Inception-v3 in half at batch 7 660 -> 619 us, in bfloat16 at batch 64 2298 -> 2248.
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
-        bool plain = false;
-        if constexpr (TERMS == 2) plain = a.pre_relu == 0 && (POINT ? a.ICg % BK == 0 : (a.ICg & 3) == 0);
+        const bool plain = a.pre_relu == 0 && (POINT ? a.ICg % BK == 0 : (a.ICg & 3) == 0);
         unsigned limit;
-        if (plain) limit = attempt<RES, true, TERMS == 2>(a, smem, tile, g, z, kNoLimit);
+        if (plain) limit = attempt<RES, true, true>(a, smem, tile, g, z, kNoLimit);
         else limit = attempt<RES, true, false>(a, smem, tile, g, z, kNoLimit);
         if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES, false, false>(a, smem, tile, g, z, limit);
     }
@@ -195,7 +195,12 @@ struct ConvPipe {
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
             float v[8];
-            octet_of(br[i], left, v);
+            if constexpr (PLAIN) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = br[i][j >> 2][j & 3];
+            } else {
+                octet_of(br[i], left, v);
+            }
             if constexpr (TERMS == 2) {
                 watch.octet(octet_peak(v), limit);
                 split_half2(v, limit_scale(limit), hi[i], lo[i]);
@@ -247,7 +252,7 @@ struct ConvPipe {
             const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
             const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
             // operands of the next unit are read ahead of a unit's matrix work, where registers allow it
-            constexpr int TURN = PLAIN && KU > 1 && TMW * TNW != 2 ? 1 : 0;
+            constexpr int TURN = PLAIN && TERMS == 2 && KU > 1 && TMW * TNW != 2 ? 1 : 0;
             uintx4 av[TURN + 1][TERMS][TM], bv[TURN + 1][TERMS][TN];
             auto read_unit = [&](int u) {
 #pragma unroll
@@ -260,7 +265,7 @@ struct ConvPipe {
             };
             const uintx4 (&ar)[A_IT] = a_reg[(s + 1) % PD];
             const floatx4 (&br)[B_IT][2] = b_reg[(s + 1) % PD];
-            if constexpr (PLAIN) {
+            if constexpr (PLAIN && TERMS == 2) {
                 // The octets of the next stage are split between the matrix instructions of this one, a pair of values at a time.
                 constexpr int SLOTS = 3 * TM * TN * KU, PIECES = 5 * B_IT;
                 uintx4 hi[B_IT], lo[B_IT];
