@@ -26,7 +26,9 @@ extern "C" {
  * Latency of a whole graph under its schedule.  Replaces graph_latency (src/ios/ios_runtime.cu:1480-1484).
  * results[repeat]: milliseconds per forward pass, each the mean of `number` individually timed passes.
  * stage_results[repeat * num_stages] (row-major, caller-zeroed): per-stage milliseconds, written only when
- * profile_stage_latency != 0; num_stages = total number of stages over all blocks.
+ * profile_stage_latency != 0; num_stages = total number of stages over all blocks.  A pass whose stages are timed
+ * runs every operator in the stage that the schedule gives it: convolutions of different stages share no launch in it
+ * (see option "batch_convs"), so that it may take longer than one that is timed as a whole.
  */
 int graph_latency(const char *graph_json, int batch_size, int warmup, int number, int repeat,
                   int profile_stage_latency, float *results, float *stage_results);
@@ -122,7 +124,9 @@ const char *ios_last_error(void);
  *       block) share a launch where a measurement finds that faster (with "autotune" = "1"; pinned configurations that have such a
  *       kernel always).  They then run in the stage of the first of them; the same results bit for bit as apart on the same
  *       configuration.  Convolutions that the groups of a stage begin with, and those of one view through different windows, share
- *       launches by the same rule, and a pool beside them goes along.  "host_plan_batches" = "0" (default) | "1" | "2": plans made
+ *       launches by the same rule, and a pool beside them goes along.  "batch_across_stages" = "1" (default) | "0": the former may
+ *       lie in different stages of the schedule (also of one that was searched with stage_latency, which sees a stage at a time)
+ *       | only within one.  "host_plan_batches" = "0" (default) | "1" | "2": plans made
  *       without a device batch the former ("1") or both ("2") wherever they may;
  *   "host_threads" = N: threads that share a large copy between a caller's arrays and pinned memory, the caller among them
  *       (12 at most; 1: the caller alone).  "0" (default): three quarters of the processors the process is bound to or that its

@@ -54,7 +54,9 @@ int latency_call(ios::PlanMode mode, const char *doc_json, const char *extra_jso
         const ios::Json doc = ios::Json::parse(doc_json);
         ios::Json extra;
         if (extra_json != nullptr) extra = ios::Json::parse(extra_json);
-        ios::Plan plan = ios::build_plan(mode, doc, extra_json ? &extra : nullptr, batch_size, device_chooser(), ios::InputUse::Resident, device_batches());
+        // (the time of a stage is that of its own operations: none of them moves into another stage's launch)
+        ios::Plan plan = ios::build_plan(mode, doc, extra_json ? &extra : nullptr, batch_size, device_chooser(), ios::InputUse::Resident, device_batches(),
+                                         /*across_stages=*/profile_stage_latency == 0);
         ios::Session session(std::move(plan), /*shared=*/true);
         if (mode == ios::PlanMode::Stage) {
             if (profile_stage_latency) throw std::runtime_error("stage_latency cannot profile stages (profile_stage_latency must be 0)");

@@ -79,8 +79,8 @@ int act_code(const std::string &name) {
 
 class Planner {
 public:
-    Planner(int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches)
-        : batch_(batch), input_use_(input), chooser_(chooser), batch_chooser_(batches) {
+    Planner(int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches, bool across_stages)
+        : batch_(batch), input_use_(input), chooser_(chooser), batch_chooser_(batches), across_stages_(across_stages) {
         if (batch < 1) throw std::runtime_error("batch size must be positive");
         plan_.batch = batch;
     }
@@ -714,6 +714,7 @@ private:
         for (const PlanOp &op : plan_.ops) {
             touch(op.in.offset, op.stage);
             touch(op.out.offset, op.stage);
+            touch(op.in.offset, op.scheduled_stage());   // (a pass whose stages are timed runs it there)
             for (const ViewRef &v : op.srcs) touch(v.offset, op.stage);
             if (op.has_residual) touch(op.residual.offset, op.stage);
             if (op.conv >= 0 && plan_.convs[op.conv].ws_floats > 0) touch(plan_.convs[op.conv].ws_off, op.stage);
@@ -1167,7 +1168,7 @@ private:
             if (op.kind != OpKind::ConvMfma || op.has_residual || !plan_.convs[op.conv].matrix_path) continue;
             const ConvProblem &p = plan_.convs[op.conv].problem;
             if (!conv_batchable(p, p)) continue;
-            readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W, p.sh, p.sw, p.ph, p.pw}].push_back((int)i);
+            readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W, p.sh, p.sw, p.ph, p.pw, within(op)}].push_back((int)i);
         }
         for (auto &entry : readers) {
             const std::vector<int> ops = behind_their_view(entry.second);
@@ -1212,7 +1213,7 @@ private:
         std::map<std::vector<long long>, std::vector<int>> readers;
         for (size_t i = 0; i < plan_.ops.size(); i++) {
             const PlanOp &op = plan_.ops[i];
-            if (may_share(op, share)) readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W}].push_back((int)i);
+            if (may_share(op, share)) readers[{(long long)op.in.base, op.in.first, op.in.pstride, op.in.C, op.in.H, op.in.W, within(op)}].push_back((int)i);
         }
         for (auto &entry : readers) {
             const std::vector<int> ops = behind_their_view(entry.second);
@@ -1222,6 +1223,9 @@ private:
             }
         }
     }
+
+    // what operations have in common that may share a launch: nothing, or their stage
+    int within(const PlanOp &op) const { return across_stages_ ? 0 : op.stage; }
 
     // of operations that read one view: those of later stages than the last that writes into it, by stage
     std::vector<int> behind_their_view(std::vector<int> ops) const {
@@ -1269,6 +1273,10 @@ private:
             PlanOp &op = plan_.ops[i];
             auto &group = plan_.stages[op.stage][op.group];
             group.erase(std::find(group.begin(), group.end(), i));
+            if (op.stage != batch.stage) {
+                batch.across_stages = true;
+                op.moved_from = op.stage;
+            }
             op.stage = batch.stage;
             op.batch = (int)plan_.batches.size();
             if (op.conv < 0) continue;
@@ -1323,6 +1331,7 @@ private:
     int level_unit_ = -2, level_base_ = 0, level_top_ = 0;   // PlanOp::level of the operations being emitted
     const LaunchChooser &chooser_;
     const BatchChooser &batch_chooser_;
+    const bool across_stages_;   // operations of different stages may share a launch
     Plan plan_;
     std::vector<PNode> nodes_;
     std::map<std::string, int> by_name_;
@@ -1359,6 +1368,7 @@ long long g_thin_conv_min_pixels = 1LL << 18;
 int g_host_split_k = 0;
 bool g_commute_pool_conv = true;
 bool g_batch_convs = true;
+bool g_batch_across_stages = true;
 int g_host_batches = 0;
 }
 
@@ -1373,6 +1383,10 @@ bool set_planner_option(const std::string &key, const std::string &value) {
     }
     if (key == "batch_convs") {
         g_batch_convs = !(value == "0" || value == "false" || value == "off" || value.empty());
+        return true;
+    }
+    if (key == "batch_across_stages") {
+        g_batch_across_stages = !(value == "0" || value == "false" || value == "off" || value.empty());
         return true;
     }
     if (key == "host_plan_batches") {   // plans made without a device put every convolution that may share a launch into one ("2": mixed ones too)
@@ -1399,8 +1413,9 @@ bool planner_batch_convs() { return g_batch_convs; }
 int planner_host_batches() { return g_host_batches; }
 bool planner_commute_pool_conv() { return g_commute_pool_conv; }
 
-Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches) {
-    Planner planner(batch, chooser, mode == PlanMode::Graph ? input : InputUse::Resident, batches);
+Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input, const BatchChooser &batches,
+                bool across_stages) {
+    Planner planner(batch, chooser, mode == PlanMode::Graph ? input : InputUse::Resident, batches, across_stages && g_batch_across_stages);
     return planner.run(mode, doc, extra);
 }
 
@@ -1436,6 +1451,7 @@ std::string describe_plan(const Plan &plan) {
         if (op.conv >= 0 && plan.convs[op.conv].linear) os << ",\"linear\":true";
         if (op.has_residual) os << ",\"residual\":true,\"post_relu\":" << op.post_relu;
         if (op.batch >= 0) os << ",\"batch\":" << op.batch;
+        if (op.moved_from >= 0) os << ",\"scheduled_stage\":" << op.moved_from;
         os << ",\"level\":" << op.level;
         // arena extents in floats, one [begin, end) per image: what the operation writes and what it reads
         auto ranges = [&](const char *key, const std::vector<ViewRef> &views) {

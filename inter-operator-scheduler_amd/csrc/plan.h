@@ -92,6 +92,8 @@ struct PlanOp {
     ViewRef part_in, part_out;
     bool part_in_whole = true, part_out_whole = true;
     int batch = -1;       // index into Plan::batches
+    int moved_from = -1;  // its stage in the schedule, where a batch takes it ahead
+    int scheduled_stage() const { return moved_from >= 0 ? moved_from : stage; }
     double flops = 0.0, bytes = 0.0;
 };
 
@@ -101,6 +103,7 @@ struct PlanBatch {
     int stage = 0;
     int variant = -1;
     bool mixed = false;     // (a pool may be among its operations, the last of them)
+    bool across_stages = false;   // the schedule puts some of them into later stages
     std::vector<int> ops;
 };
 
@@ -153,8 +156,9 @@ typedef std::function<int(const std::vector<ConvProblem> &, const std::vector<in
 // Compile a document.  `extra` is the input-shape document of stage mode ({name: [C, H, W]}).
 // Throws std::runtime_error on malformed documents, unknown operator types, non-topological schedules
 // and stages with too many groups.
+// across_stages: convolutions of different stages may share a launch (as far as option batch_across_stages allows it).
 Plan build_plan(PlanMode mode, const Json &doc, const Json *extra, int batch, const LaunchChooser &chooser, InputUse input = InputUse::Resident,
-                const BatchChooser &batches = nullptr);
+                const BatchChooser &batches = nullptr, bool across_stages = true);
 
 std::string describe_plan(const Plan &plan);   // JSON array, one object per op
 

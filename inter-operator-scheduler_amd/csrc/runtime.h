@@ -194,11 +194,12 @@ private:
     TensorView part_of(const ViewRef &whole_view, const ViewRef &part_view, bool whole, int first, int images) const;
     void launch_batch(const PlanBatch &batch, int first = 0, int images = 0);   // on the main stream
     void launch_batches(size_t stage, int first = 0, int images = 0);           // those at the beginning of a stage
+    void launch_scheduled_batches(size_t stage);
     unsigned *counters_of(const PlanConv &c) const;
     const float *bias_of(const PlanConv &c) const { return base_ + (c.linear ? c.zero_bias_off : c.bias_off); }
     void ready_executor();
     void enqueue(size_t first, bool stage_events);   // issue the stages from `first` on according to the execution mode
-    void enqueue_stage(size_t s);
+    void enqueue_stage(size_t s, bool timed = false);
     void enqueue_stage_streams(size_t s);
     void enqueue_stage_fused(size_t s);
     void enqueue_stage_serial(size_t s);

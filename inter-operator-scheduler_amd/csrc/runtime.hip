@@ -1015,6 +1015,18 @@ void Session::launch_batches(size_t stage, int first, int images) {
         if (batch.stage == (int)stage) launch_batch(batch, first, images);
 }
 
+// The same where the stages are timed: what a batch would take ahead runs in the stage that the schedule gives it, by itself.
+void Session::launch_scheduled_batches(size_t stage) {
+    for (const PlanBatch &batch : plan_.batches) {
+        if (!batch.across_stages) {
+            if (batch.stage == (int)stage) launch_batch(batch);
+            continue;
+        }
+        for (int op : batch.ops)
+            if (plan_.ops[op].scheduled_stage() == (int)stage) launch_op(plan_.ops[op], 0);
+    }
+}
+
 void Session::launch_op(const PlanOp &op, int group, int first, int images) {
     hipStream_t stream = ctx_.stream(group);
     const int count = images > 0 ? images : plan_.batch;
@@ -1093,8 +1105,9 @@ void Session::enqueue_stage_serial(size_t s) {
         for (int op : group) launch_op(plan_.ops[op], 0);
 }
 
-void Session::enqueue_stage(size_t s) {
-    launch_batches(s);
+void Session::enqueue_stage(size_t s, bool timed) {
+    if (timed) launch_scheduled_batches(s);
+    else launch_batches(s);
     if (static_) enqueue_stage_serial(s);
     else if (ctx_.fused_executor()) enqueue_stage_fused(s);
     else enqueue_stage_streams(s);
@@ -1112,7 +1125,7 @@ void Session::enqueue(size_t first, bool stage_events) {
     if (static_ && stage_events) throw std::runtime_error("a session in the static scratch cannot profile stages");
     ready_executor();
     for (size_t s = first; s < plan_.stages.size(); s++) {
-        enqueue_stage(s);
+        enqueue_stage(s, stage_events);
         if (stage_events) IOS_HIP(hipEventRecord(stage_events_[s], ctx_.stream(0)));
     }
 }
