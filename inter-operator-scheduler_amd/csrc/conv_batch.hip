@@ -4,10 +4,11 @@
 
 namespace ios {
 
-#define IOS_PIPE3_BATCH(IDX, NAME, ...) conv_batch_kernel<ConvPipe<2, true, __VA_ARGS__, true>>,
-#define IOS_PIPE_BF16_BATCH(IDX, NAME, ...) conv_batch_kernel<ConvPipe<1, false, __VA_ARGS__, true>>,
-#define IOS_PIPE_FP16_BATCH(IDX, NAME, ...) conv_batch_kernel<ConvPipe<1, true, __VA_ARGS__, true>>,
-extern const ConvBatchKernelFn kPipeBatchKernels[] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_BATCH) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_BATCH)
+#define IOS_BATCH(...) {conv_batch_kernel<ConvPipe<__VA_ARGS__, true, false>>, conv_batch_kernel<ConvPipe<__VA_ARGS__, true, true>>},
+#define IOS_PIPE3_BATCH(IDX, NAME, ...) IOS_BATCH(2, true, __VA_ARGS__)
+#define IOS_PIPE_BF16_BATCH(IDX, NAME, ...) IOS_BATCH(1, false, __VA_ARGS__)
+#define IOS_PIPE_FP16_BATCH(IDX, NAME, ...) IOS_BATCH(1, true, __VA_ARGS__)
+extern const ConvBatchKernelFn kPipeBatchKernels[][2] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_BATCH) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_BATCH)
                                                           IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_BATCH)};
 
 }  // namespace ios

@@ -38,6 +38,8 @@ __global__ __launch_bounds__(Body::THREADS) __attribute__((amdgpu_waves_per_eu(w
 // alone, 64 x 64 tiles of 768 -> 192 channels on 17 x 17 take 16 us at batch 3 as at batch 7.  Four such convolutions together put three to
 // seven blocks on a compute unit instead of one or two: 27 -> 12 us (half, batch 7), 41 -> 19 us (bfloat16, batch 16), 133 -> 99 us (fp32, batch 64: 606
 // TFLOP/s of half products).
+// Six of the two-term kernels (64 x 128 and 128 x 64 outputs) keep 16 bytes a lane in scratch memory over the sums' tests: two stores and
+// two loads per tile behind its K loop, for the fourth wavefront on a SIMD.
 struct ConvBatchArgs {
     int xcd_q, xcd_r, tile_div, weights_major;   // as in ConvKernelArgs, of all members' tiles
     FastDiv div_tile;
@@ -45,7 +47,7 @@ struct ConvBatchArgs {
     ConvKernelArgs item[kMaxConvBatch];          // (numbered by rows of tiles of channels, without XCDs)
 };
 typedef void (*ConvBatchKernelFn)(ConvBatchArgs);
-extern const ConvBatchKernelFn kPipeBatchKernels[];   // conv_batch.hip, in the order of conv_pipe.h
+extern const ConvBatchKernelFn kPipeBatchKernels[][2];   // conv_batch.hip, in the order of conv_pipe.h; [1]: all members PLAIN
 template <typename Body>
 __global__ __launch_bounds__(Body::THREADS) __attribute__((amdgpu_waves_per_eu(waves_per_simd<Body>::value))) void conv_batch_kernel(ConvBatchArgs b) {
     extern __shared__ floatx4 conv_smem[];

@@ -75,7 +75,7 @@ struct VariantEntry {
       false, 16, false, false, PRECISION, TERMS},                                                                                     \
      kPipeKernels[IDX - kFirstPipeVariant][0], \
      ConvPipe<TERMS, HALF, KU, PD, TMW, TNW, WM, WN>::SMEM_FLOATS,                                                                   \
-     {kPipeKernels[IDX - kFirstPipeVariant][1], {}}},
+     {kPipeKernels[IDX - kFirstPipeVariant][1], kPipePlainKernels[IDX - kFirstPipeVariant][0], kPipePlainKernels[IDX - kFirstPipeVariant][1]}},
 #define IOS_PIPE3_ENTRY(...) IOS_PIPE_ENTRY(2, true, PREC_FP32, __VA_ARGS__)
 #define IOS_PIPE_BF16_ENTRY(...) IOS_PIPE_ENTRY(1, false, PREC_BF16, __VA_ARGS__)
 #define IOS_PIPE_FP16_ENTRY(...) IOS_PIPE_ENTRY(1, true, PREC_FP16, __VA_ARGS__)
@@ -397,8 +397,13 @@ ConvDispatch make_conv_dispatch(const ConvProblem &p, const ConvLaunch &l, const
     return d;
 }
 
+// Pipelined kernels: inputs that need neither a ReLU nor channels masked, for kernels of 1 x 1 filters (`point`) in whole stages, for others in
+// whole quads
+static bool pipe_plain(const ConvProblem &p, const VariantEntry &e, bool point) { return p.pre_relu == 0 && p.ICg() % (point ? e.v.BK : 4) == 0; }
+
 // Which of an entry's kernels serves the problem: 0 any, else the special ones.  Pipelined kernels: [1] 1 x 1 filters without groups,
-// whose addresses stay the same over K (at batch 64 768 -> 192 on 17 x 17 39.7 -> 34.8 us, 2048 -> 320 on 8 x 8 51.2 -> 43.1).  Window kernels:
+// whose addresses stay the same over K (at batch 64 768 -> 192 on 17 x 17 39.7 -> 34.8 us, 2048 -> 320 on 8 x 8 51.2 -> 43.1), [2] and [3] any filter
+// and these where pipe_plain holds.  Window kernels:
 // [1] seven taps, [2] nine (see known_chunk; other numbers are rare, 1 x 3 and 5 x 5), [3] and [4] the same where the window fits three rounds.
 static int kernel_of(const ConvProblem &p, const VariantEntry &e) {
     const int taps = p.KH * p.KW;
@@ -406,7 +411,9 @@ static int kernel_of(const ConvProblem &p, const VariantEntry &e) {
         const int known = taps == 7 ? 1 : taps == 9 ? 2 : 0;
         return known != 0 && window_span(p, e.v.BN) <= short_rounds(INT_MAX) * (e.v.threads() / 2) ? known + 2 : known;
     }
-    return e.special[0].kernel != nullptr && taps == 1 && p.groups == 1 ? 1 : 0;
+    if (e.special[0].kernel == nullptr) return 0;
+    const int point = taps == 1 && p.groups == 1 ? 1 : 0;
+    return pipe_plain(p, e, point != 0) ? 2 + point : point;
 }
 
 void launch_conv_mfma(const ConvProblem &p, const ConvLaunch &l, const TensorView &x, const float *packed, const float *filters,
@@ -446,7 +453,7 @@ void launch_conv_batch(const ConvBatchMember *members, int count, int variant, h
     ConvLaunch l;
     l.variant = variant;
     ConvBatchArgs b;
-    int tiles_m = 0, tiles_n = 0, threads = 0, smem_bytes = 0;
+    int tiles_m = 0, tiles_n = 0, threads = 0, smem_bytes = 0, plain = 1;
     double filters = 0.0;
     for (int i = 0; i < kMaxConvBatch; i++) {
         const ConvBatchMember &m = members[std::min(i, count - 1)];
@@ -463,6 +470,7 @@ void launch_conv_batch(const ConvBatchMember *members, int count, int variant, h
         threads = d.threads;
         smem_bytes = d.smem_bytes;
         filters += (double)m.p.OC * m.p.K();
+        plain &= pipe_plain(m.p, e, true) ? 1 : 0;
     }
     const ConvProblem &p = members[0].p;
     b.weights_major = filters > (double)p.B * p.IC * p.H * p.W ? 1 : 0;
@@ -470,13 +478,13 @@ void launch_conv_batch(const ConvBatchMember *members, int count, int variant, h
     b.div_tile = make_fast_div((unsigned)b.tile_div);
     b.xcd_q = (tiles_m * tiles_n) >> 3;
     b.xcd_r = (tiles_m * tiles_n) & 7;
-    const ConvBatchKernelFn kernel = kPipeBatchKernels[variant - kFirstPipeVariant];
+    const ConvBatchKernelFn kernel = kPipeBatchKernels[variant - kFirstPipeVariant][plain];
     if (smem_bytes > 64 * 1024) {
-        static bool raised[kNumConvVariants] = {};
-        if (!raised[variant]) {
+        static bool raised[kNumConvVariants][2] = {};
+        if (!raised[variant][plain]) {
             if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes) != hipSuccess)
                 throw std::runtime_error(std::string("conv: cannot reserve LDS for a batch on configuration ") + e.v.name);
-            raised[variant] = true;
+            raised[variant][plain] = true;
         }
     }
     hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(threads), smem_bytes, stream, b);
@@ -495,7 +503,7 @@ void launch_conv_mixed(const ConvBatchMember *members, int count, const MixedPoo
     l.variant = variant;
     ConvMixedArgs b;
     long long blocks = 0;
-    int threads = 0, smem_bytes = 0, which = -1;
+    int threads = 0, smem_bytes = 0, which = -1, plain = 1;
     for (int i = 0; i < kMaxConvBatch; i++) {
         const ConvBatchMember &m = members[std::min(i, count - 1)];
         if (!conv_mixable(m.p, variant)) throw std::runtime_error(std::string("conv: configuration ") + e.v.name + " does not take a member of a launch");
@@ -508,6 +516,7 @@ void launch_conv_mixed(const ConvBatchMember *members, int count, const MixedPoo
         smem_bytes = d.smem_bytes;
         const int here = e.v.window != 0 ? kernel_of(m.p, e) : 0;
         which = which < 0 || which == here ? here : 0;
+        plain &= pipe_plain(m.p, e, false) ? 1 : 0;
     }
     b.pool_first = INT_MAX;
     b.pool_blocks = 0;
@@ -521,11 +530,11 @@ void launch_conv_mixed(const ConvBatchMember *members, int count, const MixedPoo
     if (blocks >= INT_MAX) throw std::runtime_error("conv: grid too large");
     const int index = variant - (e.v.window != 0 ? kFirstWindowVariant : kFirstPipeVariant);
     // (windows of more than three rounds with a known number of taps are rare here: the kernel for any number serves them)
-    const ConvMixedKernelFn *kernels = e.v.window == 0 ? kPipeMixedKernels : which == 3 ? kWindow7MixedKernels : which == 4 ? kWindow9MixedKernels : kWindowMixedKernels;
-    const ConvMixedKernelFn kernel = kernels[index];
+    const ConvMixedKernelFn *windows = which == 3 ? kWindow7MixedKernels : which == 4 ? kWindow9MixedKernels : kWindowMixedKernels;
+    const ConvMixedKernelFn kernel = e.v.window != 0 ? windows[index] : kPipeMixedKernels[index][plain];
     if (smem_bytes > 64 * 1024) {
         static bool raised[kNumConvVariants][3] = {};
-        bool &done = raised[variant][which >= 3 ? which - 2 : 0];
+        bool &done = raised[variant][e.v.window == 0 ? plain : which >= 3 ? which - 2 : 0];
         if (!done) {
             if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem_bytes) != hipSuccess)
                 throw std::runtime_error(std::string("conv: cannot reserve LDS for mixed convolutions on configuration ") + e.v.name);

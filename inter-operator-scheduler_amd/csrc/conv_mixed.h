@@ -18,7 +18,8 @@ struct ConvMixedArgs {
     ConvKernelArgs item[kMaxConvBatch];
 };
 typedef void (*ConvMixedKernelFn)(ConvMixedArgs);
-extern const ConvMixedKernelFn kPipeMixedKernels[], kWindowMixedKernels[];     // conv_mixed.hip, in the order of conv_pipe.h and conv_window.h
+// conv_mixed.hip, in the order of conv_pipe.h ([1]: all members PLAIN) and conv_window.h
+extern const ConvMixedKernelFn kPipeMixedKernels[][2], kWindowMixedKernels[];
 extern const ConvMixedKernelFn kWindow7MixedKernels[], kWindow9MixedKernels[];   // conv_mixed7.hip, conv_mixed9.hip
 // (Where four wavefronts a SIMD fit, the address of the member's arguments is one value too many.)
 template <typename Body>

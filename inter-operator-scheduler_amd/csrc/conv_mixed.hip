@@ -4,10 +4,11 @@
 
 namespace ios {
 
-#define IOS_PIPE3_MIXED(IDX, NAME, ...) conv_mixed_kernel<ConvPipe<2, true, __VA_ARGS__, false>>,
-#define IOS_PIPE_BF16_MIXED(IDX, NAME, ...) conv_mixed_kernel<ConvPipe<1, false, __VA_ARGS__, false>>,
-#define IOS_PIPE_FP16_MIXED(IDX, NAME, ...) conv_mixed_kernel<ConvPipe<1, true, __VA_ARGS__, false>>,
-extern const ConvMixedKernelFn kPipeMixedKernels[] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_MIXED) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_MIXED)
+#define IOS_MIXED(...) {conv_mixed_kernel<ConvPipe<__VA_ARGS__, false, false>>, conv_mixed_kernel<ConvPipe<__VA_ARGS__, false, true>>},
+#define IOS_PIPE3_MIXED(IDX, NAME, ...) IOS_MIXED(2, true, __VA_ARGS__)
+#define IOS_PIPE_BF16_MIXED(IDX, NAME, ...) IOS_MIXED(1, false, __VA_ARGS__)
+#define IOS_PIPE_FP16_MIXED(IDX, NAME, ...) IOS_MIXED(1, true, __VA_ARGS__)
+extern const ConvMixedKernelFn kPipeMixedKernels[][2] = {IOS_PIPE3_VARIANTS(IOS_PIPE3_MIXED) IOS_PIPE_BF16_VARIANTS(IOS_PIPE_BF16_MIXED)
                                                           IOS_PIPE_FP16_VARIANTS(IOS_PIPE_FP16_MIXED)};
 
 #define IOS_WINDOW3_MIXED(IDX, NAME, ...) conv_mixed_kernel<ConvWindow<2, true, __VA_ARGS__>>,

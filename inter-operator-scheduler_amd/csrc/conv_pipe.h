@@ -19,7 +19,8 @@
 
 namespace ios {
 
-template <int TERMS, bool HALF, int KU, int PD, int TMW, int TNW, int WM, int WN, bool POINT = false>
+// POINT: 1 x 1 filters without groups.  PLAIN: inputs that need neither a ReLU nor channels masked (pipe_plain).
+template <int TERMS, bool HALF, int KU, int PD, int TMW, int TNW, int WM, int WN, bool POINT = false, bool PLAIN = false>
 struct ConvPipe {
     static_assert(TERMS == 1 || (TERMS == 2 && HALF), "one rounded term, or two terms of half");
     static constexpr int MT = 32;
@@ -29,7 +30,9 @@ struct ConvPipe {
     static constexpr int THREADS = T;
     static constexpr int CPAD = 16;
     static constexpr bool FUSABLE = false;
-    static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : 4;
+    // (stages of four units fill the LDS with two blocks: no fewer registers than three wavefronts leave, or the PLAIN form spills: 256 -> 256 3 x 3 on
+    // 14 x 14 at batch 7 38.5 -> 33.0 us)
+    static constexpr int WAVES_PER_SIMD = TERMS == 1 ? 1 : TMW * TNW >= 3 ? 2 : KU == 4 ? 3 : 4;
     static constexpr int OCT = 2 * KU;                 // octets (eight consecutive k) of a pixel or filter row in a stage
     static constexpr int B_IT = OCT * BN / T;          // pixels a thread stages, T / OCT apart
     static constexpr int A_SLOTS = OCT * TERMS * BM;   // slots of 16 bytes (eight 16-bit values)
@@ -44,23 +47,22 @@ struct ConvPipe {
 
     // Two terms: one limit for the inputs of the tile, by those of its first stage.  Where that does not serve all of them, the tile is
     // computed again.  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to 100
-    // registers.  And once more, PLAIN, for inputs that need neither a ReLU nor channels masked: what a tile with nothing beside it on its
-    // compute unit waits for is the sum of its steps (768 -> 192 on 17 x 17, a block of 64 x 128, per 16 k: 230 cycles for the operands from LDS, 320 for the
+    // registers.  The PLAIN form of the first attempt: what a tile with nothing beside it on its compute unit waits for is the sum of its steps (768 -> 192 on 17 x 17, a block of 64 x 128, per 16 k: 230 cycles for the operands from LDS, 320 for the
     // matrix instructions, 450 to split an octet, 250 to store and for the barrier), and without the branches between them the split work lies
     // under the matrix instructions.  That layer at batch 3 23.6 -> 21.7 us, at batch 64 31.8 -> 29.0; four such convolutions in a launch, 704 outputs,
     // batch 16 31.6 -> 29.2, batch 64 94.2 -> 92.2.  With one term the matrix work is a third of that and the two ways out of each test cost as much as the
     // conversion: passes of Inception-v3 in half at batch 7 660 -> 619 us, in bfloat16 at batch 64 2298 -> 2248.
+    // A kernel holds one of the two forms: both in one take the registers of the larger for either (one term, 64 x 64 outputs, any filter 106
+    // instead of 82, four wavefronts a SIMD instead of five).  Masked forms, both in one -> apart: 256 -> 256 3 x 3 behind a folded
+    // ReLU on 14 x 14, half at batch 7, 26.1 -> 23.2 us; 768 -> 192 behind one on 17 x 17, bfloat16 at batch 64, 64 x 128 outputs 22.1 -> 20.9.
     template <bool RES = false>
     __device__ static __forceinline__ void run(const ConvKernelArgs &a, float *smem, int tile, int g, int z) {
-        const bool plain = a.pre_relu == 0 && (POINT ? a.ICg % BK == 0 : (a.ICg & 3) == 0);
-        unsigned limit;
-        if (plain) limit = attempt<RES, true, true>(a, smem, tile, g, z, kNoLimit);
-        else limit = attempt<RES, true, false>(a, smem, tile, g, z, kNoLimit);
+        const unsigned limit = attempt<RES, true, PLAIN>(a, smem, tile, g, z, kNoLimit);
         if (TERMS == 2 && __builtin_expect(limit != 0, 0)) attempt<RES, false, false>(a, smem, tile, g, z, limit);
     }
 
     // limit: kNoLimit for the first attempt.  Returns the limit for another one, or 0.
-    template <bool RES, bool FIRST, bool PLAIN>
+    template <bool RES, bool FIRST, bool UNMASKED>
     __device__ static __forceinline__ unsigned attempt(const ConvKernelArgs &a, float *smem, int tile, int g, int z, unsigned limit) {
     constexpr int TM = TMW, TN = TNW, WTM = 32 * TMW, WTN = 32 * TNW;
     uintx4 *lds = reinterpret_cast<uintx4 *>(smem);
@@ -177,41 +179,50 @@ struct ConvPipe {
             for (int j = 0; j < 8; j++) v[j] = j < mine ? v[j] : 0.f;
         }
     };
-    auto store_octets = [&](int buf, const uintx4 (&ar)[A_IT], const uintx4 (&hi)[B_IT], const uintx4 (&lo)[B_IT]) {
+    auto store_filters = [&](int buf, const uintx4 (&ar)[A_IT]) {
         uintx4 *As = lds + buf * STAGE;
-        uintx4 *Bs = As + A_SLOTS + unit * (TERMS * UNIT);
 #pragma unroll
         for (int i = 0; i < A_IT; i++)
             if (A_SLOTS % T == 0 || tid + i * T < A_SLOTS) As[tid + i * T] = ar[i];
+    };
+    auto store_octet = [&](int buf, int i, const uintx4 &hi, const uintx4 &lo) {
+        uintx4 *Bs = lds + buf * STAGE + A_SLOTS + unit * (TERMS * UNIT);
+        const int slot = slot_of(tid / OCT + i * (T / OCT), half);
+        Bs[slot] = hi;
+        if constexpr (TERMS == 2) Bs[UNIT + slot] = lo;
+    };
+    auto convert = [&](const floatx4 (&br)[2], int left, uintx4 &hi, uintx4 &lo) {
+        float v[8];
+        if constexpr (UNMASKED) {
 #pragma unroll
-        for (int i = 0; i < B_IT; i++) {
-            const int slot = slot_of(tid / OCT + i * (T / OCT), half);
-            Bs[slot] = hi[i];
-            if constexpr (TERMS == 2) Bs[UNIT + slot] = lo[i];
+            for (int j = 0; j < 8; j++) v[j] = br[j >> 2][j & 3];
+        } else {
+            octet_of(br, left, v);
+        }
+        if constexpr (TERMS == 2) {
+            watch.octet(octet_peak(v), limit);
+            split_half2(v, limit_scale(limit), hi, lo);
+        } else if constexpr (HALF) {
+            const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+            hi = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));   // round to nearest even, overflow to infinity
+        } else {
+            hi = round_bf16x8(v);
         }
     };
+    // (With tests between them octets are stored one by one: held until the last is converted, 161 -> 160 1 x 7 on 17 x 17 at batch 16 in
+    // bfloat16, 64 x 128 outputs, takes 28.9 us instead of 24.2.)
     auto store_stage = [&](int buf, const uintx4 (&ar)[A_IT], const floatx4 (&br)[B_IT][2], int left) {
-        uintx4 hi[B_IT], lo[B_IT];
+        uintx4 hi[UNMASKED ? B_IT : 1], lo[UNMASKED ? B_IT : 1];
+        if constexpr (UNMASKED) {
+#pragma unroll
+            for (int i = 0; i < B_IT; i++) convert(br[i], left, hi[i], lo[i]);
+        }
+        store_filters(buf, ar);
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
-            float v[8];
-            if constexpr (PLAIN) {
-#pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = br[i][j >> 2][j & 3];
-            } else {
-                octet_of(br[i], left, v);
-            }
-            if constexpr (TERMS == 2) {
-                watch.octet(octet_peak(v), limit);
-                split_half2(v, limit_scale(limit), hi[i], lo[i]);
-            } else if constexpr (HALF) {
-                const floatx8 f = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
-                hi[i] = __builtin_bit_cast(uintx4, __builtin_convertvector(f, halfx8));   // round to nearest even, overflow to infinity
-            } else {
-                hi[i] = round_bf16x8(v);
-            }
+            if constexpr (!UNMASKED) convert(br[i], left, hi[0], lo[0]);
+            store_octet(buf, i, hi[UNMASKED ? i : 0], lo[UNMASKED ? i : 0]);
         }
-        store_octets(buf, ar, hi, lo);
     };
 
     typename M::acc_t acc[TM][TN];
@@ -243,7 +254,7 @@ struct ConvPipe {
     load_stage(PD, a_reg[0], b_reg[0], b_left[0]);
     __syncthreads();
     // (otherwise the compiler waits for all loads in every round, for registers that hold loads only on the way in)
-    if constexpr (PLAIN) __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    if constexpr (UNMASKED) __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
     for (int st0 = 0; st0 < stages; st0 += PD) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
@@ -252,7 +263,7 @@ struct ConvPipe {
             const uintx4 *Ab = lds + buf * STAGE + lk * (TERMS * BM) + wm * WTM + lc;
             const uintx4 *Bb = lds + buf * STAGE + A_SLOTS + slot_of(wn * WTN + lc, lk);   // (tiles are 32 pixels apart: the same exchange in all)
             // operands of the next unit are read ahead of a unit's matrix work, where registers allow it
-            constexpr int TURN = PLAIN && TERMS == 2 && KU > 1 && TMW * TNW != 2 ? 1 : 0;
+            constexpr int TURN = UNMASKED && TERMS == 2 && KU > 1 && TMW * TNW != 2 ? 1 : 0;
             uintx4 av[TURN + 1][TERMS][TM], bv[TURN + 1][TERMS][TN];
             auto read_unit = [&](int u) {
 #pragma unroll
@@ -265,7 +276,7 @@ struct ConvPipe {
             };
             const uintx4 (&ar)[A_IT] = a_reg[(s + 1) % PD];
             const floatx4 (&br)[B_IT][2] = b_reg[(s + 1) % PD];
-            if constexpr (PLAIN && TERMS == 2) {
+            if constexpr (UNMASKED && TERMS == 2) {
                 // The octets of the next stage are split between the matrix instructions of this one, a pair of values at a time.
                 constexpr int SLOTS = 3 * TM * TN * KU, PIECES = 5 * B_IT;
                 uintx4 hi[B_IT], lo[B_IT];
@@ -296,7 +307,9 @@ struct ConvPipe {
                         }
                     });
                 }
-                store_octets(buf ^ 1, ar, hi, lo);
+                store_filters(buf ^ 1, ar);
+#pragma unroll
+                for (int i = 0; i < B_IT; i++) store_octet(buf ^ 1, i, hi[i], lo[i]);
             } else {
 #pragma unroll
                 for (int u = 0; u < KU; u++) {
@@ -365,7 +378,8 @@ struct ConvPipe {
 
 constexpr int kFirstPipeVariant = 119;
 
-// The kernels of conv_pipe.hip, in the order of the lists above; [0] any filter, [1] 1 x 1 filters without groups
-extern const KernelPair kPipeKernels[][2];
+// The kernels of conv_pipe.hip and their PLAIN forms of conv_pipe_plain.hip, in the order of the lists above; [0] any filter, [1] 1 x 1 filters
+// without groups
+extern const KernelPair kPipeKernels[][2], kPipePlainKernels[][2];
 
 }  // namespace ios
