@@ -27,8 +27,9 @@ ios::LaunchChooser device_chooser() {
 
 ios::BatchChooser device_batches() {
     ios::DeviceContext &ctx = ios::DeviceContext::get();
-    return [&ctx](const std::vector<ios::ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const ios::PoolProblem *pool) {
-        return ctx.choose_batch(problems, share, remains, mixed, pool);
+    return [&ctx](const std::vector<ios::ConvProblem> &problems, const std::vector<int> &share, const std::vector<int> &stage, bool remains, bool mixed,
+                  const ios::PoolProblem *pool) {
+        return ctx.choose_batch(problems, share, stage, remains, mixed, pool);
     };
 }
 
@@ -236,7 +237,7 @@ static ios::LaunchChooser host_chooser() {
 
 static ios::BatchChooser host_batches() {
     if (!ios::planner_host_batches()) return nullptr;
-    return [](const std::vector<ios::ConvProblem> &, const std::vector<int> &, bool, bool mixed, const ios::PoolProblem *) {
+    return [](const std::vector<ios::ConvProblem> &, const std::vector<int> &, const std::vector<int> &, bool, bool mixed, const ios::PoolProblem *) {
         if (mixed && ios::planner_host_batches() < 2) return -1;
         int v = 0;
         while (!ios::conv_variant_batches(v)) v++;   // (the first of them takes any member of a mixed launch too)

@@ -47,9 +47,9 @@ struct ConvPipe {
 
     // Two terms: one limit for the inputs of the tile, by those of its first stage.  Where that does not serve all of them, the tile is
     // computed again.  The code is there twice: as a loop the compiler holds addresses, masks and zeros for the second time, 40 to 100
-    // registers.  The PLAIN form of the first attempt: what a tile with nothing beside it on its compute unit waits for is the sum of its steps (768 -> 192 on 17 x 17, a block of 64 x 128, per 16 k: 230 cycles for the operands from LDS, 320 for the
-    // matrix instructions, 450 to split an octet, 250 to store and for the barrier), and without the branches between them the split work lies
-    // under the matrix instructions.  That layer at batch 3 23.6 -> 21.7 us, at batch 64 31.8 -> 29.0; four such convolutions in a launch, 704 outputs,
+    // registers.  The PLAIN form of the first attempt: what a tile with nothing beside it on its compute unit waits for is the sum of its
+    // steps (768 -> 192 on 17 x 17, a block of 64 x 128, per 16 k: 230 cycles for the operands from LDS, 320 for the matrix instructions, 450 to
+    // split an octet, 250 to store and for the barrier), and without the branches between them the split work lies under the matrix instructions.  That layer at batch 3 23.6 -> 21.7 us, at batch 64 31.8 -> 29.0; four such convolutions in a launch, 704 outputs,
     // batch 16 31.6 -> 29.2, batch 64 94.2 -> 92.2.  With one term the matrix work is a third of that and the two ways out of each test cost as much as the
     // conversion: passes of Inception-v3 in half at batch 7 660 -> 619 us, in bfloat16 at batch 64 2298 -> 2248.
     // A kernel holds one of the two forms: both in one take the registers of the larger for either (one term, 64 x 64 outputs, any filter 106

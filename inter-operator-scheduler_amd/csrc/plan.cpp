@@ -1253,7 +1253,7 @@ private:
         batch.ops = std::move(ops);
         batch.stage = plan_.ops[batch.ops[0]].stage;
         std::vector<ConvProblem> problems;
-        std::vector<int> their_share;
+        std::vector<int> their_share, their_stage;
         bool remains = false;
         const PoolProblem *pool = nullptr;
         for (int i : batch.ops) {
@@ -1263,11 +1263,12 @@ private:
             }
             problems.push_back(plan_.convs[plan_.ops[i].conv].problem);
             their_share.push_back(share[plan_.ops[i].conv]);
+            their_stage.push_back(plan_.ops[i].stage);
             if (plan_.stages[plan_.ops[i].stage].size() == 1) continue;
             for (const auto &group : plan_.stages[plan_.ops[i].stage])   // (what runs at the beginning of their stages)
                 remains = remains || (!group.empty() && std::find(batch.ops.begin(), batch.ops.end(), group[0]) == batch.ops.end());
         }
-        batch.variant = batch_chooser_(problems, their_share, remains, mixed, pool);
+        batch.variant = batch_chooser_(problems, their_share, their_stage, remains, mixed, pool);
         if (batch.variant < 0) return;
         for (int i : batch.ops) {
             PlanOp &op = plan_.ops[i];

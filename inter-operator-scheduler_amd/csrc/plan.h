@@ -149,9 +149,11 @@ enum class InputUse { Resident, InParts, Once };
 typedef std::function<ConvLaunch(const ConvProblem &, int share)> LaunchChooser;
 
 // Kernel configuration on which convolutions of one input (`mixed`: of any inputs and windows) run in a launch of their own, or -1 where
-// they are faster by themselves; `share` of each as above.  `remains`: other operations of their stage lose the launch that they shared
-// with them.  `pool`: it runs beside mixed convolutions.
-typedef std::function<int(const std::vector<ConvProblem> &, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool)> BatchChooser;
+// they are faster by themselves; `share` of each as above, `stage`: in the schedule (those of one run beside each other where the share is
+// more than one).  `remains`: other operations of their stage lose the launch that they shared with them.  `pool`: it runs beside mixed
+// convolutions.
+typedef std::function<int(const std::vector<ConvProblem> &, const std::vector<int> &share, const std::vector<int> &stage, bool remains, bool mixed,
+                          const PoolProblem *pool)> BatchChooser;
 
 // Compile a document.  `extra` is the input-shape document of stage mode ({name: [C, H, W]}).
 // Throws std::runtime_error on malformed documents, unknown operator types, non-topological schedules

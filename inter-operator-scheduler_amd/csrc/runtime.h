@@ -80,7 +80,8 @@ public:
 
     // Kernel configuration on which these convolutions of one input share a launch, or -1 where the measurement finds them faster by
     // themselves (as choose_launch has them); see BatchChooser.  Without autotuning there are no batches, but on a forced configuration.
-    int choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool);
+    int choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, const std::vector<int> &stage, bool remains, bool mixed,
+                     const PoolProblem *pool);
 
     // Static device scratch of the entry point that allocates nothing: address on device 0 (resolved once, when the
     // context is created) and size in bytes.
@@ -95,7 +96,8 @@ public:
 
 private:
     bool serves_batch(const std::vector<ConvProblem> &problems, int variant, bool mixed) const;
-    int tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool);
+    int tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, const std::vector<int> &stage, bool remains, bool mixed,
+                   const PoolProblem *pool);
     DeviceContext();
     TunedConv tune_conv(const ConvProblem &p);
     float *tuning_buffer(int which, size_t floats);

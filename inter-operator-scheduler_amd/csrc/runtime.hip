@@ -19,6 +19,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <set>
 #include <sstream>
 #include <stdexcept>
 
@@ -470,9 +472,11 @@ bool DeviceContext::serves_batch(const std::vector<ConvProblem> &problems, int v
     return true;
 }
 
-// Both ways on scratch tensors of the real shapes: every convolution as it runs without a batch (beside the others where one of them
-// shares its stage), and all of them in a launch on every configuration that has such a kernel.
-int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool) {
+// Both ways on scratch tensors of the real shapes: every convolution as it runs without a batch (those of one stage whose share is more than
+// one beside each other, in a fused launch or on streams, as the executor has them), and all of them in a launch on every configuration that
+// has such a kernel.
+int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, const std::vector<int> &stage, bool remains, bool mixed,
+                              const PoolProblem *pool) {
     const size_t count = problems.size();
     bool parallel = false;
     for (int s : share) parallel = parallel || s > 1;
@@ -550,51 +554,106 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
     };
     constexpr int kReps = 8;
     // by themselves
-    std::vector<WorkItem> items;
-    FusedHeader header{};
-    int blocks = 0, smem_bytes = 0, threads = 256;
+    struct Level {   // what a stage has in a fused launch
+        std::vector<WorkItem> items;
+        std::vector<size_t> members;
+        FusedHeader header{};
+        int blocks = 0, smem_bytes = 0, threads = 256;
+        bool wide = false, pool = false;
+        size_t first_item = 0;
+        void add(WorkItem item) {
+            item.first_block = blocks;
+            header.first_block[items.size()] = blocks;
+            blocks += item.num_blocks;
+            items.push_back(item);
+            header.num_items = (int)items.size();
+        }
+    };
+    std::map<int, Level> levels;
     std::vector<size_t> single;
-    bool wide = false;
     for (size_t i = 0; i < count; i++) {
         launch_pack_filters(problems[i], alone[i], memory + filters_at[i], memory + packed_at[i], stream);
         const ConvDispatch d = make_conv_dispatch(problems[i], alone[i], x[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
                                                   workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr));
-        if (!parallel || !fused_executor() || !conv_variant(d.variant).fusable() || d.has_reduce) {
+        if (share[i] <= 1 || !fused_executor() || !conv_variant(d.variant).fusable() || d.has_reduce) {
             single.push_back(i);
             continue;
         }
-        WorkItem item = conv_work_item(d);
-        item.first_block = blocks;
-        header.first_block[items.size()] = blocks;
-        blocks += item.num_blocks;
-        smem_bytes = std::max(smem_bytes, d.smem_bytes);
-        threads = std::max(threads, d.threads);
-        wide = wide || conv_variant(d.variant).needs_wide();
-        items.push_back(item);
+        Level &level = levels[stage[i]];
+        level.add(conv_work_item(d));
+        level.members.push_back(i);
+        level.smem_bytes = std::max(level.smem_bytes, d.smem_bytes);
+        level.threads = std::max(level.threads, d.threads);
+        level.wide = level.wide || conv_variant(d.variant).needs_wide();
     }
-    if (pool != nullptr && !items.empty()) {
+    for (auto it = levels.begin(); it != levels.end();) {   // (no fused launch holds both: build_fused launches such a level one by one)
+        const Level &level = it->second;
+        if (level.wide && level.threads > 512) {
+            single.insert(single.end(), level.members.begin(), level.members.end());
+            it = levels.erase(it);
+        } else {
+            ++it;
+        }
+    }
+    const bool pool_alone = pool != nullptr && levels.empty();
+    if (pool != nullptr && !pool_alone) {   // (of the stage that all members are of)
+        Level &level = levels.begin()->second;
         WorkItem item;
         memset(&item, 0, sizeof(item));
         item.kind = WORK_POOL;
         item.pool = make_pool_args(beside.p, beside.x, beside.y, false, &item.num_blocks);
-        item.num_blocks = std::max(1, (item.num_blocks * 256 + threads - 1) / threads);
-        item.threads = threads;
-        item.first_block = blocks;
-        header.first_block[items.size()] = blocks;
-        blocks += item.num_blocks;
-        items.push_back(item);
+        item.num_blocks = std::max(1, (item.num_blocks * 256 + level.threads - 1) / level.threads);
+        item.threads = level.threads;
+        level.add(item);
     }
-    const bool pool_alone = pool != nullptr && items.empty();
-    if (wide && threads > 512) return -1;   // (a level of such operators is not one launch: see build_fused)
-    header.num_items = (int)items.size();
+    std::vector<WorkItem> items;
+    for (auto &entry : levels) {
+        entry.second.first_item = items.size();
+        items.insert(items.end(), entry.second.items.begin(), entry.second.items.end());
+    }
     WorkItem *device_items = reinterpret_cast<WorkItem *>(memory + items_at);
     if (!items.empty()) stage_.upload(device_items, items.data(), items.size() * sizeof(WorkItem), stream);
-    const float apart = measure(kReps, (int)single.size() + 1, [&] {
+    struct Joins {   // of streams beside the main one
+        std::vector<hipEvent_t> events;
+        ~Joins() {
+            for (hipEvent_t event : events) (void)hipEventDestroy(event);
+        }
+    } joins;
+    auto beside_others = [&](size_t i) {   // on a stream of its own
+        return !fused_executor() && share[i] > 1 && std::count(stage.begin(), stage.end(), stage[i]) > 1;
+    };
+    for (size_t i = 0; i <= count; i++) {   // (one event to fork)
+        joins.events.push_back(nullptr);
+        IOS_HIP(hipEventCreateWithFlags(&joins.events.back(), hipEventDisableTiming));
+    }
+    auto launch_alone = [&](size_t i, hipStream_t on) {
+        launch_conv_mfma(problems[i], alone[i], x[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
+                         workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr), on);
+    };
+    const int launches_apart = (int)(3 * single.size() + levels.size() + 2);   // (the joins among them)
+    const float apart = measure(kReps, launches_apart, [&] {
         if (pool_alone) launch_pool(beside.p, beside.x, beside.y, stream);
-        if (!items.empty()) launch_fused(threads, device_items, items.data(), header, blocks, smem_bytes, num_cus_, stream);
-        for (size_t i : single)
-            launch_conv_mfma(problems[i], alone[i], x[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
-                             workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr), stream);
+        for (const auto &entry : levels) {
+            const Level &level = entry.second;
+            launch_fused(level.threads, device_items + level.first_item, items.data() + level.first_item, level.header, level.blocks, level.smem_bytes, num_cus_, stream);
+        }
+        for (size_t n = 0; n < single.size(); n++) {
+            const size_t i = single[n];
+            if (!beside_others(i)) {
+                launch_alone(i, stream);
+                continue;
+            }
+            size_t end = n;   // (members come by stage)
+            while (end < single.size() && stage[single[end]] == stage[i] && beside_others(single[end])) end++;
+            IOS_HIP(hipEventRecord(joins.events[count], stream));
+            for (size_t m = n + 1; m < end; m++) IOS_HIP(hipStreamWaitEvent(streams_[m - n], joins.events[count], 0));
+            for (size_t m = n; m < end; m++) launch_alone(single[m], streams_[m - n]);
+            for (size_t m = n + 1; m < end; m++) {
+                IOS_HIP(hipEventRecord(joins.events[m], streams_[m - n]));
+                IOS_HIP(hipStreamWaitEvent(stream, joins.events[m], 0));
+            }
+            n = end - 1;
+        }
     });
     // together
     float best = 1e30f;
@@ -622,14 +681,21 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
     return best + (remains ? kLaunchMs : 0.f) < kNoise * apart ? variant : -1;
 }
 
-int DeviceContext::choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, bool remains, bool mixed, const PoolProblem *pool) {
+int DeviceContext::choose_batch(const std::vector<ConvProblem> &problems, const std::vector<int> &share, const std::vector<int> &stage, bool remains, bool mixed,
+                                const PoolProblem *pool) {
     if (forced_variant_ >= 0) {
         const bool serves = mixed ? serves_batch(problems, forced_variant_, true) : conv_variant_batches(forced_variant_);
         return forced_split_k_ <= 1 && serves ? forced_variant_ : -1;
     }
     if (!autotune_ || forced_split_k_ > 0) return -1;
     std::string key = (mixed ? "mixed " : "") + settings_token() + (precision_ == PREC_BF16 ? " bf16" : precision_ == PREC_FP16 ? " fp16" : "") + (remains ? " remains" : "");
-    for (size_t i = 0; i < problems.size(); i++) key += " | " + conv_signature(problems[i]) + " " + std::to_string(share[i]);
+    const std::set<int> stages(stage.begin(), stage.end());
+    bool parallel = false;
+    for (int s : share) parallel = parallel || s > 1;
+    for (size_t i = 0; i < problems.size(); i++) {
+        key += " | " + conv_signature(problems[i]) + " " + std::to_string(share[i]);
+        if (parallel) key += "@" + std::to_string(std::distance(stages.begin(), stages.find(stage[i])));   // (who runs beside whom)
+    }
     if (pool != nullptr) {
         key += " | pool";
         for (int n : {pool->C, pool->H, pool->W, pool->KH, pool->KW, pool->sh, pool->sw, pool->ph, pool->pw, pool->is_max})
@@ -643,7 +709,7 @@ int DeviceContext::choose_batch(const std::vector<ConvProblem> &problems, const 
         }
     }
     if (it == batched.end()) {
-        it = batched.emplace(key, tune_batch(problems, share, remains, mixed, pool)).first;
+        it = batched.emplace(key, tune_batch(problems, share, stage, remains, mixed, pool)).first;
         FILE *f = tune_cache_path_.empty() ? nullptr : fopen(tune_cache_path_.c_str(), "a");
         if (f != nullptr) {
             fprintf(f, "batch\t%s\t%s\n", key.c_str(), it->second >= 0 ? conv_variant(it->second).name : "none");
