@@ -215,13 +215,13 @@ void launch_pack_depthwise(const ConvProblem &p, const float *w, float *packed, 
 constexpr int kLine = 16;   // floats
 constexpr int kTileRow = 240, kTileChannels = 32;
 
-// Floats [at, at + 4) of `total`, at a multiple of four; those outside are zero.
-__device__ __forceinline__ pw_floatx4 line_quad(const float *nchw, long long at, long long total) {
-    if (at + 4 <= total) return *reinterpret_cast<const pw_floatx4 *>(nchw + at);
+// Floats [at, at + 4) behind `line`, at a multiple of four; those outside [lead, total) are zero and not read.
+__device__ __forceinline__ pw_floatx4 line_quad(const float *line, long long at, int lead, long long total) {
+    if (at >= lead && at + 4 <= total) return *reinterpret_cast<const pw_floatx4 *>(line + at);
     pw_floatx4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        if (at + j < total) v[j] = nchw[at + j];
+        if (at + j >= lead && at + j < total) v[j] = line[at + j];
     return v;
 }
 
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void to_view_kernel(const float *nchw, float *
         }
         return;
     }
-    nchw -= lead;
+    const float *line = nchw - lead;   // (what lies in front of the first element is not read)
     constexpr int STRIDE = kTileRow + kLine + 4;
     __shared__ float rows[kTileChannels * STRIDE];
     const int tid = threadIdx.x;
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void to_view_kernel(const float *nchw, float *
             const int c = wave + 4 * i;
             const long long at = first + c * plane, from = at & ~(long long)(kLine - 1);
             v[i] = pw_floatx4{0.f, 0.f, 0.f, 0.f};
-            if (c0 + c < C && 4 * lane < (int)(at - from) + pixels) v[i] = line_quad(nchw, from + 4 * lane, total);
+            if (c0 + c < C && 4 * lane < (int)(at - from) + pixels) v[i] = line_quad(line, from + 4 * lane, lead, total);
         }
         __syncthreads();
 #pragma unroll
