@@ -97,8 +97,10 @@ struct ConvWindow {
     const unsigned plane_bytes = (unsigned)a.OCgP * 16u;
     const unsigned tap_bytes = (unsigned)(a.ICgP >> 3) * TERMS * plane_bytes, chunk_bytes = 2u * TERMS * plane_bytes;
 
-    // The filters of a pass fit no L2: all of what the block will read is requested at once, a word of every line, shared out over the
-    // blocks of the XCD that read the same.  Requested two taps ahead only, each of them waits for memory.  With filters that no cache
+    // The filters of a pass fit no L2: what the block will read is requested at once, a word of every line, shared out over the
+    // blocks of the XCD that read the same: the first kTouches * T lines for each of them, all of a tile's where enough of them share it (a tile of
+    // 448 channels 3 x 3, two terms and 64 outputs has 8064; three blocks of 256 threads request 3072).  Requested two taps ahead only, each
+    // of them waits for memory.  With filters that no cache
     // holds, bfloat16 at batch 64, 192 -> 192 1 x 7 on 17 x 17 took 25.7 us (20.6 with filters in the L2) and takes 20.2, 256 -> 256 3 x 3 on
     // 14 x 14 38.8 (26.8) -> 27.2, 448 -> 384 3 x 3 on 8 x 8 48.7 (32.3) -> 34.3; two terms at batch 7, 256 -> 256 38.5 -> 32.8.  It costs
     // 0.2 to 1 us where they are in the L2.
