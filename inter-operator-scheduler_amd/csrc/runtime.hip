@@ -626,9 +626,11 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
         joins.events.push_back(nullptr);
         IOS_HIP(hipEventCreateWithFlags(&joins.events.back(), hipEventDisableTiming));
     }
-    auto launch_alone = [&](size_t i, hipStream_t on) {
+    const bool placement_known = !(parallel && exec_mode_ == ExecMode::Graph);   // (captured forks run on streams that nobody knows)
+    auto launch_alone = [&](size_t i, size_t group) {
         launch_conv_mfma(problems[i], alone[i], x[i], memory + packed_at[i], memory + filters_at[i], memory + filters_at[i], y[i],
-                         workspace != nullptr ? workspace + ws_at[i] : nullptr, split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr), on);
+                         workspace != nullptr ? workspace + ws_at[i] : nullptr,
+                         split_reduce(tickets != nullptr ? tickets + ctr_at[i] : nullptr, (int)group, placement_known), streams_[group]);
     };
     const int launches_apart = (int)(3 * single.size() + levels.size() + 2);   // (the joins among them)
     const float apart = measure(kReps, launches_apart, [&] {
@@ -640,14 +642,14 @@ int DeviceContext::tune_batch(const std::vector<ConvProblem> &problems, const st
         for (size_t n = 0; n < single.size(); n++) {
             const size_t i = single[n];
             if (!beside_others(i)) {
-                launch_alone(i, stream);
+                launch_alone(i, 0);
                 continue;
             }
             size_t end = n;   // (members come by stage)
             while (end < single.size() && stage[single[end]] == stage[i] && beside_others(single[end])) end++;
             IOS_HIP(hipEventRecord(joins.events[count], stream));
             for (size_t m = n + 1; m < end; m++) IOS_HIP(hipStreamWaitEvent(streams_[m - n], joins.events[count], 0));
-            for (size_t m = n; m < end; m++) launch_alone(single[m], streams_[m - n]);
+            for (size_t m = n; m < end; m++) launch_alone(single[m], m - n);
             for (size_t m = n + 1; m < end; m++) {
                 IOS_HIP(hipEventRecord(joins.events[m], streams_[m - n]));
                 IOS_HIP(hipStreamWaitEvent(stream, joins.events[m], 0));

@@ -14,13 +14,13 @@ import ios
 from ios.contrib import ios_runtime as rt
 from test_conv_batches import heads
 from test_gpu_parity import assert_close, ios_oracle
-graph = heads((384, 17, 17), (192, 160, 160, 192), 1, 0, 'sequential')
+graph = heads(*SHAPE, 1, 0, 'sequential')
 block = graph.blocks[0]
 names = [name for stage in block.stages for group in stage for name in group]
 block.stages = [[[n] for n in names[first:first + WIDTH]] if 1 <= first < 5 else [[names[first]]] for first in [0, *range(1, 5, WIDTH), *range(5, len(names))]]
 rt.set_option('executor', EXECUTOR)
-x = np.random.default_rng(1).standard_normal((12, *graph.enter_node.output_shape)).astype(np.float32)
-with rt.Session(graph, 12) as session:
+x = np.random.default_rng(1).standard_normal((BATCH, *graph.enter_node.output_shape)).astype(np.float32)
+with rt.Session(graph, BATCH) as session:
     session.load_weights()
     session.set_input(x)
     for _ in range(3):
@@ -30,10 +30,10 @@ with rt.Session(graph, 12) as session:
 '''
 
 
-def run(path, executor, width):
+def run(path, executor, width, shape=((384, 17, 17), (192, 160, 160, 192)), batch=12):
     here = os.path.dirname(os.path.abspath(__file__))
     env = dict(os.environ, IOS_TUNE_CACHE=str(path), PYTHONPATH=os.path.join(os.path.dirname(here), 'inter-operator-scheduler_amd') + ':' + here)
-    done = subprocess.run([sys.executable, '-c', f'EXECUTOR, WIDTH = {executor!r}, {width}\n' + PROGRAM], env=env, capture_output=True, text=True, timeout=100)
+    done = subprocess.run([sys.executable, '-c', f'EXECUTOR, WIDTH, SHAPE, BATCH = {executor!r}, {width}, {shape!r}, {batch}\n' + PROGRAM], env=env, capture_output=True, text=True, timeout=100)
     assert done.returncode == 0, done.stderr[-2000:]
     return done.stdout
 
@@ -61,3 +61,19 @@ def test_wide_registers_beside_1024_threads(tmp_path):
     path.write_text('\n'.join(' '.join(line) for line in lines) + '\n')
     assert 'shared 4' in run(path, 'fused', 4)
     assert 'none' not in [line.split('\t')[2] for line in path.read_text().splitlines() if line.startswith('batch\t') and 'mixed' not in line]
+
+
+@pytest.mark.parametrize('executor', ['streams', 'graph'])
+def test_sums_in_slices_beside_each_other(tmp_path, executor):
+    """Slices of K that meet in the L2 of one XCD: which one it is depends on the stream, and on a captured fork nobody knows."""
+    path = tmp_path / 'choices'
+    shape, batch = ((640, 8, 8), (96, 64, 128, 80)), 2
+    run(path, executor, 4, shape, batch)
+    lines = [line.split() for line in path.read_text().splitlines() if not line.startswith('batch\t')]
+    heads = [line for line in lines if line[1] == '640']
+    assert len(heads) == 4
+    for line in heads:
+        line[13:] = ['wq_m32n32_w4_t16', '4'] * 4
+    path.write_text('\n'.join(' '.join(line) for line in lines) + '\n')
+    run(path, executor, 4, shape, batch)
+    assert sum(line.startswith('batch\t') and 'mixed' not in line for line in path.read_text().splitlines()) == 1   # (measured again)
