@@ -62,6 +62,18 @@ def network_roofline_ms(ops, parallel):
     return sum(max(groups.values()) for groups in stages.values())
 
 
+def result_line(result):
+    """One line of JSON, numbers to seven digits, no spaces: with all of them, and the kernels that a run happens to choose, it came to more than
+    20 KB at times, which is where readers of the end of an output may cut it."""
+    def short(value):
+        if isinstance(value, dict):
+            return {key: short(v) for key, v in value.items()}
+        if isinstance(value, (list, tuple)):
+            return [short(v) for v in value]
+        return float(f'{value:.7g}') if isinstance(value, float) else value
+    return json.dumps(short(result), separators=(',', ':'))
+
+
 def progress(text):
     """A line on stderr per phase: a run that takes minutes says what it is doing (stdout carries the one JSON line)."""
     print(f'bench.py [{time.strftime("%H:%M:%S")}] {text}', file=sys.stderr, flush=True)
@@ -684,7 +696,7 @@ def main():
                                             f'(torch-CPU fp32, {threads} threads), {cpu_ms:.1f} ms each'}
         result['oracle'] = oracle_check(np, opt_out, cpu_out)
         result['matches_cpu_oracle'] = result['oracle']['matches_cpu_oracle']
-    print(json.dumps(result))
+    print(result_line(result))
 
 
 if __name__ == '__main__':
